@@ -133,16 +133,20 @@ class RaggedBatch:
             self._tiles[key] = (both[:len(rec)], both[len(rec):])
         return self._tiles[key]
 
-    def tiles(self, tq: int) -> torch.Tensor:
-        """[n_tiles, 4] int32 {b, first query position, count, first row}: each request's rows cut into runs of at most ``tq``."""
-        t = self._tiles.get(tq)
+    def tiles(self, tq: int, longest_first: bool = False) -> torch.Tensor:
+        """[n_tiles, 4] int32 {b, first query position, count, first row}: each request's rows cut into runs of at most ``tq``; with
+        ``longest_first`` those with the most positions in front of them come first."""
+        key = ("longest first", tq) if longest_first else tq
+        t = self._tiles.get(key)
         if t is None:
             rows, r0 = [], 0
             for b, (c, s) in enumerate(zip(self.counts, self.starts)):
                 for o in range(0, c, tq):
                     rows.append((b, s + o, min(tq, c - o), r0 + o))
                 r0 += c
-            t = self._tiles[tq] = torch.tensor(rows, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
+            if longest_first:
+                rows.sort(key=lambda r: -r[1])
+            t = self._tiles[key] = torch.tensor(rows, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
         return t
 
 
@@ -326,7 +330,9 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
         wide = int(N.layers().jl_attn_sweep_wide_tile_rows(_code(q.dtype), H, G, Gv, D, Dv, k_cache.stride(0), v_cache.stride(0),
                                                            int(v_cache.data_ptr() == k_cache.data_ptr())))
         if wide > 0:
-            tq, tiles = wide, batch.tiles(wide)
+            # what starts last should be short (4 x 2048 tokens, 16 heads of 128 over 4 key heads: 175 -> 137 us).  The 32-row kernel keeps the
+            # requests' order, in which neighbours share keys (over a latent of 512 the sorted order was 3 % slower)
+            tq, tiles = wide, batch.tiles(wide, longest_first=True)
     elif groups < SWEEP_SPLIT_BELOW_GROUPS:
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
         splits = max(1, min(-(-reach // 128), SWEEP_SPLIT_WORKGROUPS // groups, 64))

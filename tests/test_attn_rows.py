@@ -1,0 +1,71 @@
+"""The 128-row attention tiles of long portions at the sizes where they can go wrong, against attention in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, starts, counts, pages, page, H, G, Gv, D, Dv, scale, window, chunk, cap, sink):
+    out, r0 = [], 0
+    for s, n, tab in zip(starts, counts, pages):
+        total = s + n
+        tok = torch.tensor([tab[j // page] * page + j % page for j in range(total)], device=q.device)
+        qq = q[r0:r0 + n].double().view(n, H, D).transpose(0, 1)
+        kk = k[tok].double().view(total, G, D).transpose(0, 1).repeat_interleave(H // G, 0)
+        vv = v[tok].double().view(total, Gv, Dv).transpose(0, 1)[torch.arange(H, device=q.device) // (H // G) % Gv]
+        z = qq @ kk.transpose(1, 2) * scale
+        if cap:
+            z = cap * torch.tanh(z / cap)
+        i, j = torch.arange(s, total, device=q.device).view(n, 1), torch.arange(total, device=q.device).view(1, total)
+        see = j <= i
+        if window:
+            see = see & (i - j < window)
+        if chunk:
+            see = see & (i // chunk == j // chunk)
+        z = z.masked_fill(~see, float("-inf"))
+        if sink is not None:
+            z = torch.cat([z, sink.double().view(H, 1, 1).expand(H, n, 1)], -1)
+        w = torch.softmax(z, -1)[..., :total]
+        out.append((w @ vv).transpose(0, 1).reshape(n, H * Dv))
+        r0 += n
+    return torch.cat(out)
+
+
+# key and value widths at and beside the multiples of 64 (key rows in LDS) and 32 / 64 / 128 (value rows)
+@pytest.mark.parametrize("H,G,Gv,D,Dv,window,chunk,cap,page,pad", [
+    (16, 4, 4, 128, 128, 0, 0, 0.0, 64, 0), (16, 16, 16, 64, 64, 0, 0, 0.0, 64, 0), (16, 2, 2, 8, 32, 0, 0, 0.0, 64, 0), (24, 4, 4, 72, 96, 100, 0, 0.0, 64, 0),
+    (16, 4, 2, 136, 64, 0, 0, 0.0, 48, 0), (20, 20, 20, 192, 128, 65, 0, 0.0, 64, 0), (40, 1, 1, 200, 96, 0, 0, 0.0, 64, 4), (16, 2, 2, 256, 128, 0, 0, 0.0, 64, 0),
+    (16, 4, 4, 128, 128, 0, 100, 5.0, 64, 0), (16, 1, 0, 160, 128, 0, 0, 0.0, 64, 0), (16, 1, 0, 96, 64, 63, 0, 0.0, 64, 4), (33, 1, 0, 256, 32, 0, 64, 2.0, 40, 0),
+])
+def test_wide_tiles(H, G, Gv, D, Dv, window, chunk, cap, page, pad):
+    """Unequal requests, two of them continuing inside a page; ``pad``: rows of the pools start at 8-byte borders only; Gv 0: the values are the key
+    rows' first columns; pools hold NaN wherever nothing was written."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt = "cuda", torch.bfloat16
+    starts, counts = [0, 37, 1, 0], [-(-16384 // H), 131, 64, 33]
+    g = torch.Generator(device=dev).manual_seed(D + H)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dt)
+    need = [-(-(s + n) // page) for s, n in zip(starts, counts)]
+    ids = torch.randperm(sum(need) + 3, generator=torch.Generator().manual_seed(H)).tolist()
+    pages = [[ids.pop() for _ in range(n)] for n in need]
+    tokens = (sum(need) + 3) * page
+    nan = lambda width: torch.full((tokens, width), float("nan"), dtype=dt, device=dev)
+    kp = nan(G * D + pad)
+    k = kp[:, :G * D]
+    v = k[:, :Dv] if Gv == 0 else nan(Gv * Dv + pad)[:, :Gv * Dv]
+    for s, n, tab in zip(starts, counts, pages):
+        tok = torch.tensor([tab[j // page] * page + j % page for j in range(s + n)], device=dev)
+        k[tok] = rnd(s + n, G * D)
+        if Gv:
+            v[tok] = rnd(s + n, Gv * Dv)
+    q, sink = rnd(sum(counts), H * D), torch.randn(H, generator=g, device=dev)
+    batch = LO.RaggedBatch.build(counts, starts, [0, 1, 2, 3], pages, page, dev)
+    gate = rnd(sum(counts), H)
+    got = LO.attn_sweep(q, k, v, batch, H, G, D, Dv, D ** -0.5, window, value_heads=Gv, float_out=True, sink=sink, gate=gate, gate_per_head=True, chunk=chunk, softcap=cap)
+    assert ("longest first", 128 // min(H // G, 32)) in batch._tiles, "the 128-row form did not run"
+    want = reference(q, k, v, starts, counts, pages, page, H, G, Gv or 1, D, Dv, D ** -0.5, window, chunk, cap, sink)
+    want = (want.view(-1, H, Dv) * torch.sigmoid(gate.double()).unsqueeze(-1)).view_as(want)
+    assert torch.isfinite(got).all()
+    # weights are rounded to bfloat16 (2 ** -9 relative, independently): a sum of them is off by less than that of its largest terms
+    err = (got.double() - want).abs()
+    assert err.max() < 2.0 ** -7 * want.abs().max() and err.norm() < 2.0 ** -8 * want.norm()
