@@ -322,7 +322,6 @@ class _LayerLibs:
 
     def __init__(self):
         self._libs = {}
-        self._last = None
 
     def _load(self, group: str):
         from . import _build
@@ -356,11 +355,13 @@ class _LayerLibs:
     def __getattr__(self, name: str):
         if name.startswith("_"):
             raise AttributeError(name)
-        if name == "jl_last_error":                  # the message of the library that was called last
-            return (self._last or self._libs.get("layers") or self._load("layers")).jl_last_error
+        fn = getattr(self._library(name), name)
+        setattr(self, name, fn)                      # the next call finds it without coming here
+        return fn
+
+    def _library(self, name: str):
         group = "layers_seq" if name in _SEQ_SYMBOLS else "layers"
-        self._last = self._libs.get(group) or self._load(group)
-        return getattr(self._last, name)
+        return self._libs.get(group) or self._load(group)
 
 
 _LAYERS = None
@@ -378,7 +379,7 @@ def layers():
 def check_layers(rc: int, what: str = ""):
     if rc == 0:
         return
-    msg = layers().jl_last_error()
+    msg = layers()._library(what.split("(")[0]).jl_last_error()          # each library keeps its own message
     msg = msg.decode() if isinstance(msg, (bytes, bytearray)) else str(msg)
     text = f"{what}: {msg}" if what else msg
     if rc == -1:

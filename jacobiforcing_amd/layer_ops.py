@@ -26,11 +26,14 @@ DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(device: torch.device):
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream) if device.type == "cuda" else None
+    """The current stream's handle (the raw one: no stream object is made for every launch)."""
+    if device.type != "cuda":
+        return None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _code(dt: torch.dtype) -> int:
@@ -90,11 +93,21 @@ class RaggedBatch:
                 raise ValueError(f"request {b}: {t.size} pages do not hold {starts[b] + counts[b]} tokens")
             kv[row0[b]:row0[b + 1]] = t[pos // page_size] * page_size + pos % page_size
             row_pos[row0[b]:row0[b + 1]] = pos
-        dev = torch.device(device)
+        # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on
+        tables = [seq.ravel(), bt.ravel(), np.repeat(np.arange(B, dtype=np.int32), np.asarray(counts, dtype=np.int64)), row_pos]
+        at = [2 * (kv.size + kv.size % 2)]
+        for t in tables:
+            at.append(at[-1] + (t.size + 3) // 4 * 4)
+        host = np.empty(at[-1] // 2, dtype=np.int64)
+        host[:kv.size] = kv
+        words = host.view(np.int32)
+        for t, a in zip(tables, at):
+            words[a:a + t.size] = t
+        up = torch.from_numpy(host).to(torch.device(device))
+        w32 = up.view(torch.int32)
+        d_seq, d_bt, d_req, d_pos = (w32[a:a + t.size] for t, a in zip(tables, at))
         return cls(B=B, N=int(row0[-1]), counts=list(map(int, counts)), starts=list(map(int, starts)),
-                   seq=torch.from_numpy(seq).to(dev), kv_slot=torch.from_numpy(kv).to(dev), tables=torch.from_numpy(bt).to(dev),
-                   row_req=torch.from_numpy(np.repeat(np.arange(B, dtype=np.int32), np.asarray(counts, dtype=np.int64))).to(dev),
-                   pos=torch.from_numpy(row_pos).to(dev),
+                   seq=d_seq.view(B, 4), kv_slot=up[:kv.size], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos,
                    page_size=int(page_size), max_pos=max(int(s) + int(c) for s, c in zip(starts, counts)), max_page=int(bt.max()),
                    max_slot=int(max(slots)), slots=list(map(int, slots)), _tiles={})
 

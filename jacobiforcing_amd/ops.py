@@ -46,13 +46,14 @@ def _stage(name: str, nbytes: int):
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(device: torch.device):
-    if device.type == "cuda":
-        return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
-    return None
+    """The current stream's handle (the raw one: no stream object is made for every launch)."""
+    if device.type != "cuda":
+        return None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _dtype_code(t: torch.Tensor) -> int:
