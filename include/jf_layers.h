@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 126
+#define JL_VERSION 127
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -101,6 +101,12 @@ typedef struct {
     float softcap;                /* > 0: scores pass softcap * tanh(s / softcap) behind scale and bias (the sink does not)            */
     float out_scale;              /* the outputs times this (1 when there is nothing to scale)                                        */
     int64_t out_ld;               /* row stride of `out` in elements (0: H*Dv)                                                       */
+    /* jl_attn_expanded only                                                                                                          */
+    const int32_t *key_base;      /* [B] the key / value row of request b's position j is key_base[b] + j (no pages)                  */
+    const void *k_tail;           /* the last k_tail_cols columns of every key head, shared by the heads: row stride k_tail_ld         */
+    int64_t k_tail_ld, q_ld;      /* q_ld: row stride of q                                                                            */
+    int32_t k_tail_cols;
+    int32_t reserved;
 } jl_attn_args;
 #define JL_OUT_SAME 0
 #define JL_OUT_F32 2
@@ -126,6 +132,19 @@ JL_API int64_t jl_attn_sweep_scratch_floats(int32_t n_tiles, int32_t H, int32_t 
  * rows to itself (scores, weights and outputs never leave its registers). */
 JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld,
                                         int32_t v_in_k);
+
+/* The wide form over keys and values that were built per head for this step (long portions of latent attention: keys and values from the latent
+ * by a product instead of queries brought to the latent), bfloat16, G = H, contiguous rows per request instead of pages: key head c of a row is
+ * columns c * (D - k_tail_cols) .. of k_cache followed by the row's k_tail_cols shared columns; value head c is columns c * Dv .. of v_cache.
+ * D, k_tail_cols % 8 == 0, D <= 256, Dv % 32 == 0 up to 128, row strides % 4 == 0.  Of jl_attn_args it reads what jl_attn_sweep reads except pages and splits;
+ * tiles of jl_attn_expanded_tile_rows() queries, in any order. */
+JL_API int jl_attn_expanded(const jl_attn_args *a, void *stream);
+JL_API int jl_attn_expanded_tile_rows(void);
+
+/* Rotation in place of the columns behind each head's first D: heads of D + rd columns side by side in q [N, ld], the first rot_dims of a head's rd
+ * columns turned by position (cos / sin [table_len, rot_dims / 2] float), pairs as `pairing` says. */
+JL_API int jl_rotate_heads(void *q, int dtype, int64_t N, int64_t ld, int32_t H, int32_t D, int32_t rd, int32_t rot_dims, const int32_t *pos, const float *cos_t,
+                           const float *sin_t, int64_t table_len, int32_t pairing, void *stream);
 
 /* Residual update, weighted sum over the streams of all depths, RMS norm — the layer whose result is kept beside the results of all
  * layers before it, and whose successor reads a learned mixture of them:

@@ -38,9 +38,14 @@ constexpr size_t ar_lds_bytes(int KU, int VU) { return 2 * (size_t)ar_tile_keys(
 template <int U> __device__ __forceinline__ int ar_key_unit(int r, int u) { return U % 16 == 0 ? u ^ (r & 15) : u ^ ((r >> 1) & 7); }
 template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { return U == 16 ? u ^ ((r & 3) << 2) : u ^ ((r & 2) << 1); }
 
-template <int KU, int VU, bool V_IN_K>                                                  // D <= 8 * KU, Dv <= 8 * VU; V_IN_K: the values are the key rows' first columns
+// where keys and values come from: pages of pools, pages whose key rows hold the values in their first columns, or contiguous rows per request whose heads
+// share their last columns (keys and values built for this step)
+enum { AR_PAGED, AR_V_IN_K, AR_BUILT };
+
+template <int KU, int VU, int SRC>                                                      // D <= 8 * KU, Dv <= 8 * VU
 __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a, int HF, int TQ, int HB) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    constexpr bool V_IN_K = SRC == AR_V_IN_K, BUILT = SRC == AR_BUILT;
     constexpr int KT = ar_tile_keys(KU), HALVES = KT / 32, NDV = VU / 4, VROWS = V_IN_K ? 0 : KT * VU;
     constexpr int KPF = KT * KU / AR_THREADS, VPF = KT * VU / AR_THREADS;
     const int H = a.H, D = a.D, Dv = a.Dv, per_group = H / a.G;
@@ -59,10 +64,12 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     const int chunk = a.chunk;
     const int lo = chunk > 0 ? i0 - i0 % chunk : (i0 - window + 1 > 0 ? i0 - window + 1 : 0);      // lowest key the tile's first row sees
     const int n_keys = i_max + 1 - lo;
-    const int *bt = a.block_tables + (int64_t)b * a.bt_stride;
-    const bf16_t *kc = (const bf16_t *)a.k_cache + (int64_t)c * D;
+    const int *bt = BUILT ? nullptr : a.block_tables + (int64_t)b * a.bt_stride;
+    const int key_base = BUILT ? a.key_base[b] : 0;
+    const int Dh = BUILT ? D - a.k_tail_cols : D;                   // columns of a key head that are its own
+    const bf16_t *kc = (const bf16_t *)a.k_cache + (int64_t)c * Dh, *kt = (const bf16_t *)a.k_tail;
     const bf16_t *vc = (const bf16_t *)a.v_cache + (int64_t)(c % a.Gv) * Dv;
-    const int page_shift = (a.page_size & (a.page_size - 1)) == 0 ? __builtin_ctz(a.page_size) : -1;
+    const int page_shift = !BUILT && (a.page_size & (a.page_size - 1)) == 0 ? __builtin_ctz(a.page_size) : -1;
     for (int e = tid; e < 2 * BUF; e += AR_THREADS) buf0[e] = make_uint4(0, 0, 0, 0);      // columns beyond D / Dv and rows beyond the last key stay zero or finite
     __syncthreads();
 
@@ -72,7 +79,7 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     const int qi = i0 + ii, q_lo = chunk > 0 ? qi - qi % chunk : qi - window + 1;                 // the row's keys: q_lo .. qi
     ar_bf16x8 qf[KU / 2];
     {
-        const bf16_t *qp = (const bf16_t *)a.q + ((int64_t)(row0 + ii) * H + hh) * D + 8 * hi;
+        const bf16_t *qp = (const bf16_t *)a.q + (int64_t)(row0 + ii) * a.q_ld + hh * D + 8 * hi;
 #pragma unroll
         for (int x = 0; x < KU / 2; ++x) {
             uint2 w[2] = {make_uint2(0, 0), make_uint2(0, 0)};
@@ -100,7 +107,8 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     const bool wave_full = 32 * wave + 31 < TQ * HF && (32 * wave + 31) / HF < cnt && h0 + HF <= h_end;     // all 32 rows are rows of the tile
 
     // 16-byte loads where rows and columns start at 16-byte borders, else two of 8
-    const bool wide = ((uintptr_t)a.k_cache & 15) == 0 && ((uintptr_t)a.v_cache & 15) == 0 && a.k_ld % 8 == 0 && a.v_ld % 8 == 0;
+    const bool wide = ((uintptr_t)a.k_cache & 15) == 0 && ((uintptr_t)a.v_cache & 15) == 0 && a.k_ld % 8 == 0 && a.v_ld % 8 == 0 &&
+                      (!BUILT || (((uintptr_t)a.k_tail & 15) == 0 && a.k_tail_ld % 8 == 0));
     uint4 kreg[KPF], vreg[VPF];
     auto load16 = [&](const bf16_t *p) -> uint4 {
         if (wide) return *(const uint4 *)p;
@@ -111,7 +119,9 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     int tok_next = 0;
     auto look_up = [&](int u0) {
         if (tid >= KT || u0 + tid >= n_keys) return;
-        const int j = lo + u0 + tid, pg = page_shift >= 0 ? j >> page_shift : j / a.page_size;
+        const int j = lo + u0 + tid;
+        if (BUILT) { tok_next = key_base + j; return; }
+        const int pg = page_shift >= 0 ? j >> page_shift : j / a.page_size;
         tok_next = bt[pg] * a.page_size + (j - pg * a.page_size);
     };
     auto tokens_out = [&](int sel) { if (tid < KT) tokS[sel * KT + tid] = tok_next; };
@@ -120,7 +130,8 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
 #pragma unroll
         for (int it = 0; it < KPF; ++it) {
             const int e = tid + it * AR_THREADS, jj = e / KU, u = e % KU;
-            if (jj < nk && 8 * u < D) kreg[it] = load16(kc + (int64_t)tok[jj] * a.k_ld + 8 * u);
+            if (jj < nk && 8 * u < D)
+                kreg[it] = load16(BUILT && 8 * u >= Dh ? kt + (int64_t)tok[jj] * a.k_tail_ld + (8 * u - Dh) : kc + (int64_t)tok[jj] * a.k_ld + 8 * u);
         }
         if (V_IN_K) return;
 #pragma unroll
@@ -287,9 +298,9 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     }
 }
 
-template <int KU, int VU, bool V_IN_K> static int ar_launch(const jl_attn_args &a, int hf, int hb, hipStream_t st) {
+template <int KU, int VU, int SRC> static int ar_launch(const jl_attn_args &a, int hf, int hb, hipStream_t st) {
     constexpr size_t lds = ar_lds_bytes(KU, VU);
-    auto kern = attn_rows_kernel<KU, VU, V_IN_K>;
+    auto kern = attn_rows_kernel<KU, VU, SRC>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_sweep: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
@@ -298,10 +309,12 @@ template <int KU, int VU, bool V_IN_K> static int ar_launch(const jl_attn_args &
     return jl_check_launch("attn_rows_kernel");
 }
 template <int KU, int VU> static int ar_launch_v(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st) {
-    return v_in_k ? ar_launch<KU, VU, true>(a, hf, hb, st) : ar_launch<KU, VU, false>(a, hf, hb, st);
+    return v_in_k ? ar_launch<KU, VU, AR_V_IN_K>(a, hf, hb, st) : ar_launch<KU, VU, AR_PAGED>(a, hf, hb, st);
 }
 
-int jl_attn_rows_launch(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st) {
+int jl_attn_rows_launch(const jl_attn_args &args, int hf, int hb, bool v_in_k, hipStream_t st) {
+    jl_attn_args a = args;
+    a.q_ld = (int64_t)a.H * a.D;
     if (a.n_tiles > 65535) return jl_fail(JL_E_INVALID, "jl_attn_sweep: at most 65535 tiles");
     const int ku = 8 * ((a.D + 63) / 64), vu = a.Dv <= 64 ? 8 : 16;      // 16-byte units of a row in LDS
 #define AR_CASE(K, V) if (ku == K && vu == V) return ar_launch_v<K, V>(a, hf, hb, v_in_k, st)
@@ -311,4 +324,31 @@ int jl_attn_rows_launch(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipS
     AR_CASE(32, 8); AR_CASE(32, 16);
 #undef AR_CASE
     return jl_fail(JL_E_INVALID, "jl_attn_sweep: 128-row tiles take key widths up to 256, value widths up to 128");
+}
+
+extern "C" int jl_attn_expanded_tile_rows(void) { return AR_ROWS; }
+
+extern "C" int jl_attn_expanded(const jl_attn_args *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_attn_expanded: null arguments");
+    const jl_attn_args &a = *ap;
+    if (a.n_tiles <= 0) return JL_OK;
+    if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.tiles || !a.key_base || (a.k_tail_cols > 0 && !a.k_tail)) return jl_fail(JL_E_INVALID, "jl_attn_expanded: null pointer");
+    const int64_t own = a.D - a.k_tail_cols;
+    if (a.dtype != JL_BF16 || a.H <= 0 || a.G != a.H || (a.Gv > 0 && a.Gv != a.H) || a.D <= 0 || a.D % 8 || a.D > 256 || a.k_tail_cols < 0 || a.k_tail_cols % 8 || own < 0 ||
+        a.Dv < 32 || a.Dv % 32 || a.Dv > 128 || a.TQ != AR_ROWS || a.n_tiles > 65535)
+        return jl_fail(JL_E_INVALID, "jl_attn_expanded: bfloat16, a key and a value head per query head, key widths in multiples of 8 up to 256, value widths in multiples of 32 up to 128");
+    if (a.k_ld < a.H * own || a.v_ld < (int64_t)a.H * a.Dv || a.q_ld < (int64_t)a.H * a.D || a.out_ld < (int64_t)a.H * a.Dv || (a.k_tail_cols > 0 && a.k_tail_ld < a.k_tail_cols) ||
+        a.k_ld % 4 || a.v_ld % 4 || a.q_ld % 4 || a.out_ld % 4 || a.k_tail_ld % 4)
+        return jl_fail(JL_E_INVALID, "jl_attn_expanded: row strides hold a row and are multiples of four");
+    if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_expanded: unknown out_dtype");
+    if (a.chunk > 0 && a.window > 0) return jl_fail(JL_E_INVALID, "jl_attn_expanded: chunks exclude a window");
+    hipStream_t st = (hipStream_t)stream;
+    const int ku = 8 * ((a.D + 63) / 64), vu = a.Dv <= 64 ? 8 : 16;
+#define AR_CASE(K, V) if (ku == K && vu == V) return ar_launch<K, V, AR_BUILT>(a, 1, 1, st)
+    AR_CASE(8, 8); AR_CASE(8, 16);
+    AR_CASE(16, 8); AR_CASE(16, 16);
+    AR_CASE(24, 8); AR_CASE(24, 16);
+    AR_CASE(32, 8); AR_CASE(32, 16);
+#undef AR_CASE
+    return jl_fail(JL_E_INVALID, "jl_attn_expanded: sizes");
 }

@@ -100,6 +100,37 @@ extern "C" int jl_latent_q_pack(const void *qa, const void *q, int64_t q_ld, int
     return jl_check_launch("latent_q_pack_kernel");
 }
 
+// q[n, h, D + d] for d < rot_dims <- rotated, in place: a thread owns a pair.  A workgroup of 256 walks 256 / half heads of consecutive rows at a time; what
+// it moves is the rotary columns only (8 192 rows x 16 heads x 64 of 192 columns: 9 us).
+template <typename T>
+__global__ __launch_bounds__(256) void rotate_heads_kernel(T *__restrict__ q, int64_t N, int64_t ld, int H, int D, int rd, int rot_dims, const int32_t *__restrict__ pos,
+                                                            const float *__restrict__ cos_t, const float *__restrict__ sin_t, int pairing) {
+    const int half = rot_dims >> 1, per_row = H * half;
+    for (int64_t n = blockIdx.x; n < N; n += gridDim.x) {
+        const float *cs = cos_t + (int64_t)pos[n] * half, *sn = sin_t + (int64_t)pos[n] * half;
+        T *row = q + n * ld + D;
+        for (int e = threadIdx.x; e < per_row; e += 256) {
+            const int h = e / half, i = e - h * half;
+            T *v = row + (int64_t)h * (D + rd);
+            const int x = pairing == JL_ROT_NEIGHBOURS ? 2 * i : i, y = pairing == JL_ROT_NEIGHBOURS ? 2 * i + 1 : i + half;
+            const float a = ld_f(v + x), b = ld_f(v + y);
+            st_f(v + x, a * cs[i] - b * sn[i]);
+            st_f(v + y, b * cs[i] + a * sn[i]);
+        }
+    }
+}
+
+extern "C" int jl_rotate_heads(void *q, int dtype, int64_t N, int64_t ld, int32_t H, int32_t D, int32_t rd, int32_t rot_dims, const int32_t *pos, const float *cos_t,
+                               const float *sin_t, int64_t table_len, int32_t pairing, void *stream) {
+    if (N <= 0 || rot_dims == 0) return JL_OK;
+    if (!q || !pos || !cos_t || !sin_t || table_len <= 0 || H <= 0 || D < 0 || rd <= 0 || ld < (int64_t)H * (D + rd)) return jl_fail(JL_E_INVALID, "jl_rotate_heads: null pointer or bad sizes");
+    if (rot_dims < 0 || rot_dims > rd || (rot_dims & 1)) return jl_fail(JL_E_INVALID, "jl_rotate_heads: rot_dims must be even and at most rd");
+    if (pairing != JL_ROT_HALVES && pairing != JL_ROT_NEIGHBOURS) return jl_fail(JL_E_INVALID, "jl_rotate_heads: unknown pairing %d", pairing);
+    JL_DISPATCH(dtype, rotate_heads_kernel<T><<<dim3((unsigned)(N < 65535 * 16 ? N : 65535 * 16)), 256, 0, (hipStream_t)stream>>>((T *)q, N, ld, H, D, rd, rot_dims, pos, cos_t,
+                                                                                                                                sin_t, pairing));
+    return jl_check_launch("rotate_heads_kernel");
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void heads_gate_kernel(const T *__restrict__ ov, const T *__restrict__ gate, int64_t gate_ld, int64_t N, int H, int Dv,
                                                           T *__restrict__ out) {

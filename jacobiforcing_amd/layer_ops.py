@@ -12,6 +12,7 @@ from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
+import torch.nn.functional as F
 
 from . import _native as N
 
@@ -74,6 +75,7 @@ class RaggedBatch:
     max_slot: int
     slots: List[int]
     _tiles: dict
+    _host_tables: Optional[np.ndarray] = None         # block_tables on the host (what key_rows reads)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
@@ -109,7 +111,7 @@ class RaggedBatch:
         return cls(B=B, N=int(row0[-1]), counts=list(map(int, counts)), starts=list(map(int, starts)),
                    seq=d_seq.view(B, 4), kv_slot=up[:kv.size], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos,
                    page_size=int(page_size), max_pos=max(int(s) + int(c) for s, c in zip(starts, counts)), max_page=int(bt.max()),
-                   max_slot=int(max(slots)), slots=list(map(int, slots)), _tiles={})
+                   max_slot=int(max(slots)), slots=list(map(int, slots)), _tiles={}, _host_tables=bt)
 
     def chunks(self, size: int):
         """A portion of at least two chunks is cut into chunks of ``size`` tokens that the recurrent layers run side by side.
@@ -146,15 +148,42 @@ class RaggedBatch:
             self._tiles[key] = (both[:len(rec)], both[len(rec):])
         return self._tiles[key]
 
-    def tiles(self, tq: int, longest_first: bool = False) -> torch.Tensor:
+    def key_rows(self, requests: Sequence[int], window: int):
+        """The pool tokens that ``requests`` read under ``window`` (0: all before them), request by request in order of position: (tokens [K] int64,
+        base [B] int32 with the place of request b's position j at base[b] + j)."""
+        key = ("keys", tuple(requests), window)
+        if key not in self._tiles:
+            tok, base, at = [], np.zeros(self.B, dtype=np.int32), 0
+            for b in requests:
+                end = self.starts[b] + self.counts[b]
+                pos = np.arange(max(0, self.starts[b] - window + 1) if window > 0 else 0, end, dtype=np.int64)
+                tok.append(self._host_tables[b][pos // self.page_size].astype(np.int64) * self.page_size + pos % self.page_size)
+                base[b] = at - int(pos[0])
+                at += pos.size
+            dev = self.seq.device
+            self._tiles[key] = (torch.from_numpy(np.concatenate(tok)).to(dev), torch.from_numpy(base).to(dev))
+        return self._tiles[key]
+
+    def part(self, requests: Sequence[int]):
+        """``requests`` as a batch of their own and the rows of this batch that are theirs ([n] int64)."""
+        key = ("part", tuple(requests))
+        if key not in self._tiles:
+            row0 = np.concatenate([[0], np.cumsum(self.counts)])
+            rows = np.concatenate([np.arange(row0[b], row0[b + 1], dtype=np.int64) for b in requests])
+            sub = RaggedBatch.build([self.counts[b] for b in requests], [self.starts[b] for b in requests], [self.slots[b] for b in requests],
+                                    [self._host_tables[b] for b in requests], self.page_size, self.seq.device)
+            self._tiles[key] = (sub, torch.from_numpy(rows).to(self.seq.device))
+        return self._tiles[key]
+
+    def tiles(self, tq: int, longest_first: bool = False, requests: Optional[Sequence[int]] = None) -> torch.Tensor:
         """[n_tiles, 4] int32 {b, first query position, count, first row}: each request's rows cut into runs of at most ``tq``; with
-        ``longest_first`` those with the most positions in front of them come first."""
-        key = ("longest first", tq) if longest_first else tq
+        ``longest_first`` those with the most positions in front of them come first; only those of ``requests`` when given."""
+        key = ("longest first", tq, None if requests is None else tuple(requests)) if longest_first or requests is not None else tq
         t = self._tiles.get(key)
         if t is None:
             rows, r0 = [], 0
             for b, (c, s) in enumerate(zip(self.counts, self.starts)):
-                for o in range(0, c, tq):
+                for o in range(0, c if requests is None or b in requests else 0, tq):
                     rows.append((b, s + o, min(tq, c - o), r0 + o))
                 r0 += c
             if longest_first:
@@ -748,6 +777,90 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
             ov = torch.bmm(o, wv) if ov is None else torch.baddbmm(ov, o, wv)
         parts.append(ov)
     return parts[0] if len(parts) == 1 else torch.cat(parts, 0)
+
+
+# What the two forms of latent attention run at (this card): attention over the latent on the 32-row and (narrow latents) the 128-row tiles, attention over
+# keys and values built per head, the product that builds them; plus what the built form's extra launches cost, alone and beside the other form's.
+LATENT_RATES = dict(narrow=330e12, wide=105e12, built=420e12, product=600e12, launches=20e-6, both=80e-6)
+LATENT_BUILT_BYTES = 2 << 30          # keys and values built at a time
+LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth building keys for fewer
+
+
+def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, window: int) -> List[int]:
+    """The requests of a step whose keys and values are better built per head.  Over the latent a visible pair costs 2 H (2 R + rd) operations, over
+    built keys 2 H (D + rd + Dv) — a third of it at R = 512, D = Dv = 128, rd = 64 — but every key is built first, 2 H R (D + Dv): worth it from some
+    hundred new tokens per request on, never for a decoded token."""
+    key = ("built", H, D, R, rd, Dv, window)
+    chosen = batch._tiles.get(key)
+    if chosen is None:
+        r = LATENT_RATES
+        over = r["narrow"] if R <= 128 and R + rd <= 256 else r["wide"]
+        pair, one = 2.0 * H * ((2 * R + rd) / over - (D + rd + Dv) / r["built"]), 2.0 * H * R * (D + Dv) / r["product"]      # seconds won per pair, spent per key
+        w, won, keys, chosen = window if window > 0 else 1 << 40, 0.0, 0, []
+        for b, c in enumerate(batch.counts):
+            if c < LATENT_BUILT_FROM:
+                continue
+            s = batch.starts[b]
+            full = min(c, max(0, s + c - w))              # queries that see a whole window; the others see s + 1, s + 2, .. keys
+            n = s + c - max(0, s - w + 1)
+            gain = pair * (full * w + (c - full) * (s + 0.5 * (1 + c - full))) - one * n
+            if gain > 0 and (keys + n) * 2 * H * (D + Dv) <= LATENT_BUILT_BYTES:
+                chosen.append(b)
+                won += gain
+                keys += n
+        if won <= (r["launches"] if len(chosen) == batch.B else r["both"]):
+            chosen = []
+        batch._tiles[key] = chosen
+    return chosen
+
+
+def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w_uk: torch.Tensor, w_uv: torch.Tensor, batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, rot_dims: int,
+                     cos, sin, pairing: int, scale: float, window: int, sink: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+                     gate_per_head: bool = False) -> torch.Tensor:
+    """Latent attention from the queries to the heads' outputs [N, H*Dv]: q [N, H*(D + rd)] not yet rotated (row stride free; its rotary columns are
+    OVERWRITTEN), pool [tokens, R + rd] with this step's rows in place, w_ukv [H*D + H*Dv, R] the key up-projections of all heads on the value up-projections,
+    w_uk [H, D, R] and w_uv [H, R, Dv] the same per head, the latter turned.  ``window`` 0: plain causal; ``sink`` float [H]; ``gate`` a [N, H*Dv] view, or [N, H] with
+    ``gate_per_head``: sigmoid gates on the outputs.
+    Decoded tokens and short portions bring their queries to the latent (``latent_q_pack``, ``latent_attend``); for long portions in bfloat16 keys and values
+    are built per head (``_latent_built_requests``) and attended on the 128-row tiles; a step may hold both."""
+    _dev(q)
+    n, dt = q.shape[0], q.dtype
+    _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] == H * (D + rd) and n == batch.N, "latent_attention: q [N, H*(D + rd)] of the batch")
+    built: List[int] = []
+    if dt == torch.bfloat16 and D % 8 == 0 and rd % 8 == 0 and D + rd <= 256 and Dv % 32 == 0 and Dv <= 128 and q.stride(0) % 4 == 0 and q.data_ptr() % 8 == 0:
+        built = _latent_built_requests(batch, H, D, R, rd, Dv, window)
+
+    def over_latent(q, batch, gate):
+        m = q.shape[0]
+        qa = torch.bmm(q.view(m, H, D + rd)[:, :, :D].transpose(0, 1), w_uk)      # [H, N, R]: query . (W_uk c) = (W_uk^T query) . c
+        qf = latent_q_pack(qa, q, H, D, R, rd, rot_dims, batch, cos, sin, pairing=pairing)
+        return heads_gate(latent_attend(qf, pool, w_uv, batch, H, R, rd, scale, window, sink=sink, gate=gate if gate_per_head else None), None if gate_per_head else gate)
+
+    if not built:
+        return over_latent(q, batch, gate)
+    _need(w_ukv.is_contiguous() and w_ukv.dtype == dt and tuple(w_ukv.shape) == (H * (D + Dv), R), "latent_attention: up-projections [H*D + H*Dv, R]")
+    _need(pool.dtype == dt and pool.is_contiguous() and pool.shape[-1] == R + rd and pool.shape[0] % batch.page_size == 0 and
+          batch.max_page < pool.shape[0] // batch.page_size, "latent_attention: pool [tokens, R + rd] that holds the batch's pages")
+    _check_gate_sink(gate, sink, gate_per_head, n, H, Dv, dt, "latent_attention")
+    out = torch.empty((n, H * Dv), dtype=dt, device=q.device)
+    if len(built) < batch.B:                              # the other requests' rows, before the rotation below reaches them
+        rest, rows = batch.part(sorted(set(range(batch.B)) - set(built)))
+        out.index_copy_(0, rows, over_latent(q.index_select(0, rows), rest, None if gate is None else gate.index_select(0, rows)))
+    keys, base = batch.key_rows(built, window)
+    lat = pool.index_select(0, keys)
+    kv = F.linear(lat[:, :R], w_ukv)
+    tl = _angle_tables(rot_dims, cos, sin, batch, "latent_attention")
+    st = _stream(q.device)
+    N.check_layers(N.layers().jl_rotate_heads(_ptr(q), _code(dt), n, q.stride(0), H, D, rd, rot_dims, _ptr(batch.pos), _ptr(cos), _ptr(sin), tl, int(pairing), st), "jl_rotate_heads")
+    tq = int(N.layers().jl_attn_expanded_tile_rows())
+    tiles = batch.tiles(tq, longest_first=True, requests=built)
+    a = N.AttnArgs(q=q.data_ptr(), k_cache=kv.data_ptr(), v_cache=kv.data_ptr() + 2 * H * D, out=out.data_ptr(), tiles=tiles.data_ptr(), n_tiles=tiles.shape[0], H=H, G=H, D=D + rd,
+                   Dv=Dv, window=int(window), TQ=tq, dtype=_code(dt), scale=float(scale), n_rows=n, k_ld=kv.shape[1], v_ld=kv.shape[1], Gv=H, out_dtype=N.JL_OUT_SAME,
+                   sink=sink.data_ptr() if sink is not None else None, gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0,
+                   gate_heads=int(gate_per_head), out_scale=1.0, out_ld=H * Dv, key_base=base.data_ptr(), k_tail=lat.data_ptr() + 2 * R if rd else None, k_tail_ld=R + rd,
+                   q_ld=q.stride(0), k_tail_cols=rd)
+    N.check_layers(N.layers().jl_attn_expanded(C.byref(a), st), "jl_attn_expanded")
+    return out
 
 
 def heads_gate(ov: torch.Tensor, gate: Optional[torch.Tensor]) -> torch.Tensor:

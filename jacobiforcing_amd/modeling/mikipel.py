@@ -98,8 +98,8 @@ def _delta_sizes(m: Dict[str, Any]):
 class MikipelWeights:
     """Tensors by their checkpoint names (``embed``, ``l<i>.norm1``, ``l<i>.shift``, ``l<i>.dwa``, ``l<i>.mix.*``, ``l<i>.mlp.*``,
     ``final.norm``), regrouped per layer for the forward: a mixer's input projections stacked into one matrix (ending with zero rows up
-    to a multiple of eight, so that the product's rows start at 16-byte borders), the latent up-projections per head ([H, D, R] for keys,
-    [H, R, Dv] for values), the three convolutions' taps stacked like their channels, every expert's gate rows on its up rows
+    to a multiple of eight, so that the product's rows start at 16-byte borders), the latent up-projections (keys of all heads on values, and the
+    values' once more as [H, R, Dv]), the three convolutions' taps stacked like their channels, every expert's gate rows on its up rows
     ([E, 2*ff, W]); norm weights, shift, depth weights, decay constants and the router in float."""
 
     def __init__(self, cfg: MikipelConfig, tensors: Dict[str, torch.Tensor], device, dtype=torch.bfloat16):
@@ -131,7 +131,8 @@ class MikipelWeights:
             elif L["type"] == "latent_attention":
                 H, D, rd, Dv, R = (int(m[k]) for k in ("heads", "dim", "rot_dim", "vdim", "kv_rank"))
                 w.update(w_in=stack(i, [p + "mix.q", p + "mix.dkv"], H * (D + rd) + R + rd), kv_col=H * (D + rd), dkv_norm=act(p + "mix.dkv.norm"),
-                         w_uk=act(p + "mix.uk").view(H, D, R).contiguous(), w_uv=act(p + "mix.uv").view(H, Dv, R).transpose(1, 2).contiguous())
+                         w_ukv=torch.cat([act(p + "mix.uk"), act(p + "mix.uv")], 0), w_uv=act(p + "mix.uv").view(H, Dv, R).transpose(1, 2).contiguous())
+                w["w_uk"] = w["w_ukv"][:H * D].view(H, D, R)
                 if w["dkv_norm"].numel() != R:
                     raise ValueError(f"layer {i}: dkv.norm has {w['dkv_norm'].numel()} entries, kv_rank is {R}")
                 out_in = H * Dv
@@ -273,13 +274,10 @@ class MikipelModel:
         m, w, eps = self.cfg.layers[li]["mixer"], self.w.layers[li], self.cfg.norm_eps
         H, D, rd, Dv, R = (int(m[k]) for k in ("heads", "dim", "rot_dim", "vdim", "kv_rank"))
         dims, cos, sin = self._tables(m)
-        n, pool, scale = h.shape[0], cache.k[li], float(m["scale"])
+        pool, scale = cache.k[li], float(m["scale"])
         proj = F.linear(h, w["w_in"])
         LO.latent_prep(proj, 0, 0, w["kv_col"], R, rd, dims, None, w["dkv_norm"], eps, batch, cos, sin, pool, pairing=LO.ROT_NEIGHBOURS)
-        q = proj[:, :H * (D + rd)]
-        qa = torch.bmm(q.view(n, H, D + rd)[:, :, :D].transpose(0, 1), w["w_uk"])                  # [H, N, R]: query . (W_uk c) = (W_uk^T query) . c
-        qf = LO.latent_q_pack(qa, q, H, D, R, rd, dims, batch, cos, sin, pairing=LO.ROT_NEIGHBOURS)
-        return LO.heads_gate(LO.latent_attend(qf, pool, w["w_uv"], batch, H, R, rd, scale, 0), None)
+        return LO.latent_attention(proj[:, :H * (D + rd)], pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, dims, cos, sin, LO.ROT_NEIGHBOURS, scale, 0)
 
     def _delta(self, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]

@@ -104,7 +104,7 @@ def _experts(f: Dict[str, Any]):
 class VoboraxWeights:
     """Tensors by their checkpoint names (``embed``, ``l<i>.norm1``, ``l<i>.mix.*``, ``l<i>.mlp.*``, ``final.norm``, ``head``), regrouped per
     layer for the forward: a mixer's input projections (query latent, key/value latent with the rotary key, head gate) stacked into one matrix
-    that ends with zero rows up to a multiple of eight, the latent up-projections per head ([H, D, R] for keys, [H, R, Dv] for values), every
+    that ends with zero rows up to a multiple of eight, the latent up-projections (keys of all heads on values, and the values' once more as [H, R, Dv]), every
     expert's gate rows on its up rows ([E, 2*ff, W]), the shared expert's likewise; stream norms, sinks, router and correction in float."""
 
     def __init__(self, cfg: VoboraxConfig, tensors: Dict[str, torch.Tensor], device, dtype=torch.bfloat16):
@@ -135,8 +135,9 @@ class VoboraxWeights:
             rows.append(torch.zeros(((-n) % 8, W), dtype=dtype, device=dev))
             w = dict(norm1=f32(p + "norm1", W), w_in=torch.cat(rows, 0), kv_col=Rq, g_col=Rq + (R + rd if own else 0), dq_norm=act(p + "mix.dq.norm", Rq),
                      dkv_norm=act(p + "mix.dkv.norm", R) if own else None, w_uq=act(p + "mix.uq", H * (D + rd), Rq),
-                     w_uk=act(p + "mix.uk", H * D, R).view(H, D, R), w_uv=act(p + "mix.uv", H * Dv, R).view(H, Dv, R).transpose(1, 2).contiguous(),
+                     w_ukv=torch.cat([act(p + "mix.uk", H * D, R), act(p + "mix.uv", H * Dv, R)], 0), w_uv=act(p + "mix.uv", H * Dv, R).view(H, Dv, R).transpose(1, 2).contiguous(),
                      w_o=act(p + "mix.o", W, H * Dv), sink=f32(p + "mix.sink", H) if L["type"] == CAUSAL else None)
+            w["w_uk"] = w["w_ukv"][:H * D].view(H, D, R)
             f = L.get("mlp")
             if f is not None:
                 w["norm2"] = f32(p + "norm2", W)
@@ -238,17 +239,16 @@ class VoboraxModel:
         windowed, src = L["type"] == WINDOWED, self.cfg.pool_layer(li)
         key = _rot_key(m) if windowed else (0, 0.0)
         cos, sin = self._angles[key] if key[0] else (None, None)
-        n, pool = h.shape[0], cache.k[src]
+        pool = cache.k[src]
         proj = F.linear(h, w["w_in"])
         cq = LO.latent_prep(proj, 0, Rq, w["kv_col"], R, rd, key[0], w["dq_norm"], w["dkv_norm"], eps, batch, cos, sin, pool if src == li else None,
                             pairing=LO.ROT_NEIGHBOURS)
         q = F.linear(cq, w["w_uq"])
-        qa = torch.bmm(q.view(n, H, D + rd)[:, :, :D].transpose(0, 1), w["w_uk"])                  # [H, N, R]: query . (W_uk c) = (W_uk^T query) . c
-        qf = LO.latent_q_pack(qa, q, H, D, R, rd, key[0], batch, cos, sin, pairing=LO.ROT_NEIGHBOURS)
         gate = proj[:, w["g_col"]:w["g_col"] + H] if windowed else None
         window = int((m.get("mask") or {}).get("size", 0)) if windowed else 0
-        ov = LO.latent_attend(qf, pool, w["w_uv"], batch, H, R, rd, float(m["scale"]), window, sink=w["sink"], gate=gate)
-        return F.linear(LO.heads_gate(ov, None), w["w_o"])
+        o = LO.latent_attention(q, pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, key[0], cos, sin, LO.ROT_NEIGHBOURS, float(m["scale"]), window, sink=w["sink"],
+                                gate=gate, gate_per_head=windowed)
+        return F.linear(o, w["w_o"])
 
     # ---- feed-forward: the addends of its output, and the choices among which there are identity experts ----------------------------------
     def _feed_forward(self, li: int, h: torch.Tensor, x: torch.Tensor):

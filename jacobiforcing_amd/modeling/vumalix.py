@@ -125,7 +125,8 @@ class VumalixWeights:
                 H, D, rd, Dv, R, Rq = (int(m[k]) for k in ("heads", "dim", "rot_dim", "vdim", "kv_rank", "q_rank"))
                 w.update(w_in=torch.cat([act(p + "mix.dq"), act(p + "mix.dkv"), act(p + "mix.g")], 0), cols=(0, Rq, Rq + R + rd),
                          dq_norm=act(p + "mix.dq.norm"), dkv_norm=act(p + "mix.dkv.norm"), w_uq=act(p + "mix.uq"),
-                         w_uk=act(p + "mix.uk").view(H, D, R).contiguous(), w_uv=act(p + "mix.uv").view(H, Dv, R).transpose(1, 2).contiguous())
+                         w_ukv=torch.cat([act(p + "mix.uk"), act(p + "mix.uv")], 0), w_uv=act(p + "mix.uv").view(H, Dv, R).transpose(1, 2).contiguous())
+                w["w_uk"] = w["w_ukv"][:H * D].view(H, D, R)
                 want = Rq + R + rd + H * Dv
                 if tuple(w["w_uq"].shape) != (H * (D + rd), Rq):
                     raise ValueError(f"layer {i}: uq is {tuple(w['w_uq'].shape)}, the config's sizes give {(H * (D + rd), Rq)}")
@@ -245,15 +246,12 @@ class VumalixModel:
         rot = m.get("rot") or {}
         dims = int(rot.get("dims", 0))
         cos, sin = self._angles[(dims, float(rot.get("base", 10000.0)))] if dims else (None, None)
-        n = h.shape[0]
         pool = cache.k[li]
         proj = F.linear(h, w["w_in"])
         cq = LO.latent_prep(proj, w["cols"][0], Rq, w["cols"][1], R, rd, dims, w["dq_norm"], w["dkv_norm"], eps, batch, cos, sin, pool)
         q = F.linear(cq, w["w_uq"])
-        qa = torch.bmm(q.view(n, H, D + rd)[:, :, :D].transpose(0, 1), w["w_uk"])                    # [H, N, R]: query . (W_uk c) = (W_uk^T query) . c
-        qf = LO.latent_q_pack(qa, q, H, D, R, rd, dims, batch, cos, sin)
-        ov = LO.latent_attend(qf, pool, w["w_uv"], batch, H, R, rd, float(m["scale"]), int((m.get("mask") or {}).get("size", 0)))      # [H, N, Dv]
-        return LO.heads_gate(ov, proj[:, w["cols"][2]:w["cols"][2] + H * Dv])
+        return LO.latent_attention(q, pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, dims, cos, sin, LO.ROT_HALVES, float(m["scale"]),
+                                   int((m.get("mask") or {}).get("size", 0)), gate=proj[:, w["cols"][2]:w["cols"][2] + H * Dv])
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------
     @torch.inference_mode()

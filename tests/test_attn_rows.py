@@ -62,10 +62,58 @@ def test_wide_tiles(H, G, Gv, D, Dv, window, chunk, cap, page, pad):
     batch = LO.RaggedBatch.build(counts, starts, [0, 1, 2, 3], pages, page, dev)
     gate = rnd(sum(counts), H)
     got = LO.attn_sweep(q, k, v, batch, H, G, D, Dv, D ** -0.5, window, value_heads=Gv, float_out=True, sink=sink, gate=gate, gate_per_head=True, chunk=chunk, softcap=cap)
-    assert ("longest first", 128 // min(H // G, 32)) in batch._tiles, "the 128-row form did not run"
+    assert ("longest first", 128 // min(H // G, 32), None) in batch._tiles, "the 128-row form did not run"
     want = reference(q, k, v, starts, counts, pages, page, H, G, Gv or 1, D, Dv, D ** -0.5, window, chunk, cap, sink)
     want = (want.view(-1, H, Dv) * torch.sigmoid(gate.double()).unsqueeze(-1)).view_as(want)
     assert torch.isfinite(got).all()
     # weights are rounded to bfloat16 (2 ** -9 relative, independently): a sum of them is off by less than that of its largest terms
     err = (got.double() - want).abs()
     assert err.max() < 2.0 ** -7 * want.abs().max() and err.norm() < 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("H,D,R,rd,Dv,rot,pairing,window,gate,built", [
+    (5, 64, 128, 32, 64, 32, "ROT_NEIGHBOURS", 0, None, (0, 1, 2, 3)), (16, 128, 512, 64, 128, 64, "ROT_HALVES", 100, "full", (0, 1, 2, 3)), (3, 8, 64, 8, 32, 4, "ROT_NEIGHBOURS", 1, "head", (1, 3)),
+    (2, 248, 32, 8, 96, 8, "ROT_HALVES", 0, "full", (0,)), (4, 64, 96, 0, 128, 0, "ROT_HALVES", 37, "head", (0, 1, 3)), (33, 120, 40, 72, 64, 72, "ROT_NEIGHBOURS", 300, None, (1, 2)),
+])
+def test_latent_attention_with_built_keys(monkeypatch, H, D, R, rd, Dv, rot, pairing, window, gate, built):
+    """Some or all requests of a step on keys and values built per head, the others over the latent; the last request brings one token."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt, page = "cuda", torch.bfloat16, 32
+    monkeypatch.setattr(LO, "_latent_built_requests", lambda *a: list(built))
+    starts, counts = [0, 45, 3, 200], [129, 300, 128, 1]
+    g = torch.Generator(device=dev).manual_seed(H + R)
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g, device=dev) * std).to(dt)
+    need = [-(-(s + n) // page) for s, n in zip(starts, counts)]
+    ids = torch.randperm(sum(need) + 2, generator=torch.Generator().manual_seed(H)).tolist()
+    pages = [[ids.pop() for _ in range(n)] for n in need]
+    pool = torch.full(((sum(need) + 2) * page, R + rd), float("nan"), dtype=dt, device=dev)
+    for s, n, tab in zip(starts, counts, pages):
+        pool[torch.tensor([tab[j // page] * page + j % page for j in range(s + n)], device=dev)] = rnd(s + n, R + rd)
+    n = sum(counts)
+    wide = rnd(n, H * (D + rd) + 8)                       # the queries are a column range of wider rows
+    w_uk, w_uv, sink = rnd(H * D, R, std=R ** -0.5), rnd(H * Dv, R, std=R ** -0.5), torch.randn(H, generator=g, device=dev)
+    gates = None if gate is None else rnd(n, H if gate == "head" else H * Dv)
+    batch = LO.RaggedBatch.build(counts, starts, [0, 1, 2, 3], pages, page, dev)
+    a = torch.arange(512, dtype=torch.float32, device=dev).view(-1, 1) * torch.rand(max(rot, 2) // 2, generator=g, device=dev).view(1, -1)
+    cos, sin = (a.cos().contiguous(), a.sin().contiguous()) if rot else (None, None)
+    q64 = wide[:, :H * (D + rd)].double().view(n, H, D + rd)
+    tail = q64[..., D:D + rot]
+    if rot:
+        c, s = cos.double()[batch.pos.long()].unsqueeze(1), sin.double()[batch.pos.long()].unsqueeze(1)
+        near = pairing == "ROT_NEIGHBOURS"
+        u, v = (tail[..., 0::2], tail[..., 1::2]) if near else (tail[..., :rot // 2], tail[..., rot // 2:])
+        x, y = u * c - v * s, v * c + u * s
+        tail = torch.stack([x, y], -1).flatten(-2) if near else torch.cat([x, y], -1)
+    q64 = torch.cat([q64[..., :D], tail, q64[..., D + rot:]], -1)
+    lat = pool.double()
+    k64 = torch.cat([(lat[:, :R] @ w_uk.double().T).view(-1, H, D), lat[:, R:].unsqueeze(1).expand(-1, H, rd)], -1).flatten(1)
+    scale = (D + rd) ** -0.5
+    want = reference(q64.flatten(1), k64, lat[:, :R] @ w_uv.double().T, starts, counts, pages, page, H, H, H, D + rd, Dv, scale, window, 0, 0.0, sink)
+    if gate is not None:
+        gg = torch.sigmoid(gates.double())
+        want = want * (gg if gate == "full" else gg.repeat_interleave(Dv, 1))
+    got = LO.latent_attention(wide[:, :H * (D + rd)], pool, torch.cat([w_uk, w_uv]), w_uk.view(H, D, R), w_uv.view(H, Dv, R).transpose(1, 2).contiguous(), batch, H, D, R, rd, Dv, rot, cos, sin,
+                              getattr(LO, pairing), scale, window, sink=sink, gate=gates, gate_per_head=gate == "head")
+    # queries, keys, values, weights and the result are rounded to bfloat16 once each (2 ** -9 relative); a score of size 3 moves its weight by 1.2 %
+    err = (got.double() - want).abs()
+    assert torch.isfinite(got).all() and err.norm() < 2.0 ** -6 * want.norm() and err.max() < 2.0 ** -4 * want.abs().max()
