@@ -779,9 +779,11 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
     return parts[0] if len(parts) == 1 else torch.cat(parts, 0)
 
 
-# What the two forms of latent attention run at (this card): attention over the latent on the 32-row and (narrow latents) the 128-row tiles, attention over
-# keys and values built per head, the product that builds them; plus what the built form's extra launches cost, alone and beside the other form's.
-LATENT_RATES = dict(narrow=330e12, wide=105e12, built=420e12, product=600e12, launches=20e-6, both=80e-6)
+# What the two forms of latent attention run at (this card): attention over the latent on the 32-row and (narrow latents, many rows) the 128-row tiles,
+# attention over keys and values built per head, the product that builds them.  ``key`` is the time the built form takes per key of its longest tile when the
+# chip is not full (a tile walks its keys in order; the 32-row kernel shares few tiles' keys out).  A step wholly on built keys has fewer launches (bmm, packing, bmm
+# and head order go: 95 -> 55 us of host time for small steps), a step that mixes the forms has more.
+LATENT_RATES = dict(narrow=330e12, wide=105e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
 LATENT_BUILT_BYTES = 2 << 30          # keys and values built at a time
 LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth building keys for fewer
 
@@ -789,26 +791,27 @@ LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth build
 def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, window: int) -> List[int]:
     """The requests of a step whose keys and values are better built per head.  Over the latent a visible pair costs 2 H (2 R + rd) operations, over
     built keys 2 H (D + rd + Dv) — a third of it at R = 512, D = Dv = 128, rd = 64 — but every key is built first, 2 H R (D + Dv): worth it from some
-    hundred new tokens per request on, never for a decoded token."""
+    hundred new tokens per request on, never for a decoded token.  Measured, us over the latent / built: 4 x 1024 tokens at 16 heads x 128, R 512: 1044 / 110,
+    one request of 128 behind 4000: 303 / 288, of 32: 132 / 259; 8 heads x 64, R 128, 4 x 256 behind 1500: 132 / 92, 1 x 256 behind 4000: 116 / 163."""
     key = ("built", H, D, R, rd, Dv, window)
     chosen = batch._tiles.get(key)
     if chosen is None:
         r = LATENT_RATES
-        over = r["narrow"] if R <= 128 and R + rd <= 256 else r["wide"]
-        pair, one = 2.0 * H * ((2 * R + rd) / over - (D + rd + Dv) / r["built"]), 2.0 * H * R * (D + Dv) / r["product"]      # seconds won per pair, spent per key
-        w, won, keys, chosen = window if window > 0 else 1 << 40, 0.0, 0, []
+        over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["wide"])
+        pair, one = 2.0 * H * (D + rd + Dv) / r["built"], 2.0 * H * R * (D + Dv) / r["product"]
+        step = r["key64"] if D + rd <= 128 else r["key32"]
+        w, won, attend, chain, keys, chosen = window if window > 0 else 1 << 40, 0.0, 0.0, 0.0, 0, []
         for b, c in enumerate(batch.counts):
             if c < LATENT_BUILT_FROM:
                 continue
             s = batch.starts[b]
             full = min(c, max(0, s + c - w))              # queries that see a whole window; the others see s + 1, s + 2, .. keys
-            n = s + c - max(0, s - w + 1)
-            gain = pair * (full * w + (c - full) * (s + 0.5 * (1 + c - full))) - one * n
-            if gain > 0 and (keys + n) * 2 * H * (D + Dv) <= LATENT_BUILT_BYTES:
+            n, pairs = s + c - max(0, s - w + 1), full * w + (c - full) * (s + 0.5 * (1 + c - full))
+            if (keys + n) * 2 * H * (D + Dv) <= LATENT_BUILT_BYTES:
                 chosen.append(b)
-                won += gain
-                keys += n
-        if won <= (r["launches"] if len(chosen) == batch.B else r["both"]):
+                won += pairs * over - n * one
+                attend, chain, keys = attend + pairs * pair, max(chain, step * min(n, w + 127)), keys + n
+        if won - max(attend, chain) <= (r["launches"] if len(chosen) == batch.B else r["both"]):
             chosen = []
         batch._tiles[key] = chosen
     return chosen
