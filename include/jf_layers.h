@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 127
+#define JL_VERSION 128
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -343,13 +343,14 @@ JL_API int jl_linear_scan_chunked_ok(int dtype, int32_t D, int32_t Dv);
 JL_API int jl_moe_route(const float *logits, const float *correction, int64_t N, int32_t E, int32_t top, float scale, int32_t *ids,
                         float *weights, int32_t kind, float renorm_eps, void *stream);
 
-/* Rows (token, choice) grouped by expert; a choice outside 0 .. E-1 (an expert without weights) is left out.  perm [N*top]: sorted row -> flat index n*top + s; offsets [E+1]; tile_expert /
+/* Rows (token, choice) grouped by expert; a choice outside 0 .. E-1 (an expert without weights) is left out.  perm [N*top]: sorted row -> flat index n*top + s; offsets [E+2] (the last: tiles in use); tile_expert /
  * tile_row0 [max_tiles] (max_tiles >= N*top/tile_rows + E): row tiles of at most tile_rows rows of one expert, unused entries -1. */
 JL_API int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, int32_t tile_rows, int32_t *perm, int32_t *offsets,
                         int32_t *tile_expert, int32_t *tile_row0, int32_t max_tiles, void *stream);
-JL_API int jl_moe_tile_rows(void);
+/* tile_rows for a step of `rows` (token, choice) rows over E experts of width ff behind a stream of width W: 32, 64 or 128 */
+JL_API int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff);
 
-/* Grouped product over the sorted rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].
+/* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].
  *   mode 0 (up):   in(r) = perm[r] / top;  out[r, :] = relu(C)^2, stored in `dtype` ([N*top, n_out], sorted order)
  *   mode 1 (down): in(r) = r;              out[perm[r], :] = C * weights[perm[r]], stored as float ([N*top, n_out])
  *   mode JL_MOE_UP_PLAIN: as mode 0 without the activation (out[r, :] = C): a gated unit stacks its gate and linear branch in W and
@@ -357,13 +358,13 @@ JL_API int jl_moe_tile_rows(void);
 #define JL_MOE_UP_PLAIN 2
 JL_API int jl_moe_gemm(const void *X, const void *Wt, int dtype, int32_t mode, int32_t K, int32_t n_out, int32_t top,
                        const int32_t *perm, const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0,
-                       int32_t max_tiles, const float *weights, void *out, void *stream);
+                       int32_t max_tiles, int32_t E, int32_t tile_rows, const float *weights, void *out, void *stream);
 
 /* The up product of gated experts with the unit applied in its epilogue: W [E, 2*ff, K] stacks every expert's gate rows on its
  * linear rows; out[r, c] = unit(X[in(r)] . W[e(r), c], X[in(r)] . W[e(r), ff + c]) with in(r) = perm[r] / top, stored in `dtype`
  * ([N*top, ff], sorted order); kind / limit / alpha / shift as for jl_gated_act. */
 JL_API int jl_moe_gemm_gated(const void *X, const void *Wt, int dtype, int32_t K, int32_t ff, int32_t top, const int32_t *perm,
-                             const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t kind,
+                             const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t E, int32_t tile_rows, int32_t kind,
                              float limit, float alpha, float shift, void *out, void *stream);
 
 #ifdef __cplusplus

@@ -3,8 +3,10 @@
 // the grouped products: up with relu^2, plain, or with the gated unit in its epilogue, down with the routing weights.
 #include "jl_common.h"
 #include <stdlib.h>
+#include <type_traits>
 
 constexpr int MOE_MAX_E = 4096;   // experts (router outputs) at most
+struct MoeAct { int kind; float limit, alpha, shift; };       // the gated unit of JL_MOE_UP_GATED (jl_gated_act's kinds)
 
 // ---- router: one wavefront per token, NJ router outputs per lane (lane + 64 j) -------------------------------------------------------
 // Every lane keeps its outputs' comparison values and scores in registers; `top` rounds find the largest comparison value (ties: the lowest
@@ -87,46 +89,103 @@ extern "C" int jl_moe_route(const float *logits, const float *correction, int64_
 }
 
 // ---- grouping: one workgroup counts, scans and places (a step holds at most a few 10^5 rows) ----------------------------------------
-constexpr int MOE_TM = 64;        // rows of a tile
-constexpr int MOE_TN = 64;        // output columns of a tile
+constexpr int MOE_TM = 64;        // rows and output columns of a tile of the product for any size
+constexpr int MOE_TN = 64;
 constexpr int MOE_TK = 32;        // depth of one LDS stage
 
+// Its time is the latency of the trips to memory and of the counters, so a thread has MG_IN_FLIGHT ids on the way at once, and up to 16 wavefronts count in
+// tables of their own (8 192 rows x 4 choices over 32 experts: 53 us with one id at a time on shared counters, 15 us so).
+constexpr int MG_IN_FLIGHT = 16, MG_COUNTERS = 8192;
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *__restrict__ ids, int64_t rows, int E, int tile_rows,
                                                           int32_t *__restrict__ perm, int32_t *__restrict__ offsets,
                                                           int32_t *__restrict__ tile_expert, int32_t *__restrict__ tile_row0, int max_tiles) {
-    __shared__ int cnt[MOE_MAX_E];
-    __shared__ int base[MOE_MAX_E + 1];
-    for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
+    __shared__ int cnt[MG_COUNTERS];                                  // [tables][E]: counts, then the next free place of a table's rows
+    __shared__ int first_tile[MOE_MAX_E + 1];
+    __shared__ int wave_sum[2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tables = MG_COUNTERS / E < 16 ? MG_COUNTERS / E : 16;
+    int *mine = cnt + (wave % tables) * E;
+    for (int e = tid; e < tables * E; e += 1024) cnt[e] = 0;
     __syncthreads();
-    for (int64_t r = threadIdx.x; r < rows; r += 1024) {
-        const int e = ids[r];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);                   // an expert without weights has no rows
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int o = 0, t = 0;
-        for (int e = 0; e < E; ++e) {
-            base[e] = o;
-            offsets[e] = o;
-            for (int r = 0; r < cnt[e]; r += tile_rows)
-                if (t < max_tiles) { tile_expert[t] = e; tile_row0[t] = o + r; ++t; }
-            o += cnt[e];
+    auto each = [&](auto &&f) {
+        for (int64_t r0 = 0; r0 < rows; r0 += 1024 * MG_IN_FLIGHT) {
+            int e[MG_IN_FLIGHT];
+#pragma unroll
+            for (int i = 0; i < MG_IN_FLIGHT; ++i) {
+                const int64_t r = r0 + i * 1024 + tid;
+                e[i] = r < rows ? ids[r] : -1;
+            }
+#pragma unroll
+            for (int i = 0; i < MG_IN_FLIGHT; ++i)
+                if (e[i] >= 0 && e[i] < E) f((int32_t)(r0 + i * 1024 + tid), e[i]);      // an expert without weights has no rows
         }
-        offsets[E] = o;
-        for (; t < max_tiles; ++t) { tile_expert[t] = -1; tile_row0[t] = 0; }
+    };
+    each([&](int32_t, int e) { atomicAdd(&mine[e], 1); });
+    __syncthreads();
+    // a thread owns MOE_MAX_E / 1024 neighbouring experts: their rows and tiles, summed over the threads in front of it
+    constexpr int PER = MOE_MAX_E / 1024;
+    int n_rows[PER], sum_r = 0, sum_t = 0;
+#pragma unroll
+    for (int x = 0; x < PER; ++x) {
+        const int e = tid * PER + x;
+        n_rows[x] = 0;
+        if (e < E)
+            for (int t = 0; t < tables; ++t) n_rows[x] += cnt[t * E + e];
+        sum_r += n_rows[x];
+        sum_t += (n_rows[x] + tile_rows - 1) / tile_rows;
+    }
+    int inc_r = sum_r, inc_t = sum_t;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int a = __shfl_up(inc_r, off, 64), b = __shfl_up(inc_t, off, 64);
+        if (lane >= off) { inc_r += a; inc_t += b; }
+    }
+    if (lane == 63) { wave_sum[0][wave] = inc_r; wave_sum[1][wave] = inc_t; }
+    __syncthreads();
+    int o = inc_r - sum_r, t0 = inc_t - sum_t;
+    for (int w = 0; w < wave; ++w) { o += wave_sum[0][w]; t0 += wave_sum[1][w]; }
+#pragma unroll
+    for (int x = 0; x < PER; ++x) {
+        const int e = tid * PER + x;
+        if (e < E) {
+            offsets[e] = o;
+            first_tile[e] = t0;
+            int at = o;
+            for (int t = 0; t < tables; ++t) { const int c = cnt[t * E + e]; cnt[t * E + e] = at; at += c; }
+        }
+        o += n_rows[x];
+        t0 += (n_rows[x] + tile_rows - 1) / tile_rows;
+    }
+    if (tid == 1023) { offsets[E] = o; offsets[E + 1] = t0 < max_tiles ? t0 : max_tiles; first_tile[E] = t0; }
+    __syncthreads();
+    const int tiles = first_tile[E];
+    for (int t = tid; t < max_tiles; t += 1024) {
+        int lo = 0, hi = E;                                           // the expert whose tiles t is among: the last with first_tile <= t that has rows
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (first_tile[mid] <= t) lo = mid; else hi = mid;
+        }
+        tile_expert[t] = t < tiles ? lo : -1;
+        tile_row0[t] = t < tiles ? cnt[lo] + (t - first_tile[lo]) * tile_rows : 0;      // table 0's first place is the expert's first row
     }
     __syncthreads();
     // placement: a row's place within its expert is whatever the counter says when it arrives.  The order of an expert's rows
     // changes nothing in the results (every row is computed by itself); only which tile a row lands in differs from run to run.
-    for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
-    __syncthreads();
-    for (int64_t r = threadIdx.x; r < rows; r += 1024) {
-        const int e = ids[r];
-        if (e >= 0 && e < E) perm[base[e] + atomicAdd(&cnt[e], 1)] = (int32_t)r;
-    }
+    each([&](int32_t r, int e) { perm[atomicAdd(&mine[e], 1)] = r; });
 }
 
-extern "C" int jl_moe_tile_rows(void) { return MOE_TM; }
+// Rows of a tile.  High tiles read the weights less often and do more per byte of LDS, low ones pad less, give more workgroups and overlap their starts and ends.
+// 128 rows need both products to fill the chip and enough depth to pay for a tile's start; 64 need as many blocks as the chip takes at once.  Measured, experts
+// alone, bfloat16, us at 32 / 64 / 128 rows: 8 192 tokens x 4 of 32 (2048 x 1024) 1333 / 841 / 706; 512 tokens 163 / 159 / 156; 256 tokens 120 / 128 / 142;
+// 4 096 x 4 of 16 (1024 x 512) 227 / 141 / 168; 512 tokens 59 / 60 / 86; 1 024 x 4 of 8 (1024 x 2048) 216 / 146 / 169; float, 2 048 x 4 of 16: 418 / 356 / 432.
+// Sizes the matrix-core product does not take (rows that do not start at 16-byte borders) go in tiles of MOE_TM.
+static bool moe_mm_sizes(int dtype, int64_t K) { return (dtype == JL_BF16 && K % 8 == 0) || (dtype == JL_F32 && K % 4 == 0); }
+extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff) {
+    if (E <= 0 || !moe_mm_sizes(dtype, W) || !moe_mm_sizes(dtype, ff)) return MOE_TM;
+    auto blocks = [&](int tm, int width, int tn) { return (rows / tm + E / 2) * ((width + tn - 1) / tn); };
+    if (dtype == JL_BF16 && W + ff >= 3072 && blocks(128, ff, 128) >= 256 && blocks(128, W, 256) >= 256 && rows >= (int64_t)48 * E) return 128;
+    return rows >= (int64_t)48 * E && blocks(64, ff, 128) + blocks(64, W, 256) >= 512 ? 64 : 32;
+}
 
 extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, int32_t tile_rows, int32_t *perm, int32_t *offsets,
                             int32_t *tile_expert, int32_t *tile_row0, int32_t max_tiles, void *stream) {
@@ -139,21 +198,21 @@ extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t 
 }
 
 // ---- grouped product, any dtype and size: a 64 x 64 tile of one expert's rows per workgroup, float FMAs ------------------------------------
-struct MoeAct { int kind; float limit, alpha, shift; };       // the gated unit of JL_MOE_UP_GATED (jl_gated_act's kinds)
 
 // GATED: W holds 2 * n_out rows per expert, gate rows on linear rows; a tile forms both products of its columns and stores the unit
 template <typename T, bool GATED>
 __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, const T *__restrict__ Wt, int mode, int K, int n_out, int top,
                                                         const int32_t *__restrict__ perm, const int32_t *__restrict__ offsets,
                                                         const int32_t *__restrict__ tile_expert, const int32_t *__restrict__ tile_row0,
-                                                        const float *__restrict__ weights, void *__restrict__ out, MoeAct act) {
+                                                        const float *__restrict__ weights, void *__restrict__ out, MoeAct act, int tile_rows) {
     __shared__ float Xs[MOE_TM][MOE_TK + 1];
     __shared__ float Ws[(GATED ? 2 : 1) * MOE_TN][MOE_TK + 1];
     __shared__ int rin[MOE_TM];
     const int e = tile_expert[blockIdx.x];
     if (e < 0) return;
-    const int r0 = tile_row0[blockIdx.x];
-    const int nr = offsets[e + 1] - r0 < MOE_TM ? offsets[e + 1] - r0 : MOE_TM;
+    const int r0 = tile_row0[blockIdx.x] + blockIdx.z * MOE_TM, left = offsets[e + 1] - r0 < tile_rows - (int)blockIdx.z * MOE_TM ? offsets[e + 1] - r0 : tile_rows - (int)blockIdx.z * MOE_TM;
+    const int nr = left < MOE_TM ? left : MOE_TM;
+    if (nr <= 0) return;
     const int n0 = blockIdx.y * MOE_TN;
     const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
     if (tid < MOE_TM) rin[tid] = tid < nr ? (mode != 1 ? perm[r0 + tid] / top : r0 + tid) : -1;
@@ -214,148 +273,221 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
     }
 }
 
-// ---- grouped product on the matrix cores (bfloat16, K a multiple of 8) -----------------------------------------------------------------
-// A 64 x 128 tile per workgroup, four wavefronts side by side over the columns: each holds two 32 x 32 accumulators (rows 0-31 and
-// 32-63) and feeds v_mfma_f32_32x32x8_bf16 from LDS stages of depth 32.  Operand layout of that instruction: lane l supplies row
-// (A) or column (B) l % 32 with the four consecutive depths 4 * (l / 32) ..; accumulator i of lane l is row 8 * (i / 4) + 4 * (l / 32)
-// + i % 4, column l % 32.
-typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4_t;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
-constexpr int MM_TN = 128, MM_TK = 32, MM_LD = 36;     // LDS row stride in bf16 (72 bytes: rows 16 apart share a bank, no worse)
-
-// GATED: the tile's 128 columns of the gate AND of the linear branch (rows n_out further on in W): every wavefront holds four
-// accumulators, the A fragments serve both products, and the epilogue stores the gated unit.
-template <bool GATED>
-__global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16_t *__restrict__ X, const bf16_t *__restrict__ Wt, int mode, int K, int n_out,
-                                                             int top, const int32_t *__restrict__ perm, const int32_t *__restrict__ offsets,
-                                                             const int32_t *__restrict__ tile_expert, const int32_t *__restrict__ tile_row0,
-                                                             const float *__restrict__ weights, void *__restrict__ out, MoeAct act) {
-    __shared__ __attribute__((aligned(16))) bf16_t As[MOE_TM * MM_LD];
-    __shared__ __attribute__((aligned(16))) bf16_t Bs[(GATED ? 2 : 1) * MM_TN * MM_LD];
-    __shared__ int rin[MOE_TM];
-    const int e = tile_expert[blockIdx.x];
-    if (e < 0) return;
-    const int r0 = tile_row0[blockIdx.x];
-    const int nr = offsets[e + 1] - r0 < MOE_TM ? offsets[e + 1] - r0 : MOE_TM;
-    const int n0 = blockIdx.y * MM_TN;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if (tid < MOE_TM) rin[tid] = tid < nr ? (mode != 1 ? perm[r0 + tid] / top : r0 + tid) : -1;
-    __syncthreads();
-    const bf16_t *We = Wt + (int64_t)e * (GATED ? 2 : 1) * n_out * K;
-    // loaders: 8 bf16 (16 bytes) per thread and row segment; A 64 x 32 = 256 segments, B 128 x 32 = 512 segments (twice that when GATED)
-    const int a_row = tid >> 2, a_seg = (tid & 3) * 8;
-    const int64_t a_src = rin[a_row] >= 0 ? (int64_t)rin[a_row] * K : -1;
-    f32x16_t acc0 = {0}, acc1 = {0}, acu0 = {0}, acu1 = {0};
-    // a stage's rows travel from memory while the previous stage is multiplied: loaded into registers one iteration ahead
-    constexpr int NB = GATED ? 4 : 2;
-    uint4 av, bv[NB];
-    auto fetch = [&](int k0) {
-        av = make_uint4(0, 0, 0, 0);
-        if (a_src >= 0 && k0 + a_seg < K) av = *(const uint4 *)(X + a_src + k0 + a_seg);
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int n = (tid >> 2) + 64 * (i & 1);
-            bv[i] = make_uint4(0, 0, 0, 0);
-            if (n0 + n < n_out && k0 + a_seg < K) bv[i] = *(const uint4 *)(We + (int64_t)((i >> 1) * n_out + n0 + n) * K + k0 + a_seg);
-        }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += MM_TK) {
-        __syncthreads();                                   // the previous stage's readers are done
-        {
-            uint2 *d = (uint2 *)(As + a_row * MM_LD + a_seg);       // rows are 72 bytes apart: 8-byte stores stay aligned
-            d[0] = make_uint2(av.x, av.y);
-            d[1] = make_uint2(av.z, av.w);
-        }
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            uint2 *d = (uint2 *)(Bs + ((tid >> 2) + 64 * i) * MM_LD + a_seg);     // rows 0-127: gate (or the only) columns, 128-255: linear branch
-            d[0] = make_uint2(bv[i].x, bv[i].y);
-            d[1] = make_uint2(bv[i].z, bv[i].w);
-        }
-        __syncthreads();
-        if (k0 + MM_TK < K) fetch(k0 + MM_TK);
-#pragma unroll
-        for (int kk = 0; kk < MM_TK; kk += 8) {
-            const int ko = kk + 4 * (lane >> 5);
-            const bf16x4_t b = *(const bf16x4_t *)(Bs + (wave * 32 + (lane & 31)) * MM_LD + ko);
-            const bf16x4_t a0 = *(const bf16x4_t *)(As + (lane & 31) * MM_LD + ko);
-            const bf16x4_t a1 = *(const bf16x4_t *)(As + (32 + (lane & 31)) * MM_LD + ko);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a0, b, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a1, b, acc1, 0, 0, 0);
-            if (GATED) {
-                const bf16x4_t bu = *(const bf16x4_t *)(Bs + (MM_TN + wave * 32 + (lane & 31)) * MM_LD + ko);
-                acu0 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a0, bu, acu0, 0, 0, 0);
-                acu1 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a1, bu, acu1, 0, 0, 0);
-            }
-        }
+// ---- grouped product on the matrix cores -------------------------------------------------------------------------------------------------
+// A tile of TM rows of one expert by WR of its weight rows, both K-major, walked in stages of TKU 16-byte units per row (8 bfloat16 or 4 floats each)
+// through two LDS buffers: the next stage's units travel from memory while this one is multiplied, one barrier per stage.  NW wavefronts (two over the
+// rows when TM is 128) hold 32 x 32 accumulators; the weights are the A operand, the rows the B operand, so that a lane ends with four neighbouring
+// output columns of ONE row and stores them together.  A lane's operand is one 16-byte unit: in bfloat16 the eight depths 8 (lane / 32) .. of
+// v_mfma_f32_32x32x16_bf16; in float four v_mfma_f32_32x32x2_f32, one for each of its floats (the depths meet in the order 0, 4, 1, 5, ..: a sum of
+// products rounded one by one, as a chain of multiply-adds is).  Units of a row are permuted so that 16 neighbouring rows meet different banks.
+// GATED: the WR weight rows are WR / 2 of the gate and the WR / 2 of the linear branch that belong to them (rows n_out further on); both products
+// of a column end in the same lane, which stores the gated unit.
+// TM = 128 (an expert has about a hundred rows or more) is bound by the matrix cores and LDS: 128 x 256 reads 48 KB of LDS per 64 products, so two
+// workgroups fit a CU and cover each other's barriers.  Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an
+// expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading the weights: single wavefronts, many per CU, 12 KB on the way each.
+struct MoeMM {
+    const void *X, *Wt;
+    const int32_t *perm, *offsets, *tile_expert, *tile_row0;
+    const float *weights;
+    void *out;
+    int mode, K, n_out, top, E, col_blocks, max_tiles;
+    MoeAct act;
+};
+typedef __bf16 mm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float mm_f32x16 __attribute__((ext_vector_type(16)));
+template <typename T> struct mm_type;
+template <> struct mm_type<bf16_t> {
+    static constexpr int UNIT = 8;
+    static __device__ __forceinline__ mm_f32x16 mma(uint4 a, uint4 b, mm_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mm_bf16x8, a), __builtin_bit_cast(mm_bf16x8, b), c, 0, 0, 0);
     }
-    const int n = n0 + wave * 32 + (lane & 31);
-    if (n >= n_out) return;
+};
+template <> struct mm_type<float> {
+    static constexpr int UNIT = 4;
+    static __device__ __forceinline__ mm_f32x16 mma(uint4 a, uint4 b, mm_f32x16 c) {
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+    }
+};
+
+template <typename T, int TM, int NW, int WR, int TKU, bool GATED>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM a) {
+    constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
+    constexpr int XPF = TM * TKU / THREADS, WPF = WR * TKU / THREADS, TN = GATED ? WR / 2 : WR, STAGE = TKU * UNIT;
+    static_assert(XPF * THREADS == TM * TKU && WPF * THREADS == WR * TKU && (!GATED || NT % 2 == 0), "tile");
+    __shared__ uint4 smem[2 * (TM + WR) * TKU];
+    int tile, col;
+    if (TM >= 64) {                                                 // workgroups with the same remainder by 8 share an XCD
+        const int per_xcd = (a.offsets[a.E + 1] + 7) / 8, xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
+        if (s >= per_xcd * a.col_blocks) return;
+        tile = xcd * per_xcd + s / a.col_blocks;
+        col = s % a.col_blocks;
+        if (tile >= a.max_tiles) return;
+    } else {
+        tile = blockIdx.x / a.col_blocks;
+        col = blockIdx.x - tile * a.col_blocks;
+    }
+    const int e = a.tile_expert[tile];
+    if (e < 0) return;
+    const int r0 = a.tile_row0[tile], K = a.K, n_out = a.n_out, n0 = col * TN;
+    const int nr = a.offsets[e + 1] - r0 < TM ? a.offsets[e + 1] - r0 : TM;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave / WN, wn = wave % WN;
+    auto at = [](int row, int u) { return row * TKU + (u ^ (TKU == 4 ? (row >> 2) & 3 : (row >> 1) & 7)); };
+    // loaders: unit tid % TKU of rows tid / TKU + x * THREADS / TKU; a row that does not exist is zero (and stays zero in LDS)
+    const int lu = tid % TKU, lr = tid / TKU;
+    const T *xp[XPF], *wp[WPF];
 #pragma unroll
-    for (int half = 0; half < 2; ++half)
+    for (int x = 0; x < XPF; ++x) {
+        const int m = lr + x * (THREADS / TKU);
+        xp[x] = m < nr ? (const T *)a.X + (int64_t)(a.mode != 1 ? a.perm[r0 + m] / a.top : r0 + m) * K + lu * UNIT : nullptr;
+    }
+    const T *We = (const T *)a.Wt + (int64_t)e * (GATED ? 2 : 1) * n_out * K;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = 32 * half + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-            if (m >= nr) continue;
-            const float c = half ? acc1[i] : acc0[i];
-            const int r = r0 + m;
-            if (GATED) {
-                st_f((bf16_t *)out + (int64_t)r * n_out + n, gated_unit_f<true>(c, half ? acu1[i] : acu0[i], act.kind, act.limit, act.alpha, act.shift));
-            } else if (mode == JL_MOE_UP_PLAIN) {
-                st_f((bf16_t *)out + (int64_t)r * n_out + n, c);
-            } else if (mode == 0) {
-                const float v = fmaxf(c, 0.f);
-                st_f((bf16_t *)out + (int64_t)r * n_out + n, v * v);
-            } else {
-                const int p = perm[r];
-                ((float *)out)[(int64_t)p * n_out + n] = c * weights[p];
-            }
+    for (int x = 0; x < WPF; ++x) {
+        const int j = lr + x * (THREADS / TKU), c = GATED ? j % TN : j;
+        wp[x] = n0 + c < n_out ? We + (int64_t)((GATED && j >= TN ? n_out : 0) + n0 + c) * K + lu * UNIT : nullptr;
+    }
+    uint4 reg[2][XPF + WPF];                                        // stages on their way: even ones in reg[0], odd ones in reg[1]
+    auto fetch = [&](uint4 (&r)[XPF + WPF], int k0) {
+        const bool in = k0 + lu * UNIT < K;
+#pragma unroll
+        for (int x = 0; x < XPF; ++x) r[x] = in && xp[x] ? *(const uint4 *)(xp[x] + k0) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int x = 0; x < WPF; ++x) r[XPF + x] = in && wp[x] ? *(const uint4 *)(wp[x] + k0) : make_uint4(0, 0, 0, 0);
+    };
+    auto stash = [&](const uint4 (&r)[XPF + WPF], int sel) {
+        uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
+#pragma unroll
+        for (int x = 0; x < XPF; ++x) Xs[at(lr + x * (THREADS / TKU), lu)] = r[x];
+#pragma unroll
+        for (int x = 0; x < WPF; ++x) Ws[at(lr + x * (THREADS / TKU), lu)] = r[XPF + x];
+    };
+    mm_f32x16 acc[XT][NT];
+#pragma unroll
+    for (int x = 0; x < XT; ++x)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[x][t][i] = 0.f;
+    // weight row (within the tile) of this wavefront's tile t: gate tiles first, then the linear branch's
+    auto w_row = [&](int t) { return GATED ? (t < NT / 2 ? 0 : TN) + wn * (TN / WN) + 32 * (t % (NT / 2 > 0 ? NT / 2 : 1)) : wn * (WR / WN) + 32 * t; };
+    fetch(reg[0], 0);
+    fetch(reg[1], STAGE);
+    stash(reg[0], 0);
+    __syncthreads();
+    auto stage = [&](int k0, auto sel_c) {
+        constexpr int sel = decltype(sel_c)::value;
+        fetch(reg[sel], k0 + 2 * STAGE);                            // two stages ahead: a trip to memory takes longer than one stage's products
+        const uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
+#pragma unroll
+        for (int s = 0; s < TKU / 2; ++s) {
+            uint4 xf[XT], wf[NT];
+#pragma unroll
+            for (int x = 0; x < XT; ++x) xf[x] = Xs[at(wm * (TM / WM) + 32 * x + l32, 2 * s + hi)];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wf[t] = Ws[at(w_row(t) + l32, 2 * s + hi)];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int x = 0; x < XT; ++x) acc[x][t] = mm_type<T>::mma(wf[t], xf[x], acc[x][t]);
         }
+        stash(reg[sel ^ 1], sel ^ 1);
+        __syncthreads();
+    };
+    for (int k0 = 0; k0 < K; k0 += 2 * STAGE) {
+        stage(k0, std::integral_constant<int, 0>());
+        if (k0 + STAGE < K) stage(k0 + STAGE, std::integral_constant<int, 1>());
+    }
+    constexpr int OT = GATED ? NT / 2 : NT;
+    const bool whole = n_out % 4 == 0;
+#pragma unroll
+    for (int x = 0; x < XT; ++x) {
+        const int m = wm * (TM / WM) + 32 * x + l32;
+        if (m >= nr) continue;
+        const int64_t r = r0 + m;
+        const int64_t p = a.mode == 1 ? a.perm[r] : r;
+        const float w = a.mode == 1 ? a.weights[p] : 1.0f;
+#pragma unroll
+        for (int t = 0; t < OT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n = n0 + w_row(t) + 8 * g + 4 * hi;       // four neighbouring columns
+                if (n >= n_out) continue;
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float c = acc[x][t][4 * g + i];
+                    if (GATED) v[i] = gated_unit_f<sizeof(T) == 2>(c, acc[x][t + (GATED ? OT : 0)][4 * g + i], a.act.kind, a.act.limit, a.act.alpha, a.act.shift);
+                    else if (a.mode == JL_MOE_UP_PLAIN) v[i] = c;
+                    else if (a.mode == 0) { const float q = fmaxf(c, 0.f); v[i] = q * q; }
+                    else v[i] = c * w;
+                }
+                const int64_t o = p * n_out + n;
+                if (!GATED && a.mode == 1) {
+                    if (whole) st4_f((float *)a.out + o, v);
+                    else for (int i = 0; i < 4 && n + i < n_out; ++i) ((float *)a.out)[o + i] = v[i];
+                } else {
+                    if (whole) st4_f((T *)a.out + o, v);
+                    else for (int i = 0; i < 4 && n + i < n_out; ++i) st_f((T *)a.out + o + i, v[i]);
+                }
+            }
+    }
+}
+
+template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(MoeMM &a, bool gated, hipStream_t st) {
+    const int tn = gated ? WR / 2 : WR;
+    a.col_blocks = (a.n_out + tn - 1) / tn;
+    const int64_t groups = (int64_t)(TM >= 64 ? (a.max_tiles + 7) / 8 * 8 : a.max_tiles) * a.col_blocks;
+    if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
+    if (gated) moe_mm_kernel<T, TM, NW, WR, TKU, true><<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
+    else moe_mm_kernel<T, TM, NW, WR, TKU, false><<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
+    return jl_check_launch("moe_mm_kernel");
+}
+template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated, hipStream_t st) {
+    if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
+    if (tile_rows == 64) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
+    return moe_mm_launch<T, 32, 1, 64, 8>(a, gated, st);
 }
 
 static int moe_gemm_launch(const void *X, const void *Wt, int dtype, int32_t mode, int32_t K, int32_t n_out, int32_t top, const int32_t *perm,
-                           const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, const float *weights,
-                           void *out, const MoeAct *act, void *stream) {
+                           const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t E, int32_t tile_rows,
+                           const float *weights, void *out, const MoeAct *act, void *stream) {
     static const bool no_mfma = getenv("JL_MOE_NO_MFMA") != nullptr;      // A/B switch for measurements
-    const MoeAct none = {0, 0.f, 0.f, 0.f};
-    if (!no_mfma && dtype == JL_BF16 && K % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)Wt % 16) == 0) {
-        const dim3 mgrid((unsigned)max_tiles, (unsigned)((n_out + MM_TN - 1) / MM_TN));
-        if (act)
-            moe_gemm_mfma_kernel<true><<<mgrid, 256, 0, (hipStream_t)stream>>>((const bf16_t *)X, (const bf16_t *)Wt, mode, K, n_out, top, perm, offsets,
-                                                                              tile_expert, tile_row0, weights, out, *act);
-        else
-            moe_gemm_mfma_kernel<false><<<mgrid, 256, 0, (hipStream_t)stream>>>((const bf16_t *)X, (const bf16_t *)Wt, mode, K, n_out, top, perm, offsets,
-                                                                               tile_expert, tile_row0, weights, out, none);
-        return jl_check_launch("moe_gemm_mfma_kernel");
+    if (E <= 0 || (tile_rows != 32 && tile_rows != 64 && tile_rows != 128)) return jl_fail(JL_E_INVALID, "jl_moe_gemm: tiles of 32, 64 or 128 rows");
+    MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}};
+    if (!no_mfma && moe_mm_sizes(dtype, K) && ((uintptr_t)X % 16) == 0 && ((uintptr_t)Wt % 16) == 0 && ((uintptr_t)out % 16) == 0) {
+        if (dtype == JL_BF16) return moe_mm_rows<bf16_t>(a, tile_rows, act != nullptr, (hipStream_t)stream);
+        return moe_mm_rows<float>(a, tile_rows, act != nullptr, (hipStream_t)stream);
     }
-    const dim3 grid((unsigned)max_tiles, (unsigned)((n_out + MOE_TN - 1) / MOE_TN));
+    const dim3 grid((unsigned)max_tiles, (unsigned)((n_out + MOE_TN - 1) / MOE_TN), (unsigned)((tile_rows + MOE_TM - 1) / MOE_TM));
     if (act)
         JL_DISPATCH(dtype, moe_gemm_kernel<T, true><<<grid, 256, 0, (hipStream_t)stream>>>((const T *)X, (const T *)Wt, mode, K, n_out, top, perm, offsets,
-                                                                                           tile_expert, tile_row0, weights, out, *act));
+                                                                                           tile_expert, tile_row0, weights, out, a.act, tile_rows));
     else
         JL_DISPATCH(dtype, moe_gemm_kernel<T, false><<<grid, 256, 0, (hipStream_t)stream>>>((const T *)X, (const T *)Wt, mode, K, n_out, top, perm, offsets,
-                                                                                            tile_expert, tile_row0, weights, out, none));
+                                                                                            tile_expert, tile_row0, weights, out, a.act, tile_rows));
     return jl_check_launch("moe_gemm_kernel");
 }
 
 extern "C" int jl_moe_gemm(const void *X, const void *Wt, int dtype, int32_t mode, int32_t K, int32_t n_out, int32_t top,
                            const int32_t *perm, const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0,
-                           int32_t max_tiles, const float *weights, void *out, void *stream) {
+                           int32_t max_tiles, int32_t E, int32_t tile_rows, const float *weights, void *out, void *stream) {
     if (max_tiles <= 0) return JL_OK;
     if (!X || !Wt || !perm || !offsets || !tile_expert || !tile_row0 || !out || (mode == 1 && !weights))
         return jl_fail(JL_E_INVALID, "jl_moe_gemm: null pointer");
     if (K <= 0 || n_out <= 0 || top <= 0 || (mode != 0 && mode != 1 && mode != JL_MOE_UP_PLAIN)) return jl_fail(JL_E_INVALID, "jl_moe_gemm: bad sizes or mode");
-    return moe_gemm_launch(X, Wt, dtype, mode, K, n_out, top, perm, offsets, tile_expert, tile_row0, max_tiles, weights, out, nullptr, stream);
+    return moe_gemm_launch(X, Wt, dtype, mode, K, n_out, top, perm, offsets, tile_expert, tile_row0, max_tiles, E, tile_rows, weights, out, nullptr, stream);
 }
 
 extern "C" int jl_moe_gemm_gated(const void *X, const void *Wt, int dtype, int32_t K, int32_t ff, int32_t top, const int32_t *perm,
-                                 const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t kind,
-                                 float limit, float alpha, float shift, void *out, void *stream) {
+                                 const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t E,
+                                 int32_t tile_rows, int32_t kind, float limit, float alpha, float shift, void *out, void *stream) {
     if (max_tiles <= 0) return JL_OK;
     if (!X || !Wt || !perm || !offsets || !tile_expert || !tile_row0 || !out) return jl_fail(JL_E_INVALID, "jl_moe_gemm_gated: null pointer");
     if (K <= 0 || ff <= 0 || top <= 0 || kind < JL_ACT_GELU_TANH || kind > JL_ACT_GELU_ERF)
         return jl_fail(JL_E_INVALID, "jl_moe_gemm_gated: bad sizes or kind");
     const MoeAct act = {kind, limit, alpha, shift};
-    return moe_gemm_launch(X, Wt, dtype, JL_MOE_UP_PLAIN, K, ff, top, perm, offsets, tile_expert, tile_row0, max_tiles, nullptr, out, &act, stream);
+    return moe_gemm_launch(X, Wt, dtype, JL_MOE_UP_PLAIN, K, ff, top, perm, offsets, tile_expert, tile_row0, max_tiles, E, tile_rows, nullptr, out, &act, stream);
 }

@@ -461,26 +461,26 @@ def moe_experts(h: torch.Tensor, router_logits: torch.Tensor, correction: Option
     wts = torch.empty((n, top), dtype=torch.float32, device=dev)
     N.check_layers(L.jl_moe_route(_ptr(router_logits), _ptr(correction), n, Er, top, float(scale), _ptr(ids), _ptr(wts),
                                   _ROUTES[route], float(renorm_eps), st), "jl_moe_route")
-    tm = int(L.jl_moe_tile_rows())
     rows = n * top
+    tm = int(L.jl_moe_tile_rows(_code(dt), rows, E, W, ff))
     max_tiles = rows // tm + E
     perm = torch.empty((rows,), dtype=torch.int32, device=dev)
-    offsets = torch.empty((E + 1,), dtype=torch.int32, device=dev)
+    offsets = torch.empty((E + 2,), dtype=torch.int32, device=dev)
     tile_e = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
     tile_r = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
     N.check_layers(L.jl_moe_group(_ptr(ids), n, top, E, tm, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, st), "jl_moe_group")
     if gated is not None and not os.environ.get("JL_MOE_UNFUSED_ACT"):          # the unit in the product's epilogue (A/B switch for measurements)
         act = torch.empty((rows, ff), dtype=dt, device=dev)
-        N.check_layers(L.jl_moe_gemm_gated(_ptr(h), _ptr(w_up), _code(dt), W, ff, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles,
+        N.check_layers(L.jl_moe_gemm_gated(_ptr(h), _ptr(w_up), _code(dt), W, ff, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm,
                                            int(gated[0]), float(gated[1]), float(gated[2]), float(gated[3]), _ptr(act), st), "jl_moe_gemm_gated")
     else:
         act = torch.empty((rows, up_rows), dtype=dt, device=dev)
         N.check_layers(L.jl_moe_gemm(_ptr(h), _ptr(w_up), _code(dt), N.JL_MOE_UP_PLAIN if gated is not None else N.JL_MOE_UP_RELU2, W, up_rows, top, _ptr(perm),
-                                     _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, None, _ptr(act), st), "jl_moe_gemm(up)")
+                                     _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm, None, _ptr(act), st), "jl_moe_gemm(up)")
         if gated is not None:
             act = gated_act(act, 0, ff, ff, *gated)
     y = torch.empty((n, top, W), dtype=torch.float32, device=dev)
-    N.check_layers(L.jl_moe_gemm(_ptr(act), _ptr(w_down), _code(dt), N.JL_MOE_DOWN, ff, W, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles,
+    N.check_layers(L.jl_moe_gemm(_ptr(act), _ptr(w_down), _code(dt), N.JL_MOE_DOWN, ff, W, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm,
                                  _ptr(wts), _ptr(y), st), "jl_moe_gemm(down)")
     return (y, ids, wts) if identity else y
 
