@@ -117,8 +117,8 @@ JL_API int jl_attn_window(const jl_attn_args *a, void *stream);
 JL_API int jl_attn_tile_rows(int dtype, int32_t H, int32_t G, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
 
 /* The same attention without bias and head mixing (sink and gate as above), in ONE sweep over the keys on the matrix cores, for heads in groups that
- * share a key head (H / G query heads per key head c, value head c % Gv): bfloat16, D % 8 == 0 up to 640, Dv % 32 == 0 up to 512,
- * row strides % 4 == 0.  v_cache == k_cache (with G = 1, Dv <= D): the values are the first Dv columns of the key rows — the pool
+ * share a key head (H / G query heads per key head c, value head c % Gv): bfloat16, D % 8 == 0 up to 640, Dv % 32 == 0 up to 512; float, D % 4 == 0 up to 256,
+ * Dv % 32 == 0 up to 128, rows at 16-byte borders; row strides % 4 == 0.  v_cache == k_cache (with G = 1, Dv <= D): the values are the first Dv columns of the key rows — the pool
  * of latent attention — and are not loaded a second time.  Of jl_attn_args it reads q, k_cache, v_cache, k_ld, v_ld, out, out_dtype,
  * block_tables, bt_stride, tiles, n_tiles, page_size, H, G, Gv, D, Dv, window, scale, dtype, sink, gate, gate_ld, gate_heads, splits, scratch and TQ, which must be
  * what jl_attn_sweep_tile_rows returns (0: sizes not taken).  splits in 2 .. 64: the keys of every tile are shared out over that
@@ -134,7 +134,7 @@ JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t
                                         int32_t v_in_k);
 
 /* The wide form over keys and values that were built per head for this step (long portions of latent attention: keys and values from the latent
- * by a product instead of queries brought to the latent), bfloat16, G = H, contiguous rows per request instead of pages: key head c of a row is
+ * by a product instead of queries brought to the latent), G = H, contiguous rows per request instead of pages: key head c of a row is
  * columns c * (D - k_tail_cols) .. of k_cache followed by the row's k_tail_cols shared columns; value head c is columns c * Dv .. of v_cache.
  * D, k_tail_cols % 8 == 0, D <= 256, Dv % 32 == 0 up to 128, row strides % 4 == 0.  Of jl_attn_args it reads what jl_attn_sweep reads except pages and splits;
  * tiles of jl_attn_expanded_tile_rows() queries, in any order. */

@@ -9,4 +9,12 @@ constexpr int AR_ROWS = 128;          // (query, head) rows of a tile of the wid
 // the wide form's launch (jl_attn_rows.hip); sizes as jl_attn_sweep has checked them, ``hf`` heads of a.TQ queries per tile, ``hb`` tiles per group
 int jl_attn_rows_launch(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st);
 
+// where keys and values come from: pages of pools, pages whose key rows hold the values in their first columns, or contiguous rows per request whose heads
+// share their last columns (keys and values built for this step)
+enum { AR_PAGED, AR_V_IN_K, AR_BUILT };
+
+// float activations (jl_attn_f32.hip): tiles of 128 rows (``wide``) or of 32, whose keys may be shared out
+bool jl_attn_f32_fits(int H, int G, int Gv, int D, int Dv, int64_t k_ld, int64_t v_ld, bool v_in_k);
+int jl_attn_f32_launch(const jl_attn_args &a, int hf, int hb, int src, bool wide, hipStream_t st);
+
 #endif

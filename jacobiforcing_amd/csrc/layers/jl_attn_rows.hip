@@ -38,10 +38,6 @@ constexpr size_t ar_lds_bytes(int KU, int VU) { return 2 * (size_t)ar_tile_keys(
 template <int U> __device__ __forceinline__ int ar_key_unit(int r, int u) { return U % 16 == 0 ? u ^ (r & 15) : u ^ ((r >> 1) & 7); }
 template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { return U == 16 ? u ^ ((r & 3) << 2) : u ^ ((r & 2) << 1); }
 
-// where keys and values come from: pages of pools, pages whose key rows hold the values in their first columns, or contiguous rows per request whose heads
-// share their last columns (keys and values built for this step)
-enum { AR_PAGED, AR_V_IN_K, AR_BUILT };
-
 template <int KU, int VU, int SRC>                                                      // D <= 8 * KU, Dv <= 8 * VU
 __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a, int HF, int TQ, int HB) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -334,15 +330,16 @@ extern "C" int jl_attn_expanded(const jl_attn_args *ap, void *stream) {
     if (a.n_tiles <= 0) return JL_OK;
     if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.tiles || !a.key_base || (a.k_tail_cols > 0 && !a.k_tail)) return jl_fail(JL_E_INVALID, "jl_attn_expanded: null pointer");
     const int64_t own = a.D - a.k_tail_cols;
-    if (a.dtype != JL_BF16 || a.H <= 0 || a.G != a.H || (a.Gv > 0 && a.Gv != a.H) || a.D <= 0 || a.D % 8 || a.D > 256 || a.k_tail_cols < 0 || a.k_tail_cols % 8 || own < 0 ||
+    if ((a.dtype != JL_BF16 && a.dtype != JL_F32) || a.H <= 0 || a.G != a.H || (a.Gv > 0 && a.Gv != a.H) || a.D <= 0 || a.D % 8 || a.D > 256 || a.k_tail_cols < 0 || a.k_tail_cols % 8 || own < 0 ||
         a.Dv < 32 || a.Dv % 32 || a.Dv > 128 || a.TQ != AR_ROWS || a.n_tiles > 65535)
-        return jl_fail(JL_E_INVALID, "jl_attn_expanded: bfloat16, a key and a value head per query head, key widths in multiples of 8 up to 256, value widths in multiples of 32 up to 128");
+        return jl_fail(JL_E_INVALID, "jl_attn_expanded: a key and a value head per query head, key widths in multiples of 8 up to 256, value widths in multiples of 32 up to 128");
     if (a.k_ld < a.H * own || a.v_ld < (int64_t)a.H * a.Dv || a.q_ld < (int64_t)a.H * a.D || a.out_ld < (int64_t)a.H * a.Dv || (a.k_tail_cols > 0 && a.k_tail_ld < a.k_tail_cols) ||
         a.k_ld % 4 || a.v_ld % 4 || a.q_ld % 4 || a.out_ld % 4 || a.k_tail_ld % 4)
         return jl_fail(JL_E_INVALID, "jl_attn_expanded: row strides hold a row and are multiples of four");
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_expanded: unknown out_dtype");
     if (a.chunk > 0 && a.window > 0) return jl_fail(JL_E_INVALID, "jl_attn_expanded: chunks exclude a window");
     hipStream_t st = (hipStream_t)stream;
+    if (a.dtype == JL_F32) return jl_attn_f32_launch(a, 1, 1, AR_BUILT, true, st);
     const int ku = 8 * ((a.D + 63) / 64), vu = a.Dv <= 64 ? 8 : 16;
 #define AR_CASE(K, V) if (ku == K && vu == V) return ar_launch<K, V, AR_BUILT>(a, 1, 1, st)
     AR_CASE(8, 8); AR_CASE(8, 16);

@@ -241,6 +241,7 @@ __global__ __launch_bounds__(AS_THREADS) void attn_sweep_kernel(jl_attn_args a, 
 // out[row] = sum_s part_s[row] * exp(m_s - M) / sum_s l_s * exp(m_s - M), outputs summed in share order.  A workgroup joins AJ_ROWS of a
 // tile's rows; a row's weights are formed by one wavefront, lane s holding share s (at most 64).
 constexpr int AJ_ROWS = 4;
+template <typename T>                                                                    // of the gate, and of the outputs where they are not float anyway
 __global__ __launch_bounds__(256) void attn_sweep_join_kernel(jl_attn_args a, int HF, int TQ, int HB) {
     __shared__ float wS[AJ_ROWS * 64];
     const int H = a.H, Dv = a.Dv, S = a.splits, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r0 = blockIdx.z * AJ_ROWS;
@@ -256,12 +257,12 @@ __global__ __launch_bounds__(256) void attn_sweep_join_kernel(jl_attn_args a, in
         float M = m;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-        const float w = m > -INFINITY ? __expf(m - M) : 0.f;
+        const float w = m > -INFINITY ? (sizeof(T) == 4 ? expf(m - M) : __expf(m - M)) : 0.f;
         const float L = wave_sum_f32(w * l);
         wS[r * 64 + lane] = L > 0.f ? w / L : 0.f;
     }
     __syncthreads();
-    bf16_t *out = (bf16_t *)a.out;
+    T *out = (T *)a.out;
     for (int e = tid; e < AJ_ROWS * Dv; e += 256) {
         const int r = e / Dv, col = e - r * Dv, row = r0 + r, ii = row / HF, hh = h0 + row % HF;
         if (row >= TQ * HF || ii >= cnt || hh >= h_end) continue;
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(256) void attn_sweep_join_kernel(jl_attn_args a, in
         for (int sp = 0; sp < S; ++sp) v += wS[r * 64 + sp] * base[sp * share + r * (Dv + 2) + col];
         const int64_t o = (int64_t)(row0 + ii) * a.out_ld + hh * Dv + col;
         v *= a.out_scale;
-        if (a.gate) v *= 1.0f / (1.0f + __expf(-ld_f((const bf16_t *)a.gate + (int64_t)(row0 + ii) * a.gate_ld + (a.gate_heads ? hh : hh * Dv + col))));
+        if (a.gate) v *= sigmoid_f<false>(ld_f((const T *)a.gate + (int64_t)(row0 + ii) * a.gate_ld + (a.gate_heads ? hh : hh * Dv + col)));
         if (a.out_dtype == JL_OUT_F32) ((float *)a.out)[o] = v;
         else st_f(out + o, v);
     }
@@ -285,6 +286,7 @@ extern "C" int64_t jl_attn_sweep_scratch_floats(int32_t n_tiles, int32_t H, int3
 }
 
 static bool as_fits(int dtype, int H, int G, int Gv, int D, int Dv, int64_t k_ld, int64_t v_ld, bool v_in_k) {
+    if (dtype == JL_F32) return jl_attn_f32_fits(H, G, Gv, D, Dv, k_ld, v_ld, v_in_k);
     if (!(dtype == JL_BF16 && H >= 1 && G >= 1 && H % G == 0 && Gv >= 1 && G % Gv == 0 && D % 8 == 0 && D <= 8 * AS_WAVES * AS_QSTEPS && Dv % 32 == 0 &&
           Dv >= 32 && Dv <= 512 && k_ld % 4 == 0 && v_ld % 4 == 0 && k_ld >= (int64_t)G * D))
         return false;
@@ -304,7 +306,7 @@ static bool ar_fits(int dtype, int H, int G, int Gv, int D, int Dv, int64_t k_ld
 }
 
 extern "C" int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld, int32_t v_in_k) {
-    if (!ar_fits(dtype, H, G, Gv > 0 ? Gv : G, D, Dv, k_ld, v_in_k ? k_ld : v_ld, v_in_k != 0)) return 0;
+    if (dtype == JL_F32 ? !as_fits(dtype, H, G, Gv > 0 ? Gv : G, D, Dv, k_ld, v_in_k ? k_ld : v_ld, v_in_k != 0) : !ar_fits(dtype, H, G, Gv > 0 ? Gv : G, D, Dv, k_ld, v_in_k ? k_ld : v_ld, v_in_k != 0)) return 0;
     return AR_ROWS / as_heads_per_tile(H, G);
 }
 
@@ -319,17 +321,21 @@ extern "C" int jl_attn_sweep(const jl_attn_args *ap, void *stream) {
     const bool v_in_k = a.v_cache == a.k_cache;
     if (a.v_ld <= 0) a.v_ld = v_in_k ? a.k_ld : (int64_t)a.Gv * a.Dv;
     if (!as_fits(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld, v_in_k))
-        return jl_fail(JL_E_INVALID, "jl_attn_sweep: bfloat16, key width a multiple of 8 up to %d, value width a multiple of 32 up to 512, row strides in "
-                       "multiples of 4; values inside the key rows need one key head", 8 * AS_WAVES * AS_QSTEPS);
+        return jl_fail(JL_E_INVALID, "jl_attn_sweep: key width a multiple of 8 up to %d, value width a multiple of 32 up to 512 (float: of 4 up to 256, of 32 up to 128), row "
+                       "strides in multiples of 4; values inside the key rows need one key head", 8 * AS_WAVES * AS_QSTEPS);
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_sweep: unknown out_dtype");
     if (a.out_ld <= 0) a.out_ld = (int64_t)a.H * a.Dv;
     if (a.out_ld < (int64_t)a.H * a.Dv || a.out_ld % 4) return jl_fail(JL_E_INVALID, "jl_attn_sweep: the output's row stride holds a row and is a multiple of four");
     if (a.chunk > 0 && a.window > 0) return jl_fail(JL_E_INVALID, "jl_attn_sweep: chunks exclude a window");
     const int hf = as_heads_per_tile(a.H, a.G), hb = as_head_blocks(a.H, a.G), tq = AS_T / hf;
     if (a.TQ == AR_ROWS / hf && a.TQ != tq) {                       // tiles of up to 128 rows: every wavefront keeps its rows to itself
-        if (a.splits > 1 || !ar_fits(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld, v_in_k))
+        if (a.splits > 1 || (a.dtype == JL_BF16 && !ar_fits(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld, v_in_k)))
             return jl_fail(JL_E_INVALID, "jl_attn_sweep: 128-row tiles take key widths up to 256, value widths up to 128 and no shared-out keys");
         hipStream_t st = (hipStream_t)stream;
+        if (a.dtype == JL_F32) {
+            a.q_ld = (int64_t)a.H * a.D;
+            return jl_attn_f32_launch(a, hf, hb, v_in_k ? AR_V_IN_K : AR_PAGED, true, st);
+        }
         return jl_attn_rows_launch(a, hf, hb, v_in_k, st);
     }
     if (a.TQ != tq) return jl_fail(JL_E_INVALID, "jl_attn_sweep: tiles of %d queries wanted (ask jl_attn_sweep_tile_rows)", tq);
@@ -337,6 +343,13 @@ extern "C" int jl_attn_sweep(const jl_attn_args *ap, void *stream) {
     const size_t lds = as_lds_bytes(a.D, a.Dv, v_in_k);
     const dim3 grid((unsigned)a.n_tiles, (unsigned)(a.G * hb), (unsigned)(a.splits > 1 ? a.splits : 1));
     hipStream_t st = (hipStream_t)stream;
+    if (a.dtype == JL_F32) {
+        a.q_ld = (int64_t)a.H * a.D;
+        const int rc = jl_attn_f32_launch(a, hf, hb, v_in_k ? AR_V_IN_K : AR_PAGED, false, st);
+        if (rc != JL_OK || a.splits <= 1) return rc;
+        attn_sweep_join_kernel<float><<<dim3(grid.x, grid.y, AS_T / AJ_ROWS), 256, 0, st>>>(a, hf, tq, hb);
+        return jl_check_launch("attn_sweep_join_kernel");
+    }
 #define AS_CASE(NTV)                                                                                                              \
     case NTV: {                                                                                                                   \
         auto kern = attn_sweep_kernel<NTV>;                                                                                       \
@@ -351,6 +364,6 @@ extern "C" int jl_attn_sweep(const jl_attn_args *ap, void *stream) {
         AS_CASE(1) AS_CASE(2) AS_CASE(3) AS_CASE(4)
     }
 #undef AS_CASE
-    if (a.splits > 1) attn_sweep_join_kernel<<<dim3(grid.x, grid.y, AS_T / AJ_ROWS), 256, 0, st>>>(a, hf, tq, hb);
+    if (a.splits > 1) attn_sweep_join_kernel<bf16_t><<<dim3(grid.x, grid.y, AS_T / AJ_ROWS), 256, 0, st>>>(a, hf, tq, hb);
     return jl_check_launch("attn_sweep_kernel");
 }

@@ -337,7 +337,7 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
 def attn_sweep_tile_rows(dtype: torch.dtype, H: int, G: int, D: int, Dv: int, k_cache: torch.Tensor, v_cache: torch.Tensor, value_heads: int = 0) -> int:
     """Queries per tile of the one-sweep kernel (heads in groups over a key head) for these sizes and pools; 0 when it does not
     take them."""
-    if dtype != torch.bfloat16 or os.environ.get("JL_ATTN_NO_SWEEP"):                          # A/B switch for measurements
+    if os.environ.get("JL_ATTN_NO_SWEEP") or (dtype == torch.float32 and (k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16)):      # A/B switch for measurements; float rows are read 16 bytes at a time
         return 0
     v_in_k = v_cache.data_ptr() == k_cache.data_ptr()
     return int(N.layers().jl_attn_sweep_tile_rows(_code(dtype), H, G, value_heads or G, D, Dv, k_cache.stride(0), v_cache.stride(0), int(v_in_k)))
@@ -347,7 +347,7 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
                window: int, value_heads: int = 0, float_out: bool = False, sink: Optional[torch.Tensor] = None,
                gate: Optional[torch.Tensor] = None, gate_per_head: bool = False, chunk: int = 0, softcap: float = 0.0, out_scale: float = 1.0,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Attention without bias or head mixing (``sink`` / ``gate`` / ``chunk`` / ``softcap`` / ``out_scale`` / ``out`` as for ``attn_window``) in one sweep on the matrix cores: q [N, H*D] bfloat16, pools as for
+    """Attention without bias or head mixing (``sink`` / ``gate`` / ``chunk`` / ``softcap`` / ``out_scale`` / ``out`` as for ``attn_window``) in one sweep on the matrix cores: q [N, H*D], pools as for
     ``attn_window`` (column ranges of wider rows allowed); ``v_cache`` may be the first Dv columns of ``k_cache`` itself (one key
     head whose rows hold the values: the latent pool).  Returns [N, H*Dv].  Sizes as ``attn_sweep_tile_rows`` accepts them."""
     _dev(q)
@@ -366,8 +366,11 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
     out = _attn_out(out, n, H * Dv, torch.float32 if float_out else q.dtype, q.device, "attn_sweep")
     # few tiles with many keys (decoding): share each tile's keys out over workgroups until the chip is full
     groups = tiles.shape[0] * G * -(-(H // G) // 32)
+    # float tiles take 16 times as long per key, so the chip has to be fuller before their keys are left whole: 3 x 1000 tokens, 8 heads over 2 (648 groups)
+    # 160 us shared out, 218 us in 128-row tiles; 1 x 4096 (1024 groups) 916 and 805 us
+    below = SWEEP_SPLIT_BELOW_GROUPS if q.dtype == torch.bfloat16 else 2 * SWEEP_SPLIT_BELOW_GROUPS
     splits, scratch = 1, None
-    if groups >= SWEEP_SPLIT_BELOW_GROUPS and n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B:
+    if groups >= below and n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B:
         # long portions: tiles of up to 128 (query, head) rows, every wavefront keeps its rows to itself
         wide = int(N.layers().jl_attn_sweep_wide_tile_rows(_code(q.dtype), H, G, Gv, D, Dv, k_cache.stride(0), v_cache.stride(0),
                                                            int(v_cache.data_ptr() == k_cache.data_ptr())))
@@ -375,7 +378,7 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
             # what starts last should be short (4 x 2048 tokens, 16 heads of 128 over 4 key heads: 175 -> 137 us).  The 32-row kernel keeps the
             # requests' order, in which neighbours share keys (over a latent of 512 the sorted order was 3 % slower)
             tq, tiles = wide, batch.tiles(wide, longest_first=True)
-    elif groups < SWEEP_SPLIT_BELOW_GROUPS:
+    elif groups < below:
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
         splits = max(1, min(-(-reach // 128), SWEEP_SPLIT_WORKGROUPS // groups, 64))
         if splits > 1:
@@ -754,7 +757,7 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
     n, W, dt = qf.shape[0], R + rd, qf.dtype
     per_head = gate is not None
     up = lambda o, c0, c1, h0, h1: (o.view(n, h1 - h0, c1 - c0).transpose(0, 1), w_uv[h0:h1] if c1 - c0 == R else w_uv[h0:h1, c0:c1].contiguous())
-    if attn_sweep_tile_rows(dt, H, 1, W, R, pool, pool[:, :R]):                    # bfloat16, latents in multiples of 32 up to 512
+    if attn_sweep_tile_rows(dt, H, 1, W, R, pool, pool[:, :R]):                    # latents in multiples of 32 up to 512 (float: 128)
         o = attn_sweep(qf, pool, pool[:, :R], batch, H, 1, W, R, scale, window, sink=sink, gate=gate, gate_per_head=per_head)
         return torch.bmm(*up(o, 0, R, 0, H))
     fits = lambda h, c: int(N.layers().jl_attn_tile_rows(_code(dt), h, 1, W, c, pool.stride(0), pool.stride(0))) > 0
@@ -784,19 +787,21 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
 # chip is not full (a tile walks its keys in order; the 32-row kernel shares few tiles' keys out).  A step wholly on built keys has fewer launches (bmm, packing, bmm
 # and head order go: 95 -> 55 us of host time for small steps), a step that mixes the forms has more.
 LATENT_RATES = dict(narrow=330e12, wide=105e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
+# in float: the matrix form of the one-sweep kernel (narrow) or float multiply-adds (wide) over the latent
+LATENT_RATES_FLOAT = dict(narrow=60e12, wide=1.5e12, built=60e12, product=90e12, key64=130e-9, key32=180e-9, launches=-35e-6, both=80e-6)
 LATENT_BUILT_BYTES = 2 << 30          # keys and values built at a time
 LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth building keys for fewer
 
 
-def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, window: int) -> List[int]:
+def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, window: int, dtype: torch.dtype = torch.bfloat16) -> List[int]:
     """The requests of a step whose keys and values are better built per head.  Over the latent a visible pair costs 2 H (2 R + rd) operations, over
     built keys 2 H (D + rd + Dv) — a third of it at R = 512, D = Dv = 128, rd = 64 — but every key is built first, 2 H R (D + Dv): worth it from some
     hundred new tokens per request on, never for a decoded token.  Measured, us over the latent / built: 4 x 1024 tokens at 16 heads x 128, R 512: 1044 / 110,
     one request of 128 behind 4000: 303 / 288, of 32: 132 / 259; 8 heads x 64, R 128, 4 x 256 behind 1500: 132 / 92, 1 x 256 behind 4000: 116 / 163."""
-    key = ("built", H, D, R, rd, Dv, window)
+    key = ("built", H, D, R, rd, Dv, window, dtype)
     chosen = batch._tiles.get(key)
     if chosen is None:
-        r = LATENT_RATES
+        r = LATENT_RATES if dtype == torch.bfloat16 else LATENT_RATES_FLOAT
         over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["wide"])
         pair, one = 2.0 * H * (D + rd + Dv) / r["built"], 2.0 * H * R * (D + Dv) / r["product"]
         step = r["key64"] if D + rd <= 128 else r["key32"]
@@ -830,8 +835,8 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
     n, dt = q.shape[0], q.dtype
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] == H * (D + rd) and n == batch.N, "latent_attention: q [N, H*(D + rd)] of the batch")
     built: List[int] = []
-    if dt == torch.bfloat16 and D % 8 == 0 and rd % 8 == 0 and D + rd <= 256 and Dv % 32 == 0 and Dv <= 128 and q.stride(0) % 4 == 0 and q.data_ptr() % 8 == 0:
-        built = _latent_built_requests(batch, H, D, R, rd, Dv, window)
+    if D % 8 == 0 and rd % 8 == 0 and D + rd <= 256 and Dv % 32 == 0 and Dv <= 128 and q.stride(0) % 4 == 0 and q.data_ptr() % (2 * 4 if dt == torch.bfloat16 else 16) == 0 and R % 4 == 0:
+        built = _latent_built_requests(batch, H, D, R, rd, Dv, window, dt)
 
     def over_latent(q, batch, gate):
         m = q.shape[0]
@@ -855,12 +860,12 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
     tl = _angle_tables(rot_dims, cos, sin, batch, "latent_attention")
     st = _stream(q.device)
     N.check_layers(N.layers().jl_rotate_heads(_ptr(q), _code(dt), n, q.stride(0), H, D, rd, rot_dims, _ptr(batch.pos), _ptr(cos), _ptr(sin), tl, int(pairing), st), "jl_rotate_heads")
-    tq = int(N.layers().jl_attn_expanded_tile_rows())
+    tq, es = int(N.layers().jl_attn_expanded_tile_rows()), q.element_size()
     tiles = batch.tiles(tq, longest_first=True, requests=built)
-    a = N.AttnArgs(q=q.data_ptr(), k_cache=kv.data_ptr(), v_cache=kv.data_ptr() + 2 * H * D, out=out.data_ptr(), tiles=tiles.data_ptr(), n_tiles=tiles.shape[0], H=H, G=H, D=D + rd,
+    a = N.AttnArgs(q=q.data_ptr(), k_cache=kv.data_ptr(), v_cache=kv.data_ptr() + es * H * D, out=out.data_ptr(), tiles=tiles.data_ptr(), n_tiles=tiles.shape[0], H=H, G=H, D=D + rd,
                    Dv=Dv, window=int(window), TQ=tq, dtype=_code(dt), scale=float(scale), n_rows=n, k_ld=kv.shape[1], v_ld=kv.shape[1], Gv=H, out_dtype=N.JL_OUT_SAME,
                    sink=sink.data_ptr() if sink is not None else None, gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0,
-                   gate_heads=int(gate_per_head), out_scale=1.0, out_ld=H * Dv, key_base=base.data_ptr(), k_tail=lat.data_ptr() + 2 * R if rd else None, k_tail_ld=R + rd,
+                   gate_heads=int(gate_per_head), out_scale=1.0, out_ld=H * Dv, key_base=base.data_ptr(), k_tail=lat.data_ptr() + es * R if rd else None, k_tail_ld=R + rd,
                    q_ld=q.stride(0), k_tail_cols=rd)
     N.check_layers(N.layers().jl_attn_expanded(C.byref(a), st), "jl_attn_expanded")
     return out

@@ -266,7 +266,7 @@ class MikipelModel:
         proj = F.linear(h, w["w_in"])
         kp, vp, scale = cache.k[li], cache.v[li], float(m["scale"])
         q = LO.head_norm_append(proj, w["cols"], H, G, 1, D, Dv, None, None, eps, 0.0, 1, batch, kp, vp, rot_dims=dims, cos=cos, sin=sin)
-        if LO.attn_sweep_tile_rows(self.dtype, H, G, D, Dv, kp, vp) > 0:      # bfloat16, head sizes the one-sweep matrix-core kernel takes
+        if LO.attn_sweep_tile_rows(self.dtype, H, G, D, Dv, kp, vp) > 0:      # head sizes the one-sweep matrix-core kernels take
             return LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, scale, 0)
         return LO.attn_window(q, None, kp, vp, batch, H, G, D, Dv, scale, 0, 0, None, None, None)
 

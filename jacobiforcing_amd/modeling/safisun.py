@@ -320,7 +320,7 @@ class SafisunModel:
                               pairing=LO.ROT_NEIGHBOURS, batch=batch, cos=cos, sin=sin)
         kw = dict(sink=w["sink"], gate_per_head=True, chunk=int((m.get("mask") or {}).get("size", 0)), softcap=float(m.get("softcap") or 0.0), out_scale=scale, out=out)
         gate = proj[:, cols[3]:cols[3] + H]
-        if LO.attn_sweep_tile_rows(self.dtype, H, G, D, Dv, kp, vp) > 0:      # bfloat16, head sizes the one-sweep matrix-core kernel takes
+        if LO.attn_sweep_tile_rows(self.dtype, H, G, D, Dv, kp, vp) > 0:      # head sizes the one-sweep matrix-core kernels take
             return LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, float(m["scale"]), 0, gate=gate, **kw)
         return LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, float(m["scale"]), 0, 0, None, None, None, **kw)
 

@@ -32,17 +32,18 @@ def reference(q, k, v, starts, counts, pages, page, H, G, Gv, D, Dv, scale, wind
 
 
 # key and value widths at and beside the multiples of 64 (key rows in LDS) and 32 / 64 / 128 (value rows)
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("H,G,Gv,D,Dv,window,chunk,cap,page,pad", [
     (16, 4, 4, 128, 128, 0, 0, 0.0, 64, 0), (16, 16, 16, 64, 64, 0, 0, 0.0, 64, 0), (16, 2, 2, 8, 32, 0, 0, 0.0, 64, 0), (24, 4, 4, 72, 96, 100, 0, 0.0, 64, 0),
     (16, 4, 2, 136, 64, 0, 0, 0.0, 48, 0), (20, 20, 20, 192, 128, 65, 0, 0.0, 64, 0), (40, 1, 1, 200, 96, 0, 0, 0.0, 64, 4), (16, 2, 2, 256, 128, 0, 0, 0.0, 64, 0),
     (16, 4, 4, 128, 128, 0, 100, 5.0, 64, 0), (16, 1, 0, 160, 128, 0, 0, 0.0, 64, 0), (16, 1, 0, 96, 64, 63, 0, 0.0, 64, 4), (33, 1, 0, 256, 32, 0, 64, 2.0, 40, 0),
 ])
-def test_wide_tiles(H, G, Gv, D, Dv, window, chunk, cap, page, pad):
+def test_wide_tiles(dtype, H, G, Gv, D, Dv, window, chunk, cap, page, pad):
     """Unequal requests, two of them continuing inside a page; ``pad``: rows of the pools start at 8-byte borders only; Gv 0: the values are the key
     rows' first columns; pools hold NaN wherever nothing was written."""
     from jacobiforcing_amd import layer_ops as LO
-    dev, dt = "cuda", torch.bfloat16
-    starts, counts = [0, 37, 1, 0], [-(-16384 // H), 131, 64, 33]
+    dev, dt = "cuda", getattr(torch, dtype)
+    starts, counts = [0, 37, 1, 0], [-(-16384 * (1 if dtype == "bfloat16" else 2) // H), 131, 64, 33]
     g = torch.Generator(device=dev).manual_seed(D + H)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dt)
     need = [-(-(s + n) // page) for s, n in zip(starts, counts)]
@@ -66,19 +67,49 @@ def test_wide_tiles(H, G, Gv, D, Dv, window, chunk, cap, page, pad):
     want = reference(q, k, v, starts, counts, pages, page, H, G, Gv or 1, D, Dv, D ** -0.5, window, chunk, cap, sink)
     want = (want.view(-1, H, Dv) * torch.sigmoid(gate.double()).unsqueeze(-1)).view_as(want)
     assert torch.isfinite(got).all()
-    # weights are rounded to bfloat16 (2 ** -9 relative, independently): a sum of them is off by less than that of its largest terms
+    # weights are rounded to bfloat16 (2 ** -9 relative, independently): a sum of them is off by less than that of its largest terms; in float a score of
+    # size 5 (sums of D products) is 2 ** -21 off and moves its weight by as much
+    err, tol = (got.double() - want).abs(), 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -20
+    assert err.max() < 2 * tol * want.abs().max() and err.norm() < tol * want.norm()
+
+
+@pytest.mark.parametrize("H,G,Gv,D,Dv,window,chunk,cap,page", [
+    (8, 2, 2, 128, 128, 0, 0, 0.0, 64), (3, 3, 3, 20, 32, 50, 0, 0.0, 32), (40, 1, 0, 160, 128, 0, 0, 0.0, 64), (12, 4, 2, 252, 96, 0, 128, 3.0, 48), (6, 1, 0, 68, 64, 300, 0, 0.0, 64),
+])
+def test_float_tiles_with_shared_out_keys(H, G, Gv, D, Dv, window, chunk, cap, page):
+    """Decoded tokens and short portions in float: 32-row tiles whose keys several workgroups share."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt = "cuda", torch.float32
+    starts, counts = [700, 0, 333, 1023, 64], [1, 1, 5, 1, 33]
+    g = torch.Generator(device=dev).manual_seed(D + H)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    need = [-(-(s + n) // page) for s, n in zip(starts, counts)]
+    ids = torch.randperm(sum(need) + 3, generator=torch.Generator().manual_seed(H)).tolist()
+    pages = [[ids.pop() for _ in range(n)] for n in need]
+    k = torch.full(((sum(need) + 3) * page, G * D), float("nan"), device=dev)
+    v = k[:, :Dv] if Gv == 0 else torch.full((k.shape[0], Gv * Dv), float("nan"), device=dev)
+    for s, n, tab in zip(starts, counts, pages):
+        tok = torch.tensor([tab[j // page] * page + j % page for j in range(s + n)], device=dev)
+        k[tok] = rnd(s + n, G * D)
+        if Gv:
+            v[tok] = rnd(s + n, Gv * Dv)
+    q, sink, gate = rnd(sum(counts), H * D), rnd(H), rnd(sum(counts), H * Dv)
+    batch = LO.RaggedBatch.build(counts, starts, list(range(5)), pages, page, dev)
+    got = LO.attn_sweep(q, k, v, batch, H, G, D, Dv, D ** -0.5, window, value_heads=Gv, sink=sink, gate=gate, chunk=chunk, softcap=cap, out_scale=0.7)
+    want = reference(q, k, v, starts, counts, pages, page, H, G, Gv or 1, D, Dv, D ** -0.5, window, chunk, cap, sink) * torch.sigmoid(gate.double()) * 0.7
     err = (got.double() - want).abs()
-    assert err.max() < 2.0 ** -7 * want.abs().max() and err.norm() < 2.0 ** -8 * want.norm()
+    assert torch.isfinite(got).all() and err.max() < 2.0 ** -19 * want.abs().max() and err.norm() < 2.0 ** -20 * want.norm()
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("H,D,R,rd,Dv,rot,pairing,window,gate,built", [
     (5, 64, 128, 32, 64, 32, "ROT_NEIGHBOURS", 0, None, (0, 1, 2, 3)), (16, 128, 512, 64, 128, 64, "ROT_HALVES", 100, "full", (0, 1, 2, 3)), (3, 8, 64, 8, 32, 4, "ROT_NEIGHBOURS", 1, "head", (1, 3)),
     (2, 248, 32, 8, 96, 8, "ROT_HALVES", 0, "full", (0,)), (4, 64, 96, 0, 128, 0, "ROT_HALVES", 37, "head", (0, 1, 3)), (33, 120, 40, 72, 64, 72, "ROT_NEIGHBOURS", 300, None, (1, 2)),
 ])
-def test_latent_attention_with_built_keys(monkeypatch, H, D, R, rd, Dv, rot, pairing, window, gate, built):
+def test_latent_attention_with_built_keys(monkeypatch, dtype, H, D, R, rd, Dv, rot, pairing, window, gate, built):
     """Some or all requests of a step on keys and values built per head, the others over the latent; the last request brings one token."""
     from jacobiforcing_amd import layer_ops as LO
-    dev, dt, page = "cuda", torch.bfloat16, 32
+    dev, dt, page = "cuda", getattr(torch, dtype), 32
     monkeypatch.setattr(LO, "_latent_built_requests", lambda *a: list(built))
     starts, counts = [0, 45, 3, 200], [129, 300, 128, 1]
     g = torch.Generator(device=dev).manual_seed(H + R)
@@ -115,5 +146,5 @@ def test_latent_attention_with_built_keys(monkeypatch, H, D, R, rd, Dv, rot, pai
     got = LO.latent_attention(wide[:, :H * (D + rd)], pool, torch.cat([w_uk, w_uv]), w_uk.view(H, D, R), w_uv.view(H, Dv, R).transpose(1, 2).contiguous(), batch, H, D, R, rd, Dv, rot, cos, sin,
                               getattr(LO, pairing), scale, window, sink=sink, gate=gates, gate_per_head=gate == "head")
     # queries, keys, values, weights and the result are rounded to bfloat16 once each (2 ** -9 relative); a score of size 3 moves its weight by 1.2 %
-    err = (got.double() - want).abs()
-    assert torch.isfinite(got).all() and err.norm() < 2.0 ** -6 * want.norm() and err.max() < 2.0 ** -4 * want.abs().max()
+    err, tol = (got.double() - want).abs(), 2.0 ** -6 if dtype == "bfloat16" else 2.0 ** -19
+    assert torch.isfinite(got).all() and err.norm() < tol * want.norm() and err.max() < 4 * tol * want.abs().max()
