@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 128
+#define JL_VERSION 129
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -293,6 +293,24 @@ JL_API int jl_retention(const void *proj, int dtype, int64_t ld, int32_t q_col, 
 /* req [B, 4] int32 = {first chunk, chunks, pos0, slot}; chunk_len [chunks] int32; scratch [chunks, H, D, Dv] float as above. */
 JL_API int jl_retention_join(const int32_t *req, int32_t B, const int32_t *chunk_len, int32_t H, int32_t D, int32_t Dv,
                              const float *decay, float *state, float *scratch, void *stream);
+
+/* The same for long portions on the matrix cores: every request's portion cut into pieces of piece_tokens (a multiple of 64) tokens, the last of a request
+ * what is left, that run side by side (own contributions to the state, the state each starts from, outputs).  piece_rec [pieces, 4] int32 {row0, count, slot,
+ * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}; pos [N] int32 position of every row; scratch [pieces, H, D, Dv] float.
+ * Sizes as jl_retention_pieces_ok takes them; ld and columns in multiples of four, rows and tables at the borders of four elements. */
+typedef struct jl_retention_pieces {
+    const void *proj;
+    const int32_t *piece_rec, *req, *pos;
+    const float *cos_t, *sin_t, *decay;
+    float *state, *scratch;
+    void *out;
+    int64_t ld, table_len;
+    int32_t q_col, k_col, v_col, g_col, dtype, B, pieces, piece_tokens, H, D, Dv, rot_dims;
+    float eps;
+    int32_t reserved;
+} jl_retention_pieces;
+JL_API int jl_retention_pieces_ok(int dtype, int32_t D, int32_t Dv, int32_t rot_dims);
+JL_API int jl_retention_pieces_run(const jl_retention_pieces *a, void *stream);
 
 /* Gated delta rule over the ragged batch, state carried in float.  Per head h (key head c = h / (H / G)) and token t:
  *   q, k = unit vectors (x / sqrt(sum x^2 + unit_eps)) of the head's D query / key values, q also times q_scale;

@@ -1,6 +1,7 @@
 // jl_retention.hip — retention: linear attention with a fixed decay per head and a float state per (request slot, head),
 // scanned token by token for prompt portions and decoded tokens alike.
 #include "jl_common.h"
+#include <type_traits>
 
 // One workgroup per (request, head); thread j owns column j of the state S [D, Dv] in registers.  Tokens are taken TT at a
 // time: the rotated queries / keys of a group go through LDS, each thread runs the recurrence for its column, the per-token
@@ -163,4 +164,310 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
     const unsigned gy = (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64);
     retention_join_kernel<<<dim3((unsigned)(B * H), gy), 256, 0, (hipStream_t)stream>>>(req, chunk_len, H, ddv, decay, state, scratch);
     return jl_check_launch("retention_join_kernel");
+}
+
+// ---- long portions on the float matrix instructions: pieces side by side, 64 tokens at a time -------------------------------------------------
+// With g = the head's decay, a group of n tokens is three products on the state S the group starts from:
+//   o_i = g^(i+1) S^T q_i + sum_{j <= i} g^(i-j) (q_i . k_j) v_j,          S <- g^n S + sum_j g^(n-1-j) k_j v_j^T.
+// A portion is cut into pieces (whole groups, except the last) that run side by side: every piece's own contribution to the state (RM_LOCAL, not for a
+// request's last piece), the state every piece starts from (retention_pieces_join_kernel), outputs (RM_OUT; the last piece leaves the final state in its slot).
+// A workgroup owns one head of one piece; wavefront w holds columns 32 w .. + 31 of S [D, Dv] in accumulators.  v_mfma_f32_32x32x2_f32: lane l supplies
+// row (A) or column (B) l % 32 at depth l / 32, accumulator r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 — so the state's accumulators are the B operand of
+// S^T q as they are (register r against the query's element of the same row), and never cross LDS.  Everything is a 32-bit number from the projection on, as in
+// the scan: no operand is split or rounded.  q, k (rotated, scaled), v and the pairs' weights of the group lie in LDS as floats; the next group's rows
+// are on their way meanwhile.
+// What bounds it: 368 matrix instructions of 64 cycles per wavefront and group of 64 tokens at 128 x 128, and the phases of a group at one workgroup per CU.
+// Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 261 us, one prompt of 128
+// 985 -> 70, 8 x 8 tokens 84 -> 39; float, 1021 + 851 + 681 tokens: 1091 -> 156.
+constexpr int RM_T = 64, RM_OUT = 0, RM_LOCAL = 1;
+typedef float rm_f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ rm_f32x16 rm_mma(float a, float b, rm_f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+static constexpr size_t rm_lds_bytes(int DP, bool out) { return ((size_t)RM_T * DP * (out ? 2 : 1) + RM_T * 128 + (out ? RM_T * RM_T + 4 * RM_T : 0) + 2 * RM_T) * 4; }
+
+template <typename T, int DP, int MODE>
+__global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_pieces a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    constexpr bool OUT = MODE == RM_OUT;
+    constexpr int U = DP / 4, KPF = RM_T * U / 256, VPF = RM_T * 32 / 256, NS = DP / 32;
+    const int piece = blockIdx.x, h = blockIdx.y, H = a.H, D = a.D, Dv = a.Dv;
+    const int row0 = a.piece_rec[4 * piece], cnt = a.piece_rec[4 * piece + 1], slot = a.piece_rec[4 * piece + 2], last = a.piece_rec[4 * piece + 3];
+    if (cnt <= 0 || (!OUT && last)) return;
+    float4 *Ks = (float4 *)smem, *Qs = Ks + RM_T * U;               // [64][D], 16-byte units permuted by the row
+    float *Vs = (float *)(OUT ? Qs + RM_T * U : Qs);                // [64][128]
+    float4 *Ps = (float4 *)(Vs + RM_T * 128);                       // [64][64] decayed q . k of the pairs, permuted likewise
+    float *red = (float *)Ps + (OUT ? RM_T * RM_T : 0);             // [64][4] sums of squares
+    float *gp = red + (OUT ? 4 * RM_T : 0);                         // g^0 .. g^64
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, nw = (Dv + 31) / 32, col = 32 * wave + l32;
+    const float gamma = a.decay[h], kscale = 1.0f / sqrtf((float)D);
+    if (wave == 0) {                                                // powers by doubling, which doubles a rounding error too: in 64 bits.  Lane l holds g^(l+1)
+        double p = gamma;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double y = __shfl_up(p, off, 64);
+            if (lane >= off) p *= y;
+        }
+        gp[lane + 1] = (float)p;
+        if (lane == 0) gp[0] = 1.0f;
+    }
+    auto at = [](int row, int u) { return u ^ (row & 15); };        // U is a multiple of 16
+    const T *src = (const T *)a.proj + (int64_t)row0 * a.ld;
+    const int half = a.rot_dims >> 1, hu = half / 4;
+
+    rm_f32x16 S[NS];
+    float *sp = a.scratch + ((int64_t)piece * H + h) * D * Dv;
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int d = 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
+            S[t][r] = (OUT && d < D && col < Dv) ? sp[(int64_t)d * Dv + col] : 0.f;
+        }
+    // a group's rows on their way: four elements of a row per unit
+    typedef typename std::conditional<sizeof(T) == 2, uint2, float4>::type unit_t;
+    unit_t rq[KPF], rk[KPF], rv[VPF];
+    auto to_float = [](const unit_t &w) -> float4 {
+        float v[4];
+        ld4_f((const T *)&w, v);
+        return make_float4(v[0], v[1], v[2], v[3]);
+    };
+    auto fetch = [&](int t0) {
+        const int nt = cnt - t0;
+        const T *base = src + (int64_t)t0 * a.ld;
+        const unit_t zero = {};
+#pragma unroll
+        for (int it = 0; it < KPF; ++it) {
+            const int e = tid + it * 256, tt = e / U, u = e % U;
+            rk[it] = rq[it] = zero;
+            if (tt < nt && 4 * u < D) {
+                const T *row = base + (int64_t)tt * a.ld + h * D + 4 * u;
+                rk[it] = *(const unit_t *)(row + a.k_col);
+                if (OUT) rq[it] = *(const unit_t *)(row + a.q_col);
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < VPF; ++it) {
+            const int e = tid + it * 256, tt = e >> 5, u = e & 31;
+            rv[it] = zero;
+            if (tt < nt && 4 * u < Dv) rv[it] = *(const unit_t *)(base + (int64_t)tt * a.ld + a.v_col + h * Dv + 4 * u);
+        }
+    };
+    fetch(0);
+    for (int t0 = 0; t0 < cnt; t0 += RM_T) {
+        const int nt = cnt - t0 < RM_T ? cnt - t0 : RM_T;
+        __syncthreads();                                            // the group before has been read
+#pragma unroll
+        for (int it = 0; it < KPF; ++it) {
+            const int e = tid + it * 256, tt = e / U, u = e % U;
+            const float4 k = to_float(rk[it]);
+            Ks[tt * U + at(tt, u)] = make_float4(k.x * kscale, k.y * kscale, k.z * kscale, k.w * kscale);
+            if (OUT) Qs[tt * U + at(tt, u)] = to_float(rq[it]);
+        }
+#pragma unroll
+        for (int it = 0; it < VPF; ++it) {
+            const int e = tid + it * 256;
+            ((float4 *)Vs)[e] = to_float(rv[it]);                   // rows of 128 columns, those beyond Dv and tokens beyond the portion zero
+        }
+        __syncthreads();
+        if (t0 + RM_T < cnt) fetch(t0 + RM_T);                      // in flight while this group is multiplied
+        for (int e = tid; e < nt * hu; e += 256) {                  // rotation in place: units u and u + half / 4 of a row
+            const int tt = e / hu, u = e - tt * hu;
+            int64_t p = a.pos[row0 + t0 + tt];
+            if (p >= a.table_len) p = a.table_len - 1;
+            const float4 c = *(const float4 *)(a.cos_t + p * half + 4 * u), s = *(const float4 *)(a.sin_t + p * half + 4 * u);
+            auto turn = [&](float4 *rows) {
+                float4 *x = rows + tt * U + at(tt, u), *y = rows + tt * U + at(tt, u + hu);
+                const float4 v = *x, w = *y;
+                *x = make_float4(v.x * c.x - w.x * s.x, v.y * c.y - w.y * s.y, v.z * c.z - w.z * s.z, v.w * c.w - w.w * s.w);
+                *y = make_float4(w.x * c.x + v.x * s.x, w.y * c.y + v.y * s.y, w.z * c.z + v.z * s.z, w.w * c.w + v.w * s.w);
+            };
+            turn(Ks);
+            if (OUT) turn(Qs);
+        }
+        __syncthreads();
+        if (OUT) {
+            for (int part = wave; part < 3; part += 4) {            // quadrants (queries, keys) of the pairs: (0, 0), (1, 0), (1, 1)
+                const int qi = part > 0, qj = part > 1;
+                rm_f32x16 s;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = 0.f;
+                const int ki = 32 * qj + l32, ii = 32 * qi + l32;
+#pragma unroll 4
+                for (int x = 0; x < U / 2; ++x) {
+                    const float4 k = Ks[ki * U + at(ki, 2 * x + hi)], q = Qs[ii * U + at(ii, 2 * x + hi)];
+                    s = rm_mma(k.x, q.x, s);
+                    s = rm_mma(k.y, q.y, s);
+                    s = rm_mma(k.z, q.z, s);
+                    s = rm_mma(k.w, q.w, s);
+                }
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int j0 = 32 * qj + 8 * g + 4 * hi;
+                    float v[4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[x] = j0 + x <= ii ? s[4 * g + x] * gp[ii - j0 - x > 0 ? ii - j0 - x : 0] : 0.f;
+                    Ps[ii * 16 + at(ii, j0 >> 2)] = make_float4(v[0], v[1], v[2], v[3]);
+                }
+            }
+            __syncthreads();
+            rm_f32x16 o[2];
+            if (wave < nw) {
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[rt][r] = 0.f;
+                }
+#pragma unroll
+                for (int x = 0; x < U / 2; ++x) {
+                    if (x % 2 == 0) __builtin_amdgcn_sched_barrier(0);      // all operands at once would not fit the registers
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt) {
+                        const int i = 32 * rt + l32;
+                        const float4 q = Qs[i * U + at(i, 2 * x + hi)];
+                        o[rt] = rm_mma(q.x, S[x >> 2][4 * (x & 3)], o[rt]);
+                        o[rt] = rm_mma(q.y, S[x >> 2][4 * (x & 3) + 1], o[rt]);
+                        o[rt] = rm_mma(q.z, S[x >> 2][4 * (x & 3) + 2], o[rt]);
+                        o[rt] = rm_mma(q.w, S[x >> 2][4 * (x & 3) + 3], o[rt]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[rt][r] *= gp[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3) + 1];
+                auto pairs = [&](int x, int first) {                // eight keys; no key of the second half is visible to the first half's queries
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = Vs[(8 * x + 4 * hi + i) * 128 + col];
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt) {
+                        if (rt < first) continue;
+                        const int i = 32 * rt + l32;
+                        const float4 p = Ps[i * 16 + at(i, 2 * x + hi)];
+                        o[rt] = rm_mma(p.x, v[0], o[rt]);
+                        o[rt] = rm_mma(p.y, v[1], o[rt]);
+                        o[rt] = rm_mma(p.z, v[2], o[rt]);
+                        o[rt] = rm_mma(p.w, v[3], o[rt]);
+                    }
+                };
+#pragma unroll 2
+                for (int x = 0; x < 4; ++x) pairs(x, 0);
+#pragma unroll 2
+                for (int x = 4; x < 8; ++x) pairs(x, 1);
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {                  // columns beyond Dv are zero
+                        if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                        float ss = o[rt][r] * o[rt][r];
+#pragma unroll
+                        for (int off = 16; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+                        if (l32 == 0) red[(32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3)) * 4 + wave] = ss;
+                    }
+            }
+            __syncthreads();
+            if (col < Dv) {
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                        const int i = 32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3);
+                        if (i >= nt) continue;
+                        float ss = 0.f;
+                        for (int w = 0; w < nw; ++w) ss += red[i * 4 + w];
+                        const float rn = 1.0f / sqrtf(ss / (float)Dv + a.eps), g = ld_f(src + (int64_t)(t0 + i) * a.ld + a.g_col + h * Dv + col);
+                        st_f((T *)a.out + (int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col, o[rt][r] * rn * (g / (1.0f + expf(-g))));
+                    }
+            }
+        }
+        if (wave < nw && (!OUT || last || t0 + RM_T < cnt)) {       // the state behind the group
+            const float gn = gp[nt];
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) S[t][r] *= gn;
+#pragma unroll 1
+            for (int x = 0; 8 * x < nt; ++x) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = 8 * x + 4 * hi + i;
+                    const float v = Vs[j * 128 + col] * gp[nt - 1 - j > 0 ? nt - 1 - j : 0];
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        const int d = 32 * t + l32;
+                        S[t] = rm_mma(((const float *)(Ks + j * U + at(j, d >> 2)))[d & 3], v, S[t]);
+                    }
+                }
+            }
+        }
+    }
+    float *dst = OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : sp;
+    if (col < Dv && (!OUT || last))
+#pragma unroll
+        for (int t = 0; t < NS; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int d = 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
+                if (d < D) dst[(int64_t)d * Dv + col] = S[t][r];
+            }
+}
+
+// The state every piece of a request starts from, in place of the piece's own contribution: S = the slot's state (zero at position 0), then for every piece but
+// the last S <- g^tokens S + contribution.  Every piece but the last of a request is `tokens` long.
+__global__ __launch_bounds__(256) void retention_pieces_join_kernel(jl_retention_pieces a) {
+    const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
+    const int p0 = a.req[4 * b], np = a.req[4 * b + 1], pos0 = a.req[4 * b + 2], slot = a.req[4 * b + 3];
+    const int64_t ddv = (int64_t)a.D * a.Dv;
+    double power = 1.0, g2 = a.decay[h];
+    for (int n = a.piece_tokens; n; n >>= 1) {
+        if (n & 1) power *= g2;
+        g2 *= g2;
+    }
+    const float gn = (float)power;
+    const float *sp = a.state + ((int64_t)slot * a.H + h) * ddv;
+    for (int64_t e = (int64_t)blockIdx.y * 256 + threadIdx.x; e < ddv; e += (int64_t)gridDim.y * 256) {
+        float S = pos0 > 0 ? sp[e] : 0.f;
+        float next = np > 1 ? a.scratch[((int64_t)p0 * a.H + h) * ddv + e] : 0.f;
+        for (int p = p0; p < p0 + np; ++p) {
+            float *lp = a.scratch + ((int64_t)p * a.H + h) * ddv + e;
+            const float local = next;
+            next = p + 2 < p0 + np ? lp[(int64_t)a.H * ddv] : 0.f;  // the last piece has none
+            *lp = S;
+            S = gn * S + local;
+        }
+    }
+}
+
+extern "C" int jl_retention_pieces_ok(int dtype, int32_t D, int32_t Dv, int32_t rot_dims) {
+    return (dtype == JL_BF16 || dtype == JL_F32) && D > 0 && D <= 128 && D % 4 == 0 && Dv > 0 && Dv <= 128 && Dv % 4 == 0 && rot_dims >= 0 && rot_dims <= D && rot_dims % 8 == 0;
+}
+
+template <typename T, int DP> static int rm_launch(const jl_retention_pieces &a, hipStream_t st) {
+    auto local = retention_pieces_kernel<T, DP, RM_LOCAL>;
+    auto outs = retention_pieces_kernel<T, DP, RM_OUT>;
+    constexpr size_t l0 = rm_lds_bytes(DP, false), l1 = rm_lds_bytes(DP, true);
+    hipError_t e = hipFuncSetAttribute((const void *)local, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l0);
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void *)outs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l1);
+    if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_retention_pieces_run: cannot get %zu bytes of LDS: %s", l1, hipGetErrorString(e));
+    const dim3 grid((unsigned)a.pieces, (unsigned)a.H);
+    if (a.pieces > a.B) local<<<grid, 256, l0, st>>>(a);
+    const int64_t ddv = (int64_t)a.D * a.Dv;
+    retention_pieces_join_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64)), 256, 0, st>>>(a);
+    outs<<<grid, 256, l1, st>>>(a);
+    return jl_check_launch("retention_pieces_kernel");
+}
+
+extern "C" int jl_retention_pieces_run(const jl_retention_pieces *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_retention_pieces_run: null arguments");
+    const jl_retention_pieces &a = *ap;
+    if (a.B <= 0 || a.pieces <= 0) return JL_OK;
+    if (!a.proj || !a.decay || !a.state || !a.out || !a.scratch || !a.piece_rec || !a.req || !a.pos || (a.rot_dims && (!a.cos_t || !a.sin_t || a.table_len <= 0)))
+        return jl_fail(JL_E_INVALID, "jl_retention_pieces_run: null pointer");
+    if (!jl_retention_pieces_ok(a.dtype, a.D, a.Dv, a.rot_dims) || a.H <= 0 || a.H > 65535 || a.piece_tokens <= 0 || a.piece_tokens % RM_T || a.ld % 4 || (a.q_col | a.k_col | a.v_col) % 4 ||
+        ((uintptr_t)a.proj % (a.dtype == JL_BF16 ? 8 : 16)) || ((uintptr_t)a.cos_t % 16) || ((uintptr_t)a.sin_t % 16))
+        return jl_fail(JL_E_INVALID, "jl_retention_pieces_run: sizes, columns or alignment (ask jl_retention_pieces_ok)");
+    hipStream_t st = (hipStream_t)stream;
+    if (a.D <= 64) JL_DISPATCH(a.dtype, return (rm_launch<T, 64>(a, st)));
+    JL_DISPATCH(a.dtype, return (rm_launch<T, 128>(a, st)));
+    return JL_OK;
 }

@@ -21,6 +21,7 @@ ATTN_SPLIT_BELOW_TILES, ATTN_SPLIT_WORKGROUPS = 128, 512     # attention: split 
 ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-core attention kernel takes in one workgroup
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
+RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
 SCAN_PIECES_FROM, SCAN_WORKGROUPS = 32, 512     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
@@ -417,6 +418,19 @@ def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: Ragged
         N.check_layers(L.jl_retention(_ptr(proj), _code(proj.dtype), ld, cols[0], cols[1], cols[2], cols[3], _ptr(records), count, H, D, Dv,
                                       rot_dims, _ptr(cos), _ptr(sin), tl, _ptr(decay), float(eps), _ptr(where), _ptr(out), mode, st), what)
 
+    longest = max(batch.counts)
+    if (longest >= RETENTION_PIECES_FROM and L.jl_retention_pieces_ok(_code(proj.dtype), D, Dv, rot_dims) and ld % 4 == 0 and not any(c % 4 for c in cols[:3]) and
+            proj.data_ptr() % (8 if proj.dtype == torch.bfloat16 else 16) == 0 and (not rot_dims or (cos.data_ptr() | sin.data_ptr()) % 16 == 0)):
+        total = sum(batch.counts)
+        size = min(max(64, -(-total * H // RETENTION_WORKGROUPS) // 64 * 64), 1024)        # whole groups, as many pieces as the chip takes workgroups
+        rec, req = batch.pieces(size)
+        scratch = torch.empty((rec.shape[0], H, D, Dv), dtype=torch.float32, device=proj.device)
+        a = N.RetentionPieces(proj=proj.data_ptr(), piece_rec=rec.data_ptr(), req=req.data_ptr(), pos=batch.pos.data_ptr(), cos_t=cos.data_ptr() if rot_dims else None,
+                              sin_t=sin.data_ptr() if rot_dims else None, decay=decay.data_ptr(), state=state.data_ptr(), scratch=scratch.data_ptr(), out=out.data_ptr(), ld=ld,
+                              table_len=tl, q_col=cols[0], k_col=cols[1], v_col=cols[2], g_col=cols[3], dtype=_code(proj.dtype), B=batch.B, pieces=rec.shape[0], piece_tokens=size,
+                              H=H, D=D, Dv=Dv, rot_dims=rot_dims, eps=float(eps))
+        N.check_layers(L.jl_retention_pieces_run(C.byref(a), st), "jl_retention_pieces_run")
+        return out
     plan = batch.chunks(RETENTION_CHUNK)
     if plan is None:                                    # decoded tokens and short portions: one scan per request
         scan(batch.seq, batch.B, state, 0, "jl_retention")

@@ -1,0 +1,58 @@
+"""Retention of long portions in pieces on the matrix cores, at the edges of its groups of 64 tokens, tiles of 32 and pieces, against the recurrence in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("H,D,Dv,rot,workgroups,counts,starts", [
+    (3, 128, 128, 128, 256, [200, 64, 1], [0, 30, 5]), (2, 64, 32, 16, 64, [129, 65, 63, 300], [0, 0, 7, 1]), (4, 20, 100, 0, 8, [1000, 33], [3, 0]),
+    (1, 128, 4, 8, 2, [128, 127, 66], [9, 0, 0]), (2, 100, 128, 96, 1, [640], [0]), (1, 4, 68, 0, 256, [32], [1]),
+])
+def test_pieces(monkeypatch, dtype, H, D, Dv, rot, workgroups, counts, starts):
+    """Unequal portions (one token among them), slots of new requests hold NaN; decays of one, nearly none, zero and beyond one."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt, eps = "cuda", getattr(torch, dtype), 1e-5
+    monkeypatch.setattr(LO, "RETENTION_WORKGROUPS", workgroups)
+    g = torch.Generator(device=dev).manual_seed(D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    B, n = len(counts), sum(counts)
+    ld = 2 * H * D + 2 * H * Dv + 12
+    cols = (4, 4 + H * D, 4 + 2 * H * D, 4 + 2 * H * D + H * Dv)
+    proj = rnd(n, ld).to(dt)
+    decay = torch.tensor([0.97, 1.0, 0.0, 1.001][:H] if H > 1 else [1e-30], device=dev)
+    slots = list(range(1, B + 1))
+    state = rnd(B + 2, H, D, Dv)
+    for s, sl in zip(starts, slots):
+        if s == 0:
+            state[sl] = float("nan")
+    before = state.clone()
+    a = torch.arange(2048, dtype=torch.float32, device=dev).view(-1, 1) * torch.rand(max(rot, 2) // 2, generator=g, device=dev).view(1, -1)
+    cos, sin = (a.cos().contiguous(), a.sin().contiguous()) if rot else (None, None)
+    pages = [[b * 40 + i for i in range(40)] for b in range(B)]
+    batch = LO.RaggedBatch.build(counts, starts, slots, pages, 64, dev)
+    got = LO.retention(proj, cols, batch, H, D, Dv, rot, cos, sin, decay, eps, state)
+    assert any(isinstance(k, tuple) and k[0] == "pieces" for k in batch._tiles), "the form in pieces did not run"
+    p64, r0 = proj.double(), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        rows = p64[r0:r0 + c]
+        q, k = (rows[:, x:x + H * D].view(c, H, D) for x in cols[:2])
+        v, gate = (rows[:, x:x + H * Dv].view(c, H, Dv) for x in cols[2:])
+        if rot:
+            co, si = cos.double()[s:s + c].unsqueeze(1), sin.double()[s:s + c].unsqueeze(1)
+            turn = lambda x: torch.cat([x[..., :rot // 2] * co - x[..., rot // 2:rot] * si, x[..., rot // 2:rot] * co + x[..., :rot // 2] * si, x[..., rot:]], -1)
+            q, k = turn(q), turn(k)
+        S = before[slots[b]].double() if s else torch.zeros(H, D, Dv, dtype=torch.float64, device=dev)
+        o = []
+        for t in range(c):
+            S = decay.double().view(H, 1, 1) * S + (k[t] * D ** -0.5).unsqueeze(-1) * v[t].unsqueeze(-2)
+            o.append((q[t].unsqueeze(-2) @ S).squeeze(-2))
+        o = torch.stack(o)
+        o = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * torch.nn.functional.silu(gate)
+        r = got[r0:r0 + c].double().view(c, H, Dv)
+        # sums of up to c * D products of 32 bits; bfloat16 outputs round once more
+        assert (state[slots[b]].double() - S).norm() <= 2e-6 * S.norm(), (b, "state")
+        assert (r - o).norm() <= (2.0 ** -8 if dtype == "bfloat16" else 5e-6) * o.norm(), (b, "outputs")
+        r0 += c
+    assert torch.equal(state[0], before[0]) and torch.equal(state[B + 1], before[B + 1])
