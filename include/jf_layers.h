@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 129
+#define JL_VERSION 130
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -165,6 +165,17 @@ JL_API int jl_depth_mix_norm(const float *x_in, const jl_addend *addends, int32_
  * becomes the h of the request's last row of this step.  row_req [N] int32, seq [B, 4] as above. */
 JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_req, const int32_t *seq, float *tail, int64_t N, int32_t W,
                           void *out, int dtype, void *stream);
+
+/* out[n] = W x[n] + bias for up to JL_LINEAR_SMALL_ROWS rows: x [N, x_ld] of `dtype` and W [O, K] of `w_dtype` (x's, or float) with rows at 16-byte borders, bias [O] of `w_dtype` or
+ * null; sums in float.  One launch; W's rows are split into tiles of 16 for up to JL_LINEAR_ONE_TILE of them, into larger ones beyond.
+ * out rows out_ld elements apart: of `dtype`, float, or float after rounding to `dtype`. */
+#define JL_LINEAR_SMALL_ROWS 64
+#define JL_LINEAR_ONE_TILE 4096
+#define JL_LINEAR_SAME 0
+#define JL_LINEAR_FLOAT 1
+#define JL_LINEAR_ROUNDED_FLOAT 2
+JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
+                           int32_t out_mode, void *stream);
 
 /* z <- cap * tanh(z / cap) in place over `total` floats (soft cap of the logits). */
 JL_API int jl_softcap(float *z, int64_t total, float cap, void *stream);

@@ -1,0 +1,138 @@
+// jl_linear.hip — dense products of a few rows (decoding): out[n] = W x[n] (+ bias), W [O, K] read once.
+#include "jl_common.h"
+
+// What bounds such a product is W's bytes when W is large and the way there when it is small (a launch alone is 3 us, a trip to memory 2 us).  So a workgroup's NW wavefronts
+// share the depth of 16 * OT rows of W, every lane has LS_AHEAD pairs of 16-byte units of each of its rows of W and x (which comes from L2) on the way at once, straight into the
+// operands of 16 x 16 products — no LDS in between, no barrier before the end.  The order of the depths is free as long as both operands agree: lane l supplies units l / 16 and
+// 4 + l / 16 of each 128 bytes of row l % 16, so that a load takes 64 neighbouring bytes of every row.  The shares meet in LDS; a lane ends with four neighbouring columns of a row.
+//
+// The split (us of GPU time for 16 * OT rows of W and NW wavefronts, bfloat16, W from memory: 1 x 8 / 1 x 4 / 2 x 4 / 4 x 4):
+//   W 1024 x 1024, 32 rows:  5.7 / 5.6 /  6.7 /  9.3     W 5120 x 2048, 32 rows: 16.3 / 15.8 / 12.8 / 18.0     W 32000 x 1024, 32 rows: 29.4 / 30.5 / 23.6 / 21.5
+//   W 2048 x 4096, 16 rows: 11.3 / 11.4 / 16.2 / 25.8    W 5120 x 2048,  1 row:   8.7 /  9.0 /  9.2 / 13.4     W 32000 x 1024,  1 row:  17.7 / 14.5 / 16.3 / 17.4
+// As long as 16 rows of W per workgroup come to no more workgroups than the chip has CUs, that is the best; beyond, x is read again by every workgroup that a CU runs, and more rows
+// of W per workgroup pay (not for one row of x).  Library products of the same shapes take 8.2, 12.4, 24.0 / 14.9, 12.2, 18.7 us, and 11 us more of host time per call (19.5 / 8.6).
+// Rows beyond 16 cost x's reads: the caller's rule (layer_ops.linear) leaves products to the library where a CU would read more than 128 KB of x.
+constexpr int LS_AHEAD = 4;
+
+typedef float ls_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 ls_bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ ls_f32x4 ls_mma(const bf16_t *, uint4 a, uint4 b, ls_f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ls_bf16x8, a), __builtin_bit_cast(ls_bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ ls_f32x4 ls_mma(const float *, uint4 a, uint4 b, ls_f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint4 ls_unit(const bf16_t *p, const bf16_t *) { return *(const uint4 *)p; }
+__device__ __forceinline__ uint4 ls_unit(const float *p, const float *) { return *(const uint4 *)p; }
+__device__ __forceinline__ uint4 ls_unit(const bf16_t *p, const float *) {        // four 16-bit values for a float product
+    const uint2 v = *(const uint2 *)p;
+    return make_uint4(v.x << 16, v.x & 0xffff0000u, v.y << 16, v.y & 0xffff0000u);
+}
+
+template <typename TX, typename T, int NT, int OT, int NW>          // N <= 16 * NT rows of x, 16 * OT rows of W, NW wavefronts
+__global__ __launch_bounds__(64 * NW) void linear_small_kernel(const TX *__restrict__ x, int64_t x_ld, const T *__restrict__ w, const T *__restrict__ bias, void *__restrict__ out,
+                                                               int64_t out_ld, int N, int K, int O, int out_mode) {
+    __shared__ ls_f32x4 part[NW][OT][NT][64];
+    constexpr int UNIT = 16 / sizeof(T), LINE = 8 * UNIT;           // elements of a unit, of the 128 bytes that a step takes from every row
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4, o0 = blockIdx.x * 16 * OT;
+    const int k_lane = UNIT * g;
+    const T *wp[OT];
+    const TX *xp[NT];
+    ls_f32x4 acc[OT][NT];
+#pragma unroll
+    for (int o = 0; o < OT; ++o) {
+        const int r = o0 + 16 * o + r16;
+        wp[o] = w + (int64_t)(r < O ? r : O - 1) * K + k_lane;      // rows and columns that do not exist repeat the last one and are not stored
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[o][t] = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int n = 16 * t + r16;
+        xp[t] = x + (int64_t)(n < N ? n : N - 1) * x_ld + k_lane;
+    }
+    const int steps = (K + LINE - 1) / LINE, s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW;
+    for (int s = s0; s < s1; s += LS_AHEAD) {
+        uint4 wr[LS_AHEAD][2][OT], xr[LS_AHEAD][2][NT];
+#pragma unroll
+        for (int i = 0; i < LS_AHEAD; ++i)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const int k = (s + i) * LINE + 4 * UNIT * y;
+                const bool in = s + i < s1 && k + k_lane < K;
+#pragma unroll
+                for (int o = 0; o < OT; ++o) wr[i][y][o] = in ? *(const uint4 *)(wp[o] + k) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) xr[i][y][t] = in ? ls_unit(xp[t] + k, (const T *)nullptr) : make_uint4(0, 0, 0, 0);
+            }
+#pragma unroll
+        for (int i = 0; i < LS_AHEAD; ++i)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int o = 0; o < OT; ++o)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[o][t] = ls_mma((const T *)nullptr, wr[i][y][o], xr[i][y][t], acc[o][t]);
+    }
+#pragma unroll
+    for (int o = 0; o < OT; ++o)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) part[wave][o][t][lane] = acc[o][t];
+    __syncthreads();
+    for (int e = threadIdx.x; e < OT * NT * 64; e += 64 * NW) {
+        const int l = e & 63, t = (e >> 6) % NT, ot = (e >> 6) / NT, n = 16 * t + (l & 15), o = o0 + 16 * ot + 4 * (l >> 4);
+        if (n >= N || o >= O) continue;
+        ls_f32x4 s = part[0][ot][t][l];
+#pragma unroll
+        for (int i = 1; i < NW; ++i) s += part[i][ot][t][l];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (o + i >= O) continue;
+            float v = s[i];
+            if (bias) v += ld_f(bias + o + i);
+            if (out_mode == JL_LINEAR_FLOAT) ((float *)out)[n * out_ld + o + i] = v;
+            else if (out_mode == JL_LINEAR_ROUNDED_FLOAT) {
+                TX r;
+                st_f(&r, v);
+                ((float *)out)[n * out_ld + o + i] = ld_f(&r);
+            } else st_f((TX *)out + n * out_ld + o + i, v);
+        }
+    }
+}
+
+template <typename TX, typename T, int NT>
+static void linear_small_launch(const void *x, int64_t x_ld, const void *w, const void *bias, void *out, int64_t out_ld, int N, int K, int O, int out_mode, hipStream_t st) {
+#define LS_LAUNCH(OT, NW) linear_small_kernel<TX, T, NT, OT, NW><<<dim3((unsigned)((O + 16 * OT - 1) / (16 * OT))), 64 * NW, 0, st>>>((const TX *)x, x_ld, (const T *)w, (const T *)bias, out, \
+                                                                                                                                 out_ld, N, K, O, out_mode)
+    if (O <= JL_LINEAR_ONE_TILE) LS_LAUNCH(1, 8);
+    else if (N == 1) LS_LAUNCH(1, 4);
+    else if (O <= 4 * JL_LINEAR_ONE_TILE) LS_LAUNCH(2, 4);
+    else LS_LAUNCH(4, 4);
+#undef LS_LAUNCH
+}
+
+extern "C" int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
+                               int32_t out_mode, void *stream) {
+    if (N <= 0 || O <= 0) return JL_OK;
+    if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < O) return jl_fail(JL_E_INVALID, "jl_linear_small: null pointer or bad sizes");
+    if ((dtype != JL_BF16 && dtype != JL_F32) || (w_dtype != dtype && w_dtype != JL_F32)) return jl_fail(JL_E_INVALID, "jl_linear_small: W of x's type, or float");
+    const int x_unit = dtype == JL_BF16 ? 8 : 4, w_unit = w_dtype == JL_BF16 ? 8 : 4;
+    if (N > JL_LINEAR_SMALL_ROWS || K % w_unit || x_ld % x_unit || (((uintptr_t)x | (uintptr_t)w) & 15))
+        return jl_fail(JL_E_INVALID, "jl_linear_small: up to %d rows, rows of x and W at 16-byte borders", JL_LINEAR_SMALL_ROWS);
+    if (out_mode < JL_LINEAR_SAME || out_mode > JL_LINEAR_ROUNDED_FLOAT) return jl_fail(JL_E_INVALID, "jl_linear_small: unknown out_mode");
+#define LS_TYPES(TX, T)                                                                                                                        \
+    do {                                                                                                                                       \
+        if (N <= 16) linear_small_launch<TX, T, 1>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (hipStream_t)stream);                 \
+        else if (N <= 32) linear_small_launch<TX, T, 2>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (hipStream_t)stream);            \
+        else linear_small_launch<TX, T, 4>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (hipStream_t)stream);                         \
+    } while (0)
+    if (dtype == JL_F32) LS_TYPES(float, float);
+    else if (w_dtype == JL_F32) LS_TYPES(bf16_t, float);
+    else LS_TYPES(bf16_t, bf16_t);
+#undef LS_TYPES
+    return jl_check_launch("linear_small_kernel");
+}

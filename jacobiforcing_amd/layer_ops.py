@@ -193,6 +193,40 @@ class RaggedBatch:
         return t
 
 
+LINEAR_SMALL_ROWS, LINEAR_ONE_TILE = 64, 4096       # jl_linear_small: rows at most; W's rows up to which a workgroup takes 16 of them
+LINEAR_X_BYTES = 128 << 10           # ... and the bytes of x that a CU reads up to which it is the faster one
+_LINEAR_SAME, _LINEAR_FLOAT, _LINEAR_ROUNDED_FLOAT = 0, 1, 2
+
+
+def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
+    """Whether ``linear`` takes n rows of k values times [o, k] to the package's launch.  Every workgroup reads all rows of x: 16 of W's rows each up to LINEAR_ONE_TILE, then 32 and 64.
+    us of GPU time, own / library, at the line (bfloat16): 32 rows of 2048 by 2048 8.3 / 8.5, by 5120 12.8 / 12.4, 64 rows of 1024 by 4096 8.1 / 8.7; beyond it: 32 rows of 4096 by
+    2048 15.4 / 12.3, 64 rows of 2048 by 2048 12.1 / 9.2, 32 rows of 2048 by 32000 36.8 / 31.1.  float: 16 rows of 2048 by 2048 11.9 / 12.1; beyond, 32 rows 17.5 / 12.5."""
+    tile = 16 if o <= LINEAR_ONE_TILE or n == 1 else 32 if o <= 4 * LINEAR_ONE_TILE else 64
+    return 0 < n <= LINEAR_SMALL_ROWS and n * k * itemsize * -(-o // (tile * 256)) <= LINEAR_X_BYTES
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:
+    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launch for few rows (decoding, ``linear_small``), the library's product for more.
+    ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then counts as
+    float: give ``float_out`` True."""
+    _dev(x)
+    n, k = x.shape
+    o, size = w.shape[0], w.element_size()
+    _need(w.dtype == x.dtype or (w.dtype == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
+    if n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, size) and w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and \
+            (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous())):
+        out = torch.empty((n, o), dtype=x.dtype if float_out is None else torch.float32, device=x.device)
+        N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), _code(w.dtype), k, o, _ptr(bias), out.data_ptr(), o,
+                                                 _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT, _stream(x.device)), "jl_linear_small")
+        return out
+    if float_out and w.dtype != torch.float32:
+        y = torch.mm(x, w.t(), out_dtype=torch.float32)
+        return y if bias is None else y + bias
+    y = F.linear(x.to(w.dtype), w, bias)
+    return y if float_out is None else y.float()
+
+
 def embed_scale(embed: torch.Tensor, ids: torch.Tensor, scale: float, want_copy: bool,
                 out: Optional[torch.Tensor] = None, copy_dtype: torch.dtype = torch.float32) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """Rows ``ids`` of ``embed`` times ``scale`` as float [N, W] (written into ``out`` when given), and a second copy with ``want_copy``
@@ -602,8 +636,7 @@ def output_norm(x: torch.Tensor, addends: Sequence[Tuple[torch.Tensor, Optional[
 
 def product_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """a [N, K] . w [M, K]^T with a float result [N, M] (not rounded to the operands' dtype): a product that becomes the residual stream."""
-    _dev(a)
-    return torch.mm(a, w.t()) if a.dtype == torch.float32 else torch.mm(a, w.t(), out_dtype=torch.float32)
+    return linear(a, w, float_out=True)
 
 
 def sandwich_norm(x_in: torch.Tensor, y: Optional[torch.Tensor], w_post: Optional[torch.Tensor], eps: float, w_next: Optional[torch.Tensor] = None,

@@ -25,7 +25,6 @@ from pathlib import Path
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -243,7 +242,7 @@ class BamanexModel:
         H, G, D, Dv = (int(m[k]) for k in ("heads", "kv_heads", "dim", "vdim"))
         key = _rot_key(m)
         cos, sin = self._angles[key] if key[0] else (None, None)
-        proj = F.linear(h, w["w_in"], w["b_in"])
+        proj = LO.linear(h, w["w_in"], w["b_in"])
         kp, vp = cache.k[run], cache.v[run]
         q = LO.head_norm_append(proj, w["cols"][:3], H, G, 1, D, Dv, None, None, eps, 0.0, 1, batch, kp, vp, rot_dims=key[0], cos=cos, sin=sin)
         gate = proj[:, w["cols"][3]:w["cols"][3] + H]
@@ -252,7 +251,7 @@ class BamanexModel:
             a = LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, scale, window, sink=w["sink"], gate=gate, gate_per_head=True)
         else:
             a = LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, scale, window, 0, None, None, None, sink=w["sink"], gate_per_head=True)
-        return F.linear(a, w["w_o"], w["b_o"])
+        return LO.linear(a, w["w_o"], w["b_o"])
 
     # ---- feed-forward: the addends (tensor, channel scale) its result contributes to the residual sum -----------------------------------
     def _feed_forward(self, li: int, h: torch.Tensor, h_float: Optional[torch.Tensor] = None) -> list:
@@ -260,14 +259,14 @@ class BamanexModel:
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
             ff = int(f["ff"])
-            return [(F.linear(LO.gated_act(F.linear(h, w["w_gu"]), 0, ff, ff, LO.ACT_GELU_TANH), w["w_down"]), w["ls2"])]
+            return [(LO.linear(LO.gated_act(LO.linear(h, w["w_gu"]), 0, ff, ff, LO.ACT_GELU_TANH), w["w_down"]), w["ls2"])]
         unit = lambda c: (LO.ACT_CLAMPED_SWISH, float(c["limit"]), SWISH_ALPHA, UNIT_SHIFT)
-        out = [(LO.moe_experts(h, F.linear(h_float if h_float is not None else h.float(), w["router"]), None, int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
+        out = [(LO.moe_experts(h, LO.linear(h_float if h_float is not None else h, w["router"], float_out=True), None, int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
                                renorm_eps=ROUTER_RENORM_EPS, gated=unit(f["expert"])), w["ls2"])]
         if f.get("shared") is not None:                 # the token gate multiplies the activation: down() is linear, so the result is the gated output
             fs = int(f["shared"]["ff"])
-            z = F.linear(h, w["w_sh"])
-            out.append((F.linear(LO.gated_act(z, 0, fs, fs, *unit(f["shared"]), row_gate=z[:, 2 * fs]), w["w_sh_down"]), w["ls2"]))
+            z = LO.linear(h, w["w_sh"])
+            out.append((LO.linear(LO.gated_act(z, 0, fs, fs, *unit(f["shared"]), row_gate=z[:, 2 * fs]), w["w_sh_down"]), w["ls2"]))
         return out
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------
@@ -297,7 +296,7 @@ class BamanexModel:
         hf = LO.scaled_add_norms(x, pending, w.final_norm, None, 1.0, eps, dt)
         if logit_rows is not None:
             hf = hf.index_select(0, logit_rows)
-        return F.linear(hf, w.head).float() * cfg.logit_scale
+        return LO.linear(hf, w.head, float_out=False) * cfg.logit_scale
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):

@@ -22,7 +22,6 @@ from typing import Any, Dict, List, Optional
 
 import numpy as np
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -234,7 +233,7 @@ class LokizenModel:
     def _attention(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
         m, w, eps = self.cfg.layers[li]["mixer"], self.w.layers[li], self.cfg.norm_eps
         H, G, D, Dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         q = LO.qk_norm_append(proj, w["cols"][:3], H, G, D, Dv, w["q_norm"], w["k_norm"], eps, cache.k[run], cache.v[run], batch.kv_slot)
         gate = proj[:, w["cols"][3]:w["cols"][3] + H * Dv]
         mask = m.get("mask") or {}
@@ -248,7 +247,7 @@ class LokizenModel:
         rot = m.get("rot") or {}
         dims = int(rot.get("dims", 0))
         cos, sin = self._angles[(dims, float(rot.get("base", 10000.0)))] if dims else (None, None)
-        return LO.retention(F.linear(h, w["w_in"]), w["cols"], batch, m["heads"], m["dim"], m["vdim"], dims, cos, sin, w["decay"],
+        return LO.retention(LO.linear(h, w["w_in"]), w["cols"], batch, m["heads"], m["dim"], m["vdim"], dims, cos, sin, w["decay"],
                             self.cfg.norm_eps, cache.state[run])
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------
@@ -266,11 +265,11 @@ class LokizenModel:
             L, lw = cfg.layers[li], w.layers[li]
             h = LO.add_rmsnorm(x, pending, x0 if readd else None, lw["norm1"], eps, dt)
             a = self._attention(run, li, h, batch, cache) if L["type"] == "attention" else self._retention(run, li, h, batch, cache)
-            pending = F.linear(a, lw["w_o"])
+            pending = LO.linear(a, lw["w_o"])
             if L.get("mlp") is not None:
                 r = L["mlp"]["router"]
                 h2 = LO.add_rmsnorm(x, pending, None, lw["norm2"], eps, dt)
-                pending = LO.moe_experts(h2, F.linear(h2.float(), lw["router"]), lw["correction"], int(r["top"]), float(r["scale"]),
+                pending = LO.moe_experts(h2, LO.linear(h2, lw["router"], float_out=True), lw["correction"], int(r["top"]), float(r["scale"]),
                                          lw["w_up"], lw["w_down"])
             if trace is not None:
                 LO.add_rmsnorm(x, pending, None, None, eps, None)
@@ -279,7 +278,7 @@ class LokizenModel:
         hf = LO.add_rmsnorm(x, pending, None, w.final_norm, eps, dt)
         if logit_rows is not None:
             hf = hf.index_select(0, logit_rows)
-        return F.linear(hf, w.head).float()
+        return LO.linear(hf, w.head, float_out=False)
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):

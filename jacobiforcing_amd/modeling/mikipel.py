@@ -26,7 +26,6 @@ from pathlib import Path
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -263,7 +262,7 @@ class MikipelModel:
         m, w, eps = self.cfg.layers[li]["mixer"], self.w.layers[li], self.cfg.norm_eps
         H, G, D, Dv = (int(m[k]) for k in ("heads", "kv_heads", "dim", "vdim"))
         dims, cos, sin = self._tables(m)
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         kp, vp, scale = cache.k[li], cache.v[li], float(m["scale"])
         q = LO.head_norm_append(proj, w["cols"], H, G, 1, D, Dv, None, None, eps, 0.0, 1, batch, kp, vp, rot_dims=dims, cos=cos, sin=sin)
         if LO.attn_sweep_tile_rows(self.dtype, H, G, D, Dv, kp, vp) > 0:      # head sizes the one-sweep matrix-core kernels take
@@ -275,14 +274,14 @@ class MikipelModel:
         H, D, rd, Dv, R = (int(m[k]) for k in ("heads", "dim", "rot_dim", "vdim", "kv_rank"))
         dims, cos, sin = self._tables(m)
         pool, scale = cache.k[li], float(m["scale"])
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         LO.latent_prep(proj, 0, 0, w["kv_col"], R, rd, dims, None, w["dkv_norm"], eps, batch, cos, sin, pool, pairing=LO.ROT_NEIGHBOURS)
         return LO.latent_attention(proj[:, :H * (D + rd)], pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, dims, cos, sin, LO.ROT_NEIGHBOURS, scale, 0)
 
     def _delta(self, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]
         H, G, D, Dv, taps = _delta_sizes(m)
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         qkv = LO.short_conv(proj, 0, 2 * G * D + H * Dv, w["conv"], batch, cache.tails[li].get("conv"), LO.ACT_SILU)
         return LO.delta_rule(qkv, (0, G * D, 2 * G * D), proj, w["pcols"], w["a_log"], w["dt_bias"], w["out_norm"], batch, H, G, D, Dv, UNIT_EPS,
                              D ** -0.5, self.cfg.norm_eps, cache.state[li])
@@ -293,8 +292,8 @@ class MikipelModel:
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
             ff = int(f["ff"])
-            return [(F.linear(LO.gated_act(F.linear(h, w["w_up"]), 0, -1, ff, LO.ACT_GELU_ERF), w["w_down"]), None)]
-        logits = torch.addmm(w["router_b"], h_float, w["router"].t())
+            return [(LO.linear(LO.gated_act(LO.linear(h, w["w_up"]), 0, -1, ff, LO.ACT_GELU_ERF), w["w_down"]), None)]
+        logits = LO.linear(h_float, w["router"], w["router_b"])
         return [(LO.moe_experts(h, logits, None, int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="top_softmax", gated=(LO.ACT_SILU, 0.0, 1.0, 0.0)), None)]
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------
@@ -335,7 +334,7 @@ class MikipelModel:
                 h, hf = hs if both else (hs, hs)
                 shifted = LO.token_shift(hf, lw["shift"], batch, cache.tails[li]["shift"], dt)
             mixer = self._attention if L["type"] == "attention" else self._latent_attention if L["type"] == "latent_attention" else self._delta
-            pending = [(F.linear(mixer(li, shifted, batch, cache), lw["w_o"]), None)]
+            pending = [(LO.linear(mixer(li, shifted, batch, cache), lw["w_o"]), None)]
             if L.get("mlp") is not None:
                 pending += self._feed_forward(li, h, hf)
             if trace is not None:
@@ -344,7 +343,7 @@ class MikipelModel:
         hl = hand_on(nl, w.final_norm, dt)
         if logit_rows is not None:
             hl = hl.index_select(0, logit_rows)
-        z = F.linear(hl, w.embed).float()
+        z = LO.linear(hl, w.embed, float_out=False)
         return LO.softcap(z, cfg.logit_softcap) if cfg.logit_softcap > 0 else z
 
 

@@ -24,7 +24,6 @@ from pathlib import Path
 from typing import Any, Dict, List, Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -299,17 +298,17 @@ class SafisunModel:
 
     def _lightning(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
         w = self.w.layers[li]
-        return F.linear(self._linear_attention(self.cfg.layers[li]["mixer"], w, F.linear(h, w["w_in"]), run, batch, cache, 1.0, None), w["w_o"])
+        return LO.linear(self._linear_attention(self.cfg.layers[li]["mixer"], w, LO.linear(h, w["w_in"]), run, batch, cache, 1.0, None), w["w_o"])
 
     def _mamba2(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]
         H, G, N, Dv, taps, C_ = _mamba_sizes(m)
         inner = H * Dv
-        proj = F.linear(h, w["w_in"])                   # z | x | B | C | dt
+        proj = LO.linear(h, w["w_in"])                   # z | x | B | C | dt
         xbc = LO.short_conv(proj, inner, C_, w["conv"], batch, cache.tails[run].get("conv"), LO.ACT_SILU, bias=w["conv_b"], out_dtype=self.dtype)
         y = LO.linear_scan(xbc, (inner + G * N, inner, 0), batch, H, G, N, Dv, cache.state[run], dt=proj[:, inner + C_:inner + C_ + H], a_log=w["a_log"],
                            dt_bias=w["dt_bias"], skip=w["skip"])
-        return F.linear(LO.gated_norm(y, proj[:, :inner], w["out_norm"], self.cfg.norm_eps, LO.ACT_SILU, True, parts=int(m["norm_groups"])), w["w_o"])
+        return LO.linear(LO.gated_norm(y, proj[:, :inner], w["out_norm"], self.cfg.norm_eps, LO.ACT_SILU, True, parts=int(m["norm_groups"])), w["w_o"])
 
     def _attention(self, m, w, proj: torch.Tensor, run: int, batch: LO.RaggedBatch, cache: PagedStateCache, scale: float, out: torch.Tensor) -> torch.Tensor:
         """The parallel mixer's left side on its columns of the product, up to (not with) its output projection."""
@@ -328,13 +327,13 @@ class SafisunModel:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]
         H, _, _, Dv = _attention_sizes(m["left"])
         n, left, width = h.shape[0], H * Dv, w["w_o"].shape[1]
-        proj = F.linear(h, w["w_in"], w["b_in"])
+        proj = LO.linear(h, w["w_in"], w["b_in"])
         # both sides write their columns of one matrix, scaled; the output product over all of them is the weighted sum.  Rows start at
         # 16-byte borders; the right side starts where the left one ends
         both = torch.empty((n, width + (-width) % 8), dtype=h.dtype, device=h.device)[:, :width]
         self._attention(m["left"], w, proj, run, batch, cache, float(m["left_scale"]), both[:, :left])
         self._linear_attention(m["right"], w, proj, run, batch, cache, float(m["right_scale"]), both[:, left:])
-        return F.linear(both, w["w_o"])
+        return LO.linear(both, w["w_o"])
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------
     @torch.inference_mode()
@@ -373,7 +372,7 @@ class SafisunModel:
             if L.get("mlp") is not None:
                 ff = int(L["mlp"]["ff"])
                 h = norm(lw["norm2"])
-                pending = (F.linear(LO.gated_act(F.linear(h, lw["w_gu"]), 0, ff, ff, LO.ACT_SILU), lw["w_down"]), lw["norm2b"])
+                pending = (LO.linear(LO.gated_act(LO.linear(h, lw["w_gu"]), 0, ff, ff, LO.ACT_SILU), lw["w_down"]), lw["norm2b"])
             if trace is not None:
                 LO.sandwich_norm(x, *pending, eps)
                 pending = None
@@ -381,7 +380,7 @@ class SafisunModel:
         hl = norm(w.final_norm)
         if logit_rows is not None:
             hl = hl.index_select(0, logit_rows)
-        return F.linear(hl, w.head).float()
+        return LO.linear(hl, w.head, float_out=False)
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):

@@ -25,7 +25,6 @@ from pathlib import Path
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -240,31 +239,31 @@ class VoboraxModel:
         key = _rot_key(m) if windowed else (0, 0.0)
         cos, sin = self._angles[key] if key[0] else (None, None)
         pool = cache.k[src]
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         cq = LO.latent_prep(proj, 0, Rq, w["kv_col"], R, rd, key[0], w["dq_norm"], w["dkv_norm"], eps, batch, cos, sin, pool if src == li else None,
                             pairing=LO.ROT_NEIGHBOURS)
-        q = F.linear(cq, w["w_uq"])
+        q = LO.linear(cq, w["w_uq"])
         gate = proj[:, w["g_col"]:w["g_col"] + H] if windowed else None
         window = int((m.get("mask") or {}).get("size", 0)) if windowed else 0
         o = LO.latent_attention(q, pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, key[0], cos, sin, LO.ROT_NEIGHBOURS, float(m["scale"]), window, sink=w["sink"],
                                 gate=gate, gate_per_head=windowed)
-        return F.linear(o, w["w_o"])
+        return LO.linear(o, w["w_o"])
 
     # ---- feed-forward: the addends of its output, and the choices among which there are identity experts ----------------------------------
     def _feed_forward(self, li: int, h: torch.Tensor, x: torch.Tensor):
         """``h`` the stream in the products' dtype, ``x`` the stream itself (float): the router and the identity experts read that."""
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
-            z = F.linear(h, w["w_up"], w["b_up"])
-            return [(F.linear(LO.gated_act(z, 0, -1, z.shape[1], LO.ACT_GELU_TANH), w["w_down"], w["b_down"]), None)], None
+            z = LO.linear(h, w["w_up"], w["b_up"])
+            return [(LO.linear(LO.gated_act(z, 0, -1, z.shape[1], LO.ACT_GELU_TANH), w["w_down"], w["b_down"]), None)], None
         E, ident = _experts(f)
-        y = LO.moe_experts(h, F.linear(x, w["router"]), w["correction"], int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
+        y = LO.moe_experts(h, LO.linear(x, w["router"]), w["correction"], int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
                            renorm_eps=ROUTER_RENORM_EPS, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0), identity=ident)
         y, choices = (y[0], (y[1], y[2], E)) if ident else (y, None)
         out = [(y, None)]
         if f.get("shared") is not None:
             fs = int(f["shared"]["ff"])
-            out.append((F.linear(LO.gated_act(F.linear(h, w["w_sh"]), 0, fs, fs, LO.ACT_SILU), w["w_sh_down"]), None))
+            out.append((LO.linear(LO.gated_act(LO.linear(h, w["w_sh"]), 0, fs, fs, LO.ACT_SILU), w["w_sh_down"]), None))
         return out, choices
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------
@@ -291,7 +290,7 @@ class VoboraxModel:
             h = LO.output_norm(x, [], None, eps, LO.NORM_LAYER, w_next=w.final_norm, out_dtype=dt)
         if logit_rows is not None:
             h = h.index_select(0, logit_rows)
-        return F.linear(h, w.head).float()
+        return LO.linear(h, w.head, float_out=False)
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):

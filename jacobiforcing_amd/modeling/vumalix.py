@@ -22,7 +22,6 @@ from pathlib import Path
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from . import read_tensors
 from .. import layer_ops as LO
@@ -222,7 +221,7 @@ class VumalixModel:
         m, w, eps = self.cfg.layers[li]["mixer"], self.w.layers[li], self.cfg.norm_eps
         H, G, D, Dv = int(m["heads"]), int(m["kv_heads"]), int(m["dim"]), int(m["vdim"])
         qt = m.get("q_temp") or {}
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         kp, vp, scale = cache.k[li], cache.v[li], float(m["scale"])
         window = int((m.get("mask") or {}).get("size", 0))                                          # none in the design: plain causal
         sweep = LO.attn_sweep_tile_rows(self.dtype, 2 * H, 2 * G, D, Dv, kp, vp, G) > 0
@@ -247,9 +246,9 @@ class VumalixModel:
         dims = int(rot.get("dims", 0))
         cos, sin = self._angles[(dims, float(rot.get("base", 10000.0)))] if dims else (None, None)
         pool = cache.k[li]
-        proj = F.linear(h, w["w_in"])
+        proj = LO.linear(h, w["w_in"])
         cq = LO.latent_prep(proj, w["cols"][0], Rq, w["cols"][1], R, rd, dims, w["dq_norm"], w["dkv_norm"], eps, batch, cos, sin, pool)
-        q = F.linear(cq, w["w_uq"])
+        q = LO.linear(cq, w["w_uq"])
         return LO.latent_attention(q, pool, w["w_ukv"], w["w_uk"], w["w_uv"], batch, H, D, R, rd, Dv, dims, cos, sin, LO.ROT_HALVES, float(m["scale"]),
                                    int((m.get("mask") or {}).get("size", 0)), gate=proj[:, w["cols"][2]:w["cols"][2] + H * Dv])
 
@@ -267,11 +266,11 @@ class VumalixModel:
             lw = w.layers[li]
             h = LO.causal_conv(x, lw["canon"], batch, cache.tail[li])
             a = self._attention(li, h, batch, cache) if L["type"] == "attention" else self._latent_attention(li, h, batch, cache)
-            y = F.linear(a, lw["w_o"])
+            y = LO.linear(a, lw["w_o"])
             if L.get("mlp") is not None:
                 h2 = LO.norm_add(x, y, lw["norm1"], eps, dt)
-                act = LO.polynorm(F.linear(h2, lw["w_up"]), lw["act"], eps)
-                LO.norm_add(x, F.linear(act, lw["w_down"]), lw["norm2"], eps, None)
+                act = LO.polynorm(LO.linear(h2, lw["w_up"]), lw["act"], eps)
+                LO.norm_add(x, LO.linear(act, lw["w_down"]), lw["norm2"], eps, None)
             else:
                 LO.norm_add(x, y, lw["norm1"], eps, None)
             if trace is not None:
@@ -279,7 +278,7 @@ class VumalixModel:
         hf = LO.add_rmsnorm(x, None, None, w.final_norm, eps, dt)
         if logit_rows is not None:
             hf = hf.index_select(0, logit_rows)
-        return F.linear(hf, w.head).float()
+        return LO.linear(hf, w.head, float_out=False)
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):
