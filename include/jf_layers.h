@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 130
+#define JL_VERSION 131
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -338,6 +338,26 @@ JL_API int jl_delta_rule(const void *qkv, int qkv_dtype, int64_t qkv_ld, int32_t
                          int64_t ld, int32_t a_col, int32_t b_col, int32_t g_col, const float *A_log, const float *dt_bias, const float *norm_w,
                          const int32_t *seq, int32_t B, int64_t N, int32_t H, int32_t G, int32_t D, int32_t Dv, float unit_eps, float q_scale, float eps,
                          float *state, float *raw, void *out, void *stream);
+
+/* The same for long portions on the matrix cores, in chunks of 64 tokens (a request's last one of what is left).  chunk_rec [chunks, 4] int32 {row0, count, slot, 1 for a
+ * request's last chunk}; req [B, 4] int32 {first chunk, chunks, pos0, slot}; raw [N, H * Dv] float; scratch_floats floats of scratch for pass_heads heads at a time (a
+ * multiple of H / G; jl_delta_chunks_floats).  D and Dv as jl_delta_chunks_ok takes them; qkv_ld, q_col and k_col in multiples of four, qkv and scratch at 16-byte borders;
+ * at most INT32_MAX / 256 chunks times heads.  `out` null: raw is left to a following jl_delta_rule's norm and gate.  Requests not named in req are not touched. */
+typedef struct jl_delta_chunks {
+    const float *qkv;
+    const void *proj;
+    const float *A_log, *dt_bias, *norm_w;
+    const int32_t *chunk_rec, *req;
+    float *state, *raw, *scratch;
+    void *out;
+    int64_t qkv_ld, ld, N, scratch_floats;
+    int32_t q_col, k_col, v_col, a_col, b_col, g_col, dtype, B, chunks, H, G, D, Dv, pass_heads;
+    float unit_eps, q_scale, eps;
+    int32_t reserved;
+} jl_delta_chunks;
+JL_API int jl_delta_chunks_ok(int32_t D, int32_t Dv);
+JL_API int64_t jl_delta_chunks_floats(int32_t chunks, int32_t heads, int32_t H, int32_t G, int32_t D, int32_t Dv);
+JL_API int jl_delta_chunks_run(const jl_delta_chunks *a, void *stream);
 
 /* Linear recurrence with one decay per head (and token) over the ragged batch, state carried in float — lightning attention and the
  * state-space duality of Mamba-2 in one form.  Per head h (q / k head c = h / (H / G)) and token t:

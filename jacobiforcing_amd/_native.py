@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 130                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 131                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -262,6 +262,14 @@ class RetentionPieces(C.Structure):
     """jl_retention_pieces (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("proj", "piece_rec", "req", "pos", "cos_t", "sin_t", "decay", "state", "scratch", "out")] + [("ld", _i64), ("table_len", _i64)] + \
                [(k, _i32) for k in ("q_col", "k_col", "v_col", "g_col", "dtype", "B", "pieces", "piece_tokens", "H", "D", "Dv", "rot_dims")] + [("eps", _f32), ("reserved", _i32)]
+
+
+class DeltaChunks(C.Structure):
+    """jl_delta_chunks (include/jf_layers.h)."""
+    _fields_ = [(k, _vp) for k in ("qkv", "proj", "A_log", "dt_bias", "norm_w", "chunk_rec", "req", "state", "raw", "scratch", "out")] + \
+               [(k, _i64) for k in ("qkv_ld", "ld", "N", "scratch_floats")] + \
+               [(k, _i32) for k in ("q_col", "k_col", "v_col", "a_col", "b_col", "g_col", "dtype", "B", "chunks", "H", "G", "D", "Dv", "pass_heads")] + \
+               [(k, _f32) for k in ("unit_eps", "q_scale", "eps")] + [("reserved", _i32)]
 
 
 class Addend(C.Structure):
@@ -308,6 +316,9 @@ _LAYER_SIGNATURES = {
     "jl_gated_norm": (C.c_int, [_vp, _vp, C.c_int, _i64, _vp, _f32, _i32, _i32, _f32, _vp, _i64, _i64, _i32, _i32, _vp]),
     "jl_linear_scan": (C.c_int, [C.POINTER(ScanArgs), _vp]),
     "jl_linear_scan_chunked_ok": (C.c_int, [C.c_int, _i32, _i32]),
+    "jl_delta_chunks_ok": (C.c_int, [_i32, _i32]),
+    "jl_delta_chunks_floats": (_i64, [_i32] * 6),
+    "jl_delta_chunks_run": (C.c_int, [_vp, _vp]),
     "jl_delta_rule": (C.c_int, [_vp, C.c_int, _i64, _i32, _i32, _i32, _vp, C.c_int, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                 _i32, _i32, _f32, _f32, _f32, _vp, _vp, _vp, _vp]),
     "jl_linear_small": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, C.c_int, _i32, _i32, _vp, _vp, _i64, _i32, _vp]),
@@ -325,7 +336,7 @@ _LAYER_SIGNATURES = {
 }
 LAYER_SYMBOLS = tuple(_LAYER_SIGNATURES)
 # which library a symbol lives in (jacobiforcing_amd/_build.py: LAYER_GROUPS); both carry their own jl_version / jl_last_error
-_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_gemm", "jl_moe_gemm_gated")
+_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_gemm", "jl_moe_gemm_gated")
 
 
 class _LayerLibs:

@@ -237,21 +237,433 @@ __global__ __launch_bounds__(64) void delta_cols_kernel(const float *__restrict_
             if (d0 + i < D) sp[(int64_t)(d0 + i) * Dv + j] = S[i];
 }
 
-// out_h(t) = o / sqrt(mean(o^2) + eps) * norm_w * silu(gate_h(t)): a wavefront per (token, head)
-template <typename T>
+// out_h(t) = o / sqrt(mean(o^2) + eps) * norm_w * silu(gate_h(t)): 32 lanes per (token, head), four values at a time where rows lie at their borders (bytes bound it:
+// 134 MB at 8192 tokens x 16 heads of 128, a wavefront per row and a value per lane 59 us)
+template <typename T, int VW>
 __global__ __launch_bounds__(256) void delta_out_kernel(const float *__restrict__ raw, const T *__restrict__ proj, int64_t ld, int g_col,
                                                          const float *__restrict__ norm_w, int64_t NH, int H, int Dv, float eps, T *__restrict__ out) {
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t r = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
     if (r >= NH) return;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 31;
     const int64_t n = r / H;
     const int h = (int)(r - n * H);
     const float *o = raw + r * Dv;
-    float ss = 0.f;
-    for (int c = lane; c < Dv; c += 64) ss += o[c] * o[c];
-    ss = wave_sum_f32(ss);
+    const T *gate = proj + n * ld + g_col + (int64_t)h * Dv;
+    float ss = 0.f, v[VW], g[VW];
+    auto load = [&](int c) {
+        if constexpr (VW == 4) ld4_f(o + c, v);
+        else v[0] = o[c];
+    };
+    for (int c = VW * lane; c < Dv; c += 32 * VW) {
+        load(c);
+#pragma unroll
+        for (int i = 0; i < VW; ++i) ss += v[i] * v[i];
+    }
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
     const float rr = 1.0f / sqrtf(ss / (float)Dv + eps);
-    for (int c = lane; c < Dv; c += 64) st_f(out + r * Dv + c, o[c] * rr * norm_w[c] * silu_f(ld_f(proj + n * ld + g_col + h * Dv + c)));
+    for (int c = VW * lane; c < Dv; c += 32 * VW) {
+        if (Dv > 32 * VW) load(c);                                  // otherwise it is still there
+        if constexpr (VW == 4) ld4_f(gate + c, g);
+        else g[0] = ld_f(gate + c);
+#pragma unroll
+        for (int i = 0; i < VW; ++i) g[i] = v[i] * rr * norm_w[c + i] * silu_f(g[i]);
+        if constexpr (VW == 4) st4_f(out + r * Dv + c, g);
+        else st_f(out + r * Dv + c, g[0]);
+    }
+}
+template <typename T>
+static int delta_out_launch(const float *raw, const void *proj, int64_t ld, int g_col, const float *norm_w, int64_t NH, int H, int Dv, float eps, void *out, hipStream_t st) {
+    const dim3 grid((unsigned)((NH + 7) / 8));
+    if ((ld | g_col | Dv) % 4 == 0 && !(((uintptr_t)raw & 15) | (((uintptr_t)proj | (uintptr_t)out) & (4 * sizeof(T) - 1))))
+        delta_out_kernel<T, 4><<<grid, 256, 0, st>>>(raw, (const T *)proj, ld, g_col, norm_w, NH, H, Dv, eps, (T *)out);
+    else delta_out_kernel<T, 1><<<grid, 256, 0, st>>>(raw, (const T *)proj, ld, g_col, norm_w, NH, H, Dv, eps, (T *)out);
+    return jl_check_launch("delta_out_kernel");
+}
+
+// ---- long portions on the float matrix instructions: 64 tokens at a time ------------------------------------------------------------------------
+// With c_t = the running sum of ln g within a chunk of 64 tokens, S the state the chunk starts from, and u_t the corrections, the recurrence is
+//   (I + A) U = diag(beta) V - diag(beta e^c) K S,   A_tj = beta_t e^(c_t - c_j) (k_t . k_j) for j < t        (unit lower triangular)
+//   o_t = e^(c_t) S^T q_t + sum_{j <= t} e^(c_t - c_j) (q_t . k_j) u_j,        S <- e^(c_63) S + sum_j e^(c_63 - c_j) k_j u_j^T
+// so with T = (I + A)^-1, W1 = T diag(beta) V and W2 = T diag(beta e^c) K a chunk costs the chain four products: U = W1 - W2 S, then o and S.
+// delta_chunk_kernel makes unit vectors, T, W1, -W2 and P_tj = e^(c_t - c_j) (q_t . k_j) for all chunks and heads side by side; delta_chain_kernel walks a request's
+// chunks with 32 columns of one head's state in accumulators.  Everything is a 32-bit number, as in the scan; the sums c are 64-bit (differences of long sums).  A token
+// that does not exist has k = q = v = 0, beta = 0, g = 1.  ln g below -1e4 counts as -1e4: e^ of it is zero all the same, and differences stay numbers.
+//
+// v_mfma_f32_32x32x2_f32: lane l supplies row (A) or column (B) l % 32 at depth l / 32; accumulator r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  Four
+// instructions take a unit of 16 bytes per lane, depths 8 u + 4 (l / 32) + i of unit u — which is also how four accumulators of a lane lie, so results are the next
+// product's operand as they are: between the kernels (every operand as units [unit][lane], read as 1 KB per wavefront straight into registers, a chunk ahead) and in LDS
+// between the wavefronts of a chain.  T comes from 16 x 16 blocks by substitution, joined by products, on one wavefront while the others make P.
+// What bounds it: the chain's 128 matrix instructions of 64 cycles per chunk on the busiest of its four wavefronts (D = 128; 58 % of its time), and in the chunks' kernel the
+// phases of a workgroup that wait for each other (two workgroups per CU at 77.5 KB of LDS; with one, 302 us instead of 198).
+// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 446 us (chunks 198, chain 214,
+// norm 34); 8 heads, one portion of 128 80 -> 45; 16 heads, 777 + 300 tokens beside 30 single ones 566 -> 148; float, 8 heads, 1021 + 851 + 681 tokens 587 -> 149.
+constexpr int DK_T = 64;
+typedef float dk_f32x16 __attribute__((ext_vector_type(16)));
+typedef float dk_f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ dk_f32x16 dk_mma(float4 a, float4 b, dk_f32x16 c) {
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, c, 0, 0, 0);
+}
+__device__ __forceinline__ dk_f32x4 dk_mma16(float4 a, float4 b, dk_f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+__device__ __forceinline__ void dk_wave_sync() {        // LDS written by some lanes is read by others of the same wavefront
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// floats of scratch: per chunk and head W2, W1, P, e^c and e^(c_63 - c); per chunk and key head the unit vectors
+struct dk_sizes { int64_t w2, w1, p, head, group; };
+static __host__ __device__ inline dk_sizes dk_layout(int DP, int Dv) {
+    dk_sizes z;
+    z.w2 = 0;
+    z.w1 = (int64_t)DK_T * DP;
+    z.p = z.w1 + (int64_t)DK_T * ((Dv + 31) / 32 * 32);
+    z.head = z.p + 3 * 1024 + 2 * DK_T;
+    z.group = (int64_t)2 * DK_T * DP;
+    return z;
+}
+
+template <typename T, int DP>
+__global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, int h0, int nh) {
+    constexpr int U = DP / 4, DT = DP / 32;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float4 *Ks = (float4 *)smem, *Qs = Ks + DK_T * U, *Am = Qs + DK_T * U;          // rows of units, permuted by the row
+    double *cs = (double *)(Am + 3 * 256);                                         // [64] sums of ln g
+    float *bs = (float *)(cs + DK_T), *bg = bs + DK_T;                             // [64] beta; -beta e^c
+    const int hl = blockIdx.x % nh, h = h0 + hl, chunk = blockIdx.x / nh, per = a.H / a.G, kh = h / per, D = a.D, Dv = a.Dv;
+    const int row0 = a.chunk_rec[4 * chunk], cnt = a.chunk_rec[4 * chunk + 1];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+    const dk_sizes z = dk_layout(DP, Dv);
+    float *head = a.scratch + ((int64_t)chunk * nh + hl) * z.head;
+    float *group = a.scratch + (int64_t)a.chunks * nh * z.head + ((int64_t)chunk * (nh / per) + hl / per) * z.group;
+    const bool leader = hl % per == 0;                                             // writes its key head's unit vectors
+    auto at = [](int row, int u) { return u ^ (row & 15); };                        // rows have a multiple of 16 units
+    auto am_at = [](int t, int u) { return t < 32 ? t * 8 + (u ^ (t & 7)) : 256 + (t - 32) * 16 + (u ^ (t & 15)); };    // A, then T: the first 32 rows have 32 columns
+    const float *src = a.qkv + (int64_t)row0 * a.qkv_ld + kh * D;
+#pragma unroll
+    for (int it = 0; it < DK_T * U / 256; ++it) {                                  // unit vectors: U adjacent lanes hold a row
+        const int e = tid + it * 256, tt = e / U, u = e % U;
+        float4 q = make_float4(0.f, 0.f, 0.f, 0.f), k = q;
+        if (tt < cnt && 4 * u < D) {
+            const float *row = src + (int64_t)tt * a.qkv_ld + 4 * u;
+            q = *(const float4 *)(row + a.q_col);
+            k = *(const float4 *)(row + a.k_col);
+        }
+        float sq = (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w), sk = (k.x * k.x + k.y * k.y) + (k.z * k.z + k.w * k.w);
+#pragma unroll
+        for (int off = 1; off < U; off <<= 1) { sq += __shfl_xor(sq, off, 64); sk += __shfl_xor(sk, off, 64); }
+        const float rq = tt < cnt ? a.q_scale / sqrtf(sq + a.unit_eps) : 0.f, rk = tt < cnt ? 1.0f / sqrtf(sk + a.unit_eps) : 0.f;
+        Qs[tt * U + at(tt, u)] = make_float4(q.x * rq, q.y * rq, q.z * rq, q.w * rq);
+        Ks[tt * U + at(tt, u)] = make_float4(k.x * rk, k.y * rk, k.z * rk, k.w * rk);
+    }
+    if (wave == 0) {
+        float lg = 0.f, beta = 0.f;
+        if (lane < cnt) {
+            const T *row = (const T *)a.proj + (int64_t)(row0 + lane) * a.ld;
+            lg = -expf(a.A_log[h]) * softplus_f(ld_f(row + a.a_col + h) + a.dt_bias[h]);
+            lg = lg < -1e4f ? -1e4f : lg;
+            beta = 1.0f / (1.0f + expf(-ld_f(row + a.b_col + h)));
+        }
+        double c = lg;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double y = __shfl_up(c, off, 64);
+            if (lane >= off) c += y;
+        }
+        const double end = __shfl(c, 63, 64);
+        const float gam = expf((float)c);
+        cs[lane] = c;
+        bs[lane] = beta;
+        bg[lane] = -beta * gam;
+        head[z.p + 3 * 1024 + lane] = gam;
+        head[z.p + 3 * 1024 + DK_T + lane] = expf((float)(end - c));
+    }
+    __syncthreads();
+    // a quarter [32 t, 32 j] of K K^T or Q K^T: lane l ends with t = 32 ti + l % 32, unit y the four j at 32 tj + 8 y + 4 (l / 32)
+    auto pairs = [&](const float4 *rows, int ti, int tj, bool diagonal, float row_factor, auto &&store) {
+        const int t = 32 * ti + l32, j = 32 * tj + l32;
+        dk_f32x16 s, s2;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = s2[r] = 0.f;
+#pragma unroll 2
+        for (int x = 0; x < U / 2; x += 2) {
+            s = dk_mma(Ks[j * U + at(j, 2 * x + hi)], rows[t * U + at(t, 2 * x + hi)], s);
+            s2 = dk_mma(Ks[j * U + at(j, 2 * x + 2 + hi)], rows[t * U + at(t, 2 * x + 2 + hi)], s2);
+        }
+        s += s2;
+        const double ct = cs[t];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int jj = 32 * tj + 8 * y + 4 * hi + i;
+                v[i] = jj < t || (diagonal && jj == t) ? s[4 * y + i] * row_factor * expf((float)(ct - cs[jj])) : 0.f;
+            }
+            store(t, y, make_float4(v[0], v[1], v[2], v[3]));
+        }
+    };
+    if (wave < 3) {
+        const int ti = wave > 0, tj = wave > 1;
+        pairs(Ks, ti, tj, false, bs[32 * ti + l32], [&](int t, int y, float4 v) { Am[am_at(t, 8 * tj + 2 * y + hi)] = v; });
+    } else if (leader) {
+#pragma unroll 4
+        for (int e = 0; e < 2 * (DP / 8); ++e) {
+            const int t = 32 * (e / (DP / 8)) + l32, x = e % (DP / 8);
+            ((float4 *)group)[e * 64 + lane] = Qs[t * U + at(t, 2 * x + hi)];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // (I + A)^-1 in place.  The four 16 x 16 blocks of the diagonal by substitution, a lane per column
+        float *am = (float *)Am;
+        auto el = [&](int t, int j) -> float & { return am[4 * am_at(t, j >> 2) + (j & 3)]; };
+        {
+            const int b0 = 16 * (lane >> 4), c = lane & 15;
+            float x[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float s = r == c ? 1.0f : 0.f;
+#pragma unroll
+                for (int y = 0; y < (r + 3) / 4; ++y) {
+                    const float4 v = Am[am_at(b0 + r, b0 / 4 + y)];
+                    if (4 * y < r) s -= v.x * x[4 * y];
+                    if (4 * y + 1 < r) s -= v.y * x[4 * y + 1];
+                    if (4 * y + 2 < r) s -= v.z * x[4 * y + 2];
+                    if (4 * y + 3 < r) s -= v.w * x[4 * y + 3];
+                }
+                x[r] = s;
+            }
+            dk_wave_sync();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) el(b0 + r, b0 + c) = x[r];
+            dk_wave_sync();
+        }
+        // below the diagonal: T_10 = -T_11 (A_10 T_00), of 16 x 16 blocks, then of 32 x 32 blocks
+#pragma unroll
+        for (int b0 = 0; b0 < 64; b0 += 32) {
+            const int r16 = lane & 15, g = lane >> 4;
+            const int t = b0 + 16 + r16;
+            dk_f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            x = dk_mma16(Am[am_at(t, b0 / 4 + g)], make_float4(el(b0 + 4 * g, b0 + r16), el(b0 + 4 * g + 1, b0 + r16), el(b0 + 4 * g + 2, b0 + r16), el(b0 + 4 * g + 3, b0 + r16)), x);
+            dk_f32x4 w = {0.f, 0.f, 0.f, 0.f};
+            w = dk_mma16(Am[am_at(t, b0 / 4 + 4 + g)], make_float4(x[0], x[1], x[2], x[3]), w);
+            dk_wave_sync();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) el(b0 + 16 + 4 * g + i, b0 + r16) = -w[i];
+            dk_wave_sync();
+        }
+        {
+            const int t = 32 + l32;
+            dk_f32x16 x, w;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[r] = w[r] = 0.f;
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                const int j = 8 * y + 4 * hi;
+                x = dk_mma(Am[am_at(t, 2 * y + hi)], make_float4(el(j, l32), el(j + 1, l32), el(j + 2, l32), el(j + 3, l32)), x);
+            }
+#pragma unroll
+            for (int y = 0; y < 4; ++y) w = dk_mma(Am[am_at(t, 8 + 2 * y + hi)], make_float4(x[4 * y], x[4 * y + 1], x[4 * y + 2], x[4 * y + 3]), w);
+            dk_wave_sync();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) el(32 + 8 * (r >> 2) + 4 * hi + (r & 3), l32) = -w[r];
+        }
+    } else {
+        const int ti = wave > 1, tj = wave > 2, tile = wave - 1;
+        pairs(Qs, ti, tj, true, 1.0f, [&](int, int y, float4 v) { ((float4 *)(head + z.p))[(4 * tile + y) * 64 + lane] = v; });
+    }
+    __syncthreads();
+    auto trow = [&](int ti, int y) { const int t = 32 * ti + l32; return Am[am_at(t, 2 * y + hi)]; };
+    const int nv = (Dv + 31) / 32;
+    for (int task = wave; task < DT + nv; task += 4) {
+        float4 f[8];                                                               // 32 columns of K or V at all 64 depths
+        dk_f32x16 acc[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+        if (task < DT) {                                                           // -W2 transposed: rows of K^T, columns t
+            const float *kf = (const float *)Ks;
+            const int d = 32 * task + l32;
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = kf[4 * (t * U + at(t, d >> 2)) + (d & 3)]; }
+                f[y] = make_float4(v[0], v[1], v[2], v[3]);
+                if (leader) ((float4 *)group)[(DP / 4 + 8 * task + y) * 64 + lane] = f[y];
+            }
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                const float4 s = *(const float4 *)(bg + 8 * y + 4 * hi), v = make_float4(f[y].x * s.x, f[y].y * s.y, f[y].z * s.z, f[y].w * s.w);
+                if (y < 4) acc[0] = dk_mma(v, trow(0, y), acc[0]);
+                acc[1] = dk_mma(v, trow(1, y), acc[1]);
+            }
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    ((float4 *)(head + z.w2))[(ti * (DP / 8) + 4 * task + y) * 64 + lane] = make_float4(acc[ti][4 * y], acc[ti][4 * y + 1], acc[ti][4 * y + 2], acc[ti][4 * y + 3]);
+        } else {                                                                   // W1: rows t, 32 columns of beta V
+            const int vt = task - DT, col = 32 * vt + l32;
+            const float *vp = a.qkv + (int64_t)row0 * a.qkv_ld + a.v_col + (int64_t)h * Dv + col;
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = t < cnt && col < Dv ? vp[t * a.qkv_ld] * bs[t] : 0.f; }
+                f[y] = make_float4(v[0], v[1], v[2], v[3]);
+            }
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                if (y < 4) acc[0] = dk_mma(trow(0, y), f[y], acc[0]);
+                acc[1] = dk_mma(trow(1, y), f[y], acc[1]);
+            }
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    ((float4 *)(head + z.w1))[((vt * 2 + ti) * 4 + y) * 64 + lane] = make_float4(acc[ti][4 * y], acc[ti][4 * y + 1], acc[ti][4 * y + 2], acc[ti][4 * y + 3]);
+        }
+    }
+}
+
+// Workgroup (request, head, 32 columns); the column blocks of a head lie eight apart, on one XCD, since they read the same operands.  Wavefronts 0 and 1 make U, 2 and 3 the
+// outputs of 32 tokens each; every one of the first D / 32 owns 32 rows of S.
+template <int DP>
+__global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, int h0, int nh, float *__restrict__ raw) {
+    constexpr int NU = DP / 8, DT = DP / 32;
+    __shared__ float4 Sf[NU * 64], Uf[8 * 64], Ug[8 * 64];
+    const int nv = (a.Dv + 31) / 32, lin = blockIdx.x >> 3, vt = lin % nv, bh = (lin / nv) * 8 + (blockIdx.x & 7);
+    if (bh >= a.B * nh) return;
+    const int b = bh / nh, hl = bh - b * nh, h = h0 + hl, per = a.H / a.G, D = a.D, Dv = a.Dv;
+    const int first = a.req[4 * b], n = a.req[4 * b + 1], pos0 = a.req[4 * b + 2], slot = a.req[4 * b + 3];
+    if (n <= 0) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * vt + l32, ti = wave & 1;
+    const bool maker = wave < 2, owner = wave < DT;
+    const dk_sizes z = dk_layout(DP, Dv);
+    const float *heads = a.scratch + (int64_t)hl * z.head, *groups = a.scratch + (int64_t)a.chunks * nh * z.head + (int64_t)(hl / per) * z.group;
+    const int64_t head_step = nh * z.head, group_step = (nh / per) * z.group;
+    float *sp = a.state + ((int64_t)slot * a.H + h) * D * Dv;
+    dk_f32x16 S;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int d = 32 * wave + 8 * (r >> 2) + 4 * hi + (r & 3);
+        S[r] = owner && d < D && col < Dv && pos0 > 0 ? sp[(int64_t)d * Dv + col] : 0.f;
+    }
+    auto share_state = [&]() {
+        if (owner)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) Sf[(4 * wave + y) * 64 + lane] = make_float4(S[4 * y], S[4 * y + 1], S[4 * y + 2], S[4 * y + 3]);
+    };
+    share_state();
+    float4 fa[NU], fk[8], fp[8], w1[4], sc[4];
+    float gend;
+    // what U, or the outputs, take of S, and their scales; the keys that the owned rows of S take up, and the pairs
+    struct sources { const float4 *a, *w1, *sc, *k, *p; const float *gend; };
+    auto sources_of = [&](int c) {
+        const float *hp = heads + (int64_t)c * head_step, *gp = groups + (int64_t)c * group_step;
+        sources q;
+        q.a = (const float4 *)(maker ? hp + z.w2 : gp) + ti * NU * 64 + lane;
+        q.w1 = (const float4 *)(hp + z.w1) + ((vt * 2 + ti) * 4) * 64 + lane;
+        q.sc = (const float4 *)(hp + z.p + 3 * 1024 + (maker ? DK_T : 0) + 32 * ti + 4 * hi);
+        q.k = (const float4 *)gp + (DP / 4 + (owner ? 8 * wave : 0)) * 64 + lane;
+        q.p = (const float4 *)(hp + z.p) + 4 * ti * 64 + lane;
+        q.gend = hp + z.p + 3 * 1024 + DK_T - 1;
+        return q;
+    };
+    {
+        const sources q = sources_of(first);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) fa[u] = q.a[u * 64];
+#pragma unroll
+        for (int y = 0; y < 8; ++y) {
+            if (owner) fk[y] = q.k[y * 64];
+            if (!maker && (y < 4 || ti)) fp[y] = q.p[y * 64];
+            if (y < 4) {
+                if (maker) w1[y] = q.w1[y * 64];
+                sc[y] = q.sc[2 * y];
+            }
+        }
+        gend = *q.gend;
+    }
+    for (int c = first; c < first + n; ++c) {
+        const int row0 = a.chunk_rec[4 * c], cnt = a.chunk_rec[4 * c + 1];
+        const sources q = sources_of(c + 1 < first + n ? c + 1 : c);    // every operand's successor sets out when it has been used: a whole chunk ahead, in its registers
+        __syncthreads();                                            // S is there, U has been read
+        dk_f32x16 acc, part[3];                                     // four shorter sums: a rounding each, and what 128 in a row lose is more than the scan's lanes do
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc[r] = maker ? ((const float *)&w1[r >> 2])[r & 3] : 0.f;
+            part[0][r] = part[1][r] = part[2][r] = 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < NU; u += 4) {
+            part[0] = dk_mma(fa[u], Sf[u * 64 + lane], part[0]);
+            part[1] = dk_mma(fa[u + 1], Sf[(u + 1) * 64 + lane], part[1]);
+            part[2] = dk_mma(fa[u + 2], Sf[(u + 2) * 64 + lane], part[2]);
+            acc = dk_mma(fa[u + 3], Sf[(u + 3) * 64 + lane], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fa[u + i] = q.a[(u + i) * 64];
+        }
+        acc += (part[0] + part[1]) + part[2];
+        if (maker) {
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                Uf[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y], acc[4 * y + 1], acc[4 * y + 2], acc[4 * y + 3]);
+                Ug[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y] * sc[y].x, acc[4 * y + 1] * sc[y].y, acc[4 * y + 2] * sc[y].z, acc[4 * y + 3] * sc[y].w);
+            }
+        } else
+#pragma unroll
+            for (int y = 0; y < 4; ++y) { acc[4 * y] *= sc[y].x; acc[4 * y + 1] *= sc[y].y; acc[4 * y + 2] *= sc[y].z; acc[4 * y + 3] *= sc[y].w; }
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            if (maker) w1[y] = q.w1[y * 64];
+            sc[y] = q.sc[2 * y];
+        }
+        __syncthreads();                                            // U is there, S has been read
+        if (owner) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) S[r] *= gend;
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                S = dk_mma(fk[y], Ug[y * 64 + lane], S);
+                fk[y] = q.k[y * 64];
+            }
+            gend = *q.gend;
+            share_state();
+        }
+        if (!maker) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[0][r] = 0.f;
+#pragma unroll
+            for (int y = 0; y < 4; ++y) part[0] = dk_mma(fp[y], Uf[y * 64 + lane], part[0]);
+            if (ti)
+#pragma unroll
+                for (int y = 4; y < 8; ++y) acc = dk_mma(fp[y], Uf[y * 64 + lane], acc);
+            acc += part[0];
+#pragma unroll
+            for (int y = 0; y < 8; ++y)
+                if (y < 4 || ti) fp[y] = q.p[y * 64];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int t = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3);
+                if (t < cnt && col < Dv) raw[(int64_t)(row0 + t) * ((int64_t)a.H * Dv) + (int64_t)h * Dv + col] = acc[r];
+            }
+        }
+    }
+    if (owner && col < Dv)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int d = 32 * wave + 8 * (r >> 2) + 4 * hi + (r & 3);
+            if (d < D) sp[(int64_t)d * Dv + col] = S[r];
+        }
 }
 
 template <typename T, int DMAX>
@@ -264,9 +676,7 @@ static int delta_cols_launch(const void *qkv, int64_t qkv_ld, int q_col, int k_c
                                                          D, Dv, unit_eps, q_scale, state, raw);
     int rc = jl_check_launch("delta_cols_kernel");
     if (rc != JL_OK) return rc;
-    const int64_t NH = N * H;
-    delta_out_kernel<T><<<dim3((unsigned)((NH + 3) / 4)), 256, 0, st>>>(raw, (const T *)proj, ld, g_col, norm_w, NH, H, Dv, eps, (T *)out);
-    return jl_check_launch("delta_out_kernel");
+    return delta_out_launch<T>(raw, proj, ld, g_col, norm_w, N * H, H, Dv, eps, out, st);
 }
 
 template <typename T, typename TQ, int DMAX, int LPC>
@@ -315,5 +725,48 @@ extern "C" int jl_delta_rule(const void *qkv, int qkv_dtype, int64_t qkv_ld, int
     else DL_CASE(256);
 #undef DL_CASE
 #undef DL_ARGS
+    return JL_OK;
+}
+
+extern "C" int jl_delta_chunks_ok(int32_t D, int32_t Dv) { return D > 0 && D <= 128 && D % 4 == 0 && Dv > 0 && Dv <= 1024; }
+
+// heads come in whole key groups
+extern "C" int64_t jl_delta_chunks_floats(int32_t chunks, int32_t heads, int32_t H, int32_t G, int32_t D, int32_t Dv) {
+    if (chunks <= 0 || heads <= 0 || G <= 0 || H <= 0 || H % G || !jl_delta_chunks_ok(D, Dv)) return 0;
+    const dk_sizes z = dk_layout(D <= 64 ? 64 : 128, Dv);
+    return (int64_t)chunks * (heads * z.head + heads / (H / G) * z.group);
+}
+
+template <typename T, int DP> static int delta_chunks_launch(const jl_delta_chunks &a, hipStream_t st) {
+    const size_t lds = (size_t)(2 * DK_T * DP + 3 * 1024 + 2 * DK_T) * 4 + DK_T * 8;
+    auto chunk = delta_chunk_kernel<T, DP>;
+    hipError_t e = hipFuncSetAttribute((const void *)chunk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_delta_chunks_run: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+    const int nv = (a.Dv + 31) / 32;
+    for (int h0 = 0; h0 < a.H; h0 += a.pass_heads) {                 // as many heads at a time as the scratch holds
+        const int nh = a.H - h0 < a.pass_heads ? a.H - h0 : a.pass_heads;
+        chunk<<<dim3((unsigned)nh * (unsigned)a.chunks), 256, lds, st>>>(a, h0, nh);
+        delta_chain_kernel<DP><<<dim3((unsigned)((a.B * nh + 7) / 8 * nv * 8)), 256, 0, st>>>(a, h0, nh, a.raw);
+    }
+    int rc = jl_check_launch("delta_chunk_kernel");
+    if (rc != JL_OK) return rc;
+    return a.out ? delta_out_launch<T>(a.raw, a.proj, a.ld, a.g_col, a.norm_w, a.N * a.H, a.H, a.Dv, a.eps, a.out, st) : JL_OK;
+}
+
+extern "C" int jl_delta_chunks_run(const jl_delta_chunks *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: null arguments");
+    const jl_delta_chunks &a = *ap;
+    if (a.B <= 0 || a.chunks <= 0) return JL_OK;
+    if (!a.qkv || !a.proj || !a.A_log || !a.dt_bias || !a.norm_w || !a.chunk_rec || !a.req || !a.state || !a.scratch || !a.raw)
+        return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: null pointer");
+    if (!jl_delta_chunks_ok(a.D, a.Dv) || a.H <= 0 || a.G <= 0 || a.H % a.G || a.N <= 0 || (int64_t)a.chunks * a.H > INT32_MAX / 256 || a.pass_heads <= 0 || a.pass_heads % (a.H / a.G) || a.qkv_ld % 4 ||
+        (a.q_col | a.k_col) % 4 || (((uintptr_t)a.qkv | (uintptr_t)a.scratch) & 15) || (a.dtype != JL_BF16 && a.dtype != JL_F32))
+        return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: sizes, columns or alignment (ask jl_delta_chunks_ok)");
+    if (a.q_col < 0 || a.k_col < 0 || a.v_col < 0 || a.a_col < 0 || a.b_col < 0 || a.g_col < 0 || a.q_col + (int64_t)a.G * a.D > a.qkv_ld || a.k_col + (int64_t)a.G * a.D > a.qkv_ld ||
+        a.v_col + (int64_t)a.H * a.Dv > a.qkv_ld || a.a_col + (int64_t)a.H > a.ld || a.b_col + (int64_t)a.H > a.ld || a.g_col + (int64_t)a.H * a.Dv > a.ld)
+        return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: columns do not fit the rows");
+    if (a.scratch_floats < jl_delta_chunks_floats(a.chunks, a.pass_heads < a.H ? a.pass_heads : a.H, a.H, a.G, a.D, a.Dv))
+        return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: scratch is too small");
+    JL_DISPATCH(a.dtype, return a.D <= 64 ? delta_chunks_launch<T, 64>(a, (hipStream_t)stream) : delta_chunks_launch<T, 128>(a, (hipStream_t)stream));
     return JL_OK;
 }

@@ -25,6 +25,8 @@ RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions f
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
 SCAN_PIECES_FROM, SCAN_WORKGROUPS = 32, 512     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
+DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
+DELTA_SCRATCH_FLOATS = 256 << 20     # scratch of those chunks at most (1 GiB: more heads than it holds take turns), as long as it holds one key head's
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -147,6 +149,22 @@ class RaggedBatch:
                 r0 += c
             both = torch.tensor(rec + req, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
             self._tiles[key] = (both[:len(rec)], both[len(rec):])
+        return self._tiles[key]
+
+    def long_pieces(self, size: int, least: int):
+        """``pieces`` of the requests with at least ``least`` tokens alone (request records of those), the other requests' rows of ``seq`` and their longest portion (0: none)."""
+        key = ("long", size, least)
+        if key not in self._tiles:
+            rec, req, rest, r0 = [], [], [], 0
+            for c, s, sl in zip(self.counts, self.starts, self.slots):
+                if c >= least:
+                    req.append((len(rec), -(-c // size), s, sl))
+                    rec += [(r0 + o, min(size, c - o), sl, int(o + size >= c)) for o in range(0, c, size)]
+                else:
+                    rest.append((r0, c, s, sl))
+                r0 += c
+            every = torch.tensor(rec + req + rest, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
+            self._tiles[key] = (every[:len(rec)], every[len(rec):len(rec) + len(req)], every[len(rec) + len(req):], max((r[1] for r in rest), default=0))
         return self._tiles[key]
 
     def key_rows(self, requests: Sequence[int], window: int):
@@ -1045,10 +1063,27 @@ def delta_rule(qkv: torch.Tensor, cols: Tuple[int, int, int], proj: torch.Tensor
     for t, k in ((a_log, H), (dt_bias, H), (norm_w, Dv)):
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == k, "delta_rule: a_log, dt_bias float [H], norm_w float [Dv]")
     out = torch.empty((n, H * Dv), dtype=proj.dtype, device=proj.device)
-    long_portions = max(batch.counts) >= DELTA_COLUMNS_FROM and not os.environ.get("JL_DELTA_NO_COLUMNS")          # A/B switch for measurements
-    raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device) if long_portions else None
+    longest = max(batch.counts) if not os.environ.get("JL_DELTA_NO_COLUMNS") else 1          # A/B switch for measurements
+    raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device) if longest >= DELTA_COLUMNS_FROM else None
+    seq, B = batch.seq, batch.B
+    if longest >= DELTA_CHUNKS_FROM and N.layers().jl_delta_chunks_ok(D, Dv) and (qkv.shape[1] | cols[0] | cols[1]) % 4 == 0 and qkv.data_ptr() % 16 == 0:
+        rec, req, seq, longest = batch.long_pieces(64, DELTA_CHUNKS_FROM)
+        B, chunks, per = seq.shape[0], rec.shape[0], H // G
+        floats = lambda heads: N.layers().jl_delta_chunks_floats(chunks, heads, H, G, D, Dv)
+        heads = min(H, max(1, DELTA_SCRATCH_FLOATS // floats(per)) * per)
+        scratch = torch.empty((floats(heads),), dtype=torch.float32, device=proj.device)
+        columns = longest >= DELTA_COLUMNS_FROM                             # portions of lengths between: their launch norms and gates all rows
+        a = N.DeltaChunks(qkv=qkv.data_ptr(), proj=proj.data_ptr(), A_log=a_log.data_ptr(), dt_bias=dt_bias.data_ptr(), norm_w=norm_w.data_ptr(), chunk_rec=rec.data_ptr(),
+                          req=req.data_ptr(), state=state.data_ptr(), raw=raw.data_ptr(), scratch=scratch.data_ptr(), out=None if columns else out.data_ptr(), qkv_ld=qkv.shape[1],
+                          ld=ld, N=n, scratch_floats=scratch.numel(), q_col=cols[0], k_col=cols[1], v_col=cols[2], a_col=pcols[0], b_col=pcols[1], g_col=pcols[2],
+                          dtype=_code(proj.dtype), B=req.shape[0], chunks=chunks, H=H, G=G, D=D, Dv=Dv, pass_heads=heads, unit_eps=unit_eps, q_scale=q_scale, eps=eps)
+        N.check_layers(N.layers().jl_delta_chunks_run(C.byref(a), _stream(proj.device)), "jl_delta_chunks_run")
+        if B == 0:
+            return out
+        if not columns:
+            raw = None                                                      # a workgroup per request and head, which writes its rows' outputs itself
     N.check_layers(N.layers().jl_delta_rule(_ptr(qkv), N.JL_F32, qkv.shape[1], cols[0], cols[1], cols[2], _ptr(proj), _code(proj.dtype), ld, pcols[0], pcols[1],
-                                           pcols[2], _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), _ptr(batch.seq), batch.B, n, H, G, D, Dv, float(unit_eps),
+                                           pcols[2], _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), _ptr(seq), B, n, H, G, D, Dv, float(unit_eps),
                                            float(q_scale), float(eps), _ptr(state), _ptr(raw), _ptr(out), _stream(proj.device)), "jl_delta_rule")
     return out
 

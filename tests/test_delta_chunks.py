@@ -1,0 +1,74 @@
+"""The delta rule of long portions in chunks on the matrix cores, at the edges of its chunks of 64 tokens and tiles of 32 columns, against the recurrence in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("H,G,D,Dv,counts,starts,keys,floats", [
+    (4, 2, 128, 128, [200, 64, 1, 40], [0, 30, 5, 2], "random", 1 << 30), (3, 3, 64, 33, [129, 65, 63, 300], [0, 0, 7, 1], "random", 1 << 30), (6, 2, 24, 20, [500, 33], [3, 0], "alike", 1),
+    (4, 1, 100, 300, [128, 127, 66], [9, 0, 0], "random", 200000), (1, 1, 4, 1, [32], [1], "alike", 1 << 30), (2, 2, 68, 128, [1000], [0], "alike", 1 << 30), (8, 4, 128, 96, [96], [4], "zero", 40000),
+])
+def test_chunks(monkeypatch, dtype, H, G, D, Dv, counts, starts, keys, floats):
+    """Unequal portions (one token among them), slots of new requests hold NaN; decays of one, ordinary ones, beyond the exponent's range; keys that hardly differ; scratch
+    (``floats``) for all heads, some, one key head's."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt, eps, unit_eps = "cuda", getattr(torch, dtype), 1e-5, 1e-6
+    monkeypatch.setattr(LO, "DELTA_SCRATCH_FLOATS", floats)
+    monkeypatch.setattr(LO, "DELTA_CHUNKS_FROM", min(max(counts), 64))
+    g = torch.Generator(device=dev).manual_seed(D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    B, n = len(counts), sum(counts)
+    qkv = rnd(n, 2 * G * D + H * Dv + 4 + (-H * Dv) % 4)
+    cols = (4, 4 + G * D, 4 + 2 * G * D)
+    if keys == "alike":
+        qkv[:, cols[1]:cols[1] + G * D] = 1 + 0.01 * qkv[:, cols[1]:cols[1] + G * D]
+    if keys == "zero":
+        qkv[::3, cols[1]:cols[1] + G * D] = 0
+    proj = rnd(n, 2 * H + H * Dv + 3).to(dt)
+    pcols = (1, 1 + H, 1 + 2 * H)
+    proj[5:9, 1:1 + H] = 300.0                                       # a decay of nothing
+    proj[:, 1 + H:1 + 2 * H] += 2.0
+    a_log, dt_bias = torch.linspace(-12.0, 6.0, H, device=dev), 0.3 * rnd(H)
+    norm_w = 1 + 0.1 * rnd(Dv)
+    slots = list(range(1, B + 1))
+    state = rnd(B + 2, H, D, Dv)
+    for s, sl in zip(starts, slots):
+        if s == 0:
+            state[sl] = float("nan")
+    before = state.clone()
+    batch = LO.RaggedBatch.build(counts, starts, slots, [[b * 40 + i for i in range(40)] for b in range(B)], 64, dev)
+    run = lambda st: LO.delta_rule(qkv, cols, proj, pcols, a_log, dt_bias, norm_w, batch, H, G, D, Dv, unit_eps, D ** -0.5, eps, st)
+    got = run(state)
+    assert any(k[0] == "long" for k in batch._tiles if isinstance(k, tuple)), "the form in chunks did not run"
+    scan_state = before.clone()
+    monkeypatch.setattr(LO, "DELTA_CHUNKS_FROM", 1 << 30)
+    scan = run(scan_state)
+    x64, p64, r0 = qkv.double(), proj.double(), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        rows, p = x64[r0:r0 + c], p64[r0:r0 + c]
+        unit = lambda x: (x / torch.sqrt((x * x).sum(-1, keepdim=True) + unit_eps)).repeat_interleave(H // G, 1)
+        q, k = (unit(rows[:, x:x + G * D].view(c, G, D)) for x in cols[:2])
+        v = rows[:, cols[2]:cols[2] + H * Dv].view(c, H, Dv)
+        gate = p[:, pcols[2]:pcols[2] + H * Dv].view(c, H, Dv)
+        dec = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, pcols[0]:pcols[0] + H] + dt_bias.double()))
+        beta = torch.sigmoid(p[:, pcols[1]:pcols[1] + H])
+        S = before[slots[b]].double() if s else torch.zeros(H, D, Dv, dtype=torch.float64, device=dev)
+        o = []
+        for t in range(c):
+            S = dec[t].view(H, 1, 1) * S
+            u = beta[t].view(H, 1) * (v[t] - (k[t].unsqueeze(-2) @ S).squeeze(-2))
+            S = S + k[t].unsqueeze(-1) * u.unsqueeze(-2)
+            o.append((q[t].unsqueeze(-2) @ S).squeeze(-2) * D ** -0.5)
+        o = torch.stack(o)
+        o = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * norm_w.double() * torch.nn.functional.silu(gate)
+        # 32-bit sums of products either way: as far off as the token by token form, which may be lucky: 5 roundings.  Where keys hardly differ the corrections of a chunk cancel in
+        # the outputs: a rounding of each of up to 64
+        slack = 64 * 2.0 ** -24 if keys == "alike" else 5 * 2.0 ** -24
+        err = lambda x, want: ((x.double() - want).norm() / want.norm()).item()
+        sl = slots[b]
+        assert err(state[sl], S) <= 1.5 * err(scan_state[sl], S) + slack, (b, "state")
+        assert err(got[r0:r0 + c].view(c, H, Dv), o) <= 1.5 * err(scan[r0:r0 + c].view(c, H, Dv), o) + slack, (b, "outputs")
+        r0 += c
+    assert torch.equal(state[0], before[0]) and torch.equal(state[B + 1], before[B + 1])
