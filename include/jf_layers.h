@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 131
+#define JL_VERSION 132
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -132,6 +132,14 @@ JL_API int64_t jl_attn_sweep_scratch_floats(int32_t n_tiles, int32_t H, int32_t 
  * rows to itself (scores, weights and outputs never leave its registers). */
 JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld,
                                         int32_t v_in_k);
+
+/* jl_attn_window with `talk` (heads mixed after the softmax) in one sweep over the keys, for the sizes jl_attn_talk_ok takes; no sink, chunks or cap.  Tiles of
+ * jl_attn_talk_tile_rows(H, G, wide) queries in any order (wide: 128 (query, head) rows per workgroup, else 32), a tile's keys shared out over `splits` workgroups;
+ * scratch of jl_attn_talk_scratch_floats for pass_tiles tiles at a time.  q, pools and scratch at 16-byte borders, k_ld and v_ld in multiples of 8, out_ld of 4. */
+JL_API int jl_attn_talk(const jl_attn_args *a, int32_t wide, int32_t pass_tiles, void *stream);
+JL_API int jl_attn_talk_ok(int dtype, int32_t H, int32_t G, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
+JL_API int jl_attn_talk_tile_rows(int32_t H, int32_t G, int32_t wide);
+JL_API int64_t jl_attn_talk_scratch_floats(int32_t tiles, int32_t TQ, int32_t H, int32_t G, int32_t Dv, int32_t splits);
 
 /* The wide form over keys and values that were built per head for this step (long portions of latent attention: keys and values from the latent
  * by a product instead of queries brought to the latent), G = H, contiguous rows per request instead of pages: key head c of a row is

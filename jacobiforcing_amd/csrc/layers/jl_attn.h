@@ -4,6 +4,18 @@
 
 #include "jl_common.h"
 
+// floats -> bfloat16 (round to nearest even) through the compiler's own conversion: one packed instruction per pair
+typedef __bf16 ar_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float ar_f32x8 __attribute__((ext_vector_type(8)));
+typedef float ar_f32x16 __attribute__((ext_vector_type(16)));
+typedef short ar_s16x4 __attribute__((ext_vector_type(4)));
+typedef short ar_s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) ar_s16x4 ar_lds_s16x4;
+
+// where 16-byte unit u of row r sits in a row of U units
+template <int U> __device__ __forceinline__ int ar_key_unit(int r, int u) { return U % 16 == 0 ? u ^ (r & 15) : u ^ ((r >> 1) & 7); }
+template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { return U == 16 ? u ^ ((r & 3) << 2) : u ^ ((r & 2) << 1); }
+
 constexpr int AR_ROWS = 128;          // (query, head) rows of a tile of the wide form
 
 // the wide form's launch (jl_attn_rows.hip); sizes as jl_attn_sweep has checked them, ``hf`` heads of a.TQ queries per tile, ``hb`` tiles per group

@@ -23,20 +23,8 @@ constexpr int AR_THREADS = 256;
 //   4 x 2048 tokens, 16 heads of 192 / 128 apart           806 -> 180 us (479 TFLOP/s)
 //   4 x 2048 tokens, 8 heads of 128 over 2, window 1024    180 -> 66 us
 
-// floats -> bfloat16 (round to nearest even) through the compiler's own conversion: one packed instruction per pair
-typedef __bf16 ar_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float ar_f32x8 __attribute__((ext_vector_type(8)));
-typedef float ar_f32x16 __attribute__((ext_vector_type(16)));
-typedef short ar_s16x4 __attribute__((ext_vector_type(4)));
-typedef short ar_s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) ar_s16x4 ar_lds_s16x4;
-
 constexpr int ar_tile_keys(int KU) { return KU <= 16 ? 64 : 32; }
 constexpr size_t ar_lds_bytes(int KU, int VU) { return 2 * (size_t)ar_tile_keys(KU) * (KU + VU) * 16 + 2 * ar_tile_keys(KU) * 4; }
-
-// where 16-byte unit u of row r sits in a row of U units
-template <int U> __device__ __forceinline__ int ar_key_unit(int r, int u) { return U % 16 == 0 ? u ^ (r & 15) : u ^ ((r >> 1) & 7); }
-template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { return U == 16 ? u ^ ((r & 3) << 2) : u ^ ((r & 2) << 1); }
 
 template <int KU, int VU, int SRC>                                                      // D <= 8 * KU, Dv <= 8 * VU
 __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a, int HF, int TQ, int HB) {

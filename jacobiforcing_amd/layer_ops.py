@@ -19,6 +19,9 @@ from . import _native as N
 
 ATTN_SPLIT_BELOW_TILES, ATTN_SPLIT_WORKGROUPS = 128, 512     # attention: split a tile's keys while tiles x splits stays below ~2 per CU
 ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-core attention kernel takes in one workgroup
+# mixed heads: workgroups of 4 wavefronts to aim at (of one: three times as many); scratch at most (1 GiB: more tiles than it holds take turns), as long as it holds a tile's.  us, 8 heads
+# over 2 of 128 under a window of 1024, for 512 / 640 / 1024: 777 + 300 tokens beside 30 single ones 105 / 79 / 81, one portion of 1000 54 / 56 / 65
+TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
 RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
@@ -361,9 +364,27 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
     if rel is not None:                                  # rel [rows, H] with lut [positions] -> row, or rel [positions, H] by distance itself
         _need(rel.shape[1] == H and (lut is None or lut.dtype == torch.int32), "attn_window: rel [rows, H] (+ int32 lut)")
     _need(chunk <= 0 or (window <= 0 and keep_first <= 0), "attn_window: chunks exclude a window and kept first tokens")
+    out = _attn_out(out, n, H * Dv, torch.float32 if float_out else dt, q.device, "attn_window")
+    if (talk is not None and sink is None and chunk <= 0 and softcap <= 0 and Gv == G and N.layers().jl_attn_talk_ok(_code(dt), H, G, D, Dv, k_ld, v_ld) and out.stride(0) % 4 == 0 and
+            not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and not os.environ.get("JL_ATTN_NO_MFMA")):
+        wide = n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B
+        tq = int(N.layers().jl_attn_talk_tile_rows(H, G, int(wide)))
+        tiles = batch.tiles(tq, longest_first=wide)
+        reach = batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + int(keep_first) + tq)
+        splits = max(1, min(-(-reach // 64), (TALK_WORKGROUPS if wide else 3 * TALK_WORKGROUPS) // (tiles.shape[0] * G * G), 64))
+        per_tile = int(N.layers().jl_attn_talk_scratch_floats(1, tq, H, G, Dv, splits))
+        pass_tiles = min(tiles.shape[0], max(1, TALK_SCRATCH_FLOATS // per_tile))
+        scratch = torch.empty((per_tile * pass_tiles,), dtype=torch.float32, device=q.device)
+        a = N.AttnArgs(q=q.data_ptr(), gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0, k_cache=k_cache.data_ptr(),
+                       v_cache=v_cache.data_ptr(), out=out.data_ptr(), block_tables=batch.tables.data_ptr(), tiles=tiles.data_ptr(), rel=rel.data_ptr() if rel is not None else None,
+                       lut=lut.data_ptr() if lut is not None else None, talk=talk.data_ptr(), bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0],
+                       lut_len=(lut.numel() if lut is not None else rel.shape[0]) if rel is not None else 0, page_size=batch.page_size, H=H, G=G, D=D, Dv=Dv, window=int(window),
+                       keep_first=max(0, int(keep_first)), TQ=tq, dtype=_code(dt), scale=float(scale), splits=splits, n_rows=n, scratch=scratch.data_ptr(), k_ld=k_ld, v_ld=v_ld, Gv=Gv,
+                       out_dtype=N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME, gate_heads=int(gate_per_head), out_scale=float(out_scale), out_ld=out.stride(0))
+        N.check_layers(N.layers().jl_attn_talk(C.byref(a), int(wide), pass_tiles, _stream(q.device)), "jl_attn_talk")
+        return out
     tq = attn_tile_rows(dt, H, G, D, Dv, k_ld, v_ld)
     tiles = batch.tiles(tq)
-    out = _attn_out(out, n, H * Dv, torch.float32 if float_out else dt, q.device, "attn_window")
     # few tiles with many keys (decoding): share each tile's keys out over workgroups until the chip is full
     splits, scratch = 1, None
     if tq == 32 and tiles.shape[0] < ATTN_SPLIT_BELOW_TILES:

@@ -1,0 +1,55 @@
+"""Attention with mixed heads in one sweep, at the edges of its tiles (32 keys, 32 or 128 rows), windows and kept tokens, against the same in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,G,D,Dv,window,keep,counts,starts,bias,floats,wgs", [
+    (8, 2, 128, 128, 100, 4, [129, 64, 1], [0, 300, 70], "direct", 1 << 28, 512), (4, 4, 64, 32, 0, 0, [200, 33], [5, 0], "lut", 1 << 28, 1), (6, 2, 96, 72, 33, 40, [90, 47, 31], [0, 64, 1000], "direct", 1, 512),
+    (16, 1, 8, 8, 64, 70, [50, 20], [150, 0], None, 1 << 28, 64), (12, 4, 40, 128, 1, 3, [40], [7], "lut", 30000, 512), (5, 5, 128, 56, 300, 0, [65, 200], [0, 512], "direct", 1 << 28, 512),
+    (8, 2, 128, 128, 1000, 4, [1] * 5, [0, 31, 32, 1500, 999], "direct", 1 << 28, 512), (3, 1, 64, 128, 0, 0, [1, 2, 1], [700, 40, 3], "lut", 1, 512), (16, 8, 24, 16, 50, 2, [3, 1], [64, 10], None, 1 << 28, 1), (32, 1, 16, 24, 40, 1, [1, 2], [90, 33], "lut", 1 << 28, 512), (16, 1, 128, 64, 0, 0, [60, 1], [0, 200], "lut", 1 << 28, 512),
+])
+def test_talk(monkeypatch, H, G, D, Dv, window, keep, counts, starts, bias, floats, wgs):
+    """Portions and single tokens; scratch (``floats``) for all tiles or one at a time, keys whole or shared out (``wgs``); gates per value, strided pools."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, page = "cuda", 16
+    monkeypatch.setattr(LO, "TALK_SCRATCH_FLOATS", floats)
+    monkeypatch.setattr(LO, "TALK_WORKGROUPS", wgs)
+    g = torch.Generator(device=dev).manual_seed(H * D + Dv + len(counts))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    n, B = sum(counts), len(counts)
+    need = [-(-(c + s) // page) for c, s in zip(counts, starts)]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(1)).tolist()
+    pages = [[order.pop() for _ in range(x)] for x in need]
+    batch = LO.RaggedBatch.build(counts, starts, list(range(B)), pages, page, dev)
+    kp, vp = rnd(sum(need) * page, G * D + 8).bfloat16()[:, :G * D], rnd(sum(need) * page, G * Dv + 16).bfloat16()[:, 8:8 + G * Dv]
+    q, gate, talk = rnd(n, H * D).bfloat16(), rnd(n, H * Dv + 4).bfloat16()[:, 4:], torch.eye(H, device=dev) + 0.4 * rnd(H, H)
+    longest = max(c + s for c, s in zip(counts, starts))
+    lut = (torch.arange(longest + 50, device=dev).float().sqrt() * 2).int() if bias == "lut" else None
+    rel = rnd(int(lut.max()) + 1 if bias == "lut" else 40, H) if bias else None      # direct: distances beyond the table read its last row
+    scale = D ** -0.5
+    import jacobiforcing_amd._native as N
+    assert N.layers().jl_attn_talk_ok(1 if N.JL_BF16 == 1 else N.JL_BF16, H, G, D, Dv, kp.stride(0), vp.stride(0))
+    out = LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, scale, window, keep, rel, lut, talk, float_out=True)
+    rounded = LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, scale, window, keep, rel, lut, talk)
+    assert torch.equal(rounded, out.bfloat16())
+    r0, rep = 0, H // G
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // page] * page + j % page for j in range(c + s)], device=dev)
+        k, v = kp[tok].double().view(-1, G, D).repeat_interleave(rep, 1), vp[tok].double().view(-1, G, Dv).repeat_interleave(rep, 1)
+        qq = q[r0:r0 + c].double().view(c, H, D)
+        sc = (qq.permute(1, 0, 2).contiguous() @ k.permute(1, 2, 0).contiguous()) * scale
+        i, j = torch.arange(s, s + c, device=dev).view(-1, 1), torch.arange(c + s, device=dev).view(1, -1)
+        if rel is not None:
+            d = (i - j).clamp(min=0)
+            d = lut[d.clamp(max=lut.numel() - 1)].long() if lut is not None else d.clamp(max=rel.shape[0] - 1)
+            sc = sc + rel.double()[d].permute(2, 0, 1)
+        see = (j <= i) & (((i - j) < window) | (j < keep) if window > 0 else torch.ones_like(i - j, dtype=torch.bool))
+        p = torch.softmax(sc.masked_fill(~see, float("-inf")), -1)
+        mixed = torch.einsum("yx,xij->yij", talk.double(), p)
+        o = (mixed.contiguous() @ v.permute(1, 0, 2).contiguous()).permute(1, 0, 2) * torch.sigmoid(gate[r0:r0 + c].double().view(c, H, Dv))
+        err = (out[r0:r0 + c].double().view(c, H, Dv) - o).norm() / o.norm()
+        # scores: float sums of D products times the scale (a few 2 ** -24 of their size, up to about 10); weights to 16 bits of mantissa (2 ** -17), weights and sums cancel by up to 8
+        assert err <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24), (b, err.item())
+        r0 += c
