@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 132
+#define JL_VERSION 133
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -140,6 +140,29 @@ JL_API int jl_attn_talk(const jl_attn_args *a, int32_t wide, int32_t pass_tiles,
 JL_API int jl_attn_talk_ok(int dtype, int32_t H, int32_t G, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
 JL_API int jl_attn_talk_tile_rows(int32_t H, int32_t G, int32_t wide);
 JL_API int64_t jl_attn_talk_scratch_floats(int32_t tiles, int32_t TQ, int32_t H, int32_t G, int32_t Dv, int32_t splits);
+
+/* Attention of a draft block: q [R, nkv, G * T, D] (a key head's heads, then tokens), k and v [blocks, nkv, page_size, D], all bfloat16 and contiguous.  Token t of row r sees the keys
+ * 0 .. kv_len[r] + min(t + 1, row_len[r]) - 1 of the row, at most max_keys: of cache row row_prompt[r] (tables null; page_size the cache's row length) or of the blocks
+ * tables[r * table_ld ..] in order (table_cols of them; a negative one counts as block 0).  With cand_rows > 0 a row whose row_cand is not negative has its keys from kv_len on in
+ * ck / cv [cand_rows, nkv, cand_max, D].  out [R * T, nkv * G * D].  Indexes beyond their tables are clamped.  Keys shared out over `splits` workgroups
+ * (scratch of jl_attn_block_scratch_floats). */
+typedef struct jl_block_args {
+    const void *q, *k, *v, *ck, *cv;
+    const int32_t *kv_len, *row_len, *row_prompt, *row_cand, *tables;
+    void *out;
+    float *scratch;
+    int64_t table_ld;
+    int32_t R, T, nkv, G, D, blocks, page_size, table_cols, cand_rows, cand_max, max_keys, splits;
+    float scale;
+    int32_t reserved;
+} jl_block_args;
+JL_API int jl_attn_block(const jl_block_args *a, void *stream);
+/* Cache slots of the block's tokens, [R * T] int64: row_prompt * S_max + position where row_cand is negative and the token is one of the row's row_len, else -1; slot_cand (may be
+ * null): row_cand * T_max + t where it is not. */
+JL_API int jl_block_slots(const int32_t *positions, const int32_t *row_prompt, const int32_t *row_cand, const int32_t *row_len, int64_t R, int32_t T, int64_t S_max, int64_t T_max,
+                          int64_t *slot_main, int64_t *slot_cand, void *stream);
+JL_API int jl_attn_block_ok(int dtype, int32_t D);
+JL_API int64_t jl_attn_block_scratch_floats(int64_t R, int32_t T, int32_t nkv, int32_t G, int32_t D, int32_t splits);
 
 /* The wide form over keys and values that were built per head for this step (long portions of latent attention: keys and values from the latent
  * by a product instead of queries brought to the latent), G = H, contiguous rows per request instead of pages: key head c of a row is

@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 132                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 133                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -262,6 +262,12 @@ class RetentionPieces(C.Structure):
     """jl_retention_pieces (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("proj", "piece_rec", "req", "pos", "cos_t", "sin_t", "decay", "state", "scratch", "out")] + [("ld", _i64), ("table_len", _i64)] + \
                [(k, _i32) for k in ("q_col", "k_col", "v_col", "g_col", "dtype", "B", "pieces", "piece_tokens", "H", "D", "Dv", "rot_dims")] + [("eps", _f32), ("reserved", _i32)]
+
+
+class BlockArgs(C.Structure):
+    """jl_block_args (include/jf_layers.h)."""
+    _fields_ = [(k, _vp) for k in ("q", "k", "v", "ck", "cv", "kv_len", "row_len", "row_prompt", "row_cand", "tables", "out", "scratch")] + [("table_ld", _i64)] + \
+               [(k, _i32) for k in ("R", "T", "nkv", "G", "D", "blocks", "page_size", "table_cols", "cand_rows", "cand_max", "max_keys", "splits")] + [("scale", _f32), ("reserved", _i32)]
 
 
 class DeltaChunks(C.Structure):
@@ -302,6 +308,10 @@ _LAYER_SIGNATURES = {
     "jl_diff_combine": (C.c_int, [_vp, _vp, _i64, _i64, _i32, _i32, _f32, _f32, _f32, _vp, C.c_int, _vp]),
     "jl_latent_prep": (C.c_int, [_vp, C.c_int, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _f32, _vp, _vp, _vp, _i64, _vp, _vp,
                                  _vp, _i32, _vp]),
+    "jl_attn_block": (C.c_int, [_vp, _vp]),
+    "jl_block_slots": (C.c_int, [_vp, _vp, _vp, _vp, _i64, _i32, _i64, _i64, _vp, _vp, _vp]),
+    "jl_attn_block_ok": (C.c_int, [C.c_int, _i32]),
+    "jl_attn_block_scratch_floats": (_i64, [_i64] + [_i32] * 5),
     "jl_attn_talk": (C.c_int, [C.POINTER(AttnArgs), _i32, _i32, _vp]),
     "jl_attn_talk_ok": (C.c_int, [C.c_int, _i32, _i32, _i32, _i32, _i64, _i64]),
     "jl_attn_talk_tile_rows": (C.c_int, [_i32, _i32, _i32]),

@@ -22,6 +22,7 @@ ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-co
 # mixed heads: workgroups of 4 wavefronts to aim at (of one: three times as many); scratch at most (1 GiB: more tiles than it holds take turns), as long as it holds a tile's.  us, 8 heads
 # over 2 of 128 under a window of 1024, for 512 / 640 / 1024: 777 + 300 tokens beside 30 single ones 105 / 79 / 81, one portion of 1000 54 / 56 / 65
 TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
+BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
 RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
@@ -405,6 +406,53 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
                    sink=sink.data_ptr() if sink is not None else None, gate_heads=int(gate_per_head), chunk=int(chunk), softcap=float(softcap),
                    out_scale=float(out_scale), out_ld=out.stride(0))
     N.check_layers(N.layers().jl_attn_window(C.byref(a), _stream(q.device)), "jl_attn_window")
+    return out
+
+
+def attn_block_ok(dtype: torch.dtype, device: torch.device, D: int) -> bool:
+    """Whether ``attn_block`` takes heads of D values of this dtype."""
+    return device.type == "cuda" and dtype == torch.bfloat16 and bool(N.layers().jl_attn_block_ok(N.JL_BF16, D))
+
+
+def block_slots(positions: torch.Tensor, T: int, row_prompt: torch.Tensor, row_cand: torch.Tensor, row_len: torch.Tensor, S_max: int, T_max: int, candidates: bool):
+    """Cache slots of a draft block's tokens (int64 [R*T], -1: none) and, with ``candidates``, their slots in the candidate scratch (else None); inputs int32."""
+    _dev(positions)
+    for t in (positions, row_prompt, row_cand, row_len):
+        _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() * (1 if t is positions else T) == positions.numel(), "block_slots: contiguous int32 [R*T] positions, [R] rows")
+    out = torch.empty((2 if candidates else 1, positions.numel()), dtype=torch.int64, device=positions.device)
+    N.check_layers(N.layers().jl_block_slots(positions.data_ptr(), row_prompt.data_ptr(), row_cand.data_ptr(), row_len.data_ptr(), row_len.numel(), T, S_max, T_max, out[0].data_ptr(),
+                                             out[1].data_ptr() if candidates else None, _stream(positions.device)), "jl_block_slots")
+    return out[0], out[1] if candidates else None
+
+
+def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len: torch.Tensor, row_len: torch.Tensor, max_keys: int, row_prompt: Optional[torch.Tensor] = None,
+               tables: Optional[torch.Tensor] = None, row_cand: Optional[torch.Tensor] = None, ck: Optional[torch.Tensor] = None, cv: Optional[torch.Tensor] = None,
+               scale: Optional[float] = None) -> torch.Tensor:
+    """Attention of a draft block: q [R, nkv, G*T, D] over k, v [blocks, nkv, page, D].  Token t of row r sees the row's first kv_len[r] keys and the block's tokens up to
+    min(t, row_len[r] - 1), at most ``max_keys`` in all: in cache row row_prompt[r], or in the blocks tables[r] lists; with ``ck`` / ``cv`` [rows, nkv, T_max, D], rows whose row_cand is
+    not negative have the block's keys there.  Integers int32.  Returns [R*T, nkv*G*D]."""
+    _dev(q)
+    R, nkv, GT, D = q.shape
+    G = GT // T
+    for t in (q, k, v) + ((ck, cv) if ck is not None else ()):
+        _need(t.is_contiguous() and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[1] == nkv and t.shape[3] == D, "attn_block: contiguous bfloat16 [., nkv, ., D]")
+    for t in (kv_len, row_len) + ((row_prompt,) if tables is None else ()) + ((row_cand,) if ck is not None else ()):
+        _need(t is not None and t.dtype == torch.int32 and t.numel() == R and t.is_contiguous(), "attn_block: int32 [R] lengths and rows")
+    _need(GT == G * T and k.shape == v.shape and (tables is None or (tables.dtype == torch.int32 and tables.dim() == 2 and tables.shape[0] == R and tables.stride(1) == 1)) and
+          (ck is None or (ck.shape == cv.shape and ck.shape[2] >= T)), "attn_block: shapes")
+    out = torch.empty((R * T, nkv * G * D), dtype=q.dtype, device=q.device)
+    max_keys = min(int(max_keys), k.shape[2] * (1 if tables is None else tables.shape[1]))
+    groups = R * nkv * -(-GT // 128)
+    splits = max(1, min(BLOCK_WORKGROUPS // max(1, groups), -(-max_keys // 128), 32))
+    scratch = None
+    if splits > 1:
+        scratch = torch.empty((int(N.layers().jl_attn_block_scratch_floats(R, T, nkv, G, D, splits)),), dtype=torch.float32, device=q.device)
+    a = N.BlockArgs(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), ck=_ptr(ck), cv=_ptr(cv), kv_len=kv_len.data_ptr(), row_len=row_len.data_ptr(),
+                    row_prompt=row_prompt.data_ptr() if tables is None else None, row_cand=row_cand.data_ptr() if ck is not None else None, tables=_ptr(tables), out=out.data_ptr(),
+                    scratch=_ptr(scratch), table_ld=tables.stride(0) if tables is not None else 0, R=R, T=T, nkv=nkv, G=G, D=D, blocks=k.shape[0], page_size=k.shape[2],
+                    table_cols=tables.shape[1] if tables is not None else 0, cand_rows=ck.shape[0] if ck is not None else 0, cand_max=ck.shape[2] if ck is not None else 0,
+                    max_keys=max_keys, splits=splits, scale=D ** -0.5 if scale is None else float(scale))
+    N.check_layers(N.layers().jl_attn_block(C.byref(a), _stream(q.device)), "jl_attn_block")
     return out
 
 

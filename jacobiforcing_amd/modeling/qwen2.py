@@ -25,6 +25,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from .. import layer_ops as LO
 from .. import ops
 
 
@@ -290,14 +291,15 @@ class Qwen2Model:
         PAGED layout (``Config.kv_cache_layout = "paged"``, the reference's cache: layers/attention.py:10-40, MR:1204-1265): ``cache`` is a
         pool ``[num_blocks, H_kv, block_size, D]`` per layer (a StaticKVCache whose "rows" are blocks), ``paged_slots`` [R*T] the slot of
         every new token (block * block_size + offset, -1 = padding: jf_engine_fill's slot_mapping) and ``block_tables`` [R, C] the blocks
-        of each row in order (-1 = none).  The append is the same launch; a row's keys are its blocks gathered in table order (stock
-        SDPA has no block-table argument; flash_attn_with_kvcache is not in this image), so logical key index = position."""
+        of each row in order (-1 = none).  The append is the same launch; logical key index = position.
+
+        bfloat16 on the GPU goes through the package's attention kernel (layer_ops.attn_block), which reads lengths, cache rows, blocks and candidate scratch itself; anything else
+        (32-bit weights, the CPU) through torch's attention over a mask and gathered prefixes / blocks."""
         cfg, w = self.cfg, self.w
         R, T = input_ids.shape
         nq, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         G = nq // nkv
         dev = self.device
-        pos = positions.long()
         if s_cur is None:
             s_cur = (int(kv_len_rows.max().item()) + T) if R else T
         paged = block_tables is not None
@@ -305,10 +307,14 @@ class Qwen2Model:
         S_cur = min(int(s_cur), S_cap)
         if self.cos.shape[0] < S_cap:                        # a cache longer than max_position_embeddings: never read past the table
             self._rope_tables(S_cap)
+        if R and T and LO.attn_block_ok(self.dtype, dev, hd):    # lengths, cache rows, pages and candidate scratch are read by the attention kernel itself
+            return self._forward_native(input_ids, positions, cache, row_prompt, row_cand, row_len, kv_len_rows, any_candidates or (n_main is not None and R > int(n_main)), S_cur,
+                                        paged, paged_slots, block_tables, n_main, logits_rows, logit_index)
+        pos = positions.long()
         ar_t = torch.arange(T, device=dev)
-        ar_s = torch.arange(S_cur, device=dev)
         kvl = kv_len_rows.long()
         rlen = row_len.long()
+        ar_s = torch.arange(S_cur, device=dev)
         rel = ar_s.view(1, 1, S_cur) - kvl.view(R, 1, 1)                            # key index relative to the new block
         mask = (rel < 0) | ((rel <= ar_t.view(1, T, 1)) & (rel < rlen.view(R, 1, 1)))
         mask = mask.view(R, 1, 1, T, S_cur).expand(R, 1, G, T, S_cur).reshape(R, 1, G * T, S_cur)
@@ -397,9 +403,37 @@ class Qwen2Model:
             o = o.view(R, nkv, G, T, hd).permute(0, 3, 1, 2, 4).reshape(R * T, nq * hd)
             x.addmm_(o, L["wo"].t())                                                  # residual in the GEMM epilogue, in place
             x = self._mlp_residual(L, x, self._norm(x, L["ln2"]))
-        flat = self._norm(x, w.norm)
+        return self._head(x, logits_rows, logit_index)
+
+    def _head(self, x: torch.Tensor, logits_rows: Optional[slice], logit_index: Optional[torch.Tensor]) -> torch.Tensor:
+        flat = self._norm(x, self.w.norm)
         if logits_rows is not None:
             flat = flat[logits_rows]
         if logit_index is not None:
             flat = flat.index_select(0, logit_index.clamp(min=0).long())
-        return F.linear(flat, w.lm_head)
+        return F.linear(flat, self.w.lm_head)
+
+    def _forward_native(self, input_ids, positions, cache, row_prompt, row_cand, row_len, kv_len_rows, candidates, S_cur, paged, paged_slots, block_tables, n_main, logits_rows,
+                        logit_index) -> torch.Tensor:
+        """``forward`` on the package's attention kernel: no mask, no gathered prefixes, no copy of the outputs."""
+        cfg, w = self.cfg, self.w
+        R, T = input_ids.shape
+        nq, nkv, hd = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        i32 = lambda t: t.to(torch.int32).contiguous()
+        pos32, kv, lens, prompts, cands = i32(positions).reshape(-1), i32(kv_len_rows), i32(row_len), i32(row_prompt), i32(row_cand)
+        slot_cand = tables = None
+        if paged:
+            if candidates or n_main is not None:
+                raise NotImplementedError("candidate rows over the paged layout (the engine's decoders are single-block: MR:1468-1473)")
+            slot_main, tables = paged_slots.long().reshape(-1), block_tables.to(torch.int32)
+        else:
+            slot_main, slot_cand = LO.block_slots(pos32, T, prompts, cands, lens, cache.S_max, cache.T_max, bool(candidates))
+        x = w.embed[input_ids].view(R * T, cfg.hidden_size)
+        for li, L in enumerate(w.layers):
+            qkv = F.linear(self._norm(x, L["ln1"]), L["wqkv"], L["bqkv"])
+            ck, cv = (cache.ck[li], cache.cv[li]) if candidates else (None, None)
+            qh = ops.rope_kv_append(qkv, T, nq, nkv, hd, pos32, self.cos, self.sin, cache.k[li], cache.v[li], slot_main, ck, cv, slot_cand)
+            o = LO.attn_block(qh, T, cache.k[li], cache.v[li], kv, lens, S_cur, prompts, tables, cands, ck, cv)
+            x.addmm_(o, L["wo"].t())
+            x = self._mlp_residual(L, x, self._norm(x, L["ln2"]))
+        return self._head(x, logits_rows, logit_index)

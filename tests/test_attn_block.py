@@ -1,0 +1,68 @@
+"""Attention of draft blocks at the edges of its tiles (64 keys, 128 (head, token) rows, shared-out keys), over cache rows, pages and candidate scratch, against 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,T,nkv,G,D,kv,lens,kind,wgs", [
+    (3, 32, 2, 4, 128, [512, 63, 0], [32, 7, 32], "rows", 384), (2, 16, 2, 7, 64, [64, 1000], [16, 16], "rows", 1), (5, 5, 1, 3, 72, [0, 1, 130, 64, 200], [5, 0, 3, 5, 1], "cand", 384),
+    (1, 64, 2, 8, 128, [777], [64], "rows", 384), (4, 33, 3, 1, 8, [100, 31, 32, 33], [33, 30, 33, 2], "pages", 384), (2, 1, 2, 16, 96, [300, 15], [1, 1], "pages", 1),
+    (6, 32, 2, 4, 128, [250] * 6, [32, 32, 20, 1, 32, 9], "cand", 1),
+])
+def test_block(monkeypatch, R, T, nkv, G, D, kv, lens, kind, wgs):
+    from jacobiforcing_amd import layer_ops as LO
+    dev = "cuda"
+    monkeypatch.setattr(LO, "BLOCK_WORKGROUPS", wgs)
+    g = torch.Generator(device=dev).manual_seed(R * T + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    q = rnd(R, nkv, G * T, D)
+    longest = max(a + b for a, b in zip(kv, lens))
+    if kind == "pages":
+        page = 16
+        cols = -(-longest // page)
+        order = torch.randperm(R * cols, generator=torch.Generator().manual_seed(3)).view(R, cols)
+        k, v = rnd(R * cols, nkv, page, D), rnd(R * cols, nkv, page, D)
+        tables = i32([[int(order[r, c]) if c * page < kv[r] + lens[r] else -1 for c in range(cols)] for r in range(R)])
+        out = LO.attn_block(q, T, k, v, i32(kv), i32(lens), longest, tables=tables)
+        key = lambda x, r: torch.cat([x[order[r, c]] for c in range(cols)], 1)
+    else:
+        P = R + 1
+        k, v = rnd(P, nkv, longest + 3, D), rnd(P, nkv, longest + 3, D)
+        prompt = [(2 * r + 1) % P for r in range(R)]
+        cand = [r // 2 if kind == "cand" and r % 2 else -1 for r in range(R)]
+        ck, cv = (rnd(R, nkv, T + 4, D), rnd(R, nkv, T + 4, D)) if kind == "cand" else (None, None)
+        out = LO.attn_block(q, T, k, v, i32(kv), i32(lens), longest, i32(prompt), None, i32(cand), ck, cv)
+
+        def key(x, r):
+            row = x[prompt[r]].clone()
+            if cand[r] >= 0:
+                row[:, kv[r]:kv[r] + lens[r]] = (ck if x is k else cv)[cand[r], :, :lens[r]]
+            return row
+    out = out.double().view(R, T, nkv, G, D)
+    for r in range(R):
+        n = kv[r] + lens[r]
+        kk, vv = key(k, r).double()[:, :n], key(v, r).double()[:, :n]
+        s = (q[r].double().view(nkv, G * T, D) @ kk.transpose(1, 2).contiguous() * D ** -0.5).view(nkv, G, T, n)
+        t, j = torch.arange(T, device=dev).view(T, 1), torch.arange(n, device=dev).view(1, n)
+        see = (j < kv[r]) | (j - kv[r] <= t)
+        want = torch.softmax(s.masked_fill(~see, float("-inf")), -1).view(nkv, G * T, n) @ vv if n else torch.zeros(nkv, G * T, D, dtype=torch.float64, device=dev)
+        want = want.view(nkv, G, T, D).permute(2, 0, 1, 3)
+        err = (out[r] - want).abs().max().item()
+        # weights and outputs are rounded to bfloat16 (2 ** -9 each of values up to 4 or so), scores keep a few 2 ** -24 of their size
+        assert err <= 4 * 2.0 ** -8 * max(1.0, want.abs().max().item() / 4), (r, err)
+
+
+@pytest.mark.parametrize("R,T,candidates", [(1, 1, False), (5, 33, True), (64, 32, True), (3, 200, False)])
+def test_slots(R, T, candidates):
+    from jacobiforcing_amd import layer_ops as LO
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(R)
+    i32 = lambda lo, hi, *s: torch.randint(lo, hi, s, generator=g, device=dev, dtype=torch.int32)
+    pos, prompt, cand, lens = i32(0, 3000, R * T), i32(0, 60000, R), i32(-2, 4, R), i32(0, T + 1, R)
+    main, scratch = LO.block_slots(pos, T, prompt, cand, lens, 70000, T + 3, candidates)       # beyond 32 bits
+    t, valid = torch.arange(T, device=dev).view(1, T), torch.arange(T, device=dev).view(1, T) < lens.view(R, 1)
+    neg = torch.full((), -1, dtype=torch.int64, device=dev)
+    assert torch.equal(main.view(R, T), torch.where(valid & (cand < 0).view(R, 1), prompt.long().view(R, 1) * 70000 + pos.view(R, T), neg))
+    assert scratch is None if not candidates else torch.equal(scratch.view(R, T), torch.where(valid & (cand >= 0).view(R, 1), cand.long().view(R, 1) * (T + 3) + t, neg))
