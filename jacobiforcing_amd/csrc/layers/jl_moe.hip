@@ -175,15 +175,16 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *__restri
 }
 
 // Rows of a tile.  High tiles read the weights less often and do more per byte of LDS, low ones pad less, give more workgroups and overlap their starts and ends.
-// 128 rows need both products to fill the chip and enough depth to pay for a tile's start; 64 need as many blocks as the chip takes at once.  Measured, experts
-// alone, bfloat16, us at 32 / 64 / 128 rows: 8 192 tokens x 4 of 32 (2048 x 1024) 1333 / 841 / 706; 512 tokens 163 / 159 / 156; 256 tokens 120 / 128 / 142;
-// 4 096 x 4 of 16 (1024 x 512) 227 / 141 / 168; 512 tokens 59 / 60 / 86; 1 024 x 4 of 8 (1024 x 2048) 216 / 146 / 169; float, 2 048 x 4 of 16: 418 / 356 / 432.
+// 128 rows need both products to fill the chip and about a tile of rows per expert; 64 need as many blocks as the chip takes at once.  Measured, experts alone, gated,
+// bfloat16, us at 32 / 64 / 128 rows: 8192 tokens x 4 of 32 (2048 x 1024) 1059 / 790 / 623, 1024 tokens 213 / 171 / 160, 512 tokens 147 / 140 / 155, 256 tokens 121 / 124 / 142;
+// 4096 x 4 of 16 (1024 x 512) 180 / 135 / 123, 1024 tokens 75 / 66 / 79, 512 tokens 51 / 57 / 77; 4096 x 4 of 12 (768 x 512) 151 / 117 / 104, 2048 tokens 95 / 77 / 80;
+// float, 2048 x 4 of 16 (1024 x 512): 341 / 311 / 401.
 // Sizes the matrix-core product does not take (rows that do not start at 16-byte borders) go in tiles of MOE_TM.
 static bool moe_mm_sizes(int dtype, int64_t K) { return (dtype == JL_BF16 && K % 8 == 0) || (dtype == JL_F32 && K % 4 == 0); }
 extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff) {
     if (E <= 0 || !moe_mm_sizes(dtype, W) || !moe_mm_sizes(dtype, ff)) return MOE_TM;
     auto blocks = [&](int tm, int width, int tn) { return (rows / tm + E / 2) * ((width + tn - 1) / tn); };
-    if (dtype == JL_BF16 && W + ff >= 3072 && blocks(128, ff, 128) >= 256 && blocks(128, W, 256) >= 256 && rows >= (int64_t)48 * E) return 128;
+    if (dtype == JL_BF16 && blocks(128, ff, 128) >= 256 && blocks(128, W, 256) >= 256 && rows >= (int64_t)96 * E) return 128;
     return rows >= (int64_t)48 * E && blocks(64, ff, 128) + blocks(64, W, 256) >= 512 ? 64 : 32;
 }
 
@@ -282,12 +283,14 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
 // products rounded one by one, as a chain of multiply-adds is).  Units of a row are permuted so that 16 neighbouring rows meet different banks.
 // GATED: the WR weight rows are WR / 2 of the gate and the WR / 2 of the linear branch that belong to them (rows n_out further on); both products
 // of a column end in the same lane, which stores the gated unit.
-// TM = 128 (an expert has about a hundred rows or more) is bound by the matrix cores and LDS: 128 x 256 reads 48 KB of LDS per 64 products, so two
-// workgroups fit a CU and cover each other's barriers.  Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an
-// expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading the weights: single wavefronts, many per CU, 12 KB on the way each.
+// TM = 128 (an expert has about a hundred rows or more) is bound by the matrix cores and LDS: 128 x 256 reads 48 KB of LDS per 64 products.  Rows go from memory straight into LDS
+// (16 bytes per lane, every lane fetching the unit that the permutation puts into its place), one stage ahead: no registers and no LDS writes for them, so that three workgroups fit a
+// CU and cover each other's barriers (through registers, two of them: gated product at 8192 x 4 of 32 experts of 2048 x 1024 406 -> 363 us, the way down 290 -> 252).
+// Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading
+// the weights: single wavefronts, many per CU, 12 KB on the way each, in registers.
 // Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from one base, rows that do not exist repeat another, stages behind the last repeat the
-// first, depths beyond the last whole stage come after the loop (a condition per load had cost six vector instructions per product, 431 us instead of 406 for the gated
-// product at 8192 x 4 of 32 experts of 2048 x 1024; us for up and down at 32 rows x 4 of 16 of 1024 x 512: 49 -> 41, float 16 rows 100 -> 79, 400 rows 53 -> 45).
+// first, depths beyond the last whole stage come after the loop (a condition per load had cost six vector instructions per product: 431 us instead of 406 for the gated product
+// above; us for up and down at 32 rows x 4 of 16 of 1024 x 512: 49 -> 41, float 16 rows 100 -> 79, 400 rows 53 -> 45).
 struct MoeMM {
     const void *X, *Wt;
     const int32_t *perm, *offsets, *tile_expert, *tile_row0;
@@ -316,8 +319,13 @@ template <> struct mm_type<float> {
     }
 };
 
+// 16 bytes per lane from base + off into LDS at `lds` + 16 * lane (`base`, `lds` the same for the wavefront); the caller waits for vmcnt before the barrier that publishes them
+__device__ __forceinline__ void mm_load_lds(const char *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+
 template <typename T, int TM, int NW, int WR, int TKU, bool GATED>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM a) {
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM a) {
     constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
     constexpr int XPF = TM * TKU / THREADS, WPF = WR * TKU / THREADS, TN = GATED ? WR / 2 : WR, STAGE = TKU * UNIT;
     static_assert(XPF * THREADS == TM * TKU && WPF * THREADS == WR * TKU && (!GATED || NT % 2 == 0), "tile");
@@ -340,21 +348,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave / WN, wn = wave % WN;
     auto at = [](int row, int u) { return row * TKU + (u ^ (TKU == 4 ? (row >> 2) & 3 : (row >> 1) & 7)); };
     // loaders: unit tid % TKU of rows tid / TKU + x * THREADS / TKU; a row that does not exist repeats another and is not stored
-    const int lu = tid % TKU, lr = tid / TKU;
+    const int lr = tid / TKU;
+    constexpr bool DMA = NW > 1;
+    auto unit_of = [&](int x) { return DMA ? at(lr + x * (THREADS / TKU), tid % TKU) % TKU : tid % TKU; };      // DMA: what belongs into this thread's place of LDS
     // byte offsets from a base that is the same for all lanes: a load is one instruction (the launch has checked that 32 bits hold them)
     uint32_t xo[XPF], wo[WPF];
 #pragma unroll
     for (int x = 0; x < XPF; ++x) {
         const int m = lr + x * (THREADS / TKU), row = r0 + (m < nr ? m : 0);
-        xo[x] = (uint32_t)((a.mode != 1 ? a.perm[row] / a.top : row) * (int64_t)K + lu * UNIT) * sizeof(T);
+        xo[x] = (uint32_t)((a.mode != 1 ? a.perm[row] / a.top : row) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
     }
     const char *Xb = (const char *)a.X, *Wb = (const char *)((const T *)a.Wt + (int64_t)e * (GATED ? 2 : 1) * n_out * K);
 #pragma unroll
     for (int x = 0; x < WPF; ++x) {
         const int j = lr + x * (THREADS / TKU), c = n0 + (GATED ? j % TN : j);
-        wo[x] = (uint32_t)(((GATED && j >= TN ? n_out : 0) + (c < n_out ? c : n_out - 1)) * (int64_t)K + lu * UNIT) * sizeof(T);
+        wo[x] = (uint32_t)(((GATED && j >= TN ? n_out : 0) + (c < n_out ? c : n_out - 1)) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
     }
-    mm_u32x4 reg[2][XPF + WPF];                                     // stages on their way: even ones in reg[0], odd ones in reg[1]
+    mm_u32x4 reg[DMA ? 1 : 2][XPF + WPF];                                     // stages on their way: even ones in reg[0], odd ones in reg[1]
     const int full = K / STAGE;                                     // whole stages; what is left of K comes last
     auto fetch = [&](mm_u32x4 (&r)[XPF + WPF], int i) {             // without branches: behind the last stage, stage 0 again (never used)
         const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
@@ -367,9 +377,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM 
     auto stash = [&](const mm_u32x4 (&r)[XPF + WPF], int sel) {
         uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
 #pragma unroll
-        for (int x = 0; x < XPF; ++x) Xs[at(lr + x * (THREADS / TKU), lu)] = __builtin_bit_cast(uint4, r[x]);
+        for (int x = 0; x < XPF; ++x) Xs[at(lr + x * (THREADS / TKU), unit_of(x))] = __builtin_bit_cast(uint4, r[x]);
 #pragma unroll
-        for (int x = 0; x < WPF; ++x) Ws[at(lr + x * (THREADS / TKU), lu)] = __builtin_bit_cast(uint4, r[XPF + x]);
+        for (int x = 0; x < WPF; ++x) Ws[at(lr + x * (THREADS / TKU), unit_of(x))] = __builtin_bit_cast(uint4, r[XPF + x]);
     };
     mm_f32x16 acc[XT][NT];
 #pragma unroll
@@ -390,26 +400,59 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM 
             for (int x = 0; x < XT; ++x) xf[x] = Xs[at(wm * (TM / WM) + 32 * x + l32, 2 * s + hi)];
 #pragma unroll
             for (int t = 0; t < NT; ++t) wf[t] = Ws[at(w_row(t) + l32, 2 * s + hi)];
+
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int x = 0; x < XT; ++x) acc[x][t] = mm_type<T>::mma(wf[t], xf[x], acc[x][t]);
+
         }
     };
     std::integral_constant<int, 0> even;
     std::integral_constant<int, 1> odd;
-    if (full > 0) {
+    if (DMA && full > 0) {
+        // straight into LDS: a wavefront's 64 places of 16 bytes per load, one stage ahead
+        const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(smem + wave * 64));
+        auto issue = [&](int i, int sel) {
+            const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
+            const uint32_t dst = lds + sel * (TM + WR) * TKU * 16;
+#pragma unroll
+            for (int x = 0; x < XPF; ++x) mm_load_lds(Xb + k, xo[x], dst + x * THREADS * 16);
+#pragma unroll
+            for (int x = 0; x < WPF; ++x) mm_load_lds(Wb + k, wo[x], dst + (XPF + x) * THREADS * 16);
+        };
+        auto arrived = [&]() {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        };
+        issue(0, 0);
+        int i = 0;
+        for (; i + 1 < full; i += 2) {
+            arrived();
+            issue(i + 1, 1);
+            products(even);
+            arrived();
+            issue(i + 2, 0);
+            products(odd);
+        }
+        arrived();
+        if (i < full) {
+            products(even);
+            __syncthreads();
+        }
+    } else if (full > 0) {
         fetch(reg[0], 0);
-        fetch(reg[1], 1);
+        constexpr int R1 = DMA ? 0 : 1;
+        fetch(reg[R1], 1);
         stash(reg[0], 0);
         __syncthreads();
         int i = 0;
         for (; i + 1 < full; i += 2) {                              // two stages ahead: a trip to memory takes longer than one stage's products
             fetch(reg[0], i + 2);
             products(even);
-            stash(reg[1], 1);
+            stash(reg[R1], 1);
             __syncthreads();
-            fetch(reg[1], i + 3);
+            fetch(reg[R1], i + 3);
             products(odd);
             stash(reg[0], 0);
             __syncthreads();
@@ -420,13 +463,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void moe_mm_kernel(MoeMM 
         }
     }
     if (full * STAGE < K) {                                         // depths beyond K are zero
-        const bool in = full * STAGE + lu * UNIT < K;
-        const int64_t k = in ? (int64_t)full * STAGE * sizeof(T) : -(int64_t)(lu * UNIT * sizeof(T));      // a lane beyond K reads its row's first unit: a row may be shorter than a stage
         const mm_u32x4 zero = {0, 0, 0, 0};
+        auto last = [&](const char *base, uint32_t off, int u) {    // a lane beyond K reads its row's first unit: a row may be shorter than a stage
+            const bool in = full * STAGE + u * UNIT < K;
+            const mm_u32x4 v = *(const mm_u32x4 *)(base + off + (in ? (int64_t)full * STAGE * sizeof(T) : -(int64_t)(u * UNIT * sizeof(T))));
+            return in ? v : zero;
+        };
 #pragma unroll
-        for (int x = 0; x < XPF; ++x) { const mm_u32x4 v = *(const mm_u32x4 *)(Xb + xo[x] + k); reg[0][x] = in ? v : zero; }
+        for (int x = 0; x < XPF; ++x) reg[0][x] = last(Xb, xo[x], unit_of(x));
 #pragma unroll
-        for (int x = 0; x < WPF; ++x) { const mm_u32x4 v = *(const mm_u32x4 *)(Wb + wo[x] + k); reg[0][XPF + x] = in ? v : zero; }
+        for (int x = 0; x < WPF; ++x) reg[0][XPF + x] = last(Wb, wo[x], unit_of(x));
         stash(reg[0], 0);
         __syncthreads();
         products(even);
