@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 133
+#define JL_VERSION 134
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -207,6 +207,9 @@ JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_re
 #define JL_LINEAR_ROUNDED_FLOAT 2
 JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                            int32_t out_mode, void *stream);
+/* The same for more rows (a few hundred), W of x's type, the result at a 16-byte border, operands of up to 4 GB. */
+JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
+                         void *stream);
 
 /* z <- cap * tanh(z / cap) in place over `total` floats (soft cap of the logits). */
 JL_API int jl_softcap(float *z, int64_t total, float cap, void *stream);

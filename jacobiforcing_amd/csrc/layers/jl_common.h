@@ -97,6 +97,12 @@ __device__ __forceinline__ float gated_unit_f(float g, float u, int kind, float 
     return g * sigmoid_f<FAST>(alpha * g) * (u + shift);
 }
 
+// 16 bytes per lane from base + off into LDS at `lds` + 16 * lane (`base`, `lds` the same for the wavefront).  The compiler does not count these loads: the caller waits for vmcnt
+// before the barrier that publishes them, and before the workgroup ends
+__device__ __forceinline__ void jl_load_lds(const char *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+
 #define JL_DISPATCH(dtype, ...)                                   \
     do {                                                          \
         if ((dtype) == JL_BF16) { typedef bf16_t T; __VA_ARGS__; } \

@@ -115,6 +115,129 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 #undef LS_LAUNCH
 }
 
+// ---- a few hundred rows: 64 of x by 64 of W per workgroup ---------------------------------------------------------------------------------------
+// Stages of 128 bytes of every row go from memory straight into a ring of three buffers in LDS (16 bytes per lane, every lane fetching the unit that the permutation puts into its
+// place), two stages ahead of the products; four wavefronts hold a 32 x 32 quarter each, W's rows are the A operand, so that a lane ends with four neighbouring columns of a row.
+// What bounds it: a workgroup's way through its stages, 0.27 us each however many workgroups there are, until two per CU are busy.  us of GPU time against the library's product
+// (bfloat16, W from memory): 1024 x 1024 by 256 rows 7.8 / 8.3, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 520 x 1000 by 1024 7.0 / 10.1, by 1600 10.0 / 12.0; 192 x 768 by 1600 5.4 / 5.9;
+// 1024 x 3072 by 256 8.3 / 9.0; and 11 us less of host time.  Beyond the caller's line (layer_ops.linear_mid) it loses: 2048 x 2048 by 512 13.3 / 11.2, 1024 x 3072 by 1024 16.1 / 13.6, float
+// 1024 x 1024 by 512 22.5 / 12.7.  Larger tiles and deeper rings gained nothing there (128 x 128 by 8192 rows 100 / 52), nor did a share of the depth per wavefront without barriers.
+typedef float ld_f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ ld_f32x16 ld_mma(const bf16_t *, uint4 a, uint4 b, ld_f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ls_bf16x8, a), __builtin_bit_cast(ls_bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ ld_f32x16 ld_mma(const float *, uint4 a, uint4 b, ld_f32x16 c) {
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+}
+constexpr int LD_RING = 3, LD_UNITS = 8, LD_TILE = 64;              // 16-byte units of a row per stage
+
+template <typename T>
+__global__ __launch_bounds__(256) void linear_mid_kernel(const T *__restrict__ x, int64_t x_ld, const T *__restrict__ w, const T *__restrict__ bias, void *__restrict__ out, int64_t out_ld,
+                                                         int N, int K, int O, int out_mode, int row_tiles) {
+    constexpr int UNIT = 16 / sizeof(T), STAGE = LD_UNITS * UNIT, BUF = 2 * LD_TILE * LD_UNITS;
+    __shared__ uint4 ldS[LD_RING * BUF];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    const int n0 = blockIdx.x % row_tiles * LD_TILE, o0 = blockIdx.x / row_tiles * LD_TILE;      // neighbouring workgroups share W's rows
+    auto at = [](int row, int u) { return row * LD_UNITS + (u ^ (row & 7)); };
+    const int lr = tid / LD_UNITS, lu = (tid % LD_UNITS) ^ (lr & 7);   // the unit whose place in LDS is this thread's (rows step by 32: the permutation is the same)
+    uint32_t xo[2], wo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {                                   // rows that do not exist repeat the last one
+        const int n = n0 + lr + 32 * i, o = o0 + lr + 32 * i;
+        xo[i] = (uint32_t)((n < N ? n : N - 1) * x_ld + lu * UNIT) * sizeof(T);
+        wo[i] = (uint32_t)((o < O ? o : O - 1) * (int64_t)K + lu * UNIT) * sizeof(T);
+    }
+    const char *xb = (const char *)x, *wb = (const char *)w;
+    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(ldS + wave * 64));
+    const int full = K / STAGE;
+    auto issue = [&](int s, int sel) {                              // behind the last stage, stage 0 again (never used): the number of loads on their way stays the same
+        const int64_t k = s < full ? (int64_t)s * 128 : 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) jl_load_lds(xb + k, xo[i], lds + (sel * BUF + i * 256) * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) jl_load_lds(wb + k, wo[i], lds + (sel * BUF + (2 + i) * 256) * 16);
+    };
+    ld_f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    auto products = [&](const uint4 *Xs) {
+        const uint4 *Ws = Xs + LD_TILE * LD_UNITS;
+#pragma unroll
+        for (int s = 0; s < LD_UNITS / 2; ++s) acc = ld_mma((const T *)nullptr, Ws[at(32 * wn + l32, 2 * s + hi)], Xs[at(32 * wm + l32, 2 * s + hi)], acc);
+    };
+    if (full > 0) {
+#pragma unroll
+        for (int s = 0; s < LD_RING - 1; ++s) issue(s, s);
+        int sel = 0;
+        for (int s = 0; s < full; ++s) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LD_RING - 2) * 4) : "memory");
+            __syncthreads();                                        // stage s is there for everybody, stage s - 1 has been read
+            issue(s + LD_RING - 1, sel == 0 ? LD_RING - 1 : sel - 1);
+            products(ldS + sel * BUF);
+            sel = sel == LD_RING - 1 ? 0 : sel + 1;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    if (full * STAGE < K) {                                         // depths beyond K are zero; a lane beyond K reads its row's first unit: a row may be shorter than a stage
+        const bool in = full * STAGE + lu * UNIT < K;
+        const int64_t k = in ? (int64_t)full * 128 : -(int64_t)lu * 16;
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const u32x4 v = *(const u32x4 *)(xb + xo[i] + k), u = *(const u32x4 *)(wb + wo[i] + k);
+            ldS[i * 256 + tid] = __builtin_bit_cast(uint4, in ? v : zero);
+            ldS[(2 + i) * 256 + tid] = __builtin_bit_cast(uint4, in ? u : zero);
+        }
+        __syncthreads();
+        products(ldS);
+    }
+    const int n = n0 + 32 * wm + l32;
+    if (n >= N) return;
+    const bool whole = O % 4 == 0 && out_ld % 4 == 0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int o = o0 + 32 * wn + 8 * g + 4 * hi;                // four neighbouring columns
+        if (o >= O) continue;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[4 * g + e] + (bias && o + e < O ? ld_f(bias + o + e) : 0.f);
+        if (out_mode == JL_LINEAR_ROUNDED_FLOAT)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { T r; st_f(&r, v[e]); v[e] = ld_f(&r); }
+        if (out_mode == JL_LINEAR_SAME) {
+            T *p = (T *)out + n * out_ld + o;
+            if (whole) st4_f(p, v);
+            else for (int e = 0; e < 4 && o + e < O; ++e) st_f(p + e, v[e]);
+        } else {
+            float *p = (float *)out + n * out_ld + o;
+            if (whole) st4_f(p, v);
+            else for (int e = 0; e < 4 && o + e < O; ++e) p[e] = v[e];
+        }
+    }
+}
+
+extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
+                             void *stream) {
+    if (N <= 0 || O <= 0) return JL_OK;
+    if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < O) return jl_fail(JL_E_INVALID, "jl_linear_mid: null pointer or bad sizes");
+    const int64_t unit = dtype == JL_BF16 ? 8 : 4, size = 16 / unit;
+    if ((dtype != JL_BF16 && dtype != JL_F32) || K % unit || x_ld % unit || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15))
+        return jl_fail(JL_E_INVALID, "jl_linear_mid: rows of x and W and the result at 16-byte borders");
+    if (N > INT32_MAX / 64 || N * x_ld * size > UINT32_MAX || (int64_t)O * K * size > UINT32_MAX) return jl_fail(JL_E_INVALID, "jl_linear_mid: operands of up to 4 GB");
+    if (out_mode < JL_LINEAR_SAME || out_mode > JL_LINEAR_ROUNDED_FLOAT) return jl_fail(JL_E_INVALID, "jl_linear_mid: unknown out_mode");
+    const int row_tiles = (int)((N + LD_TILE - 1) / LD_TILE);
+    const int64_t groups = (int64_t)row_tiles * ((O + LD_TILE - 1) / LD_TILE);
+    if (groups > INT32_MAX / 256) return jl_fail(JL_E_INVALID, "jl_linear_mid: too many tiles");
+    JL_DISPATCH(dtype, linear_mid_kernel<T><<<dim3((unsigned)groups), 256, 0, (hipStream_t)stream>>>((const T *)x, x_ld, (const T *)w, (const T *)bias, out, out_ld, (int)N, K, O, out_mode,
+                                                                                                    row_tiles));
+    return jl_check_launch("linear_mid_kernel");
+}
+
 extern "C" int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                                int32_t out_mode, void *stream) {
     if (N <= 0 || O <= 0) return JL_OK;

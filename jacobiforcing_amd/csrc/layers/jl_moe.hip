@@ -319,11 +319,6 @@ template <> struct mm_type<float> {
     }
 };
 
-// 16 bytes per lane from base + off into LDS at `lds` + 16 * lane (`base`, `lds` the same for the wavefront); the caller waits for vmcnt before the barrier that publishes them
-__device__ __forceinline__ void mm_load_lds(const char *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-
 template <typename T, int TM, int NW, int WR, int TKU, bool GATED>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM a) {
     constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
@@ -417,9 +412,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
             const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
             const uint32_t dst = lds + sel * (TM + WR) * TKU * 16;
 #pragma unroll
-            for (int x = 0; x < XPF; ++x) mm_load_lds(Xb + k, xo[x], dst + x * THREADS * 16);
+            for (int x = 0; x < XPF; ++x) jl_load_lds(Xb + k, xo[x], dst + x * THREADS * 16);
 #pragma unroll
-            for (int x = 0; x < WPF; ++x) mm_load_lds(Wb + k, wo[x], dst + (XPF + x) * THREADS * 16);
+            for (int x = 0; x < WPF; ++x) jl_load_lds(Wb + k, wo[x], dst + (XPF + x) * THREADS * 16);
         };
         auto arrived = [&]() {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

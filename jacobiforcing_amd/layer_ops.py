@@ -228,20 +228,33 @@ def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
     return 0 < n <= LINEAR_SMALL_ROWS and n * k * itemsize * -(-o // (tile * 256)) <= LINEAR_X_BYTES
 
 
+def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
+    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for a few hundred rows: 16-bit rows of up to 2 KB and no more than two 64 x 64 tiles per CU.  There its GPU
+    time is the library's give or take 2 us (1024 x 1024 by 128 rows 7.6 / 5.4, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4), and the call costs 11 us less of the host."""
+    return dtype == torch.bfloat16 and n > 0 and k <= 1024 and -(-n // 64) * -(-o // 64) <= 512
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:
-    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launch for few rows (decoding, ``linear_small``), the library's product for more.
-    ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then counts as
-    float: give ``float_out`` True."""
+    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``) and a few hundred (``linear_mid``), the library's product
+    for more.  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
+    counts as float: give ``float_out`` True."""
     _dev(x)
     n, k = x.shape
     o, size = w.shape[0], w.element_size()
     _need(w.dtype == x.dtype or (w.dtype == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
-    if n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, size) and w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and \
-            (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous())):
+    small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, size)
+    if ((small or (w.dtype == x.dtype and linear_mid(n, k, o, x.dtype))) and w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and
+            x.stride(0) * x.element_size() % 16 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous()))):
         out = torch.empty((n, o), dtype=x.dtype if float_out is None else torch.float32, device=x.device)
-        N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), _code(w.dtype), k, o, _ptr(bias), out.data_ptr(), o,
-                                                 _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT, _stream(x.device)), "jl_linear_small")
-        return out
+        mode = _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT
+        if small:
+            N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), _code(w.dtype), k, o, _ptr(bias), out.data_ptr(), o, mode,
+                                                     _stream(x.device)), "jl_linear_small")
+            return out
+        if n * x.stride(0) * size < 1 << 32:
+            N.check_layers(N.layers().jl_linear_mid(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), k, o, _ptr(bias), out.data_ptr(), o, mode, _stream(x.device)),
+                           "jl_linear_mid")
+            return out
     if float_out and w.dtype != torch.float32:
         y = torch.mm(x, w.t(), out_dtype=torch.float32)
         return y if bias is None else y + bias

@@ -41,3 +41,23 @@ def test_forms_it_does_not_take():
         LO.linear(torch.randn(3, 60, device=dev), w)
     with pytest.raises(ValueError):
         LO.linear(torch.randn(3, 64, device=dev), w.bfloat16())
+
+
+@pytest.mark.parametrize("N,K,O,bias", [(65, 8, 1, True), (127, 56, 63, False), (129, 64, 65, True), (1000, 72, 130, False), (64, 1024, 4099, True), (700, 1016, 1000, True), (1, 512, 32000, False)])
+def test_a_few_hundred_rows(N, K, O, bias):
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt = "cuda", torch.bfloat16
+    assert LO.linear_mid(N, K, O, dt)
+    g = torch.Generator(device=dev).manual_seed(N + K + O)
+    x = torch.randn(N, K + 16, generator=g, device=dev).to(dt)[:, 8:8 + K]                  # rows apart, 16-byte borders
+    w, b = torch.randn(O, K, generator=g, device=dev).to(dt), torch.randn(O, generator=g, device=dev).to(dt) if bias else None
+    want = x.double() @ w.double().T + (b.double() if bias else 0)
+    size = x.double().abs() @ w.double().abs().T + (b.double().abs() if bias else 0)
+    for float_out in (None, True, False):
+        got = LO.linear(x, w, b, float_out)
+        assert got.dtype == (torch.float32 if float_out is not None else dt) and got.shape == (N, O)
+        # float sums of K exact products: at most K roundings; then one of the result
+        tol = (K + 16) * 2.0 ** -24 * size + (2.0 ** -8 * want.abs() if not float_out else 0)
+        assert bool(((got.double() - want).abs() <= tol).all())
+        if float_out is False:
+            assert torch.equal(got, got.to(dt).float())
