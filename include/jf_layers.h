@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 134
+#define JL_VERSION 135
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -137,6 +137,10 @@ JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t
  * jl_attn_talk_tile_rows(H, G, wide) queries in any order (wide: 128 (query, head) rows per workgroup, else 32), a tile's keys shared out over `splits` workgroups;
  * scratch of jl_attn_talk_scratch_floats for pass_tiles tiles at a time.  q, pools and scratch at 16-byte borders, k_ld and v_ld in multiples of 8, out_ld of 4. */
 JL_API int jl_attn_talk(const jl_attn_args *a, int32_t wide, int32_t pass_tiles, void *stream);
+/* jl_attn_sweep for portions of a few tokens (decoding), the same arguments, in tiles of jl_attn_talk_tile_rows(H, G, 0) queries; scratch of
+ * jl_attn_talk_scratch_floats(tiles, TQ, H, 1, Dv, splits); sizes as jl_attn_narrow_ok takes them, alignment as for jl_attn_talk. */
+JL_API int jl_attn_narrow(const jl_attn_args *a, void *stream);
+JL_API int jl_attn_narrow_ok(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
 JL_API int jl_attn_talk_ok(int dtype, int32_t H, int32_t G, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
 JL_API int jl_attn_talk_tile_rows(int32_t H, int32_t G, int32_t wide);
 JL_API int64_t jl_attn_talk_scratch_floats(int32_t tiles, int32_t TQ, int32_t H, int32_t G, int32_t Dv, int32_t splits);

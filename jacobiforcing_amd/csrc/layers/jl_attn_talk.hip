@@ -21,7 +21,7 @@ constexpr int AT_BIAS = 5;              // bias entries per thread and tile at m
 static __host__ __device__ inline int at_bias_row(int TQ, int HF) { return (TQ + AT_KT - 1 + 31) / 32 * 32 + (HF < 32 ? 32 / HF : 1); }   // heads of a query meet different banks
 static size_t at_lds_bytes(int KU, int VU, int TQ, int HF, int NW) { return (NW > 1 ? 2 : 1) * ((size_t)AT_KT * (KU + VU) * 16 + AT_KT * 4 + (size_t)HF * at_bias_row(TQ, HF) * 4); }
 
-template <int KU, int VU, int NW>                                                      // D <= 8 * KU, Dv <= 8 * VU, wavefronts
+template <int KU, int VU, int NW, bool MIX>                                            // D <= 8 * KU, Dv <= 8 * VU, wavefronts; MIX: products with all value heads
 __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, int HF, int tile0, int n_tiles) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int THREADS = 64 * NW, BUFS = NW > 1 ? 2 : 1, KT = AT_KT, NDV = VU / 4, BUF = KT * (KU + VU);
@@ -29,7 +29,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     const int H = a.H, G = a.G, D = a.D, Dv = a.Dv, TQ = a.TQ, S = a.splits;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
     // key heads (and the value heads' groups) side by side: neighbouring workgroups go to different XCDs, so each keeps few heads' keys in its L2
-    const int side = blockIdx.x % (G * G), rest = blockIdx.x / (G * G), split = rest % S, ti = rest / S, c = side / G, g = side - c * G;
+    const int sides = MIX ? G * G : G, side = blockIdx.x % sides, rest = blockIdx.x / sides, split = rest % S, ti = rest / S, c = MIX ? side / G : side, g = MIX ? side - c * G : c % a.Gv;
     const int *tile = a.tiles + 4 * (int64_t)(tile0 + ti);
     const int b = tile[0], i0 = tile[1], cnt = tile[2], row0 = tile[3], h0 = c * HF;
     if (b < 0 || cnt <= 0) return;
@@ -39,8 +39,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     const int BR = at_bias_row(TQ, HF);
     const int window = a.window > 0 ? a.window : 0x3fffffff;
     const int i_max = i0 + cnt - 1;
-    const int lo = i0 - window + 1 > 0 ? i0 - window + 1 : 0;       // lowest key of the first row's window
-    const int kept = a.keep_first < lo ? a.keep_first : lo;         // kept first tokens in front of it
+    const int chunk = MIX ? 0 : a.chunk, keep_first = MIX ? a.keep_first : 0;
+    auto lowest = [&](int i) { return chunk > 0 ? i - i % chunk : i - window + 1; };        // first key that query i sees
+    const int lo = lowest(i0) > 0 ? lowest(i0) : 0;                 // of the first row's
+    const int kept = keep_first < lo ? keep_first : lo;             // kept first tokens in front of them
     const int kept_tiles = (kept + KT - 1) / KT, n_kt = kept_tiles + (i_max + 1 - lo + KT - 1) / KT;
     const int share = (n_kt + S - 1) / S, t_lo = split * share, t_hi = t_lo + share < n_kt ? t_lo + share : n_kt;
     // a tile's first position and its keys
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     // this lane's row: (query R / HF, head h0 + R % HF); both half-wavefronts hold it
     const int R = 32 * wave + l32, ii = R / HF, hl = R - ii * HF;
     const bool ok = ii < TQ && ii < cnt;
-    const int qi = i0 + ii, q_lo = qi - window + 1;
+    const int qi = i0 + ii, q_lo = lowest(qi);
     ar_bf16x8 qf[KU / 2];
 #pragma unroll
     for (int x = 0; x < KU / 2; ++x) {
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
             const int e = tid + it * THREADS, jj = e / VU, u = e % VU;
             if (jj < nk && 8 * u < Dv) vreg[it] = load16(vc + (int64_t)tok[jj] * a.v_ld + 8 * u);
         }
-        if (NW > 1 && a.rel)
+        if (MIX && NW > 1 && a.rel)
 #pragma unroll
             for (int it = 0; it < AT_BIAS; ++it) {
                 const int e = tid + it * THREADS;
@@ -124,13 +126,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
             const int e = tid + it * THREADS, jj = e / VU, u = e % VU;
             if (jj < nk && 8 * u < Dv) Ks[KT * KU + jj * VU + ar_value_unit<VU>(jj, u)] = vreg[it];
         }
-        if (NW > 1 && a.rel)
+        if (MIX && NW > 1 && a.rel)
 #pragma unroll
             for (int it = 0; it < AT_BIAS; ++it) {
                 const int e = tid + it * THREADS;
                 if (e < n_bias) { const int y = e / HF; bias[(e - y * HF) * BR + y] = breg[it] * LOG2E; }
             }
-        if (NW == 1 && a.rel) {
+        if (MIX && NW == 1 && a.rel) {
             const int j0 = first_of(t);
 #pragma unroll 4
             for (int e = tid; e < n_bias; e += THREADS) { const int y = e / HF; bias[(e - y * HF) * BR + y] = bias_of(e, j0) * LOG2E; }
@@ -160,14 +162,17 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
         const uint4 *Ks = buf0 + sel * BUF;
         const int j0 = first_of(t), nk = keys_of(t);
         // wavefront-uniform: keys all behind its last query, or all before its first query's window and not kept
-        if (wave_live && j0 <= i0 + wq_last && (j0 < a.keep_first || j0 + nk - 1 >= i0 + wq_first - window + 1)) {
+        if (wave_live && j0 <= i0 + wq_last && (j0 < keep_first || j0 + nk - 1 >= lowest(i0 + wq_first))) {
             ar_f32x16 sc;
 #pragma unroll
             for (int r = 0; r < 16; ++r) sc[r] = 0.f;
 #pragma unroll
             for (int x = 0; x < KU / 2; ++x)
                 sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ar_bf16x8, Ks[l32 * KU + ar_key_unit<KU>(l32, 2 * x + hi)]), qf[x], sc, 0, 0, 0);
-            if (a.rel) {
+            if (!MIX && a.softcap > 0.f) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] = soft_cap_fast(sc[r] * a.scale, a.softcap) * LOG2E;
+            } else if (MIX && a.rel) {
                 const float *bias = biasS + sel * HF * BR + hl * BR + (ok ? ii : 0) + KT - 1 - 4 * hi;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[r] = fmaf(sc[r], c2, bias[-(8 * (r >> 2) + (r & 3))]);
@@ -175,9 +180,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[r] *= c2;
             // wavefront-uniform: a full tile whose keys every row of the wavefront sees needs no mask
-            const bool inside = nk == KT && wave_full && j0 + KT - 1 <= i0 + wq_first && (j0 >= i0 + wq_last - window + 1 || j0 + KT <= a.keep_first);
+            const bool inside = nk == KT && wave_full && j0 + KT - 1 <= i0 + wq_first && (j0 >= lowest(i0 + wq_last) || j0 + KT <= keep_first);
             if (!inside) {
-                const int first = ok ? q_lo - j0 : KT, last = qi - j0 < nk - 1 ? qi - j0 : nk - 1, keep = ok ? a.keep_first - j0 : 0;
+                const int first = ok ? q_lo - j0 : KT, last = qi - j0 < nk - 1 ? qi - j0 : nk - 1, keep = ok ? keep_first - j0 : 0;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int kk = 8 * (r >> 2) + 4 * hi + (r & 3);
@@ -220,7 +225,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
                     }
                     const ar_bf16x8 va = __builtin_bit_cast(ar_bf16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
                     acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, acc[y], 0, 0, 0);
-                    acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[y], 0, 0, 0);
+                    if (MIX) acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[y], 0, 0, 0);
                 }
             }
         }
@@ -234,10 +239,11 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     if (!ok) return;
     // shares of the pass's rows: [tile, query][split][head][value head][Dv], and their maxima and sums [..][head][2] behind all of them
     const int64_t row = ((int64_t)ti * TQ + ii) * S + split;
-    float *ml = a.scratch + (int64_t)n_tiles * TQ * S * H * G * Dv + (row * H + h0 + hl) * 2;
-    if (g == 0 && hi == 0) { ml[0] = m_run; ml[1] = l_run; }
+    const int GW = MIX ? G : 1;
+    float *ml = a.scratch + (int64_t)n_tiles * TQ * S * H * GW * Dv + (row * H + h0 + hl) * 2;
+    if ((!MIX || g == 0) && hi == 0) { ml[0] = m_run; ml[1] = l_run; }
     if (!(l_run > 0.f) && m_run == -INFINITY) return;               // nothing seen: the share is not read
-    float *o = a.scratch + ((row * H + h0 + hl) * G + g) * Dv;
+    float *o = a.scratch + ((row * H + h0 + hl) * GW + (MIX ? g : 0)) * Dv;
 #pragma unroll
     for (int y = 0; y < NDV; ++y)
 #pragma unroll
@@ -346,7 +352,7 @@ template <int KU, int VU, int NW> static int at_launch(const jl_attn_args &a, in
     const bool spread = a.splits > 1;
     const size_t lds = at_lds_bytes(KU, VU, a.TQ, HF, NW), mix = (size_t)((spread ? a.H * (a.G * a.Dv > 2 * a.splits ? a.G * a.Dv : 2 * a.splits) + a.splits * a.H : 4 * a.H) + a.H * a.H) * 4;
     if (NW > 1 && HF * (a.TQ + AT_KT - 1) > AT_BIAS * 64 * NW) return jl_fail(JL_E_INVALID, "jl_attn_talk: too many biases per tile");
-    auto kern = attn_talk_kernel<KU, VU, NW>;
+    auto kern = attn_talk_kernel<KU, VU, NW, true>;
     auto join = spread ? attn_talk_mix_kernel<true> : attn_talk_mix_kernel<false>;
     hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess && mix > 64 * 1024) e = hipFuncSetAttribute((const void *)join, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix);
@@ -379,4 +385,79 @@ extern "C" int jl_attn_talk(const jl_attn_args *ap, int32_t wide, int32_t pass_t
     AT_CASE(8, 8); AT_CASE(8, 16); AT_CASE(16, 8); AT_CASE(16, 16);
 #undef AT_CASE
     return jl_fail(JL_E_INVALID, "jl_attn_talk: unsupported size");
+}
+
+// ---- the same for single tokens without mixed heads: a wavefront's keys once, one product with the values -----------------------------------------
+// Decoding's attention is bound by the way to its keys: four wavefronts that meet at three barriers per 32 keys and fetch each tile's rows behind its page numbers (jl_attn_sweep.hip)
+// read keys and values at 1.3 TB/s; single wavefronts, eight to a CU, that keep their rows to themselves at 3.1.  us for both launches, sweep / this (20 and less are the host's): 32 tokens at 2048,
+// 16 heads of 128 over 4 100 / 43, 8 over 2 68 / 32; 200 tokens at 1000, 16 over 4 538 / 103; 48 at 500 40 / 25; 30 portions of 10 at 1000, 8 over 2 63 / 30; 512 tokens 50 / 31.
+// A (token, head) row's shares joined: w = 2 ** (m - M) / L with the sink as one more share that holds nothing, times the gate
+__global__ __launch_bounds__(256) void attn_narrow_join_kernel(jl_attn_args a, int64_t groups) {
+    const int64_t r = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
+    if (r >= groups) return;
+    const int H = a.H, Dv = a.Dv, S = a.splits, lane = threadIdx.x & 31, h = (int)(r % H);
+    const int64_t rt = r / H;
+    const int ti = (int)(rt / a.TQ), ii = (int)(rt - (int64_t)ti * a.TQ);
+    const int *tile = a.tiles + 4 * (int64_t)ti;
+    if (tile[0] < 0 || ii >= tile[2]) return;
+    const int64_t n = tile[3] + ii;
+    const float *ml = a.scratch + (int64_t)a.n_tiles * a.TQ * S * H * Dv + (rt * S * H + h) * 2, *po = a.scratch + (rt * S * H + h) * Dv + 4 * lane;
+    constexpr float LOG2E = 1.44269504088896341f;
+    const float sink = a.sink ? a.sink[h] * LOG2E : -INFINITY;
+    float M = sink;
+    for (int s = 0; s < S; ++s) M = fmaxf(M, ml[s * H * 2]);
+    float L = a.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
+    const bool in = 4 * lane < Dv;
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+        const float m = ml[s * H * 2], l = ml[s * H * 2 + 1], w = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+        const float4 p = in ? *(const float4 *)(po + (int64_t)s * H * Dv) : make_float4(0.f, 0.f, 0.f, 0.f);
+        L += w * l;                                                 // an empty share (m = -inf) holds nothing and is not looked at
+        v[0] = m > -INFINITY ? fmaf(w, p.x, v[0]) : v[0];
+        v[1] = m > -INFINITY ? fmaf(w, p.y, v[1]) : v[1];
+        v[2] = m > -INFINITY ? fmaf(w, p.z, v[2]) : v[2];
+        v[3] = m > -INFINITY ? fmaf(w, p.w, v[3]) : v[3];
+    }
+    if (!in) return;
+    const float inv = L > 0.f ? a.out_scale / L : 0.f;
+    const bf16_t *gate = (const bf16_t *)a.gate;
+    const int col = h * Dv + 4 * lane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[i] *= inv;
+        if (gate) v[i] *= 1.0f / (1.0f + __expf(-ld_f(gate + n * a.gate_ld + (a.gate_heads ? h : col + i))));
+    }
+    if (a.out_dtype == JL_OUT_F32) st4_f((float *)a.out + n * a.out_ld + col, v);
+    else st4_f((bf16_t *)a.out + n * a.out_ld + col, v);
+}
+
+extern "C" int jl_attn_narrow_ok(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld) {
+    return jl_attn_talk_ok(dtype, H, G, D, Dv, k_ld, v_ld) && Gv > 0 && G % Gv == 0;
+}
+
+template <int KU, int VU> static int an_launch(const jl_attn_args &a, hipStream_t st) {
+    const size_t lds = at_lds_bytes(KU, VU, a.TQ, a.H / a.G, 1);
+    auto kern = attn_talk_kernel<KU, VU, 1, false>;
+    kern<<<dim3((unsigned)(a.n_tiles * a.splits * a.G)), 64, lds, st>>>(a, a.H / a.G, 0, a.n_tiles);
+    const int64_t groups = (int64_t)a.n_tiles * a.TQ * a.H;
+    attn_narrow_join_kernel<<<dim3((unsigned)((groups + 7) / 8)), 256, 0, st>>>(a, groups);
+    return jl_check_launch("attn_talk_kernel (single tokens)");
+}
+
+extern "C" int jl_attn_narrow(const jl_attn_args *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null arguments");
+    const jl_attn_args &a = *ap;
+    if (a.n_tiles <= 0) return JL_OK;
+    if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.block_tables || !a.tiles || !a.scratch) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null pointer");
+    if (!jl_attn_narrow_ok(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld) || a.k_ld < (int64_t)a.G * a.D || a.v_ld < (int64_t)a.Gv * a.Dv ||
+        (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.v_cache | (uintptr_t)a.scratch) & 15))
+        return jl_fail(JL_E_INVALID, "jl_attn_narrow: sizes or alignment (ask jl_attn_narrow_ok)");
+    if (a.talk || a.rel || a.keep_first > 0 || (a.chunk > 0 && a.window > 0) || a.page_size <= 0) return jl_fail(JL_E_INVALID, "jl_attn_narrow: no bias, mixed heads or kept tokens; chunks exclude a window");
+    if (a.TQ != jl_attn_talk_tile_rows(a.H, a.G, 0) || a.splits <= 0 || a.splits > 64 || a.out_ld < (int64_t)a.H * a.Dv || a.out_ld % 4 ||
+        (int64_t)a.n_tiles * a.splits * a.G > INT32_MAX / 64 || (int64_t)a.n_tiles * a.TQ * a.H > INT32_MAX)
+        return jl_fail(JL_E_INVALID, "jl_attn_narrow: tiles, splits or output rows");
+    if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_narrow: unknown out_dtype");
+    hipStream_t st = (hipStream_t)stream;
+    if (a.D <= 64) return a.Dv <= 64 ? an_launch<8, 8>(a, st) : an_launch<8, 16>(a, st);
+    return a.Dv <= 64 ? an_launch<16, 8>(a, st) : an_launch<16, 16>(a, st);
 }

@@ -22,6 +22,7 @@ ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-co
 # mixed heads: workgroups of 4 wavefronts to aim at (of one: three times as many); scratch at most (1 GiB: more tiles than it holds take turns), as long as it holds a tile's.  us, 8 heads
 # over 2 of 128 under a window of 1024, for 512 / 640 / 1024: 777 + 300 tokens beside 30 single ones 105 / 79 / 81, one portion of 1000 54 / 56 / 65
 TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
+NARROW_WORKGROUPS = 2048              # attention of a few tokens per request: single wavefronts to aim at when keys are shared out
 BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
@@ -497,10 +498,9 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
     tq = attn_sweep_tile_rows(q.dtype, H, G, D, Dv, k_cache, v_cache, Gv)
     _need(tq > 0, f"attn_sweep: heads={H} kv_heads={G} dim={D} vdim={Dv} are not sizes of this kernel")
     _need(chunk <= 0 or window <= 0, "attn_sweep: chunks exclude a window")
-    tiles = batch.tiles(tq)
     out = _attn_out(out, n, H * Dv, torch.float32 if float_out else q.dtype, q.device, "attn_sweep")
     # few tiles with many keys (decoding): share each tile's keys out over workgroups until the chip is full
-    groups = tiles.shape[0] * G * -(-(H // G) // 32)
+    tiles, groups = None, sum(-(-c // tq) for c in batch.counts) * G * -(-(H // G) // 32)
     # float tiles take 16 times as long per key, so the chip has to be fuller before their keys are left whole: 3 x 1000 tokens, 8 heads over 2 (648 groups)
     # 160 us shared out, 218 us in 128-row tiles; 1 x 4096 (1024 groups) 916 and 805 us
     below = SWEEP_SPLIT_BELOW_GROUPS if q.dtype == torch.bfloat16 else 2 * SWEEP_SPLIT_BELOW_GROUPS
@@ -513,11 +513,22 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
             # what starts last should be short (4 x 2048 tokens, 16 heads of 128 over 4 key heads: 175 -> 137 us).  The 32-row kernel keeps the
             # requests' order, in which neighbours share keys (over a latent of 512 the sorted order was 3 % slower)
             tq, tiles = wide, batch.tiles(wide, longest_first=True)
-    elif groups < below:
+    narrow = False
+    if tiles is None and q.dtype == torch.bfloat16 and out.stride(0) % 4 == 0 and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and \
+            N.layers().jl_attn_narrow_ok(N.JL_BF16, H, G, Gv, D, Dv, k_cache.stride(0), v_cache.stride(0)):
+        # few tokens per request: single wavefronts, each with a share of a tile's keys
+        narrow, tq = True, int(N.layers().jl_attn_talk_tile_rows(H, G, 0))
+        tiles = batch.tiles(tq)
+        reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
+        splits = max(1, min(-(-reach // 64), NARROW_WORKGROUPS // (tiles.shape[0] * G), 64))
+        scratch = torch.empty((int(N.layers().jl_attn_talk_scratch_floats(tiles.shape[0], tq, H, 1, Dv, splits)),), dtype=torch.float32, device=q.device)
+    elif tiles is None and groups < below:
+        tiles = batch.tiles(tq)
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
         splits = max(1, min(-(-reach // 128), SWEEP_SPLIT_WORKGROUPS // groups, 64))
         if splits > 1:
             scratch = torch.empty((int(N.layers().jl_attn_sweep_scratch_floats(tiles.shape[0], H, G, Dv, splits)),), dtype=torch.float32, device=q.device)
+    tiles = batch.tiles(tq) if tiles is None else tiles
     a = N.AttnArgs(q=q.data_ptr(), k_cache=k_cache.data_ptr(), v_cache=v_cache.data_ptr(), out=out.data_ptr(), block_tables=batch.tables.data_ptr(),
                    tiles=tiles.data_ptr(), bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0], page_size=batch.page_size, H=H, G=G, D=D, Dv=Dv,
                    window=int(window), TQ=tq, dtype=_code(q.dtype), scale=float(scale), n_rows=n, k_ld=k_cache.stride(0), v_ld=v_cache.stride(0), Gv=Gv,
@@ -525,6 +536,9 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
                    out_dtype=N.JL_OUT_F32 if float_out else N.JL_OUT_SAME, sink=sink.data_ptr() if sink is not None else None,
                    gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0, gate_heads=int(gate_per_head),
                    chunk=int(chunk), softcap=float(softcap), out_scale=float(out_scale), out_ld=out.stride(0))
+    if narrow:
+        N.check_layers(N.layers().jl_attn_narrow(C.byref(a), _stream(q.device)), "jl_attn_narrow")
+        return out
     N.check_layers(N.layers().jl_attn_sweep(C.byref(a), _stream(q.device)), "jl_attn_sweep")
     return out
 

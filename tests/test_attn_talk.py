@@ -53,3 +53,57 @@ def test_talk(monkeypatch, H, G, D, Dv, window, keep, counts, starts, bias, floa
         # scores: float sums of D products times the scale (a few 2 ** -24 of their size, up to about 10); weights to 16 bits of mantissa (2 ** -17), weights and sums cancel by up to 8
         assert err <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24), (b, err.item())
         r0 += c
+
+
+@pytest.mark.parametrize("H,G,Gv,D,Dv,counts,starts,kw,wgs", [
+    (16, 4, 4, 128, 128, [1] * 4, [0, 31, 2000, 999], {}, 2048), (6, 2, 2, 72, 64, [3, 1, 20], [100, 64, 0], dict(window=50, sink=True, gate="head"), 2048),
+    (4, 4, 2, 64, 128, [1, 2], [700, 90], dict(chunk=64, float_out=True), 64), (8, 1, 1, 8, 64, [1, 1], [33, 1], dict(softcap=5.0, gate="value", out_scale=0.5), 1),
+    (32, 1, 1, 128, 32, [2, 1], [300, 5], dict(sink=True, into=True), 2048), (12, 3, 1, 104, 96, [1] * 3, [63, 64, 500], dict(window=1), 2048),
+])
+def test_few_tokens(monkeypatch, H, G, Gv, D, Dv, counts, starts, kw, wgs):
+    """The form for a few tokens per request without mixed heads: windows, chunks, caps, sinks, gates, shared values, results into wider rows."""
+    from jacobiforcing_amd import _native as N
+    from jacobiforcing_amd import layer_ops as LO
+    dev, page = "cuda", 16
+    monkeypatch.setattr(LO, "NARROW_WORKGROUPS", wgs)
+    g = torch.Generator(device=dev).manual_seed(H * D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    n, B, rep = sum(counts), len(counts), H // G
+    need = [-(-(c + s) // page) for c, s in zip(counts, starts)]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(1)).tolist()
+    pages = [[order.pop() for _ in range(x)] for x in need]
+    batch = LO.RaggedBatch.build(counts, starts, list(range(B)), pages, page, dev)
+    kp, vp = rnd(sum(need) * page, G * D + 8).bfloat16()[:, :G * D], rnd(sum(need) * page, Gv * Dv + 16).bfloat16()[:, 8:8 + Gv * Dv]
+    q = rnd(n, H * D).bfloat16()
+    window, chunk, cap = kw.get("window", 0), kw.get("chunk", 0), kw.get("softcap", 0.0)
+    sink = rnd(H) if kw.get("sink") else None
+    gate = None if "gate" not in kw else rnd(n, H if kw["gate"] == "head" else H * Dv).bfloat16()
+    wider = torch.zeros(n, H * Dv + 12, device=dev, dtype=torch.bfloat16) if kw.get("into") else None
+    assert N.layers().jl_attn_narrow_ok(N.JL_BF16, H, G, Gv, D, Dv, kp.stride(0), vp.stride(0))
+    calls, real = [], N.layers().jl_attn_narrow
+    monkeypatch.setattr(N.layers(), "jl_attn_narrow", lambda *a: calls.append(1) or real(*a), raising=False)
+    out = LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, D ** -0.5, window, value_heads=Gv, float_out=kw.get("float_out", False), sink=sink, gate=gate, gate_per_head=kw.get("gate") == "head",
+                        chunk=chunk, softcap=cap, out_scale=kw.get("out_scale", 1.0), out=wider[:, 4:4 + H * Dv] if wider is not None else None)
+    assert calls, "the form for a few tokens did not run"
+    if wider is not None:
+        assert not wider[:, :4].any() and not wider[:, 4 + H * Dv:].any()
+    r0 = 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // page] * page + j % page for j in range(c + s)], device=dev)
+        heads = torch.arange(H, device=dev) // rep
+        k, v = kp[tok].double().view(-1, G, D)[:, heads], vp[tok].double().view(-1, Gv, Dv)[:, heads % Gv]
+        sc = (q[r0:r0 + c].double().view(c, H, D).permute(1, 0, 2).contiguous() @ k.permute(1, 2, 0).contiguous()) * D ** -0.5
+        sc = cap * torch.tanh(sc / cap) if cap else sc
+        i, j = torch.arange(s, s + c, device=dev).view(-1, 1), torch.arange(c + s, device=dev).view(1, -1)
+        see = (j <= i) & ((i - j) < window if window else (j >= i - i % chunk) if chunk else torch.ones_like(i - j, dtype=torch.bool))
+        sc = sc.masked_fill(~see, float("-inf"))
+        if sink is not None:
+            sc = torch.cat([sc, sink.double().view(H, 1, 1).expand(H, c, 1)], -1)
+        o = (torch.softmax(sc, -1)[..., :c + s].contiguous() @ v.permute(1, 0, 2).contiguous()).permute(1, 0, 2) * kw.get("out_scale", 1.0)
+        if gate is not None:
+            z = torch.sigmoid(gate[r0:r0 + c].double())
+            o = o * (z.view(c, H, 1) if kw["gate"] == "head" else z.view(c, H, Dv))
+        err = (out[r0:r0 + c].double().reshape(c, H, Dv) - o).norm() / o.norm()
+        # weights and results are rounded to bfloat16, 2 ** -9 each; the cap's tanh is a few 1e-7 of the cap off
+        assert err <= 2 * 2.0 ** -8, (b, err.item())
+        r0 += c
