@@ -14,6 +14,10 @@
 //      beside the keys — or ARE the keys' first columns.
 // Few tiles with many keys (decoding): the key tiles of a row tile are shared out over blockIdx.z; every share leaves its
 // unnormalised outputs with its maximum and sum in a scratch, and attn_sweep_join_kernel combines them.
+// The next tile's rows travel in registers (16 bytes per lane, all at once) while this one is computed, its pool tokens were looked up a tile before.  What bounds it now: three
+// barriers per 32 keys at two or three workgroups per CU.  us before (rows fetched 8 bytes at a time between two barriers, each behind its page number) and after: 32 tokens at 2048 over
+// latents of 512 + 64, 16 heads 83 -> 49; 4 x 200 tokens at 500 over them 246 -> 149; 777 + 300 tokens beside 30 single ones over 128 + 32, 8 heads 91 -> 69; 32 tokens at 2048, 16 heads
+// of 192 / 128 over 4 119 -> 61.
 // Accumulator r of lane l of a 32 x 32 MFMA is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32; lane l supplies row (A) or
 // column (B) l % 32 with depths 4 * (l / 32) .. + 3.
 #include "jl_attn.h"
@@ -31,11 +35,11 @@ __device__ __forceinline__ short as_bf16(float v) {
 }
 
 static size_t as_lds_bytes(int D, int Dv, bool v_in_k) {
-    return (size_t)AS_T * (D + 4) * 2 + (v_in_k ? 0 : (size_t)AS_T * (Dv + 4) * 2) + (size_t)AS_WAVES * AS_T * 33 * 4 + (size_t)AS_T * AS_PROW * 2 + 2 * AS_T * 4;
+    return (size_t)AS_T * (D + 4) * 2 + (v_in_k ? 0 : (size_t)AS_T * (Dv + 4) * 2) + (size_t)AS_WAVES * AS_T * 33 * 4 + (size_t)AS_T * AS_PROW * 2 + 4 * AS_T * 4;
 }
 
-template <int NT>                                                                       // value tiles (32 columns) per wavefront: Dv <= 128 * NT
-__global__ __launch_bounds__(AS_THREADS) void attn_sweep_kernel(jl_attn_args a, int HF, int TQ, int HB, int v_in_k) {
+template <int NT, int KPF, bool v_in_k>                                                 // value tiles (32 columns) per wavefront: Dv <= 128 * NT; D <= 64 * KPF
+__global__ __launch_bounds__(AS_THREADS, KPF > 3 || NT > 1 ? 2 : 3) void attn_sweep_kernel(jl_attn_args a, int HF, int TQ, int HB) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int H = a.H, D = a.D, Dv = a.Dv, KROW = D + 4, VROW = v_in_k ? KROW : Dv + 4, per_group = H / a.G;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
@@ -50,6 +54,7 @@ __global__ __launch_bounds__(AS_THREADS) void attn_sweep_kernel(jl_attn_args a, 
     bf16_t *Pb = (bf16_t *)(Sp + AS_WAVES * AS_T * 33);             // [32][36] weights
     float *alphaS = (float *)(Pb + AS_T * AS_PROW);                 // [32] rescale factor of the tile
     float *lS = alphaS + AS_T;                                      // [32] final sums
+    int *tokS = (int *)(lS + AS_T);                                 // [2][32] pool tokens of a tile's keys
     const int window = a.window > 0 ? a.window : 0x3fffffff;
     const int i_max = i0 + cnt - 1;
     const int chunk = a.chunk;
@@ -87,48 +92,71 @@ __global__ __launch_bounds__(AS_THREADS) void attn_sweep_kernel(jl_attn_args a, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
 
-    const int units = D / 4;                                        // 8-byte units per key row
-    const int jj0 = tid / units, u0r = tid - jj0 * units, dj = AS_THREADS / units, dr = AS_THREADS - dj * units;
-    const int vunits = Dv / 4;
-    const int vj0 = tid / vunits, v0r = tid - vj0 * vunits, vdj = AS_THREADS / vunits, vdr = AS_THREADS - vdj * vunits;
-
+    // 16 bytes per load where rows and columns start at 16-byte borders, else two of 8; into rows of LDS that start at 8-byte borders
+    const int units = D / 8, vunits = Dv / 8;
+    const bool whole = ((uintptr_t)a.k_cache & 15) == 0 && a.k_ld % 8 == 0 && ((uintptr_t)a.v_cache & 15) == 0 && a.v_ld % 8 == 0;
+    typedef uint32_t as_u32x4 __attribute__((ext_vector_type(4)));
+    auto load16 = [&](const bf16_t *p) -> as_u32x4 {
+        if (whole) return *(const as_u32x4 *)p;
+        const uint2 x = *(const uint2 *)p, y = *(const uint2 *)(p + 4);
+        return (as_u32x4){x.x, x.y, y.x, y.y};
+    };
+    auto store16 = [](bf16_t *p, as_u32x4 v) {
+        *(uint2 *)p = make_uint2(v[0], v[1]);
+        *(uint2 *)(p + 4) = make_uint2(v[2], v[3]);
+    };
+    constexpr int VPF = v_in_k ? 1 : 2 * NT;
+    as_u32x4 kreg[KPF], vreg[VPF];
     const int S = a.splits > 1 ? a.splits : 1, split = blockIdx.z;
     const int per = ((n_keys + AS_T - 1) / AS_T + S - 1) / S;       // key tiles per share
     const int key_lo = split * per * AS_T, key_hi = (split + 1) * per * AS_T < n_keys ? (split + 1) * per * AS_T : n_keys;
-    for (int u0 = key_lo; u0 < key_hi; u0 += AS_T) {
+    // the next tile's rows travel while this one is computed, the tokens of the tile behind it are looked up meanwhile
+    int tok_next = 0;
+    auto look_up = [&](int u) {
+        if (tid >= AS_T || u + tid >= key_hi) return;
+        const int j = lo + u + tid, pg = page_shift >= 0 ? j >> page_shift : j / a.page_size;
+        tok_next = bt[pg] * a.page_size + (j - pg * a.page_size);
+    };
+    const as_u32x4 zero = {0, 0, 0, 0};
+    auto fetch = [&](int u, const int *tok) {
+        const int nk = key_hi - u < AS_T ? key_hi - u : AS_T;
+#pragma unroll
+        for (int it = 0; it < KPF; ++it) {
+            const int e = tid + it * AS_THREADS, jj = e / units, x = e - jj * units;
+            kreg[it] = zero;                                        // rows beyond the last key are zero
+            if (jj < nk) kreg[it] = load16(kc + (int64_t)tok[jj] * a.k_ld + 8 * x);
+        }
+        if (!v_in_k)
+#pragma unroll
+            for (int it = 0; it < VPF; ++it) {
+                const int e = tid + it * AS_THREADS, jj = e / vunits, x = e - jj * vunits;
+                vreg[it] = zero;
+                if (jj < nk) vreg[it] = load16(vc + (int64_t)tok[jj] * a.v_ld + 8 * x);
+            }
+    };
+    look_up(key_lo);
+    if (tid < AS_T) tokS[tid] = tok_next;
+    look_up(key_lo + AS_T);
+    __syncthreads();
+    if (key_lo < key_hi) fetch(key_lo, tokS);
+    for (int u0 = key_lo, sel = 1; u0 < key_hi; u0 += AS_T, sel ^= 1) {
         const int nk = key_hi - u0 < AS_T ? key_hi - u0 : AS_T;
         __syncthreads();                                            // the previous tile's readers are done with Ks / Pb
-        {
-            int jj = jj0, r = u0r;
-            for (int e = tid; e < AS_T * units; e += AS_THREADS) {
-                uint2 v = make_uint2(0, 0);
-                if (jj < nk) {
-                    const int j = lo + u0 + jj;
-                    const int pg = page_shift >= 0 ? j >> page_shift : j / a.page_size;
-                    const int64_t tok = (int64_t)bt[pg] * a.page_size + (j - pg * a.page_size);
-                    v = *(const uint2 *)(kc + tok * a.k_ld + 4 * r);
-                }
-                *(uint2 *)(Ks + jj * KROW + 4 * r) = v;
-                jj += dj; r += dr;
-                if (r >= units) { r -= units; ++jj; }
-            }
+#pragma unroll
+        for (int it = 0; it < KPF; ++it) {
+            const int e = tid + it * AS_THREADS, jj = e / units;
+            if (jj < AS_T) store16(Ks + jj * KROW + 8 * (e - jj * units), kreg[it]);
         }
-        if (!v_in_k) {
-            int jj = vj0, r = v0r;
-            for (int e = tid; e < AS_T * vunits; e += AS_THREADS) {
-                uint2 v = make_uint2(0, 0);
-                if (jj < nk) {
-                    const int j = lo + u0 + jj;
-                    const int pg = page_shift >= 0 ? j >> page_shift : j / a.page_size;
-                    const int64_t tok = (int64_t)bt[pg] * a.page_size + (j - pg * a.page_size);
-                    v = *(const uint2 *)(vc + tok * a.v_ld + 4 * r);
-                }
-                *(uint2 *)(Vs + jj * VROW + 4 * r) = v;
-                jj += vdj; r += vdr;
-                if (r >= vunits) { r -= vunits; ++jj; }
+        if (!v_in_k)
+#pragma unroll
+            for (int it = 0; it < VPF; ++it) {
+                const int e = tid + it * AS_THREADS, jj = e / vunits;
+                if (jj < AS_T) store16(Vs + jj * VROW + 8 * (e - jj * vunits), vreg[it]);
             }
-        }
+        if (tid < AS_T) tokS[sel * AS_T + tid] = tok_next;
         __syncthreads();
+        if (u0 + AS_T < key_hi) fetch(u0 + AS_T, tokS + sel * AS_T);
+        look_up(u0 + 2 * AS_T);
         {   // 1. partial scores of this wavefront's share of the key width
             as_f32x16 sc;
 #pragma unroll
@@ -350,20 +378,26 @@ extern "C" int jl_attn_sweep(const jl_attn_args *ap, void *stream) {
         attn_sweep_join_kernel<float><<<dim3(grid.x, grid.y, AS_T / AJ_ROWS), 256, 0, st>>>(a, hf, tq, hb);
         return jl_check_launch("attn_sweep_join_kernel");
     }
-#define AS_CASE(NTV)                                                                                                              \
-    case NTV: {                                                                                                                   \
-        auto kern = attn_sweep_kernel<NTV>;                                                                                       \
-        if (lds > 64 * 1024) {                                                                                                    \
-            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
-            if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_sweep: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e)); \
-        }                                                                                                                         \
-        kern<<<grid, AS_THREADS, lds, st>>>(a, hf, tq, hb, v_in_k ? 1 : 0);                                                       \
-        break;                                                                                                                    \
-    }
+    auto launch = [&](auto kern) -> int {
+        if (lds > 64 * 1024) {
+            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_sweep: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        }
+        kern<<<grid, AS_THREADS, lds, st>>>(a, hf, tq, hb);
+        return JL_OK;
+    };
+    int rc = JL_OK;
+#define AS_CASE(NTV)                                                                                                                   \
+    case NTV: rc = v_in_k ? (a.D <= 192 ? launch(attn_sweep_kernel<NTV, 3, true>) : launch(attn_sweep_kernel<NTV, 10, true>))           \
+                          : (a.D <= 192 ? launch(attn_sweep_kernel<NTV, 3, false>) : launch(attn_sweep_kernel<NTV, 10, false>)); break
     switch ((a.Dv + 127) / 128) {
-        AS_CASE(1) AS_CASE(2) AS_CASE(3) AS_CASE(4)
+        AS_CASE(1);
+        AS_CASE(2);
+        AS_CASE(3);
+        AS_CASE(4);
     }
 #undef AS_CASE
+    if (rc != JL_OK) return rc;
     if (a.splits > 1) attn_sweep_join_kernel<bf16_t><<<dim3(grid.x, grid.y, AS_T / AJ_ROWS), 256, 0, st>>>(a, hf, tq, hb);
     return jl_check_launch("attn_sweep_kernel");
 }
