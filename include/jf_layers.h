@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 135
+#define JL_VERSION 136
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -345,7 +345,8 @@ JL_API int jl_retention_join(const int32_t *req, int32_t B, const int32_t *chunk
 
 /* The same for long portions on the matrix cores: every request's portion cut into pieces of piece_tokens (a multiple of 64) tokens, the last of a request
  * what is left, that run side by side (own contributions to the state, the state each starts from, outputs).  piece_rec [pieces, 4] int32 {row0, count, slot,
- * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}; pos [N] int32 position of every row; scratch [pieces, H, D, Dv] float.
+ * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}; pos [N] int32 position of every row; scratch [pieces, H, D, Dv] and raw
+ * [N, H * Dv] float.
  * Sizes as jl_retention_pieces_ok takes them; ld and columns in multiples of four, rows and tables at the borders of four elements. */
 typedef struct jl_retention_pieces {
     const void *proj;
@@ -353,7 +354,8 @@ typedef struct jl_retention_pieces {
     const float *cos_t, *sin_t, *decay;
     float *state, *scratch;
     void *out;
-    int64_t ld, table_len;
+    float *raw;
+    int64_t ld, table_len, N;
     int32_t q_col, k_col, v_col, g_col, dtype, B, pieces, piece_tokens, H, D, Dv, rot_dims;
     float eps;
     int32_t reserved;

@@ -97,6 +97,9 @@ __device__ __forceinline__ float gated_unit_f(float g, float u, int kind, float 
     return g * sigmoid_f<FAST>(alpha * g) * (u + shift);
 }
 
+// out = raw / sqrt(mean(raw^2) + eps) (* norm_w) * silu(gate) per (row, head) of Dv values, gates at g_col of proj's rows (jl_delta.hip)
+int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int g_col, const float *norm_w, int64_t NH, int H, int Dv, float eps, void *out, hipStream_t st);
+
 // 16 bytes per lane from base + off into LDS at `lds` + 16 * lane (`base`, `lds` the same for the wavefront).  The compiler does not count these loads: the caller waits for vmcnt
 // before the barrier that publishes them, and before the workgroup ends
 __device__ __forceinline__ void jl_load_lds(const char *base, uint32_t off, uint32_t lds) {

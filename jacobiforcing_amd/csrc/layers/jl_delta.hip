@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const float *__restrict_
         if constexpr (VW == 4) ld4_f(gate + c, g);
         else g[0] = ld_f(gate + c);
 #pragma unroll
-        for (int i = 0; i < VW; ++i) g[i] = v[i] * rr * norm_w[c + i] * silu_f(g[i]);
+        for (int i = 0; i < VW; ++i) g[i] = v[i] * rr * (norm_w ? norm_w[c + i] : 1.0f) * silu_f(g[i]);
         if constexpr (VW == 4) st4_f(out + r * Dv + c, g);
         else st_f(out + r * Dv + c, g[0]);
     }
@@ -279,6 +279,11 @@ static int delta_out_launch(const float *raw, const void *proj, int64_t ld, int 
         delta_out_kernel<T, 4><<<grid, 256, 0, st>>>(raw, (const T *)proj, ld, g_col, norm_w, NH, H, Dv, eps, (T *)out);
     else delta_out_kernel<T, 1><<<grid, 256, 0, st>>>(raw, (const T *)proj, ld, g_col, norm_w, NH, H, Dv, eps, (T *)out);
     return jl_check_launch("delta_out_kernel");
+}
+
+int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int g_col, const float *norm_w, int64_t NH, int H, int Dv, float eps, void *out, hipStream_t st) {
+    JL_DISPATCH(dtype, return delta_out_launch<T>(raw, proj, ld, g_col, norm_w, NH, H, Dv, eps, out, st));
+    return JL_OK;
 }
 
 // ---- long portions on the float matrix instructions: 64 tokens at a time ------------------------------------------------------------------------

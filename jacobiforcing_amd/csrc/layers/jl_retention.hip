@@ -177,12 +177,14 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // the scan: no operand is split or rounded.  q, k (rotated, scaled), v and the pairs' weights of the group lie in LDS as floats; the next group's rows
 // are on their way meanwhile.
 // What bounds it: 368 matrix instructions of 64 cycles per wavefront and group of 64 tokens at 128 x 128, and the phases of a group at one workgroup per CU.
-// Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 261 us, one prompt of 128
-// 985 -> 70, 8 x 8 tokens 84 -> 39; float, 1021 + 851 + 681 tokens: 1091 -> 156.
+// Outputs leave as floats and are normed and gated by rows in a launch of their own: in this one, a wavefront's sums over its 32 columns cost 160 exchanges per group and the gates
+// came two bytes at a time, four on their way (outputs 211 us then, 112 and 18 now).
+// Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 182 us, one prompt of 128
+// 985 -> 53, 8 x 8 tokens 84 -> 34; float, 1021 + 851 + 681 tokens: 1091 -> 105.
 constexpr int RM_T = 64, RM_OUT = 0, RM_LOCAL = 1;
 typedef float rm_f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ rm_f32x16 rm_mma(float a, float b, rm_f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-static constexpr size_t rm_lds_bytes(int DP, bool out) { return ((size_t)RM_T * DP * (out ? 2 : 1) + RM_T * 128 + (out ? RM_T * RM_T + 4 * RM_T : 0) + 2 * RM_T) * 4; }
+static constexpr size_t rm_lds_bytes(int DP, bool out) { return ((size_t)RM_T * DP * (out ? 2 : 1) + RM_T * 128 + (out ? RM_T * RM_T : 0) + 2 * RM_T) * 4; }
 
 template <typename T, int DP, int MODE>
 __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_pieces a) {
@@ -195,8 +197,7 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
     float4 *Ks = (float4 *)smem, *Qs = Ks + RM_T * U;               // [64][D], 16-byte units permuted by the row
     float *Vs = (float *)(OUT ? Qs + RM_T * U : Qs);                // [64][128]
     float4 *Ps = (float4 *)(Vs + RM_T * 128);                       // [64][64] decayed q . k of the pairs, permuted likewise
-    float *red = (float *)Ps + (OUT ? RM_T * RM_T : 0);             // [64][4] sums of squares
-    float *gp = red + (OUT ? 4 * RM_T : 0);                         // g^0 .. g^64
+    float *gp = (float *)Ps + (OUT ? RM_T * RM_T : 0);              // g^0 .. g^64
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, nw = (Dv + 31) / 32, col = 32 * wave + l32;
     const float gamma = a.decay[h], kscale = 1.0f / sqrtf((float)D);
     if (wave == 0) {                                                // powers by doubling, which doubles a rounding error too: in 64 bits.  Lane l holds g^(l+1)
@@ -353,31 +354,15 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
                 for (int x = 0; x < 4; ++x) pairs(x, 0);
 #pragma unroll 2
                 for (int x = 4; x < 8; ++x) pairs(x, 1);
+                if (col < Dv) {                                     // as they are: the norm over a head's Dv columns spans wavefronts, and a gate's bytes are better read in rows
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt)
+                    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {                  // columns beyond Dv are zero
-                        if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-                        float ss = o[rt][r] * o[rt][r];
-#pragma unroll
-                        for (int off = 16; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-                        if (l32 == 0) red[(32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3)) * 4 + wave] = ss;
-                    }
-            }
-            __syncthreads();
-            if (col < Dv) {
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-                        const int i = 32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3);
-                        if (i >= nt) continue;
-                        float ss = 0.f;
-                        for (int w = 0; w < nw; ++w) ss += red[i * 4 + w];
-                        const float rn = 1.0f / sqrtf(ss / (float)Dv + a.eps), g = ld_f(src + (int64_t)(t0 + i) * a.ld + a.g_col + h * Dv + col);
-                        st_f((T *)a.out + (int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col, o[rt][r] * rn * (g / (1.0f + expf(-g))));
-                    }
+                        for (int r = 0; r < 16; ++r) {
+                            const int i = 32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3);
+                            if (i < nt) a.raw[(int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col] = o[rt][r];
+                        }
+                }
             }
         }
         if (wave < nw && (!OUT || last || t0 + RM_T < cnt)) {       // the state behind the group
@@ -454,14 +439,15 @@ template <typename T, int DP> static int rm_launch(const jl_retention_pieces &a,
     const int64_t ddv = (int64_t)a.D * a.Dv;
     retention_pieces_join_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64)), 256, 0, st>>>(a);
     outs<<<grid, 256, l1, st>>>(a);
-    return jl_check_launch("retention_pieces_kernel");
+    const int rc = jl_check_launch("retention_pieces_kernel");
+    return rc != JL_OK ? rc : jl_heads_out(a.raw, a.proj, a.dtype, a.ld, a.g_col, nullptr, a.N * a.H, a.H, a.Dv, a.eps, a.out, st);
 }
 
 extern "C" int jl_retention_pieces_run(const jl_retention_pieces *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_retention_pieces_run: null arguments");
     const jl_retention_pieces &a = *ap;
     if (a.B <= 0 || a.pieces <= 0) return JL_OK;
-    if (!a.proj || !a.decay || !a.state || !a.out || !a.scratch || !a.piece_rec || !a.req || !a.pos || (a.rot_dims && (!a.cos_t || !a.sin_t || a.table_len <= 0)))
+    if (!a.proj || !a.decay || !a.state || !a.out || !a.scratch || !a.raw || a.N <= 0 || !a.piece_rec || !a.req || !a.pos || (a.rot_dims && (!a.cos_t || !a.sin_t || a.table_len <= 0)))
         return jl_fail(JL_E_INVALID, "jl_retention_pieces_run: null pointer");
     if (!jl_retention_pieces_ok(a.dtype, a.D, a.Dv, a.rot_dims) || a.H <= 0 || a.H > 65535 || a.piece_tokens <= 0 || a.piece_tokens % RM_T || a.ld % 4 || (a.q_col | a.k_col | a.v_col) % 4 ||
         ((uintptr_t)a.proj % (a.dtype == JL_BF16 ? 8 : 16)) || ((uintptr_t)a.cos_t % 16) || ((uintptr_t)a.sin_t % 16))

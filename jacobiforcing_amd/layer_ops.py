@@ -573,7 +573,8 @@ def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: Ragged
         size = min(max(64, -(-total * H // RETENTION_WORKGROUPS) // 64 * 64), 1024)        # whole groups, as many pieces as the chip takes workgroups
         rec, req = batch.pieces(size)
         scratch = torch.empty((rec.shape[0], H, D, Dv), dtype=torch.float32, device=proj.device)
-        a = N.RetentionPieces(proj=proj.data_ptr(), piece_rec=rec.data_ptr(), req=req.data_ptr(), pos=batch.pos.data_ptr(), cos_t=cos.data_ptr() if rot_dims else None,
+        raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device)
+        a = N.RetentionPieces(raw=raw.data_ptr(), N=n, proj=proj.data_ptr(), piece_rec=rec.data_ptr(), req=req.data_ptr(), pos=batch.pos.data_ptr(), cos_t=cos.data_ptr() if rot_dims else None,
                               sin_t=sin.data_ptr() if rot_dims else None, decay=decay.data_ptr(), state=state.data_ptr(), scratch=scratch.data_ptr(), out=out.data_ptr(), ld=ld,
                               table_len=tl, q_col=cols[0], k_col=cols[1], v_col=cols[2], g_col=cols[3], dtype=_code(proj.dtype), B=batch.B, pieces=rec.shape[0], piece_tokens=size,
                               H=H, D=D, Dv=Dv, rot_dims=rot_dims, eps=float(eps))
@@ -947,7 +948,7 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
 # attention over keys and values built per head, the product that builds them.  ``key`` is the time the built form takes per key of its longest tile when the
 # chip is not full (a tile walks its keys in order; the 32-row kernel shares few tiles' keys out).  A step wholly on built keys has fewer launches (bmm, packing, bmm
 # and head order go: 95 -> 55 us of host time for small steps), a step that mixes the forms has more.
-LATENT_RATES = dict(narrow=330e12, wide=105e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
+LATENT_RATES = dict(narrow=330e12, wide=140e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
 # in float: the matrix form of the one-sweep kernel (narrow) or float multiply-adds (wide) over the latent
 LATENT_RATES_FLOAT = dict(narrow=60e12, wide=1.5e12, built=60e12, product=90e12, key64=130e-9, key32=180e-9, launches=-35e-6, both=80e-6)
 LATENT_BUILT_BYTES = 2 << 30          # keys and values built at a time
@@ -957,8 +958,8 @@ LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth build
 def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, window: int, dtype: torch.dtype = torch.bfloat16) -> List[int]:
     """The requests of a step whose keys and values are better built per head.  Over the latent a visible pair costs 2 H (2 R + rd) operations, over
     built keys 2 H (D + rd + Dv) — a third of it at R = 512, D = Dv = 128, rd = 64 — but every key is built first, 2 H R (D + Dv): worth it from some
-    hundred new tokens per request on, never for a decoded token.  Measured, us over the latent / built: 4 x 1024 tokens at 16 heads x 128, R 512: 1044 / 110,
-    one request of 128 behind 4000: 303 / 288, of 32: 132 / 259; 8 heads x 64, R 128, 4 x 256 behind 1500: 132 / 92, 1 x 256 behind 4000: 116 / 163."""
+    hundred new tokens per request on, never for a decoded token.  Measured, us over the latent / built: 4 x 1024 tokens at 16 heads x 128, R 512: 581 / 110,
+    one request of 512 behind 4000: 430 / 300, of 128: 193 / 286, of 32: 108 / 258; 8 heads x 64, R 128, 4 x 256 behind 1500: 108 / 91, 1 x 256 behind 4000: 105 / 165."""
     key = ("built", H, D, R, rd, Dv, window, dtype)
     chosen = batch._tiles.get(key)
     if chosen is None:
