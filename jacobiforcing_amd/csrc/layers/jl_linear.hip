@@ -120,7 +120,8 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 // place), two stages ahead of the products; four wavefronts hold a 32 x 32 quarter each, W's rows are the A operand, so that a lane ends with four neighbouring columns of a row.
 // What bounds it: a workgroup's way through its stages, 0.27 us each however many workgroups there are, until two per CU are busy.  us of GPU time against the library's product
 // (bfloat16, W from memory): 1024 x 1024 by 256 rows 7.8 / 8.3, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 520 x 1000 by 1024 7.0 / 10.1, by 1600 10.0 / 12.0; 192 x 768 by 1600 5.4 / 5.9;
-// 1024 x 3072 by 256 8.3 / 9.0; and 11 us less of host time.  Beyond the caller's line (layer_ops.linear_mid) it loses: 2048 x 2048 by 512 13.3 / 11.2, 1024 x 3072 by 1024 16.1 / 13.6, float
+// 1024 x 3072 by 256 8.3 / 9.0; 2048 x 2048 by 512 13.3 / 11.2; and 11 us less of host time.  Beyond the caller's line (layer_ops.linear_mid) it loses more: 4096 x 2048 by 256 20.4 / 14.4,
+// 1024 x 3072 by 1024 16.1 / 13.6, float
 // 1024 x 1024 by 512 22.5 / 12.7.  Larger tiles and deeper rings gained nothing there (128 x 128 by 8192 rows 100 / 52), nor did a share of the depth per wavefront without barriers.
 typedef float ld_f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ ld_f32x16 ld_mma(const bf16_t *, uint4 a, uint4 b, ld_f32x16 c) {

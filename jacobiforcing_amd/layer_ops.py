@@ -230,9 +230,12 @@ def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
 
 
 def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
-    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for a few hundred rows: 16-bit rows of up to 2 KB and no more than two 64 x 64 tiles per CU.  There its GPU
-    time is the library's give or take 2 us (1024 x 1024 by 128 rows 7.6 / 5.4, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4), and the call costs 11 us less of the host."""
-    return dtype == torch.bfloat16 and n > 0 and k <= 1024 and -(-n // 64) * -(-o // 64) <= 512
+    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for a few hundred rows: 16-bit rows of up to 2 KB and no more than two 64 x 64 tiles per CU, or of up to 4 KB
+    and one.  There its GPU time is the library's give or take 3 us (1024 x 1024 by 128 rows 7.6 / 5.4, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 2048 x 2048 by 512 13.3 / 11.2), and the call
+    costs 11 us less of the host, which such steps wait for (two portions of 50 beside 16 decoding requests at widths of 2048, us without / with the second line: Mikipel 1180 / 1122,
+    Safisun 1050 / 936, Voborax 1400 / 1247)."""
+    tiles = -(-n // 64) * -(-o // 64)
+    return dtype == torch.bfloat16 and n > 0 and (k <= 1024 and tiles <= 512 or k <= 2048 and tiles <= 256)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:

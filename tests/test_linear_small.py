@@ -43,7 +43,7 @@ def test_forms_it_does_not_take():
         LO.linear(torch.randn(3, 64, device=dev), w.bfloat16())
 
 
-@pytest.mark.parametrize("N,K,O,bias", [(65, 8, 1, True), (127, 56, 63, False), (129, 64, 65, True), (1000, 72, 130, False), (64, 1024, 4099, True), (700, 1016, 1000, True), (1, 512, 32000, False)])
+@pytest.mark.parametrize("N,K,O,bias", [(65, 8, 1, True), (127, 56, 63, False), (129, 64, 65, True), (1000, 72, 130, False), (64, 1024, 4099, True), (700, 1016, 1000, True), (1, 512, 32000, False), (100, 2048, 8000, True), (513, 1032, 1500, False)])
 def test_a_few_hundred_rows(N, K, O, bias):
     from jacobiforcing_amd import layer_ops as LO
     dev, dt = "cuda", torch.bfloat16
