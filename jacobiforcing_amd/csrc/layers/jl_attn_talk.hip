@@ -18,6 +18,12 @@
 constexpr int AT_KT = 32;
 constexpr int AT_BIAS = 5;              // bias entries per thread and tile at most (checked by the launch)
 
+// a bias times log2(e); a finite one stays finite (a mask of the type's lowest value is a number: a row that sees nothing else still has weights)
+__device__ __forceinline__ float at_log2_bias(float b) {
+    const float v = b * 1.44269504088896341f;
+    return __builtin_isinf(v) && !__builtin_isinf(b) ? __builtin_copysignf(__FLT_MAX__, b) : v;
+}
+
 static __host__ __device__ inline int at_bias_row(int TQ, int HF) { return (TQ + AT_KT - 1 + 31) / 32 * 32 + (HF < 32 ? 32 / HF : 1); }   // heads of a query meet different banks
 static size_t at_lds_bytes(int KU, int VU, int TQ, int HF, int NW) { return (NW > 1 ? 2 : 1) * ((size_t)AT_KT * (KU + VU) * 16 + AT_KT * 4 + (size_t)HF * at_bias_row(TQ, HF) * 4); }
 
@@ -130,12 +136,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
 #pragma unroll
             for (int it = 0; it < AT_BIAS; ++it) {
                 const int e = tid + it * THREADS;
-                if (e < n_bias) { const int y = e / HF; bias[(e - y * HF) * BR + y] = breg[it] * LOG2E; }
+                if (e < n_bias) { const int y = e / HF; bias[(e - y * HF) * BR + y] = at_log2_bias(breg[it]); }
             }
         if (MIX && NW == 1 && a.rel) {
             const int j0 = first_of(t);
 #pragma unroll 4
-            for (int e = tid; e < n_bias; e += THREADS) { const int y = e / HF; bias[(e - y * HF) * BR + y] = bias_of(e, j0) * LOG2E; }
+            for (int e = tid; e < n_bias; e += THREADS) { const int y = e / HF; bias[(e - y * HF) * BR + y] = at_log2_bias(bias_of(e, j0)); }
         }
     };
     look_up(t_lo);
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     const int GW = MIX ? G : 1;
     float *ml = a.scratch + (int64_t)n_tiles * TQ * S * H * GW * Dv + (row * H + h0 + hl) * 2;
     if ((!MIX || g == 0) && hi == 0) { ml[0] = m_run; ml[1] = l_run; }
-    if (!(l_run > 0.f) && m_run == -INFINITY) return;               // nothing seen: the share is not read
+    if (!(l_run > 0.f) && m_run == -INFINITY) return;               // nothing seen: the share counts for nothing (or, all shares like it, the row is not a number)
     float *o = a.scratch + ((row * H + h0 + hl) * GW + (MIX ? g : 0)) * Dv;
 #pragma unroll
     for (int y = 0; y < NDV; ++y)
@@ -253,7 +259,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
         }
 }
 
-// w[split][head] = 2 ** (m - M) / L, then out_h = sum over heads x of talk[h, x] sum over splits of w O_(x, g(h)), gated.  A wavefront per token where shares are whole (bytes bound it:
+// w[split][head] = 2 ** (m - M) / L (not a number where L is none or zero, as the softmax of such scores), then out_h = sum over heads x of talk[h, x] sum over splits of w O_(x, g(h)), gated.  A wavefront per token where shares are whole (bytes bound it:
 // 8192 tokens, 8 heads over 2 of 128 in 22 us); a workgroup per token (SPREAD), which adds up the shares of different heads on different wavefronts first, where they are not
 constexpr int AM_HEADS = 32;
 template <bool SPREAD>
@@ -282,10 +288,10 @@ __global__ __launch_bounds__(256) void attn_talk_mix_kernel(jl_attn_args a, int 
                 w[s * H + x] = e;
                 L += mls[s * H + x].y * e;
             }
-            const float inv = L > 0.f ? 1.0f / L : 0.f;
+            const float inv = L > 0.f ? 1.0f / L : NAN;
             for (int s = 0; s < S; ++s) w[s * H + x] *= inv;
         }
-    } else if (live && lane < H) w[lane] = ml[2 * lane + 1] > 0.f ? 1.0f / ml[2 * lane + 1] : 0.f;
+    } else if (live && lane < H) w[lane] = ml[2 * lane + 1] > 0.f ? 1.0f / ml[2 * lane + 1] : NAN;
     __syncthreads();
     // a head's sum over the shares, four columns of all value heads; an empty share (weight zero) holds nothing and is not looked at
     auto head_sum = [&](int x, int e) {
@@ -419,7 +425,7 @@ __global__ __launch_bounds__(256) void attn_narrow_join_kernel(jl_attn_args a, i
         v[3] = m > -INFINITY ? fmaf(w, p.w, v[3]) : v[3];
     }
     if (!in) return;
-    const float inv = L > 0.f ? a.out_scale / L : 0.f;
+    const float inv = L != 0.f ? a.out_scale / L : 0.f;             // a sum that is not a number reaches the outputs
     const bf16_t *gate = (const bf16_t *)a.gate;
     const int col = h * Dv + 4 * lane;
 #pragma unroll

@@ -107,3 +107,51 @@ def test_few_tokens(monkeypatch, H, G, Gv, D, Dv, counts, starts, kw, wgs):
         # weights and results are rounded to bfloat16, 2 ** -9 each; the cap's tanh is a few 1e-7 of the cap off
         assert err <= 2 * 2.0 ** -8, (b, err.item())
         r0 += c
+
+
+@pytest.mark.parametrize("what", ["lowest", "minus infinity", "not a number"])
+@pytest.mark.parametrize("counts,starts,wgs", [([70], [0], 1), ([70], [0], 4096), ([1, 1, 2, 1], [0, 5, 0, 900], 4096), ([1, 1, 2, 1], [0, 5, 0, 900], 1)])
+def test_values_at_the_types_ends(monkeypatch, what, counts, starts, wgs):
+    """A distance bias of the lowest value or of minus infinity on a query's own key (position 0 sees nothing else), and a cached key that is not a number: as the softmax in 64 bits."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, page, H, G, D = "cuda", 16, 4, 2, 64
+    monkeypatch.setattr(LO, "TALK_WORKGROUPS", wgs)
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    n, need = sum(counts), [-(-(c + s) // page) for c, s in zip(counts, starts)]
+    at = [sum(need[:b]) for b in range(len(need))]
+    batch = LO.RaggedBatch.build(counts, starts, list(range(len(counts))), [list(range(a, a + x)) for a, x in zip(at, need)], page, dev)
+    kp, vp, q, talk, rel = rnd(sum(need) * page, G * D).bfloat16(), rnd(sum(need) * page, G * D).bfloat16(), rnd(n, H * D).bfloat16(), torch.eye(H, device=dev) + 0.3 * rnd(H, H), rnd(1000, H)
+    if what == "not a number":
+        kp[[a * page + 3 for a in at], :D] = float("nan")            # position 3 of every request, under the first key head
+    else:
+        rel[0, 1] = torch.finfo(torch.float32).min if what == "lowest" else float("-inf")
+    stale = torch.full((1 << 22,), float("inf"), device=dev)         # what an allocation of the call may find in its memory
+    del stale
+    out, r0 = LO.attn_window(q, None, kp, vp, batch, H, G, D, D, D ** -0.5, 0, 0, rel, None, talk, float_out=True).double().view(n, H, D), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.arange(at[b] * page, at[b] * page + c + s, device=dev)
+        k, v = (x[tok].double().view(-1, G, D).repeat_interleave(H // G, 1).permute(1, 0, 2).contiguous() for x in (kp, vp))
+        i, j = torch.arange(s, s + c, device=dev).view(-1, 1), torch.arange(c + s, device=dev).view(1, -1)
+        sc = q[r0:r0 + c].double().view(c, H, D).permute(1, 0, 2).contiguous() @ k.transpose(1, 2).contiguous() * D ** -0.5 + rel.double()[(i - j).clamp(min=0)].permute(2, 0, 1)
+        p = torch.softmax(sc.masked_fill(j > i, float("-inf")), -1)
+        want = (torch.einsum("yx,xij->yij", talk.double(), p).contiguous() @ v).permute(1, 0, 2)
+        dead = torch.isnan(want).flatten(1).any(1)                   # rows with a sum that is none: all heads, they are mixed
+        assert (what != "lowest" or not bool(dead.any())) and torch.equal(torch.isnan(out[r0:r0 + c]).flatten(1).all(1), dead), (b, dead)
+        live = out[r0:r0 + c][~dead]
+        # as in test_talk
+        assert bool(torch.isfinite(live).all()) and (live - want[~dead]).norm() <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24) * want[~dead].norm(), b
+        r0 += c
+
+
+def test_a_key_that_is_not_a_number_reaches_a_decoded_token():
+    """... in the form without mixed heads: alone in its share of the keys it must not drop out."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, page, H, G, D = "cuda", 64, 4, 2, 64
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    batch = LO.RaggedBatch.build([1, 1], [640, 0], [0, 1], [list(range(11)), [11]], page, dev)
+    kp, vp, q = rnd(12 * page, G * D), rnd(12 * page, G * D), rnd(2, H * D)
+    kp[640, :D] = kp[11 * page, :D] = float("nan")                   # the last key of one request, the only one of the other
+    out = LO.attn_sweep(q, kp, vp, batch, H, G, D, D, D ** -0.5, 0).view(2, G, -1)
+    assert bool(torch.isnan(out[:, 0]).all()) and bool(torch.isfinite(out[:, 1]).all())
