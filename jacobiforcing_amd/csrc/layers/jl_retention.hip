@@ -177,6 +177,7 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // the scan: no operand is split or rounded.  q, k (rotated, scaled), v and the pairs' weights of the group lie in LDS as floats; the next group's rows
 // are on their way meanwhile.
 // What bounds it: 368 matrix instructions of 64 cycles per wavefront and group of 64 tokens at 128 x 128, and the phases of a group at one workgroup per CU.
+// Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups (a second pass over a group that holds one).
 // Outputs leave as floats and are normed and gated by rows in a launch of their own: in this one, a wavefront's sums over its 32 columns cost 160 exchanges per group and the gates
 // came two bytes at a time, four on their way (outputs 211 us then, 112 and 18 now).
 // Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 182 us, one prompt of 128
@@ -269,6 +270,7 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
             ((float4 *)Vs)[e] = to_float(rv[it]);                   // rows of 128 columns, those beyond Dv and tokens beyond the portion zero
         }
         __syncthreads();
+        int broken = RM_T;                                          // the group's first token whose value in this lane's column is not finite
         if (t0 + RM_T < cnt) fetch(t0 + RM_T);                      // in flight while this group is multiplied
         for (int e = tid; e < nt * hu; e += 256) {                  // rotation in place: units u and u + half / 4 of a row
             const int tt = e / hu, u = e - tt * hu;
@@ -312,55 +314,66 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
             __syncthreads();
             rm_f32x16 o[2];
             if (wave < nw) {
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[rt][r] = 0.f;
-                }
-#pragma unroll
-                for (int x = 0; x < U / 2; ++x) {
-                    if (x % 2 == 0) __builtin_amdgcn_sched_barrier(0);      // all operands at once would not fit the registers
+                for (bool first_time = true;; first_time = false) {
 #pragma unroll
                     for (int rt = 0; rt < 2; ++rt) {
-                        const int i = 32 * rt + l32;
-                        const float4 q = Qs[i * U + at(i, 2 * x + hi)];
-                        o[rt] = rm_mma(q.x, S[x >> 2][4 * (x & 3)], o[rt]);
-                        o[rt] = rm_mma(q.y, S[x >> 2][4 * (x & 3) + 1], o[rt]);
-                        o[rt] = rm_mma(q.z, S[x >> 2][4 * (x & 3) + 2], o[rt]);
-                        o[rt] = rm_mma(q.w, S[x >> 2][4 * (x & 3) + 3], o[rt]);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[rt][r] = 0.f;
                     }
+#pragma unroll
+                    for (int x = 0; x < U / 2; ++x) {
+                        if (x % 2 == 0) __builtin_amdgcn_sched_barrier(0);      // all operands at once would not fit the registers
+#pragma unroll
+                        for (int rt = 0; rt < 2; ++rt) {
+                            const int i = 32 * rt + l32;
+                            const float4 q = Qs[i * U + at(i, 2 * x + hi)];
+                            o[rt] = rm_mma(q.x, S[x >> 2][4 * (x & 3)], o[rt]);
+                            o[rt] = rm_mma(q.y, S[x >> 2][4 * (x & 3) + 1], o[rt]);
+                            o[rt] = rm_mma(q.z, S[x >> 2][4 * (x & 3) + 2], o[rt]);
+                            o[rt] = rm_mma(q.w, S[x >> 2][4 * (x & 3) + 3], o[rt]);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[rt][r] *= gp[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3) + 1];
+                    auto pairs = [&](int x, int first) {                // eight keys; no key of the second half is visible to the first half's queries
+                        float v[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = Vs[(8 * x + 4 * hi + i) * 128 + col];
+#pragma unroll
+                        for (int rt = 0; rt < 2; ++rt) {
+                            if (rt < first) continue;
+                            const int i = 32 * rt + l32;
+                            const float4 p = Ps[i * 16 + at(i, 2 * x + hi)];
+                            o[rt] = rm_mma(p.x, v[0], o[rt]);
+                            o[rt] = rm_mma(p.y, v[1], o[rt]);
+                            o[rt] = rm_mma(p.z, v[2], o[rt]);
+                            o[rt] = rm_mma(p.w, v[3], o[rt]);
+                        }
+                    };
+#pragma unroll 2
+                    for (int x = 0; x < 4; ++x) pairs(x, 0);
+#pragma unroll 2
+                    for (int x = 4; x < 8; ++x) pairs(x, 1);
+                    // A value that is not finite makes every sum of its column none, through weights of zero also those of tokens in front of it.  Then, once more without it: what it
+                    // reaches is set below.  (All keys enter a row of the second half.)
+                    if (!first_time || !__any(!__builtin_isfinite(o[1][0]))) break;
+                    for (int j = RM_T - 1; j >= 0; --j)
+                        if (!__builtin_isfinite(Vs[j * 128 + col])) {
+                            broken = j;
+                            if (hi) Vs[j * 128 + col] = 0.f;        // the column's other lane looks at it in the same instruction
+                        }
+                    if (!__any(broken < RM_T)) break;
                 }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[rt][r] *= gp[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3) + 1];
-                auto pairs = [&](int x, int first) {                // eight keys; no key of the second half is visible to the first half's queries
-                    float v[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = Vs[(8 * x + 4 * hi + i) * 128 + col];
-#pragma unroll
-                    for (int rt = 0; rt < 2; ++rt) {
-                        if (rt < first) continue;
-                        const int i = 32 * rt + l32;
-                        const float4 p = Ps[i * 16 + at(i, 2 * x + hi)];
-                        o[rt] = rm_mma(p.x, v[0], o[rt]);
-                        o[rt] = rm_mma(p.y, v[1], o[rt]);
-                        o[rt] = rm_mma(p.z, v[2], o[rt]);
-                        o[rt] = rm_mma(p.w, v[3], o[rt]);
-                    }
-                };
-#pragma unroll 2
-                for (int x = 0; x < 4; ++x) pairs(x, 0);
-#pragma unroll 2
-                for (int x = 4; x < 8; ++x) pairs(x, 1);
                 if (col < Dv) {                                     // as they are: the norm over a head's Dv columns spans wavefronts, and a gate's bytes are better read in rows
 #pragma unroll
                     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const int i = 32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3);
-                            if (i < nt) a.raw[(int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col] = o[rt][r];
+                            if (i < nt) a.raw[(int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col] = i < broken ? o[rt][r] : NAN;
                         }
                 }
             }
@@ -384,6 +397,11 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
                     }
                 }
             }
+            if (OUT && broken < RM_T)
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) S[t][r] = NAN;
         }
     }
     float *dst = OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : sp;

@@ -56,3 +56,27 @@ def test_pieces(monkeypatch, dtype, H, D, Dv, rot, workgroups, counts, starts):
         assert (r - o).norm() <= (2.0 ** -8 if dtype == "bfloat16" else 5e-6) * o.norm(), (b, "outputs")
         r0 += c
     assert torch.equal(state[0], before[0]) and torch.equal(state[B + 1], before[B + 1])
+
+
+@pytest.mark.parametrize("dtype,value", [("bfloat16", float("inf")), ("float32", float("nan")), ("float32", float("-inf"))])
+def test_values_that_are_not_finite_reach_later_tokens_only(dtype, value):
+    """... of their own head and request: what other rows hold is what it is without them, bit for bit."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt, H, D, Dv = "cuda", getattr(torch, dtype), 3, 64, 96
+    g = torch.Generator(device=dev).manual_seed(5)
+    counts = [300, 70]
+    batch = LO.RaggedBatch.build(counts, [0, 0], [0, 1], [[0, 1, 2, 3, 4], [5, 6]], 64, dev)
+    cols = (0, H * D, 2 * H * D, 2 * H * D + H * Dv)
+    proj = torch.randn(370, cols[3] + H * Dv, generator=g, device=dev).to(dt)
+    run = lambda p, st: LO.retention(p, cols, batch, H, D, Dv, 0, None, None, torch.full((H,), 0.9, device=dev), 1e-5, st).view(370, H, Dv)
+    states = [torch.zeros(2, H, D, Dv, device=dev) for _ in range(2)]
+    want = run(proj, states[0])
+    first = {0: 37, 1: 63, 2: 64}                                    # per head: within a group of 64, its last token, the next one's first
+    for h, t in first.items():
+        proj[t, cols[2] + h * Dv + 11 * h] = value
+    proj[300 + 69, cols[2] + 5] = value                              # the other request's last token
+    got = run(proj, states[1])
+    for h, t in first.items():
+        assert torch.equal(got[:t, h], want[:t, h]) and bool(torch.isnan(got[t:300, h]).any(-1).all()), h
+        assert torch.equal(got[300:369, h], want[300:369, h]) and not bool(torch.isfinite(states[1][0, h]).all())
+    assert bool(torch.isnan(got[369, 0]).any()) and torch.equal(got[369, 1:], want[369, 1:]) and torch.equal(states[1][1, 1:], states[0][1, 1:])
