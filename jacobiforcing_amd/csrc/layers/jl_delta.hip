@@ -295,12 +295,15 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 // chunks with 32 columns of one head's state in accumulators.  Everything is a 32-bit number, as in the scan; the sums c are 64-bit (differences of long sums).  A token
 // that does not exist has k = q = v = 0, beta = 0, g = 1.  ln g below -1e4 counts as -1e4: e^ of it is zero all the same, and differences stay numbers.
 //
+// What is not finite in a token's key, value, decay or beta reaches its own and later tokens' outputs and the state, as in the scan, though products run over whole chunks: it is left
+// out of them and set afterwards (in rare branches: W1's rows from that token on, the outputs' rows from a correction's token on).
+//
 // v_mfma_f32_32x32x2_f32: lane l supplies row (A) or column (B) l % 32 at depth l / 32; accumulator r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  Four
 // instructions take a unit of 16 bytes per lane, depths 8 u + 4 (l / 32) + i of unit u — which is also how four accumulators of a lane lie, so results are the next
 // product's operand as they are: between the kernels (every operand as units [unit][lane], read as 1 KB per wavefront straight into registers, a chunk ahead) and in LDS
 // between the wavefronts of a chain.  T comes from 16 x 16 blocks by substitution, joined by products, on one wavefront while the others make P.
 // What bounds it: the chain's 128 matrix instructions of 64 cycles per chunk on the busiest of its four wavefronts (D = 128; 58 % of its time), and in the chunks' kernel the
-// phases of a workgroup that wait for each other (two workgroups per CU at 77.5 KB of LDS; with one, 302 us instead of 198).
+// phases of a workgroup that wait for each other (two workgroups per CU at 79 104 bytes of LDS; with one, 302 us instead of 198).
 // Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 446 us (chunks 198, chain 214,
 // norm 34); 8 heads, one portion of 128 80 -> 45; 16 heads, 777 + 300 tokens beside 30 single ones 566 -> 148; float, 8 heads, 1021 + 851 + 681 tokens 587 -> 149.
 constexpr int DK_T = 64;
@@ -342,6 +345,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
     float4 *Ks = (float4 *)smem, *Qs = Ks + DK_T * U, *Am = Qs + DK_T * U;          // rows of units, permuted by the row
     double *cs = (double *)(Am + 3 * 256);                                         // [64] sums of ln g
     float *bs = (float *)(cs + DK_T), *bg = bs + DK_T;                             // [64] beta; -beta e^c
+    int *flawS = (int *)(bg + DK_T);                                               // [64] a key that is not a number
     const int hl = blockIdx.x % nh, h = h0 + hl, chunk = blockIdx.x / nh, per = a.H / a.G, kh = h / per, D = a.D, Dv = a.Dv;
     const int row0 = a.chunk_rec[4 * chunk], cnt = a.chunk_rec[4 * chunk + 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
@@ -366,7 +370,15 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
         for (int off = 1; off < U; off <<= 1) { sq += __shfl_xor(sq, off, 64); sk += __shfl_xor(sk, off, 64); }
         const float rq = tt < cnt ? a.q_scale / sqrtf(sq + a.unit_eps) : 0.f, rk = tt < cnt ? 1.0f / sqrtf(sk + a.unit_eps) : 0.f;
         Qs[tt * U + at(tt, u)] = make_float4(q.x * rq, q.y * rq, q.z * rq, q.w * rq);
-        Ks[tt * U + at(tt, u)] = make_float4(k.x * rk, k.y * rk, k.z * rk, k.w * rk);
+        k = make_float4(k.x * rk, k.y * rk, k.z * rk, k.w * rk);
+        const uint64_t none = __ballot(__builtin_isnan((k.x + k.y) + (k.z + k.w)));   // elements of a unit vector: what is not finite before is not a number now
+        bool flaw = false;                                                          // the row's
+        if (none) {
+            flaw = none >> (lane & ~(U - 1)) & ((1ull << U) - 1);
+            if (flaw) k = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        Ks[tt * U + at(tt, u)] = k;
+        if (u == 0) flawS[tt] = flaw;
     }
     if (wave == 0) {
         float lg = 0.f, beta = 0.f;
@@ -391,6 +403,14 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
         head[z.p + 3 * 1024 + DK_T + lane] = expf((float)(end - c));
     }
     __syncthreads();
+    // from the first token with a key, decay or beta that is not a number on: nothing here that zeros would spread to the tokens in front of it; W1 says so instead
+    const uint64_t flaws = __ballot(flawS[lane] || !__builtin_isfinite((float)cs[lane]) || !__builtin_isfinite(bs[lane]));
+    const int broken = flaws ? __builtin_ctzll(flaws) : DK_T;                       // the same in all wavefronts
+    if (broken < DK_T) {
+        __syncthreads();
+        if (wave == 0 && lane >= broken) { bs[lane] = bg[lane] = 0.f; cs[lane] = broken > 0 ? cs[broken - 1] : 0.0; }
+        __syncthreads();
+    }
     // a quarter [32 t, 32 j] of K K^T or Q K^T: lane l ends with t = 32 ti + l % 32, unit y the four j at 32 tj + 8 y + 4 (l / 32)
     auto pairs = [&](const float4 *rows, int ti, int tj, bool diagonal, float row_factor, auto &&store) {
         const int t = 32 * ti + l32, j = 32 * tj + l32;
@@ -530,6 +550,29 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
                 if (y < 4) acc[0] = dk_mma(trow(0, y), f[y], acc[0]);
                 acc[1] = dk_mma(trow(1, y), f[y], acc[1]);
             }
+            // all values of a column enter a row of the second half, one that is not finite as not a number: the same without it
+            if (broken < DK_T || __any(!__builtin_isfinite(acc[1][0]))) {
+                int none = broken;                                                 // this lane's column is not a number from here on
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+#pragma unroll 1
+                for (int y = 0; y < 8; ++y) {
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int t = 8 * y + 4 * hi + i;
+                        v[i] = t < cnt && col < Dv ? vp[t * a.qkv_ld] * bs[t] : 0.f;
+                        if (!__builtin_isfinite(v[i])) { v[i] = 0.f; none = min(none, t); }
+                    }
+                    if (y < 4) acc[0] = dk_mma(trow(0, y), make_float4(v[0], v[1], v[2], v[3]), acc[0]);
+                    acc[1] = dk_mma(trow(1, y), make_float4(v[0], v[1], v[2], v[3]), acc[1]);
+                }
+                none = min(none, __shfl_xor(none, 32, 64));
+#pragma unroll
+                for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[ti][r] = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3) < none ? acc[ti][r] : NAN;
+            }
 #pragma unroll
             for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
@@ -545,6 +588,7 @@ template <int DP>
 __global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, int h0, int nh, float *__restrict__ raw) {
     constexpr int NU = DP / 8, DT = DP / 32;
     __shared__ float4 Sf[NU * 64], Uf[8 * 64], Ug[8 * 64];
+    __shared__ int noneS[2][32];                                    // the first token of a half chunk whose correction is not finite, per column
     const int nv = (a.Dv + 31) / 32, lin = blockIdx.x >> 3, vt = lin % nv, bh = (lin / nv) * 8 + (blockIdx.x & 7);
     if (bh >= a.B * nh) return;
     const int b = bh / nh, hl = bh - b * nh, h = h0 + hl, per = a.H / a.G, D = a.D, Dv = a.Dv;
@@ -619,9 +663,21 @@ __global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, 
         }
         acc += (part[0] + part[1]) + part[2];
         if (maker) {
+            float zero[4] = {0.f, 0.f, 0.f, 0.f};                   // not a number if a correction is not finite
+#pragma unroll
+            for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(acc[r], 0.f, zero[r & 3]);
+            dk_f32x16 u = acc;
+            int none = DK_T;
+            if (__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f)) {      // the state takes it up, the outputs of the tokens in front of it must not meet it
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (!__builtin_isfinite(acc[r])) { u[r] = 0.f; none = min(none, 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3)); }
+                none = min(none, __shfl_xor(none, 32, 64));
+            }
+            if (hi == 0) noneS[ti][l32] = none;
 #pragma unroll
             for (int y = 0; y < 4; ++y) {
-                Uf[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y], acc[4 * y + 1], acc[4 * y + 2], acc[4 * y + 3]);
+                Uf[(4 * ti + y) * 64 + lane] = make_float4(u[4 * y], u[4 * y + 1], u[4 * y + 2], u[4 * y + 3]);
                 Ug[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y] * sc[y].x, acc[4 * y + 1] * sc[y].y, acc[4 * y + 2] * sc[y].z, acc[4 * y + 3] * sc[y].w);
             }
         } else
@@ -653,6 +709,10 @@ __global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, 
 #pragma unroll
                 for (int y = 4; y < 8; ++y) acc = dk_mma(fp[y], Uf[y * 64 + lane], acc);
             acc += part[0];
+            const int none = min(noneS[0][l32], noneS[1][l32]);
+            if (__any(none < DK_T))
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[r] = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3) < none ? acc[r] : NAN;
 #pragma unroll
             for (int y = 0; y < 8; ++y)
                 if (y < 4 || ti) fp[y] = q.p[y * 64];
@@ -743,7 +803,7 @@ extern "C" int64_t jl_delta_chunks_floats(int32_t chunks, int32_t heads, int32_t
 }
 
 template <typename T, int DP> static int delta_chunks_launch(const jl_delta_chunks &a, hipStream_t st) {
-    const size_t lds = (size_t)(2 * DK_T * DP + 3 * 1024 + 2 * DK_T) * 4 + DK_T * 8;
+    const size_t lds = (size_t)(2 * DK_T * DP + 3 * 1024 + 3 * DK_T) * 4 + DK_T * 8;
     auto chunk = delta_chunk_kernel<T, DP>;
     hipError_t e = hipFuncSetAttribute((const void *)chunk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_delta_chunks_run: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));

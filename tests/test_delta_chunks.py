@@ -72,3 +72,32 @@ def test_chunks(monkeypatch, dtype, H, G, D, Dv, counts, starts, keys, floats):
         assert err(got[r0:r0 + c].view(c, H, Dv), o) <= 1.5 * err(scan[r0:r0 + c].view(c, H, Dv), o) + slack, (b, "outputs")
         r0 += c
     assert torch.equal(state[0], before[0]) and torch.equal(state[B + 1], before[B + 1])
+
+
+@pytest.mark.parametrize("what,value", [("v", float("nan")), ("v", float("inf")), ("k", float("nan")), ("k", float("-inf")), ("a", float("nan")), ("b", float("nan")), ("q", float("inf"))])
+@pytest.mark.parametrize("D,Dv", [(64, 40), (128, 128)])
+def test_what_is_not_finite_reaches_later_tokens_only(D, Dv, what, value):
+    """... of the heads that read it: what other rows and heads hold is what it is without it, bit for bit."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, G, n = "cuda", 4, 2, 300
+    g = torch.Generator(device=dev).manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    batch = LO.RaggedBatch.build([n, 70], [0, 9], [0, 1], [[0, 1, 2, 3, 4], [5, 6]], 64, dev)
+    cols, pcols = (0, G * D, 2 * G * D), (0, H, 2 * H)
+    qkv, proj = rnd(n + 70, 2 * G * D + H * Dv), rnd(n + 70, 2 * H + H * Dv)
+    a_log, bias, w, start = rnd(H), rnd(H), 1 + 0.1 * rnd(Dv), rnd(2, H, D, Dv)
+    run = lambda st: LO.delta_rule(qkv, cols, proj, pcols, a_log, bias, w, batch, H, G, D, Dv, 1e-6, D ** -0.5, 1e-5, st).view(n + 70, H, Dv)
+    for t in (0, 21, 40, 63, 64, 190, n - 1):                        # within blocks of 16, 32 and 64 tokens, at their ends, in the last chunk
+        states = [start.clone(), start.clone()]
+        want = run(states[0])
+        x, at, heads = {"q": (qkv, cols[0] + D + 3, [2, 3]), "k": (qkv, cols[1] + D + 3, [2, 3]), "v": (qkv, cols[2] + 2 * Dv + 3, [2]), "a": (proj, pcols[0] + 2, [2]),
+                        "b": (proj, pcols[1] + 2, [2])}[what]
+        kept, x[t, at] = x[t, at].clone(), value
+        got = run(states[1])
+        x[t, at] = kept
+        others = [h for h in range(H) if h not in heads]
+        assert torch.equal(got[:t], want[:t]) and torch.equal(got[n:], want[n:]) and torch.equal(got[:, others], want[:, others]), t
+        assert torch.equal(states[1][1], states[0][1]) and torch.equal(states[1][0, others], states[0][0, others]), t
+        last = t + 1 if what == "q" else n
+        assert bool(torch.isnan(got[t:last, heads]).any(-1).all()) and torch.equal(got[last:n], want[last:n]), t
+        assert all(bool(torch.isfinite(states[1][0, h]).all()) == (what == "q") for h in heads), t
