@@ -26,7 +26,7 @@ NARROW_WORKGROUPS = 2048              # attention of a few tokens per request: s
 BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
-RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
+RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
 SCAN_PIECES_FROM, SCAN_WORKGROUPS = 32, 512     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
@@ -546,6 +546,20 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
     return out
 
 
+def retention_pieces_from(counts: Sequence[int], H: int, D: int) -> int:
+    """From how many tokens on the requests of a step run in pieces, the others in the scan behind them (0: all in the scan).  A round of pieces (one workgroup per CU) takes 37 us at
+    128 x 128, 18 at 64 x 64, however few tokens they hold; the scan 8.5 and 5.3 us per token of its longest portion, up to 1024 or 4096 (request, head) pairs at a time, and the more
+    requests it has besides, the less a longer portion shows.  us, scan of all / all in pieces / this rule: 8 heads of 128, 8 tokens and 250 x 1 101 / 319 / 101, 777 + 300 and 30 x 1
+    1063 / 101 / 93, 100 x 8 96 / 151 / 96, 100 x 16 165 / 158 / 158; 32 heads, 8 and 30 x 1 95 / 163 / 71, 40 + 10 and 60 x 1 360 / 323 / 113, 10 x 10 and 60 x 1 116 / 359 / 116; 16 heads
+    of 64, 200 x 20 153 / 255 / 153, 700, 40 x 10 and 40 x 1 746 / 130 / 112."""
+    long = sum(c >= RETENTION_PIECES_FROM for c in counts)
+    rounds = -(-long * H // 256)
+    least = max(RETENTION_PIECES_FROM, min(4 * rounds, 16) if D > 64 else min(3 * rounds, 48), 3 + (len(counts) - long) * H // 230)
+    if max(counts) < least:
+        return 0
+    return 1 if len(counts) * H < 256 else least                     # single tokens beside them where CUs are free: a launch less (8 heads, 8 and 30 x 1 53 / 62 us)
+
+
 def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: RaggedBatch, H: int, D: int, Dv: int, rot_dims: int,
               cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], decay: torch.Tensor, eps: float, state: torch.Tensor) -> torch.Tensor:
     """proj [N, ld] with q, k, v, gate at ``cols``; state [slots, H, D, Dv] float (updated in place).  Returns [N, H*Dv]."""
@@ -569,19 +583,23 @@ def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: Ragged
         N.check_layers(L.jl_retention(_ptr(proj), _code(proj.dtype), ld, cols[0], cols[1], cols[2], cols[3], _ptr(records), count, H, D, Dv,
                                       rot_dims, _ptr(cos), _ptr(sin), tl, _ptr(decay), float(eps), _ptr(where), _ptr(out), mode, st), what)
 
-    longest = max(batch.counts)
-    if (longest >= RETENTION_PIECES_FROM and L.jl_retention_pieces_ok(_code(proj.dtype), D, Dv, rot_dims) and ld % 4 == 0 and not any(c % 4 for c in cols[:3]) and
+    least = batch._tiles.get(("retention", H, D))
+    if least is None:
+        least = batch._tiles[("retention", H, D)] = retention_pieces_from(batch.counts, H, D)
+    if (least and L.jl_retention_pieces_ok(_code(proj.dtype), D, Dv, rot_dims) and ld % 4 == 0 and not any(c % 4 for c in cols[:3]) and
             proj.data_ptr() % (8 if proj.dtype == torch.bfloat16 else 16) == 0 and (not rot_dims or (cos.data_ptr() | sin.data_ptr()) % 16 == 0)):
-        total = sum(batch.counts)
+        total = sum(c for c in batch.counts if c >= least)
         size = min(max(64, -(-total * H // RETENTION_WORKGROUPS) // 64 * 64), 1024)        # whole groups, as many pieces as the chip takes workgroups
-        rec, req = batch.pieces(size)
+        rec, req, rest = (*batch.pieces(size), None) if least == 1 else batch.long_pieces(size, least)[:3]
         scratch = torch.empty((rec.shape[0], H, D, Dv), dtype=torch.float32, device=proj.device)
         raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device)
         a = N.RetentionPieces(raw=raw.data_ptr(), N=n, proj=proj.data_ptr(), piece_rec=rec.data_ptr(), req=req.data_ptr(), pos=batch.pos.data_ptr(), cos_t=cos.data_ptr() if rot_dims else None,
                               sin_t=sin.data_ptr() if rot_dims else None, decay=decay.data_ptr(), state=state.data_ptr(), scratch=scratch.data_ptr(), out=out.data_ptr(), ld=ld,
-                              table_len=tl, q_col=cols[0], k_col=cols[1], v_col=cols[2], g_col=cols[3], dtype=_code(proj.dtype), B=batch.B, pieces=rec.shape[0], piece_tokens=size,
+                              table_len=tl, q_col=cols[0], k_col=cols[1], v_col=cols[2], g_col=cols[3], dtype=_code(proj.dtype), B=req.shape[0], pieces=rec.shape[0], piece_tokens=size,
                               H=H, D=D, Dv=Dv, rot_dims=rot_dims, eps=float(eps))
         N.check_layers(L.jl_retention_pieces_run(C.byref(a), st), "jl_retention_pieces_run")
+        if rest is not None and rest.shape[0]:                       # behind it: its norm passes over all rows
+            scan(rest, rest.shape[0], state, 0, "jl_retention")
         return out
     plan = batch.chunks(RETENTION_CHUNK)
     if plan is None:                                    # decoded tokens and short portions: one scan per request

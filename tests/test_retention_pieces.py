@@ -80,3 +80,26 @@ def test_values_that_are_not_finite_reach_later_tokens_only(dtype, value):
         assert torch.equal(got[:t, h], want[:t, h]) and bool(torch.isnan(got[t:300, h]).any(-1).all()), h
         assert torch.equal(got[300:369, h], want[300:369, h]) and not bool(torch.isfinite(states[1][0, h]).all())
     assert bool(torch.isnan(got[369, 0]).any()) and torch.equal(got[369, 1:], want[369, 1:]) and torch.equal(states[1][1, 1:], states[0][1, 1:])
+
+
+@pytest.mark.parametrize("H,D,counts,least", [(32, 128, [8] + [1] * 20 + [40, 7], 8), (64, 64, [70, 3, 9, 1, 200], 8), (40, 100, [20, 130] + [1] * 11 + [6], 8), (48, 20, [1] * 50 + [20, 9], 13)])
+def test_portions_of_both_kinds(H, D, counts, least):
+    """Steps whose short portions go through the scan behind the others' pieces: as all of them through the scan."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, g, n, B = "cuda", torch.Generator(device="cuda").manual_seed(H), sum(counts), len(counts)
+    assert LO.retention_pieces_from(counts, H, D) == least
+    starts = [(7 * b) % 30 for b in range(B)]
+    run = lambda batch, st: LO.retention(proj, (0, H * D, 2 * H * D, 3 * H * D), batch, H, D, D, 0, None, None, decay, 1e-5, st)
+    proj, decay, start = torch.randn(n, 4 * H * D, generator=g, device=dev), torch.linspace(0.9, 1.0, H, device=dev), torch.randn(B, H, D, D, generator=g, device=dev)
+    outs, states = [], []
+    for scan in (False, True):
+        batch, st = LO.RaggedBatch.build(counts, starts, list(range(B)), [list(range(4 * b, 4 * b + 4)) for b in range(B)], 64, dev), start.clone()
+        if scan:
+            batch._tiles[("retention", H, D)] = 0
+        outs.append(run(batch, st).double())
+        states.append(st.double())
+        assert any(k[0] == "long" for k in batch._tiles if isinstance(k, tuple)) != scan
+    short = torch.repeat_interleave(torch.tensor([c < least for c in counts], device=dev), torch.tensor(counts, device=dev))
+    assert torch.equal(outs[0][short], outs[1][short])
+    # sums of 32-bit products in another order, normed: as in test_pieces
+    assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[1].norm() and (states[0] - states[1]).norm() <= 4e-6 * states[1].norm()
