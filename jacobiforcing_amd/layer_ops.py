@@ -30,7 +30,7 @@ RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions f
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
 SCAN_PIECES_FROM, SCAN_WORKGROUPS = 32, 512     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
-DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
+DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (alone in its step; else delta_chunks_from.  us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
 DELTA_SCRATCH_FLOATS = 256 << 20     # scratch of those chunks at most (1 GiB: more heads than it holds take turns), as long as it holds one key head's
 
 
@@ -1165,6 +1165,33 @@ def short_conv(x: torch.Tensor, col: int, C_: int, w: torch.Tensor, batch: Ragge
     return out
 
 
+def delta_chunks_from(counts: Sequence[int], H: int, D: int) -> int:
+    """From how many tokens on the requests of a step go through the delta rule in chunks, the others behind them in the forms for short portions (0: none of them).  Portions of
+    DELTA_CHUNKS_FROM tokens on are worth it alone; beside other requests the times of both ways are estimated, us per chunk of the longest, chunk and head, token of the columns' longest, token
+    and head, request and head, token of the others' longest.  At widths of 64 the columns' walk is the faster one as soon as it fills the chip.  us, columns / chunks from 64 tokens on /
+    this rule: 16 heads of 64, 100 x 100 214 / 404 / 214, 30 x 200 164 / 227 / 164; 8 heads of 128, 70 and 10 x 31 56 / 140 / 56, 300 + 63 174 / 104 / 65, 64 and 200 x 1 131 / 117 / 117,
+    100 x 64 333 / 225 / 225."""
+    if max(counts) < DELTA_CHUNKS_FROM or len(counts) == 1:
+        return DELTA_CHUNKS_FROM if max(counts) >= DELTA_CHUNKS_FROM else 0
+    c = np.asarray(counts)
+    first, chain, chunk, step, token, request, alone, single = (30, 6.7, 0.28, 0.6, 5.5e-3, 0.05, 2.7, 0.045) if D > 64 else (24, 4.9, 0.145, 0.49, 1.34e-3, 6e-3, 1.4, 0.012)
+
+    def others(r):
+        if r.size == 0:
+            return 0.0
+        longest, tokens, pairs = int(r.max()), int(r.sum()) * H, r.size * H
+        if longest >= DELTA_COLUMNS_FROM:
+            return 8 + max(step * longest, 0.6 * step * longest + token * tokens + request * pairs)
+        return 8 + max(alone * longest, single * pairs + 0.012 * (tokens - pairs))
+
+    best, least = others(c), 0
+    for m in (2, 8, 16, DELTA_COLUMNS_FROM, 64):
+        n = -(-c[c >= m] // 64)
+        t = first + max(chain * int(n.max()), chunk * int(n.sum()) * H) + others(c[c < m]) if n.size else best
+        best, least = (t, m) if t < best else (best, least)
+    return least
+
+
 def delta_rule(qkv: torch.Tensor, cols: Tuple[int, int, int], proj: torch.Tensor, pcols: Tuple[int, int, int], a_log: torch.Tensor, dt_bias: torch.Tensor,
                norm_w: torch.Tensor, batch: RaggedBatch, H: int, G: int, D: int, Dv: int, unit_eps: float, q_scale: float, eps: float,
                state: torch.Tensor) -> torch.Tensor:
@@ -1181,11 +1208,15 @@ def delta_rule(qkv: torch.Tensor, cols: Tuple[int, int, int], proj: torch.Tensor
     for t, k in ((a_log, H), (dt_bias, H), (norm_w, Dv)):
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == k, "delta_rule: a_log, dt_bias float [H], norm_w float [Dv]")
     out = torch.empty((n, H * Dv), dtype=proj.dtype, device=proj.device)
-    longest = max(batch.counts) if not os.environ.get("JL_DELTA_NO_COLUMNS") else 1          # A/B switch for measurements
+    longest, least = max(batch.counts), batch._tiles.get(("delta", H, D))
+    if least is None:
+        least = batch._tiles[("delta", H, D)] = delta_chunks_from(batch.counts, H, D)
+    if os.environ.get("JL_DELTA_NO_COLUMNS"):                               # A/B switch for measurements
+        longest, least = 1, 0
     raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device) if longest >= DELTA_COLUMNS_FROM else None
     seq, B = batch.seq, batch.B
-    if longest >= DELTA_CHUNKS_FROM and N.layers().jl_delta_chunks_ok(D, Dv) and (qkv.shape[1] | cols[0] | cols[1]) % 4 == 0 and qkv.data_ptr() % 16 == 0:
-        rec, req, seq, longest = batch.long_pieces(64, DELTA_CHUNKS_FROM)
+    if least and N.layers().jl_delta_chunks_ok(D, Dv) and (qkv.shape[1] | cols[0] | cols[1]) % 4 == 0 and qkv.data_ptr() % 16 == 0:
+        rec, req, seq, longest = batch.long_pieces(64, least)
         B, chunks, per = seq.shape[0], rec.shape[0], H // G
         floats = lambda heads: N.layers().jl_delta_chunks_floats(chunks, heads, H, G, D, Dv)
         heads = min(H, max(1, DELTA_SCRATCH_FLOATS // floats(per)) * per)

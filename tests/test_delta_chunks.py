@@ -101,3 +101,22 @@ def test_what_is_not_finite_reaches_later_tokens_only(D, Dv, what, value):
         last = t + 1 if what == "q" else n
         assert bool(torch.isnan(got[t:last, heads]).any(-1).all()) and torch.equal(got[last:n], want[last:n]), t
         assert all(bool(torch.isfinite(states[1][0, h]).all()) == (what == "q") for h in heads), t
+
+
+@pytest.mark.parametrize("H,G,D,counts,least", [(16, 16, 64, [777] + [40] * 100 + [1], 64), (8, 2, 128, [300, 63, 5, 1, 1], 2), (8, 2, 128, [300] + [8] * 50 + [1], 16), (16, 16, 64, [100] * 30, 0)])
+def test_portions_of_all_kinds(H, G, D, counts, least):
+    """Steps whose requests go through chunks, columns and the form for short portions behind each other: as without chunks."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, g, n, B = "cuda", torch.Generator(device="cuda").manual_seed(H), sum(counts), len(counts)
+    assert LO.delta_chunks_from(counts, H, D) == least
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    qkv, proj, a_log, bias, w, start = rnd(n, 2 * G * D + H * D), rnd(n, 2 * H + H * D), rnd(H), rnd(H), 1 + 0.1 * rnd(D), rnd(B, H, D, D)
+    outs, states = [], []
+    for chunks in (least, 0):
+        batch, st = LO.RaggedBatch.build(counts, [b % 5 for b in range(B)], list(range(B)), [list(range(13 * b, 13 * b + 13)) for b in range(B)], 64, dev), start.clone()
+        batch._tiles[("delta", H, D)] = chunks
+        outs.append(LO.delta_rule(qkv, (0, G * D, 2 * G * D), proj, (0, H, 2 * H), a_log, bias, w, batch, H, G, D, D, 1e-6, D ** -0.5, 1e-5, st).double())
+        states.append(st.double())
+        assert any(k[0] == "long" for k in batch._tiles if isinstance(k, tuple)) == (chunks > 0)
+    # 32-bit sums in another order, a few roundings of 2 ** -24 each, normed
+    assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[1].norm() and (states[0] - states[1]).norm() <= 4e-6 * states[1].norm()
