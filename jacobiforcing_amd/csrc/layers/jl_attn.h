@@ -18,6 +18,9 @@ template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { re
 
 constexpr int AR_ROWS = 128;          // (query, head) rows of a tile of the wide form
 
+// tiles and groups (``hb`` per key head) lie along one axis of the grid: up to 2 ** 32 threads of workgroups of 256
+static inline bool jl_attn_grid_fits(const jl_attn_args &a, int hb) { return (int64_t)a.n_tiles * a.G * hb < (1 << 24); }
+
 // the wide form's launch (jl_attn_rows.hip); sizes as jl_attn_sweep has checked them, ``hf`` heads of a.TQ queries per tile, ``hb`` tiles per group
 int jl_attn_rows_launch(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st);
 

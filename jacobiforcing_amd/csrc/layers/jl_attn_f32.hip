@@ -26,11 +26,12 @@ __global__ __launch_bounds__(64 * NW) void attn_f32_kernel(jl_attn_args a, int H
     constexpr int THREADS = 64 * NW, VU = 8 * NDV, BUF = AF_KT * (KU + VU), KPF = AF_KT * KU / THREADS, VPF = AF_KT * VU / THREADS;
     const int H = a.H, D = a.D, Dv = a.Dv, per_group = H / a.G;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
-    const int *tile = a.tiles + 4 * (int64_t)blockIdx.y;
+    const int groups = a.G * HB, group = blockIdx.x % groups, tile_i = blockIdx.x / groups;
+    const int *tile = a.tiles + 4 * (int64_t)tile_i;
     const int b = tile[0], i0 = tile[1], cnt = tile[2], row0 = tile[3];
     if (b < 0 || cnt <= 0) return;
-    const int c = blockIdx.x / HB;
-    const int h0 = c * per_group + (blockIdx.x - c * HB) * HF, h_end = (c + 1) * per_group;
+    const int c = group / HB;
+    const int h0 = c * per_group + (group - c * HB) * HF, h_end = (c + 1) * per_group;
     uint4 *buf0 = (uint4 *)smem;
     int *tokS = (int *)(buf0 + (NW > 1 ? 2 : 1) * BUF);             // [2][32] pool tokens of a tile's keys
     const int window = a.window > 0 ? a.window : 0x3fffffff, chunk = a.chunk, i_max = i0 + cnt - 1;
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(64 * NW) void attn_f32_kernel(jl_attn_args a, int H
     }
     l_run += __shfl_xor(l_run, 32, 64);
     if (S > 1) {                                                    // this share's rows: [Dv] unnormalised outputs, maximum, sum
-        float *part = a.scratch + ((((int64_t)split * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 32 + l32) * (int64_t)(Dv + 2);
+        float *part = a.scratch + ((((int64_t)split * a.n_tiles + tile_i) * groups + group) * 32 + l32) * (int64_t)(Dv + 2);
         if (hi == 0) { part[Dv] = m_run; part[Dv + 1] = l_run; }
 #pragma unroll
         for (int t = 0; t < NDV; ++t) {
@@ -252,12 +253,12 @@ template <int KU, int NDV, int NW, int SRC> static int af_launch(const jl_attn_a
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_sweep: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     }
-    kern<<<dim3((unsigned)(a.G * hb), (unsigned)a.n_tiles, (unsigned)(a.splits > 1 ? a.splits : 1)), 64 * NW, lds, st>>>(a, hf, a.TQ, hb);
+    kern<<<dim3((unsigned)(a.n_tiles * a.G * hb), 1, (unsigned)(a.splits > 1 ? a.splits : 1)), 64 * NW, lds, st>>>(a, hf, a.TQ, hb);
     return jl_check_launch("attn_f32_kernel");
 }
 
 int jl_attn_f32_launch(const jl_attn_args &a, int hf, int hb, int src, bool wide, hipStream_t st) {
-    if (a.n_tiles > 65535) return jl_fail(JL_E_INVALID, "jl_attn_sweep: at most 65535 tiles");
+    if (!jl_attn_grid_fits(a, hb)) return jl_fail(JL_E_INVALID, "jl_attn_sweep: too many tiles");
     if (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.v_cache | (uintptr_t)a.k_tail) & 15) return jl_fail(JL_E_INVALID, "jl_attn_sweep: float rows start at 16-byte borders");
     const int ku = a.D <= 64 ? 16 : a.D <= 128 ? 32 : a.D <= 192 ? 48 : 64, ndv = a.Dv <= 64 ? 2 : 4;
 #define AF_CASE(K, V)                                                                               \

@@ -35,11 +35,12 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     const int H = a.H, D = a.D, Dv = a.Dv, per_group = H / a.G;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
     // groups side by side: neighbouring workgroups go to different XCDs, so each keeps few groups' keys in its L2
-    const int *tile = a.tiles + 4 * (int64_t)blockIdx.y;
+    const int groups = a.G * HB, group = blockIdx.x % groups;
+    const int *tile = a.tiles + 4 * (int64_t)(blockIdx.x / groups);
     const int b = tile[0], i0 = tile[1], cnt = tile[2], row0 = tile[3];
     if (b < 0 || cnt <= 0) return;
-    const int c = blockIdx.x / HB;
-    const int h0 = c * per_group + (blockIdx.x - c * HB) * HF, h_end = (c + 1) * per_group;
+    const int c = group / HB;
+    const int h0 = c * per_group + (group - c * HB) * HF, h_end = (c + 1) * per_group;
     constexpr int BUF = KT * KU + VROWS;                            // one buffer in 16-byte units: the keys, then the values (or none: the keys' own rows)
     uint4 *buf0 = (uint4 *)smem;
     int *tokS = (int *)(buf0 + 2 * (KT * KU + KT * VU));            // [2][KT] pool tokens of a tile's keys
@@ -289,7 +290,7 @@ template <int KU, int VU, int SRC> static int ar_launch(const jl_attn_args &a, i
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_sweep: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     }
-    kern<<<dim3((unsigned)(a.G * hb), (unsigned)a.n_tiles), AR_THREADS, lds, st>>>(a, hf, a.TQ, hb);
+    kern<<<dim3((unsigned)(a.n_tiles * a.G * hb)), AR_THREADS, lds, st>>>(a, hf, a.TQ, hb);
     return jl_check_launch("attn_rows_kernel");
 }
 template <int KU, int VU> static int ar_launch_v(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st) {
@@ -299,7 +300,7 @@ template <int KU, int VU> static int ar_launch_v(const jl_attn_args &a, int hf, 
 int jl_attn_rows_launch(const jl_attn_args &args, int hf, int hb, bool v_in_k, hipStream_t st) {
     jl_attn_args a = args;
     a.q_ld = (int64_t)a.H * a.D;
-    if (a.n_tiles > 65535) return jl_fail(JL_E_INVALID, "jl_attn_sweep: at most 65535 tiles");
+    if (!jl_attn_grid_fits(a, hb)) return jl_fail(JL_E_INVALID, "jl_attn_sweep: too many tiles");
     const int ku = 8 * ((a.D + 63) / 64), vu = a.Dv <= 64 ? 8 : 16;      // 16-byte units of a row in LDS
 #define AR_CASE(K, V) if (ku == K && vu == V) return ar_launch_v<K, V>(a, hf, hb, v_in_k, st)
     AR_CASE(8, 8); AR_CASE(8, 16);
@@ -319,7 +320,7 @@ extern "C" int jl_attn_expanded(const jl_attn_args *ap, void *stream) {
     if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.tiles || !a.key_base || (a.k_tail_cols > 0 && !a.k_tail)) return jl_fail(JL_E_INVALID, "jl_attn_expanded: null pointer");
     const int64_t own = a.D - a.k_tail_cols;
     if ((a.dtype != JL_BF16 && a.dtype != JL_F32) || a.H <= 0 || a.G != a.H || (a.Gv > 0 && a.Gv != a.H) || a.D <= 0 || a.D % 8 || a.D > 256 || a.k_tail_cols < 0 || a.k_tail_cols % 8 || own < 0 ||
-        a.Dv < 32 || a.Dv % 32 || a.Dv > 128 || a.TQ != AR_ROWS || a.n_tiles > 65535)
+        a.Dv < 32 || a.Dv % 32 || a.Dv > 128 || a.TQ != AR_ROWS || !jl_attn_grid_fits(a, 1))
         return jl_fail(JL_E_INVALID, "jl_attn_expanded: a key and a value head per query head, key widths in multiples of 8 up to 256, value widths in multiples of 32 up to 128");
     if (a.k_ld < a.H * own || a.v_ld < (int64_t)a.H * a.Dv || a.q_ld < (int64_t)a.H * a.D || a.out_ld < (int64_t)a.H * a.Dv || (a.k_tail_cols > 0 && a.k_tail_ld < a.k_tail_cols) ||
         a.k_ld % 4 || a.v_ld % 4 || a.q_ld % 4 || a.out_ld % 4 || a.k_tail_ld % 4)

@@ -148,3 +148,27 @@ def test_latent_attention_with_built_keys(monkeypatch, dtype, H, D, R, rd, Dv, r
     # queries, keys, values, weights and the result are rounded to bfloat16 once each (2 ** -9 relative); a score of size 3 moves its weight by 1.2 %
     err, tol = (got.double() - want).abs(), 2.0 ** -6 if dtype == "bfloat16" else 2.0 ** -19
     assert torch.isfinite(got).all() and err.norm() < tol * want.norm() and err.max() < 4 * tol * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype,single", [("bfloat16", False), ("float32", False), ("float32", True)])
+def test_more_tiles_than_a_short_grid_axis_holds(dtype, single):
+    """One portion in more than 65 535 tiles of 128 rows (``single``: as many decoding requests, tiles of 32 rows), as in two steps."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt, page, H, D, Dv, window = "cuda", getattr(torch, dtype), 64, 32, 8, 32, 5
+    n = 65600 if single else 262400
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dt)
+    q, half = rnd(n, H * D), n // 2
+    pages = list(range(n // page))
+    k, v = rnd(n, D), rnd(n, Dv)
+
+    def run(lo, hi):
+        if single:                                                   # request b attends to the keys of page b % pages
+            batch = LO.RaggedBatch.build([1] * (hi - lo), [b % page for b in range(lo, hi)], [0] * (hi - lo), [[b % len(pages)] for b in range(lo, hi)], page, dev)
+        else:
+            batch = LO.RaggedBatch.build([hi - lo], [lo], [0], [pages], page, dev)
+        out = LO.attn_sweep(q[lo:hi].contiguous(), k, v, batch, H, 1, D, Dv, D ** -0.5, window)
+        assert any(t.shape[0] > 65535 for key, t in batch._tiles.items() if torch.is_tensor(t)) == (hi - lo == n)
+        return out
+
+    assert torch.equal(run(0, n), torch.cat([run(0, half), run(half, n)]))
