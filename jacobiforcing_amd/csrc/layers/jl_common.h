@@ -105,6 +105,10 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 __device__ __forceinline__ void jl_load_lds(const char *base, uint32_t off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
+// the same from an address per lane
+__device__ __forceinline__ void jl_load_lds_far(const char *from, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "memory");
+}
 
 #define JL_DISPATCH(dtype, ...)                                   \
     do {                                                          \

@@ -288,7 +288,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
 // CU and cover each other's barriers (through registers, two of them: gated product at 8192 x 4 of 32 experts of 2048 x 1024 406 -> 363 us, the way down 290 -> 252).
 // Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading
 // the weights: single wavefronts, many per CU, 12 KB on the way each, in registers.
-// Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from one base, rows that do not exist repeat another, stages behind the last repeat the
+// Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from a base (of the tile where its rows lie together; FAR: rows gathered from more than
+// 4 GiB have 64-bit addresses), rows that do not exist repeat another, stages behind the last repeat the
 // first, depths beyond the last whole stage come after the loop (a condition per load had cost six vector instructions per product: 431 us instead of 406 for the gated product
 // above; us for up and down at 32 rows x 4 of 16 of 1024 x 512: 49 -> 41, float 16 rows 100 -> 79, 400 rows 53 -> 45).
 struct MoeMM {
@@ -319,7 +320,7 @@ template <> struct mm_type<float> {
     }
 };
 
-template <typename T, int TM, int NW, int WR, int TKU, bool GATED>
+template <typename T, int TM, int NW, int WR, int TKU, bool GATED, bool FAR>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM a) {
     constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
     constexpr int XPF = TM * TKU / THREADS, WPF = WR * TKU / THREADS, TN = GATED ? WR / 2 : WR, STAGE = TKU * UNIT;
@@ -348,26 +349,35 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
     auto unit_of = [&](int x) { return DMA ? at(lr + x * (THREADS / TKU), tid % TKU) % TKU : tid % TKU; };      // DMA: what belongs into this thread's place of LDS
     // byte offsets from a base that is the same for all lanes: a load is one instruction (the launch has checked that 32 bits hold them)
     uint32_t xo[XPF], wo[WPF];
+    const char *xfar[FAR ? XPF : 1];
+    const char *Xb = (const char *)((const T *)a.X + (a.mode != 1 ? 0 : (int64_t)r0 * K));
 #pragma unroll
     for (int x = 0; x < XPF; ++x) {
-        const int m = lr + x * (THREADS / TKU), row = r0 + (m < nr ? m : 0);
-        xo[x] = (uint32_t)((a.mode != 1 ? a.perm[row] / a.top : row) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
+        const int m = lr + x * (THREADS / TKU), row = m < nr ? m : 0;
+        const int64_t at_x = (a.mode != 1 ? a.perm[r0 + row] / a.top : row) * (int64_t)K + unit_of(x) * UNIT;
+        if constexpr (FAR) xfar[x] = Xb + at_x * sizeof(T);
+        xo[x] = (uint32_t)at_x * sizeof(T);
     }
-    const char *Xb = (const char *)a.X, *Wb = (const char *)((const T *)a.Wt + (int64_t)e * (GATED ? 2 : 1) * n_out * K);
+    // the first half of a gated tile's rows are the gate's, the others the linear branch's, n_out further on
+    const char *Wb = (const char *)((const T *)a.Wt + ((int64_t)e * (GATED ? 2 : 1) * n_out + n0) * K), *Wl = Wb + (int64_t)(GATED ? n_out : 0) * K * sizeof(T);
 #pragma unroll
     for (int x = 0; x < WPF; ++x) {
-        const int j = lr + x * (THREADS / TKU), c = n0 + (GATED ? j % TN : j);
-        wo[x] = (uint32_t)(((GATED && j >= TN ? n_out : 0) + (c < n_out ? c : n_out - 1)) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
+        const int j = lr + x * (THREADS / TKU), c = GATED ? j % TN : j;
+        wo[x] = (uint32_t)((n0 + c < n_out ? c : n_out - 1 - n0) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
     }
+    auto w_base = [&](int x) { return GATED && x >= WPF / 2 ? Wl : Wb; };
     mm_u32x4 reg[DMA ? 1 : 2][XPF + WPF];                                     // stages on their way: even ones in reg[0], odd ones in reg[1]
     const int full = K / STAGE;                                     // whole stages; what is left of K comes last
     auto fetch = [&](mm_u32x4 (&r)[XPF + WPF], int i) {             // without branches: behind the last stage, stage 0 again (never used)
         const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
-        const char *xb = Xb + k, *wb = Wb + k;
+        const char *xb = Xb + k;
 #pragma unroll
-        for (int x = 0; x < XPF; ++x) r[x] = *(const mm_u32x4 *)(xb + xo[x]);
+        for (int x = 0; x < XPF; ++x) {
+            if constexpr (FAR) r[x] = *(const mm_u32x4 *)(xfar[x] + k);
+            else r[x] = *(const mm_u32x4 *)(xb + xo[x]);
+        }
 #pragma unroll
-        for (int x = 0; x < WPF; ++x) r[XPF + x] = *(const mm_u32x4 *)(wb + wo[x]);
+        for (int x = 0; x < WPF; ++x) r[XPF + x] = *(const mm_u32x4 *)(w_base(x) + k + wo[x]);
     };
     auto stash = [&](const mm_u32x4 (&r)[XPF + WPF], int sel) {
         uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
@@ -412,9 +422,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
             const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
             const uint32_t dst = lds + sel * (TM + WR) * TKU * 16;
 #pragma unroll
-            for (int x = 0; x < XPF; ++x) jl_load_lds(Xb + k, xo[x], dst + x * THREADS * 16);
+            for (int x = 0; x < XPF; ++x) {
+                if constexpr (FAR) jl_load_lds_far(xfar[x] + k, dst + x * THREADS * 16);
+                else jl_load_lds(Xb + k, xo[x], dst + x * THREADS * 16);
+            }
 #pragma unroll
-            for (int x = 0; x < WPF; ++x) jl_load_lds(Wb + k, wo[x], dst + (XPF + x) * THREADS * 16);
+            for (int x = 0; x < WPF; ++x) jl_load_lds(w_base(x) + k, wo[x], dst + (XPF + x) * THREADS * 16);
         };
         auto arrived = [&]() {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -459,15 +472,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
     }
     if (full * STAGE < K) {                                         // depths beyond K are zero
         const mm_u32x4 zero = {0, 0, 0, 0};
-        auto last = [&](const char *base, uint32_t off, int u) {    // a lane beyond K reads its row's first unit: a row may be shorter than a stage
+        auto last = [&](const char *from, int u) {                  // a lane beyond K reads its row's first unit: a row may be shorter than a stage
             const bool in = full * STAGE + u * UNIT < K;
-            const mm_u32x4 v = *(const mm_u32x4 *)(base + off + (in ? (int64_t)full * STAGE * sizeof(T) : -(int64_t)(u * UNIT * sizeof(T))));
+            const mm_u32x4 v = *(const mm_u32x4 *)(from + (in ? (int64_t)full * STAGE * sizeof(T) : -(int64_t)(u * UNIT * sizeof(T))));
             return in ? v : zero;
         };
 #pragma unroll
-        for (int x = 0; x < XPF; ++x) reg[0][x] = last(Xb, xo[x], unit_of(x));
+        for (int x = 0; x < XPF; ++x) reg[0][x] = last(FAR ? xfar[FAR ? x : 0] : Xb + xo[x], unit_of(x));
 #pragma unroll
-        for (int x = 0; x < WPF; ++x) reg[0][XPF + x] = last(Wb, wo[x], unit_of(x));
+        for (int x = 0; x < WPF; ++x) reg[0][XPF + x] = last(w_base(x) + wo[x], unit_of(x));
         stash(reg[0], 0);
         __syncthreads();
         products(even);
@@ -513,8 +526,10 @@ template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(
     a.col_blocks = (a.n_out + tn - 1) / tn;
     const int64_t groups = (int64_t)(TM >= 64 ? (a.max_tiles + 7) / 8 * 8 : a.max_tiles) * a.col_blocks;
     if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
-    if (gated) moe_mm_kernel<T, TM, NW, WR, TKU, true><<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
-    else moe_mm_kernel<T, TM, NW, WR, TKU, false><<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
+    const bool far = a.mode != 1 && ((int64_t)a.max_tiles * TM / a.top + 1) * a.K * (int64_t)sizeof(T) > UINT32_MAX;      // gathered rows beyond what 32 bits reach
+    auto kern = gated ? (far ? moe_mm_kernel<T, TM, NW, WR, TKU, true, true> : moe_mm_kernel<T, TM, NW, WR, TKU, true, false>)
+                      : (far ? moe_mm_kernel<T, TM, NW, WR, TKU, false, true> : moe_mm_kernel<T, TM, NW, WR, TKU, false, false>);
+    kern<<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
     return jl_check_launch("moe_mm_kernel");
 }
 template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated, hipStream_t st) {
@@ -531,8 +546,7 @@ static int moe_gemm_launch(const void *X, const void *Wt, int dtype, int32_t mod
     const int64_t dtype_bytes = dtype == JL_BF16 ? 2 : 4;
     MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}};
     if (!no_mfma && moe_mm_sizes(dtype, K) && ((uintptr_t)X % 16) == 0 && ((uintptr_t)Wt % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
-        ((int64_t)max_tiles * tile_rows / top + 1) * K * dtype_bytes <= UINT32_MAX && ((int64_t)max_tiles * tile_rows + 1) * (mode == 1 ? K : 0) * dtype_bytes <= UINT32_MAX &&
-        (int64_t)(act ? 2 : 1) * n_out * K * dtype_bytes <= UINT32_MAX) {
+        256 * (int64_t)K * dtype_bytes <= UINT32_MAX) {                     // a tile's rows, of X or of W
         if (dtype == JL_BF16) return moe_mm_rows<bf16_t>(a, tile_rows, act != nullptr, (hipStream_t)stream);
         return moe_mm_rows<float>(a, tile_rows, act != nullptr, (hipStream_t)stream);
     }

@@ -37,3 +37,55 @@ def test_experts(dtype, N, E, top, W, ff, gated, identity, skew):
     # float: sums of K products rounded one by one, 2 ** -24 each, in two products; bfloat16: the units may round the other way (2 ** -8 of each, averaged by the sum)
     tol = (W + ff) ** 0.5 * 2.0 ** -22 if dtype == "float32" else 2.0 ** -8
     assert err.norm() <= tol * want.norm() and err.abs().max() <= 16 * tol * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype,K,gated", [("bfloat16", 1032, True), ("bfloat16", 2048, False), ("float32", 516, True), ("float32", 1028, False)])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+@pytest.mark.parametrize("far", ["rows gathered from", "rows in order", "weights"])
+def test_operands_beyond_4_gib(dtype, K, gated, tile, far):
+    """The tiles of the matrix instructions reach them, in the same order of sums: bit for bit what the same rows give as a small product."""
+    from jacobiforcing_amd import _native as N
+    from jacobiforcing_amd import layer_ops as LO
+    if dtype == "float32" and tile == 128:
+        pytest.skip("float tiles have up to 64 rows")
+    dev, dt, lib, E, n_out = "cuda", getattr(torch, dtype), N.layers(), 2, 24
+    size, code, st = dt.itemsize, LO._code(dt), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(K)
+    rows, beyond = 300, (1 << 32) // (K * size) + 5                  # rows of 32 bits' reach and five more
+    mode = 1 if far == "rows in order" else N.JL_MOE_UP_PLAIN
+    if far == "weights":
+        if gated:
+            pytest.skip("one product's columns reach as far")
+        X, W, cols = torch.randn(rows, K, generator=g, device=dev).to(dt), torch.zeros(E, beyond + n_out, K, dtype=dt, device=dev), beyond + n_out
+        W[:, -n_out:] = torch.randn(E, n_out, K, generator=g, device=dev).to(dt)
+    else:
+        X, W, cols = torch.zeros(beyond + rows, K, dtype=dt, device=dev), torch.randn(E, (2 if gated and mode != 1 else 1) * n_out, K, generator=g, device=dev).to(dt), n_out
+        X[-rows:] = torch.randn(rows, K, generator=g, device=dev).to(dt)
+
+    def run(x, w, n_cols, first_row):
+        """Expert 0 has 170 of the 300 rows, expert 1 the others; gathered backwards, or in order from ``first_row`` on."""
+        total = x.shape[0]
+        perm = torch.arange(total - 1, total - 1 - rows, -1, dtype=torch.int32, device=dev) if mode != 1 else torch.arange(first_row + rows, dtype=torch.int32, device=dev)
+        start = 0 if mode != 1 else first_row
+        t_e, t_r = [], []
+        for e, (lo, hi) in enumerate(((start, start + 170), (start + 170, start + 300))):
+            t_e += [e] * len(range(lo, hi, tile))
+            t_r += list(range(lo, hi, tile))
+        offs = torch.tensor([start, start + 170, start + rows, len(t_e)], dtype=torch.int32, device=dev)
+        count = total // tile + E if mode != 1 else len(t_e)          # as many tiles as a step of all rows would have: the launch goes by it
+        te, tr = torch.full((count,), -1, dtype=torch.int32, device=dev), torch.zeros(count, dtype=torch.int32, device=dev)
+        te[:len(t_e)], tr[:len(t_e)] = torch.tensor(t_e, device=dev), torch.tensor(t_r, device=dev)
+        out = torch.empty(start + rows, n_cols, dtype=torch.float32 if mode == 1 else dt, device=dev)
+        wts = torch.ones(start + rows, device=dev)
+        if gated and mode != 1:
+            rc = lib.jl_moe_gemm_gated(x.data_ptr(), w.data_ptr(), code, K, n_cols, 1, perm.data_ptr(), offs.data_ptr(), te.data_ptr(), tr.data_ptr(), count, E, tile, N.JL_ACT_SILU, 0.0, 1.0,
+                                       0.0, out.data_ptr(), st)
+        else:
+            rc = lib.jl_moe_gemm(x.data_ptr(), w.data_ptr(), code, mode, K, n_cols, 1, perm.data_ptr(), offs.data_ptr(), te.data_ptr(), tr.data_ptr(), count, E, tile,
+                                 wts.data_ptr() if mode == 1 else None, out.data_ptr(), st)
+        assert rc == 0
+        return out[start:, -n_out:].clone()
+
+    got = run(X, W, cols, X.shape[0] - rows)
+    want = run(X[-rows:].contiguous(), W[:, -n_out:].contiguous() if far == "weights" else W, n_out, 0)
+    assert torch.equal(got, want) and bool(want.any())
