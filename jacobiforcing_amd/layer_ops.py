@@ -995,7 +995,7 @@ def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, 
             s = batch.starts[b]
             full = min(c, max(0, s + c - w))              # queries that see a whole window; the others see s + 1, s + 2, .. keys
             n, pairs = s + c - max(0, s - w + 1), full * w + (c - full) * (s + 0.5 * (1 + c - full))
-            if (keys + n) * 2 * H * (D + Dv) <= LATENT_BUILT_BYTES:
+            if (keys + n) * dtype.itemsize * H * (D + Dv) <= LATENT_BUILT_BYTES:
                 chosen.append(b)
                 won += pairs * over - n * one
                 attend, chain, keys = attend + pairs * pair, max(chain, step * min(n, w + 127)), keys + n

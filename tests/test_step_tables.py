@@ -1,0 +1,24 @@
+"""What a step's tables and rules on the host hold (no kernel runs)."""
+import pytest
+import torch
+
+from jacobiforcing_amd import layer_ops as LO
+
+
+def batch(counts, starts, page=64):
+    need = [-(-(c + s) // page) for c, s in zip(counts, starts)]
+    at = [sum(need[:b]) for b in range(len(need))]
+    return LO.RaggedBatch.build(counts, starts, list(range(len(counts))), [list(range(a, a + n)) for a, n in zip(at, need)], page, "cpu")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_keys_built_per_head_stay_within_their_bytes(monkeypatch, dtype):
+    """The bytes of keys and values that a step builds, in the activations' type."""
+    H, D, R, rd, Dv = 16, 128, 512, 64, 128
+    b = batch([4096] * 6, [0] * 6)
+    per = 4096 * H * (D + Dv) * dtype.itemsize
+    for room in (6, 3, 1):
+        monkeypatch.setattr(LO, "LATENT_BUILT_BYTES", room * per)
+        b._tiles.clear()
+        chosen = LO._latent_built_requests(b, H, D, R, rd, Dv, 0, dtype)
+        assert len(chosen) == room and sum(b.counts[i] for i in chosen) * H * (D + Dv) * dtype.itemsize <= LO.LATENT_BUILT_BYTES
