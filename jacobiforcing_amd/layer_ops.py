@@ -202,7 +202,7 @@ class RaggedBatch:
     def tiles(self, tq: int, longest_first: bool = False, requests: Optional[Sequence[int]] = None) -> torch.Tensor:
         """[n_tiles, 4] int32 {b, first query position, count, first row}: each request's rows cut into runs of at most ``tq``; with
         ``longest_first`` those with the most positions in front of them come first; only those of ``requests`` when given."""
-        key = ("longest first", tq, None if requests is None else tuple(requests)) if longest_first or requests is not None else tq
+        key = ("longest first" if longest_first else "in order", tq, None if requests is None else tuple(requests)) if longest_first or requests is not None else tq
         t = self._tiles.get(key)
         if t is None:
             rows, r0 = [], 0

@@ -22,3 +22,12 @@ def test_keys_built_per_head_stay_within_their_bytes(monkeypatch, dtype):
         b._tiles.clear()
         chosen = LO._latent_built_requests(b, H, D, R, rd, Dv, 0, dtype)
         assert len(chosen) == room and sum(b.counts[i] for i in chosen) * H * (D + Dv) * dtype.itemsize <= LO.LATENT_BUILT_BYTES
+
+
+def test_tiles_of_some_requests_keep_the_order_they_were_asked_for():
+    b = batch([5, 3, 9], [0, 7, 2])
+    for first in (False, True):
+        b._tiles.clear()
+        asked = [b.tiles(4, longest_first=x, requests=[1, 2]).tolist() for x in (first, not first)]
+        in_order = asked[0] if not first else asked[1]
+        assert in_order == [[1, 7, 3, 5], [2, 2, 4, 8], [2, 6, 4, 12], [2, 10, 1, 16]] and sorted(in_order, key=lambda r: -r[1]) == asked[1 if not first else 0]
