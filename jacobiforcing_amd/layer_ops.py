@@ -83,7 +83,7 @@ class RaggedBatch:
     max_slot: int
     slots: List[int]
     _tiles: dict
-    _host_tables: Optional[np.ndarray] = None         # block_tables on the host (what key_rows reads)
+    _host_tables: Optional[np.ndarray] = None         # tables on the host, for key_rows and part (None: read back when they need it)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
@@ -172,6 +172,11 @@ class RaggedBatch:
             self._tiles[key] = (every[:len(rec)], every[len(rec):len(rec) + len(req)], every[len(rec) + len(req):], max((r[1] for r in rest), default=0))
         return self._tiles[key]
 
+    def _pages(self) -> np.ndarray:
+        if self._host_tables is None:
+            self._host_tables = self.tables.cpu().numpy()
+        return self._host_tables
+
     def key_rows(self, requests: Sequence[int], window: int):
         """The pool tokens that ``requests`` read under ``window`` (0: all before them), request by request in order of position: (tokens [K] int64,
         base [B] int32 with the place of request b's position j at base[b] + j)."""
@@ -181,7 +186,7 @@ class RaggedBatch:
             for b in requests:
                 end = self.starts[b] + self.counts[b]
                 pos = np.arange(max(0, self.starts[b] - window + 1) if window > 0 else 0, end, dtype=np.int64)
-                tok.append(self._host_tables[b][pos // self.page_size].astype(np.int64) * self.page_size + pos % self.page_size)
+                tok.append(self._pages()[b][pos // self.page_size].astype(np.int64) * self.page_size + pos % self.page_size)
                 base[b] = at - int(pos[0])
                 at += pos.size
             dev = self.seq.device
@@ -195,7 +200,7 @@ class RaggedBatch:
             row0 = np.concatenate([[0], np.cumsum(self.counts)])
             rows = np.concatenate([np.arange(row0[b], row0[b + 1], dtype=np.int64) for b in requests])
             sub = RaggedBatch.build([self.counts[b] for b in requests], [self.starts[b] for b in requests], [self.slots[b] for b in requests],
-                                    [self._host_tables[b] for b in requests], self.page_size, self.seq.device)
+                                    [self._pages()[b] for b in requests], self.page_size, self.seq.device)
             self._tiles[key] = (sub, torch.from_numpy(rows).to(self.seq.device))
         return self._tiles[key]
 

@@ -31,3 +31,14 @@ def test_tiles_of_some_requests_keep_the_order_they_were_asked_for():
         asked = [b.tiles(4, longest_first=x, requests=[1, 2]).tolist() for x in (first, not first)]
         in_order = asked[0] if not first else asked[1]
         assert in_order == [[1, 7, 3, 5], [2, 2, 4, 8], [2, 6, 4, 12], [2, 10, 1, 16]] and sorted(in_order, key=lambda r: -r[1]) == asked[1 if not first else 0]
+
+
+def test_a_batch_without_its_tables_on_the_host():
+    """One that was put together from its tensors: key rows and parts read them back."""
+    import dataclasses
+    b = batch([70, 3, 9], [0, 130, 2])
+    bare = dataclasses.replace(b, _tiles={}, _host_tables=None)
+    for window in (0, 50):
+        assert all(torch.equal(x, y) for x, y in zip(b.key_rows([0, 1], window), bare.key_rows([0, 1], window)))
+    (s1, r1), (s2, r2) = b.part([1, 2]), bare.part([1, 2])
+    assert torch.equal(r1, r2) and torch.equal(s1.kv_slot, s2.kv_slot) and torch.equal(s1.tables, s2.tables)
