@@ -224,6 +224,7 @@ class RaggedBatch:
 LINEAR_SMALL_ROWS, LINEAR_ONE_TILE = 64, 4096       # jl_linear_small: rows at most; W's rows up to which a workgroup takes 16 of them
 LINEAR_X_BYTES = 128 << 10           # ... and the bytes of x that a CU reads up to which it is the faster one
 _LINEAR_SAME, _LINEAR_FLOAT, _LINEAR_ROUNDED_FLOAT = 0, 1, 2
+_LINEAR_TYPES = (torch.bfloat16, torch.float32)
 
 
 def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
@@ -246,14 +247,16 @@ def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:
     """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``) and a few hundred (``linear_mid``), the library's product
     for more.  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
-    counts as float: give ``float_out`` True."""
+    counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
     n, k = x.shape
     o, size = w.shape[0], w.element_size()
     _need(w.dtype == x.dtype or (w.dtype == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
     small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, size)
     if ((small or (w.dtype == x.dtype and linear_mid(n, k, o, x.dtype))) and w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and
-            x.stride(0) * x.element_size() % 16 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous()))):
+            x.stride(0) * x.element_size() % 16 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous())) and
+            x.dtype in _LINEAR_TYPES and k > 0 and w.get_device() == x.get_device() and (bias is None or bias.get_device() == x.get_device()) and
+            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))):
         out = torch.empty((n, o), dtype=x.dtype if float_out is None else torch.float32, device=x.device)
         mode = _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT
         if small:

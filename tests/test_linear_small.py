@@ -61,3 +61,23 @@ def test_a_few_hundred_rows(N, K, O, bias):
         assert bool(((got.double() - want).abs() <= tol).all())
         if float_out is False:
             assert torch.equal(got, got.to(dt).float())
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32", "float16"])
+@pytest.mark.parametrize("n", [3, 100])
+def test_operands_on_other_devices_and_gradients(dtype, n):
+    """Weights or a bias in host memory are refused, types the launches do not know and gradients come from the library, a product over nothing is zero."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, dt = "cuda", getattr(torch, dtype)
+    x, w, b = torch.randn(n, 64, device=dev).to(dt), torch.randn(32, 64, device=dev).to(dt), torch.randn(32, device=dev).to(dt)
+    for args in ((x, w.cpu()), (x, w, b.cpu()), (x, w.cpu(), b)):
+        for float_out in (None, True):
+            with pytest.raises(RuntimeError):
+                LO.linear(*args, float_out=float_out)
+    want = x.double() @ w.double().T + b.double()
+    assert torch.allclose(LO.linear(x, w, b).double(), want, atol=0.2)
+    for i in range(3):
+        leaf = [t.clone().requires_grad_(j == i) for j, t in enumerate((x, w, b))]
+        LO.linear(*leaf).sum().backward()
+        assert leaf[i].grad is not None and bool(leaf[i].grad.any())
+    assert torch.equal(LO.linear(x[:, :0].contiguous(), w[:, :0].contiguous()), torch.zeros(n, 32, dtype=dt, device=dev))
