@@ -443,7 +443,8 @@ def block_slots(positions: torch.Tensor, T: int, row_prompt: torch.Tensor, row_c
     """Cache slots of a draft block's tokens (int64 [R*T], -1: none) and, with ``candidates``, their slots in the candidate scratch (else None); inputs int32."""
     _dev(positions)
     for t in (positions, row_prompt, row_cand, row_len):
-        _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() * (1 if t is positions else T) == positions.numel(), "block_slots: contiguous int32 [R*T] positions, [R] rows")
+        _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() * (1 if t is positions else T) == positions.numel() and t.get_device() == positions.get_device(),
+              "block_slots: contiguous int32 [R*T] positions, [R] rows on one device")
     out = torch.empty((2 if candidates else 1, positions.numel()), dtype=torch.int64, device=positions.device)
     N.check_layers(N.layers().jl_block_slots(positions.data_ptr(), row_prompt.data_ptr(), row_cand.data_ptr(), row_len.data_ptr(), row_len.numel(), T, S_max, T_max, out[0].data_ptr(),
                                              out[1].data_ptr() if candidates else None, _stream(positions.device)), "jl_block_slots")
@@ -460,10 +461,11 @@ def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len
     R, nkv, GT, D = q.shape
     G = GT // T
     for t in (q, k, v) + ((ck, cv) if ck is not None else ()):
-        _need(t.is_contiguous() and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[1] == nkv and t.shape[3] == D, "attn_block: contiguous bfloat16 [., nkv, ., D]")
+        _need(t.is_contiguous() and t.dtype == torch.bfloat16 and t.dim() == 4 and t.shape[1] == nkv and t.shape[3] == D and t.get_device() == q.get_device(),
+              "attn_block: contiguous bfloat16 [., nkv, ., D] on one device")
     for t in (kv_len, row_len) + ((row_prompt,) if tables is None else ()) + ((row_cand,) if ck is not None else ()):
-        _need(t is not None and t.dtype == torch.int32 and t.numel() == R and t.is_contiguous(), "attn_block: int32 [R] lengths and rows")
-    _need(GT == G * T and k.shape == v.shape and (tables is None or (tables.dtype == torch.int32 and tables.dim() == 2 and tables.shape[0] == R and tables.stride(1) == 1)) and
+        _need(t is not None and t.dtype == torch.int32 and t.numel() == R and t.is_contiguous() and t.get_device() == q.get_device(), "attn_block: int32 [R] lengths and rows on q's device")
+    _need(GT == G * T and k.shape == v.shape and (tables is None or (tables.dtype == torch.int32 and tables.dim() == 2 and tables.shape[0] == R and tables.stride(1) == 1 and tables.get_device() == q.get_device())) and
           (ck is None or (ck.shape == cv.shape and ck.shape[2] >= T)), "attn_block: shapes")
     out = torch.empty((R * T, nkv * G * D), dtype=q.dtype, device=q.device)
     max_keys = min(int(max_keys), k.shape[2] * (1 if tables is None else tables.shape[1]))

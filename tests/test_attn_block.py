@@ -66,3 +66,22 @@ def test_slots(R, T, candidates):
     neg = torch.full((), -1, dtype=torch.int64, device=dev)
     assert torch.equal(main.view(R, T), torch.where(valid & (cand < 0).view(R, 1), prompt.long().view(R, 1) * 70000 + pos.view(R, T), neg))
     assert scratch is None if not candidates else torch.equal(scratch.view(R, T), torch.where(valid & (cand >= 0).view(R, 1), cand.long().view(R, 1) * (T + 3) + t, neg))
+
+
+def test_operands_in_host_memory_are_refused():
+    from jacobiforcing_amd import layer_ops as LO
+    dev, R, T, D = "cuda", 2, 4, 64
+    q, k, v, ck, cv = (torch.zeros(R, 2, n, D, dtype=torch.bfloat16, device=dev) for n in (3 * T, 32, 32, T, T))
+    lens, tables, pos = torch.full((R,), T, dtype=torch.int32, device=dev), torch.zeros(R, 1, dtype=torch.int32, device=dev), torch.zeros(R * T, dtype=torch.int32, device=dev)
+    good = dict(k=k, v=v, kv_len=lens, row_len=lens, row_prompt=lens * 0, row_cand=lens * 0, ck=ck, cv=cv)
+    for name in good:
+        with pytest.raises(ValueError):
+            LO.attn_block(q, T, max_keys=32, **{**good, name: good[name].cpu()})
+    with pytest.raises(ValueError):
+        LO.attn_block(q, T, k, v, lens, lens, 32, tables=tables.cpu())
+    rows = [pos, lens, lens, lens]
+    for i in range(1, 4):
+        args = [x.cpu() if j == i else x for j, x in enumerate(rows)]
+        with pytest.raises(ValueError):
+            LO.block_slots(args[0], T, *args[1:], 32, T, True)
+    assert LO.attn_block(q, T, max_keys=32, **good).shape == (R * T, 6 * D)
