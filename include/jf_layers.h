@@ -135,7 +135,7 @@ JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t
 
 /* jl_attn_window with `talk` (heads mixed after the softmax) in one sweep over the keys, for the sizes jl_attn_talk_ok takes; no sink, chunks or cap.  Tiles of
  * jl_attn_talk_tile_rows(H, G, wide) queries in any order (wide: 128 (query, head) rows per workgroup, else 32), a tile's keys shared out over `splits` workgroups;
- * scratch of jl_attn_talk_scratch_floats for pass_tiles tiles at a time.  q, pools and scratch at 16-byte borders, k_ld and v_ld in multiples of 8, out_ld of 4. */
+ * scratch of jl_attn_talk_scratch_floats for pass_tiles tiles at a time.  q, pools and scratch at 16-byte borders, k_ld and v_ld in multiples of 8, out_ld of 4; out at the borders of four values. */
 JL_API int jl_attn_talk(const jl_attn_args *a, int32_t wide, int32_t pass_tiles, void *stream);
 /* jl_attn_sweep for portions of a few tokens (decoding), the same arguments, in tiles of jl_attn_talk_tile_rows(H, G, 0) queries; scratch of
  * jl_attn_talk_scratch_floats(tiles, TQ, H, 1, Dv, splits); sizes as jl_attn_narrow_ok takes them, alignment as for jl_attn_talk. */

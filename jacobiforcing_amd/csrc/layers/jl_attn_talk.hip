@@ -385,6 +385,7 @@ extern "C" int jl_attn_talk(const jl_attn_args *ap, int32_t wide, int32_t pass_t
         (int64_t)(pass_tiles < a.n_tiles ? pass_tiles : a.n_tiles) * a.splits * a.G * a.G > INT32_MAX / 256)
         return jl_fail(JL_E_INVALID, "jl_attn_talk: tiles, splits or output rows");
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_talk: unknown out_dtype");
+    if ((uintptr_t)a.out & (a.out_dtype == JL_OUT_F32 ? 15 : 7)) return jl_fail(JL_E_INVALID, "jl_attn_talk: output rows start at the borders of four values");
     hipStream_t st = (hipStream_t)stream;
     const int ku = a.D <= 64 ? 8 : 16, vu = a.Dv <= 64 ? 8 : 16;
 #define AT_CASE(K, V) if (ku == K && vu == V) return wide ? at_launch<K, V, 4>(a, pass_tiles, st) : at_launch<K, V, 1>(a, pass_tiles, st)
@@ -463,6 +464,7 @@ extern "C" int jl_attn_narrow(const jl_attn_args *ap, void *stream) {
         (int64_t)a.n_tiles * a.splits * a.G > INT32_MAX / 64 || (int64_t)a.n_tiles * a.TQ * a.H > INT32_MAX)
         return jl_fail(JL_E_INVALID, "jl_attn_narrow: tiles, splits or output rows");
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_narrow: unknown out_dtype");
+    if ((uintptr_t)a.out & (a.out_dtype == JL_OUT_F32 ? 15 : 7)) return jl_fail(JL_E_INVALID, "jl_attn_narrow: output rows start at the borders of four values");
     hipStream_t st = (hipStream_t)stream;
     if (a.D <= 64) return a.Dv <= 64 ? an_launch<8, 8>(a, st) : an_launch<8, 16>(a, st);
     return a.Dv <= 64 ? an_launch<16, 8>(a, st) : an_launch<16, 16>(a, st);

@@ -353,6 +353,11 @@ def _attn_out(out: Optional[torch.Tensor], n: int, width: int, dtype: torch.dtyp
     return out
 
 
+def _fours(out: torch.Tensor) -> bool:
+    """Whether rows of ``out`` can be stored four values at a time."""
+    return out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0
+
+
 def attn_tile_rows(dtype: torch.dtype, H: int, G: int, D: int, Dv: int, k_ld: int = 0, v_ld: int = 0) -> int:
     tq = int(N.layers().jl_attn_tile_rows(_code(dtype), H, G, D, Dv, k_ld, v_ld))
     if tq <= 0:
@@ -391,7 +396,7 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
         _need(rel.shape[1] == H and (lut is None or lut.dtype == torch.int32), "attn_window: rel [rows, H] (+ int32 lut)")
     _need(chunk <= 0 or (window <= 0 and keep_first <= 0), "attn_window: chunks exclude a window and kept first tokens")
     out = _attn_out(out, n, H * Dv, torch.float32 if float_out else dt, q.device, "attn_window")
-    if (talk is not None and sink is None and chunk <= 0 and softcap <= 0 and Gv == G and N.layers().jl_attn_talk_ok(_code(dt), H, G, D, Dv, k_ld, v_ld) and out.stride(0) % 4 == 0 and
+    if (talk is not None and sink is None and chunk <= 0 and softcap <= 0 and Gv == G and N.layers().jl_attn_talk_ok(_code(dt), H, G, D, Dv, k_ld, v_ld) and _fours(out) and
             not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and not os.environ.get("JL_ATTN_NO_MFMA")):
         wide = n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B
         tq = int(N.layers().jl_attn_talk_tile_rows(H, G, int(wide)))
@@ -527,7 +532,7 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
             # requests' order, in which neighbours share keys (over a latent of 512 the sorted order was 3 % slower)
             tq, tiles = wide, batch.tiles(wide, longest_first=True)
     narrow = False
-    if tiles is None and q.dtype == torch.bfloat16 and out.stride(0) % 4 == 0 and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and \
+    if tiles is None and q.dtype == torch.bfloat16 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and \
             N.layers().jl_attn_narrow_ok(N.JL_BF16, H, G, Gv, D, Dv, k_cache.stride(0), v_cache.stride(0)):
         # few tokens per request: single wavefronts, each with a share of a tile's keys
         narrow, tq = True, int(N.layers().jl_attn_talk_tile_rows(H, G, 0))

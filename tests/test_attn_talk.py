@@ -155,3 +155,28 @@ def test_a_key_that_is_not_a_number_reaches_a_decoded_token():
     kp[640, :D] = kp[11 * page, :D] = float("nan")                   # the last key of one request, the only one of the other
     out = LO.attn_sweep(q, kp, vp, batch, H, G, D, D, D ** -0.5, 0).view(2, G, -1)
     assert bool(torch.isnan(out[:, 0]).all()) and bool(torch.isfinite(out[:, 1]).all())
+
+
+@pytest.mark.parametrize("mixed", [True, False])
+@pytest.mark.parametrize("first", [0, 1, 2, 4])
+def test_results_into_rows_that_start_anywhere(monkeypatch, mixed, first):
+    """Columns of wider rows: stored four at a time where they start at such borders, otherwise by the forms that store single values."""
+    from jacobiforcing_amd import _native as N
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, G, D = "cuda", 4, 2, 64
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    batch = LO.RaggedBatch.build([1, 3], [100, 60], [0, 1], [[0, 1], [2]], 64, dev)
+    kp, vp, q, talk = rnd(192, G * D), rnd(192, G * D), rnd(4, H * D), torch.eye(H, device=dev) + 0.2 * torch.randn(H, H, generator=g, device=dev)
+    wider = torch.zeros(4, H * D + 8, dtype=torch.bfloat16, device=dev)
+    calls, name = [], "jl_attn_talk" if mixed else "jl_attn_narrow"
+    real = getattr(N.layers(), name)
+    monkeypatch.setattr(N.layers(), name, lambda *a: calls.append(1) or real(*a), raising=False)
+    run = (lambda out: LO.attn_window(q, None, kp, vp, batch, H, G, D, D, D ** -0.5, 0, 0, None, None, talk, out=out)) if mixed else \
+        lambda out: LO.attn_sweep(q, kp, vp, batch, H, G, D, D, D ** -0.5, 0, out=out)
+    want = run(None)
+    run(wider[:, first:first + H * D])
+    assert len(calls) == (2 if first % 4 == 0 else 1)
+    assert not bool(wider[:, :first].any()) and not bool(wider[:, first + H * D:].any())
+    # both forms round weights (to bfloat16, or 16 bits) and results
+    assert (wider[:, first:first + H * D].double() - want.double()).abs().max() <= 2 * 2.0 ** -8 * want.double().abs().max()
