@@ -211,7 +211,7 @@ JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_re
 #define JL_LINEAR_ROUNDED_FLOAT 2
 JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                            int32_t out_mode, void *stream);
-/* The same for more rows (a few hundred), W of x's type, the result at a 16-byte border, operands of up to 4 GB. */
+/* The same for more rows (a few hundred), all bfloat16, the result at a 16-byte border, operands of up to 4 GB. */
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                          void *stream);
 
@@ -436,7 +436,7 @@ JL_API int jl_moe_route(const float *logits, const float *correction, int64_t N,
  * tile_row0 [max_tiles] (max_tiles >= N*top/tile_rows + E): row tiles of at most tile_rows rows of one expert, unused entries -1. */
 JL_API int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, int32_t tile_rows, int32_t *perm, int32_t *offsets,
                         int32_t *tile_expert, int32_t *tile_row0, int32_t max_tiles, void *stream);
-/* tile_rows for a step of `rows` (token, choice) rows over E experts of width ff behind a stream of width W: 32, 64 or 128 */
+/* tile_rows for a step of `rows` (token, choice) rows over E experts of width ff behind a stream of width W: 32, 64 or (bfloat16) 128 */
 JL_API int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff);
 
 /* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].

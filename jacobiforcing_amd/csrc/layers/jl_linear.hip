@@ -121,23 +121,16 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 // What bounds it: a workgroup's way through its stages, 0.27 us each however many workgroups there are, until two per CU are busy.  us of GPU time against the library's product
 // (bfloat16, W from memory): 1024 x 1024 by 256 rows 7.8 / 8.3, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 520 x 1000 by 1024 7.0 / 10.1, by 1600 10.0 / 12.0; 192 x 768 by 1600 5.4 / 5.9;
 // 1024 x 3072 by 256 8.3 / 9.0; 2048 x 2048 by 512 13.3 / 11.2; and 11 us less of host time.  Beyond the caller's line (layer_ops.linear_mid) it loses more: 4096 x 2048 by 256 20.4 / 14.4,
-// 1024 x 3072 by 1024 16.1 / 13.6, float
-// 1024 x 1024 by 512 22.5 / 12.7.  Larger tiles and deeper rings gained nothing there (128 x 128 by 8192 rows 100 / 52), nor did a share of the depth per wavefront without barriers.
+// 1024 x 3072 by 1024 16.1 / 13.6, and on the float matrix instructions everywhere (1024 x 1024 by 512 22.5 / 12.7): float rows stay with the library.  Larger tiles and deeper rings gained nothing there (128 x 128 by 8192 rows 100 / 52), nor did a share of the depth per wavefront without barriers.
 typedef float ld_f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ ld_f32x16 ld_mma(const bf16_t *, uint4 a, uint4 b, ld_f32x16 c) {
+__device__ __forceinline__ ld_f32x16 ld_mma(uint4 a, uint4 b, ld_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ls_bf16x8, a), __builtin_bit_cast(ls_bf16x8, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ ld_f32x16 ld_mma(const float *, uint4 a, uint4 b, ld_f32x16 c) {
-    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
 }
 constexpr int LD_RING = 3, LD_UNITS = 8, LD_TILE = 64;              // 16-byte units of a row per stage
 
-template <typename T>
-__global__ __launch_bounds__(256) void linear_mid_kernel(const T *__restrict__ x, int64_t x_ld, const T *__restrict__ w, const T *__restrict__ bias, void *__restrict__ out, int64_t out_ld,
-                                                         int N, int K, int O, int out_mode, int row_tiles) {
+__global__ __launch_bounds__(256) void linear_mid_kernel(const bf16_t *__restrict__ x, int64_t x_ld, const bf16_t *__restrict__ w, const bf16_t *__restrict__ bias, void *__restrict__ out,
+                                                         int64_t out_ld, int N, int K, int O, int out_mode, int row_tiles) {
+    typedef bf16_t T;
     constexpr int UNIT = 16 / sizeof(T), STAGE = LD_UNITS * UNIT, BUF = 2 * LD_TILE * LD_UNITS;
     __shared__ uint4 ldS[LD_RING * BUF];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave >> 1, wn = wave & 1;
@@ -167,7 +160,7 @@ __global__ __launch_bounds__(256) void linear_mid_kernel(const T *__restrict__ x
     auto products = [&](const uint4 *Xs) {
         const uint4 *Ws = Xs + LD_TILE * LD_UNITS;
 #pragma unroll
-        for (int s = 0; s < LD_UNITS / 2; ++s) acc = ld_mma((const T *)nullptr, Ws[at(32 * wn + l32, 2 * s + hi)], Xs[at(32 * wm + l32, 2 * s + hi)], acc);
+        for (int s = 0; s < LD_UNITS / 2; ++s) acc = ld_mma(Ws[at(32 * wn + l32, 2 * s + hi)], Xs[at(32 * wm + l32, 2 * s + hi)], acc);
     };
     if (full > 0) {
 #pragma unroll
@@ -226,16 +219,15 @@ extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, 
                              void *stream) {
     if (N <= 0 || O <= 0) return JL_OK;
     if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < O) return jl_fail(JL_E_INVALID, "jl_linear_mid: null pointer or bad sizes");
-    const int64_t unit = dtype == JL_BF16 ? 8 : 4, size = 16 / unit;
-    if ((dtype != JL_BF16 && dtype != JL_F32) || K % unit || x_ld % unit || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15))
-        return jl_fail(JL_E_INVALID, "jl_linear_mid: rows of x and W and the result at 16-byte borders");
-    if (N > INT32_MAX / 64 || N * x_ld * size > UINT32_MAX || (int64_t)O * K * size > UINT32_MAX) return jl_fail(JL_E_INVALID, "jl_linear_mid: operands of up to 4 GB");
+    if (dtype != JL_BF16 || K % 8 || x_ld % 8 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15))
+        return jl_fail(JL_E_INVALID, "jl_linear_mid: bfloat16, rows of x and W and the result at 16-byte borders");
+    if (N > INT32_MAX / 64 || N * x_ld * 2 > UINT32_MAX || (int64_t)O * K * 2 > UINT32_MAX) return jl_fail(JL_E_INVALID, "jl_linear_mid: operands of up to 4 GB");
     if (out_mode < JL_LINEAR_SAME || out_mode > JL_LINEAR_ROUNDED_FLOAT) return jl_fail(JL_E_INVALID, "jl_linear_mid: unknown out_mode");
     const int row_tiles = (int)((N + LD_TILE - 1) / LD_TILE);
     const int64_t groups = (int64_t)row_tiles * ((O + LD_TILE - 1) / LD_TILE);
     if (groups > INT32_MAX / 256) return jl_fail(JL_E_INVALID, "jl_linear_mid: too many tiles");
-    JL_DISPATCH(dtype, linear_mid_kernel<T><<<dim3((unsigned)groups), 256, 0, (hipStream_t)stream>>>((const T *)x, x_ld, (const T *)w, (const T *)bias, out, out_ld, (int)N, K, O, out_mode,
-                                                                                                    row_tiles));
+    linear_mid_kernel<<<dim3((unsigned)groups), 256, 0, (hipStream_t)stream>>>((const bf16_t *)x, x_ld, (const bf16_t *)w, (const bf16_t *)bias, out, out_ld, (int)N, K, O, out_mode,
+                                                                              row_tiles);
     return jl_check_launch("linear_mid_kernel");
 }
 

@@ -533,7 +533,9 @@ template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(
     return jl_check_launch("moe_mm_kernel");
 }
 template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated, hipStream_t st) {
-    if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
+    if constexpr (sizeof(T) == 2) {
+        if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
+    } else if (tile_rows == 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32 or 64 rows");
     if (tile_rows == 64) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
     return moe_mm_launch<T, 32, 1, 64, 8>(a, gated, st);
 }

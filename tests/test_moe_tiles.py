@@ -89,3 +89,13 @@ def test_operands_beyond_4_gib(dtype, K, gated, tile, far):
     got = run(X, W, cols, X.shape[0] - rows)
     want = run(X[-rows:].contiguous(), W[:, -n_out:].contiguous() if far == "weights" else W, n_out, 0)
     assert torch.equal(got, want) and bool(want.any())
+
+
+def test_tile_heights_of_each_type():
+    """Float rows never get the 128-row tiles, and asking for them is refused."""
+    from jacobiforcing_amd import _native as N
+    lib = N.layers()
+    heights = {dt: {lib.jl_moe_tile_rows(dt, rows, E, W, ff) for rows in (4, 500, 5000, 100000) for E in (2, 16, 64) for W in (64, 1024, 4096) for ff in (64, 1024)} for dt in (N.JL_BF16, N.JL_F32)}
+    assert heights[N.JL_BF16] == {32, 64, 128} and heights[N.JL_F32] == {32, 64}
+    x, i = torch.zeros(64, 64, device="cuda"), torch.zeros(64, dtype=torch.int32, device="cuda")
+    assert lib.jl_moe_gemm(x.data_ptr(), x.data_ptr(), N.JL_F32, N.JL_MOE_UP_PLAIN, 64, 64, 1, i.data_ptr(), i.data_ptr(), i.data_ptr(), i.data_ptr(), 1, 1, 128, None, x.data_ptr(), None) == -1
