@@ -99,3 +99,25 @@ def test_tile_heights_of_each_type():
     assert heights[N.JL_BF16] == {32, 64, 128} and heights[N.JL_F32] == {32, 64}
     x, i = torch.zeros(64, 64, device="cuda"), torch.zeros(64, dtype=torch.int32, device="cuda")
     assert lib.jl_moe_gemm(x.data_ptr(), x.data_ptr(), N.JL_F32, N.JL_MOE_UP_PLAIN, 64, 64, 1, i.data_ptr(), i.data_ptr(), i.data_ptr(), i.data_ptr(), 1, 1, 128, None, x.data_ptr(), None) == -1
+
+
+@pytest.mark.parametrize("dtype,tile", [("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128), ("float32", 32), ("float32", 64)])
+@pytest.mark.parametrize("N,E,top,W,ff,gated,identity,skew", [
+    (1, 3, 2, 8, 8, True, 0, 0.0), (130, 3, 2, 24, 32, True, 0, 0.0), (259, 4, 2, 64, 96, True, 1, 0.0), (257, 2, 1, 96, 64, False, 0, 0.0), (300, 5, 2, 72, 264, True, 0, 0.0), (200, 3, 1, 64, 50, True, 0, 0.0),
+    (513, 9, 1, 160, 136, False, 0, 9.0), (1100, 2, 1, 520, 264, True, 0, 1.0), (640, 40, 2, 40, 256, True, 4, 3.0), (385, 4, 3, 1024, 520, True, 0, 0.0),
+])
+def test_every_tile_height(monkeypatch, dtype, tile, N, E, top, W, ff, gated, identity, skew):
+    """The same with tiles of one height: depths of one, two, three and more stages, beside and below them, columns beside their fours, experts with few rows, many or none."""
+    from jacobiforcing_amd import _native as N_
+    asked = []
+    monkeypatch.setattr(N_.layers(), "jl_moe_tile_rows", lambda *a: asked.append(a) or tile, raising=False)
+    test_experts(dtype, N, E, top, W, ff, gated, identity, skew)
+    assert asked
+
+
+@pytest.mark.parametrize("dtype,tile,N,E,W,ff", [("bfloat16", 128, 4096, 16, 1024, 512), ("bfloat16", 64, 3000, 40, 520, 256), ("float32", 64, 2048, 16, 1024, 256)])
+def test_tile_heights_that_the_rule_chooses(dtype, tile, N, E, W, ff):
+    from jacobiforcing_amd import _native as N_
+    from jacobiforcing_amd import layer_ops as LO
+    assert N_.layers().jl_moe_tile_rows(LO._code(getattr(torch, dtype)), 4 * N, E, W, ff) == tile
+    test_experts(dtype, N, E, 4, W, ff, True, 0, 0.0)
