@@ -304,7 +304,7 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 // between the wavefronts of a chain.  T comes from 16 x 16 blocks by substitution, joined by products, on one wavefront while the others make P.
 // What bounds it: the chain's 128 matrix instructions of 64 cycles per chunk on the busiest of its four wavefronts (D = 128; 58 % of its time), and in the chunks' kernel the
 // phases of a workgroup that wait for each other (two workgroups per CU at 79 104 bytes of LDS; with one, 302 us instead of 198).
-// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 446 us (chunks 198, chain 214,
+// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 430 us (chunks 198, chain 214,
 // norm 34); 8 heads, one portion of 128 80 -> 45; 16 heads, 777 + 300 tokens beside 30 single ones 566 -> 148; float, 8 heads, 1021 + 851 + 681 tokens 587 -> 149.
 constexpr int DK_T = 64;
 typedef float dk_f32x16 __attribute__((ext_vector_type(16)));
@@ -324,6 +324,12 @@ __device__ __forceinline__ dk_f32x4 dk_mma16(float4 a, float4 b, dk_f32x4 c) {
 __device__ __forceinline__ void dk_wave_sync() {        // LDS written by some lanes is read by others of the same wavefront
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// e ** x of a 64-bit sum: the float next to x, and what is left of x to first order (rounding x itself would cost |x| 2 ** -25)
+__device__ __forceinline__ float dk_exp(double x) {
+    const float hi = (float)x, e = expf(hi);
+    return fmaf(e, (float)(x - (double)hi), e);
 }
 
 // floats of scratch: per chunk and head W2, W1, P, e^c and e^(c_63 - c); per chunk and key head the unit vectors
@@ -395,12 +401,12 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
             if (lane >= off) c += y;
         }
         const double end = __shfl(c, 63, 64);
-        const float gam = expf((float)c);
+        const float gam = dk_exp(c);
         cs[lane] = c;
         bs[lane] = beta;
         bg[lane] = -beta * gam;
         head[z.p + 3 * 1024 + lane] = gam;
-        head[z.p + 3 * 1024 + DK_T + lane] = expf((float)(end - c));
+        head[z.p + 3 * 1024 + DK_T + lane] = dk_exp(end - c);
     }
     __syncthreads();
     // from the first token with a key, decay or beta that is not a number on: nothing here that zeros would spread to the tokens in front of it; W1 says so instead
@@ -414,15 +420,25 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
     // a quarter [32 t, 32 j] of K K^T or Q K^T: lane l ends with t = 32 ti + l % 32, unit y the four j at 32 tj + 8 y + 4 (l / 32)
     auto pairs = [&](const float4 *rows, int ti, int tj, bool diagonal, float row_factor, auto &&store) {
         const int t = 32 * ti + l32, j = 32 * tj + l32;
-        dk_f32x16 s, s2;
+        dk_f32x16 s;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = s2[r] = 0.f;
-#pragma unroll 2
-        for (int x = 0; x < U / 2; x += 2) {
-            s = dk_mma(Ks[j * U + at(j, 2 * x + hi)], rows[t * U + at(t, 2 * x + hi)], s);
-            s2 = dk_mma(Ks[j * U + at(j, 2 * x + 2 + hi)], rows[t * U + at(t, 2 * x + 2 + hi)], s2);
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll 1
+        for (int x0 = 0; x0 < U / 2; x0 += U / 4) {               // sums of 8 products in a row, met in pairs: what 64 in a row lose shows in the outputs
+            dk_f32x16 half;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) half[r] = 0.f;
+#pragma unroll 1
+            for (int x = x0; x < x0 + U / 4; x += 2) {
+                dk_f32x16 s1, s2;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s1[r] = s2[r] = 0.f;
+                s1 = dk_mma(Ks[j * U + at(j, 2 * x + hi)], rows[t * U + at(t, 2 * x + hi)], s1);
+                s2 = dk_mma(Ks[j * U + at(j, 2 * x + 2 + hi)], rows[t * U + at(t, 2 * x + 2 + hi)], s2);
+                half += s1 + s2;
+            }
+            s += half;
         }
-        s += s2;
         const double ct = cs[t];
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
@@ -430,7 +446,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int jj = 32 * tj + 8 * y + 4 * hi + i;
-                v[i] = jj < t || (diagonal && jj == t) ? s[4 * y + i] * row_factor * expf((float)(ct - cs[jj])) : 0.f;
+                v[i] = jj < t || (diagonal && jj == t) ? s[4 * y + i] * row_factor * dk_exp(ct - cs[jj]) : 0.f;
             }
             store(t, y, make_float4(v[0], v[1], v[2], v[3]));
         }
@@ -646,23 +662,23 @@ __global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, 
         const int row0 = a.chunk_rec[4 * c], cnt = a.chunk_rec[4 * c + 1];
         const sources q = sources_of(c + 1 < first + n ? c + 1 : c);    // every operand's successor sets out when it has been used: a whole chunk ahead, in its registers
         __syncthreads();                                            // S is there, U has been read
-        dk_f32x16 acc, part[3];                                     // four shorter sums: a rounding each, and what 128 in a row lose is more than the scan's lanes do
+        // Short sums that start from nothing, then met: what 128 products in a row lose, or as many onto a W1 larger than they are, is more than the lanes of the other forms do
+        dk_f32x16 acc, part[4];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            acc[r] = maker ? ((const float *)&w1[r >> 2])[r & 3] : 0.f;
-            part[0][r] = part[1][r] = part[2][r] = 0.f;
-        }
+        for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = part[2][r] = part[3][r] = 0.f;
 #pragma unroll
         for (int u = 0; u < NU; u += 4) {
             part[0] = dk_mma(fa[u], Sf[u * 64 + lane], part[0]);
             part[1] = dk_mma(fa[u + 1], Sf[(u + 1) * 64 + lane], part[1]);
             part[2] = dk_mma(fa[u + 2], Sf[(u + 2) * 64 + lane], part[2]);
-            acc = dk_mma(fa[u + 3], Sf[(u + 3) * 64 + lane], acc);
+            part[3] = dk_mma(fa[u + 3], Sf[(u + 3) * 64 + lane], part[3]);
 #pragma unroll
             for (int i = 0; i < 4; ++i) fa[u + i] = q.a[(u + i) * 64];
         }
-        acc += (part[0] + part[1]) + part[2];
+        acc = (part[0] + part[1]) + (part[2] + part[3]);
         if (maker) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] += ((const float *)&w1[r >> 2])[r & 3];
             float zero[4] = {0.f, 0.f, 0.f, 0.f};                   // not a number if a correction is not finite
 #pragma unroll
             for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(acc[r], 0.f, zero[r & 3]);
@@ -680,35 +696,37 @@ __global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, 
                 Uf[(4 * ti + y) * 64 + lane] = make_float4(u[4 * y], u[4 * y + 1], u[4 * y + 2], u[4 * y + 3]);
                 Ug[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y] * sc[y].x, acc[4 * y + 1] * sc[y].y, acc[4 * y + 2] * sc[y].z, acc[4 * y + 3] * sc[y].w);
             }
-        } else
-#pragma unroll
-            for (int y = 0; y < 4; ++y) { acc[4 * y] *= sc[y].x; acc[4 * y + 1] *= sc[y].y; acc[4 * y + 2] *= sc[y].z; acc[4 * y + 3] *= sc[y].w; }
+        }
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
-            if (maker) w1[y] = q.w1[y * 64];
-            sc[y] = q.sc[2 * y];
+            if (maker) { w1[y] = q.w1[y * 64]; sc[y] = q.sc[2 * y]; }
         }
         __syncthreads();                                            // U is there, S has been read
         if (owner) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) S[r] *= gend;
+            for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = 0.f;
 #pragma unroll
             for (int y = 0; y < 8; ++y) {
-                S = dk_mma(fk[y], Ug[y * 64 + lane], S);
+                part[y >> 2] = dk_mma(fk[y], Ug[y * 64 + lane], part[y >> 2]);
                 fk[y] = q.k[y * 64];
             }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) S[r] = fmaf(S[r], gend, part[0][r] + part[1][r]);
             gend = *q.gend;
             share_state();
         }
         if (!maker) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) part[0][r] = 0.f;
+            for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = 0.f;
 #pragma unroll
-            for (int y = 0; y < 4; ++y) part[0] = dk_mma(fp[y], Uf[y * 64 + lane], part[0]);
+            for (int y = 0; y < 4; ++y) part[y & 1] = dk_mma(fp[y], Uf[y * 64 + lane], part[y & 1]);
             if (ti)
 #pragma unroll
-                for (int y = 4; y < 8; ++y) acc = dk_mma(fp[y], Uf[y * 64 + lane], acc);
-            acc += part[0];
+                for (int y = 4; y < 8; ++y) part[y & 1] = dk_mma(fp[y], Uf[y * 64 + lane], part[y & 1]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] = fmaf(acc[r], ((const float *)&sc[r >> 2])[r & 3], part[0][r] + part[1][r]);
+#pragma unroll
+            for (int y = 0; y < 4; ++y) sc[y] = q.sc[2 * y];
             const int none = min(noneS[0][l32], noneS[1][l32]);
             if (__any(none < DK_T))
 #pragma unroll

@@ -120,3 +120,34 @@ def test_portions_of_all_kinds(H, G, D, counts, least):
         assert any(k[0] == "long" for k in batch._tiles if isinstance(k, tuple)) == (chunks > 0)
     # 32-bit sums in another order, a few roundings of 2 ** -24 each, normed
     assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[1].norm() and (states[0] - states[1]).norm() <= 4e-6 * states[1].norm()
+
+
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (8, 8, 64)])
+@pytest.mark.parametrize("lo,hi", [(-3.0, 1.0), (-6.0, -4.0)])
+def test_chunks_lose_no_more_bits_than_the_columns(H, G, D, lo, hi):
+    """Errors against 64 bits of both forms in float, short and long memories: the state's is no larger, the outputs' (normed, so that errors of a row's size drop out of both) at most a sixth larger."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, n, errs = "cuda", 1021, {}
+    for seed in range(3):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+        qkv, proj = torch.nn.functional.silu(rnd(n, 2 * G * D + H * D)), rnd(n, 2 * H + H * D)
+        a_log, bias, w, start = lo + (hi - lo) * torch.rand(H, generator=g, device=dev), rnd(H), 1 + 0.1 * rnd(D), 0.1 * rnd(1, H, D, D)
+        x, p = qkv.double(), proj.double()
+        unit = lambda y: (y / torch.sqrt((y * y).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(H // G, 1)
+        q, k = (unit(x[:, c:c + G * D].view(n, G, D)) for c in (0, G * D))
+        v, dec, beta = x[:, 2 * G * D:].view(n, H, D), torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, :H] + bias.double())), torch.sigmoid(p[:, H:2 * H])
+        S, o = start[0].double(), []
+        for t in range(n):
+            S = dec[t].view(H, 1, 1) * S
+            S = S + k[t].unsqueeze(-1) * (beta[t].view(H, 1) * (v[t] - (k[t].unsqueeze(-2) @ S).squeeze(-2))).unsqueeze(-2)
+            o.append((q[t].unsqueeze(-2) @ S).squeeze(-2) * D ** -0.5)
+        o = torch.stack(o)
+        o = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * w.double() * torch.nn.functional.silu(p[:, 2 * H:].view(n, H, D))
+        for form in (0, 64):
+            batch, st = LO.RaggedBatch.build([n], [100], [0], [list(range(18))], 64, dev), start.clone()
+            batch._tiles[("delta", H, D)] = form
+            got = LO.delta_rule(qkv, (0, G * D, 2 * G * D), proj, (0, H, 2 * H), a_log, bias, w, batch, H, G, D, D, 1e-6, D ** -0.5, 1e-5, st)
+            for name, a, b in (("out", got.double().view(n, H, D), o), ("state", st[0].double(), S)):
+                errs[name, form] = errs.get((name, form), 0.0) + ((a - b).norm() / b.norm()).item()
+    assert errs["state", 64] <= errs["state", 0] and errs["out", 64] <= 7 / 6 * errs["out", 0], errs
