@@ -303,8 +303,8 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 // product's operand as they are: between the kernels (every operand as units [unit][lane], read as 1 KB per wavefront straight into registers, a chunk ahead) and in LDS
 // between the wavefronts of a chain.  T comes from 16 x 16 blocks by substitution, joined by products, on one wavefront while the others make P.
 // What bounds it: the chain's 128 matrix instructions of 64 cycles per chunk on the busiest of its four wavefronts (D = 128; 58 % of its time), and in the chunks' kernel the
-// phases of a workgroup that wait for each other (two workgroups per CU at 79 104 bytes of LDS; with one, 302 us instead of 198).
-// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 430 us (chunks 198, chain 214,
+// phases of a workgroup that wait for each other (two workgroups per CU at 79 104 bytes of LDS; with one, 302 us instead of 198, measured then).
+// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 430 us (chunks 210, chain 210,
 // norm 34); 8 heads, one portion of 128 80 -> 45; 16 heads, 777 + 300 tokens beside 30 single ones 566 -> 148; float, 8 heads, 1021 + 851 + 681 tokens 587 -> 149.
 constexpr int DK_T = 64;
 typedef float dk_f32x16 __attribute__((ext_vector_type(16)));

@@ -179,7 +179,7 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // What bounds it: 368 matrix instructions of 64 cycles per wavefront and group of 64 tokens at 128 x 128, and the phases of a group at one workgroup per CU.
 // Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups (a second pass over a group that holds one).
 // Outputs leave as floats and are normed and gated by rows in a launch of their own: in this one, a wavefront's sums over its 32 columns cost 160 exchanges per group and the gates
-// came two bytes at a time, four on their way (outputs 211 us then, 112 and 18 now).
+// came two bytes at a time, four on their way (outputs 211 us then, 119 and 18 now).
 // Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 182 us, one prompt of 128
 // 985 -> 53, 8 x 8 tokens 84 -> 34; float, 1021 + 851 + 681 tokens: 1091 -> 105.
 constexpr int RM_T = 64, RM_OUT = 0, RM_LOCAL = 1;

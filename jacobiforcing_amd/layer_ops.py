@@ -20,9 +20,12 @@ from . import _native as N
 ATTN_SPLIT_BELOW_TILES, ATTN_SPLIT_WORKGROUPS = 128, 512     # attention: split a tile's keys while tiles x splits stays below ~2 per CU
 ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-core attention kernel takes in one workgroup
 # mixed heads: workgroups of 4 wavefronts to aim at (of one: three times as many); scratch at most (1 GiB: more tiles than it holds take turns), as long as it holds a tile's.  us, 8 heads
-# over 2 of 128 under a window of 1024, for 512 / 640 / 1024: 777 + 300 tokens beside 30 single ones 105 / 79 / 81, one portion of 1000 54 / 56 / 65
+# over 2 of 128 under a window of 1024, for 512 / 640 / 1024: 777 + 300 tokens beside 30 single ones 105 / 79 / 81, one portion of 1000 54 / 56 / 65.  The form costs a product with the
+# values per value head, and is taken for up to 8 of them: us, two sweeps / this, 4 x 2048 tokens, 32 single ones: 8 heads over 1 688 / 102, 122 / 29; 4 over 4 1011 / 179, 196 / 81; 16 over 4
+# 1891 / 585, 299 / 93; sizes that went to float multiply-adds before: 12 over 6 51800 / 689, 16 over 8 70400 / 1270
 TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
-NARROW_WORKGROUPS = 2048              # attention of a few tokens per request: single wavefronts to aim at when keys are shared out
+NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, and of portions too few for the 128-row tiles (one of 1000 / 2040 tokens, 8 heads over 2 of 128: 66 -> 36, 193 -> 67 us;
+                                      # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
 BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
