@@ -42,3 +42,22 @@ def test_a_batch_without_its_tables_on_the_host():
         assert all(torch.equal(x, y) for x, y in zip(b.key_rows([0, 1], window), bare.key_rows([0, 1], window)))
     (s1, r1), (s2, r2) = b.part([1, 2]), bare.part([1, 2])
     assert torch.equal(r1, r2) and torch.equal(s1.kv_slot, s2.kv_slot) and torch.equal(s1.tables, s2.tables)
+
+
+@pytest.mark.parametrize("counts,starts,page,window", [([70, 3, 9], [0, 130, 2], 64, 0), ([70, 3, 9], [0, 130, 2], 64, 50), ([1, 33, 16, 65], [31, 0, 48, 640], 16, 17), ([5], [0], 1, 0),
+                                                       ([64, 64], [64, 0], 64, 64), ([7, 2, 90], [100, 64, 3], 48, 1)])
+def test_key_rows_are_those_of_the_pages_in_one_upload(monkeypatch, counts, starts, page, window):
+    b = batch(counts, starts, page)
+    for requests in (list(range(len(counts))), [len(counts) - 1], [0, len(counts) - 1][:len(counts)]):
+        b._tiles.clear()
+        want, base = [], [0] * len(counts)
+        for r in requests:
+            first = max(0, starts[r] - window + 1) if window else 0
+            base[r] = len(want) - first
+            want += [int(b.tables[r, p // page]) * page + p % page for p in range(first, starts[r] + counts[r])]
+        uploads, to = [], torch.Tensor.to
+        monkeypatch.setattr(torch.Tensor, "to", lambda t, *a, **k: uploads.append(t.shape) or to(t, *a, **k))
+        tokens, places = b.key_rows(requests, window)
+        monkeypatch.undo()
+        assert tokens.dtype == torch.int64 and places.dtype == torch.int32 and tokens.tolist() == want and places.tolist() == base
+        assert len(uploads) == 1                                        # each waits for everything queued before it
