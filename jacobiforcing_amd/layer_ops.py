@@ -5,7 +5,9 @@ A step's tokens form one ragged batch (``RaggedBatch``): N token rows, the rows 
 records and tiles the kernels read."""
 from __future__ import annotations
 
+import bisect
 import ctypes as C
+import itertools
 import os
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
@@ -1198,21 +1200,23 @@ def delta_chunks_from(counts: Sequence[int], H: int, D: int) -> int:
     100 x 64 333 / 225 / 225."""
     if max(counts) < DELTA_CHUNKS_FROM or len(counts) == 1:
         return DELTA_CHUNKS_FROM if max(counts) >= DELTA_CHUNKS_FROM else 0
-    c = np.asarray(counts)
     first, chain, chunk, step, token, request, alone, single = (30, 6.7, 0.28, 0.6, 5.5e-3, 0.05, 2.7, 0.045) if D > 64 else (24, 4.9, 0.145, 0.49, 1.34e-3, 6e-3, 1.4, 0.012)
+    c = sorted(counts)
+    held = [0, *itertools.accumulate(c)]                  # tokens of the shortest ones
 
-    def others(r):
-        if r.size == 0:
+    def others(k):                                        # of the k shortest
+        if k == 0:
             return 0.0
-        longest, tokens, pairs = int(r.max()), int(r.sum()) * H, r.size * H
+        longest, tokens, pairs = c[k - 1], held[k] * H, k * H
         if longest >= DELTA_COLUMNS_FROM:
             return 8 + max(step * longest, 0.6 * step * longest + token * tokens + request * pairs)
         return 8 + max(alone * longest, single * pairs + 0.012 * (tokens - pairs))
 
-    best, least = others(c), 0
+    best, least, k64 = others(len(c)), 0, bisect.bisect_left(c, 64)
+    chunks = sum(-(-x // 64) for x in c[k64:])            # of 64 tokens and more; each shorter one is one
     for m in (2, 8, 16, DELTA_COLUMNS_FROM, 64):
-        n = -(-c[c >= m] // 64)
-        t = first + max(chain * int(n.max()), chunk * int(n.sum()) * H) + others(c[c < m]) if n.size else best
+        k = bisect.bisect_left(c, m)
+        t = first + max(chain * -(-c[-1] // 64), chunk * H * (chunks + k64 - k)) + others(k)
         best, least = (t, m) if t < best else (best, least)
     return least
 

@@ -1,4 +1,7 @@
 """What a step's tables and rules on the host hold (no kernel runs)."""
+import random
+
+import numpy as np
 import pytest
 import torch
 
@@ -61,3 +64,28 @@ def test_key_rows_are_those_of_the_pages_in_one_upload(monkeypatch, counts, star
         monkeypatch.undo()
         assert tokens.dtype == torch.int64 and places.dtype == torch.int32 and tokens.tolist() == want and places.tolist() == base
         assert len(uploads) == 1                                        # each waits for everything queued before it
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_the_rule_is_the_cheapest_of_its_estimates(seed):
+    """Against the same estimates over whole lists, for steps of all kinds; no kernel runs."""
+    r = random.Random(seed)
+    for _ in range(500):
+        counts = [r.choice([1, r.randint(1, r.choice([3, 31, 64, 300, 2000]))]) for _ in range(r.randint(2, 60))] + [r.randint(64, 700)]
+        H, D = r.choice([1, 4, 8, 16, 32]), r.choice([64, 128])
+        c = np.asarray(counts)
+        first, chain, chunk, step, token, request, alone, single = (30, 6.7, 0.28, 0.6, 5.5e-3, 0.05, 2.7, 0.045) if D > 64 else (24, 4.9, 0.145, 0.49, 1.34e-3, 6e-3, 1.4, 0.012)
+
+        def others(r):
+            if r.size == 0:
+                return 0.0
+            longest, tokens, pairs = int(r.max()), int(r.sum()) * H, r.size * H
+            if longest >= LO.DELTA_COLUMNS_FROM:
+                return 8 + max(step * longest, 0.6 * step * longest + token * tokens + request * pairs)
+            return 8 + max(alone * longest, single * pairs + 0.012 * (tokens - pairs))
+
+        ways = {0: others(c)}
+        for m in (2, 8, 16, LO.DELTA_COLUMNS_FROM, 64):
+            n = -(-c[c >= m] // 64)
+            ways[m] = first + max(chain * int(n.max()), chunk * int(n.sum()) * H) + others(c[c < m])
+        assert ways[LO.delta_chunks_from(counts, H, D)] == min(ways.values())
