@@ -138,7 +138,7 @@ JL_API int jl_attn_sweep_wide_tile_rows(int dtype, int32_t H, int32_t G, int32_t
  * scratch of jl_attn_talk_scratch_floats for pass_tiles tiles at a time.  q, pools and scratch at 16-byte borders, k_ld and v_ld in multiples of 8, out_ld of 4; out at the borders of four values. */
 JL_API int jl_attn_talk(const jl_attn_args *a, int32_t wide, int32_t pass_tiles, void *stream);
 /* jl_attn_sweep for portions of a few tokens (decoding), the same arguments, in tiles of jl_attn_talk_tile_rows(H, G, 0) queries; scratch of
- * jl_attn_talk_scratch_floats(tiles, TQ, H, 1, Dv, splits); sizes as jl_attn_narrow_ok takes them, alignment as for jl_attn_talk. */
+ * jl_attn_talk_scratch_floats(tiles, TQ, H, 1, Dv, splits) where keys are shared out (splits > 1); sizes as jl_attn_narrow_ok takes them, alignment as for jl_attn_talk. */
 JL_API int jl_attn_narrow(const jl_attn_args *a, void *stream);
 JL_API int jl_attn_narrow_ok(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);
 JL_API int jl_attn_talk_ok(int dtype, int32_t H, int32_t G, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld);

@@ -243,6 +243,29 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     }
     l_run += __shfl_xor(l_run, 32, 64);
     if (!ok) return;
+    if (!MIX && S == 1) {                                           // keys not shared out: what attn_narrow_join_kernel does with one share, without the way through the scratch
+        const int h = h0 + hl;
+        const float sink = a.sink ? a.sink[h] * LOG2E : -INFINITY, M = fmaxf(sink, m_run), w = m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - M) : 0.f;
+        const float L = (a.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f) + w * l_run, inv = L != 0.f ? a.out_scale / L : 0.f;
+        const int64_t n = row0 + ii;
+        const bf16_t *gate = (const bf16_t *)a.gate;
+#pragma unroll
+        for (int y = 0; y < NDV; ++y)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = 32 * y + 8 * q + 4 * hi;
+                if (col >= Dv) continue;
+                float v[4];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    v[x] = (m_run > -INFINITY ? w * acc[y][4 * q + x] : 0.f) * inv;
+                    if (gate) v[x] *= 1.0f / (1.0f + __expf(-ld_f(gate + n * a.gate_ld + (a.gate_heads ? h : h * Dv + col + x))));
+                }
+                if (a.out_dtype == JL_OUT_F32) st4_f((float *)a.out + n * a.out_ld + h * Dv + col, v);
+                else st4_f((bf16_t *)a.out + n * a.out_ld + h * Dv + col, v);
+            }
+        return;
+    }
     // shares of the pass's rows: [tile, query][split][head][value head][Dv], and their maxima and sums [..][head][2] behind all of them
     const int64_t row = ((int64_t)ti * TQ + ii) * S + split;
     const int GW = MIX ? G : 1;
@@ -397,7 +420,8 @@ extern "C" int jl_attn_talk(const jl_attn_args *ap, int32_t wide, int32_t pass_t
 // ---- the same for single tokens without mixed heads: a wavefront's keys once, one product with the values -----------------------------------------
 // Decoding's attention is bound by the way to its keys: four wavefronts that meet at three barriers per 32 keys and fetch each tile's rows behind its page numbers (jl_attn_sweep.hip)
 // read keys and values at 1.3 TB/s; single wavefronts, eight to a CU, that keep their rows to themselves at 3.1.  us for both launches, sweep / this (20 and less are the host's): 32 tokens at 2048,
-// 16 heads of 128 over 4 100 / 43, 8 over 2 68 / 32; 200 tokens at 1000, 16 over 4 538 / 103; 48 at 500 40 / 25; 30 portions of 10 at 1000, 8 over 2 63 / 30; 512 tokens 50 / 31.
+// 16 heads of 128 over 4 100 / 43, 8 over 2 68 / 32; 200 tokens at 1000, 16 over 4 538 / 103; 48 at 500 40 / 25; 30 portions of 10 at 1000, 8 over 2 63 / 30; 512 tokens 50 / 31.  Few keys are not shared out (layer_ops.NARROW_WHOLE): their
+// rows leave finished, in one launch.
 // A (token, head) row's shares joined: w = 2 ** (m - M) / L with the sink as one more share that holds nothing, times the gate
 __global__ __launch_bounds__(256) void attn_narrow_join_kernel(jl_attn_args a, int64_t groups) {
     const int64_t r = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
@@ -446,6 +470,7 @@ template <int KU, int VU> static int an_launch(const jl_attn_args &a, hipStream_
     const size_t lds = at_lds_bytes(KU, VU, a.TQ, a.H / a.G, 1);
     auto kern = attn_talk_kernel<KU, VU, 1, false>;
     kern<<<dim3((unsigned)(a.n_tiles * a.splits * a.G)), 64, lds, st>>>(a, a.H / a.G, 0, a.n_tiles);
+    if (a.splits == 1) return jl_check_launch("attn_talk_kernel (single tokens)");
     const int64_t groups = (int64_t)a.n_tiles * a.TQ * a.H;
     attn_narrow_join_kernel<<<dim3((unsigned)((groups + 7) / 8)), 256, 0, st>>>(a, groups);
     return jl_check_launch("attn_talk_kernel (single tokens)");
@@ -455,7 +480,7 @@ extern "C" int jl_attn_narrow(const jl_attn_args *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null arguments");
     const jl_attn_args &a = *ap;
     if (a.n_tiles <= 0) return JL_OK;
-    if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.block_tables || !a.tiles || !a.scratch) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null pointer");
+    if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.block_tables || !a.tiles || (a.splits > 1 && !a.scratch)) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null pointer");
     if (!jl_attn_narrow_ok(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld) || a.k_ld < (int64_t)a.G * a.D || a.v_ld < (int64_t)a.Gv * a.Dv ||
         (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.v_cache | (uintptr_t)a.scratch) & 15))
         return jl_fail(JL_E_INVALID, "jl_attn_narrow: sizes or alignment (ask jl_attn_narrow_ok)");

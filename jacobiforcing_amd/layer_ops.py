@@ -28,6 +28,8 @@ ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-co
 TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
 NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, and of portions too few for the 128-row tiles (one of 1000 / 2040 tokens, 8 heads over 2 of 128: 66 -> 36, 193 -> 67 us;
                                       # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
+NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
+                                      # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
 BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
@@ -549,8 +551,9 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
         narrow, tq = True, int(N.layers().jl_attn_talk_tile_rows(H, G, 0))
         tiles = batch.tiles(tq)
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
-        splits = max(1, min(-(-reach // 64), NARROW_WORKGROUPS // (tiles.shape[0] * G), 64))
-        scratch = torch.empty((int(N.layers().jl_attn_talk_scratch_floats(tiles.shape[0], tq, H, 1, Dv, splits)),), dtype=torch.float32, device=q.device)
+        splits = max(1, min(-(-reach // 64), NARROW_WORKGROUPS // (tiles.shape[0] * G), 64)) if reach > NARROW_WHOLE else 1
+        if splits > 1:
+            scratch = torch.empty((int(N.layers().jl_attn_talk_scratch_floats(tiles.shape[0], tq, H, 1, Dv, splits)),), dtype=torch.float32, device=q.device)
     elif tiles is None and groups < below:
         tiles = batch.tiles(tq)
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)

@@ -180,3 +180,34 @@ def test_results_into_rows_that_start_anywhere(monkeypatch, mixed, first):
     assert not bool(wider[:, :first].any()) and not bool(wider[:, first + H * D:].any())
     # both forms round weights (to bfloat16, or 16 bits) and results
     assert (wider[:, first:first + H * D].double() - want.double()).abs().max() <= 2 * 2.0 ** -8 * want.double().abs().max()
+
+
+@pytest.mark.parametrize("H,G,Gv,D,Dv,counts,starts,kw", [
+    (8, 2, 2, 128, 128, [1] * 3, [127, 0, 60], {}), (8, 2, 2, 128, 128, [1] * 3, [128, 0, 60], {}), (6, 2, 1, 72, 96, [3, 1, 20], [100, 64, 0], dict(gate="value")),
+    (4, 1, 1, 64, 32, [2, 1], [700, 3], dict(window=120, sink=True, gate="head")), (4, 1, 1, 64, 64, [2, 1], [700, 3], dict(window=121)), (32, 1, 1, 40, 64, [5], [0], dict(sink=True, chunk=3, float_out=True)),
+])
+def test_few_keys_are_not_shared_out(monkeypatch, H, G, Gv, D, Dv, counts, starts, kw):
+    """Up to NARROW_WHOLE keys: one launch without a scratch, whose results are those of the shares."""
+    from jacobiforcing_amd import _native as N
+    from jacobiforcing_amd import layer_ops as LO
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    n, need = sum(counts), [-(-(c + s) // 16) for c, s in zip(counts, starts)]
+    at = [sum(need[:b]) for b in range(len(need))]
+    batch = LO.RaggedBatch.build(counts, starts, list(range(len(counts))), [list(range(a, a + x)) for a, x in zip(at, need)], 16, dev)
+    kp, vp, q = rnd(sum(need) * 16, G * D).bfloat16(), rnd(sum(need) * 16, Gv * Dv).bfloat16(), rnd(n, H * D).bfloat16()
+    gate = None if "gate" not in kw else rnd(n, H if kw["gate"] == "head" else H * Dv).bfloat16()
+    sink = rnd(H) if kw.get("sink") else None
+    seen, real = [], N.layers().jl_attn_narrow
+    monkeypatch.setattr(N.layers(), "jl_attn_narrow", lambda a, st: seen.append((a._obj.splits, a._obj.scratch)) or real(a, st), raising=False)
+    run = lambda: LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, D ** -0.5, kw.get("window", 0), value_heads=Gv, float_out=kw.get("float_out", False), sink=sink, gate=gate,
+                                gate_per_head=kw.get("gate") == "head", chunk=kw.get("chunk", 0), out_scale=0.75)
+    whole = run()
+    monkeypatch.setattr(LO, "NARROW_WHOLE", 0)
+    shared = run()
+    tq = int(N.layers().jl_attn_talk_tile_rows(H, G, 0))
+    reach = min(batch.max_pos, kw["window"] + tq if "window" in kw else kw["chunk"] + tq if "chunk" in kw else batch.max_pos)
+    assert (seen[0] == (1, None)) == (reach <= 128) and (seen[1][0] > 1) == (reach > 64)
+    # each rounds a row's weights and results to bfloat16 once, after other partial maxima
+    assert (whole.double() - shared.double()).norm() <= 2 * 2.0 ** -8 * shared.double().norm()
