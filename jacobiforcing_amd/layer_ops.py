@@ -66,7 +66,7 @@ def _need(cond: bool, msg: str) -> None:
 
 
 def _dev(t: torch.Tensor) -> None:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise N.NativeLibraryError("the layer kernels run on the GPU only (no CPU fallback)")
 
 
@@ -263,27 +263,36 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
     n, k = x.shape
-    o, size = w.shape[0], w.element_size()
-    _need(w.dtype == x.dtype or (w.dtype == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
-    small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, size)
-    if ((small or (w.dtype == x.dtype and linear_mid(n, k, o, x.dtype))) and w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and
-            x.stride(0) * x.element_size() % 16 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == w.dtype and bias.shape == (o,) and bias.is_contiguous())) and
-            x.dtype in _LINEAR_TYPES and k > 0 and w.get_device() == x.get_device() and (bias is None or bias.get_device() == x.get_device()) and
-            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))):
-        out = torch.empty((n, o), dtype=x.dtype if float_out is None else torch.float32, device=x.device)
-        mode = _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT
-        if small:
-            N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), _code(w.dtype), k, o, _ptr(bias), out.data_ptr(), o, mode,
-                                                     _stream(x.device)), "jl_linear_small")
-            return out
-        if n * x.stride(0) * size < 1 << 32:
-            N.check_layers(N.layers().jl_linear_mid(x.data_ptr(), _code(x.dtype), n, x.stride(0), w.data_ptr(), k, o, _ptr(bias), out.data_ptr(), o, mode, _stream(x.device)),
-                           "jl_linear_mid")
-            return out
-    if float_out and w.dtype != torch.float32:
+    o, dt, wt = w.shape[0], x.dtype, w.dtype
+    same = wt == dt
+    _need(same or (wt == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
+    small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
+    if small or (same and linear_mid(n, k, o, dt)):
+        size = w.element_size()
+        if (w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and
+                (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == wt and bias.shape == (o,) and bias.is_contiguous())) and dt in _LINEAR_TYPES and k > 0 and
+                w.get_device() == x.get_device() and (bias is None or bias.get_device() == x.get_device()) and
+                not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))):
+            mode = _LINEAR_SAME if float_out is None else _LINEAR_FLOAT if float_out else _LINEAR_ROUNDED_FLOAT
+            if small:
+                out = torch.empty((n, o), dtype=dt if float_out is None else torch.float32, device=x.device)
+                N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(dt), n, x.stride(0), w.data_ptr(), _code(wt), k, o, _ptr(bias), out.data_ptr(), o, mode,
+                                                         _stream(x.device)), "jl_linear_small")
+                return out
+            if n * x.stride(0) * size < 1 << 32:
+                out = torch.empty((n, o), dtype=dt if float_out is None else torch.float32, device=x.device)
+                N.check_layers(N.layers().jl_linear_mid(x.data_ptr(), _code(dt), n, x.stride(0), w.data_ptr(), k, o, _ptr(bias), out.data_ptr(), o, mode, _stream(x.device)),
+                               "jl_linear_mid")
+                return out
+    # the library's, with as little before it as there was when models called it themselves
+    if not same:
+        x = x.float()
+    if float_out and wt != torch.float32:
         y = torch.mm(x, w.t(), out_dtype=torch.float32)
         return y if bias is None else y + bias
-    y = F.linear(x.to(w.dtype), w, bias)
+    if float_out and bias is None:
+        return torch.mm(x, w.t())
+    y = F.linear(x, w, bias)
     return y if float_out is None else y.float()
 
 
