@@ -2,6 +2,7 @@
 // Fixed decays are lightning attention, decays and step sizes from a projection (u = softplus, a = exp(-exp(A_log) u)) are the state-space
 // duality of Mamba-2; one float state [D, Dv] per (request slot, head).
 #include "jl_common.h"
+#include <type_traits>
 
 // ---- token by token: decoded tokens, short portions, float activations ----------------------------------------------------------------------
 // The columns of S never interact, so a workgroup is ONE wavefront that owns 32 columns of one head's state (grid.y walks the head's
@@ -110,282 +111,356 @@ template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t 
 }
 
 // ---- long portions on the matrix cores (bfloat16): pieces side by side, 64 tokens at a time --------------------------------------------------
-// With L_t the running sum of log a inside a group of 64 tokens, the recurrence of the group is three products:
+// With L_t the running sum of log a inside a group of 64 tokens (kept to base 2), the recurrence of the group is three products:
 //   o_i = exp(L_i) S^T q_i + sum_{j <= i} (q_i . k_j) exp(L_i - L_j) u_j v_j,        S <- exp(L_end) S + sum_j k_j (exp(L_end - L_j) u_j v_j)^T.
 // A request's portion is cut into pieces (whole groups, except the last) that run side by side in three launches: every piece's own
 // contribution to the state from a zero state (CH_LOCAL, not for a request's last piece), scan_join_kernel (the state every piece starts
-// from), outputs (CH_OUT; the last piece leaves the request's final state in its slot).  A workgroup of four wavefronts owns 64 columns of one
-// head's state and walks its piece's groups with the state in accumulators; the next group's rows travel while the current one is multiplied.
+// from), outputs (CH_OUT; the last piece leaves the request's final state in its slot).
 // q, k and v enter the products as bfloat16 (what the projection, the convolution and their activation give); everything else stays float
 // and crosses the matrix cores as the sum of THREE bfloat16 numbers, which hold all 24 bits of it: the state, the decayed weights of a pair,
-// the decayed values.  Accumulator r of lane l of a 32 x 32 product is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32; lane l supplies row (A) or column
-// (B) l % 32 with depths 8 (l / 32) .. + 7 of a 16-deep step.
+// the decayed values.
+// A wavefront keeps 32 columns of one head's state, all rows of it, in accumulators and needs nothing from the others but the rows of q, k and v, which they share in
+// LDS: heads that read the same q and k sit in one workgroup (``heads`` of them, NW wavefronts).  Accumulator r of lane l of a 32 x 32 product is row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32; lane l supplies row (A) or column (B) l % 32 with eight depths of a 16-deep step, and which depths these are is free as
+// long as both operands agree.  So registers 8s .. 8s + 7 of an accumulator are handed on as an operand over the depths 16s + 4 (l / 32) + {0 .. 3, 8 .. 11}: the state as B of
+// S^T q, the weights of the pairs (formed turned, K Q^T) as A of the sum over values, without a trip through LDS.  q and k rows are read in that order as two 8-byte halves; k and v are
+// turned by ds_read_b64_tr_b16, and the values' operand, scaled and split in registers, is the state's update too.  One staging of rows and two barriers per group are left.
+// What bounds it: latency with two wavefronts per SIMD, all that their registers allow.  Per group and wavefront 1 900 vector instructions (splits, exponentials, silu) and 138 products of 32 cycles
+// take 12 000 cycles of issue; two side by side take 40 000.  Loads, stores, splits, weights: leaving out any one of them gives 5 to 15 % of the time.
+// Before, 64 columns of one head per workgroup met in LDS five times per group, one workgroup per CU.  us of the three launches, 4 x 2048 tokens, before / now: 16 heads of 128 x 128 with silu
+// 212 / 128 (their bytes at the rate of a large copy: 78), 32 heads of 128 x 64 over one key head 201 / 119; 2 x 300 of 8 heads 42 / 34, 40 x 64 of 16 heads 121 / 91.
 typedef __bf16 ch_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 ch_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 ch_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float ch_f32x4 __attribute__((ext_vector_type(4)));
+typedef float ch_f32x8 __attribute__((ext_vector_type(8)));
 typedef float ch_f32x16 __attribute__((ext_vector_type(16)));
-constexpr int CH_T = 64, CH_C = 64, CH_THREADS = 256, CH_TROW = CH_T, CH_PROW = CH_T + 8;
-constexpr int CH_TERMS = 3;
-constexpr int CH_OUT = 0, CH_LOCAL = 1;
+typedef short ch_s16x4 __attribute__((ext_vector_type(4)));
+typedef short ch_s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) ch_s16x4 ch_lds_s16x4;
+constexpr int CH_T = 64, CH_TERMS = 3, CH_OUT = 0, CH_LOCAL = 1;
 
-__device__ __forceinline__ ch_f32x16 ch_mfma(const bf16_t *a, const bf16_t *b, ch_f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const ch_bf16x8 *)a, *(const ch_bf16x8 *)b, c, 0, 0, 0);
-}
-__device__ __forceinline__ uint2 ch_round4(const float (&v)[4]) {
-    const ch_f32x4 f = {v[0], v[1], v[2], v[3]};
-    return __builtin_bit_cast(uint2, __builtin_convertvector(f, ch_bf16x4));
-}
-// four floats as the sum of CH_TERMS bfloat16 numbers each, term x of them at dst + x * stride
-__device__ __forceinline__ void ch_split4(float (&v)[4], bf16_t *dst, int stride) {
+// eight floats as the sum of CH_TERMS bfloat16 numbers each; what a term leaves over is exact, and one product of pairs with (-1, 0) or (0, -1) gives it without unpacking the term
+__device__ __forceinline__ void ch_split8(ch_f32x8 v, ch_bf16x8 (&part)[CH_TERMS]) {
+    uint32_t low = 0x0000bf80u, high = 0xbf800000u;                 // -1 in one half.  In registers: the compiler writes (-1, 0) as the inline constant -1.0, which the instruction reads as a float's bits
+    asm("" : "+s"(low), "+s"(high));
+    const ch_bf16x2 first = __builtin_bit_cast(ch_bf16x2, low), second = __builtin_bit_cast(ch_bf16x2, high);
 #pragma unroll
     for (int x = 0; x < CH_TERMS; ++x) {
-        const uint2 w = ch_round4(v);
-        *(uint2 *)(dst + x * stride) = w;
-        v[0] -= __uint_as_float(w.x << 16); v[1] -= __uint_as_float(w.x & 0xffff0000u); v[2] -= __uint_as_float(w.y << 16); v[3] -= __uint_as_float(w.y & 0xffff0000u);
+        part[x] = __builtin_convertvector(v, ch_bf16x8);
+        if (x + 1 == CH_TERMS) break;
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            const ch_bf16x2 p = {part[x][i], part[x][i + 1]};
+            v[i] = __builtin_amdgcn_fdot2_f32_bf16(p, first, v[i], false);
+            v[i + 1] = __builtin_amdgcn_fdot2_f32_bf16(p, second, v[i + 1], false);
+        }
     }
 }
 __device__ __forceinline__ uint2 ch_silu4(uint2 w) {
     float v[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] *= __builtin_amdgcn_rcpf(1.0f + __expf(-v[i]));          // rounded to bfloat16 next
-    return ch_round4(v);
-}
-// a row of 64 tokens of a transposed tile, eight tokens (16 bytes) at a time in an order that depends on the row: writers spread over rows and
-// readers of 16 consecutive rows meet different banks
-__device__ __forceinline__ int ch_tr(int row, int t) { return row * CH_TROW + ((((t >> 3) ^ (row >> 1) ^ (row >> 4)) & 7) << 3) + (t & 7); }
-// two tokens' four values, turned into four rows' two tokens
-__device__ __forceinline__ void ch_turn(bf16_t *dst, int row, int t, uint2 a, uint2 b) {
-    *(uint32_t *)(dst + ch_tr(row, t)) = (a.x & 0xffffu) | (b.x << 16);
-    *(uint32_t *)(dst + ch_tr(row + 1, t)) = (a.x >> 16) | (b.x & 0xffff0000u);
-    *(uint32_t *)(dst + ch_tr(row + 2, t)) = (a.y & 0xffffu) | (b.y << 16);
-    *(uint32_t *)(dst + ch_tr(row + 3, t)) = (a.y >> 16) | (b.y & 0xffff0000u);
+    const ch_f32x4 f = {v[0], v[1], v[2], v[3]};
+    return __builtin_bit_cast(uint2, __builtin_convertvector(f, ch_bf16x4));
 }
 
-static constexpr size_t ch_lds_bytes(int DP, bool out) {
-    return 2 * ((size_t)DP * CH_TROW + CH_C * CH_TROW + CH_TERMS * CH_T * CH_PROW + (out ? 2 * CH_T * (DP + 8) + CH_TERMS * CH_C * (DP + 8) : 0)) + 3 * CH_T * 4;
-}
+static constexpr size_t ch_lds_bytes(int DP, int NW, bool out) { return 2 * CH_T * ((out ? 2 : 1) * (size_t)(DP + 8) + 32 * NW + 16) + NW * 4 * CH_T * 4; }
 
-template <int DP, int MODE>
-__global__ __launch_bounds__(CH_THREADS) void scan_chunk_kernel(jl_scan_args a) {
+template <int DP, int NW, int MODE>
+__global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chunk_kernel(jl_scan_args a, int heads, int blocks) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int QROW = DP + 8, UD = DP / 4, KIT = 32 * UD / CH_THREADS, VIT = 2, NS = DP >= 64 ? DP / 64 : 1, PT = CH_T * CH_PROW, ST = CH_C * QROW;
     constexpr bool OUT = MODE == CH_OUT;
-    const int H = a.H, D = a.D, Dv = a.Dv;
-    const int piece = blockIdx.x, h = blockIdx.y, kh = h / (H / a.G), c_base = blockIdx.z * CH_C;
+    constexpr int THREADS = 64 * NW, QROW = DP + 8, VROW = 32 * NW + 16, UD = DP <= 32 ? 8 : DP <= 64 ? 16 : 32, UV = 8 * NW, NT = DP / 32;
+    constexpr int KSTEP = THREADS / UD, KIT = CH_T / KSTEP, VSTEP = THREADS / UV, VIT = CH_T / VSTEP;      // rows the workgroup takes at once, and how often
+    const int D = a.D, Dv = a.Dv, H = a.H;
+    const int sharing = H / a.G, per_key = (sharing + heads - 1) / heads;                    // heads that read the same q and k, and their workgroups
+    const int piece = blockIdx.x, kh = blockIdx.y / per_key, first = (blockIdx.y % per_key) * heads, h0 = kh * sharing + first;
+    if (sharing - first < heads) heads = sharing - first;
     const int row0 = a.chunk_rec[4 * piece], cnt = a.chunk_rec[4 * piece + 1], slot = a.chunk_rec[4 * piece + 2], last = a.chunk_rec[4 * piece + 3];
     if (cnt <= 0 || (!OUT && last)) return;
-    bf16_t *KT = (bf16_t *)smem;                                    // [DP][64] keys, turned
-    bf16_t *VT = KT + DP * CH_TROW;                                 // [64][64] values, turned
-    bf16_t *Ps = VT + CH_C * CH_TROW;                               // terms x [64][72] weights of the pairs; then the decayed values (turned)
-    bf16_t *Qs = Ps + CH_TERMS * PT, *Ks = Qs + CH_T * QROW;        // [64][DP + 8]
-    bf16_t *Ss = Ks + CH_T * QROW;                                  // terms x [64][DP + 8] the state, turned
-    float *Ls = (float *)(OUT ? Ss + CH_TERMS * ST : Qs);           // [64] running log decay
-    float *us = Ls + CH_T, *es = us + CH_T;                         // [64] u; [64] exp(L_end - L) u
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, w0 = wave & 1, w1 = wave >> 1;
+    bf16_t *Ks = (bf16_t *)smem, *Vs = Ks + CH_T * QROW, *Qs = Vs + CH_T * VROW;             // [64][DP + 8] keys, [64][32 NW + 16] values, [64][DP + 8] queries
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+    float *Ls = (float *)(Vs + CH_T * VROW + (OUT ? CH_T * QROW : 0)) + wave * 4 * CH_T;     // this wavefront's: [64] running log2 decay
+    float *us = Ls + CH_T, *es = us + CH_T, *el = es + CH_T;                                 // [64] u; exp(L_end - L) u; exp(L)
+    // the columns of wavefront w: block w % blocks (of those from blockIdx.z * NW on) of head h0 + w / blocks
+    auto head_of = [&](int w) { return h0 + w / blocks; };
+    auto col_of = [&](int w) { return 32 * ((int)blockIdx.z * NW + w % blocks); };
+    const int h = head_of(wave), c_base = col_of(wave), sc = c_base + l32;
+    const bool busy = wave < heads * blocks && c_base < Dv;
     const bf16_t *src = (const bf16_t *)a.src, *dtp = (const bf16_t *)a.dt;
     const bool fixed = a.decay != nullptr, act = a.act == JL_ACT_SILU;
-    const float glog = fixed ? fmaxf(logf(a.decay[h]), -1e30f) : 0.f, rate = fixed ? 0.f : -expf(a.A_log[h]), bias = fixed ? 0.f : a.dt_bias[h];
-    const float skip = a.skip ? a.skip[h] : 0.f;
+    const float glog = fixed && busy ? fmaxf(log2f(a.decay[h]), -1e30f) : 0.f, rate = fixed || !busy ? 0.f : (float)(-1.4426950408889634 * exp((double)a.A_log[h])), bias = fixed || !busy ? 0.f : a.dt_bias[h];
+    const float skip = a.skip && busy ? a.skip[h] : 0.f;
 
-    // the state: wavefront (w1, w0) has rows 32 (w1 + 2 x) .. + 31 of columns 32 w0 .. + 31
-    ch_f32x16 S[NS];
-    const int sc = c_base + 32 * w0 + l32;
-    const float *sp = a.scratch + ((int64_t)piece * H + h) * D * Dv;
+    ch_f32x16 S[NT];                                                // rows 32 x .. 32 x + 31 of the wavefront's columns
+    // registers become f(row, byte offset in the state, register): one address that moves on, not sixty-four in registers
+    auto each_state = [&](auto &&f) {
+        uint32_t off = (uint32_t)(4 * hi * Dv + sc) * 4;
 #pragma unroll
-    for (int x = 0; x < NS; ++x)
+        for (int x = 0; x < NT; ++x)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d = 32 * (w1 + 2 * x) + 8 * (r >> 2) + 4 * hi + (r & 3);
-            S[x][r] = (OUT && d < D && sc < Dv) ? sp[(int64_t)d * Dv + sc] : 0.f;
-        }
-    auto state_out = [&]() {                                        // the state in LDS
-#pragma unroll
-        for (int x = 0; x < NS; ++x) {
-            if (32 * (w1 + 2 * x) >= DP) continue;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                float v[4] = {S[x][4 * g], S[x][4 * g + 1], S[x][4 * g + 2], S[x][4 * g + 3]};
-                ch_split4(v, Ss + (32 * w0 + l32) * QROW + 32 * (w1 + 2 * x) + 8 * g + 4 * hi, ST);
+            for (int r = 0; r < 16; ++r) {
+                asm volatile("" : "+v"(off));
+                S[x][r] = f(32 * x + 8 * (r >> 2) + 4 * hi + (r & 3), off, S[x][r]);
+                off += ((r & 3) == 3 ? 5 : 1) * Dv * 4;
             }
-        }
     };
-    if (OUT) state_out();
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[x][r] = 0.f;
+    if (OUT && busy && sc < Dv) {
+        const char *sp = (const char *)(a.scratch + ((int64_t)piece * H + h) * D * Dv);
+        each_state([&](int d, uint32_t off, float) { return d < D ? *(const float *)(sp + off) : 0.f; });
+    }
 
-    uint2 rq[KIT][2], rk[KIT][2], rv[VIT][2];
+    uint2 rq[OUT ? KIT : 1], rk[KIT], rv[VIT];
     float rd = 0.f;
-    auto fetch = [&](int t0) {
+    // this thread's unit of four values: of q and k, of v (`w`: whose columns); what does not exist is staged as zeros
+    const int kt = tid / UD, kd = (tid % UD) * 4, vt = tid / UV, vc = (tid % UV) * 4, vw = vc >> 5, vcol = col_of(vw) + (vc & 31);
+    const bool k_in = kd < D, v_in = vw < heads * blocks && vcol < Dv;
+    const uint32_t k_off = k_in ? (uint32_t)(kt * a.ld + kd) : 0u, v_off = v_in ? (uint32_t)(vt * a.ld + (int64_t)(vw / blocks) * Dv + vcol) : 0u;
+    auto fetch = [&](int t0) {                                      // rows beyond the portion repeat its last and are cleared on the way to LDS
         const int nt = cnt - t0;
-        const bf16_t *base = src + (int64_t)(row0 + t0) * a.ld;
+        const bf16_t *base = src + (int64_t)(row0 + t0) * a.ld, *kb = base + a.k_col + kh * D, *qb = base + a.q_col + kh * D, *vb = base + a.v_col + (int64_t)h0 * Dv;
+        if (nt >= CH_T) {
 #pragma unroll
-        for (int it = 0; it < KIT; ++it) {
-            const int e = tid + it * CH_THREADS, p = e / UD, d = (e - p * UD) * 4;
+            for (int it = 0; it < KIT; ++it) {
+                rk[it] = *(const uint2 *)(kb + it * KSTEP * a.ld + k_off);
+                if (OUT) rq[OUT ? it : 0] = *(const uint2 *)(qb + it * KSTEP * a.ld + k_off);
+            }
 #pragma unroll
-            for (int y = 0; y < 2; ++y) {
-                rk[it][y] = make_uint2(0, 0);
-                if (OUT) rq[it][y] = make_uint2(0, 0);
-                if (2 * p + y < nt && d < D) {
-                    const bf16_t *row = base + (int64_t)(2 * p + y) * a.ld + kh * D + d;
-                    rk[it][y] = *(const uint2 *)(row + a.k_col);
-                    if (OUT) rq[it][y] = *(const uint2 *)(row + a.q_col);
+            for (int it = 0; it < VIT; ++it) rv[it] = *(const uint2 *)(vb + it * VSTEP * a.ld + v_off);
+        } else {
+#pragma unroll
+            for (int it = 0; it < KIT; ++it) {
+                const int t = kt + it * KSTEP < nt ? kt + it * KSTEP : nt - 1;
+                const int64_t o = k_in ? t * a.ld + kd : 0;
+                rk[it] = *(const uint2 *)(kb + o);
+                if (OUT) rq[OUT ? it : 0] = *(const uint2 *)(qb + o);
+            }
+#pragma unroll
+            for (int it = 0; it < VIT; ++it) {
+                const int t = vt + it * VSTEP < nt ? vt + it * VSTEP : nt - 1;
+                rv[it] = *(const uint2 *)(vb + (v_in ? t * a.ld + (int64_t)(vw / blocks) * Dv + vcol : 0));
+            }
+        }
+        if (!fixed && busy) rd = lane < nt ? ld_f(dtp + (int64_t)(row0 + t0 + lane) * a.dt_ld + a.dt_col + h) : 0.f;
+    };
+    // turned operands: column (or row) l % 32 of 32 columns from c on, tokens 16 s + 4 hi + {0 .. 3, 8 .. 11}
+    const int tr_row = 4 * hi + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    auto turned = [&](const bf16_t *tile, int row_len, int c, int s) {
+        ch_s16x4 half[2];
+#pragma unroll
+        for (int y = 0; y < 2; ++y) half[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ch_lds_s16x4 *)(tile + (16 * s + 8 * y + tr_row) * row_len + c + tr_col));
+        return __builtin_bit_cast(ch_bf16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    auto row_of = [&](const bf16_t *tile, int t, int s) {           // row t, depths 16 s + 4 hi + {0 .. 3, 8 .. 11}
+        const ch_bf16x4 x = *(const ch_bf16x4 *)(tile + t * QROW + 16 * s + 4 * hi), y = *(const ch_bf16x4 *)(tile + t * QROW + 16 * s + 8 + 4 * hi);
+        return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto acc8 = [](const ch_f32x16 &v, int s) {
+        ch_f32x8 f;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) f[x] = v[8 * s + x];
+        return f;
+    };
+    // The outputs of a group leave behind the next group's barrier and the loads of the one after it: loads and stores share a counter, and the wait for those loads, a group
+    // later, finds the stores done too.
+    ch_f32x16 o[OUT ? 2 : 1];                                       // outputs of queries 0 .. 31, 32 ..
+    auto outputs = [&](int t0, int n) {
+        const int64_t o_ld = (int64_t)H * Dv;
+        char *to = (char *)(a.out + (row0 + t0) * o_ld + (int64_t)h * Dv + c_base);
+        const uint32_t o_row = (uint32_t)o_ld * 4;                  // (64 rows of outputs lie within 32 bits)
+        uint32_t off = 4 * hi * o_row + 4 * l32;
+        auto store = [&](auto whole) {
+#pragma unroll
+            for (int y = 0; y < (OUT ? 2 : 0); ++y)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    asm volatile("" : "+v"(off));                   // one address that moves on, not thirty-two in registers
+                    if (decltype(whole)::value || 32 * y + 8 * (r >> 2) + 4 * hi + (r & 3) < n) *(float *)(to + off) = o[y][r];
+                    off += (r & 3) == 3 ? 5 * o_row : o_row;
                 }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < VIT; ++it) {
-            const int e = tid + it * CH_THREADS, p = e >> 4, c = c_base + (e & 15) * 4;
-#pragma unroll
-            for (int y = 0; y < 2; ++y) {
-                rv[it][y] = make_uint2(0, 0);
-                if (2 * p + y < nt && c < Dv) rv[it][y] = *(const uint2 *)(base + (int64_t)(2 * p + y) * a.ld + a.v_col + (int64_t)h * Dv + c);
-            }
-        }
-        if (wave == 0 && !fixed) rd = lane < nt ? ld_f(dtp + (int64_t)(row0 + t0 + lane) * a.dt_ld + a.dt_col + h) : 0.f;
+        };
+        if (!busy || sc >= Dv) return;
+        if (n >= CH_T) store(std::true_type());
+        else store(std::false_type());
     };
     fetch(0);
-    float l_all = 0.f;                                              // log decay of the piece up to here
+    float l_all = 0.f, end = 0.f, g = 1.f;                          // log2 of the piece's decay up to here, of the group's; the group's decay (fixed decays: the same for whole groups)
     for (int t0 = 0; t0 < cnt; t0 += CH_T) {
         const int nt = cnt - t0 < CH_T ? cnt - t0 : CH_T;
-        __syncthreads();                                            // the group before has been read; the state is in LDS
+        __syncthreads();                                            // the group before has been read
+        auto stage = [&](auto silu) {                               // silu(0) = 0
+            auto put = [&](bf16_t *to, uint2 v, bool in) {
+                if (!in) v = make_uint2(0, 0);
+                *(uint2 *)to = decltype(silu)::value ? ch_silu4(v) : v;
+            };
+            if (DP == 4 * UD || kd < DP)
 #pragma unroll
-        for (int it = 0; it < KIT; ++it) {
-            const int e = tid + it * CH_THREADS, p = e / UD, d = (e - p * UD) * 4;
-            if (act) {
-#pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    rk[it][y] = ch_silu4(rk[it][y]);                // silu(0) = 0: rows and columns beyond the tile stay zero
-                    if (OUT) rq[it][y] = ch_silu4(rq[it][y]);
+                for (int it = 0; it < KIT; ++it) {
+                    const int t = kt + it * KSTEP;
+                    put(Ks + t * QROW + kd, rk[it], k_in && t < nt);
+                    if (OUT) put(Qs + t * QROW + kd, rq[OUT ? it : 0], k_in && t < nt);
                 }
-            }
-            ch_turn(KT, d, 2 * p, rk[it][0], rk[it][1]);
-            if (OUT) {
 #pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    *(uint2 *)(Ks + (2 * p + y) * QROW + d) = rk[it][y];
-                    *(uint2 *)(Qs + (2 * p + y) * QROW + d) = rq[it][y];
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < VIT; ++it) {
-            const int e = tid + it * CH_THREADS, p = e >> 4, c = (e & 15) * 4;
-            if (act) {
-                rv[it][0] = ch_silu4(rv[it][0]);
-                rv[it][1] = ch_silu4(rv[it][1]);
-            }
-            ch_turn(VT, c, 2 * p, rv[it][0], rv[it][1]);
-        }
-        if (wave == 0) {                                            // a token per lane: step size, running log decay
+            for (int it = 0; it < VIT; ++it) put(Vs + (vt + it * VSTEP) * VROW + vc, rv[it], v_in && vt + it * VSTEP < nt);
+        };
+        if (act) stage(std::true_type());
+        else stage(std::false_type());
+        if (busy && (!fixed || t0 == 0 || nt < CH_T)) {             // a token per lane: step size, running log2 decay
             const bool in = lane < nt;
             const float u = !in ? 0.f : fixed ? 1.0f : softplus_f(rd + bias);
-            float l = !in ? 0.f : fixed ? glog : rate * u;
+            double l = !in ? 0. : fixed ? (double)glog : (double)rate * u;      // far into a group with strong decays a sum in float would be off by more than the tokens' own decays
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
-                const float y = __shfl_up(l, off, 64);
+                const double y = __shfl_up(l, off, 64);
                 if (lane >= off) l += y;
             }
-            const float end = __shfl(l, 63, 64);
-            Ls[lane] = l;
-            us[lane] = u;
-            es[lane] = expf(end - l) * u;
+            const double whole = __shfl(l, 63, 64);
+            end = (float)whole;
+            es[lane] = exp2f((float)(whole - l)) * u;
+            if (OUT) {
+                Ls[lane] = (float)l;
+                us[lane] = u;
+                el[lane] = exp2f((float)l);
+            }
+            g = exp2f(end);
         }
+        l_all += end;
         __syncthreads();
         if (t0 + CH_T < cnt) fetch(t0 + CH_T);                      // in flight while this group is multiplied
-        const float l_end = Ls[CH_T - 1];
-        l_all += l_end;
-        if (OUT) {
-            if (w0 <= w1) {                                         // scores, turned: keys 32 w0 .. of queries 32 w1 ..; keys behind every query are left out
-                ch_f32x16 s;
+        if (OUT && t0 > 0) outputs(t0 - CH_T, CH_T);
+        ch_bf16x8 vf[CH_T / 16];
+        const bool more = !OUT || last || t0 + CH_T < cnt;          // else nobody reads this piece's final state: the next piece has its own
+        if (busy) {
+            if (OUT) {
+                // A step's operands (rows from LDS, splits) are made while the step before is multiplied, and no sooner (sched_barrier): all at once they do not fit the registers.
+                constexpr int KS = DP / 16;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = 0.f;
+                for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = 0.f;
+                {
+                    ch_bf16x8 q[2][2], part[2][CH_TERMS];
+                    auto operands = [&](int s) {
+                        q[s & 1][0] = row_of(Qs, l32, s);
+                        q[s & 1][1] = row_of(Qs, 32 + l32, s);
+                        ch_split8(acc8(S[s >> 1], s & 1), part[s & 1]);
+                    };
+                    operands(0);
 #pragma unroll
-                for (int kk = 0; kk < DP; kk += 16) s = ch_mfma(Ks + (32 * w0 + l32) * QROW + kk + 8 * hi, Qs + (32 * w1 + l32) * QROW + kk + 8 * hi, s);
-                const int i = 32 * w1 + l32;
-                const float li = Ls[i];
+                    for (int s = 0; s < KS; ++s) {
+                        if (s + 1 < KS) operands(s + 1);
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int j0 = 32 * w0 + 8 * g + 4 * hi;
-                    float v[4];
+                        for (int x = 0; x < CH_TERMS; ++x)
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = j0 + x <= i ? s[4 * g + x] * (__expf(li - Ls[j0 + x]) * us[j0 + x]) : 0.f;
-                    ch_split4(v, Ps + i * CH_PROW + j0, PT);
-                }
-            }
-            __syncthreads();
-            {   // outputs: queries 32 w1 .., columns 32 w0 ..
-                ch_f32x16 o;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[r] = 0.f;
-                const int ai = (32 * w1 + l32) * QROW + 8 * hi, bi = (32 * w0 + l32) * QROW + 8 * hi;
-#pragma unroll
-                for (int kk = 0; kk < DP; kk += 16) {
-#pragma unroll
-                    for (int x = 0; x < CH_TERMS; ++x) o = ch_mfma(Qs + ai + kk, Ss + x * ST + bi + kk, o);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[r] *= __expf(Ls[32 * w1 + 8 * (r >> 2) + 4 * hi + (r & 3)]);
-#pragma unroll
-                for (int kk = 0; kk < CH_T; kk += 16) {
-                    if (kk >= 32 && w1 == 0) continue;              // no key of the second half is visible to the first half's queries
-                    const bf16_t *vp = VT + ch_tr(32 * w0 + l32, kk + 8 * hi);
-#pragma unroll
-                    for (int x = 0; x < CH_TERMS; ++x) o = ch_mfma(Ps + x * PT + (32 * w1 + l32) * CH_PROW + kk + 8 * hi, vp, o);
-                }
-                if (sc < Dv) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int i = 32 * w1 + 8 * (r >> 2) + 4 * hi + (r & 3);
-                        if (i < nt) {
-                            float v = o[r];
-                            if (a.skip) v += skip * ld_f(VT + ch_tr(32 * w0 + l32, i));
-                            a.out[(int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + (int64_t)h * Dv + sc] = v;
-                        }
+                            for (int y = 0; y < 2; ++y) o[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[s & 1][y], part[s & 1][x], o[y], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
+                ch_f32x16 p[3];                                     // turned weights: keys 0 .. of queries 0 .., keys 0 .. of queries 32 .., keys 32 .. of queries 32 ..
+#pragma unroll
+                for (int r = 0; r < 16; ++r) p[0][r] = p[1][r] = p[2][r] = 0.f;
+                {
+                    ch_bf16x8 f[2][4];
+                    auto operands = [&](int s) {
+                        f[s & 1][0] = row_of(Qs, l32, s); f[s & 1][1] = row_of(Qs, 32 + l32, s); f[s & 1][2] = row_of(Ks, l32, s); f[s & 1][3] = row_of(Ks, 32 + l32, s);
+                    };
+                    operands(0);
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        if (s + 1 < KS) operands(s + 1);
+                        p[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s & 1][2], f[s & 1][0], p[0], 0, 0, 0);
+                        p[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s & 1][2], f[s & 1][1], p[1], 0, 0, 0);
+                        p[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s & 1][3], f[s & 1][1], p[2], 0, 0, 0);
+                        if (s < 2) {                                // beside the products: what S^T q is worth now
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                const ch_f32x4 e4 = *(const ch_f32x4 *)(el + 32 * s + 8 * x + 4 * hi);
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) o[s][4 * x + i] *= e4[i];
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < CH_T / 16; ++s) vf[s] = turned(Vs, VROW, 32 * wave, s);
+                {
+                    ch_bf16x8 part[2][CH_TERMS];
+                    const float li[2] = {Ls[l32], Ls[32 + l32]};
+                    int ahead = l32 - 4 * hi;                       // the query's place less the lane's first key's, in a block on the diagonal
+                    asm volatile("" : "+v"(ahead));                 // compared where it is used: sixteen masks kept would not fit the scalar registers
+                    auto weights = [&](int n) {                     // half n % 2 of block n / 2: keys 32 kb .., queries 32 qb ..
+                        const int b = n >> 1, s = n & 1, kb = b == 2, qb = b != 0;
+                        ch_f32x8 w = acc8(p[b], s);
+#pragma unroll
+                        for (int x = 0; x < 2; ++x) {
+                            const int j0 = 32 * kb + 16 * s + 8 * x + 4 * hi;
+                            const ch_f32x4 lj = *(const ch_f32x4 *)(Ls + j0), uj = *(const ch_f32x4 *)(us + j0);
+#pragma unroll
+                            for (int y = 0; y < 4; ++y) {
+                                const float f = w[4 * x + y] * (__builtin_amdgcn_exp2f(li[qb] - lj[y]) * uj[y]);
+                                w[4 * x + y] = b == 1 || 16 * s + 8 * x + y <= ahead ? f : 0.f;
+                            }
+                        }
+                        ch_split8(w, part[n & 1]);
+                    };
+                    weights(0);
+#pragma unroll
+                    for (int n = 0; n < 6; ++n) {
+                        if (n < 5) weights(n + 1);
+#pragma unroll
+                        for (int x = 0; x < CH_TERMS; ++x) o[n >= 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(part[n & 1][x], vf[2 * (n >= 4) + (n & 1)], o[n >= 2], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                if (a.skip)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[y][r] += skip * (float)vf[2 * y + (r >> 3)][r & 7];
+            } else {
+#pragma unroll
+                for (int s = 0; s < CH_T / 16; ++s) vf[s] = turned(Vs, VROW, 32 * wave, s);
             }
-            if (t0 + CH_T >= cnt && !last) break;                   // nobody reads this piece's final state: the next piece has its own
-            __syncthreads();
         }
-        {   // decayed values in the weights' place: column tid / 4, sixteen tokens
-            const int c = tid >> 2, tq = (tid & 3) * 16;
+        if (busy && more) {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int t = tq + 4 * x, o = ch_tr(c, t);
-                float v[4];
-                ld4_f(VT + o, v);
-#pragma unroll
-                for (int y = 0; y < 4; ++y) v[y] *= es[t + y];
-                ch_split4(v, Ps + o, PT);
-            }
-        }
-        __syncthreads();
-        {
-            const float g = expf(l_end);
-#pragma unroll
-            for (int x = 0; x < NS; ++x) {
-                if (32 * (w1 + 2 * x) >= DP) continue;
+            for (int x = 0; x < NT; ++x)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) S[x][r] *= g;
+            ch_bf16x8 part[2][CH_TERMS], kf[2][NT];
+            auto operands = [&](int s) {
+                ch_f32x8 w = __builtin_convertvector(vf[s], ch_f32x8);
 #pragma unroll
-                for (int kk = 0; kk < CH_T; kk += 16) {
-                    const bf16_t *kp = KT + ch_tr(32 * (w1 + 2 * x) + l32, kk + 8 * hi);
-                    const int o = ch_tr(32 * w0 + l32, kk + 8 * hi);
+                for (int x = 0; x < 2; ++x) {
+                    const ch_f32x4 e4 = *(const ch_f32x4 *)(es + 16 * s + 8 * x + 4 * hi);
 #pragma unroll
-                    for (int y = 0; y < CH_TERMS; ++y) S[x] = ch_mfma(kp, Ps + y * PT + o, S[x]);
+                    for (int y = 0; y < 4; ++y) w[4 * x + y] *= e4[y];
                 }
+                ch_split8(w, part[s & 1]);
+#pragma unroll
+                for (int x = 0; x < NT; ++x) kf[s & 1][x] = turned(Ks, QROW, 32 * x, s);
+            };
+            operands(0);
+#pragma unroll
+            for (int s = 0; s < CH_T / 16; ++s) {
+                if (s + 1 < CH_T / 16) operands(s + 1);
+#pragma unroll
+                for (int y = 0; y < CH_TERMS; ++y)
+#pragma unroll
+                    for (int x = 0; x < NT; ++x) S[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s & 1][x], part[s & 1][y], S[x], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (OUT && t0 + CH_T < cnt) state_out();                // its readers of this group are two barriers behind
         }
     }
-    if (OUT && !last) return;
-    float *dst = OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : a.scratch + ((int64_t)piece * H + h) * D * Dv;
-#pragma unroll
-    for (int x = 0; x < NS; ++x)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d = 32 * (w1 + 2 * x) + 8 * (r >> 2) + 4 * hi + (r & 3);
-            if (32 * (w1 + 2 * x) < DP && d < D && sc < Dv) dst[(int64_t)d * Dv + sc] = S[x][r];
-        }
-    if (!OUT && tid == 0 && blockIdx.z == 0) a.scratch[(int64_t)a.chunks * H * D * Dv + (int64_t)piece * H + h] = l_all;
+    if (OUT) outputs((cnt - 1) / CH_T * CH_T, cnt - (cnt - 1) / CH_T * CH_T);
+    if (!busy || (OUT && !last)) return;
+    char *dst = (char *)(OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : a.scratch + ((int64_t)piece * H + h) * D * Dv);
+    if (sc < Dv) each_state([&](int d, uint32_t off, float v) { if (d < D) *(float *)(dst + off) = v; return v; });
+    if (!OUT && lane == 0 && c_base == 0) a.scratch[(int64_t)a.chunks * H * D * Dv + (int64_t)piece * H + h] = l_all;
 }
 
 // The state every piece starts from, in place of its own contribution: S = the request's state (zero at position 0); for each piece in order
@@ -402,25 +477,28 @@ __global__ __launch_bounds__(256) void scan_join_kernel(jl_scan_args a) {
         for (int p = 0; p < np; ++p, lp += a.H * ddv) {
             const float next = p + 2 < np ? lp[a.H * ddv] : 0.f;    // on its way while this piece is joined
             *lp = S;
-            if (p + 1 < np) S = expf(ll[(int64_t)(p0 + p) * a.H + h]) * S + local;
+            if (p + 1 < np) S = exp2f(ll[(int64_t)(p0 + p) * a.H + h]) * S + local;
             local = next;
         }
     }
 }
 
-template <int DP> static int scan_chunk_launch(const jl_scan_args &a, hipStream_t st) {
-    const dim3 grid((unsigned)a.chunks, (unsigned)a.H, (unsigned)((a.Dv + CH_C - 1) / CH_C));
-    auto out = scan_chunk_kernel<DP, CH_OUT>;
-    constexpr size_t lds = ch_lds_bytes(DP, true);
-    if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)out, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_linear_scan: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    }
-    if (a.chunks > a.B) scan_chunk_kernel<DP, CH_LOCAL><<<grid, CH_THREADS, ch_lds_bytes(DP, false), st>>>(a);
+template <int DP, int NW> static int scan_chunk_launch(const jl_scan_args &a, int heads, int blocks, hipStream_t st) {
+    const int per_head = (a.Dv + 31) / 32;
+    const dim3 grid((unsigned)a.chunks, (unsigned)(a.G * ((a.H / a.G + heads - 1) / heads)), (unsigned)((per_head + NW - 1) / NW));
+    static_assert(ch_lds_bytes(DP, NW, true) <= 64 * 1024, "static limit of a launch");
+    if (a.chunks > a.B) scan_chunk_kernel<DP, NW, CH_LOCAL><<<grid, 64 * NW, ch_lds_bytes(DP, NW, false), st>>>(a, heads, blocks);
     const int64_t ddv = (int64_t)a.D * a.Dv;
     scan_join_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64)), 256, 0, st>>>(a);
-    out<<<grid, CH_THREADS, lds, st>>>(a);
+    scan_chunk_kernel<DP, NW, CH_OUT><<<grid, 64 * NW, ch_lds_bytes(DP, NW, true), st>>>(a, heads, blocks);
     return jl_check_launch("scan_chunk_kernel");
+}
+// Four wavefronts per workgroup where a head's columns or the heads that read the same q and k fill more than two of them; else two.
+template <int DP> static int scan_chunk_launch(const jl_scan_args &a, hipStream_t st) {
+    const int per_head = (a.Dv + 31) / 32, sharing = a.H / a.G;
+    const int heads = per_head >= 3 || sharing == 1 ? 1 : per_head == 1 && sharing >= 3 ? 4 : 2;
+    if (heads * per_head > 2) return scan_chunk_launch<DP, 4>(a, heads, per_head < 4 ? per_head : 4, st);
+    return scan_chunk_launch<DP, 2>(a, heads, per_head, st);
 }
 
 extern "C" int jl_linear_scan_chunked_ok(int dtype, int32_t D, int32_t Dv) { return dtype == JL_BF16 && D > 0 && D <= 128 && D % 4 == 0 && Dv > 0 && Dv % 4 == 0; }
@@ -442,6 +520,7 @@ extern "C" int jl_linear_scan(const jl_scan_args *ap, void *stream) {
             return jl_fail(JL_E_INVALID, "jl_linear_scan: pieces take bfloat16, D a multiple of four up to 128, Dv, columns and rows in multiples of four");
         if (a.D <= 32) return scan_chunk_launch<32>(a, st);
         if (a.D <= 64) return scan_chunk_launch<64>(a, st);
+        if (a.D <= 96) return scan_chunk_launch<96>(a, st);
         return scan_chunk_launch<128>(a, st);
     }
     JL_DISPATCH(a.dtype, return scan_launch<T>(a, st));

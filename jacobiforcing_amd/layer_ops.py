@@ -30,12 +30,12 @@ NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, a
                                       # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
 NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
                                       # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
-BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
+BLOCK_WORKGROUPS = 384               # a draft block's attention: wavefronts of 32 columns to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
-RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at
+RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches, 4 x 2048 of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
-SCAN_PIECES_FROM, SCAN_WORKGROUPS = 32, 512     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; workgroups to aim at
+SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches, 4 x 2048 of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
 DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (alone in its step; else delta_chunks_from.  us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
 DELTA_SCRATCH_FLOATS = 256 << 20     # scratch of those chunks at most (1 GiB: more heads than it holds take turns), as long as it holds one key head's
@@ -1302,8 +1302,8 @@ def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatc
                    act=int(act), B=batch.B, H=H, G=G, D=D, Dv=Dv)
     if (max(batch.counts) >= SCAN_PIECES_FROM and not os.environ.get("JL_SCAN_NO_PIECES") and a.ld % 4 == 0 and all(c % 4 == 0 for c in cols) and    # A/B switch for measurements
             N.layers().jl_linear_scan_chunked_ok(a.dtype, D, Dv)):
-        # long portions: pieces side by side on the matrix cores, as many as fill the chip, each at least one group of 64 tokens
-        size = 64 * max(1, min(8, n * H * -(-Dv // 64) // (SCAN_WORKGROUPS * 64)))
+        # long portions: pieces side by side on the matrix cores, as many as fill the chip with two wavefronts per SIMD, each at least one group of 64 tokens
+        size = 64 * max(1, min(8, n * H * -(-Dv // 32) // (SCAN_WAVES * 64)))
         rec, req = batch.pieces(size)
         scratch = torch.empty((rec.shape[0] * H * (D * Dv + 1),), dtype=torch.float32, device=src.device)
         a.chunk_rec, a.req, a.scratch, a.chunks = p(rec), p(req), p(scratch), rec.shape[0]

@@ -1,0 +1,48 @@
+"""The linear recurrence in pieces on the matrix cores: how columns and heads are dealt out to wavefronts (one to four blocks of 32 columns, heads that share q and k in one
+workgroup, the last of them incomplete), at the edges of groups of 64 tokens and of widths, against the recurrence in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("H,G,D,Dv,counts", [
+    (3, 3, 128, 128, [64, 1, 200]), (2, 2, 96, 96, [65, 63]), (5, 5, 72, 64, [129, 40]), (9, 1, 128, 64, [130, 33]), (6, 2, 64, 32, [64, 128]), (5, 1, 32, 20, [100, 64, 7]),
+    (2, 1, 128, 160, [320]), (1, 1, 4, 4, [191, 2]), (10, 2, 100, 12, [66, 62]),
+])
+def test_columns_and_heads(monkeypatch, H, G, D, Dv, counts, fixed):
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "SCAN_WAVES", 1)                 # pieces as long as they get: several groups per piece, and ...
+    g = torch.Generator(device="cuda").manual_seed(H * 100 + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    B, N, starts = len(counts), sum(counts), [0, 3, 0][:len(counts)]
+    x = rnd(N, H * Dv + 2 * G * D + 4).bfloat16()
+    cols = (H * Dv + G * D + 4, H * Dv, 0)
+    kw = dict(decay=torch.rand(H, generator=g, device="cuda")) if fixed else dict(dt=rnd(N, H).bfloat16(), a_log=rnd(H), dt_bias=rnd(H), skip=rnd(H))
+    state = rnd(B, H, D, Dv)
+    for b, s in enumerate(starts):
+        if s == 0:
+            state[b] = float("nan")
+    pages = [list(range(8 * b, 8 * b + 8)) for b in range(B)]
+    for waves in (1, 1 << 20):                               # ... of one group each
+        monkeypatch.setattr(LO, "SCAN_WAVES", waves)
+        batch, st = LO.RaggedBatch.build(counts, starts, list(range(B)), pages, 64, "cuda"), state.clone()
+        got = LO.linear_scan(x, cols, batch, H, G, D, Dv, st, **kw)
+        assert any(isinstance(k, tuple) and k[0] == "pieces" for k in batch._tiles), "the form in pieces did not run"
+        r0, xd = 0, x.double()
+        d = {k: v.double() for k, v in kw.items()}
+        for b, (n, s) in enumerate(zip(counts, starts)):
+            rows = xd[r0:r0 + n]
+            q, k = (rows[:, c:c + G * D].view(n, G, D).repeat_interleave(H // G, 1) for c in cols[:2])
+            v = rows[:, :H * Dv].view(n, H, Dv)
+            S = state[b].double() if s else torch.zeros(H, D, Dv, dtype=torch.float64, device="cuda")
+            for t in range(n):
+                u = torch.ones(H, dtype=torch.float64, device="cuda") if fixed else torch.nn.functional.softplus(d["dt"][r0 + t] + d["dt_bias"])
+                a = d["decay"] if fixed else torch.exp(-torch.exp(d["a_log"]) * u)
+                S = a.view(H, 1, 1) * S + k[t].unsqueeze(2) * (u.view(H, 1) * v[t]).unsqueeze(1)
+                o = (S * q[t].unsqueeze(2)).sum(1) + (0 if fixed else d["skip"].view(H, 1) * v[t])
+                # 24-bit terms, and weights whose two log decays (up to 2 ** 9 here, rounded to 2 ** -16 each) are off by 2e-5 at most where they are that large
+                assert float((got[r0 + t].double().view(H, Dv) - o).norm() / o.norm().clamp_min(1e-3 * D ** 0.5)) < 2e-5, (b, t)
+            assert float((st[b].double() - S).norm() / S.norm()) < 2e-5
+            r0 += n
