@@ -438,6 +438,8 @@ JL_API int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, i
                         int32_t *tile_expert, int32_t *tile_row0, int32_t max_tiles, void *stream);
 /* tile_rows for a step of `rows` (token, choice) rows over E experts of width ff behind a stream of width W: 32, 64 or (bfloat16) 128 */
 JL_API int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff);
+/* 1: bfloat16 tiles of 128 rows are better grouped in pairs (tile_rows 256 for jl_moe_group and the products) */
+JL_API int jl_moe_tile_pairs(int64_t rows, int32_t E, int32_t W, int32_t ff, int32_t gated);
 
 /* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].
  *   mode 0 (up):   in(r) = perm[r] / top;  out[r, :] = relu(C)^2, stored in `dtype` ([N*top, n_out], sorted order)

@@ -348,12 +348,13 @@ _LAYER_SIGNATURES = {
     "jl_moe_route": (C.c_int, [_vp, _vp, _i64, _i32, _i32, _f32, _vp, _vp, _i32, _f32, _vp]),
     "jl_moe_group": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _vp]),
     "jl_moe_tile_rows": (C.c_int, [C.c_int, _i64, _i32, _i32, _i32]),
+    "jl_moe_tile_pairs": (C.c_int, [_i64, _i32, _i32, _i32, _i32]),
     "jl_moe_gemm": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
     "jl_moe_gemm_gated": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _vp, _vp]),
 }
 LAYER_SYMBOLS = tuple(_LAYER_SIGNATURES)
 # which library a symbol lives in (jacobiforcing_amd/_build.py: LAYER_GROUPS); both carry their own jl_version / jl_last_error
-_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_gemm", "jl_moe_gemm_gated")
+_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_gemm", "jl_moe_gemm_gated")
 
 
 class _LayerLibs:

@@ -102,8 +102,9 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 
 // 16 bytes per lane from base + off into LDS at `lds` + 16 * lane (`base`, `lds` the same for the wavefront).  The compiler does not count these loads: the caller waits for vmcnt
 // before the barrier that publishes them, and before the workgroup ends
+// (s_nop 3: five states lie between a vector instruction that wrote `base` and the load, which the compiler does not see to in front of assembly)
 __device__ __forceinline__ void jl_load_lds(const char *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0", "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "m0", "memory");
 }
 // the same from an address per lane
 __device__ __forceinline__ void jl_load_lds_far(const char *from, uint32_t lds) {

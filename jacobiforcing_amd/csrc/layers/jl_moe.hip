@@ -4,7 +4,6 @@
 #include "jl_common.h"
 #include <stdlib.h>
 #include <type_traits>
-
 constexpr int MOE_MAX_E = 4096;   // experts (router outputs) at most
 struct MoeAct { int kind; float limit, alpha, shift; };       // the gated unit of JL_MOE_UP_GATED (jl_gated_act's kinds)
 
@@ -188,6 +187,16 @@ extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, i
     return rows >= (int64_t)48 * E && blocks(64, ff, 128) + blocks(64, W, 256) >= 512 ? 64 : 32;
 }
 
+// Tiles of 128 rows in pairs: the way up in tiles of 256 x 256 (moe_big_kernel), one workgroup per CU, so from two and a half rounds of the chip's CUs on; the way down walks the pairs' halves.
+// us, experts alone, gated, tiles of 128 / 256: 8192 tokens x 4 of 32 (2048 x 1024; 1152 workgroups) 656 / 598, 6554 x 4 (944) 546 / 509, 4096 x 4 (640) 372 / 355, 8192 x 4 of 24 (1536 x 768; 840)
+// 403 / 382; below: 8192 x 2 of 8 (1024 x 1024; 544) 188 / 190, 8192 x 3 of 9 (1088 x 704; 600) 216 / 221.
+// moe_big_kernel takes depths in whole stages and rows within 32 bits (gathered ones are at most as many as sorted ones).
+static bool moe_big_sizes(int64_t K, int64_t rows) { return K % 64 == 0 && rows * K * 2 <= UINT32_MAX; }
+extern "C" int jl_moe_tile_pairs(int64_t rows, int32_t E, int32_t W, int32_t ff, int32_t gated) {
+    const int cols = gated ? 128 : 256;
+    return E > 0 && rows >= (int64_t)256 * E && (rows / 256 + E / 2) * ((ff + cols - 1) / cols) >= 640 && moe_big_sizes(W, rows + (int64_t)256 * E);
+}
+
 extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, int32_t tile_rows, int32_t *perm, int32_t *offsets,
                             int32_t *tile_expert, int32_t *tile_row0, int32_t max_tiles, void *stream) {
     if (N <= 0) return JL_OK;
@@ -277,15 +286,16 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
 // ---- grouped product on the matrix cores -------------------------------------------------------------------------------------------------
 // A tile of TM rows of one expert by WR of its weight rows, both K-major, walked in stages of TKU 16-byte units per row (8 bfloat16 or 4 floats each)
 // through two LDS buffers: the next stage's units travel from memory while this one is multiplied, one barrier per stage.  NW wavefronts (two over the
-// rows when TM is 128) hold 32 x 32 accumulators; the weights are the A operand, the rows the B operand, so that a lane ends with four neighbouring
-// output columns of ONE row and stores them together.  A lane's operand is one 16-byte unit: in bfloat16 the eight depths 8 (lane / 32) .. of
+// rows when TM is 128) hold 32 x 32 accumulators; the rows are the A operand, the weights the B operand, so that a lane ends with sixteen rows of ONE output
+// column and 32 lanes store neighbouring ones (moe_store).  A lane's operand is one 16-byte unit: in bfloat16 the eight depths 8 (lane / 32) .. of
 // v_mfma_f32_32x32x16_bf16; in float four v_mfma_f32_32x32x2_f32, one for each of its floats (the depths meet in the order 0, 4, 1, 5, ..: a sum of
 // products rounded one by one, as a chain of multiply-adds is).  Units of a row are permuted so that 16 neighbouring rows meet different banks.
 // GATED: the WR weight rows are WR / 2 of the gate and the WR / 2 of the linear branch that belong to them (rows n_out further on); both products
 // of a column end in the same lane, which stores the gated unit.
 // TM = 128 (an expert has about a hundred rows or more) is bound by the matrix cores and LDS: 128 x 256 reads 48 KB of LDS per 64 products.  Rows go from memory straight into LDS
 // (16 bytes per lane, every lane fetching the unit that the permutation puts into its place), one stage ahead: no registers and no LDS writes for them, so that three workgroups fit a
-// CU and cover each other's barriers (through registers, two of them: gated product at 8192 x 4 of 32 experts of 2048 x 1024 406 -> 363 us, the way down 290 -> 252).
+// CU and cover each other's barriers (through registers, two of them: gated product at 8192 x 4 of 32 experts of 2048 x 1024 406 -> 363 us, the way down 290 -> 252).  More stages ahead in fewer
+// workgroups change nothing; without their loads the two products take 238 and 160 us, without their products 335 and 200, so where rows are many the gated one goes in larger tiles (below).
 // Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading
 // the weights: single wavefronts, many per CU, 12 KB on the way each, in registers.
 // Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from a base (of the tile where its rows lie together; FAR: rows gathered from more than
@@ -297,10 +307,12 @@ struct MoeMM {
     const int32_t *perm, *offsets, *tile_expert, *tile_row0;
     const float *weights;
     void *out;
-    int mode, K, n_out, top, E, col_blocks, max_tiles;
+    int mode, K, n_out, top, E, col_blocks, max_tiles, parts;       // parts: of TM rows, that a tile of the list is walked in
     MoeAct act;
 };
 typedef __bf16 mm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 mm_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float mm_f32x2 __attribute__((ext_vector_type(2)));
 typedef float mm_f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t mm_u32x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct mm_type;
@@ -320,17 +332,67 @@ template <> struct mm_type<float> {
     }
 };
 
+// What a wavefront's products leave: XT x NT tiles of 32 rows (from row_of(x) of the tile's) by 32 columns (from col_of(t)); a lane has sixteen rows of column lane % 32.  A store instruction writes
+// 32 neighbouring columns of two rows (float), or of four rows once neighbouring lanes have exchanged a value (bfloat16): whole lines or their halves.  (Four neighbouring columns of one row
+// per lane, 32 rows per instruction: the experts of 8192 x 4 of 32 of 2048 x 1024 took 687 us instead of 647, 8192 x 4 of 16 of 1024 x 512 174 instead of 163.)
+template <typename T, int XT, int NT, bool GATED, bool DOWN, typename Down, typename Rows, typename Cols>
+__device__ __forceinline__ void moe_store(const MoeMM &a, const mm_f32x16 (&acc)[XT][NT], int r0, int nr, int n0, Down down, Rows row_of, Cols col_of, int lane) {
+    constexpr int OT = GATED ? NT / 2 : NT;
+    const int n_out = a.n_out, l32 = lane & 31, hi = lane >> 5;
+    const bool pairs = n_out % 2 == 0, odd = lane & 1;
+#pragma unroll
+    for (int x = 0; x < XT; ++x)
+#pragma unroll
+        for (int t = 0; t < OT; ++t) {
+            const int n = n0 + col_of(t) + l32;
+            if (n - l32 >= n_out) continue;                         // the whole wavefront
+            const bool in = n < n_out;                              // both lanes of a pair, or neither, where columns come in pairs; all lanes take part in what crosses them
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const int m = row_of(x) + 8 * (r >> 2) + 4 * hi + (r & 3);
+                float v[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float c = acc[x][t][r + i];
+                    if (GATED) v[i] = gated_unit_f<sizeof(T) == 2>(c, acc[x][t + (GATED ? OT : 0)][r + i], a.act.kind, a.act.limit, a.act.alpha, a.act.shift);
+                    else if (a.mode == 0) { const float q = fmaxf(c, 0.f); v[i] = q * q; }
+                    else v[i] = c;
+                }
+                if (DOWN && a.mode == 1) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        int p;
+                        float w;
+                        down(x, 8 * (r >> 2) + 4 * hi + (r & 3) + i, p, w);
+                        if (in && m + i < nr) ((float *)a.out)[(int64_t)p * n_out + n] = v[i] * w;
+                    }
+                } else if (sizeof(T) == 2 && pairs) {
+                    const float other = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(odd ? v[0] : v[1]), 0xB1, 0xF, 0xF, true));      // quad_perm [1, 0, 3, 2]
+                    const mm_f32x2 both = {odd ? other : v[0], odd ? v[1] : other};
+                    if (in && m + odd < nr) *(uint32_t *)((bf16_t *)a.out + (int64_t)(r0 + m + odd) * n_out + n - odd) = __builtin_bit_cast(uint32_t, __builtin_convertvector(both, mm_bf16x2));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        if (in && m + i < nr) st_f((T *)a.out + (int64_t)(r0 + m + i) * n_out + n, v[i]);
+                }
+            }
+        }
+}
+
 template <typename T, int TM, int NW, int WR, int TKU, bool GATED, bool FAR>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM a) {
     constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
     constexpr int XPF = TM * TKU / THREADS, WPF = WR * TKU / THREADS, TN = GATED ? WR / 2 : WR, STAGE = TKU * UNIT;
     static_assert(XPF * THREADS == TM * TKU && WPF * THREADS == WR * TKU && (!GATED || NT % 2 == 0), "tile");
     __shared__ uint4 smem[2 * (TM + WR) * TKU];
-    int tile, col;
+    __shared__ int rows_out[TM];                                    // way down: the flat indices and weights of the tile's rows
+    __shared__ float rows_weight[TM];
+    int tile, col, part = 0;
     if (TM >= 64) {                                                 // workgroups with the same remainder by 8 share an XCD
         const int per_xcd = (a.offsets[a.E + 1] + 7) / 8, xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
-        if (s >= per_xcd * a.col_blocks) return;
-        tile = xcd * per_xcd + s / a.col_blocks;
+        if (s >= per_xcd * a.col_blocks * a.parts) return;
+        tile = xcd * per_xcd + s / (a.col_blocks * a.parts);
+        part = s / a.col_blocks % a.parts;
         col = s % a.col_blocks;
         if (tile >= a.max_tiles) return;
     } else {
@@ -339,10 +401,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
     }
     const int e = a.tile_expert[tile];
     if (e < 0) return;
-    const int r0 = a.tile_row0[tile], K = a.K, n_out = a.n_out, n0 = col * TN;
+    const int r0 = a.tile_row0[tile] + part * TM, K = a.K, n_out = a.n_out, n0 = col * TN;
+    if (a.offsets[e + 1] <= r0) return;
     const int nr = a.offsets[e + 1] - r0 < TM ? a.offsets[e + 1] - r0 : TM;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave / WN, wn = wave % WN;
     auto at = [](int row, int u) { return row * TKU + (u ^ (TKU == 4 ? (row >> 2) & 3 : (row >> 1) & 7)); };
+    if (!GATED && a.mode == 1)
+        for (int m = tid; m < nr; m += THREADS) {
+            const int p = a.perm[r0 + m];
+            rows_out[m] = p;
+            rows_weight[m] = a.weights[p];
+        }
     // loaders: unit tid % TKU of rows tid / TKU + x * THREADS / TKU; a row that does not exist repeats another and is not stored
     const int lr = tid / TKU;
     constexpr bool DMA = NW > 1;
@@ -395,8 +464,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
             for (int i = 0; i < 16; ++i) acc[x][t][i] = 0.f;
     // weight row (within the tile) of this wavefront's tile t: gate tiles first, then the linear branch's
     auto w_row = [&](int t) { return GATED ? (t < NT / 2 ? 0 : TN) + wn * (TN / WN) + 32 * (t % (NT / 2 > 0 ? NT / 2 : 1)) : wn * (WR / WN) + 32 * t; };
-    auto products = [&](auto sel_c) {
-        constexpr int sel = decltype(sel_c)::value;
+    auto products = [&](int sel) {
         const uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
 #pragma unroll
         for (int s = 0; s < TKU / 2; ++s) {
@@ -409,12 +477,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int x = 0; x < XT; ++x) acc[x][t] = mm_type<T>::mma(wf[t], xf[x], acc[x][t]);
+                for (int x = 0; x < XT; ++x) acc[x][t] = mm_type<T>::mma(xf[x], wf[t], acc[x][t]);
 
         }
     };
-    std::integral_constant<int, 0> even;
-    std::integral_constant<int, 1> odd;
     if (DMA && full > 0) {
         // straight into LDS: a wavefront's 64 places of 16 bytes per load, one stage ahead
         const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(smem + wave * 64));
@@ -429,25 +495,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
 #pragma unroll
             for (int x = 0; x < WPF; ++x) jl_load_lds(w_base(x) + k, wo[x], dst + (XPF + x) * THREADS * 16);
         };
-        auto arrived = [&]() {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-        };
         issue(0, 0);
-        int i = 0;
-        for (; i + 1 < full; i += 2) {
-            arrived();
-            issue(i + 1, 1);
-            products(even);
-            arrived();
-            issue(i + 2, 0);
-            products(odd);
-        }
-        arrived();
-        if (i < full) {
-            products(even);
+        for (int i = 0; i < full; ++i) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // stage i is in LDS; everybody has read stage i - 1, whose place is free
             __syncthreads();
+            issue(i + 1, (i + 1) & 1);
+            products(i & 1);
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
     } else if (full > 0) {
         fetch(reg[0], 0);
         constexpr int R1 = DMA ? 0 : 1;
@@ -457,16 +513,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
         int i = 0;
         for (; i + 1 < full; i += 2) {                              // two stages ahead: a trip to memory takes longer than one stage's products
             fetch(reg[0], i + 2);
-            products(even);
+            products(0);
             stash(reg[R1], 1);
             __syncthreads();
             fetch(reg[R1], i + 3);
-            products(odd);
+            products(1);
             stash(reg[0], 0);
             __syncthreads();
         }
         if (i < full) {
-            products(even);
+            products(0);
             __syncthreads();
         }
     }
@@ -483,50 +539,147 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
         for (int x = 0; x < WPF; ++x) reg[0][XPF + x] = last(w_base(x) + wo[x], unit_of(x));
         stash(reg[0], 0);
         __syncthreads();
-        products(even);
+        products(0);
     }
-    constexpr int OT = GATED ? NT / 2 : NT;
-    const bool whole = n_out % 4 == 0;
+    moe_store<T, XT, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int x, int k, int &p, float &w) { const int m = wm * (TM / WM) + 32 * x + k; p = rows_out[m]; w = rows_weight[m]; },
+                                [&](int x) { return wm * (TM / WM) + 32 * x; }, w_row, lane);
+}
+
+// ---- the same product in tiles of 256 rows by 256 weight rows (bfloat16, depths in whole stages of 64) ----------------------------------------
+// What bounds the tiles of 128 rows where experts have hundreds of rows each is not the matrix cores but the way from L2 into LDS (without their products they take 335 of 395 us for the gated product at 8192 x 4
+// of 32 experts of 2048 x 1024: 3.4 GB at 10 TB/s).  Tiles of 256 x 256 move a third less, in whole lines of 128 bytes.  One workgroup of eight wavefronts (128 rows x 64 weight rows each, two per SIMD) per CU
+// walks tile after tile: the next tile's first stage travels while the last stage of this one is multiplied, and this one's results leave while the next is multiplied.  A tile of at most 128 rows
+// (an expert's last) takes half the products: the row blocks of 32 alternate between the two rows of wavefronts.
+// Gated product of 8192 x 4 of 32 experts of 2048 x 1024: 395 -> 330 us (830 TFLOP/s); without loads 229, without products 235, without results 300.  Three stages of W in LDS instead of two,
+// so that its lines from memory have twice the time, change nothing, nor do other orders of the depths per column; on the way down the results of a whole round (67 MB) leave at once and
+// make up for the rest: 245 us against 236 of three smaller workgroups per CU.
+template <bool GATED>
+__global__ __launch_bounds__(512, 2) void moe_big_kernel(MoeMM a) {
+    constexpr int TKU = 8, STAGE = 64, XT = 4, NT = 2, TN = GATED ? 128 : 256, BUF = 512 * TKU;
+    __shared__ uint4 smem[2 * BUF];                                 // [2][rows of X, rows of W][8 units]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave >> 2, wn = wave & 3;
+    const int K = a.K, n_out = a.n_out, full = K / STAGE, in_use = __builtin_amdgcn_readfirstlane(a.offsets[a.E + 1]), tiles = in_use < a.max_tiles ? in_use : a.max_tiles;
+    const int per_xcd = (tiles + 7) / 8, first = (blockIdx.x & 7) * per_xcd, slots = gridDim.x / 8;      // workgroups with the same remainder by 8 share an XCD: neighbouring tiles and all their columns
+    const int here = tiles - first < per_xcd ? tiles - first : per_xcd;
+    auto at = [](int row, int u) { return row * TKU + (u ^ ((row >> 1) & 7)); };
+    auto w_row = [&](int t) { return GATED ? t * TN + wn * 32 : wn * 64 + 32 * t; };
+    struct Tile { int e, r0, nr, n0; };
+    auto tile_at = [&](int q) {
+        const int t = first + q / a.col_blocks, e = __builtin_amdgcn_readfirstlane(a.tile_expert[t]), r0 = __builtin_amdgcn_readfirstlane(a.tile_row0[t]);
+        const int left = __builtin_amdgcn_readfirstlane(a.offsets[e + 1]) - r0;
+        return Tile{e, r0, left < 256 ? left : 256, (q % a.col_blocks) * TN};
+    };
+    // loaders: the unit that belongs into this thread's place of LDS, of rows tid / 8 + 64 x of X and of W; a row that does not exist repeats another and is not stored
+    const int lr = tid >> 3, unit = (tid & 7) ^ ((lr >> 1) & 7);
+    uint32_t xo[XT], wo[4];
+    const char *const Xb = (const char *)a.X, *Wb, *Wl;
+    bool half;                                                      // at most 128 rows
+    auto aim = [&](const Tile &t, const int (&row)[XT]) {
+        Wb = (const char *)a.Wt + ((int64_t)t.e * (GATED ? 2 : 1) * n_out + t.n0) * K * 2;
+        Wl = Wb + (int64_t)(GATED ? n_out : 0) * K * 2;
+        half = t.nr <= 128;
 #pragma unroll
-    for (int x = 0; x < XT; ++x) {
-        const int m = wm * (TM / WM) + 32 * x + l32;
-        if (m >= nr) continue;
-        const int64_t r = r0 + m;
-        const int64_t p = a.mode == 1 ? a.perm[r] : r;
-        const float w = a.mode == 1 ? a.weights[p] : 1.0f;
+        for (int x = 0; x < XT; ++x) {
+            xo[x] = (uint32_t)(row[x] / a.top) * (uint32_t)(K * 2) + unit * 16;
+            const int j = lr + 64 * x, c = GATED ? j % TN : j;
+            wo[x] = (uint32_t)(t.n0 + c < n_out ? c : n_out - 1 - t.n0) * (uint32_t)(K * 2) + unit * 16;
+        }
+    };
+    auto rows_of = [&](const Tile &t, int (&row)[XT]) {
 #pragma unroll
-        for (int t = 0; t < OT; ++t)
+        for (int x = 0; x < XT; ++x) {
+            const int m = lr + 64 * x < t.nr ? lr + 64 * x : 0;
+            row[x] = a.perm[t.r0 + m];                              // divided by `top` where it is used: the load need not be waited for here
+        }
+    };
+    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(smem + wave * 64));
+    auto issue = [&](int i, int sel, int part) {                     // the rows of X (part 0) or of W (1) of stage i into buffer `sel`
+        const int64_t k = (int64_t)i * STAGE * 2;
+        const uint32_t dst = lds + sel * BUF * 16;
+        if (part == 0) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int n = n0 + w_row(t) + 8 * g + 4 * hi;       // four neighbouring columns
-                if (n >= n_out) continue;
-                float v[4];
+            for (int x = 0; x < XT; ++x)
+                if (x < XT / 2 || !half) jl_load_lds(Xb + k, xo[x], dst + x * 512 * 16);
+        } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float c = acc[x][t][4 * g + i];
-                    if (GATED) v[i] = gated_unit_f<sizeof(T) == 2>(c, acc[x][t + (GATED ? OT : 0)][4 * g + i], a.act.kind, a.act.limit, a.act.alpha, a.act.shift);
-                    else if (a.mode == JL_MOE_UP_PLAIN) v[i] = c;
-                    else if (a.mode == 0) { const float q = fmaxf(c, 0.f); v[i] = q * q; }
-                    else v[i] = c * w;
-                }
-                const int64_t o = p * n_out + n;
-                if (!GATED && a.mode == 1) {
-                    if (whole) st4_f((float *)a.out + o, v);
-                    else for (int i = 0; i < 4 && n + i < n_out; ++i) ((float *)a.out)[o + i] = v[i];
-                } else {
-                    if (whole) st4_f((T *)a.out + o, v);
-                    else for (int i = 0; i < 4 && n + i < n_out; ++i) st_f((T *)a.out + o + i, v[i]);
-                }
-            }
-    }
+            for (int x = 0; x < 4; ++x) jl_load_lds((GATED && x >= 2 ? Wl : Wb) + k, wo[x], dst + (XT + x) * 512 * 16);
+        }
+    };
+    auto products = [&](int sel, auto &acc, auto beside) {
+        constexpr int NX = sizeof(acc) / sizeof(acc[0]);
+        const uint4 *Xs = smem + sel * BUF, *Ws = Xs + 256 * TKU;
+#pragma unroll
+        for (int s = 0; s < TKU / 2; ++s) {
+            uint4 xf[NX], wf[NT];
+#pragma unroll
+            for (int x = 0; x < NX; ++x) xf[x] = Xs[at(64 * x + 32 * wm + l32, 2 * s + hi)];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wf[t] = Ws[at(w_row(t) + l32, 2 * s + hi)];
+            beside(s);
+            __builtin_amdgcn_s_setprio(1);                          // whoever has its operands multiplies; the SIMD's other wavefront reads meanwhile
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int x = 0; x < NX; ++x) acc[x][t] = mm_type<bf16_t>::mma(xf[x], wf[t], acc[x][t]);
+            __builtin_amdgcn_s_setprio(0);
+        }
+    };
+    const int n_q = here * a.col_blocks;
+    int q = blockIdx.x >> 3;
+    if (q >= n_q) return;                                           // the whole workgroup
+    Tile now = tile_at(q);
+    int row[XT], sel = 0;
+    rows_of(now, row);
+    aim(now, row);
+    issue(0, 0, 0);
+    issue(0, 0, 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // one tile: stage 0 of it is in buffer `sel`, as far as this wavefront loaded it.  False behind the last
+    auto walk = [&](auto n_x) {
+        constexpr int NX = decltype(n_x)::value;
+        const bool more = q + slots < n_q;
+        Tile next = now;
+        if (more) {
+            next = tile_at(q + slots);
+            rows_of(next, row);
+        }
+        mm_f32x16 acc[NX][NT];
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[x][t][i] = 0.f;
+        for (int i = 0; i + 1 < full; ++i) {
+            if (i > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();                                        // stage i is in LDS; everybody has read what the other buffer held
+            products(sel, acc, [&](int s) { if (s < 2) issue(i + 1, sel ^ 1, s); });
+            sel ^= 1;
+        }
+        if (full > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (more) {
+            aim(next, row);
+            issue(0, sel ^ 1, 0);
+            issue(0, sel ^ 1, 1);
+        }
+        products(sel, acc, [](int) {});
+        sel ^= 1;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // the next tile's first stage, before the results: what this wavefront loaded of it is there
+        moe_store<bf16_t, NX, NT, GATED, false>(a, acc, now.r0, now.nr, now.n0, [](int, int, int &, float &) {}, [&](int x) { return 64 * x + 32 * wm; }, w_row, lane);
+        now = next;
+        q += slots;
+        return more;
+    };
+    while (half ? walk(std::integral_constant<int, XT / 2>()) : walk(std::integral_constant<int, XT>())) {}
 }
 
 template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(MoeMM &a, bool gated, hipStream_t st) {
     const int tn = gated ? WR / 2 : WR;
     a.col_blocks = (a.n_out + tn - 1) / tn;
-    const int64_t groups = (int64_t)(TM >= 64 ? (a.max_tiles + 7) / 8 * 8 : a.max_tiles) * a.col_blocks;
+    const int64_t groups = (int64_t)(TM >= 64 ? (a.max_tiles + 7) / 8 * 8 : a.max_tiles) * a.col_blocks * a.parts;
     if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
-    const bool far = a.mode != 1 && ((int64_t)a.max_tiles * TM / a.top + 1) * a.K * (int64_t)sizeof(T) > UINT32_MAX;      // gathered rows beyond what 32 bits reach
+    const bool far = a.mode != 1 && ((int64_t)a.max_tiles * a.parts * TM / a.top + 1) * a.K * (int64_t)sizeof(T) > UINT32_MAX;      // gathered rows beyond what 32 bits reach
     auto kern = gated ? (far ? moe_mm_kernel<T, TM, NW, WR, TKU, true, true> : moe_mm_kernel<T, TM, NW, WR, TKU, true, false>)
                       : (far ? moe_mm_kernel<T, TM, NW, WR, TKU, false, true> : moe_mm_kernel<T, TM, NW, WR, TKU, false, false>);
     kern<<<dim3((unsigned)groups), 64 * NW, 0, st>>>(a);
@@ -534,8 +687,17 @@ template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(
 }
 template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
+        if (tile_rows == 256) {
+            a.parts = 2;
+            if (a.mode == 1 || !moe_big_sizes(a.K, (int64_t)a.max_tiles * 256)) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
+            a.col_blocks = (a.n_out + (gated ? 127 : 255)) / (gated ? 128 : 256);
+            const int64_t groups = (int64_t)(a.max_tiles + 7) / 8 * 8 * a.col_blocks;
+            if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
+            (gated ? moe_big_kernel<true> : moe_big_kernel<false>)<<<dim3((unsigned)(groups < 256 ? groups : 256)), 512, 0, st>>>(a);      // one workgroup per CU
+            return jl_check_launch("moe_big_kernel");
+        }
         if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
-    } else if (tile_rows == 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32 or 64 rows");
+    } else if (tile_rows >= 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32 or 64 rows");
     if (tile_rows == 64) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
     return moe_mm_launch<T, 32, 1, 64, 8>(a, gated, st);
 }
@@ -544,9 +706,9 @@ static int moe_gemm_launch(const void *X, const void *Wt, int dtype, int32_t mod
                            const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0, int32_t max_tiles, int32_t E, int32_t tile_rows,
                            const float *weights, void *out, const MoeAct *act, void *stream) {
     static const bool no_mfma = getenv("JL_MOE_NO_MFMA") != nullptr;      // A/B switch for measurements
-    if (E <= 0 || (tile_rows != 32 && tile_rows != 64 && tile_rows != 128)) return jl_fail(JL_E_INVALID, "jl_moe_gemm: tiles of 32, 64 or 128 rows");
+    if (E <= 0 || (tile_rows != 32 && tile_rows != 64 && tile_rows != 128 && tile_rows != 256)) return jl_fail(JL_E_INVALID, "jl_moe_gemm: tiles of 32, 64, 128 or 256 rows");
     const int64_t dtype_bytes = dtype == JL_BF16 ? 2 : 4;
-    MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}};
+    MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, 1, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}};
     if (!no_mfma && moe_mm_sizes(dtype, K) && ((uintptr_t)X % 16) == 0 && ((uintptr_t)Wt % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
         256 * (int64_t)K * dtype_bytes <= UINT32_MAX) {                     // a tile's rows, of X or of W
         if (dtype == JL_BF16) return moe_mm_rows<bf16_t>(a, tile_rows, act != nullptr, (hipStream_t)stream);

@@ -688,6 +688,8 @@ def moe_experts(h: torch.Tensor, router_logits: torch.Tensor, correction: Option
                                   _ROUTES[route], float(renorm_eps), st), "jl_moe_route")
     rows = n * top
     tm = int(L.jl_moe_tile_rows(_code(dt), rows, E, W, ff))
+    if tm == 128 and L.jl_moe_tile_pairs(rows, E, W, ff, int(gated is not None)):
+        tm = 256
     max_tiles = rows // tm + E
     perm = torch.empty((rows,), dtype=torch.int32, device=dev)
     offsets = torch.empty((E + 2,), dtype=torch.int32, device=dev)
