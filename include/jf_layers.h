@@ -441,6 +441,20 @@ JL_API int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32
 /* 1: bfloat16 tiles of 128 rows are better grouped in pairs (tile_rows 256 for jl_moe_group and the products) */
 JL_API int jl_moe_tile_pairs(int64_t rows, int32_t E, int32_t W, int32_t ff, int32_t gated);
 
+/* Router product, choice and grouping of a step of up to 32 * JL_MOE_ROUTER_BLOCKS tokens in one call: logits = x W^T (+ bias) in float (x [N, K] of x_dtype with rows x_ld apart, W [E, K] and bias float),
+ * then what jl_moe_route gives for them (`E` outputs, kind, correction) and what jl_moe_group gives for the `experts` of them that have weights.  E <= 64, K a multiple of 4, rows of x and W at
+ * 16-byte borders; counts: jl_moe_router_blocks(N) * experts int32 of scratch (not read when that is one block).  w null: x are the logits, float [N, E] (K, x_ld are not read). */
+#define JL_MOE_ROUTER_BLOCKS 512
+typedef struct {
+    const void *x; const float *w; const float *bias; const float *correction; int32_t *ids; float *weights;
+    int32_t *perm; int32_t *offsets; int32_t *tile_expert; int32_t *tile_row0; int32_t *counts;
+    int64_t N, x_ld;
+    int32_t x_dtype, K, E, experts, top, kind, tile_rows, max_tiles;
+    float scale, renorm_eps;
+} jl_moe_router;
+JL_API int jl_moe_router_blocks(int64_t N);
+JL_API int jl_moe_router_run(const jl_moe_router *a, void *stream);
+
 /* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].
  *   mode 0 (up):   in(r) = perm[r] / top;  out[r, :] = relu(C)^2, stored in `dtype` ([N*top, n_out], sorted order)
  *   mode 1 (down): in(r) = r;              out[perm[r], :] = C * weights[perm[r]], stored as float ([N*top, n_out])

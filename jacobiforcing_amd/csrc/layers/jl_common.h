@@ -111,6 +111,28 @@ __device__ __forceinline__ void jl_load_lds_far(const char *from, uint32_t lds) 
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "m0", "memory");
 }
 
+typedef __bf16 jl_bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 jl_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float jl_f32x8 __attribute__((ext_vector_type(8)));
+constexpr int JL_SPLIT_TERMS = 3;
+// eight floats as the sum of JL_SPLIT_TERMS bfloat16 numbers each; what a term leaves over is exact, and one product of pairs with (-1, 0) or (0, -1) gives it without unpacking the term
+__device__ __forceinline__ void jl_split8(jl_f32x8 v, jl_bf16x8 (&part)[JL_SPLIT_TERMS]) {
+    uint32_t low = 0x0000bf80u, high = 0xbf800000u;                 // -1 in one half.  In registers: the compiler writes (-1, 0) as the inline constant -1.0, which the instruction reads as a float's bits
+    asm("" : "+s"(low), "+s"(high));
+    const jl_bf16x2 first = __builtin_bit_cast(jl_bf16x2, low), second = __builtin_bit_cast(jl_bf16x2, high);
+#pragma unroll
+    for (int x = 0; x < JL_SPLIT_TERMS; ++x) {
+        part[x] = __builtin_convertvector(v, jl_bf16x8);
+        if (x + 1 == JL_SPLIT_TERMS) break;
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            const jl_bf16x2 p = {part[x][i], part[x][i + 1]};
+            v[i] = __builtin_amdgcn_fdot2_f32_bf16(p, first, v[i], false);
+            v[i + 1] = __builtin_amdgcn_fdot2_f32_bf16(p, second, v[i + 1], false);
+        }
+    }
+}
+
 #define JL_DISPATCH(dtype, ...)                                   \
     do {                                                          \
         if ((dtype) == JL_BF16) { typedef bf16_t T; __VA_ARGS__; } \

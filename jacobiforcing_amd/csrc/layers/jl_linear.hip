@@ -1,5 +1,5 @@
 // jl_linear.hip — dense products of a few rows (decoding): out[n] = W x[n] (+ bias), W [O, K] read once.
-#include "jl_common.h"
+#include "jl_small.h"
 
 // What bounds such a product is W's bytes when W is large and the way there when it is small (a launch alone is 3 us, a trip to memory 2 us).  So a workgroup's NW wavefronts
 // share the depth of 16 * OT rows of W, every lane has LS_AHEAD pairs of 16-byte units of each of its rows of W and x (which comes from L2) on the way at once, straight into the
@@ -12,72 +12,13 @@
 // As long as 16 rows of W per workgroup come to no more workgroups than the chip has CUs, that is the best; beyond, x is read again by every workgroup that a CU runs, and more rows
 // of W per workgroup pay (not for one row of x).  Library products of the same shapes take 8.2, 12.4, 24.0 / 14.9, 12.2, 18.7 us, and 11 us more of host time per call (19.5 / 8.6).
 // Rows beyond 16 cost x's reads: the caller's rule (layer_ops.linear) leaves products to the library where a CU would read more than 128 KB of x.
-constexpr int LS_AHEAD = 4;
-
-typedef float ls_f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 ls_bf16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ ls_f32x4 ls_mma(const bf16_t *, uint4 a, uint4 b, ls_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ls_bf16x8, a), __builtin_bit_cast(ls_bf16x8, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ ls_f32x4 ls_mma(const float *, uint4 a, uint4 b, ls_f32x4 c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ uint4 ls_unit(const bf16_t *p, const bf16_t *) { return *(const uint4 *)p; }
-__device__ __forceinline__ uint4 ls_unit(const float *p, const float *) { return *(const uint4 *)p; }
-__device__ __forceinline__ uint4 ls_unit(const bf16_t *p, const float *) {        // four 16-bit values for a float product
-    const uint2 v = *(const uint2 *)p;
-    return make_uint4(v.x << 16, v.x & 0xffff0000u, v.y << 16, v.y & 0xffff0000u);
-}
-
 template <typename TX, typename T, int NT, int OT, int NW>          // N <= 16 * NT rows of x, 16 * OT rows of W, NW wavefronts
 __global__ __launch_bounds__(64 * NW) void linear_small_kernel(const TX *__restrict__ x, int64_t x_ld, const T *__restrict__ w, const T *__restrict__ bias, void *__restrict__ out,
                                                                int64_t out_ld, int N, int K, int O, int out_mode) {
     __shared__ ls_f32x4 part[NW][OT][NT][64];
-    constexpr int UNIT = 16 / sizeof(T), LINE = 8 * UNIT;           // elements of a unit, of the 128 bytes that a step takes from every row
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4, o0 = blockIdx.x * 16 * OT;
-    const int k_lane = UNIT * g;
-    const T *wp[OT];
-    const TX *xp[NT];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, o0 = blockIdx.x * 16 * OT;
     ls_f32x4 acc[OT][NT];
-#pragma unroll
-    for (int o = 0; o < OT; ++o) {
-        const int r = o0 + 16 * o + r16;
-        wp[o] = w + (int64_t)(r < O ? r : O - 1) * K + k_lane;      // rows and columns that do not exist repeat the last one and are not stored
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[o][t] = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int n = 16 * t + r16;
-        xp[t] = x + (int64_t)(n < N ? n : N - 1) * x_ld + k_lane;
-    }
-    const int steps = (K + LINE - 1) / LINE, s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW;
-    for (int s = s0; s < s1; s += LS_AHEAD) {
-        uint4 wr[LS_AHEAD][2][OT], xr[LS_AHEAD][2][NT];
-#pragma unroll
-        for (int i = 0; i < LS_AHEAD; ++i)
-#pragma unroll
-            for (int y = 0; y < 2; ++y) {
-                const int k = (s + i) * LINE + 4 * UNIT * y;
-                const bool in = s + i < s1 && k + k_lane < K;
-#pragma unroll
-                for (int o = 0; o < OT; ++o) wr[i][y][o] = in ? *(const uint4 *)(wp[o] + k) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < NT; ++t) xr[i][y][t] = in ? ls_unit(xp[t] + k, (const T *)nullptr) : make_uint4(0, 0, 0, 0);
-            }
-#pragma unroll
-        for (int i = 0; i < LS_AHEAD; ++i)
-#pragma unroll
-            for (int y = 0; y < 2; ++y)
-#pragma unroll
-                for (int o = 0; o < OT; ++o)
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) acc[o][t] = ls_mma((const T *)nullptr, wr[i][y][o], xr[i][y][t], acc[o][t]);
-    }
+    ls_products<TX, T, NT, OT, NW>(acc, x, x_ld, w, N, K, o0, O, wave, lane);
 #pragma unroll
     for (int o = 0; o < OT; ++o)
 #pragma unroll

@@ -1,7 +1,7 @@
 // jl_moe.hip — routed experts: the router's choice (sigmoid scores with a correction, a softmax renormalised over the chosen with or without
 // a correction, or a softmax over the chosen logits alone), the rows grouped by expert (a choice of an expert without weights has none), and
 // the grouped products: up with relu^2, plain, or with the gated unit in its epilogue, down with the routing weights.
-#include "jl_common.h"
+#include "jl_small.h"
 #include <stdlib.h>
 #include <type_traits>
 constexpr int MOE_MAX_E = 4096;   // experts (router outputs) at most
@@ -205,6 +205,233 @@ extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t 
         return jl_fail(JL_E_INVALID, "jl_moe_group: experts must be <= %d and max_tiles >= rows / tile_rows + experts", MOE_MAX_E);
     moe_group_kernel<<<1, 1024, 0, (hipStream_t)stream>>>(ids, N * top, E, tile_rows, perm, offsets, tile_expert, tile_row0, max_tiles);
     return jl_check_launch("moe_group_kernel");
+}
+
+// ---- a layer's whole choice in one or two launches: router product, choice, grouping (up to 64 router outputs) --------------------------------------
+// Every workgroup takes 16 or 32 tokens: it forms their logits (the depth shared by eight wavefronts, rows of x and W straight from memory into the float matrix instructions: ls_products) or reads
+// them (LOGITS), chooses per token from LDS and counts its choices per expert; with one workgroup it groups them too.  With more, a second launch of as many workgroups adds the counts up to where each
+// one's rows go: no workgroup walks all rows.  What bounds them: what one CU takes in, 26 GB/s of x and W (more of them on the way, or the products on the bfloat16 instructions in three terms, change
+// nothing), then the table of counts.  us, product + choice + grouping in launches of their own / in these (from logits): 8192 x 1024 bfloat16 by 16 outputs 57 / 17 (9), 8192 x 2048 float by 32
+// 51 / 32 (13), by 40 56 / 45 (19), 32 x 1024 by 16 24 / 11 in one launch instead of three, 32 x 2048 float by 32 27 / 21, 2246 x 1024 float by 16 28 / 13.
+constexpr int MR_MAX_E = 64, MR_NW = 8;
+
+// lane e of the first wavefront: where expert e's rows and tiles start; offsets and the list of tiles (the first workgroup's to write)
+__device__ __forceinline__ void moe_group_list(const jl_moe_router &a, int rows_e, int lane, int &start, int *first_tile) {
+    const int tiles_e = (rows_e + a.tile_rows - 1) / a.tile_rows;
+    int inc_r = rows_e, inc_t = tiles_e;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(inc_r, off, 64), y = __shfl_up(inc_t, off, 64);
+        if (lane >= off) { inc_r += x; inc_t += y; }
+    }
+    start = inc_r - rows_e;
+    first_tile[lane] = inc_t - tiles_e;                             // an expert without rows has no tiles: the same number as the next
+    if (lane == 63) first_tile[64] = inc_t;
+    if (blockIdx.x == 0) {
+        if (lane < a.experts) a.offsets[lane] = start;
+        if (lane == 63) { a.offsets[a.experts] = inc_r; a.offsets[a.experts + 1] = inc_t < a.max_tiles ? inc_t : a.max_tiles; }
+    }
+}
+__device__ __forceinline__ void moe_tile_list(const jl_moe_router &a, const int *starts, const int *first_tile, int tid, int threads) {
+    for (int t = tid; t < a.max_tiles; t += threads) {
+        int lo = 0, hi = a.experts;                                 // the last expert with first_tile <= t
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (first_tile[mid] <= t) lo = mid; else hi = mid;
+        }
+        const bool in = t < first_tile[64];
+        a.tile_expert[t] = in ? lo : -1;
+        a.tile_row0[t] = in ? starts[lo] + (t - first_tile[lo]) * a.tile_rows : 0;
+    }
+}
+
+// the largest over groups of P lanes (16, 32 or 64); within rows of 16 by exchanges in the vector unit
+template <int P> __device__ __forceinline__ float moe_group_max(float v) {
+#define MR_STEP(ctrl) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, 0xF, 0xF, true)))
+    MR_STEP(0xB1);                                                  // quad_perm [1, 0, 3, 2], [2, 3, 0, 1], half rows and rows mirrored
+    MR_STEP(0x4E);
+    MR_STEP(0x141);
+    MR_STEP(0x140);
+#undef MR_STEP
+    if (P > 16) v = fmaxf(v, __shfl_xor(v, 16, 64));
+    if (P > 32) v = fmaxf(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+// moe_route_kernel's choice for R tokens per P lanes at once (their chains of exchanges run side by side), 64 / P groups of lanes: this lane's output is e = lane % P, the logits of token r at z[r];
+// each(r, s, e, weight) by the lane of the s-th choice.  A choice is the lowest index among the largest comparison values (one that is not a number counts as the largest): the wavefront's
+// mask of them has it without passing indices on.  The sums are those of moe_route_kernel in the same order.
+template <int P, int R, typename Each>
+__device__ __forceinline__ void moe_route_rows(const float *const (&z)[R], const float *__restrict__ correction, int E, int top, int kind, float scale, float renorm_eps, int lane, Each each) {
+    const int e = lane % P, base = lane - e;
+    const uint64_t group = P == 64 ? ~0ull : (1ull << P) - 1;
+    float cmp[R], sc[R], zmax[R], den[R], chosen[R];
+    int turn[R];                                                    // which choice this lane's output is; -1: none yet, -2: there is no such output
+#pragma unroll
+    for (int r = 0; r < R; ++r) { turn[r] = e < E ? -1 : -2; cmp[r] = e < E ? z[r][e] : -INFINITY; zmax[r] = moe_group_max<P>(cmp[r]); }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        sc[r] = e >= E ? -INFINITY : kind == JL_ROUTE_SIGMOID ? 1.0f / (1.0f + expf(-cmp[r])) : expf(cmp[r] - zmax[r]);
+        den[r] = e < E ? sc[r] : 0.f;
+        chosen[r] = 0.f;
+    }
+    if (kind == JL_ROUTE_SOFTMAX_RENORM)
+#pragma unroll
+        for (int off = P / 2; off > 0; off >>= 1)
+#pragma unroll
+            for (int r = 0; r < R; ++r) den[r] += __shfl_xor(den[r], off, 64);
+    const float add = e < E && correction && kind != JL_ROUTE_TOP_SOFTMAX ? correction[e] : 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (kind == JL_ROUTE_SOFTMAX_RENORM) sc[r] /= den[r];
+        if (kind == JL_ROUTE_SIGMOID || (kind == JL_ROUTE_SOFTMAX_RENORM && correction)) cmp[r] = sc[r];
+        if (correction && kind != JL_ROUTE_TOP_SOFTMAX) cmp[r] += add;
+        if (cmp[r] != cmp[r]) cmp[r] = INFINITY;
+    }
+    for (int s = 0; s < top; ++s) {
+        float most[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) most[r] = moe_group_max<P>(turn[r] == -1 ? cmp[r] : -INFINITY);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint64_t largest = __ballot(turn[r] == -1 && cmp[r] == most[r]) >> base & group;
+            const int be = largest ? __ffsll((unsigned long long)largest) - 1 : 0;
+            chosen[r] += __shfl(sc[r], base + be, 64);
+            if (be == e) turn[r] = s;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (turn[r] >= 0) each(r, turn[r], e, sc[r] / (kind == JL_ROUTE_SIGMOID ? 1.0f : kind == JL_ROUTE_SOFTMAX_RENORM ? chosen[r] + renorm_eps : chosen[r]) * scale);
+}
+
+template <typename TX, int NT, int OT, bool LOGITS>
+__global__ __launch_bounds__(64 * MR_NW) void moe_router_kernel(jl_moe_router a) {
+    constexpr int ROWS = 16 * NT;
+    __shared__ ls_f32x4 part[LOGITS ? 1 : MR_NW][OT][NT][64];
+    __shared__ float z[ROWS][16 * OT];
+    __shared__ int count[MR_MAX_E], starts[MR_MAX_E], first_tile[MR_MAX_E + 1];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int64_t n0 = (int64_t)blockIdx.x * ROWS;
+    const int rows = a.N - n0 < ROWS ? (int)(a.N - n0) : ROWS;
+    if (tid < MR_MAX_E) count[tid] = 0;
+    if constexpr (LOGITS) {
+        const float *from = (const float *)a.x + n0 * a.E;
+        for (int i = tid; i < rows * a.E; i += 64 * MR_NW) z[i / a.E][i % a.E] = from[i];
+    } else {
+        ls_f32x4 acc[OT][NT];
+        ls_products<TX, float, NT, OT, MR_NW, 1, true>(acc, (const TX *)a.x + n0 * a.x_ld, a.x_ld, a.w, rows, a.K, 0, a.E, wave, lane);
+#pragma unroll
+        for (int o = 0; o < OT; ++o)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) part[wave][o][t][lane] = acc[o][t];
+        __syncthreads();
+        for (int e = tid; e < OT * NT * 64; e += 64 * MR_NW) {
+            const int l = e & 63, t = (e >> 6) % NT, ot = (e >> 6) / NT, o = 16 * ot + 4 * (l >> 4);
+            ls_f32x4 s = part[0][ot][t][l];
+#pragma unroll
+            for (int i = 1; i < MR_NW; ++i) s += part[i][ot][t][l];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) z[16 * t + (l & 15)][o + i] = a.bias && o + i < a.E ? s[i] + a.bias[o + i] : s[i];
+        }
+    }
+    __syncthreads();
+    // a wavefront's tokens: its share of the rows, a few side by side
+    constexpr int P = 16 * OT <= 16 ? 16 : 16 * OT <= 32 ? 32 : 64, SHARE = ROWS / MR_NW, GROUPS = 64 / P < SHARE ? 64 / P : SHARE, R = SHARE / GROUPS;
+    const float *zr[R];
+    int64_t first[R];                                               // where the row's choices lie
+    bool real[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int g = lane / P < GROUPS ? lane / P : GROUPS - 1, row = wave * SHARE + r * GROUPS + g;
+        real[r] = lane / P < GROUPS && row < rows;
+        zr[r] = z[row];
+        first[r] = (n0 + row) * a.top;
+    }
+    moe_route_rows<P, R>(zr, a.correction, a.E, a.top, a.kind, a.scale, a.renorm_eps, lane, [&](int r, int s, int e, float weight) {
+        if (!real[r]) return;
+        a.ids[first[r] + s] = e;
+        a.weights[first[r] + s] = weight;
+        if (e < a.experts) atomicAdd(&count[e], 1);                 // an expert without weights has no rows
+    });
+    __syncthreads();
+    if (gridDim.x > 1) {
+        if (tid < a.experts) a.counts[(int64_t)blockIdx.x * a.experts + tid] = count[tid];
+        return;
+    }
+    if (wave == 0) {
+        int start;
+        moe_group_list(a, lane < a.experts ? count[lane] : 0, lane, start, first_tile);
+        starts[lane] = start;
+    }
+    __syncthreads();
+    moe_tile_list(a, starts, first_tile, tid, 64 * MR_NW);
+    __syncthreads();
+    for (int i = tid; i < rows * a.top; i += 64 * MR_NW) {
+        const int e = a.ids[i];
+        if (e >= 0 && e < a.experts) a.perm[atomicAdd(&starts[e], 1)] = i;
+    }
+}
+
+// the workgroups of moe_router_kernel again: rows_per_block tokens each
+__global__ __launch_bounds__(1024) void moe_place_kernel(jl_moe_router a, int rows_per_block) {
+    __shared__ int total[16][MR_MAX_E], before[16][MR_MAX_E], starts[MR_MAX_E], place[MR_MAX_E], first_tile[MR_MAX_E + 1];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, blocks = gridDim.x, P = a.experts <= 16 ? 16 : a.experts <= 32 ? 32 : 64, e = lane % P, per = 64 / P;
+    int tot = 0, bef = 0;
+#pragma unroll 8
+    for (int b = wave * per + lane / P; b < blocks; b += 16 * per) {
+        const int c = e < a.experts ? a.counts[(int64_t)b * a.experts + e] : 0;
+        tot += c;
+        bef += b < (int)blockIdx.x ? c : 0;
+    }
+    for (int off = P; off < 64; off <<= 1) { tot += __shfl_xor(tot, off, 64); bef += __shfl_xor(bef, off, 64); }
+    total[wave][lane] = lane < P ? tot : 0;
+    before[wave][lane] = lane < P ? bef : 0;
+    __syncthreads();
+    if (wave == 0) {
+        int rows_e = 0, in_front = 0, start;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { rows_e += total[i][lane]; in_front += before[i][lane]; }
+        moe_group_list(a, rows_e, lane, start, first_tile);
+        starts[lane] = start;
+        place[lane] = start + in_front;
+    }
+    __syncthreads();
+    const int64_t i0 = (int64_t)blockIdx.x * rows_per_block * a.top, i1 = i0 + rows_per_block * a.top < a.N * a.top ? i0 + rows_per_block * a.top : a.N * a.top;
+    for (int64_t i = i0 + tid; i < i1; i += 1024) {
+        const int x = a.ids[i];
+        if (x >= 0 && x < a.experts) a.perm[atomicAdd(&place[x], 1)] = (int32_t)i;
+    }
+    if (blockIdx.x == 0) moe_tile_list(a, starts, first_tile, tid, 1024);
+}
+
+extern "C" int jl_moe_router_blocks(int64_t N) { return (int)(N <= 16 ? 1 : (N + 31) / 32 < 0x7fffffff ? (N + 31) / 32 : 0x7fffffff); }
+extern "C" int jl_moe_router_run(const jl_moe_router *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_moe_router_run: null arguments");
+    const jl_moe_router &a = *ap;
+    if (a.N <= 0) return JL_OK;
+    const int blocks = jl_moe_router_blocks(a.N);
+    const bool logits = !a.w;
+    if (!a.x || !a.ids || !a.weights || !a.perm || !a.offsets || !a.tile_expert || !a.tile_row0 || (blocks > 1 && !a.counts)) return jl_fail(JL_E_INVALID, "jl_moe_router_run: null pointer");
+    if (a.E <= 0 || a.E > MR_MAX_E || a.experts <= 0 || a.experts > a.E || a.top <= 0 || a.top > a.E || a.kind < JL_ROUTE_SIGMOID || a.kind > JL_ROUTE_TOP_SOFTMAX)
+        return jl_fail(JL_E_INVALID, "jl_moe_router_run: up to %d router outputs, experts and choices among them", MR_MAX_E);
+    if (a.N * a.top > INT32_MAX || blocks > JL_MOE_ROUTER_BLOCKS || a.tile_rows <= 0 || (int64_t)a.max_tiles < a.N * a.top / a.tile_rows + a.experts)
+        return jl_fail(JL_E_INVALID, "jl_moe_router_run: up to %d tokens and max_tiles >= rows / tile_rows + experts", 32 * JL_MOE_ROUTER_BLOCKS);
+    const int unit = a.x_dtype == JL_BF16 ? 8 : 4;
+    if (logits && (a.x_dtype != JL_F32 || a.bias)) return jl_fail(JL_E_INVALID, "jl_moe_router_run: logits are float and whole");
+    if (!logits && ((a.x_dtype != JL_BF16 && a.x_dtype != JL_F32) || a.K <= 0 || a.K % 4 || a.x_ld < a.K || a.x_ld % unit || (((uintptr_t)a.x | (uintptr_t)a.w) & 15)))
+        return jl_fail(JL_E_INVALID, "jl_moe_router_run: rows of x and W at 16-byte borders");
+    hipStream_t st = (hipStream_t)stream;
+#define MR_CASE(NT, OT)                                                                                                          \
+    do {                                                                                                                          \
+        if (logits) moe_router_kernel<float, NT, OT, true><<<dim3((unsigned)blocks), 64 * MR_NW, 0, st>>>(a);                      \
+        else JL_DISPATCH(a.x_dtype, moe_router_kernel<T, NT, OT, false><<<dim3((unsigned)blocks), 64 * MR_NW, 0, st>>>(a));        \
+    } while (0)
+    const int ot = (a.E + 15) / 16;
+    if (a.N <= 16) { if (ot == 1) MR_CASE(1, 1); else if (ot == 2) MR_CASE(1, 2); else if (ot == 3) MR_CASE(1, 3); else MR_CASE(1, 4); }
+    else { if (ot == 1) MR_CASE(2, 1); else if (ot == 2) MR_CASE(2, 2); else if (ot == 3) MR_CASE(2, 3); else MR_CASE(2, 4); }
+#undef MR_CASE
+    if (blocks > 1) moe_place_kernel<<<dim3((unsigned)blocks), 1024, 0, st>>>(a, 32);
+    return jl_check_launch("moe_router_kernel");
 }
 
 // ---- grouped product, any dtype and size: a 64 x 64 tile of one expert's rows per workgroup, float FMAs ------------------------------------

@@ -129,34 +129,14 @@ template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t 
 // take 12 000 cycles of issue; two side by side take 40 000.  Loads, stores, splits, weights: leaving out any one of them gives 5 to 15 % of the time.
 // Before, 64 columns of one head per workgroup met in LDS five times per group, one workgroup per CU.  us of the three launches, 4 x 2048 tokens, before / now: 16 heads of 128 x 128 with silu
 // 212 / 128 (their bytes at the rate of a large copy: 78), 32 heads of 128 x 64 over one key head 201 / 119; 2 x 300 of 8 heads 42 / 34, 40 x 64 of 16 heads 121 / 91.
-typedef __bf16 ch_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 ch_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 ch_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float ch_f32x4 __attribute__((ext_vector_type(4)));
-typedef float ch_f32x8 __attribute__((ext_vector_type(8)));
 typedef float ch_f32x16 __attribute__((ext_vector_type(16)));
 typedef short ch_s16x4 __attribute__((ext_vector_type(4)));
 typedef short ch_s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) ch_s16x4 ch_lds_s16x4;
-constexpr int CH_T = 64, CH_TERMS = 3, CH_OUT = 0, CH_LOCAL = 1;
+constexpr int CH_T = 64, CH_TERMS = JL_SPLIT_TERMS, CH_OUT = 0, CH_LOCAL = 1;
 
-// eight floats as the sum of CH_TERMS bfloat16 numbers each; what a term leaves over is exact, and one product of pairs with (-1, 0) or (0, -1) gives it without unpacking the term
-__device__ __forceinline__ void ch_split8(ch_f32x8 v, ch_bf16x8 (&part)[CH_TERMS]) {
-    uint32_t low = 0x0000bf80u, high = 0xbf800000u;                 // -1 in one half.  In registers: the compiler writes (-1, 0) as the inline constant -1.0, which the instruction reads as a float's bits
-    asm("" : "+s"(low), "+s"(high));
-    const ch_bf16x2 first = __builtin_bit_cast(ch_bf16x2, low), second = __builtin_bit_cast(ch_bf16x2, high);
-#pragma unroll
-    for (int x = 0; x < CH_TERMS; ++x) {
-        part[x] = __builtin_convertvector(v, ch_bf16x8);
-        if (x + 1 == CH_TERMS) break;
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-            const ch_bf16x2 p = {part[x][i], part[x][i + 1]};
-            v[i] = __builtin_amdgcn_fdot2_f32_bf16(p, first, v[i], false);
-            v[i + 1] = __builtin_amdgcn_fdot2_f32_bf16(p, second, v[i + 1], false);
-        }
-    }
-}
 __device__ __forceinline__ uint2 ch_silu4(uint2 w) {
     float v[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
 #pragma unroll
@@ -254,14 +234,14 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
         ch_s16x4 half[2];
 #pragma unroll
         for (int y = 0; y < 2; ++y) half[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ch_lds_s16x4 *)(tile + (16 * s + 8 * y + tr_row) * row_len + c + tr_col));
-        return __builtin_bit_cast(ch_bf16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        return __builtin_bit_cast(jl_bf16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
     };
     auto row_of = [&](const bf16_t *tile, int t, int s) {           // row t, depths 16 s + 4 hi + {0 .. 3, 8 .. 11}
         const ch_bf16x4 x = *(const ch_bf16x4 *)(tile + t * QROW + 16 * s + 4 * hi), y = *(const ch_bf16x4 *)(tile + t * QROW + 16 * s + 8 + 4 * hi);
         return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
     };
     auto acc8 = [](const ch_f32x16 &v, int s) {
-        ch_f32x8 f;
+        jl_f32x8 f;
 #pragma unroll
         for (int x = 0; x < 8; ++x) f[x] = v[8 * s + x];
         return f;
@@ -333,7 +313,7 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
         __syncthreads();
         if (t0 + CH_T < cnt) fetch(t0 + CH_T);                      // in flight while this group is multiplied
         if (OUT && t0 > 0) outputs(t0 - CH_T, CH_T);
-        ch_bf16x8 vf[CH_T / 16];
+        jl_bf16x8 vf[CH_T / 16];
         const bool more = !OUT || last || t0 + CH_T < cnt;          // else nobody reads this piece's final state: the next piece has its own
         if (busy) {
             if (OUT) {
@@ -342,11 +322,11 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = 0.f;
                 {
-                    ch_bf16x8 q[2][2], part[2][CH_TERMS];
+                    jl_bf16x8 q[2][2], part[2][CH_TERMS];
                     auto operands = [&](int s) {
                         q[s & 1][0] = row_of(Qs, l32, s);
                         q[s & 1][1] = row_of(Qs, 32 + l32, s);
-                        ch_split8(acc8(S[s >> 1], s & 1), part[s & 1]);
+                        jl_split8(acc8(S[s >> 1], s & 1), part[s & 1]);
                     };
                     operands(0);
 #pragma unroll
@@ -363,7 +343,7 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
 #pragma unroll
                 for (int r = 0; r < 16; ++r) p[0][r] = p[1][r] = p[2][r] = 0.f;
                 {
-                    ch_bf16x8 f[2][4];
+                    jl_bf16x8 f[2][4];
                     auto operands = [&](int s) {
                         f[s & 1][0] = row_of(Qs, l32, s); f[s & 1][1] = row_of(Qs, 32 + l32, s); f[s & 1][2] = row_of(Ks, l32, s); f[s & 1][3] = row_of(Ks, 32 + l32, s);
                     };
@@ -388,13 +368,13 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
 #pragma unroll
                 for (int s = 0; s < CH_T / 16; ++s) vf[s] = turned(Vs, VROW, 32 * wave, s);
                 {
-                    ch_bf16x8 part[2][CH_TERMS];
+                    jl_bf16x8 part[2][CH_TERMS];
                     const float li[2] = {Ls[l32], Ls[32 + l32]};
                     int ahead = l32 - 4 * hi;                       // the query's place less the lane's first key's, in a block on the diagonal
                     asm volatile("" : "+v"(ahead));                 // compared where it is used: sixteen masks kept would not fit the scalar registers
                     auto weights = [&](int n) {                     // half n % 2 of block n / 2: keys 32 kb .., queries 32 qb ..
                         const int b = n >> 1, s = n & 1, kb = b == 2, qb = b != 0;
-                        ch_f32x8 w = acc8(p[b], s);
+                        jl_f32x8 w = acc8(p[b], s);
 #pragma unroll
                         for (int x = 0; x < 2; ++x) {
                             const int j0 = 32 * kb + 16 * s + 8 * x + 4 * hi;
@@ -405,7 +385,7 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
                                 w[4 * x + y] = b == 1 || 16 * s + 8 * x + y <= ahead ? f : 0.f;
                             }
                         }
-                        ch_split8(w, part[n & 1]);
+                        jl_split8(w, part[n & 1]);
                     };
                     weights(0);
 #pragma unroll
@@ -431,16 +411,16 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
             for (int x = 0; x < NT; ++x)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) S[x][r] *= g;
-            ch_bf16x8 part[2][CH_TERMS], kf[2][NT];
+            jl_bf16x8 part[2][CH_TERMS], kf[2][NT];
             auto operands = [&](int s) {
-                ch_f32x8 w = __builtin_convertvector(vf[s], ch_f32x8);
+                jl_f32x8 w = __builtin_convertvector(vf[s], jl_f32x8);
 #pragma unroll
                 for (int x = 0; x < 2; ++x) {
                     const ch_f32x4 e4 = *(const ch_f32x4 *)(es + 16 * s + 8 * x + 4 * hi);
 #pragma unroll
                     for (int y = 0; y < 4; ++y) w[4 * x + y] *= e4[y];
                 }
-                ch_split8(w, part[s & 1]);
+                jl_split8(w, part[s & 1]);
 #pragma unroll
                 for (int x = 0; x < NT; ++x) kf[s & 1][x] = turned(Ks, QROW, 32 * x, s);
             };

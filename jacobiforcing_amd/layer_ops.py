@@ -651,13 +651,23 @@ def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: Ragged
     return out
 
 
+ROUTER_OUTPUTS, ROUTER_TOKENS = 64, 32 * 512      # beyond: the library's product, one launch for the choices and one workgroup for the grouping
 _ROUTES = {"sigmoid": N.JL_ROUTE_SIGMOID, "softmax_renorm": N.JL_ROUTE_SOFTMAX_RENORM, "top_softmax": N.JL_ROUTE_TOP_SOFTMAX}
 
 
-def moe_experts(h: torch.Tensor, router_logits: torch.Tensor, correction: Optional[torch.Tensor], top: int, scale: float,
+def _router_in_one(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """Whether the package's launches take the router product with the choice and the grouping: up to ROUTER_OUTPUTS outputs and ROUTER_TOKENS tokens, operands as ``linear`` takes them."""
+    return (x.dim() == 2 and 0 < x.shape[0] <= ROUTER_TOKENS and w.dim() == 2 and w.shape[0] <= ROUTER_OUTPUTS and x.dtype in _LINEAR_TYPES and w.dtype == torch.float32 and w.is_contiguous() and
+            w.shape[1] == x.shape[1] and x.shape[1] % 4 == 0 and x.shape[1] > 0 and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) * x.element_size() % 16 == 0 and
+            (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.get_device() == x.get_device() and
+            (bias is None or (bias.dtype == torch.float32 and bias.shape == (w.shape[0],) and bias.is_contiguous() and bias.get_device() == x.get_device())) and
+            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad))))
+
+
+def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correction: Optional[torch.Tensor], top: int, scale: float,
                 w_up: torch.Tensor, w_down: torch.Tensor, route: str = "sigmoid", renorm_eps: float = 0.0,
-                gated: Optional[Tuple[int, float, float, float]] = None, identity: int = 0):
-    """Routed experts: h [N, W], router_logits float [N, E], w_down [E, W, ff].  Returns the weighted expert outputs per choice,
+                gated: Optional[Tuple[int, float, float, float]] = None, identity: int = 0, router: Optional[Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]] = None):
+    """Routed experts: h [N, W], router_logits float [N, E] (or None and ``router`` = (x, w, bias) that they are ``linear``'s product of), w_down [E, W, ff].  Returns the weighted expert outputs per choice,
     float [N, top, W] (their sum over the middle axis is the layer's output).
 
     ``route`` "sigmoid": sigmoid scores, choice by score + correction, weights = score * scale; "softmax_renorm": softmax over all
@@ -674,7 +684,13 @@ def moe_experts(h: torch.Tensor, router_logits: torch.Tensor, correction: Option
     Er = E + identity
     up_rows = 2 * ff if gated is not None else ff
     dev, dt = h.device, h.dtype
-    _need(h.is_contiguous() and router_logits.dtype == torch.float32 and router_logits.is_contiguous() and tuple(router_logits.shape) == (n, Er) and identity >= 0,
+    in_one = router_logits is None and router is not None and _router_in_one(*router)
+    if in_one:
+        x, rw, rb = router
+        _need(x.shape[0] == n and rw.shape[0] == Er and x.get_device() == h.get_device(), "moe_experts: router (x [N, K], w [experts + identity experts, K], bias) of h's rows")
+    elif router_logits is None and router is not None:
+        router_logits = linear(*router, float_out=True)
+    _need(h.is_contiguous() and (in_one or (router_logits.dtype == torch.float32 and router_logits.is_contiguous() and tuple(router_logits.shape) == (n, Er))) and identity >= 0,
           "moe_experts: h [N, W], logits float [N, experts + identity experts]")
     _need(tuple(w_up.shape) == (E, up_rows, W) and tuple(w_down.shape) == (E, W, ff) and w_up.dtype == dt and w_down.dtype == dt and
           w_up.is_contiguous() and w_down.is_contiguous(), "moe_experts: expert weights [E, ff (2*ff when gated), W] / [E, W, ff] in the activation dtype")
@@ -684,30 +700,41 @@ def moe_experts(h: torch.Tensor, router_logits: torch.Tensor, correction: Option
     L, st = N.layers(), _stream(dev)
     ids = torch.empty((n, top), dtype=torch.int32, device=dev)
     wts = torch.empty((n, top), dtype=torch.float32, device=dev)
-    N.check_layers(L.jl_moe_route(_ptr(router_logits), _ptr(correction), n, Er, top, float(scale), _ptr(ids), _ptr(wts),
-                                  _ROUTES[route], float(renorm_eps), st), "jl_moe_route")
     rows = n * top
     tm = int(L.jl_moe_tile_rows(_code(dt), rows, E, W, ff))
     if tm == 128 and L.jl_moe_tile_pairs(rows, E, W, ff, int(gated is not None)):
         tm = 256
     max_tiles = rows // tm + E
-    perm = torch.empty((rows,), dtype=torch.int32, device=dev)
-    offsets = torch.empty((E + 2,), dtype=torch.int32, device=dev)
-    tile_e = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
-    tile_r = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
-    N.check_layers(L.jl_moe_group(_ptr(ids), n, top, E, tm, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, st), "jl_moe_group")
+    from_logits = not in_one and 0 < n <= ROUTER_TOKENS and Er <= ROUTER_OUTPUTS
+    blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
+    lists = torch.empty((rows + E + 2 + 2 * max_tiles + blocks * E,), dtype=torch.int32, device=dev)       # the grouping's lists, one behind the other
+    perm = lists.data_ptr()
+    offsets = perm + 4 * rows
+    tile_e = offsets + 4 * (E + 2)
+    tile_r = tile_e + 4 * max_tiles
+    if from_logits:
+        x, rw, rb = router_logits, None, None
+    if in_one or from_logits:
+        a = N.MoeRouter(x=x.data_ptr(), w=_ptr(rw), bias=_ptr(rb), correction=_ptr(correction), ids=ids.data_ptr(), weights=wts.data_ptr(), perm=perm, offsets=offsets, tile_expert=tile_e,
+                        tile_row0=tile_r, counts=tile_r + 4 * max_tiles, N=n, x_ld=x.stride(0), x_dtype=_code(x.dtype), K=x.shape[1], E=Er, experts=E, top=top, kind=_ROUTES[route],
+                        tile_rows=tm, max_tiles=max_tiles, scale=float(scale), renorm_eps=float(renorm_eps))
+        N.check_layers(L.jl_moe_router_run(C.byref(a), st), "jl_moe_router_run")
+    else:
+        N.check_layers(L.jl_moe_route(_ptr(router_logits), _ptr(correction), n, Er, top, float(scale), _ptr(ids), _ptr(wts),
+                                      _ROUTES[route], float(renorm_eps), st), "jl_moe_route")
+        N.check_layers(L.jl_moe_group(_ptr(ids), n, top, E, tm, perm, offsets, tile_e, tile_r, max_tiles, st), "jl_moe_group")
     if gated is not None and not os.environ.get("JL_MOE_UNFUSED_ACT"):          # the unit in the product's epilogue (A/B switch for measurements)
         act = torch.empty((rows, ff), dtype=dt, device=dev)
-        N.check_layers(L.jl_moe_gemm_gated(_ptr(h), _ptr(w_up), _code(dt), W, ff, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm,
+        N.check_layers(L.jl_moe_gemm_gated(_ptr(h), _ptr(w_up), _code(dt), W, ff, top, perm, offsets, tile_e, tile_r, max_tiles, E, tm,
                                            int(gated[0]), float(gated[1]), float(gated[2]), float(gated[3]), _ptr(act), st), "jl_moe_gemm_gated")
     else:
         act = torch.empty((rows, up_rows), dtype=dt, device=dev)
-        N.check_layers(L.jl_moe_gemm(_ptr(h), _ptr(w_up), _code(dt), N.JL_MOE_UP_PLAIN if gated is not None else N.JL_MOE_UP_RELU2, W, up_rows, top, _ptr(perm),
-                                     _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm, None, _ptr(act), st), "jl_moe_gemm(up)")
+        N.check_layers(L.jl_moe_gemm(_ptr(h), _ptr(w_up), _code(dt), N.JL_MOE_UP_PLAIN if gated is not None else N.JL_MOE_UP_RELU2, W, up_rows, top, perm,
+                                     offsets, tile_e, tile_r, max_tiles, E, tm, None, _ptr(act), st), "jl_moe_gemm(up)")
         if gated is not None:
             act = gated_act(act, 0, ff, ff, *gated)
     y = torch.empty((n, top, W), dtype=torch.float32, device=dev)
-    N.check_layers(L.jl_moe_gemm(_ptr(act), _ptr(w_down), _code(dt), N.JL_MOE_DOWN, ff, W, top, _ptr(perm), _ptr(offsets), _ptr(tile_e), _ptr(tile_r), max_tiles, E, tm,
+    N.check_layers(L.jl_moe_gemm(_ptr(act), _ptr(w_down), _code(dt), N.JL_MOE_DOWN, ff, W, top, perm, offsets, tile_e, tile_r, max_tiles, E, tm,
                                  _ptr(wts), _ptr(y), st), "jl_moe_gemm(down)")
     return (y, ids, wts) if identity else y
 

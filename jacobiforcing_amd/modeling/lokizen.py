@@ -269,8 +269,7 @@ class LokizenModel:
             if L.get("mlp") is not None:
                 r = L["mlp"]["router"]
                 h2 = LO.add_rmsnorm(x, pending, None, lw["norm2"], eps, dt)
-                pending = LO.moe_experts(h2, LO.linear(h2, lw["router"], float_out=True), lw["correction"], int(r["top"]), float(r["scale"]),
-                                         lw["w_up"], lw["w_down"])
+                pending = LO.moe_experts(h2, None, lw["correction"], int(r["top"]), float(r["scale"]), lw["w_up"], lw["w_down"], router=(h2, lw["router"], None))
             if trace is not None:
                 LO.add_rmsnorm(x, pending, None, None, eps, None)
                 pending = None

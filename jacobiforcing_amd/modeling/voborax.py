@@ -257,8 +257,8 @@ class VoboraxModel:
             z = LO.linear(h, w["w_up"], w["b_up"])
             return [(LO.linear(LO.gated_act(z, 0, -1, z.shape[1], LO.ACT_GELU_TANH), w["w_down"], w["b_down"]), None)], None
         E, ident = _experts(f)
-        y = LO.moe_experts(h, LO.linear(x, w["router"]), w["correction"], int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
-                           renorm_eps=ROUTER_RENORM_EPS, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0), identity=ident)
+        y = LO.moe_experts(h, None, w["correction"], int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
+                           renorm_eps=ROUTER_RENORM_EPS, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0), identity=ident, router=(x, w["router"], None))
         y, choices = (y[0], (y[1], y[2], E)) if ident else (y, None)
         out = [(y, None)]
         if f.get("shared") is not None:

@@ -1,0 +1,67 @@
+"""The experts' router product, choice and grouping in one call: the same choices, weights and outputs, bit for bit, as from logits handed in.  Operands are small whole numbers, so that every
+order of the sums is exact and ties are many."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def run(monkeypatch, N, K, E, identity, top, x_dtype, bias, route, pad=0, gated=False):
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(N + K + E)
+    whole = lambda lim, *s: torch.randint(-lim, lim + 1, s, generator=g, device="cuda")
+    Er, W, ff = E + identity, 64, 32
+    x = whole(4, N, K + pad).to(x_dtype)[:, :K]
+    w = (whole(4, Er, K) / 256).float()                                        # K * 16 / 256 in steps of 1 / 256: exact in 24 bits
+    b = (whole(8, Er) / 16).float() if bias else None
+    corr = (whole(8, Er) / 32).float() if route != "top_softmax" else None
+    h = torch.randn(N, W, generator=g, device="cuda").bfloat16()
+    up, down = torch.randn(E, (2 if gated else 1) * ff, W, generator=g, device="cuda").bfloat16(), torch.randn(E, W, ff, generator=g, device="cuda").bfloat16()
+    logits = x.double() @ w.double().T
+    logits = (logits if b is None else logits + b.double()).float()
+    kw = dict(route=route, renorm_eps=1e-20, identity=identity, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0) if gated else None)
+    with monkeypatch.context() as m:
+        m.setattr(LO, "ROUTER_OUTPUTS", 0)                                     # choice and grouping in launches of their own
+        want = LO.moe_experts(h, logits, corr, top, 0.5, up, down, **kw)
+    for got in (LO.moe_experts(h, logits, corr, top, 0.5, up, down, **kw), LO.moe_experts(h, None, corr, top, 0.5, up, down, router=(x, w, b), **kw)):
+        if not identity:
+            assert torch.equal(got, want)
+            continue
+        real = want[1] < E
+        assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2]) and torch.equal(got[0][real], want[0][real])
+    return LO._router_in_one(x, w, b)
+
+
+@pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K,E,identity,top,bias,route,pad", [
+    (1, 64, 1, 0, 1, False, "sigmoid", 0), (16, 1024, 16, 0, 4, True, "top_softmax", 0), (17, 2048, 17, 5, 3, False, "softmax_renorm", 8), (32, 36, 33, 7, 4, True, "softmax_renorm", 28),
+    (33, 512, 48, 16, 8, False, "sigmoid", 0), (64, 4, 7, 1, 2, True, "top_softmax", 4), (1000, 200, 9, 0, 9, False, "softmax_renorm", 0), (4097, 1032, 32, 0, 4, True, "top_softmax", 0),
+    (8192, 128, 24, 6, 4, False, "sigmoid", 0), (16384, 32, 64, 0, 2, False, "softmax_renorm", 0), (40, 64, 3, 61, 64, False, "softmax_renorm", 0),
+])
+def test_the_same_as_from_logits(monkeypatch, x_dtype, N, K, E, identity, top, bias, route, pad):
+    """One workgroup and many, one to four blocks of outputs, depths beside whole lines, rows apart, experts without rows, choices of all outputs."""
+    assert run(monkeypatch, N, K, E, identity, top, x_dtype, bias, route, pad), "the launches did not run"
+
+
+@pytest.mark.parametrize("N,K,E", [(16385, 16, 4), (20, 30, 8), (50, 64, 65)])
+def test_what_the_launches_do_not_take(monkeypatch, N, K, E):
+    """More tokens, depths beside 16-byte borders, more outputs: the product, the choice and the grouping one after the other."""
+    assert not run(monkeypatch, N, K, E, 0, 2, torch.float32, True, "top_softmax")
+
+
+@pytest.mark.parametrize("route", ["sigmoid", "softmax_renorm", "top_softmax"])
+def test_logits_that_are_not_finite(monkeypatch, route):
+    """Infinities are chosen (or not) as before; a token with one that is not a number shows it in its outputs, and no other token does."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(3)
+    N, E, W, ff = 70, 6, 64, 32
+    h, up, down = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((N, W), (E, ff, W), (E, W, ff)))
+    z = torch.randn(N, E, generator=g, device="cuda")
+    z[3, 2], z[4, 1], z[5] = float("inf"), -float("inf"), -float("inf")
+    with monkeypatch.context() as m:
+        m.setattr(LO, "ROUTER_OUTPUTS", 0)
+        want = LO.moe_experts(h, z, None, 2, 1.0, up, down, route=route)
+    assert torch.equal(LO.moe_experts(h, z, None, 2, 1.0, up, down, route=route).nan_to_num(7.0), want.nan_to_num(7.0))
+    z[9, 4] = float("nan")
+    y = LO.moe_experts(h, z, None, 2, 1.0, up, down, route=route)
+    assert y[9].isnan().any() and torch.equal(torch.cat([y[:9], y[10:]]).nan_to_num(7.0), torch.cat([want[:9], want[10:]]).nan_to_num(7.0))
