@@ -30,12 +30,13 @@ NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, a
                                       # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
 NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
                                       # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
-BLOCK_WORKGROUPS = 384               # a draft block's attention: wavefronts of 32 columns to aim at when keys are shared out
+BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
-RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches, 4 x 2048 of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
+RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
-SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches, 4 x 2048 of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
+SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches,
+                                            # 4 x 2048 tokens of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
 DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (alone in its step; else delta_chunks_from.  us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
 DELTA_SCRATCH_FLOATS = 256 << 20     # scratch of those chunks at most (1 GiB: more heads than it holds take turns), as long as it holds one key head's
@@ -70,6 +71,35 @@ def _dev(t: torch.Tensor) -> None:
         raise N.NativeLibraryError("the layer kernels run on the GPU only (no CPU fallback)")
 
 
+_UPLOADS: dict = {}                                  # device index -> the stream its tables are copied on, and a block of its pool
+
+
+def _upload(host: np.ndarray, device) -> torch.Tensor:
+    """``host`` on ``device``, there when this returns.  A copy from ordinary host memory waits for its stream: on one of its own it waits for itself and not for the kernels queued so far (a
+    decoding step of 32 requests, kernels of 500 us: 650 -> 520 us a pass).  The memory goes back to that stream's pool once the current stream is done with it."""
+    device = torch.device(device)
+    t = torch.from_numpy(host)
+    if device.type != "cuda":
+        return t.to(device)
+    index = torch.cuda.current_device() if device.index is None else device.index
+    if index not in _UPLOADS:
+        side = torch.cuda.Stream(index)
+        with torch.cuda.stream(side):                    # a block that stays keeps the pool's first segment (2 MB) from being given back and asked for again
+            _UPLOADS.setdefault(index, (side, torch.empty(1, dtype=torch.int32, device=device)))
+    side, user = _UPLOADS[index][0], torch.cuda.current_stream(index)
+    if index == torch.cuda.current_device():             # half of what the context below takes
+        torch.cuda.set_stream(side)
+        try:
+            up = t.to(device)
+        finally:
+            torch.cuda.set_stream(user)
+    else:
+        with torch.cuda.stream(side):
+            up = t.to(device)
+    up.record_stream(user)
+    return up
+
+
 @dataclass
 class RaggedBatch:
     """What one step runs: requests b = 0..B-1 with ``counts[b]`` new tokens from position ``starts[b]``, state slot ``slots[b]``
@@ -90,43 +120,50 @@ class RaggedBatch:
     max_slot: int
     slots: List[int]
     _tiles: dict
+    _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
     _host_tables: Optional[np.ndarray] = None         # tables on the host, for key_rows and part (None: read back when they need it)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
               page_size: int, device) -> "RaggedBatch":
         B = len(counts)
-        row0 = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
-        seq = np.stack([row0[:-1], np.asarray(counts), np.asarray(starts), np.asarray(slots)], 1).astype(np.int32).reshape(B, 4)
-        C_ = max(1, max(len(t) for t in block_tables))
-        bt = np.full((B, C_), -1, dtype=np.int32)
-        kv = np.empty(int(row0[-1]), dtype=np.int64)
-        row_pos = np.empty(int(row0[-1]), dtype=np.int32)
+        held = list(map(len, block_tables))              # pages of each request
         for b in range(B):
-            t = np.asarray(block_tables[b], dtype=np.int64)
-            bt[b, :t.size] = t
-            pos = starts[b] + np.arange(counts[b], dtype=np.int64)
-            if counts[b] and (starts[b] + counts[b] + page_size - 1) // page_size > t.size:
-                raise ValueError(f"request {b}: {t.size} pages do not hold {starts[b] + counts[b]} tokens")
-            kv[row0[b]:row0[b + 1]] = t[pos // page_size] * page_size + pos % page_size
-            row_pos[row0[b]:row0[b + 1]] = pos
-        # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on
-        tables = [seq.ravel(), bt.ravel(), np.repeat(np.arange(B, dtype=np.int32), np.asarray(counts, dtype=np.int64)), row_pos]
-        at = [2 * (kv.size + kv.size % 2)]
-        for t in tables:
-            at.append(at[-1] + (t.size + 3) // 4 * 4)
+            if counts[b] and (starts[b] + counts[b] + page_size - 1) // page_size > held[b]:
+                raise ValueError(f"request {b}: {held[b]} pages do not hold {starts[b] + counts[b]} tokens")
+        counts, starts, slots = list(map(int, counts)), list(map(int, starts)), list(map(int, slots))
+        row0 = list(itertools.accumulate(counts, initial=0))
+        N_, C_ = row0[B], max(1, max(held))
+        # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on; `whole`: tiles() of steps whose requests are one tile each
+        seq = [x for r in zip(row0, counts, starts, slots) for x in r]
+        whole = [x for r in zip(range(B), starts, counts, row0) for x in r]
+        sizes = (4 * B, B * C_, N_, N_, 4 * B)
+        at = list(itertools.accumulate(((n + 3) // 4 * 4 for n in sizes), initial=2 * (N_ + N_ % 2)))
         host = np.empty(at[-1] // 2, dtype=np.int64)
-        host[:kv.size] = kv
         words = host.view(np.int32)
-        for t, a in zip(tables, at):
-            words[a:a + t.size] = t
-        up = torch.from_numpy(host).to(torch.device(device))
+        a_seq, a_bt, a_req, a_pos, a_whole = at[:5]
+        words[a_seq:a_seq + 4 * B], words[a_whole:a_whole + 4 * B] = seq, whole
+        bt = words[a_bt:a_bt + B * C_].reshape(B, C_)
+        pages = np.fromiter(itertools.chain.from_iterable(block_tables), dtype=np.int64, count=sum(held))
+        if min(held) == C_:
+            bt[:] = pages.reshape(B, C_)
+        else:
+            bt[:] = -1
+            bt[np.arange(C_) < np.asarray(held)[:, None]] = pages
+        if N_ == B and min(counts) == 1:                 # decoding: a row per request
+            words[a_req:a_req + N_], words[a_pos:a_pos + N_] = range(B), starts
+            host[:N_] = [int(t[s // page_size]) * page_size + s % page_size for t, s in zip(block_tables, starts)]
+        elif N_:
+            c = np.asarray(counts)
+            pos = np.arange(N_, dtype=np.int64) + np.repeat(np.asarray(starts) - row0[:B], c)
+            words[a_req:a_req + N_], words[a_pos:a_pos + N_] = np.repeat(np.arange(B, dtype=np.int32), c), pos
+            host[:N_] = pages[np.repeat(np.cumsum(held) - held, c) + pos // page_size] * page_size + pos % page_size
+        up = _upload(host, device)
         w32 = up.view(torch.int32)
-        d_seq, d_bt, d_req, d_pos = (w32[a:a + t.size] for t, a in zip(tables, at))
-        return cls(B=B, N=int(row0[-1]), counts=list(map(int, counts)), starts=list(map(int, starts)),
-                   seq=d_seq.view(B, 4), kv_slot=up[:kv.size], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos,
-                   page_size=int(page_size), max_pos=max(int(s) + int(c) for s, c in zip(starts, counts)), max_page=int(bt.max()),
-                   max_slot=int(max(slots)), slots=list(map(int, slots)), _tiles={}, _host_tables=bt)
+        d_seq, d_bt, d_req, d_pos, d_whole = (w32[a:a + n] for n, a in zip(sizes, at))
+        return cls(B=B, N=N_, counts=counts, starts=starts, seq=d_seq.view(B, 4), kv_slot=up[:N_], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos, page_size=int(page_size),
+                   max_pos=max(s + c for s, c in zip(starts, counts)), max_page=int(bt.max()), max_slot=max(slots), slots=slots, _tiles={}, _host_tables=bt,
+                   _whole=(max(counts), d_whole.view(B, 4)) if min(counts) > 0 else None)
 
     def chunks(self, size: int):
         """A portion of at least two chunks is cut into chunks of ``size`` tokens that the recurrent layers run side by side.
@@ -144,8 +181,7 @@ class RaggedBatch:
                         rec.append((int(seq[b, 0]) + o, min(size, c - o), s + o, len(rec)))
                 dev = self.seq.device
                 rec = np.asarray(rec, dtype=np.int32).reshape(-1, 4)
-                plan = (torch.from_numpy(rec).to(dev), torch.from_numpy(np.ascontiguousarray(rec[:, 1])).to(dev),
-                        torch.from_numpy(np.asarray(req, dtype=np.int32).reshape(-1, 4)).to(dev))
+                plan = (_upload(rec, dev), _upload(np.ascontiguousarray(rec[:, 1]), dev), _upload(np.asarray(req, dtype=np.int32).reshape(-1, 4), dev))
             self._tiles[key] = plan
         return self._tiles[key]
 
@@ -159,7 +195,7 @@ class RaggedBatch:
                 req.append((len(rec), -(-c // size), s, sl))
                 rec += [(r0 + o, min(size, c - o), sl, int(o + size >= c)) for o in range(0, c, size)]
                 r0 += c
-            both = torch.tensor(rec + req, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
+            both = _upload(np.asarray(rec + req, dtype=np.int32).reshape(-1, 4), self.seq.device)
             self._tiles[key] = (both[:len(rec)], both[len(rec):])
         return self._tiles[key]
 
@@ -175,7 +211,7 @@ class RaggedBatch:
                 else:
                     rest.append((r0, c, s, sl))
                 r0 += c
-            every = torch.tensor(rec + req + rest, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
+            every = _upload(np.asarray(rec + req + rest, dtype=np.int32).reshape(-1, 4), self.seq.device)
             self._tiles[key] = (every[:len(rec)], every[len(rec):len(rec) + len(req)], every[len(rec) + len(req):], max((r[1] for r in rest), default=0))
         return self._tiles[key]
 
@@ -202,7 +238,7 @@ class RaggedBatch:
                 host[at:at + end - first] = (pages[b, p0:(end - 1) // size + 1, None] + within).ravel()[first - p0 * size:end - p0 * size]
                 base[b] = at - first
                 at += end - first
-            up = torch.from_numpy(host).to(self.seq.device)
+            up = _upload(host, self.seq.device)
             self._tiles[key] = (up[:total], up[total:].view(torch.int32)[:self.B])
         return self._tiles[key]
 
@@ -214,7 +250,7 @@ class RaggedBatch:
             rows = np.concatenate([np.arange(row0[b], row0[b + 1], dtype=np.int64) for b in requests])
             sub = RaggedBatch.build([self.counts[b] for b in requests], [self.starts[b] for b in requests], [self.slots[b] for b in requests],
                                     [self._pages()[b] for b in requests], self.page_size, self.seq.device)
-            self._tiles[key] = (sub, torch.from_numpy(rows).to(self.seq.device))
+            self._tiles[key] = (sub, _upload(rows, self.seq.device))
         return self._tiles[key]
 
     def tiles(self, tq: int, longest_first: bool = False, requests: Optional[Sequence[int]] = None) -> torch.Tensor:
@@ -222,6 +258,8 @@ class RaggedBatch:
         ``longest_first`` those with the most positions in front of them come first; only those of ``requests`` when given."""
         key = ("longest first" if longest_first else "in order", tq, None if requests is None else tuple(requests)) if longest_first or requests is not None else tq
         t = self._tiles.get(key)
+        if t is None and key == tq and self._whole is not None and self._whole[0] <= tq:
+            t = self._tiles[key] = self._whole[1]        # came with the batch's own upload
         if t is None:
             rows, r0 = [], 0
             for b, (c, s) in enumerate(zip(self.counts, self.starts)):
@@ -230,7 +268,7 @@ class RaggedBatch:
                 r0 += c
             if longest_first:
                 rows.sort(key=lambda r: -r[1])
-            t = self._tiles[key] = torch.tensor(rows, dtype=torch.int32, device=self.seq.device).reshape(-1, 4)
+            t = self._tiles[key] = _upload(np.asarray(rows, dtype=np.int32).reshape(-1, 4), self.seq.device)
         return t
 
 
