@@ -177,7 +177,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *__restri
 // 128 rows need both products to fill the chip and about a tile of rows per expert; 64 need as many blocks as the chip takes at once.  Measured, experts alone, gated,
 // bfloat16, us at 32 / 64 / 128 rows: 8192 tokens x 4 of 32 (2048 x 1024) 1059 / 790 / 623, 1024 tokens 213 / 171 / 160, 512 tokens 147 / 140 / 155, 256 tokens 121 / 124 / 142;
 // 4096 x 4 of 16 (1024 x 512) 180 / 135 / 123, 1024 tokens 75 / 66 / 79, 512 tokens 51 / 57 / 77; 4096 x 4 of 12 (768 x 512) 151 / 117 / 104, 2048 tokens 95 / 77 / 80;
-// float, 2048 x 4 of 16 (1024 x 512): 341 / 311 / 401.
+// float, 2048 x 4 of 16 (1024 x 512): 341 / 311 / 401.  (The tiles of 32 rows have become faster since, by 7 % at 256 tokens of the first.)
 // Sizes the matrix-core product does not take (rows that do not start at 16-byte borders) go in tiles of MOE_TM.
 static bool moe_mm_sizes(int dtype, int64_t K) { return (dtype == JL_BF16 && K % 8 == 0) || (dtype == JL_F32 && K % 4 == 0); }
 extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff) {
@@ -523,8 +523,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
 // (16 bytes per lane, every lane fetching the unit that the permutation puts into its place), one stage ahead: no registers and no LDS writes for them, so that three workgroups fit a
 // CU and cover each other's barriers (through registers, two of them: gated product at 8192 x 4 of 32 experts of 2048 x 1024 406 -> 363 us, the way down 290 -> 252).  More stages ahead in fewer
 // workgroups change nothing; without their loads the two products take 238 and 160 us, without their products 335 and 200, so where rows are many the gated one goes in larger tiles (below).
-// Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an expert's weights are read into one L2.  TM = 32 (decoding) is bound by reading
-// the weights: single wavefronts, many per CU, 12 KB on the way each, in registers.
+// Workgroups of an XCD (every eighth) take neighbouring tiles and all their columns, so that an expert's weights are read into one L2.  Tiles of 32 rows (decoding) have a kernel of
+// their own.
 // Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from a base (of the tile where its rows lie together; FAR: rows gathered from more than
 // 4 GiB have 64-bit addresses), rows that do not exist repeat another, stages behind the last repeat the
 // first, depths beyond the last whole stage come after the loop (a condition per load had cost six vector instructions per product: 431 us instead of 406 for the gated product
@@ -607,25 +607,18 @@ __device__ __forceinline__ void moe_store(const MoeMM &a, const mm_f32x16 (&acc)
 }
 
 template <typename T, int TM, int NW, int WR, int TKU, bool GATED, bool FAR>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM a) {
+__global__ __launch_bounds__(64 * NW, 3) void moe_mm_kernel(MoeMM a) {
     constexpr int THREADS = 64 * NW, UNIT = mm_type<T>::UNIT, WM = TM == 128 ? 2 : 1, WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32;
     constexpr int XPF = TM * TKU / THREADS, WPF = WR * TKU / THREADS, TN = GATED ? WR / 2 : WR, STAGE = TKU * UNIT;
     static_assert(XPF * THREADS == TM * TKU && WPF * THREADS == WR * TKU && (!GATED || NT % 2 == 0), "tile");
     __shared__ uint4 smem[2 * (TM + WR) * TKU];
     __shared__ int rows_out[TM];                                    // way down: the flat indices and weights of the tile's rows
     __shared__ float rows_weight[TM];
-    int tile, col, part = 0;
-    if (TM >= 64) {                                                 // workgroups with the same remainder by 8 share an XCD
-        const int per_xcd = (a.offsets[a.E + 1] + 7) / 8, xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
-        if (s >= per_xcd * a.col_blocks * a.parts) return;
-        tile = xcd * per_xcd + s / (a.col_blocks * a.parts);
-        part = s / a.col_blocks % a.parts;
-        col = s % a.col_blocks;
-        if (tile >= a.max_tiles) return;
-    } else {
-        tile = blockIdx.x / a.col_blocks;
-        col = blockIdx.x - tile * a.col_blocks;
-    }
+    // workgroups with the same remainder by 8 share an XCD
+    const int per_xcd = (a.offsets[a.E + 1] + 7) / 8, xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
+    if (s >= per_xcd * a.col_blocks * a.parts) return;
+    const int tile = xcd * per_xcd + s / (a.col_blocks * a.parts), part = s / a.col_blocks % a.parts, col = s % a.col_blocks;
+    if (tile >= a.max_tiles) return;
     const int e = a.tile_expert[tile];
     if (e < 0) return;
     const int r0 = a.tile_row0[tile] + part * TM, K = a.K, n_out = a.n_out, n0 = col * TN;
@@ -641,8 +634,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
         }
     // loaders: unit tid % TKU of rows tid / TKU + x * THREADS / TKU; a row that does not exist repeats another and is not stored
     const int lr = tid / TKU;
-    constexpr bool DMA = NW > 1;
-    auto unit_of = [&](int x) { return DMA ? at(lr + x * (THREADS / TKU), tid % TKU) % TKU : tid % TKU; };      // DMA: what belongs into this thread's place of LDS
+    auto unit_of = [&](int x) { return at(lr + x * (THREADS / TKU), tid % TKU) % TKU; };      // what belongs into this thread's place of LDS
     // byte offsets from a base that is the same for all lanes: a load is one instruction (the launch has checked that 32 bits hold them)
     uint32_t xo[XPF], wo[WPF];
     const char *xfar[FAR ? XPF : 1];
@@ -662,26 +654,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
         wo[x] = (uint32_t)((n0 + c < n_out ? c : n_out - 1 - n0) * (int64_t)K + unit_of(x) * UNIT) * sizeof(T);
     }
     auto w_base = [&](int x) { return GATED && x >= WPF / 2 ? Wl : Wb; };
-    mm_u32x4 reg[DMA ? 1 : 2][XPF + WPF];                                     // stages on their way: even ones in reg[0], odd ones in reg[1]
     const int full = K / STAGE;                                     // whole stages; what is left of K comes last
-    auto fetch = [&](mm_u32x4 (&r)[XPF + WPF], int i) {             // without branches: behind the last stage, stage 0 again (never used)
-        const int64_t k = i < full ? (int64_t)i * STAGE * sizeof(T) : 0;
-        const char *xb = Xb + k;
-#pragma unroll
-        for (int x = 0; x < XPF; ++x) {
-            if constexpr (FAR) r[x] = *(const mm_u32x4 *)(xfar[x] + k);
-            else r[x] = *(const mm_u32x4 *)(xb + xo[x]);
-        }
-#pragma unroll
-        for (int x = 0; x < WPF; ++x) r[XPF + x] = *(const mm_u32x4 *)(w_base(x) + k + wo[x]);
-    };
-    auto stash = [&](const mm_u32x4 (&r)[XPF + WPF], int sel) {
-        uint4 *Xs = smem + sel * (TM + WR) * TKU, *Ws = Xs + TM * TKU;
-#pragma unroll
-        for (int x = 0; x < XPF; ++x) Xs[at(lr + x * (THREADS / TKU), unit_of(x))] = __builtin_bit_cast(uint4, r[x]);
-#pragma unroll
-        for (int x = 0; x < WPF; ++x) Ws[at(lr + x * (THREADS / TKU), unit_of(x))] = __builtin_bit_cast(uint4, r[XPF + x]);
-    };
     mm_f32x16 acc[XT][NT];
 #pragma unroll
     for (int x = 0; x < XT; ++x)
@@ -708,7 +681,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
 
         }
     };
-    if (DMA && full > 0) {
+    if (full > 0) {
         // straight into LDS: a wavefront's 64 places of 16 bytes per load, one stage ahead
         const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(smem + wave * 64));
         auto issue = [&](int i, int sel) {
@@ -731,27 +704,6 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-    } else if (full > 0) {
-        fetch(reg[0], 0);
-        constexpr int R1 = DMA ? 0 : 1;
-        fetch(reg[R1], 1);
-        stash(reg[0], 0);
-        __syncthreads();
-        int i = 0;
-        for (; i + 1 < full; i += 2) {                              // two stages ahead: a trip to memory takes longer than one stage's products
-            fetch(reg[0], i + 2);
-            products(0);
-            stash(reg[R1], 1);
-            __syncthreads();
-            fetch(reg[R1], i + 3);
-            products(1);
-            stash(reg[0], 0);
-            __syncthreads();
-        }
-        if (i < full) {
-            products(0);
-            __syncthreads();
-        }
     }
     if (full * STAGE < K) {                                         // depths beyond K are zero
         const mm_u32x4 zero = {0, 0, 0, 0};
@@ -761,15 +713,142 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 1) void moe_mm_kernel(MoeMM 
             return in ? v : zero;
         };
 #pragma unroll
-        for (int x = 0; x < XPF; ++x) reg[0][x] = last(FAR ? xfar[FAR ? x : 0] : Xb + xo[x], unit_of(x));
+        for (int x = 0; x < XPF; ++x) smem[tid + x * THREADS] = __builtin_bit_cast(uint4, last(FAR ? xfar[FAR ? x : 0] : Xb + xo[x], unit_of(x)));
 #pragma unroll
-        for (int x = 0; x < WPF; ++x) reg[0][XPF + x] = last(w_base(x) + wo[x], unit_of(x));
-        stash(reg[0], 0);
+        for (int x = 0; x < WPF; ++x) smem[tid + (XPF + x) * THREADS] = __builtin_bit_cast(uint4, last(w_base(x) + wo[x], unit_of(x)));
         __syncthreads();
         products(0);
     }
     moe_store<T, XT, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int x, int k, int &p, float &w) { const int m = wm * (TM / WM) + 32 * x + k; p = rows_out[m]; w = rows_weight[m]; },
                                 [&](int x) { return wm * (TM / WM) + 32 * x; }, w_row, lane);
+}
+
+// ---- the same product for few rows per expert (decoding): 32 rows by 64 weight rows, the depth shared by two or four wavefronts ----------------------
+// What bounds it is reading the weights, and with few tiles the way there: one wavefront has 24 KB of its share of the depth on the way in registers, passes it through LDS of its own (no barrier) into the
+// products, and the shares meet in the end.  Rows of x come eight at a time, as many as there are.  (Three workgroups of four per CU do not fit the registers: spills, 106 us for the first line.)
+// us of both products, gated, weights from memory, one wavefront with all of the depth / two / four: 32 rows x 4 of 32 of 2048 x 1024 92 / 79 / 80 (402 MB: 5.0 TB/s), 1 x 4 of the same 28 / 21 / 19, 32 x 4 of
+// 16 of 1024 x 512 (plain) 22 / 18 / 16, 100 x 3 of 24 of 1536 x 704 37 / 37 / 41, 400 x 4 of 16 (plain) 27 / 25 / 28; float, 16 x 4 of 16 of 1024 x 512 62 / 38 / 27, 150 x 4 66 / 65 / 46.
+template <typename T, int MF_NW, bool GATED, bool FAR>
+__global__ __launch_bounds__(64 * MF_NW, 2) void moe_few_kernel(MoeMM a) {
+    constexpr int TM = 32, WR = 64, TKU = 8, NT = 2, XPF = TM * TKU / 64, WPF = WR * TKU / 64, TN = GATED ? WR / 2 : WR, UNIT = mm_type<T>::UNIT, STAGE = TKU * UNIT, OWN = (TM + WR) * TKU;
+    __shared__ uint4 smem[MF_NW * OWN];
+    __shared__ int rows_out[TM];                                    // way down: the flat indices and weights of the tile's rows
+    __shared__ float rows_weight[TM];
+    const int tile = blockIdx.x / a.col_blocks, e = a.tile_expert[tile];
+    if (e < 0) return;
+    const int r0 = a.tile_row0[tile], K = a.K, n_out = a.n_out, n0 = (int)(blockIdx.x - tile * a.col_blocks) * TN, left = a.offsets[e + 1] - r0, nr = left < TM ? left : TM;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
+    if (!GATED && a.mode == 1 && (int)threadIdx.x < nr) {
+        const int p = a.perm[r0 + threadIdx.x];
+        rows_out[threadIdx.x] = p;
+        rows_weight[threadIdx.x] = a.weights[p];
+    }
+    auto at = [](int row, int u) { return row * TKU + (u ^ ((row >> 1) & 7)); };
+    // loaders: unit lane % 8 of rows lane / 8 + 8 x; a row that does not exist repeats another and is not stored.  Byte offsets from a base that is the same for all lanes
+    const int lr = lane / TKU, lu = lane % TKU;
+    uint32_t xo[XPF], wo[WPF];
+    const char *xfar[FAR ? XPF : 1];
+    const char *Xb = (const char *)((const T *)a.X + (a.mode != 1 ? 0 : (int64_t)r0 * K));
+#pragma unroll
+    for (int x = 0; x < XPF; ++x) {
+        const int m = lr + 8 * x, row = m < nr ? m : 0;
+        const int64_t at_x = (a.mode != 1 ? a.perm[r0 + row] / a.top : row) * (int64_t)K + lu * UNIT;
+        if constexpr (FAR) xfar[x] = Xb + at_x * sizeof(T);
+        xo[x] = (uint32_t)at_x * sizeof(T);
+    }
+    const char *Wb = (const char *)((const T *)a.Wt + ((int64_t)e * (GATED ? 2 : 1) * n_out + n0) * K), *Wl = Wb + (int64_t)(GATED ? n_out : 0) * K * sizeof(T);
+#pragma unroll
+    for (int x = 0; x < WPF; ++x) {
+        const int j = lr + 8 * x, c = GATED ? j % TN : j;
+        wo[x] = (uint32_t)((n0 + c < n_out ? c : n_out - 1 - n0) * (int64_t)K + lu * UNIT) * sizeof(T);
+    }
+    auto w_base = [&](int x) { return GATED && x >= WPF / 2 ? Wl : Wb; };
+    const int full = K / STAGE, s0 = full * wave / MF_NW, s1 = full * (wave + 1) / MF_NW;      // whole stages; what is left of K is the last wavefront's
+    mm_u32x4 reg[2][XPF + WPF];
+    auto fetch = [&](mm_u32x4 (&r)[XPF + WPF], int i) {             // behind the last stage, the first again (never used)
+        const int64_t k = i < s1 ? (int64_t)i * STAGE * sizeof(T) : 0;
+#pragma unroll
+        for (int x = 0; x < XPF; ++x) {
+            if (8 * x >= nr) continue;                              // the same for all lanes: LDS keeps whatever lies there, for rows that are not stored
+            if constexpr (FAR) r[x] = *(const mm_u32x4 *)(xfar[x] + k);
+            else r[x] = *(const mm_u32x4 *)(Xb + k + xo[x]);
+        }
+#pragma unroll
+        for (int x = 0; x < WPF; ++x) r[XPF + x] = *(const mm_u32x4 *)(w_base(x) + k + wo[x]);
+    };
+    uint4 *Xs = smem + wave * OWN, *Ws = Xs + TM * TKU;
+    auto sync = [] {                                                // LDS written by some lanes is read by others of the same wavefront
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto stash = [&](const mm_u32x4 (&r)[XPF + WPF]) {
+        sync();
+#pragma unroll
+        for (int x = 0; x < XPF; ++x)
+            if (8 * x < nr) Xs[at(lr + 8 * x, lu)] = __builtin_bit_cast(uint4, r[x]);
+#pragma unroll
+        for (int x = 0; x < WPF; ++x) Ws[at(lr + 8 * x, lu)] = __builtin_bit_cast(uint4, r[XPF + x]);
+        sync();
+    };
+    mm_f32x16 acc[1][NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[0][t][i] = 0.f;
+    auto products = [&]() {
+#pragma unroll
+        for (int s = 0; s < TKU / 2; ++s) {
+            const uint4 xf = Xs[at(l32, 2 * s + hi)];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[0][t] = mm_type<T>::mma(xf, Ws[at(32 * t + l32, 2 * s + hi)], acc[0][t]);
+        }
+    };
+    if (s0 < s1) {
+        fetch(reg[0], s0);
+        fetch(reg[1], s0 + 1);
+        for (int i = s0; i < s1; i += 2) {                          // two stages ahead: a trip to memory takes longer than one stage's products
+            stash(reg[0]);
+            fetch(reg[0], i + 2);
+            products();
+            if (i + 1 >= s1) break;
+            stash(reg[1]);
+            fetch(reg[1], i + 3);
+            products();
+        }
+    }
+    if (full * STAGE < K && wave == MF_NW - 1) {                    // depths beyond K are zero; a lane beyond K reads its row's first unit: a row may be shorter than a stage
+        const mm_u32x4 zero = {0, 0, 0, 0};
+        const bool in = full * STAGE + lu * UNIT < K;
+        const int64_t k = in ? (int64_t)full * STAGE * sizeof(T) : -(int64_t)(lu * UNIT * sizeof(T));
+#pragma unroll
+        for (int x = 0; x < XPF; ++x) { const mm_u32x4 v = *(const mm_u32x4 *)((FAR ? xfar[FAR ? x : 0] : Xb + xo[x]) + k); reg[0][x] = in ? v : zero; }
+#pragma unroll
+        for (int x = 0; x < WPF; ++x) { const mm_u32x4 v = *(const mm_u32x4 *)(w_base(x) + wo[x] + k); reg[0][XPF + x] = in ? v : zero; }
+        stash(reg[0]);
+        products();
+    }
+    // the shares meet: the first wavefront adds them in order
+    sync();
+    ls_f32x4 *mine = (ls_f32x4 *)Xs;
+    if (wave > 0)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) mine[(4 * t + g) * 64 + lane] = ls_f32x4{acc[0][t][4 * g], acc[0][t][4 * g + 1], acc[0][t][4 * g + 2], acc[0][t][4 * g + 3]};
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 1; w < MF_NW; ++w)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const ls_f32x4 v = ((const ls_f32x4 *)(smem + w * OWN))[(4 * t + g) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[0][t][4 * g + i] += v[i];
+            }
+    moe_store<T, 1, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int, int k, int &p, float &w) { p = rows_out[k]; w = rows_weight[k]; }, [](int) { return 0; },
+                                       [&](int t) { return 32 * t; }, lane);
 }
 
 // ---- the same product in tiles of 256 rows by 256 weight rows (bfloat16, depths in whole stages of 64) ----------------------------------------
@@ -904,7 +983,7 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(MoeMM a) {
 template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(MoeMM &a, bool gated, hipStream_t st) {
     const int tn = gated ? WR / 2 : WR;
     a.col_blocks = (a.n_out + tn - 1) / tn;
-    const int64_t groups = (int64_t)(TM >= 64 ? (a.max_tiles + 7) / 8 * 8 : a.max_tiles) * a.col_blocks * a.parts;
+    const int64_t groups = (int64_t)(a.max_tiles + 7) / 8 * 8 * a.col_blocks * a.parts;
     if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
     const bool far = a.mode != 1 && ((int64_t)a.max_tiles * a.parts * TM / a.top + 1) * a.K * (int64_t)sizeof(T) > UINT32_MAX;      // gathered rows beyond what 32 bits reach
     auto kern = gated ? (far ? moe_mm_kernel<T, TM, NW, WR, TKU, true, true> : moe_mm_kernel<T, TM, NW, WR, TKU, true, false>)
@@ -926,7 +1005,17 @@ template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated
         if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
     } else if (tile_rows >= 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32 or 64 rows");
     if (tile_rows == 64) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
-    return moe_mm_launch<T, 32, 1, 64, 8>(a, gated, st);
+    a.col_blocks = (a.n_out + (gated ? 31 : 63)) / (gated ? 32 : 64);
+    const int64_t groups = (int64_t)a.max_tiles * a.col_blocks;
+    if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
+    const bool far = a.mode != 1 && ((int64_t)a.max_tiles * 32 / a.top + 1) * a.K * (int64_t)sizeof(T) > UINT32_MAX;
+    // four wavefronts where experts have up to about eight rows, and for float (twice the bytes, a sixteenth of the matrix rate); two where more tiles fill the chip
+    const bool four = sizeof(T) == 4 || a.max_tiles - a.E <= a.E / 4;
+#define MF_KERNEL(NW) (gated ? (far ? moe_few_kernel<T, NW, true, true> : moe_few_kernel<T, NW, true, false>) : (far ? moe_few_kernel<T, NW, false, true> : moe_few_kernel<T, NW, false, false>))
+    if (four) MF_KERNEL(4)<<<dim3((unsigned)groups), 256, 0, st>>>(a);
+    else MF_KERNEL(2)<<<dim3((unsigned)groups), 128, 0, st>>>(a);
+#undef MF_KERNEL
+    return jl_check_launch("moe_few_kernel");
 }
 
 static int moe_gemm_launch(const void *X, const void *Wt, int dtype, int32_t mode, int32_t K, int32_t n_out, int32_t top, const int32_t *perm,
