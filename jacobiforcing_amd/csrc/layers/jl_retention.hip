@@ -3,39 +3,44 @@
 #include "jl_common.h"
 #include <type_traits>
 
-// One workgroup per (request, head); thread j owns column j of the state S [D, Dv] in registers.  Tokens are taken TT at a
-// time: the rotated queries / keys of a group go through LDS, each thread runs the recurrence for its column, the per-token
-// sums of squares (unit norm over the head's Dv outputs) are reduced once per group.
+// One workgroup per (request, head); thread (p, j) owns rows DPER p .. of column j of the state S [D, Dv] in registers, PARTS threads per column.  Tokens are taken TT at a
+// time: the rotated queries / keys of a group go through LDS, each thread runs the recurrence for its rows, the parts' sums meet in LDS, and part p finishes every PARTS-th token (unit norm over the
+// head's Dv outputs).  What bounds single tokens is the state's way in and out, so as many loads as fit are on the way: one thread per column took 34.7 us for 32 tokens of 8 heads of 128 x 128 (33.6 MB),
+// four take 12.7; a step of 32 decoding requests 516 -> 503 us, which then waits for the host.
 constexpr int RET_TT = 8;
 
 // MAXT: the largest workgroup the instantiation is launched with.  With 256 the state's DMAX rows stay in registers up to
 // DMAX = 128 (the default bound of 1 024 threads leaves 128 registers per lane and spills them).
-template <typename T, int DMAX, int MAXT>
+template <typename T, int DMAX, int PARTS, int MAXT>
 __global__ __launch_bounds__(MAXT) void retention_kernel(const T *__restrict__ proj, int64_t ld, int q_col, int k_col, int v_col, int g_col,
                                  const int32_t *__restrict__ seq, int H, int D, int Dv, int rot_dims,
                                  const float *__restrict__ cos_t, const float *__restrict__ sin_t, int64_t table_len,
                                  const float *__restrict__ decay, float eps, float *__restrict__ state, T *__restrict__ out, int mode) {
+    constexpr int DPER = DMAX / PARTS;
     extern __shared__ float lds[];
-    float *qs = lds;                                   // [TT][D]
-    float *ks = qs + RET_TT * D;                       // [TT][D]
-    float *red = ks + RET_TT * D;                      // [TT][16]
+    float *qs = lds;                                   // [TT][DMAX]
+    float *ks = qs + RET_TT * DMAX;                    // [TT][DMAX]
+    float *red = ks + RET_TT * DMAX;                   // [TT][16]
+    float *sums = red + RET_TT * 16;                   // [TT][threads]: the parts' sums
     const int b = blockIdx.x / H, h = blockIdx.x - b * H;
     const int row0 = seq[4 * b], cnt = seq[4 * b + 1], pos0 = seq[4 * b + 2], slot = seq[4 * b + 3];
     if (cnt <= 0) return;
-    const int j = threadIdx.x, wave = j >> 6, nw = (blockDim.x + 63) >> 6;
+    const int tid = threadIdx.x, width = blockDim.x / PARTS, part = PARTS > 1 ? tid / width : 0, j = PARTS > 1 ? tid - part * width : tid, wave = j >> 6, nw = width >> 6, d0 = part * DPER;
     const bool live = j < Dv;
     const float gamma = decay[h], kscale = 1.0f / sqrtf((float)D);
     const int half = rot_dims >> 1;
     float *sp = state + ((int64_t)slot * H + h) * D * Dv;
-    float S[DMAX];
+    float S[DPER];
+    const bool old = live && (mode == JL_RET_FROM_SLOT || (mode == JL_RET_SCAN && pos0 > 0));
 #pragma unroll
-    for (int d = 0; d < DMAX; ++d) S[d] = (live && d < D && (mode == JL_RET_FROM_SLOT || (mode == JL_RET_SCAN && pos0 > 0))) ? sp[(int64_t)d * Dv + j] : 0.f;
+    for (int i = 0; i < DPER; ++i) S[i] = old && d0 + i < D ? sp[(int64_t)(d0 + i) * Dv + j] : 0.f;
 
     for (int t0 = 0; t0 < cnt; t0 += RET_TT) {
         const int nt = cnt - t0 < RET_TT ? cnt - t0 : RET_TT;
         __syncthreads();
-        for (int e = j; e < nt * D; e += blockDim.x) {
-            const int tt = e / D, d = e - tt * D;
+        for (int e = tid; e < nt * DMAX; e += blockDim.x) {
+            const int tt = e / DMAX, d = e - tt * DMAX;
+            if (d >= D) { qs[e] = ks[e] = 0.f; continue; }      // rows beyond D stay zero
             const T *row = proj + (int64_t)(row0 + t0 + tt) * ld + h * D;
             float qv, kv;
             if (d < rot_dims) {
@@ -61,52 +66,67 @@ __global__ __launch_bounds__(MAXT) void retention_kernel(const T *__restrict__ p
             o[tt] = 0.f;
             if (tt < nt) {
                 const float v = live ? ld_f(proj + (int64_t)(row0 + t0 + tt) * ld + v_col + h * Dv + j) : 0.f;
-                const float *qp = qs + tt * D, *kp = ks + tt * D;
+                const float *qp = qs + tt * DMAX + d0, *kp = ks + tt * DMAX + d0;
                 float acc = 0.f;
 #pragma unroll
-                for (int d = 0; d < DMAX; ++d)
-                    if (d < D) {
-                        S[d] = gamma * S[d] + kp[d] * v;
-                        acc += S[d] * qp[d];
-                    }
-                o[tt] = acc;
-                if (mode != JL_RET_LOCAL_STATE) {
-                    const float ss = wave_sum_f32(acc * acc);
-                    if ((j & 63) == 0) red[tt * 16 + wave] = ss;
+                for (int i = 0; i < DPER; i += 4) {
+                    const float4 k4 = *(const float4 *)(kp + i), q4 = *(const float4 *)(qp + i);
+                    S[i] = gamma * S[i] + k4.x * v;             acc += S[i] * q4.x;
+                    S[i + 1] = gamma * S[i + 1] + k4.y * v;     acc += S[i + 1] * q4.y;
+                    S[i + 2] = gamma * S[i + 2] + k4.z * v;     acc += S[i + 2] * q4.z;
+                    S[i + 3] = gamma * S[i + 3] + k4.w * v;     acc += S[i + 3] * q4.w;
                 }
+                o[tt] = acc;
+                if (PARTS > 1 && mode != JL_RET_LOCAL_STATE) sums[tt * blockDim.x + tid] = acc;
             }
         }
         if (mode == JL_RET_LOCAL_STATE) continue;
+        if (PARTS > 1) __syncthreads();
+#pragma unroll
+        for (int y = 0; y < RET_TT / PARTS; ++y) {                  // this part's tokens: part, part + PARTS, ..
+            const int tt = y * PARTS + part;
+            if (tt >= nt) continue;
+            if (PARTS > 1) {
+                float acc = sums[tt * blockDim.x + j];
+#pragma unroll
+                for (int p = 1; p < PARTS; ++p) acc += sums[tt * blockDim.x + p * width + j];
+                o[y] = acc;
+            }
+            const float ss = wave_sum_f32(o[y] * o[y]);
+            if ((j & 63) == 0) red[tt * 16 + wave] = ss;
+        }
         __syncthreads();
 #pragma unroll
-        for (int tt = 0; tt < RET_TT; ++tt)
-            if (tt < nt && live) {
-                float ss = 0.f;
-                for (int w = 0; w < nw; ++w) ss += red[tt * 16 + w];
-                const float r = 1.0f / sqrtf(ss / (float)Dv + eps);
-                const int64_t n = row0 + t0 + tt;
-                const float g = ld_f(proj + n * ld + g_col + h * Dv + j);
-                st_f(out + n * ((int64_t)H * Dv) + h * Dv + j, o[tt] * r * (g / (1.0f + expf(-g))));
-            }
+        for (int y = 0; y < RET_TT / PARTS; ++y) {
+            const int tt = y * PARTS + part;
+            if (tt >= nt || !live) continue;
+            float ss = 0.f;
+            for (int w = 0; w < nw; ++w) ss += red[tt * 16 + w];
+            const float r = 1.0f / sqrtf(ss / (float)Dv + eps);
+            const int64_t n = row0 + t0 + tt;
+            const float g = ld_f(proj + n * ld + g_col + h * Dv + j);
+            st_f(out + n * ((int64_t)H * Dv) + h * Dv + j, o[y] * r * (g / (1.0f + expf(-g))));
+        }
     }
     if (live && mode != JL_RET_FROM_SLOT)
 #pragma unroll
-        for (int d = 0; d < DMAX; ++d)
-            if (d < D) sp[(int64_t)d * Dv + j] = S[d];
+        for (int i = 0; i < DPER; ++i)
+            if (d0 + i < D) sp[(int64_t)(d0 + i) * Dv + j] = S[i];
 }
 
 template <typename T, int DMAX>
 static int ret_launch(const void *proj, int64_t ld, int q_col, int k_col, int v_col, int g_col, const int32_t *seq, int B, int H, int D,
                       int Dv, int rot_dims, const float *cos_t, const float *sin_t, int64_t table_len, const float *decay, float eps,
                       float *state, void *out, int mode, hipStream_t st) {
-    const int threads = (Dv + 63) / 64 * 64;
-    const size_t lds = (size_t)(2 * RET_TT * D + RET_TT * 16) * 4;
-    if (DMAX >= 128 && threads <= 256)
-        retention_kernel<T, DMAX, 256><<<dim3((unsigned)(B * H)), threads, lds, st>>>((const T *)proj, ld, q_col, k_col, v_col, g_col, seq, H, D, Dv,
-                                                                                     rot_dims, cos_t, sin_t, table_len, decay, eps, state, (T *)out, mode);
-    else
-        retention_kernel<T, DMAX, 1024><<<dim3((unsigned)(B * H)), threads, lds, st>>>((const T *)proj, ld, q_col, k_col, v_col, g_col, seq, H, D, Dv,
-                                                                                      rot_dims, cos_t, sin_t, table_len, decay, eps, state, (T *)out, mode);
+    const int width = (Dv + 63) / 64 * 64, parts = width <= 128 ? 4 : width <= 256 ? 2 : 1;
+    const size_t lds = (size_t)(2 * RET_TT * DMAX + RET_TT * 16 + (parts > 1 ? RET_TT * width * parts : 0)) * 4;
+#define RET_LAUNCH(PARTS, MAXT)                                                                                                                          \
+    retention_kernel<T, DMAX, PARTS, MAXT><<<dim3((unsigned)(B * H)), width * PARTS, lds, st>>>((const T *)proj, ld, q_col, k_col, v_col, g_col, seq, H, D, Dv, \
+                                                                                               rot_dims, cos_t, sin_t, table_len, decay, eps, state, (T *)out, mode)
+    if (parts == 4) RET_LAUNCH(4, 512);
+    else if (parts == 2) RET_LAUNCH(2, 512);
+    else RET_LAUNCH(1, 1024);
+#undef RET_LAUNCH
     return jl_check_launch("retention_kernel");
 }
 
