@@ -217,6 +217,8 @@ JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, cons
 
 /* z <- cap * tanh(z / cap) in place over `total` floats (soft cap of the logits). */
 JL_API int jl_softcap(float *z, int64_t total, float cap, void *stream);
+/* the same of z (`dtype`) into out */
+JL_API int jl_softcap_to(const void *z, int dtype, float *out, int64_t total, float cap, void *stream);
 
 /* Sublayer-output norm + residual update: x[n] += y[n] / sqrt(mean(y[n]^2) + eps) * g[0] (x float in place, y of y_dtype, g one
  * float); when `out` is given, out[n] = x[n] in `out_dtype` (what the next sublayer's product reads). */

@@ -332,6 +332,7 @@ _LAYER_SIGNATURES = {
                                     _vp]),
     "jl_token_shift": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, C.c_int, _vp]),
     "jl_softcap": (C.c_int, [_vp, _i64, _f32, _vp]),
+    "jl_softcap_to": (C.c_int, [_vp, C.c_int, _vp, _i64, _f32, _vp]),
     "jl_short_conv": (C.c_int, [_vp, C.c_int, _i64, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _i64, _i32, _i32, _i32, _vp, C.c_int, _vp]),
     "jl_sandwich_norm": (C.c_int, [_vp, _vp, _vp, C.c_int, _vp, _vp, _f32, _vp, _vp, C.c_int, _i64, _i32, _i64, _i32, _vp]),
     "jl_output_norm": (C.c_int, [_vp, C.POINTER(Addend), _i32, _vp, _vp, _i32, _i32, _i32, _vp, _f32, _f32, _vp, _vp, C.c_int, _i64, _i32, _vp]),

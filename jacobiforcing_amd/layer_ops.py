@@ -1251,6 +1251,17 @@ def softcap(z: torch.Tensor, cap: float) -> torch.Tensor:
     return z
 
 
+def softcap_float(z: torch.Tensor, cap: float) -> torch.Tensor:
+    """cap * tanh(z / cap) as float: ``softcap`` of float z, and of bfloat16 z in the one pass that makes it float."""
+    if z.dtype != torch.bfloat16:
+        return softcap(z, cap)
+    _dev(z)
+    _need(z.is_contiguous() and cap > 0, "softcap_float: contiguous values and a positive cap")
+    out = torch.empty(z.shape, dtype=torch.float32, device=z.device)
+    N.check_layers(N.layers().jl_softcap_to(_ptr(z), _code(z.dtype), _ptr(out), z.numel(), float(cap), _stream(z.device)), "jl_softcap_to")
+    return out
+
+
 def short_conv(x: torch.Tensor, col: int, C_: int, w: torch.Tensor, batch: RaggedBatch, tail: Optional[torch.Tensor], act: int = N.JL_ACT_SILU,
                bias: Optional[torch.Tensor] = None, out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
     """act(bias + causal depthwise convolution over time, per request) of the columns col .. col + C_ of x [N, ld], with w [C_, taps]; [N, C_]

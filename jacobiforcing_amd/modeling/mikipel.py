@@ -343,8 +343,9 @@ class MikipelModel:
         hl = hand_on(nl, w.final_norm, dt)
         if logit_rows is not None:
             hl = hl.index_select(0, logit_rows)
-        z = LO.linear(hl, w.embed, float_out=False)
-        return LO.softcap(z, cfg.logit_softcap) if cfg.logit_softcap > 0 else z
+        if cfg.logit_softcap > 0:
+            return LO.softcap_float(LO.linear(hl, w.embed), cfg.logit_softcap)
+        return LO.linear(hl, w.embed, float_out=False)
 
 
 def load_model_directory(model_dir, device, dtype=torch.bfloat16, max_positions: int = 8192):
