@@ -302,10 +302,14 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 // instructions take a unit of 16 bytes per lane, depths 8 u + 4 (l / 32) + i of unit u — which is also how four accumulators of a lane lie, so results are the next
 // product's operand as they are: between the kernels (every operand as units [unit][lane], read as 1 KB per wavefront straight into registers, a chunk ahead) and in LDS
 // between the wavefronts of a chain.  T comes from 16 x 16 blocks by substitution, joined by products, on one wavefront while the others make P.
-// What bounds it: the chain's 128 matrix instructions of 64 cycles per chunk on the busiest of its four wavefronts (D = 128; 58 % of its time), and in the chunks' kernel the
-// phases of a workgroup that wait for each other (two workgroups per CU at 79 104 bytes of LDS; with one, 302 us instead of 198, measured then).
-// Measured against columns of the state walking token by token, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 1446 -> 430 us (chunks 210, chain 210,
-// norm 34); 8 heads, one portion of 128 80 -> 45; 16 heads, 777 + 300 tokens beside 30 single ones 566 -> 148; float, 8 heads, 1021 + 851 + 681 tokens 587 -> 149.
+// The chain's operands are split into three bfloat16 terms each, on the wavefronts that hold them, while the other wavefront of a SIMD multiplies: a product with S takes 48
+// instructions of 32 cycles instead of 64 of 64, one with U 24 instead of 32.  Errors against 64 bits, heads of 128, 1021 tokens: outputs 1.20e-7 and state 1.02e-7, with
+// products of floats 1.24e-7 and 1.17e-7; with long memories 1.55e-7 and 1.40e-7, 1.82e-7 and 1.76e-7.
+// What bounds it: the chain's two waits per chunk, with the product with S (about 3900 cycles), then the correction's own split and the keys' product between them; in the chunks'
+// kernel the phases of a workgroup that wait for memory and for each other (two workgroups per CU at 79 104 bytes of LDS).  Its loads set out together and V's in front of
+// the stores: a load waits for the stores in front of it, here 57 000 of a workgroup's 145 000 cycles.
+// Measured, norm and gate included, bfloat16, heads of 128: 16 heads, 4 x 2048 tokens 446 -> 328 us (chunks 210 -> 150, chain 200 -> 137, norm 40; columns walking token by token
+// took 1446); float, 8 heads, 1021 + 851 + 681 tokens 147 -> 106, heads of 64 101 -> 80.
 constexpr int DK_T = 64;
 typedef float dk_f32x16 __attribute__((ext_vector_type(16)));
 typedef float dk_f32x4 __attribute__((ext_vector_type(4)));
@@ -320,6 +324,27 @@ __device__ __forceinline__ dk_f32x4 dk_mma16(float4 a, float4 b, dk_f32x4 c) {
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+// a product 16 deep of 32-bit operands: each the sum of three bfloat16 numbers, the pairs of terms whose product is above 2 ** -26 of the whole, the greatest apart from the others
+struct dk_terms { jl_bf16x8 t[JL_SPLIT_TERMS]; };
+__device__ __forceinline__ dk_terms dk_split(float4 a, float4 b) {
+    dk_terms r;
+    jl_split8(jl_f32x8{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, r.t);
+    return r;
+}
+struct dk_sums { dk_f32x16 great, small; };
+__device__ __forceinline__ void dk_clear(dk_sums &c) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c.great[r] = c.small[r] = 0.f;
+}
+__device__ __forceinline__ dk_f32x16 dk_total(const dk_sums &c) { return c.great + c.small; }
+__device__ __forceinline__ void dk_mma_split(const dk_terms &a, const dk_terms &b, dk_sums &c) {
+    c.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[0], b.t[2], c.small, 0, 0, 0);
+    c.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[1], b.t[1], c.small, 0, 0, 0);
+    c.great = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[0], b.t[0], c.great, 0, 0, 0);
+    c.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[2], b.t[0], c.small, 0, 0, 0);
+    c.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[0], b.t[1], c.small, 0, 0, 0);
+    c.small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.t[1], b.t[0], c.small, 0, 0, 0);
 }
 __device__ __forceinline__ void dk_wave_sync() {        // LDS written by some lanes is read by others of the same wavefront
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -362,37 +387,27 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
     auto at = [](int row, int u) { return u ^ (row & 15); };                        // rows have a multiple of 16 units
     auto am_at = [](int t, int u) { return t < 32 ? t * 8 + (u ^ (t & 7)) : 256 + (t - 32) * 16 + (u ^ (t & 15)); };    // A, then T: the first 32 rows have 32 columns
     const float *src = a.qkv + (int64_t)row0 * a.qkv_ld + kh * D;
+    constexpr int IT = DK_T * U / 256;
+    float ga = 0.f, gb = 0.f;
+    if (wave == 0) {                                                               // everything that is read sets out here, V a phase later: nothing waits for memory twice
+        const T *row = (const T *)a.proj + (int64_t)(row0 + min(lane, cnt - 1)) * a.ld;
+        ga = ld_f(row + a.a_col + h);
+        gb = ld_f(row + a.b_col + h);
+    }
+    float4 qv[IT], kv[IT];
 #pragma unroll
-    for (int it = 0; it < DK_T * U / 256; ++it) {                                  // unit vectors: U adjacent lanes hold a row
-        const int e = tid + it * 256, tt = e / U, u = e % U;
-        float4 q = make_float4(0.f, 0.f, 0.f, 0.f), k = q;
-        if (tt < cnt && 4 * u < D) {
-            const float *row = src + (int64_t)tt * a.qkv_ld + 4 * u;
-            q = *(const float4 *)(row + a.q_col);
-            k = *(const float4 *)(row + a.k_col);
-        }
-        float sq = (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w), sk = (k.x * k.x + k.y * k.y) + (k.z * k.z + k.w * k.w);
-#pragma unroll
-        for (int off = 1; off < U; off <<= 1) { sq += __shfl_xor(sq, off, 64); sk += __shfl_xor(sk, off, 64); }
-        const float rq = tt < cnt ? a.q_scale / sqrtf(sq + a.unit_eps) : 0.f, rk = tt < cnt ? 1.0f / sqrtf(sk + a.unit_eps) : 0.f;
-        Qs[tt * U + at(tt, u)] = make_float4(q.x * rq, q.y * rq, q.z * rq, q.w * rq);
-        k = make_float4(k.x * rk, k.y * rk, k.z * rk, k.w * rk);
-        const uint64_t none = __ballot(__builtin_isnan((k.x + k.y) + (k.z + k.w)));   // elements of a unit vector: what is not finite before is not a number now
-        bool flaw = false;                                                          // the row's
-        if (none) {
-            flaw = none >> (lane & ~(U - 1)) & ((1ull << U) - 1);
-            if (flaw) k = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        Ks[tt * U + at(tt, u)] = k;
-        if (u == 0) flawS[tt] = flaw;
+    for (int it = 0; it < IT; ++it) {                                              // a row that does not exist: the last one's, not used
+        const int e = tid + it * 256, tt = min(e / U, cnt - 1), d = 4 * (e % U) < D ? 4 * (e % U) : 0;
+        const uint32_t at = (uint32_t)tt * (uint32_t)a.qkv_ld + d;
+        qv[it] = *(const float4 *)(src + a.q_col + at);
+        kv[it] = *(const float4 *)(src + a.k_col + at);
     }
     if (wave == 0) {
         float lg = 0.f, beta = 0.f;
         if (lane < cnt) {
-            const T *row = (const T *)a.proj + (int64_t)(row0 + lane) * a.ld;
-            lg = -expf(a.A_log[h]) * softplus_f(ld_f(row + a.a_col + h) + a.dt_bias[h]);
+            lg = -expf(a.A_log[h]) * softplus_f(ga + a.dt_bias[h]);
             lg = lg < -1e4f ? -1e4f : lg;
-            beta = 1.0f / (1.0f + expf(-ld_f(row + a.b_col + h)));
+            beta = 1.0f / (1.0f + expf(-gb));
         }
         double c = lg;
 #pragma unroll
@@ -408,6 +423,34 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
         head[z.p + 3 * 1024 + lane] = gam;
         head[z.p + 3 * 1024 + DK_T + lane] = dk_exp(end - c);
     }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {                                              // unit vectors: U adjacent lanes hold a row
+        const int e = tid + it * 256, tt = e / U, u = e % U;
+        const bool there = tt < cnt && 4 * u < D;
+        float4 q = there ? qv[it] : make_float4(0.f, 0.f, 0.f, 0.f), k = there ? kv[it] : make_float4(0.f, 0.f, 0.f, 0.f);
+        float sq = (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w), sk = (k.x * k.x + k.y * k.y) + (k.z * k.z + k.w * k.w);
+#pragma unroll
+        for (int off = 1; off < U; off <<= 1) { sq += __shfl_xor(sq, off, 64); sk += __shfl_xor(sk, off, 64); }
+        const float rq = tt < cnt ? a.q_scale / sqrtf(sq + a.unit_eps) : 0.f, rk = tt < cnt ? 1.0f / sqrtf(sk + a.unit_eps) : 0.f;
+        Qs[tt * U + at(tt, u)] = make_float4(q.x * rq, q.y * rq, q.z * rq, q.w * rq);
+        k = make_float4(k.x * rk, k.y * rk, k.z * rk, k.w * rk);
+        const uint64_t none = __ballot(__builtin_isnan((k.x + k.y) + (k.z + k.w)));   // elements of a unit vector: what is not finite before is not a number now
+        bool flaw = false;                                                          // the row's
+        if (none) {
+            flaw = none >> (lane & ~(U - 1)) & ((1ull << U) - 1);
+            if (flaw) k = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        Ks[tt * U + at(tt, u)] = k;
+        if (u == 0) flawS[tt] = flaw;
+    }
+    const int nv = (Dv + 31) / 32;
+    const float *vp = a.qkv + (int64_t)row0 * a.qkv_ld + a.v_col + (int64_t)h * Dv;
+    float vv[32];                                                                  // a wavefront's 32 columns of V, all tokens
+    auto fetch_v = [&](int vt) {
+        const int col = min(32 * vt + l32, Dv - 1);
+#pragma unroll
+        for (int i = 0; i < 32; ++i) vv[i] = vp[(uint32_t)min(8 * (i >> 2) + 4 * hi + (i & 3), cnt - 1) * (uint32_t)a.qkv_ld + col];
+    };
     __syncthreads();
     // from the first token with a key, decay or beta that is not a number on: nothing here that zeros would spread to the tokens in front of it; W1 says so instead
     const uint64_t flaws = __ballot(flawS[lane] || !__builtin_isfinite((float)cs[lane]) || !__builtin_isfinite(bs[lane]));
@@ -461,6 +504,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
             ((float4 *)group)[e * 64 + lane] = Qs[t * U + at(t, 2 * x + hi)];
         }
     }
+    if (wave < nv) fetch_v(wave);
     __syncthreads();
     if (wave == 0) {
         // (I + A)^-1 in place.  The four 16 x 16 blocks of the diagonal by substitution, a lane per column
@@ -523,42 +567,18 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
     }
     __syncthreads();
     auto trow = [&](int ti, int y) { const int t = 32 * ti + l32; return Am[am_at(t, 2 * y + hi)]; };
-    const int nv = (Dv + 31) / 32;
-    for (int task = wave; task < DT + nv; task += 4) {
+    for (int task = wave; task < nv + DT; task += 4) {                             // V first: its loads would wait for the stores of the others
         float4 f[8];                                                               // 32 columns of K or V at all 64 depths
         dk_f32x16 acc[2];
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
-        if (task < DT) {                                                           // -W2 transposed: rows of K^T, columns t
-            const float *kf = (const float *)Ks;
-            const int d = 32 * task + l32;
+        if (task < nv) {                                                           // W1: rows t, 32 columns of beta V
+            const int vt = task, col = 32 * vt + l32;
 #pragma unroll
             for (int y = 0; y < 8; ++y) {
                 float v[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = kf[4 * (t * U + at(t, d >> 2)) + (d & 3)]; }
-                f[y] = make_float4(v[0], v[1], v[2], v[3]);
-                if (leader) ((float4 *)group)[(DP / 4 + 8 * task + y) * 64 + lane] = f[y];
-            }
-#pragma unroll
-            for (int y = 0; y < 8; ++y) {
-                const float4 s = *(const float4 *)(bg + 8 * y + 4 * hi), v = make_float4(f[y].x * s.x, f[y].y * s.y, f[y].z * s.z, f[y].w * s.w);
-                if (y < 4) acc[0] = dk_mma(v, trow(0, y), acc[0]);
-                acc[1] = dk_mma(v, trow(1, y), acc[1]);
-            }
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-                for (int y = 0; y < 4; ++y)
-                    ((float4 *)(head + z.w2))[(ti * (DP / 8) + 4 * task + y) * 64 + lane] = make_float4(acc[ti][4 * y], acc[ti][4 * y + 1], acc[ti][4 * y + 2], acc[ti][4 * y + 3]);
-        } else {                                                                   // W1: rows t, 32 columns of beta V
-            const int vt = task - DT, col = 32 * vt + l32;
-            const float *vp = a.qkv + (int64_t)row0 * a.qkv_ld + a.v_col + (int64_t)h * Dv + col;
-#pragma unroll
-            for (int y = 0; y < 8; ++y) {
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = t < cnt && col < Dv ? vp[t * a.qkv_ld] * bs[t] : 0.f; }
+                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = t < cnt && col < Dv ? vv[4 * y + i] * bs[t] : 0.f; }
                 f[y] = make_float4(v[0], v[1], v[2], v[3]);
             }
 #pragma unroll
@@ -566,6 +586,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
                 if (y < 4) acc[0] = dk_mma(trow(0, y), f[y], acc[0]);
                 acc[1] = dk_mma(trow(1, y), f[y], acc[1]);
             }
+            if (vt + 4 < nv) fetch_v(vt + 4);
             // all values of a column enter a row of the second half, one that is not finite as not a number: the same without it
             if (broken < DK_T || __any(!__builtin_isfinite(acc[1][0]))) {
                 int none = broken;                                                 // this lane's column is not a number from here on
@@ -577,7 +598,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int t = 8 * y + 4 * hi + i;
-                        v[i] = t < cnt && col < Dv ? vp[t * a.qkv_ld] * bs[t] : 0.f;
+                        v[i] = t < cnt && col < Dv ? vp[(uint32_t)t * (uint32_t)a.qkv_ld + col] * bs[t] : 0.f;
                         if (!__builtin_isfinite(v[i])) { v[i] = 0.f; none = min(none, t); }
                     }
                     if (y < 4) acc[0] = dk_mma(trow(0, y), make_float4(v[0], v[1], v[2], v[3]), acc[0]);
@@ -594,159 +615,252 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 #pragma unroll
                 for (int y = 0; y < 4; ++y)
                     ((float4 *)(head + z.w1))[((vt * 2 + ti) * 4 + y) * 64 + lane] = make_float4(acc[ti][4 * y], acc[ti][4 * y + 1], acc[ti][4 * y + 2], acc[ti][4 * y + 3]);
+        } else {                                                                   // -W2 transposed: rows of K^T, columns t
+            const float *kf = (const float *)Ks;
+            const int x = task - nv, d = 32 * x + l32;
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { const int t = 8 * y + 4 * hi + i; v[i] = kf[4 * (t * U + at(t, d >> 2)) + (d & 3)]; }
+                f[y] = make_float4(v[0], v[1], v[2], v[3]);
+                if (leader) ((float4 *)group)[(DP / 4 + 8 * x + y) * 64 + lane] = f[y];
+            }
+#pragma unroll
+            for (int y = 0; y < 8; ++y) {
+                const float4 s = *(const float4 *)(bg + 8 * y + 4 * hi), v = make_float4(f[y].x * s.x, f[y].y * s.y, f[y].z * s.z, f[y].w * s.w);
+                if (y < 4) acc[0] = dk_mma(v, trow(0, y), acc[0]);
+                acc[1] = dk_mma(v, trow(1, y), acc[1]);
+            }
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    ((float4 *)(head + z.w2))[(ti * (DP / 8) + 4 * x + y) * 64 + lane] = make_float4(acc[ti][4 * y], acc[ti][4 * y + 1], acc[ti][4 * y + 2], acc[ti][4 * y + 3]);
         }
     }
 }
 
 // Workgroup (request, head, 32 columns); the column blocks of a head lie eight apart, on one XCD, since they read the same operands.  Wavefronts 0 and 1 make U, 2 and 3 the
-// outputs of 32 tokens each; every one of the first D / 32 owns 32 rows of S.
+// outputs of 32 tokens each; the D / 32 that follow own 32 rows of S each.  What a wavefront takes from memory is split while another's matrix instructions run: two to a SIMD.
 template <int DP>
-__global__ __launch_bounds__(256, 1) void delta_chain_kernel(jl_delta_chunks a, int h0, int nh, float *__restrict__ raw) {
-    constexpr int NU = DP / 8, DT = DP / 32;
-    __shared__ float4 Sf[NU * 64], Uf[8 * 64], Ug[8 * 64];
+__global__ __launch_bounds__(256 + 2 * DP, 1) void delta_chain_kernel(jl_delta_chunks a, int h0, int nh, float *__restrict__ raw) {
+    constexpr int NU = DP / 8;
+    __shared__ jl_bf16x8 Sf[NU / 2 * 3 * 64], Uf[4 * 3 * 64];       // [16 depths][term][lane]
+    __shared__ float4 Pf[2 * 4 * 64];                               // what the pairs take of U, as accumulators lie
     __shared__ int noneS[2][32];                                    // the first token of a half chunk whose correction is not finite, per column
     const int nv = (a.Dv + 31) / 32, lin = blockIdx.x >> 3, vt = lin % nv, bh = (lin / nv) * 8 + (blockIdx.x & 7);
     if (bh >= a.B * nh) return;
     const int b = bh / nh, hl = bh - b * nh, h = h0 + hl, per = a.H / a.G, D = a.D, Dv = a.Dv;
     const int first = a.req[4 * b], n = a.req[4 * b + 1], pos0 = a.req[4 * b + 2], slot = a.req[4 * b + 3];
     if (n <= 0) return;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * vt + l32, ti = wave & 1;
-    const bool maker = wave < 2, owner = wave < DT;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * vt + l32, ti = wave & 1;
     const dk_sizes z = dk_layout(DP, Dv);
     const float *heads = a.scratch + (int64_t)hl * z.head, *groups = a.scratch + (int64_t)a.chunks * nh * z.head + (int64_t)(hl / per) * z.group;
     const int64_t head_step = nh * z.head, group_step = (nh / per) * z.group;
-    float *sp = a.state + ((int64_t)slot * a.H + h) * D * Dv;
-    dk_f32x16 S;
+    auto head_of = [&](int c) { return heads + (int64_t)c * head_step; };
+    auto group_of = [&](int c) { return groups + (int64_t)c * group_step; };
+    auto after = [&](int c) { return c + 1 < first + n ? c + 1 : c; };      // every operand's successor sets out when it has been used: a whole chunk ahead, in its registers
+    auto unit_of = [&](const float *p, int u) { return ((const float4 *)p + u * 64)[(uint32_t)lane]; };
+    auto four = [](const dk_f32x16 &v, int y) { return make_float4(v[4 * y], v[4 * y + 1], v[4 * y + 2], v[4 * y + 3]); };
+    auto put = [&](jl_bf16x8 *to, int s, const dk_terms &v) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int d = 32 * wave + 8 * (r >> 2) + 4 * hi + (r & 3);
-        S[r] = owner && d < D && col < Dv && pos0 > 0 ? sp[(int64_t)d * Dv + col] : 0.f;
-    }
-    auto share_state = [&]() {
-        if (owner)
-#pragma unroll
-            for (int y = 0; y < 4; ++y) Sf[(4 * wave + y) * 64 + lane] = make_float4(S[4 * y], S[4 * y + 1], S[4 * y + 2], S[4 * y + 3]);
+        for (int x = 0; x < 3; ++x) to[(3 * s + x) * 64 + lane] = v.t[x];
     };
-    share_state();
-    float4 fa[NU], fk[8], fp[8], w1[4], sc[4];
-    float gend;
-    // what U, or the outputs, take of S, and their scales; the keys that the owned rows of S take up, and the pairs
-    struct sources { const float4 *a, *w1, *sc, *k, *p; const float *gend; };
-    auto sources_of = [&](int c) {
-        const float *hp = heads + (int64_t)c * head_step, *gp = groups + (int64_t)c * group_step;
-        sources q;
-        q.a = (const float4 *)(maker ? hp + z.w2 : gp) + ti * NU * 64 + lane;
-        q.w1 = (const float4 *)(hp + z.w1) + ((vt * 2 + ti) * 4) * 64 + lane;
-        q.sc = (const float4 *)(hp + z.p + 3 * 1024 + (maker ? DK_T : 0) + 32 * ti + 4 * hi);
-        q.k = (const float4 *)gp + (DP / 4 + (owner ? 8 * wave : 0)) * 64 + lane;
-        q.p = (const float4 *)(hp + z.p) + 4 * ti * 64 + lane;
-        q.gend = hp + z.p + 3 * 1024 + DK_T - 1;
-        return q;
+    auto get = [&](const jl_bf16x8 *from, int s) {
+        dk_terms v;
+#pragma unroll
+        for (int x = 0; x < 3; ++x) v.t[x] = from[(3 * s + x) * 64 + lane];
+        return v;
     };
-    {
-        const sources q = sources_of(first);
+    if (wave >= 4) {                                                // rows 32 (wave - 4) .. of S
+        const int w = wave - 4;
+        float *sp = a.state + ((int64_t)slot * a.H + h) * D * Dv;
+        dk_f32x16 S;
 #pragma unroll
-        for (int u = 0; u < NU; ++u) fa[u] = q.a[u * 64];
+        for (int r = 0; r < 16; ++r) {
+            const int d = 32 * w + 8 * (r >> 2) + 4 * hi + (r & 3);
+            S[r] = d < D && col < Dv && pos0 > 0 ? sp[(int64_t)d * Dv + col] : 0.f;
+        }
+        auto share = [&]() {
 #pragma unroll
-        for (int y = 0; y < 8; ++y) {
-            if (owner) fk[y] = q.k[y * 64];
-            if (!maker && (y < 4 || ti)) fp[y] = q.p[y * 64];
-            if (y < 4) {
-                if (maker) w1[y] = q.w1[y * 64];
-                sc[y] = q.sc[2 * y];
+            for (int y = 0; y < 2; ++y) put(Sf, 2 * w + y, dk_split(four(S, 2 * y), four(S, 2 * y + 1)));
+        };
+        share();
+        float4 fk[8], sc[8];                                        // keys, and what is left of a token's correction at the chunk's end
+        float gend;
+        auto fetch = [&](int c) {
+            const float *k = group_of(c);
+            const float *e = head_of(c) + z.p + 3 * 1024;
+#pragma unroll
+            for (int y = 0; y < 8; ++y) { fk[y] = unit_of(k, DP / 4 + 8 * w + y); sc[y] = ((const float4 *)(e + DK_T) + 2 * y)[(uint32_t)hi]; }
+            gend = e[DK_T - 1];
+        };
+        fetch(first);
+        for (int c = first; c < first + n; ++c) {
+            __syncthreads();                                        // S is there, U has been read
+            dk_terms k[4];
+#pragma unroll
+            for (int y = 0; y < 8; ++y) fk[y] = make_float4(fk[y].x * sc[y].x, fk[y].y * sc[y].y, fk[y].z * sc[y].z, fk[y].w * sc[y].w);
+#pragma unroll
+            for (int y = 0; y < 4; ++y) k[y] = dk_split(fk[2 * y], fk[2 * y + 1]);
+            const float end = gend;
+            fetch(after(c));
+            dk_sums sum;
+            dk_clear(sum);
+            __syncthreads();                                        // U is there, S has been read
+#pragma unroll
+            for (int y = 0; y < 4; ++y) dk_mma_split(k[y], get(Uf, y), sum);
+            const dk_f32x16 more = dk_total(sum);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) S[r] = fmaf(S[r], end, more[r]);
+            const int none = min(noneS[0][l32], noneS[1][l32]);
+            if (__any(none < DK_T))                                 // U has zeros instead
+#pragma unroll
+                for (int r = 0; r < 16; ++r) S[r] = none < DK_T ? NAN : S[r];
+            share();
+        }
+        __syncthreads();                                            // the last outputs' pairs are there
+        if (col < Dv)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int d = 32 * w + 8 * (r >> 2) + 4 * hi + (r & 3);
+                if (d < D) sp[(int64_t)d * Dv + col] = S[r];
             }
-        }
-        gend = *q.gend;
+        return;
     }
-    for (int c = first; c < first + n; ++c) {
-        const int row0 = a.chunk_rec[4 * c], cnt = a.chunk_rec[4 * c + 1];
-        const sources q = sources_of(c + 1 < first + n ? c + 1 : c);    // every operand's successor sets out when it has been used: a whole chunk ahead, in its registers
-        __syncthreads();                                            // S is there, U has been read
-        // Short sums that start from nothing, then met: what 128 products in a row lose, or as many onto a W1 larger than they are, is more than the lanes of the other forms do
-        dk_f32x16 acc, part[4];
+    const bool maker = wave < 2;
+    float4 fa[NU];                                                  // what U, or the outputs, take of S
+    auto taken = [&](int c) { return (maker ? head_of(c) + z.w2 : group_of(c)) + ti * NU * 256; };
+    {
+        const float *q = taken(first);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = part[2][r] = part[3][r] = 0.f;
+        for (int u = 0; u < NU; ++u) fa[u] = unit_of(q, u);
+    }
+    dk_terms f[2];
+    // Short sums that start from nothing, then met: what 128 products in a row lose, or as many onto a W1 larger than they are, is more than the lanes of the other forms do
+    auto product = [&](const float *next) {                        // f[0] is there already
+        dk_sums sum;
+        dk_clear(sum);
+        dk_terms s1 = get(Sf, 0);
 #pragma unroll
-        for (int u = 0; u < NU; u += 4) {
-            part[0] = dk_mma(fa[u], Sf[u * 64 + lane], part[0]);
-            part[1] = dk_mma(fa[u + 1], Sf[(u + 1) * 64 + lane], part[1]);
-            part[2] = dk_mma(fa[u + 2], Sf[(u + 2) * 64 + lane], part[2]);
-            part[3] = dk_mma(fa[u + 3], Sf[(u + 3) * 64 + lane], part[3]);
+        for (int s = 0; s < NU / 2; ++s) {
+            const dk_terms s0 = s1;
+            if (s + 1 < NU / 2) {
+                s1 = get(Sf, s + 1);
+                f[(s + 1) & 1] = dk_split(fa[2 * s + 2], fa[2 * s + 3]);
+            }
+            fa[2 * s] = unit_of(next, 2 * s);
+            fa[2 * s + 1] = unit_of(next, 2 * s + 1);
+            dk_mma_split(f[s & 1], s0, sum);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fa[u + i] = q.a[(u + i) * 64];
+            for (int i = 0; i < 6; ++i) {                           // a matrix instruction, and what the next step needs meanwhile
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        acc = (part[0] + part[1]) + (part[2] + part[3]);
-        if (maker) {
+        return dk_total(sum);
+    };
+    if (maker) {
+        float4 w1[4], fp[8];                                        // fp: the pairs
+        auto fetch = [&](int c) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] += ((const float *)&w1[r >> 2])[r & 3];
+            for (int y = 0; y < 4; ++y) w1[y] = unit_of(head_of(c) + z.w1, (vt * 2 + ti) * 4 + y);
+        };
+        auto fetch_pairs = [&](int c) {
+#pragma unroll
+            for (int y = 0; y < 8; ++y) fp[y] = unit_of(head_of(c) + z.p, 4 * ti + y);      // the first half's upper four are not used
+        };
+        fetch(first);
+        fetch_pairs(first);
+        for (int c = first; c < first + n; ++c) {
+            f[0] = dk_split(fa[0], fa[1]);
+            __syncthreads();                                        // S is there, U has been read
+            dk_f32x16 u = product(taken(after(c)));
+#pragma unroll
+            for (int r = 0; r < 16; ++r) u[r] += ((const float *)&w1[r >> 2])[r & 3];
+            fetch(after(c));
             float zero[4] = {0.f, 0.f, 0.f, 0.f};                   // not a number if a correction is not finite
 #pragma unroll
-            for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(acc[r], 0.f, zero[r & 3]);
-            dk_f32x16 u = acc;
+            for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(u[r], 0.f, zero[r & 3]);
             int none = DK_T;
-            if (__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f)) {      // the state takes it up, the outputs of the tokens in front of it must not meet it
+            if (__any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.f)) {      // the outputs of the tokens in front of it must not meet it
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    if (!__builtin_isfinite(acc[r])) { u[r] = 0.f; none = min(none, 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3)); }
+                    if (!__builtin_isfinite(u[r])) { u[r] = 0.f; none = min(none, 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3)); }
                 none = min(none, __shfl_xor(none, 32, 64));
             }
             if (hi == 0) noneS[ti][l32] = none;
 #pragma unroll
-            for (int y = 0; y < 4; ++y) {
-                Uf[(4 * ti + y) * 64 + lane] = make_float4(u[4 * y], u[4 * y + 1], u[4 * y + 2], u[4 * y + 3]);
-                Ug[(4 * ti + y) * 64 + lane] = make_float4(acc[4 * y] * sc[y].x, acc[4 * y + 1] * sc[y].y, acc[4 * y + 2] * sc[y].z, acc[4 * y + 3] * sc[y].w);
-            }
+            for (int y = 0; y < 2; ++y) put(Uf, 2 * ti + y, dk_split(four(u, 2 * y), four(u, 2 * y + 1)));
+            __syncthreads();                                        // U is there, S has been read
+            dk_sums sum;
+            dk_clear(sum);
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+                if (y < 2 || ti) dk_mma_split(dk_split(fp[2 * y], fp[2 * y + 1]), get(Uf, y), sum);
+            fetch_pairs(after(c));
+            const dk_f32x16 o = dk_total(sum);
+#pragma unroll
+            for (int y = 0; y < 4; ++y) Pf[(4 * ti + y) * 64 + lane] = four(o, y);
         }
+        __syncthreads();                                            // the last outputs' pairs are there
+        return;
+    }
+    float4 sc[4];                                                   // what is left of S at a token
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int y = 0; y < 4; ++y) sc[y] = ((const float4 *)(head_of(c) + z.p + 3 * 1024 + 32 * ti) + 2 * y)[(uint32_t)hi];
+    };
+    fetch(first);
+    // A chunk's outputs are stored while the next one's state is made.  Always 16 stores, those of tokens and columns that do not exist beyond the buffer's end: were their number
+    // not known, the next operand's loads, which came before them, could only be waited for together with them
+    dk_f32x16 o, done;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[r] = 0.f;
+    int none = DK_T, none_done, row0 = 0, cnt = 0;
+    const int ld = a.H * Dv;
+    auto add_pairs = [&]() {
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
-            if (maker) { w1[y] = q.w1[y * 64]; sc[y] = q.sc[2 * y]; }
+            const float4 p = Pf[(4 * ti + y) * 64 + lane];
+            done[4 * y] = o[4 * y] + p.x;
+            done[4 * y + 1] = o[4 * y + 1] + p.y;
+            done[4 * y + 2] = o[4 * y + 2] + p.z;
+            done[4 * y + 3] = o[4 * y + 3] + p.w;
         }
-        __syncthreads();                                            // U is there, S has been read
-        if (owner) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = 0.f;
-#pragma unroll
-            for (int y = 0; y < 8; ++y) {
-                part[y >> 2] = dk_mma(fk[y], Ug[y * 64 + lane], part[y >> 2]);
-                fk[y] = q.k[y * 64];
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) S[r] = fmaf(S[r], gend, part[0][r] + part[1][r]);
-            gend = *q.gend;
-            share_state();
-        }
-        if (!maker) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) part[0][r] = part[1][r] = 0.f;
-#pragma unroll
-            for (int y = 0; y < 4; ++y) part[y & 1] = dk_mma(fp[y], Uf[y * 64 + lane], part[y & 1]);
-            if (ti)
-#pragma unroll
-                for (int y = 4; y < 8; ++y) part[y & 1] = dk_mma(fp[y], Uf[y * 64 + lane], part[y & 1]);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] = fmaf(acc[r], ((const float *)&sc[r >> 2])[r & 3], part[0][r] + part[1][r]);
-#pragma unroll
-            for (int y = 0; y < 4; ++y) sc[y] = q.sc[2 * y];
-            const int none = min(noneS[0][l32], noneS[1][l32]);
-            if (__any(none < DK_T))
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[r] = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3) < none ? acc[r] : NAN;
-#pragma unroll
-            for (int y = 0; y < 8; ++y)
-                if (y < 4 || ti) fp[y] = q.p[y * 64];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int t = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3);
-                if (t < cnt && col < Dv) raw[(int64_t)(row0 + t) * ((int64_t)a.H * Dv) + (int64_t)h * Dv + col] = acc[r];
-            }
-        }
-    }
-    if (owner && col < Dv)
+        none_done = none;
+    };
+    auto store = [&]() {
+        const auto to = __builtin_amdgcn_make_buffer_rsrc(raw + ((int64_t)row0 * a.H + h) * Dv, 0, cnt * ld * 4, 0x00020000);
+        const int t0 = 32 * ti + 4 * hi;
+        uint32_t at = col < Dv ? (uint32_t)(t0 * ld + col) * 4 : 0x80000000u;
+        asm("" : "+v"(at));                                         // not sixteen offsets kept over the loop
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int d = 32 * wave + 8 * (r >> 2) + 4 * hi + (r & 3);
-            if (d < D) sp[(int64_t)d * Dv + col] = S[r];
+            const int x = 8 * (r >> 2) + (r & 3);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, t0 + x < none_done ? done[r] : NAN), to, at + x * ld * 4, 0, 0);
         }
+    };
+    for (int c = first; c < first + n; ++c) {
+        f[0] = dk_split(fa[0], fa[1]);
+        __syncthreads();                                            // S is there, U has been read, the pairs' part of the last outputs is there
+        add_pairs();
+        __builtin_amdgcn_sched_barrier(0);
+        o = product(taken(after(c)));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[r] *= ((const float *)&sc[r >> 2])[r & 3];
+        fetch(after(c));
+        __syncthreads();                                            // U is there, S has been read
+        store();                                                    // at first of no tokens
+        none = min(noneS[0][l32], noneS[1][l32]);
+        row0 = __builtin_amdgcn_readfirstlane(a.chunk_rec[4 * c]);
+        cnt = __builtin_amdgcn_readfirstlane(a.chunk_rec[4 * c + 1]);
+    }
+    __syncthreads();                                                // the last outputs' pairs are there
+    add_pairs();
+    store();
 }
 
 template <typename T, int DMAX>
@@ -829,7 +943,7 @@ template <typename T, int DP> static int delta_chunks_launch(const jl_delta_chun
     for (int h0 = 0; h0 < a.H; h0 += a.pass_heads) {                 // as many heads at a time as the scratch holds
         const int nh = a.H - h0 < a.pass_heads ? a.H - h0 : a.pass_heads;
         chunk<<<dim3((unsigned)nh * (unsigned)a.chunks), 256, lds, st>>>(a, h0, nh);
-        delta_chain_kernel<DP><<<dim3((unsigned)((a.B * nh + 7) / 8 * nv * 8)), 256, 0, st>>>(a, h0, nh, a.raw);
+        delta_chain_kernel<DP><<<dim3((unsigned)((a.B * nh + 7) / 8 * nv * 8)), 256 + 2 * DP, 0, st>>>(a, h0, nh, a.raw);
     }
     int rc = jl_check_launch("delta_chunk_kernel");
     if (rc != JL_OK) return rc;
@@ -842,7 +956,7 @@ extern "C" int jl_delta_chunks_run(const jl_delta_chunks *ap, void *stream) {
     if (a.B <= 0 || a.chunks <= 0) return JL_OK;
     if (!a.qkv || !a.proj || !a.A_log || !a.dt_bias || !a.norm_w || !a.chunk_rec || !a.req || !a.state || !a.scratch || !a.raw)
         return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: null pointer");
-    if (!jl_delta_chunks_ok(a.D, a.Dv) || a.H <= 0 || a.G <= 0 || a.H % a.G || a.N <= 0 || (int64_t)a.chunks * a.H > INT32_MAX / 256 || a.pass_heads <= 0 || a.pass_heads % (a.H / a.G) || a.qkv_ld % 4 ||
+    if (!jl_delta_chunks_ok(a.D, a.Dv) || a.H <= 0 || a.G <= 0 || a.H % a.G || a.N <= 0 || (int64_t)a.chunks * a.H > INT32_MAX / 256 || a.pass_heads <= 0 || a.pass_heads % (a.H / a.G) || a.qkv_ld % 4 || a.qkv_ld > 1 << 24 || (int64_t)a.H * a.Dv > 1 << 22 ||
         (a.q_col | a.k_col) % 4 || (((uintptr_t)a.qkv | (uintptr_t)a.scratch) & 15) || (a.dtype != JL_BF16 && a.dtype != JL_F32))
         return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: sizes, columns or alignment (ask jl_delta_chunks_ok)");
     if (a.q_col < 0 || a.k_col < 0 || a.v_col < 0 || a.a_col < 0 || a.b_col < 0 || a.g_col < 0 || a.q_col + (int64_t)a.G * a.D > a.qkv_ld || a.k_col + (int64_t)a.G * a.D > a.qkv_ld ||
