@@ -296,7 +296,7 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
 // that does not exist has k = q = v = 0, beta = 0, g = 1.  ln g below -1e4 counts as -1e4: e^ of it is zero all the same, and differences stay numbers.
 //
 // What is not finite in a token's key, value, decay or beta reaches its own and later tokens' outputs and the state, as in the scan, though products run over whole chunks: it is left
-// out of them and set afterwards (in rare branches: W1's rows from that token on, the outputs' rows from a correction's token on).
+// out of them and set afterwards (in rare branches: W1's rows from that token on, the outputs' rows from a correction's token on, the state's columns).
 //
 // v_mfma_f32_32x32x2_f32: lane l supplies row (A) or column (B) l % 32 at depth l / 32; accumulator r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  Four
 // instructions take a unit of 16 bytes per lane, depths 8 u + 4 (l / 32) + i of unit u — which is also how four accumulators of a lane lie, so results are the next
