@@ -347,8 +347,8 @@ JL_API int jl_retention_join(const int32_t *req, int32_t B, const int32_t *chunk
 
 /* The same for long portions on the matrix cores: every request's portion cut into pieces of piece_tokens (a multiple of 64) tokens, the last of a request
  * what is left, that run side by side (own contributions to the state, the state each starts from, outputs).  piece_rec [pieces, 4] int32 {row0, count, slot,
- * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}; pos [N] int32 position of every row; scratch [pieces, H, D, Dv] and raw
- * [N, H * Dv] float.
+ * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}, of requests that have rows alone (B counts these records: one of no rows
+ * would hide that another has several pieces); pos [N] int32 position of every row; scratch [pieces, H, D, Dv] and raw [N, H * Dv] float.
  * Sizes as jl_retention_pieces_ok takes them; ld and columns in multiples of four, rows and tables at the borders of four elements. */
 typedef struct jl_retention_pieces {
     const void *proj;
@@ -410,7 +410,8 @@ JL_API int jl_delta_chunks_run(const jl_delta_chunks *a, void *stream);
  * slot's old content is ignored); the final state is written back.  out float [N, H*Dv].  D <= 256.
  * `chunks` 0: every request's rows in one scan.  `chunks` > 0 (bfloat16, long portions): the portions are cut into `chunks` pieces that
  * run side by side on the matrix cores — chunk_rec [chunks, 4] int32 {row0, count, slot, 1 for a request's last piece}, every piece but the
- * last a multiple of 64 rows, a request's pieces consecutive; req [B, 4] int32 {first piece, pieces, pos0, slot}; scratch of
+ * last a multiple of 64 rows, a request's pieces consecutive; req [B, 4] int32 {first piece, pieces, pos0, slot}, of requests that have rows alone
+ * (B counts these records: one of no rows would hide that another has several pieces); scratch of
  * chunks * H * (D * Dv + 1) floats; sizes as jl_linear_scan_chunked_ok accepts them, rows and columns in multiples of four elements. */
 typedef struct {
     const void *src; const void *dt; const float *decay; const float *A_log; const float *dt_bias; const float *skip;

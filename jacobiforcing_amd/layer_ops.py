@@ -187,11 +187,14 @@ class RaggedBatch:
 
     def pieces(self, size: int):
         """Every request's portion cut into pieces of ``size`` tokens: (piece records [pieces, 4] int32 {row0, count, slot, 1 for a request's
-        last piece}, request records [B, 4] int32 {first piece, pieces, pos0, slot}), on the device."""
+        last piece}, request records [requests with tokens, 4] int32 {first piece, pieces, pos0, slot}), on the device.  A request without tokens has
+        no record: more pieces than records means that some request has several."""
         key = ("pieces", size)
         if key not in self._tiles:
             rec, req, r0 = [], [], 0
             for c, s, sl in zip(self.counts, self.starts, self.slots):
+                if c == 0:
+                    continue
                 req.append((len(rec), -(-c // size), s, sl))
                 rec += [(r0 + o, min(size, c - o), sl, int(o + size >= c)) for o in range(0, c, size)]
                 r0 += c
@@ -1385,6 +1388,6 @@ def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatc
         size = 64 * max(1, min(8, n * H * -(-Dv // 32) // (SCAN_WAVES * 64)))
         rec, req = batch.pieces(size)
         scratch = torch.empty((rec.shape[0] * H * (D * Dv + 1),), dtype=torch.float32, device=src.device)
-        a.chunk_rec, a.req, a.scratch, a.chunks = p(rec), p(req), p(scratch), rec.shape[0]
+        a.chunk_rec, a.req, a.scratch, a.chunks, a.B = p(rec), p(req), p(scratch), rec.shape[0], req.shape[0]
     N.check_layers(N.layers().jl_linear_scan(C.byref(a), _stream(src.device)), "jl_linear_scan")
     return out

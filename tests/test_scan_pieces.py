@@ -46,3 +46,23 @@ def test_columns_and_heads(monkeypatch, H, G, D, Dv, counts, fixed):
                 assert float((got[r0 + t].double().view(H, Dv) - o).norm() / o.norm().clamp_min(1e-3 * D ** 0.5)) < 2e-5, (b, t)
             assert float((st[b].double() - S).norm() / S.norm()) < 2e-5
             r0 += n
+
+
+@pytest.mark.parametrize("op", ["scan", "retention"])
+def test_requests_without_tokens(monkeypatch, op):
+    """Beside as many pieces as there are requests, two of them one request's: as without the request that has none, and its state stays."""
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "SCAN_WAVES", 1 << 20)           # pieces of one group each
+    monkeypatch.setattr(LO, "RETENTION_WORKGROUPS", 1 << 20)
+    g, H, D = torch.Generator(device="cuda").manual_seed(5), 2, 64
+    x, start, decay = torch.randn(128, 4 * H * D, generator=g, device="cuda").bfloat16(), torch.randn(2, H, D, D, generator=g, device="cuda"), torch.full((H,), 0.97, device="cuda")
+    got = []
+    for counts in ([0, 128], [128]):
+        b, st = LO.RaggedBatch.build(counts, [0] * len(counts), [0, 1][-len(counts):], [[0, 1]] * len(counts), 64, "cuda"), start.clone()
+        if op == "scan":
+            o = LO.linear_scan(x, (0, H * D, 2 * H * D), b, H, H, D, D, st, decay=decay)
+        else:
+            o = LO.retention(x, (0, H * D, 2 * H * D, 3 * H * D), b, H, D, D, 0, None, None, decay, 1e-5, st)
+        assert [len(v[0]) for k, v in b._tiles.items() if isinstance(k, tuple) and k[0] == "pieces"] == [2]
+        got.append((o, st))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][0], start[0])

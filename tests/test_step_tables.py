@@ -89,3 +89,10 @@ def test_the_rule_is_the_cheapest_of_its_estimates(seed):
             n = -(-c[c >= m] // 64)
             ways[m] = first + max(chain * int(n.max()), chunk * int(n.sum()) * H) + others(c[c < m])
         assert ways[LO.delta_chunks_from(counts, H, D)] == min(ways.values())
+
+
+def test_requests_without_tokens_have_no_record_of_pieces():
+    """The launches tell from more pieces than records that some request has several."""
+    b = batch([0, 128, 0, 5], [7, 0, 0, 64])
+    rec, req = b.pieces(64)
+    assert rec.tolist() == [[0, 64, 1, 0], [64, 64, 1, 1], [128, 5, 3, 1]] and req.tolist() == [[0, 2, 0, 1], [2, 1, 64, 3]]
