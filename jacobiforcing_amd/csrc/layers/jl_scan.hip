@@ -26,7 +26,7 @@ __global__ __launch_bounds__(64) void scan_kernel(jl_scan_args a) {
     const int b = blockIdx.x / H, h = blockIdx.x - b * H, kh = h / (H / a.G);
     const int row0 = a.seq[4 * b], cnt = a.seq[4 * b + 1], pos0 = a.seq[4 * b + 2], slot = a.seq[4 * b + 3];
     if (cnt <= 0) return;
-    const int lane = threadIdx.x, j = blockIdx.y * SC_COLS + (lane >> 1), sub = lane & 1, d0 = sub * DPER;
+    const int lane = threadIdx.x, j = (blockIdx.z * gridDim.y + blockIdx.y) * SC_COLS + (lane >> 1), sub = lane & 1, d0 = sub * DPER;
     const bool live = j < Dv;
     const T *src = (const T *)a.src, *dtp = (const T *)a.dt;
     const bool fixed = a.decay != nullptr, act = a.act == JL_ACT_SILU;
@@ -102,7 +102,8 @@ __global__ __launch_bounds__(64) void scan_kernel(jl_scan_args a) {
 }
 
 template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t st) {
-    const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.Dv + SC_COLS - 1) / SC_COLS));
+    const unsigned cols = (unsigned)((a.Dv + SC_COLS - 1) / SC_COLS), y = cols < 65535 ? cols : 65535;      // (a launch's second dimension ends there)
+    const dim3 grid((unsigned)(a.B * a.H), y, (cols + y - 1) / y);
     if (a.D <= 32) scan_kernel<T, 32><<<grid, 64, 0, st>>>(a);
     else if (a.D <= 64) scan_kernel<T, 64><<<grid, 64, 0, st>>>(a);
     else if (a.D <= 128) scan_kernel<T, 128><<<grid, 64, 0, st>>>(a);
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
     auto outputs = [&](int t0, int n) {
         const int64_t o_ld = (int64_t)H * Dv;
         char *to = (char *)(a.out + (row0 + t0) * o_ld + (int64_t)h * Dv + c_base);
-        const uint32_t o_row = (uint32_t)o_ld * 4;                  // (64 rows of outputs lie within 32 bits)
+        const uint32_t o_row = (uint32_t)o_ld * 4;                  // (ch_in_reach)
         uint32_t off = 4 * hi * o_row + 4 * l32;
         auto store = [&](auto whole) {
 #pragma unroll
@@ -483,6 +484,9 @@ template <int DP> static int scan_chunk_launch(const jl_scan_args &a, hipStream_
 
 extern "C" int jl_linear_scan_chunked_ok(int dtype, int32_t D, int32_t Dv) { return dtype == JL_BF16 && D > 0 && D <= 128 && D % 4 == 0 && Dv > 0 && Dv % 4 == 0; }
 
+// The pieces' kernel forms offsets of 64 rows of outputs and of src, and of a head's state, in 32 bits; wider calls take the scan.
+static bool ch_in_reach(const jl_scan_args &a) { return (int64_t)a.H * a.Dv <= 1 << 24 && a.Dv <= 1 << 22 && a.ld <= 1 << 26; }
+
 extern "C" int jl_linear_scan(const jl_scan_args *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_linear_scan: null arguments");
     const jl_scan_args &a = *ap;
@@ -498,10 +502,12 @@ extern "C" int jl_linear_scan(const jl_scan_args *ap, void *stream) {
         if (!a.chunk_rec || !a.req || !a.scratch) return jl_fail(JL_E_INVALID, "jl_linear_scan: pieces need their records and a scratch");
         if (!jl_linear_scan_chunked_ok(a.dtype, a.D, a.Dv) || a.ld % 4 || a.q_col % 4 || a.k_col % 4 || a.v_col % 4 || (uintptr_t)a.src % 8)
             return jl_fail(JL_E_INVALID, "jl_linear_scan: pieces take bfloat16, D a multiple of four up to 128, Dv, columns and rows in multiples of four");
-        if (a.D <= 32) return scan_chunk_launch<32>(a, st);
-        if (a.D <= 64) return scan_chunk_launch<64>(a, st);
-        if (a.D <= 96) return scan_chunk_launch<96>(a, st);
-        return scan_chunk_launch<128>(a, st);
+        if (ch_in_reach(a)) {
+            if (a.D <= 32) return scan_chunk_launch<32>(a, st);
+            if (a.D <= 64) return scan_chunk_launch<64>(a, st);
+            if (a.D <= 96) return scan_chunk_launch<96>(a, st);
+            return scan_chunk_launch<128>(a, st);
+        }
     }
     JL_DISPATCH(a.dtype, return scan_launch<T>(a, st));
     return JL_OK;

@@ -1383,6 +1383,7 @@ def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatc
                    ld=src.stride(0), dt_ld=dt.stride(0) if decay is None else 0, N=n, q_col=cols[0], k_col=cols[1], v_col=cols[2], dt_col=0, dtype=_code(src.dtype),
                    act=int(act), B=batch.B, H=H, G=G, D=D, Dv=Dv)
     if (max(batch.counts) >= SCAN_PIECES_FROM and not os.environ.get("JL_SCAN_NO_PIECES") and a.ld % 4 == 0 and all(c % 4 == 0 for c in cols) and    # A/B switch for measurements
+            H * Dv <= 1 << 24 and Dv <= 1 << 22 and a.ld <= 1 << 26 and         # their kernel's offsets of 32 bits; the library sends wider calls to the scan by itself
             N.layers().jl_linear_scan_chunked_ok(a.dtype, D, Dv)):
         # long portions: pieces side by side on the matrix cores, as many as fill the chip with two wavefronts per SIMD, each at least one group of 64 tokens
         size = 64 * max(1, min(8, n * H * -(-Dv // 32) // (SCAN_WAVES * 64)))

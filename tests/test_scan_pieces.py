@@ -66,3 +66,31 @@ def test_requests_without_tokens(monkeypatch, op):
         assert [len(v[0]) for k, v in b._tiles.items() if isinstance(k, tuple) and k[0] == "pieces"] == [2]
         got.append((o, st))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][0], start[0])
+
+
+@pytest.mark.parametrize("pieces", [False, True])
+def test_rows_wider_than_the_offsets_of_pieces(monkeypatch, pieces):
+    """Rows of outputs whose 64th lies beyond 2 ** 32 bytes, columns beyond a launch's second dimension: in one scan, also where the library is handed pieces."""
+    from jacobiforcing_amd import layer_ops as LO
+    lib, H, D, Dv, n = LO.N.layers(), 9, 4, (1 << 21) + 64, 40
+    g = torch.Generator(device="cuda").manual_seed(9)
+    batch = LO.RaggedBatch.build([n], [0], [0], [[0]], 64, "cuda")
+    if pieces:
+        real, (rec, req) = lib.jl_linear_scan, LO.RaggedBatch.pieces(batch, 64)
+        scratch = torch.empty(H * (D * Dv + 1), device="cuda")
+
+        def handed(ap, st):
+            a = ap._obj
+            a.chunk_rec, a.req, a.scratch, a.chunks = rec.data_ptr(), req.data_ptr(), scratch.data_ptr(), rec.shape[0]
+            return real(ap, st)
+        monkeypatch.setattr(lib, "jl_linear_scan", handed, raising=False)
+    x = torch.empty(n, 2 * D + H * Dv, device="cuda", dtype=torch.bfloat16).normal_(generator=g)
+    state, decay = torch.full((1, H, D, Dv), float("nan"), device="cuda"), torch.linspace(0.5, 1.0, H, device="cuda")
+    out = LO.linear_scan(x, (0, D, 2 * D), batch, H, 1, D, Dv, state, decay=decay).view(n, H, Dv)
+    assert pieces or ("pieces", 64) not in batch._tiles
+    q, k, back = x[:, :D].double(), x[:, D:2 * D].double(), torch.arange(n, device="cuda").view(n, 1) - torch.arange(n, device="cuda")
+    for h, c in ((0, 0), (4, 1 << 20), (8, Dv - 64)):
+        fade = (decay[h].double() ** back.clamp_min(0)).tril()
+        v = x[:, 2 * D + h * Dv + c:2 * D + h * Dv + c + 64].double()
+        want, S = (q @ k.T * fade) @ v, (k * fade[-1:].T).T @ v
+        assert (out[:, h, c:c + 64] - want).norm() <= 2e-6 * want.norm() and (state[0, h, :, c:c + 64] - S).norm() <= 2e-6 * S.norm(), (h, c)
