@@ -4,6 +4,7 @@
 // with q, k unit vectors per head (q also times q_scale), beta = sigmoid(b) and g = exp(-exp(A_log_h) softplus(a + dt_bias_h)) per head and
 // token, and the output brought to unit RMS per head, times a weight over Dv, times silu(gate).  Everything but the inputs is float.
 #include "jl_common.h"
+#include <type_traits>
 
 // One workgroup per (request, head).  The columns of S are independent of each other, so column j is owned by LPC adjacent lanes, each
 // with DMAX / LPC consecutive rows in registers; the two dot products of a token (k . S_j and q . S_j) are partial sums per lane joined by
@@ -369,8 +370,10 @@ static __host__ __device__ inline dk_sizes dk_layout(int DP, int Dv) {
     return z;
 }
 
-template <typename T, int DP>
+// FAR: rows of qkv of which 64 are not within 32 bits of each other (where they are, offsets of 64 bits cost registers and 5 to 20 % of a launch)
+template <typename T, int DP, bool FAR>
 __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, int h0, int nh) {
+    typedef typename std::conditional<FAR, int64_t, uint32_t>::type row_t;
     constexpr int U = DP / 4, DT = DP / 32;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float4 *Ks = (float4 *)smem, *Qs = Ks + DK_T * U, *Am = Qs + DK_T * U;          // rows of units, permuted by the row
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 #pragma unroll
     for (int it = 0; it < IT; ++it) {                                              // a row that does not exist: the last one's, not used
         const int e = tid + it * 256, tt = min(e / U, cnt - 1), d = 4 * (e % U) < D ? 4 * (e % U) : 0;
-        const uint32_t at = (uint32_t)tt * (uint32_t)a.qkv_ld + d;
+        const row_t at = (row_t)tt * (row_t)a.qkv_ld + d;
         qv[it] = *(const float4 *)(src + a.q_col + at);
         kv[it] = *(const float4 *)(src + a.k_col + at);
     }
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
     auto fetch_v = [&](int vt) {
         const int col = min(32 * vt + l32, Dv - 1);
 #pragma unroll
-        for (int i = 0; i < 32; ++i) vv[i] = vp[(uint32_t)min(8 * (i >> 2) + 4 * hi + (i & 3), cnt - 1) * (uint32_t)a.qkv_ld + col];
+        for (int i = 0; i < 32; ++i) vv[i] = vp[(row_t)min(8 * (i >> 2) + 4 * hi + (i & 3), cnt - 1) * (row_t)a.qkv_ld + col];
     };
     __syncthreads();
     // from the first token with a key, decay or beta that is not a number on: nothing here that zeros would spread to the tokens in front of it; W1 says so instead
@@ -598,7 +601,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int t = 8 * y + 4 * hi + i;
-                        v[i] = t < cnt && col < Dv ? vp[(uint32_t)t * (uint32_t)a.qkv_ld + col] * bs[t] : 0.f;
+                        v[i] = t < cnt && col < Dv ? vp[(row_t)t * (row_t)a.qkv_ld + col] * bs[t] : 0.f;
                         if (!__builtin_isfinite(v[i])) { v[i] = 0.f; none = min(none, t); }
                     }
                     if (y < 4) acc[0] = dk_mma(trow(0, y), make_float4(v[0], v[1], v[2], v[3]), acc[0]);
@@ -643,7 +646,8 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(jl_delta_chunks a, 
 
 // Workgroup (request, head, 32 columns); the column blocks of a head lie eight apart, on one XCD, since they read the same operands.  Wavefronts 0 and 1 make U, 2 and 3 the
 // outputs of 32 tokens each; the D / 32 that follow own 32 rows of S each.  What a wavefront takes from memory is split while another's matrix instructions run: two to a SIMD.
-template <int DP>
+// WIDE: rows of outputs of which 64 lie further apart than a buffer reaches.
+template <int DP, bool WIDE>
 __global__ __launch_bounds__(256 + 2 * DP, 1) void delta_chain_kernel(jl_delta_chunks a, int h0, int nh, float *__restrict__ raw) {
     constexpr int NU = DP / 8;
     __shared__ jl_bf16x8 Sf[NU / 2 * 3 * 64], Uf[4 * 3 * 64];       // [16 depths][term][lane]
@@ -833,6 +837,14 @@ __global__ __launch_bounds__(256 + 2 * DP, 1) void delta_chain_kernel(jl_delta_c
         none_done = none;
     };
     auto store = [&]() {
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int t = 32 * ti + 8 * (r >> 2) + 4 * hi + (r & 3);
+                if (t < cnt && col < Dv) raw[((int64_t)(row0 + t) * a.H + h) * Dv + col] = t < none_done ? done[r] : NAN;
+            }
+            return;
+        }
         const auto to = __builtin_amdgcn_make_buffer_rsrc(raw + ((int64_t)row0 * a.H + h) * Dv, 0, cnt * ld * 4, 0x00020000);
         const int t0 = 32 * ti + 4 * hi;
         uint32_t at = col < Dv ? (uint32_t)(t0 * ld + col) * 4 : 0x80000000u;
@@ -936,14 +948,15 @@ extern "C" int64_t jl_delta_chunks_floats(int32_t chunks, int32_t heads, int32_t
 
 template <typename T, int DP> static int delta_chunks_launch(const jl_delta_chunks &a, hipStream_t st) {
     const size_t lds = (size_t)(2 * DK_T * DP + 3 * 1024 + 3 * DK_T) * 4 + DK_T * 8;
-    auto chunk = delta_chunk_kernel<T, DP>;
+    auto chunk = a.qkv_ld > 1 << 26 ? delta_chunk_kernel<T, DP, true> : delta_chunk_kernel<T, DP, false>;
     hipError_t e = hipFuncSetAttribute((const void *)chunk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_delta_chunks_run: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     const int nv = (a.Dv + 31) / 32;
+    const bool wide = (int64_t)a.H * a.Dv > 1 << 22;                 // 2 GiB of 64 rows and what lies behind them
     for (int h0 = 0; h0 < a.H; h0 += a.pass_heads) {                 // as many heads at a time as the scratch holds
         const int nh = a.H - h0 < a.pass_heads ? a.H - h0 : a.pass_heads;
         chunk<<<dim3((unsigned)nh * (unsigned)a.chunks), 256, lds, st>>>(a, h0, nh);
-        delta_chain_kernel<DP><<<dim3((unsigned)((a.B * nh + 7) / 8 * nv * 8)), 256 + 2 * DP, 0, st>>>(a, h0, nh, a.raw);
+        (wide ? delta_chain_kernel<DP, true> : delta_chain_kernel<DP, false>)<<<dim3((unsigned)((a.B * nh + 7) / 8 * nv * 8)), 256 + 2 * DP, 0, st>>>(a, h0, nh, a.raw);
     }
     int rc = jl_check_launch("delta_chunk_kernel");
     if (rc != JL_OK) return rc;
@@ -956,7 +969,7 @@ extern "C" int jl_delta_chunks_run(const jl_delta_chunks *ap, void *stream) {
     if (a.B <= 0 || a.chunks <= 0) return JL_OK;
     if (!a.qkv || !a.proj || !a.A_log || !a.dt_bias || !a.norm_w || !a.chunk_rec || !a.req || !a.state || !a.scratch || !a.raw)
         return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: null pointer");
-    if (!jl_delta_chunks_ok(a.D, a.Dv) || a.H <= 0 || a.G <= 0 || a.H % a.G || a.N <= 0 || (int64_t)a.chunks * a.H > INT32_MAX / 256 || a.pass_heads <= 0 || a.pass_heads % (a.H / a.G) || a.qkv_ld % 4 || a.qkv_ld > 1 << 24 || (int64_t)a.H * a.Dv > 1 << 22 ||
+    if (!jl_delta_chunks_ok(a.D, a.Dv) || a.H <= 0 || a.G <= 0 || a.H % a.G || a.N <= 0 || (int64_t)a.chunks * a.H > INT32_MAX / 256 || a.pass_heads <= 0 || a.pass_heads % (a.H / a.G) || a.qkv_ld % 4 ||
         (a.q_col | a.k_col) % 4 || (((uintptr_t)a.qkv | (uintptr_t)a.scratch) & 15) || (a.dtype != JL_BF16 && a.dtype != JL_F32))
         return jl_fail(JL_E_INVALID, "jl_delta_chunks_run: sizes, columns or alignment (ask jl_delta_chunks_ok)");
     if (a.q_col < 0 || a.k_col < 0 || a.v_col < 0 || a.a_col < 0 || a.b_col < 0 || a.g_col < 0 || a.q_col + (int64_t)a.G * a.D > a.qkv_ld || a.k_col + (int64_t)a.G * a.D > a.qkv_ld ||

@@ -1337,8 +1337,7 @@ def delta_rule(qkv: torch.Tensor, cols: Tuple[int, int, int], proj: torch.Tensor
         longest, least = 1, 0
     raw = torch.empty((n, H * Dv), dtype=torch.float32, device=proj.device) if longest >= DELTA_COLUMNS_FROM else None
     seq, B = batch.seq, batch.B
-    if (least and N.layers().jl_delta_chunks_ok(D, Dv) and (qkv.shape[1] | cols[0] | cols[1]) % 4 == 0 and qkv.data_ptr() % 16 == 0 and
-            qkv.shape[1] <= 1 << 24 and H * Dv <= 1 << 22):                     # 64 rows' offsets in 32 bits
+    if (least and N.layers().jl_delta_chunks_ok(D, Dv) and (qkv.shape[1] | cols[0] | cols[1]) % 4 == 0 and qkv.data_ptr() % 16 == 0):
         rec, req, seq, longest = batch.long_pieces(64, least)
         B, chunks, per = seq.shape[0], rec.shape[0], H // G
         floats = lambda heads: N.layers().jl_delta_chunks_floats(chunks, heads, H, G, D, Dv)

@@ -151,3 +151,27 @@ def test_chunks_lose_no_more_bits_than_the_columns(H, G, D, lo, hi):
             for name, a, b in (("out", got.double().view(n, H, D), o), ("state", st[0].double(), S)):
                 errs[name, form] = errs.get((name, form), 0.0) + ((a - b).norm() / b.norm()).item()
     assert errs["state", 64] <= errs["state", 0] and errs["out", 64] <= 7 / 6 * errs["out", 0], errs
+
+
+@pytest.mark.parametrize("H,G,Dv,ld", [(4100, 1025, 1024, 0), (4, 2, 40, (1 << 26) + 8)])
+def test_wide_rows(H, G, Dv, ld):
+    """Rows of outputs of which 64 lie beyond what a buffer store reaches (and a chunk's last row far beyond 32 bits of bytes in qkv): as the form in columns."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, g, n, D = "cuda", torch.Generator(device="cuda").manual_seed(H), 70, 4
+    width = 2 * G * D + H * Dv
+    qkv, at = torch.empty(n, max(ld, width), device=dev), max(ld, width) - width
+    qkv[:, at:].normal_(generator=g)
+    proj = torch.empty(n, 2 * H + H * Dv, device=dev, dtype=torch.bfloat16).normal_(generator=g)
+    a_log, bias, w, start = (torch.randn(*s, generator=g, device=dev) for s in ((H,), (H,), (Dv,), (1, H, D, Dv)))
+    got = []
+    for form in (64, 0):
+        batch, st = LO.RaggedBatch.build([n], [5], [0], [[0, 1]], 64, dev), start.clone()
+        batch._tiles[("delta", H, D)] = form
+        out = LO.delta_rule(qkv, (at, at + G * D, at + 2 * G * D), proj, (0, H, 2 * H), a_log, bias, w, batch, H, G, D, Dv, 1e-6, 0.5, 1e-5, st)
+        assert any(k[0] == "long" for k in batch._tiles if isinstance(k, tuple)) == (form > 0)
+        got.append((out.view(n, H, Dv), st[0]))
+    for h in (0, H // 2, H - 1):
+        # 32-bit sums in another order, outputs rounded to 8 bits
+        o = [(x[0][:, h].double(), x[1][h].double()) for x in got]
+        assert (o[0][0] - o[1][0]).norm() <= 2.0 ** -8 * o[1][0].norm() and (o[0][1] - o[1][1]).norm() <= 4e-6 * o[1][1].norm(), h
+    assert bool(got[0][0].isfinite().all()) and bool(got[0][1].isfinite().all())
