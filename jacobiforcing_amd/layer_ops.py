@@ -8,6 +8,7 @@ from __future__ import annotations
 import bisect
 import ctypes as C
 import itertools
+import operator
 import os
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
@@ -127,13 +128,18 @@ class RaggedBatch:
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
               page_size: int, device) -> "RaggedBatch":
         B = len(counts)
-        held = list(map(len, block_tables))              # pages of each request
+        if len(starts) != B or len(slots) != B:
+            raise ValueError(f"{B} requests, {len(starts)} starts, {len(slots)} slots")
+        held = list(map(len, block_tables))              # pages of each request (tables of more requests count in the tables' width alone)
+        C_, block_tables, held = max(1, max(held)), block_tables[:B], held[:B]
         for b in range(B):
             if counts[b] and (starts[b] + counts[b] + page_size - 1) // page_size > held[b]:
                 raise ValueError(f"request {b}: {held[b]} pages do not hold {starts[b] + counts[b]} tokens")
-        counts, starts, slots = list(map(int, counts)), list(map(int, starts)), list(map(int, slots))
+        counts, starts, slots = list(map(int, counts)), list(map(operator.index, starts)), list(map(int, slots))
+        if min(counts) < 0:
+            raise ValueError("a request of fewer than no tokens")
         row0 = list(itertools.accumulate(counts, initial=0))
-        N_, C_ = row0[B], max(1, max(held))
+        N_ = row0[B]
         # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on; `whole`: tiles() of steps whose requests are one tile each
         seq = [x for r in zip(row0, counts, starts, slots) for x in r]
         whole = [x for r in zip(range(B), starts, counts, row0) for x in r]

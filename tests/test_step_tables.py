@@ -96,3 +96,16 @@ def test_requests_without_tokens_have_no_record_of_pieces():
     b = batch([0, 128, 0, 5], [7, 0, 0, 64])
     rec, req = b.pieces(64)
     assert rec.tolist() == [[0, 64, 1, 0], [64, 64, 1, 1], [128, 5, 3, 1]] and req.tolist() == [[0, 2, 0, 1], [2, 1, 64, 3]]
+
+
+def test_what_a_batch_is_built_of():
+    """Page tables beyond the requests' are left out, but for the tables' width; lists of other lengths, positions that are not whole and counts below zero are refused."""
+    build = lambda counts=[1, 70], starts=[2, 0], slots=[0, 1], tables=[[1], [2, 3], [4, 5, 6]]: LO.RaggedBatch.build(counts, starts, slots, tables, 64, "cpu")
+    for counts in ([1, 70], [1, 1]):
+        b = build(counts)
+        assert b.tables.tolist() == [[1, -1, -1], [2, 3, -1]] and b.kv_slot[:2].tolist() == [66, 128] and b.max_page == 3
+    whole = build(tables=torch.tensor([[1, 7], [2, 3], [4, 5]], dtype=torch.int32))
+    assert whole.tables.tolist() == [[1, 7], [2, 3]] and whole.kv_slot[-1] == 3 * 64 + 5
+    for bad in (dict(starts=[2, 0, 1]), dict(slots=[0, 1, 2]), dict(slots=[0]), dict(starts=[2.0, 0]), dict(counts=[1, -1]), dict(tables=[[1]])):
+        with pytest.raises((ValueError, TypeError, IndexError)):
+            build(**bad)
