@@ -10,7 +10,8 @@ import ctypes as C
 import itertools
 import operator
 import os
-from dataclasses import dataclass
+from collections import deque
+from dataclasses import dataclass, field
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -73,21 +74,34 @@ def _dev(t: torch.Tensor) -> None:
 
 
 _UPLOADS: dict = {}                                  # device index -> the stream its tables are copied on, and a block of its pool
+_GONE: dict = {}                                     # (device index, stream) -> tables uploaded from that stream whose batch is gone
 
 
-def _upload(host: np.ndarray, device) -> torch.Tensor:
-    """``host`` on ``device``, there when this returns.  A copy from ordinary host memory waits for its stream: on one of its own it waits for itself and not for the kernels queued so far (a
-    decoding step of 32 requests, kernels of 500 us: 650 -> 520 us a pass).  The memory goes back to that stream's pool once the current stream is done with it."""
+def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
+    """``host`` on ``device``, there for every stream when this returns.  A copy from ordinary host memory waits for its stream: on one of its own it waits for itself and not for the kernels
+    queued so far.  That shows where passes queue behind one another (us a pass, tables on the kernels' stream / on this one: 32 decoding requests of Mikipel 860 / 796, 4 prompts of 2048 of Lokizen
+    2402 / 2301); on an idle stream an upload costs about 10 us more (one token of Safisun 619 / 637).
+    The tensor joins ``held``, the batch's list.  Its memory goes back to the copies' stream once the stream that asked for it is done with what lies in front of its first upload behind the batch's
+    end: what a caller makes that stream wait for until then (kernels of another stream that read the tables) comes first, as it did when the memory was that stream's own."""
     device = torch.device(device)
     t = torch.from_numpy(host)
     if device.type != "cuda":
         return t.to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a step's tables cannot be copied while a graph is captured")
     index = torch.cuda.current_device() if device.index is None else device.index
     if index not in _UPLOADS:
         side = torch.cuda.Stream(index)
         with torch.cuda.stream(side):                    # a block that stays keeps the pool's first segment (2 MB) from being given back and asked for again
             _UPLOADS.setdefault(index, (side, torch.empty(1, dtype=torch.int32, device=device)))
     side, user = _UPLOADS[index][0], torch.cuda.current_stream(index)
+    key = index, user.cuda_stream
+    gone = _GONE.get(key)
+    while gone:
+        try:
+            gone.popleft().record_stream(user)
+        except IndexError:                               # another thread took the last one
+            break
     if index == torch.cuda.current_device():             # half of what the context below takes
         torch.cuda.set_stream(side)
         try:
@@ -97,7 +111,8 @@ def _upload(host: np.ndarray, device) -> torch.Tensor:
     else:
         with torch.cuda.stream(side):
             up = t.to(device)
-    up.record_stream(user)
+    up.record_stream(user)                               # (views of it may outlive the batch)
+    held.append((key, up))
     return up
 
 
@@ -121,8 +136,13 @@ class RaggedBatch:
     max_slot: int
     slots: List[int]
     _tiles: dict
-    _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
     _host_tables: Optional[np.ndarray] = None         # tables on the host, for key_rows and part (None: read back when they need it)
+    _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
+    _held: list = field(default_factory=list, repr=False, compare=False)      # what was uploaded for it, with the stream that asked
+
+    def __del__(self, gone=_GONE):
+        for key, t in self.__dict__.get("_held", ()):
+            gone.setdefault(key, deque()).append(t)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
@@ -164,12 +184,13 @@ class RaggedBatch:
             pos = np.arange(N_, dtype=np.int64) + np.repeat(np.asarray(starts) - row0[:B], c)
             words[a_req:a_req + N_], words[a_pos:a_pos + N_] = np.repeat(np.arange(B, dtype=np.int32), c), pos
             host[:N_] = pages[np.repeat(np.cumsum(held) - held, c) + pos // page_size] * page_size + pos % page_size
-        up = _upload(host, device)
+        held_by = []
+        up = _upload(host, device, held_by)
         w32 = up.view(torch.int32)
         d_seq, d_bt, d_req, d_pos, d_whole = (w32[a:a + n] for n, a in zip(sizes, at))
         return cls(B=B, N=N_, counts=counts, starts=starts, seq=d_seq.view(B, 4), kv_slot=up[:N_], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos, page_size=int(page_size),
                    max_pos=max(s + c for s, c in zip(starts, counts)), max_page=int(bt.max()), max_slot=max(slots), slots=slots, _tiles={}, _host_tables=bt,
-                   _whole=(max(counts), d_whole.view(B, 4)) if min(counts) > 0 else None)
+                   _whole=(max(counts), d_whole.view(B, 4)) if min(counts) > 0 else None, _held=held_by)
 
     def chunks(self, size: int):
         """A portion of at least two chunks is cut into chunks of ``size`` tokens that the recurrent layers run side by side.
@@ -187,7 +208,7 @@ class RaggedBatch:
                         rec.append((int(seq[b, 0]) + o, min(size, c - o), s + o, len(rec)))
                 dev = self.seq.device
                 rec = np.asarray(rec, dtype=np.int32).reshape(-1, 4)
-                plan = (_upload(rec, dev), _upload(np.ascontiguousarray(rec[:, 1]), dev), _upload(np.asarray(req, dtype=np.int32).reshape(-1, 4), dev))
+                plan = tuple(_upload(t, dev, self._held) for t in (rec, np.ascontiguousarray(rec[:, 1]), np.asarray(req, dtype=np.int32).reshape(-1, 4)))
             self._tiles[key] = plan
         return self._tiles[key]
 
@@ -204,7 +225,7 @@ class RaggedBatch:
                 req.append((len(rec), -(-c // size), s, sl))
                 rec += [(r0 + o, min(size, c - o), sl, int(o + size >= c)) for o in range(0, c, size)]
                 r0 += c
-            both = _upload(np.asarray(rec + req, dtype=np.int32).reshape(-1, 4), self.seq.device)
+            both = _upload(np.asarray(rec + req, dtype=np.int32).reshape(-1, 4), self.seq.device, self._held)
             self._tiles[key] = (both[:len(rec)], both[len(rec):])
         return self._tiles[key]
 
@@ -220,7 +241,7 @@ class RaggedBatch:
                 else:
                     rest.append((r0, c, s, sl))
                 r0 += c
-            every = _upload(np.asarray(rec + req + rest, dtype=np.int32).reshape(-1, 4), self.seq.device)
+            every = _upload(np.asarray(rec + req + rest, dtype=np.int32).reshape(-1, 4), self.seq.device, self._held)
             self._tiles[key] = (every[:len(rec)], every[len(rec):len(rec) + len(req)], every[len(rec) + len(req):], max((r[1] for r in rest), default=0))
         return self._tiles[key]
 
@@ -247,7 +268,7 @@ class RaggedBatch:
                 host[at:at + end - first] = (pages[b, p0:(end - 1) // size + 1, None] + within).ravel()[first - p0 * size:end - p0 * size]
                 base[b] = at - first
                 at += end - first
-            up = _upload(host, self.seq.device)
+            up = _upload(host, self.seq.device, self._held)
             self._tiles[key] = (up[:total], up[total:].view(torch.int32)[:self.B])
         return self._tiles[key]
 
@@ -259,7 +280,7 @@ class RaggedBatch:
             rows = np.concatenate([np.arange(row0[b], row0[b + 1], dtype=np.int64) for b in requests])
             sub = RaggedBatch.build([self.counts[b] for b in requests], [self.starts[b] for b in requests], [self.slots[b] for b in requests],
                                     [self._pages()[b] for b in requests], self.page_size, self.seq.device)
-            self._tiles[key] = (sub, _upload(rows, self.seq.device))
+            self._tiles[key] = (sub, _upload(rows, self.seq.device, self._held))
         return self._tiles[key]
 
     def tiles(self, tq: int, longest_first: bool = False, requests: Optional[Sequence[int]] = None) -> torch.Tensor:
@@ -277,7 +298,7 @@ class RaggedBatch:
                 r0 += c
             if longest_first:
                 rows.sort(key=lambda r: -r[1])
-            t = self._tiles[key] = _upload(np.asarray(rows, dtype=np.int32).reshape(-1, 4), self.seq.device)
+            t = self._tiles[key] = _upload(np.asarray(rows, dtype=np.int32).reshape(-1, 4), self.seq.device, self._held)
         return t
 
 

@@ -65,3 +65,35 @@ def test_tables_do_not_wait_and_last():
     assert not done.query(), "the tables waited for the queue"
     torch.cuda.synchronize()
     assert got.tolist() == [tables([40], [i], [0], [list(range(i, i + 8))], 64)[1] for i in range(200)] and bool(y.isfinite().all())
+
+
+@pytest.mark.gpu
+def test_tables_that_another_stream_reads():
+    """A batch built on one stream, read behind a queue on another and dropped: its memory is not written before the first stream, which waits for the other, is through."""
+    x, other, here = torch.randn(8192, 8192, device="cuda").bfloat16(), torch.cuda.Stream(), torch.cuda.current_stream()
+    for start in (7, 3):
+        b = LO.RaggedBatch.build([40], [start], [0], [[5, 9, 2]], 64, "cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            for _ in range(20):
+                y = x @ x
+            seen = torch.stack([b.kv_slot, b.kv_slot])[1]
+        del b
+        here.wait_stream(other)
+        more = [LO.RaggedBatch.build([40], [i], [0], [list(range(i, i + 8))], 64, "cuda") for i in range(20)]
+        torch.cuda.synchronize()
+        assert seen.tolist() == tables([40], [start], [0], [[5, 9, 2]], 64)[1] and bool(y.isfinite().all())
+        assert all(m.kv_slot.tolist() == tables([40], [i], [0], [list(range(i, i + 8))], 64)[1] for i, m in enumerate(more))
+
+
+@pytest.mark.gpu
+def test_tables_are_refused_in_a_capture():
+    """... before anything that would leave an error behind."""
+    build = lambda: LO.RaggedBatch.build([3, 1], [0, 5], [0, 1], [[0], [1]], 64, "cuda")
+    b = build()
+    with pytest.raises(RuntimeError, match="captured"), torch.cuda.graph(torch.cuda.CUDAGraph()):
+        build()
+    with pytest.raises(RuntimeError, match="captured"), torch.cuda.graph(torch.cuda.CUDAGraph()):
+        b.pieces(64)
+    torch.cuda.synchronize()
+    assert build().pos.tolist() == [0, 1, 2, 5] and b.pieces(64)[1].tolist() == [[0, 1, 0, 0], [1, 1, 5, 1]]
