@@ -146,7 +146,7 @@ __device__ __forceinline__ uint2 ch_silu4(uint2 w) {
     return __builtin_bit_cast(uint2, __builtin_convertvector(f, ch_bf16x4));
 }
 
-static constexpr size_t ch_lds_bytes(int DP, int NW, bool out) { return 2 * CH_T * ((out ? 2 : 1) * (size_t)(DP + 8) + 32 * NW + 16) + NW * 4 * CH_T * 4; }
+static constexpr size_t ch_lds_bytes(int DP, int NW, bool out) { return 2 * CH_T * ((out ? 2 : 1) * (size_t)(DP + 8) + 32 * NW + 16) + NW * 4 * CH_T * 4 + (out ? (NW * 32 + 2) * 4 : 0); }
 
 template <int DP, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chunk_kernel(jl_scan_args a, int heads, int blocks) {
@@ -162,8 +162,11 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
     if (cnt <= 0 || (!OUT && last)) return;
     bf16_t *Ks = (bf16_t *)smem, *Vs = Ks + CH_T * QROW, *Qs = Vs + CH_T * VROW;             // [64][DP + 8] keys, [64][32 NW + 16] values, [64][DP + 8] queries
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
-    float *Ls = (float *)(Vs + CH_T * VROW + (OUT ? CH_T * QROW : 0)) + wave * 4 * CH_T;     // this wavefront's: [64] running log2 decay
+    float *tables = (float *)(Vs + CH_T * VROW + (OUT ? CH_T * QROW : 0));
+    float *Ls = tables + wave * 4 * CH_T;                                                    // this wavefront's: [64] running log2 decay
     float *us = Ls + CH_T, *es = us + CH_T, *el = es + CH_T;                                 // [64] u; exp(L_end - L) u; exp(L)
+    int *brokenS = (int *)(tables + NW * 4 * CH_T) + wave * 32;                              // [32] the first token of a group whose value is not finite, per column (outputs only)
+    int *flawS = (int *)(tables + NW * 4 * CH_T) + NW * 32;                                  // [2] whether this group, the one before, has such a value
     // the columns of wavefront w: block w % blocks (of those from blockIdx.z * NW on) of head h0 + w / blocks
     auto head_of = [&](int w) { return h0 + w / blocks; };
     auto col_of = [&](int w) { return 32 * ((int)blockIdx.z * NW + w % blocks); };
@@ -269,15 +272,19 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
         if (n >= CH_T) store(std::true_type());
         else store(std::false_type());
     };
+    if (OUT && tid < 2) flawS[tid] = 0;
     fetch(0);
     float l_all = 0.f, end = 0.f, g = 1.f;                          // log2 of the piece's decay up to here, of the group's; the group's decay (fixed decays: the same for whole groups)
     for (int t0 = 0; t0 < cnt; t0 += CH_T) {
         const int nt = cnt - t0 < CH_T ? cnt - t0 : CH_T;
         __syncthreads();                                            // the group before has been read
+        float zero = 0.f;                                           // not a number with a value that is not finite
         auto stage = [&](auto silu) {                               // silu(0) = 0
             auto put = [&](bf16_t *to, uint2 v, bool in) {
                 if (!in) v = make_uint2(0, 0);
-                *(uint2 *)to = decltype(silu)::value ? ch_silu4(v) : v;
+                if (decltype(silu)::value) v = ch_silu4(v);
+                *(uint2 *)to = v;
+                return v;
             };
             if (DP == 4 * UD || kd < DP)
 #pragma unroll
@@ -287,7 +294,13 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
                     if (OUT) put(Qs + t * QROW + kd, rq[OUT ? it : 0], k_in && t < nt);
                 }
 #pragma unroll
-            for (int it = 0; it < VIT; ++it) put(Vs + (vt + it * VSTEP) * VROW + vc, rv[it], v_in && vt + it * VSTEP < nt);
+            for (int it = 0; it < VIT; ++it) {
+                const uint2 v = put(Vs + (vt + it * VSTEP) * VROW + vc, rv[it], v_in && vt + it * VSTEP < nt);
+                if (!OUT) continue;
+                zero = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(jl_bf16x2, v.x), jl_bf16x2{0, 0}, zero, false);
+                zero = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(jl_bf16x2, v.y), jl_bf16x2{0, 0}, zero, false);
+            }
+            if (OUT && zero != 0.f) flawS[t0 / CH_T & 1] = 1;
         };
         if (act) stage(std::true_type());
         else stage(std::false_type());
@@ -312,6 +325,32 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
         }
         l_all += end;
         __syncthreads();
+        // Weights of zero must not meet a value that is not finite, in front of whose token they stand: it is left out of the products, and its column's outputs from its token on
+        // and the column of the state are set behind them
+        bool flawed = false;
+        if (OUT) {
+            flawed = __builtin_amdgcn_readfirstlane(flawS[t0 / CH_T & 1]);
+            if (tid == 0) flawS[~(t0 / CH_T) & 1] = 0;
+            if (flawed) {
+                int broken = CH_T, here = l32;
+                asm volatile("" : "+v"(here));                      // its addresses made here, not kept over the loop
+#pragma unroll 1
+                for (int s = 0; s < CH_T / 16; ++s) {
+                    const jl_bf16x8 v = turned(Vs, VROW, 32 * wave, s);
+#pragma unroll
+                    for (int i = 7; i >= 0; --i)
+                        if (!__builtin_isfinite((float)v[i])) {
+                            const int t = 16 * s + 4 * hi + i + 4 * (i >> 2);
+                            broken = min(broken, t);
+                            Vs[t * VROW + 32 * wave + here] = (bf16_t)0;
+                        }
+                }
+                broken = min(broken, __shfl_xor(broken, 32, 64));
+                brokenS[here] = broken;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
         if (t0 + CH_T < cnt) fetch(t0 + CH_T);                      // in flight while this group is multiplied
         if (OUT && t0 > 0) outputs(t0 - CH_T, CH_T);
         jl_bf16x8 vf[CH_T / 16];
@@ -402,6 +441,15 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
                     for (int y = 0; y < 2; ++y)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) o[y][r] += skip * (float)vf[2 * y + (r >> 3)][r & 7];
+                if (flawed) {
+                    int here = l32;
+                    asm volatile("" : "+v"(here));
+                    const int broken = brokenS[here] - 4 * hi;
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[y][r] = 32 * y + 8 * (r >> 2) + (r & 3) < broken ? o[y][r] : NAN;
+                }
             } else {
 #pragma unroll
                 for (int s = 0; s < CH_T / 16; ++s) vf[s] = turned(Vs, VROW, 32 * wave, s);
@@ -434,6 +482,15 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
 #pragma unroll
                     for (int x = 0; x < NT; ++x) S[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s & 1][x], part[s & 1][y], S[x], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            if (flawed) {
+                int here = l32;
+                asm volatile("" : "+v"(here));
+                if (brokenS[here] < CH_T)
+#pragma unroll
+                    for (int x = 0; x < NT; ++x)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) S[x][r] = NAN;
             }
         }
     }

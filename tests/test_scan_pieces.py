@@ -94,3 +94,35 @@ def test_rows_wider_than_the_offsets_of_pieces(monkeypatch, pieces):
         v = x[:, 2 * D + h * Dv + c:2 * D + h * Dv + c + 64].double()
         want, S = (q @ k.T * fade) @ v, (k * fade[-1:].T).T @ v
         assert (out[:, h, c:c + 64] - want).norm() <= 2e-6 * want.norm() and (state[0, h, :, c:c + 64] - S).norm() <= 2e-6 * S.norm(), (h, c)
+
+
+@pytest.mark.parametrize("what,value", [("v", float("nan")), ("v", float("inf")), ("k", float("-inf")), ("q", float("nan")), ("dt", float("nan")), ("dt", float("inf"))])
+@pytest.mark.parametrize("H,G,D,Dv", [(6, 2, 64, 40), (4, 4, 128, 128), (5, 1, 20, 20), (2, 2, 96, 64)])
+@pytest.mark.parametrize("waves", [1, 1 << 20])
+def test_what_is_not_finite_reaches_later_tokens_only(monkeypatch, H, G, D, Dv, waves, what, value):
+    """... of the columns and heads that read it, as in the scan token by token; what other rows, columns, heads and requests hold is what it is without it, bit for bit."""
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "SCAN_WAVES", waves)             # pieces of several groups, and of one
+    n, per, g = 300, H // G, torch.Generator(device="cuda").manual_seed(H + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch = LO.RaggedBatch.build([n, 70], [0, 9], [0, 1], [[0, 1, 2, 3, 4], [5, 6]], 64, "cuda")
+    cols = (0, G * D, 2 * G * D)
+    x, dt, start, kw = rnd(n + 70, 2 * G * D + H * Dv).bfloat16(), rnd(n + 70, H).bfloat16(), rnd(2, H, D, Dv), dict(a_log=rnd(H) - 2, dt_bias=rnd(H), skip=rnd(H), act=LO.ACT_SILU)
+    if what != "dt":
+        kw = dict(decay=torch.rand(H, generator=g, device="cuda"), skip=kw["skip"])
+
+    def run(pieces):
+        st = start.clone()
+        monkeypatch.setattr(LO, "SCAN_PIECES_FROM", 32 if pieces else 1 << 30)
+        return LO.linear_scan(x, cols, batch, H, G, D, Dv, st, **(kw | (dict(dt=dt) if what == "dt" else {}))).view(n + 70, H, Dv), st
+    want, clean = run(True)
+    c, h = Dv // 2 + 1, H - 1
+    y, at = {"q": (x, cols[0] + (G - 1) * D + 3), "k": (x, cols[1] + (G - 1) * D + 3), "v": (x, cols[2] + h * Dv + c), "dt": (dt, h)}[what]
+    for t in (0, 21, 31, 32, 63, 64, 190, n - 1):            # within blocks of 32 and 64 tokens, at their ends, the last
+        kept, y[t, at] = y[t, at].clone(), value
+        (got, state), (scan, scan_state) = run(True), run(False)
+        y[t, at] = kept
+        off = torch.zeros(n + 70, H, Dv, dtype=torch.bool, device="cuda")
+        off[t:t + 1 if what == "q" else n, h if what in ("v", "dt") else slice(H - per, H), c if what == "v" else slice(0, Dv)] = True
+        assert torch.equal(~got.isfinite(), off) and torch.equal(got[~off], want[~off]), t
+        assert torch.equal(got.isfinite(), scan.isfinite()) and torch.equal(state.isfinite(), scan_state.isfinite()) and torch.equal(state[state.isfinite()], clean[state.isfinite()]), t
