@@ -140,9 +140,9 @@ class RaggedBatch:
     _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
     _held: list = field(default_factory=list, repr=False, compare=False)      # what was uploaded for it, with the stream that asked
 
-    def __del__(self, gone=_GONE):
+    def __del__(self, gone=_GONE, queue=deque):          # (module names may be gone before the last batch)
         for key, t in self.__dict__.get("_held", ()):
-            gone.setdefault(key, deque()).append(t)
+            gone.setdefault(key, queue()).append(t)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
