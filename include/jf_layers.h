@@ -412,7 +412,7 @@ JL_API int jl_delta_chunks_run(const jl_delta_chunks *a, void *stream);
  * run side by side on the matrix cores — chunk_rec [chunks, 4] int32 {row0, count, slot, 1 for a request's last piece}, every piece but the
  * last a multiple of 64 rows, a request's pieces consecutive; req [B, 4] int32 {first piece, pieces, pos0, slot}, of requests that have rows alone
  * (B counts these records: one of no rows would hide that another has several pieces); scratch of
- * chunks * H * (D * Dv + 1) floats; sizes as jl_linear_scan_chunked_ok accepts them, rows and columns in multiples of four elements.  Beyond
+ * chunks * H * (D * Dv + 1) floats (not touched where chunks = B: every request has one piece); sizes as jl_linear_scan_chunked_ok accepts them, rows and columns in multiples of four elements.  Beyond
  * H * Dv = 2^24, Dv = 2^22 or ld = 2^26 the rows go in one scan all the same (seq names these B requests too). */
 typedef struct {
     const void *src; const void *dt; const float *decay; const float *A_log; const float *dt_bias; const float *skip;

@@ -116,7 +116,8 @@ template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t 
 //   o_i = exp(L_i) S^T q_i + sum_{j <= i} (q_i . k_j) exp(L_i - L_j) u_j v_j,        S <- exp(L_end) S + sum_j k_j (exp(L_end - L_j) u_j v_j)^T.
 // A request's portion is cut into pieces (whole groups, except the last) that run side by side in three launches: every piece's own
 // contribution to the state from a zero state (CH_LOCAL, not for a request's last piece), scan_join_kernel (the state every piece starts
-// from), outputs (CH_OUT; the last piece leaves the request's final state in its slot).
+// from), outputs (CH_OUT; the last piece leaves the request's final state in its slot).  Where every request has one piece, in one: it starts from the slot (one portion of 64 tokens, 16 heads of
+// 128 x 128: 20 -> 16 us, 16 of 100 67 -> 33).
 // q, k and v enter the products as bfloat16 (what the projection, the convolution and their activation give); everything else stays float
 // and crosses the matrix cores as the sum of THREE bfloat16 numbers, which hold all 24 bits of it: the state, the decayed weights of a pair,
 // the decayed values.
@@ -129,7 +130,8 @@ template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t 
 // What bounds it: latency with two wavefronts per SIMD, all that their registers allow.  Per group and wavefront 1 900 vector instructions (splits, exponentials, silu) and 138 products of 32 cycles
 // take 12 000 cycles of issue; two side by side take 40 000.  Loads, stores, splits, weights: leaving out any one of them gives 5 to 15 % of the time.
 // Before, 64 columns of one head per workgroup met in LDS five times per group, one workgroup per CU.  us of the three launches, 4 x 2048 tokens, before / now: 16 heads of 128 x 128 with silu
-// 212 / 128 (their bytes at the rate of a large copy: 78), 32 heads of 128 x 64 over one key head 201 / 119; 2 x 300 of 8 heads 42 / 34, 40 x 64 of 16 heads 121 / 91.
+// 212 / 121 (their bytes at the rate of a large copy: 78), 32 heads of 128 x 64 over one key head 201 / 116; 3 x 1000 of 8 heads 74 / 54, 8 x 200 of 16 heads 90 / 47; but one portion of 256 of
+// 16 heads 31 / 33: a group alone takes its wavefront 9 us, and three launches' ends show.
 typedef __bf16 ch_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float ch_f32x4 __attribute__((ext_vector_type(4)));
 typedef float ch_f32x16 __attribute__((ext_vector_type(16)));
@@ -149,7 +151,7 @@ __device__ __forceinline__ uint2 ch_silu4(uint2 w) {
 static constexpr size_t ch_lds_bytes(int DP, int NW, bool out) { return 2 * CH_T * ((out ? 2 : 1) * (size_t)(DP + 8) + 32 * NW + 16) + NW * 4 * CH_T * 4 + (out ? (NW * 32 + 2) * 4 : 0); }
 
 template <int DP, int NW, int MODE>
-__global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chunk_kernel(jl_scan_args a, int heads, int blocks) {
+__global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chunk_kernel(jl_scan_args a, int heads, int blocks, int alone) {      // alone: every request has one piece
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr bool OUT = MODE == CH_OUT;
     constexpr int THREADS = 64 * NW, QROW = DP + 8, VROW = 32 * NW + 16, UD = DP <= 32 ? 8 : DP <= 64 ? 16 : 32, UV = 8 * NW, NT = DP / 32;
@@ -194,11 +196,18 @@ __global__ __launch_bounds__(64 * NW, NW == 2 && DP > 64 ? 1 : 2) void scan_chun
     for (int x = 0; x < NT; ++x)
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[x][r] = 0.f;
-    if (OUT && busy && sc < Dv) {
+    bool started = OUT && busy && sc < Dv;
+    if (started) {
         const char *sp = (const char *)(a.scratch + ((int64_t)piece * H + h) * D * Dv);
-        each_state([&](int d, uint32_t off, float) { return d < D ? *(const float *)(sp + off) : 0.f; });
+        if (alone) {                                                // from its slot, as there is nothing to join
+            int b = piece;
+            if (a.req[4 * b] != piece)
+                for (b = 0; b + 1 < a.B && a.req[4 * b] != piece;) ++b;
+            started = a.req[4 * b + 2] > 0;
+            sp = (const char *)(a.state + ((int64_t)slot * H + h) * D * Dv);
+        }
+        if (started) each_state([&](int d, uint32_t off, float) { return d < D ? *(const float *)(sp + off) : 0.f; });
     }
-
     uint2 rq[OUT ? KIT : 1], rk[KIT], rv[VIT];
     float rd = 0.f;
     // this thread's unit of four values: of q and k, of v (`w`: whose columns); what does not exist is staged as zeros
@@ -511,12 +520,19 @@ __global__ __launch_bounds__(256) void scan_join_kernel(jl_scan_args a) {
     for (int64_t e = (int64_t)blockIdx.y * 256 + threadIdx.x; e < ddv; e += (int64_t)gridDim.y * 256) {
         float S = pos0 > 0 ? sp[e] : 0.f;
         float *lp = a.scratch + ((int64_t)p0 * a.H + h) * ddv + e;
-        float local = np > 1 ? *lp : 0.f;
-        for (int p = 0; p < np; ++p, lp += a.H * ddv) {
-            const float next = p + 2 < np ? lp[a.H * ddv] : 0.f;    // on its way while this piece is joined
+        if (np == 1) {                                              // (its own way: single tokens beside a prompt are many)
             *lp = S;
-            if (p + 1 < np) S = exp2f(ll[(int64_t)(p0 + p) * a.H + h]) * S + local;
+            continue;
+        }
+        const float *l = ll + (int64_t)p0 * a.H + h;
+        float local = *lp, fade = *l;
+        for (int p = 0; p < np; ++p, lp += a.H * ddv) {
+            l += a.H;
+            const float next = p + 2 < np ? lp[a.H * ddv] : 0.f, next_fade = p + 2 < np ? *l : 0.f;      // on their way while this piece is joined
+            *lp = S;
+            if (p + 1 < np) S = exp2f(fade) * S + local;
             local = next;
+            fade = next_fade;
         }
     }
 }
@@ -525,10 +541,13 @@ template <int DP, int NW> static int scan_chunk_launch(const jl_scan_args &a, in
     const int per_head = (a.Dv + 31) / 32;
     const dim3 grid((unsigned)a.chunks, (unsigned)(a.G * ((a.H / a.G + heads - 1) / heads)), (unsigned)((per_head + NW - 1) / NW));
     static_assert(ch_lds_bytes(DP, NW, true) <= 64 * 1024, "static limit of a launch");
-    if (a.chunks > a.B) scan_chunk_kernel<DP, NW, CH_LOCAL><<<grid, 64 * NW, ch_lds_bytes(DP, NW, false), st>>>(a, heads, blocks);
-    const int64_t ddv = (int64_t)a.D * a.Dv;
-    scan_join_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64)), 256, 0, st>>>(a);
-    scan_chunk_kernel<DP, NW, CH_OUT><<<grid, 64 * NW, ch_lds_bytes(DP, NW, true), st>>>(a, heads, blocks);
+    const bool alone = a.chunks == a.B;
+    if (!alone) {
+        scan_chunk_kernel<DP, NW, CH_LOCAL><<<grid, 64 * NW, ch_lds_bytes(DP, NW, false), st>>>(a, heads, blocks, 0);
+        const int64_t ddv = (int64_t)a.D * a.Dv;
+        scan_join_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)((ddv + 255) / 256 < 64 ? (ddv + 255) / 256 : 64)), 256, 0, st>>>(a);
+    }
+    scan_chunk_kernel<DP, NW, CH_OUT><<<grid, 64 * NW, ch_lds_bytes(DP, NW, true), st>>>(a, heads, blocks, alone);
     return jl_check_launch("scan_chunk_kernel");
 }
 // Four wavefronts per workgroup where a head's columns or the heads that read the same q and k fill more than two of them; else two.

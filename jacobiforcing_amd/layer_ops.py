@@ -1386,6 +1386,17 @@ def delta_rule(qkv: torch.Tensor, cols: Tuple[int, int, int], proj: torch.Tensor
     return out
 
 
+def scan_piece_groups(counts: Sequence[int], waves: int) -> int:
+    """Groups of 64 tokens per piece of the linear recurrence, for ``waves`` wavefronts of 32 columns per request.  Portions that stay whole take one launch instead of three and half of the
+    work, but walk their groups one after the other, 9 us each: up to two of them always, more where the requests' wavefronts fill the chip on average over that walk.  us, cut / whole, 64
+    wavefronts per request: 40 tokens 21 / 16, 100 31 / 24, 192 32 / 32, 256 33 / 41, 3 x 192 40 / 34, 3 x 200 43 / 44, 8 x 200 62 / 47, 4 x 500 61 / 83, 8 x 500 109 / 88, 12 x 900 199 / 159,
+    30 x 1000 419 / 282, 8 x 2000 283 / 334, 777 and 30 x 1 104 / 133; 8 per request: 30 x 300 38 / 39, 30 x 500 44 / 59.  Else as many pieces as fill the chip with two wavefronts per SIMD."""
+    groups, longest = sum(-(-c // 64) for c in counts), -(-max(counts) // 64)
+    if longest <= 2 or groups * waves >= 48 * longest * longest:
+        return longest
+    return max(1, min(8, sum(counts) * waves // (SCAN_WAVES * 64)))
+
+
 def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatch, H: int, G: int, D: int, Dv: int, state: torch.Tensor, act: int = N.JL_ACT_NONE,
                 decay: Optional[torch.Tensor] = None, dt: Optional[torch.Tensor] = None, a_log: Optional[torch.Tensor] = None,
                 dt_bias: Optional[torch.Tensor] = None, skip: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1411,8 +1422,10 @@ def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatc
     if (max(batch.counts) >= SCAN_PIECES_FROM and not os.environ.get("JL_SCAN_NO_PIECES") and a.ld % 4 == 0 and all(c % 4 == 0 for c in cols) and    # A/B switch for measurements
             H * Dv <= 1 << 24 and Dv <= 1 << 22 and a.ld <= 1 << 26 and         # their kernel's offsets of 32 bits; the library sends wider calls to the scan by itself
             N.layers().jl_linear_scan_chunked_ok(a.dtype, D, Dv)):
-        # long portions: pieces side by side on the matrix cores, as many as fill the chip with two wavefronts per SIMD, each at least one group of 64 tokens
-        size = 64 * max(1, min(8, n * H * -(-Dv // 32) // (SCAN_WAVES * 64)))
+        waves = H * -(-Dv // 32)
+        size = batch._tiles.get(("scan", waves))
+        if size is None:
+            size = batch._tiles[("scan", waves)] = 64 * scan_piece_groups(batch.counts, waves)
         rec, req = batch.pieces(size)
         scratch = torch.empty((rec.shape[0] * H * (D * Dv + 1),), dtype=torch.float32, device=src.device)
         a.chunk_rec, a.req, a.scratch, a.chunks, a.B = p(rec), p(req), p(scratch), rec.shape[0], req.shape[0]

@@ -48,24 +48,33 @@ def test_columns_and_heads(monkeypatch, H, G, D, Dv, counts, fixed):
             r0 += n
 
 
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("H,G,D,Dv,counts", [(3, 3, 128, 128, [64, 1, 200]), (2, 2, 96, 96, [257, 63]), (9, 1, 128, 64, [130, 33]), (5, 1, 32, 20, [100, 440, 7])])
+def test_portions_that_stay_whole(monkeypatch, H, G, D, Dv, counts, fixed):
+    """One launch, from the slots: as in pieces."""
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "scan_piece_groups", lambda counts, waves: -(-max(counts) // 64))
+    test_columns_and_heads(monkeypatch, H, G, D, Dv, counts, fixed)
+
+
 @pytest.mark.parametrize("op", ["scan", "retention"])
 def test_requests_without_tokens(monkeypatch, op):
-    """Beside as many pieces as there are requests, two of them one request's: as without the request that has none, and its state stays."""
+    """Beside as many pieces as there are requests, all of them one request's: as without the requests that have none, and their states stay."""
     from jacobiforcing_amd import layer_ops as LO
     monkeypatch.setattr(LO, "SCAN_WAVES", 1 << 20)           # pieces of one group each
     monkeypatch.setattr(LO, "RETENTION_WORKGROUPS", 1 << 20)
     g, H, D = torch.Generator(device="cuda").manual_seed(5), 2, 64
-    x, start, decay = torch.randn(128, 4 * H * D, generator=g, device="cuda").bfloat16(), torch.randn(2, H, D, D, generator=g, device="cuda"), torch.full((H,), 0.97, device="cuda")
+    x, start, decay = torch.randn(192, 4 * H * D, generator=g, device="cuda").bfloat16(), torch.randn(3, H, D, D, generator=g, device="cuda"), torch.full((H,), 0.97, device="cuda")
     got = []
-    for counts in ([0, 128], [128]):
-        b, st = LO.RaggedBatch.build(counts, [0] * len(counts), [0, 1][-len(counts):], [[0, 1]] * len(counts), 64, "cuda"), start.clone()
+    for counts in ([0, 0, 192], [192]):
+        b, st = LO.RaggedBatch.build(counts, [0] * len(counts), [0, 1, 2][-len(counts):], [[0, 1, 2]] * len(counts), 64, "cuda"), start.clone()
         if op == "scan":
             o = LO.linear_scan(x, (0, H * D, 2 * H * D), b, H, H, D, D, st, decay=decay)
         else:
             o = LO.retention(x, (0, H * D, 2 * H * D, 3 * H * D), b, H, D, D, 0, None, None, decay, 1e-5, st)
-        assert [len(v[0]) for k, v in b._tiles.items() if isinstance(k, tuple) and k[0] == "pieces"] == [2]
+        assert [len(v[0]) for k, v in b._tiles.items() if isinstance(k, tuple) and k[0] == "pieces"] == [3]
         got.append((o, st))
-    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][0], start[0])
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][1][:2], start[:2])
 
 
 @pytest.mark.parametrize("pieces", [False, True])

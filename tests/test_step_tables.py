@@ -109,3 +109,10 @@ def test_what_a_batch_is_built_of():
     for bad in (dict(starts=[2, 0, 1]), dict(slots=[0, 1, 2]), dict(slots=[0]), dict(starts=[2.0, 0]), dict(counts=[1, -1]), dict(tables=[[1]])):
         with pytest.raises((ValueError, TypeError, IndexError)):
             build(**bad)
+
+
+@pytest.mark.parametrize("counts,waves,groups", [([1, 40], 64, 1), ([128], 8, 2), ([129], 64, 1), ([200] * 3, 64, 4), ([200] * 3, 63, 1), ([500] * 4, 64, 1), ([500] * 8, 64, 8), ([2048] * 4, 64, 4), ([777] + [1] * 30, 64, 1),
+                                                 ([1000] * 30, 64, 16), ([8192] * 8, 256, 8)])
+def test_pieces_of_the_linear_recurrence(counts, waves, groups):
+    """Whole up to two groups, or where the step's wavefronts fill the chip over the longest portion's walk; else as many as fill it, of at most eight groups."""
+    assert LO.scan_piece_groups(counts, waves) == groups
