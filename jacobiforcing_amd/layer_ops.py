@@ -719,12 +719,22 @@ def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: Ragged
     return out
 
 
-ROUTER_OUTPUTS, ROUTER_TOKENS = 64, 32 * 512      # beyond: the library's product, one launch for the choices and one workgroup for the grouping
+ROUTER_OUTPUTS, ROUTER_TOKENS = 64, 32 * 512      # beyond: one launch for the choices and one workgroup for the grouping
+ROUTER_DEPTH, ROUTER_DEPTH_FEW, ROUTER_FEW = 2048, 6144, 512      # router product in the same launch: depths times blocks of 16 outputs at most; for up to that many tokens (below)
 _ROUTES = {"sigmoid": N.JL_ROUTE_SIGMOID, "softmax_renorm": N.JL_ROUTE_SOFTMAX_RENORM, "top_softmax": N.JL_ROUTE_TOP_SOFTMAX}
 
 
 def _router_in_one(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
-    """Whether the package's launches take the router product with the choice and the grouping: up to ROUTER_OUTPUTS outputs and ROUTER_TOKENS tokens, operands as ``linear`` takes them."""
+    """Whether the package's launches take the router product with the choice and the grouping: up to ROUTER_OUTPUTS outputs and ROUTER_TOKENS tokens, operands as ``linear`` takes them, and
+    where that is not slower than ``linear`` in front of them.  Every 32 tokens take in all of W, so it is up to a product of the depth and the blocks of 16 outputs: ROUTER_DEPTH, for
+    bfloat16 rows, which the library's product has to convert, 1.5 per token, and ROUTER_DEPTH_FEW for steps of up to ROUTER_FEW tokens, which wait for the host's launches.  us of GPU time with choice, grouping and small experts, product of its own / in one: 32 bfloat16 rows of 1024 by 16 outputs
+    24 / 21, by 32 25 / 26, by 64 28 / 35; 1024 of 1024 by 32 33 / 31, of 2048 by 32 37 / 40, of 4096 by 64 48 / 86; 8192 of 1024 by 16 49 / 32, of 4096 by 64 100 / 101; float rows: 32 of 1024 by
+    32 25 / 25, of 2048 by 32 25 / 32; 1024 of 1024 by 32 27 / 28, of 2048 by 32 29 / 37; 8192 of 2048 by 32 42 / 47.  us a pass of four layers, widths of 2048 by 32
+    outputs: 32 decoding requests of Mikipel 817 / 796, of Lokizen 974 / 1012, one portion of 256 1106 / 1013, of 1000 1336 / 1352; by 40, 32 decoding requests of Voborax 1160 / 1119."""
+    return (x.dim() == 2 and w.dim() == 2 and x.shape[1] * -(-w.shape[0] // 16) <= max(ROUTER_DEPTH_FEW if x.shape[0] <= ROUTER_FEW else ROUTER_DEPTH, 3 * x.shape[0] // 2 if x.dtype == torch.bfloat16 else 0) and _router_operands(x, w, bias))
+
+
+def _router_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     return (x.dim() == 2 and 0 < x.shape[0] <= ROUTER_TOKENS and w.dim() == 2 and w.shape[0] <= ROUTER_OUTPUTS and x.dtype in _LINEAR_TYPES and w.dtype == torch.float32 and w.is_contiguous() and
             w.shape[1] == x.shape[1] and x.shape[1] % 4 == 0 and x.shape[1] > 0 and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.stride(0) * x.element_size() % 16 == 0 and
             (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.get_device() == x.get_device() and

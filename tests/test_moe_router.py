@@ -8,6 +8,8 @@ pytestmark = pytest.mark.gpu
 
 def run(monkeypatch, N, K, E, identity, top, x_dtype, bias, route, pad=0, gated=False):
     from jacobiforcing_amd import layer_ops as LO
+    for limit in ("ROUTER_DEPTH", "ROUTER_DEPTH_FEW"):                         # also where a product of its own is the faster one
+        monkeypatch.setattr(LO, limit, 1 << 30)
     g = torch.Generator(device="cuda").manual_seed(N + K + E)
     whole = lambda lim, *s: torch.randint(-lim, lim + 1, s, generator=g, device="cuda")
     Er, W, ff = E + identity, 64, 32
@@ -65,3 +67,12 @@ def test_logits_that_are_not_finite(monkeypatch, route):
     z[9, 4] = float("nan")
     y = LO.moe_experts(h, z, None, 2, 1.0, up, down, route=route)
     assert y[9].isnan().any() and torch.equal(torch.cat([y[:9], y[10:]]).nan_to_num(7.0), torch.cat([want[:9], want[10:]]).nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("n,K,E,dtype,one", [(32, 2048, 48, "float32", True), (512, 2048, 49, "bfloat16", False), (513, 2048, 16, "float32", True), (513, 1028, 17, "float32", False), (2048, 1024, 48, "bfloat16", True), (2048, 1024, 64, "bfloat16", False),
+                                             (8192, 2048, 32, "float32", False), (8192, 3072, 64, "bfloat16", True)])
+def test_where_the_product_is_in_the_launch(n, K, E, dtype, one):
+    """Up to a product of depth and blocks of 16 outputs that grows with the tokens in 16 bits; beyond, the same choices from ``linear``'s logits."""
+    from jacobiforcing_amd import layer_ops as LO
+    x, w = torch.zeros(n, K, device="cuda", dtype=getattr(torch, dtype)), torch.zeros(E, K, device="cuda")
+    assert LO._router_operands(x, w, None) and LO._router_in_one(x, w, None) == one
