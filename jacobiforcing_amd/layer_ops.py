@@ -74,7 +74,7 @@ def _dev(t: torch.Tensor) -> None:
 
 
 _UPLOADS: dict = {}                                  # device index -> the stream its tables are copied on, and a block of its pool
-_GONE: dict = {}                                     # (device index, stream) -> tables uploaded from that stream whose batch is gone
+_GONE: dict = {}                                     # a stream's id -> the stream, and the tables uploaded from it whose batch is gone
 
 
 def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
@@ -89,30 +89,32 @@ def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
         return t.to(device)
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("a step's tables cannot be copied while a graph is captured")
-    index = torch.cuda.current_device() if device.index is None else device.index
+    here = torch.cuda.current_device()
+    index = here if device.index is None else device.index
     if index not in _UPLOADS:
         side = torch.cuda.Stream(index)
         with torch.cuda.stream(side):                    # a block that stays keeps the pool's first segment (2 MB) from being given back and asked for again
             _UPLOADS.setdefault(index, (side, torch.empty(1, dtype=torch.int32, device=device)))
-    side, user = _UPLOADS[index][0], torch.cuda.current_stream(index)
-    key = index, user.cuda_stream
-    gone = _GONE.get(key)
+    side, user = _UPLOADS[index][0], torch._C._cuda_getCurrentStream(index)      # (the stream's id, not an object for every upload)
+    if user not in _GONE:
+        _GONE.setdefault(user, (torch.cuda.current_stream(index), deque()))
+    stream, gone = _GONE[user]
     while gone:
         try:
-            gone.popleft().record_stream(user)
+            gone.popleft().record_stream(stream)
         except IndexError:                               # another thread took the last one
             break
-    if index == torch.cuda.current_device():             # half of what the context below takes
-        torch.cuda.set_stream(side)
+    if index == here:                                    # a fifth of what the context below takes
+        torch._C._cuda_setStream(stream_id=side.stream_id, device_index=side.device_index, device_type=side.device_type)
         try:
             up = t.to(device)
         finally:
-            torch.cuda.set_stream(user)
+            torch._C._cuda_setStream(stream_id=user[0], device_index=user[1], device_type=user[2])
     else:
         with torch.cuda.stream(side):
             up = t.to(device)
-    up.record_stream(user)                               # (views of it may outlive the batch)
-    held.append((key, up))
+    up.record_stream(stream)                             # (views of it may outlive the batch)
+    held.append((gone, up))
     return up
 
 
@@ -138,11 +140,11 @@ class RaggedBatch:
     _tiles: dict
     _host_tables: Optional[np.ndarray] = None         # tables on the host, for key_rows and part (None: read back when they need it)
     _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
-    _held: list = field(default_factory=list, repr=False, compare=False)      # what was uploaded for it, with the stream that asked
+    _held: list = field(default_factory=list, repr=False, compare=False)      # what was uploaded for it, with the list it joins behind the batch's end
 
-    def __del__(self, gone=_GONE, queue=deque):          # (module names may be gone before the last batch)
-        for key, t in self.__dict__.get("_held", ()):
-            gone.setdefault(key, queue()).append(t)
+    def __del__(self):
+        for gone, t in self.__dict__.get("_held", ()):
+            gone.append(t)
 
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
