@@ -429,7 +429,8 @@ JL_API int jl_linear_scan_chunked_ok(int dtype, int32_t D, int32_t Dv);
  *   JL_ROUTE_SOFTMAX_RENORM: s = softmax(logits) over all experts; the `top` experts with the largest s + correction (null: s) are chosen
  *                            (ties: lowest index); weights = s / (sum of the chosen s + renorm_eps) * scale.
  *   JL_ROUTE_TOP_SOFTMAX:    the `top` largest logits are chosen (ties: lowest index); weights = softmax over the chosen logits
- *                            only, times scale.  `correction` is not read. */
+ *                            only, times scale.  `correction` is not read.
+ * A value to compare that is not a number counts as infinity. */
 #define JL_ROUTE_SIGMOID 0
 #define JL_ROUTE_SOFTMAX_RENORM 1
 #define JL_ROUTE_TOP_SOFTMAX 2

@@ -48,6 +48,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *__restrict_
         if (kind == JL_ROUTE_SIGMOID) cmp[j] = sc[j];
         if (kind == JL_ROUTE_SOFTMAX_RENORM && correction) cmp[j] = sc[j];
         if (correction && kind != JL_ROUTE_TOP_SOFTMAX) cmp[j] += correction[e];
+        if (cmp[j] != cmp[j]) cmp[j] = INFINITY;                    // not a number: as the largest, here as in moe_route_rows
     }
     float chosen = 0.f;
     for (int s = 0; s < top; ++s) {
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *__restrict_
             const int oe = __shfl_xor(be, off, 64);
             if (oe != 0x7fffffff && (be == 0x7fffffff || ov > bv || (!(bv > ov) && oe < be))) { bv = ov; bs = os; be = oe; }
         }
-        be = __shfl(be, 0, 64);                                     // one winner for all lanes, whatever the values compared to (not-a-numbers)
+        be = __shfl(be, 0, 64);                                     // one winner for all lanes
         bs = __shfl(bs, 0, 64);
         if ((be & 63) == lane) open &= ~(1ull << (be >> 6));
         if ((s & 63) == lane) { ids[n * top + s] = be; weights[n * top + s] = bs; }

@@ -76,3 +76,24 @@ def test_where_the_product_is_in_the_launch(n, K, E, dtype, one):
     from jacobiforcing_amd import layer_ops as LO
     x, w = torch.zeros(n, K, device="cuda", dtype=getattr(torch, dtype)), torch.zeros(E, K, device="cuda")
     assert LO._router_operands(x, w, None) and LO._router_in_one(x, w, None) == one
+
+
+@pytest.mark.parametrize("route", ["sigmoid", "softmax_renorm", "top_softmax"])
+@pytest.mark.parametrize("E,correct", [(6, False), (6, True), (64, True)])
+def test_choices_among_values_that_are_not_numbers(monkeypatch, route, E, correct):
+    """... count as the largest, ties to the lowest index, whichever launches make the choice (how many tokens a step has decides that)."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(E)
+    N, W, ff, nan = 70, 64, 32, float("nan")
+    h, up, down = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((N, W), (E - 1, ff, W), (E - 1, W, ff)))
+    z, corr = torch.randn(N, E, generator=g, device="cuda"), torch.randn(E, generator=g, device="cuda") if correct else None
+    z[2, 4], z[3, [1, E - 1]], z[4], z[5, 2:], z[6, 3], z[6, 1] = nan, nan, nan, nan, float("inf"), nan
+    run = lambda: LO.moe_experts(h, z, corr, 3, 1.0, up, down, route=route, identity=1)
+    got = run()
+    monkeypatch.setattr(LO, "ROUTER_OUTPUTS", 0)
+    want = run()
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2].nan_to_num(7.0), want[2].nan_to_num(7.0))
+    first = [[4], [1, E - 1], [0, 1, 2], [2, 3, 4]]
+    if route == "top_softmax" or (route == "sigmoid" and not correct):
+        assert all(want[1][2 + i, :len(f)].tolist() == f for i, f in enumerate(first))
+    assert all(len(set(row)) == 3 for row in want[1].tolist())
