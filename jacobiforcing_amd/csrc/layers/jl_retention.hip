@@ -11,12 +11,14 @@ constexpr int RET_TT = 8;
 
 // MAXT: the largest workgroup the instantiation is launched with.  With 256 the state's DMAX rows stay in registers up to
 // DMAX = 128 (the default bound of 1 024 threads leaves 128 registers per lane and spills them).
-template <typename T, int DMAX, int PARTS, int MAXT>
-__global__ __launch_bounds__(MAXT) void retention_kernel(const T *__restrict__ proj, int64_t ld, int q_col, int k_col, int v_col, int g_col,
+// WHOLE: D is DMAX.  Else rows beyond D, zeros times a v that may not be finite, stay out of the sums: a branch per RB rows (fewer rows where a part has few; 32 tokens of 8 heads of 96: 9.8 -> 8.5 us, with its
+// bound of registers; 300 of 4 heads of 192 in chunks 276 -> 393).
+template <typename T, int DMAX, int PARTS, int MAXT, bool WHOLE>
+__global__ __launch_bounds__(MAXT, !WHOLE && PARTS == 4 && DMAX <= 128 ? 4 : 1) void retention_kernel(const T *__restrict__ proj, int64_t ld, int q_col, int k_col, int v_col, int g_col,
                                  const int32_t *__restrict__ seq, int H, int D, int Dv, int rot_dims,
                                  const float *__restrict__ cos_t, const float *__restrict__ sin_t, int64_t table_len,
                                  const float *__restrict__ decay, float eps, float *__restrict__ state, T *__restrict__ out, int mode) {
-    constexpr int DPER = DMAX / PARTS;
+    constexpr int DPER = DMAX / PARTS, RB = WHOLE || PARTS == 4 ? 4 : 16;
     extern __shared__ float lds[];
     float *qs = lds;                                   // [TT][DMAX]
     float *ks = qs + RET_TT * DMAX;                    // [TT][DMAX]
@@ -27,6 +29,7 @@ __global__ __launch_bounds__(MAXT) void retention_kernel(const T *__restrict__ p
     if (cnt <= 0) return;
     const int tid = threadIdx.x, width = blockDim.x / PARTS, part = PARTS > 1 ? tid / width : 0, j = PARTS > 1 ? tid - part * width : tid, wave = j >> 6, nw = width >> 6, d0 = part * DPER;
     const bool live = j < Dv;
+    const int mine = __builtin_amdgcn_readfirstlane(D - d0);       // rows of this part that exist (the same for a wavefront)
     const float gamma = decay[h], kscale = 1.0f / sqrtf((float)D);
     const int half = rot_dims >> 1;
     float *sp = state + ((int64_t)slot * H + h) * D * Dv;
@@ -69,12 +72,31 @@ __global__ __launch_bounds__(MAXT) void retention_kernel(const T *__restrict__ p
                 const float *qp = qs + tt * DMAX + d0, *kp = ks + tt * DMAX + d0;
                 float acc = 0.f;
 #pragma unroll
-                for (int i = 0; i < DPER; i += 4) {
-                    const float4 k4 = *(const float4 *)(kp + i), q4 = *(const float4 *)(qp + i);
-                    S[i] = gamma * S[i] + k4.x * v;             acc += S[i] * q4.x;
-                    S[i + 1] = gamma * S[i + 1] + k4.y * v;     acc += S[i + 1] * q4.y;
-                    S[i + 2] = gamma * S[i + 2] + k4.z * v;     acc += S[i + 2] * q4.z;
-                    S[i + 3] = gamma * S[i + 3] + k4.w * v;     acc += S[i + 3] * q4.w;
+                for (int i0 = 0; i0 < DPER; i0 += RB) {
+                    float4 q4[RB / 4];
+#pragma unroll
+                    for (int y = 0; y < RB / 4; ++y) {
+                        const int i = i0 + 4 * y;
+                        const float4 k4 = *(const float4 *)(kp + i);
+                        q4[y] = *(const float4 *)(qp + i);
+                        S[i] = gamma * S[i] + k4.x * v;
+                        S[i + 1] = gamma * S[i + 1] + k4.y * v;
+                        S[i + 2] = gamma * S[i + 2] + k4.z * v;
+                        S[i + 3] = gamma * S[i + 3] + k4.w * v;
+                    }
+                    if (WHOLE || i0 + RB <= mine)
+#pragma unroll
+                        for (int y = 0; y < RB / 4; ++y) {
+                            const int i = i0 + 4 * y;
+                            acc += S[i] * q4[y].x;
+                            acc += S[i + 1] * q4[y].y;
+                            acc += S[i + 2] * q4[y].z;
+                            acc += S[i + 3] * q4[y].w;
+                        }
+                    else
+#pragma unroll
+                        for (int i = 0; i < RB; ++i)
+                            if (i0 + i < mine) acc += S[i0 + i] * qp[i0 + i];
                 }
                 o[tt] = acc;
                 if (PARTS > 1 && mode != JL_RET_LOCAL_STATE) sums[tt * blockDim.x + tid] = acc;
@@ -121,7 +143,7 @@ static int ret_launch(const void *proj, int64_t ld, int q_col, int k_col, int v_
     const int width = (Dv + 63) / 64 * 64, parts = width <= 128 ? 4 : width <= 256 ? 2 : 1;
     const size_t lds = (size_t)(2 * RET_TT * DMAX + RET_TT * 16 + (parts > 1 ? RET_TT * width * parts : 0)) * 4;
 #define RET_LAUNCH(PARTS, MAXT)                                                                                                                          \
-    retention_kernel<T, DMAX, PARTS, MAXT><<<dim3((unsigned)(B * H)), width * PARTS, lds, st>>>((const T *)proj, ld, q_col, k_col, v_col, g_col, seq, H, D, Dv, \
+    (D == DMAX ? retention_kernel<T, DMAX, PARTS, MAXT, true> : retention_kernel<T, DMAX, PARTS, MAXT, false>)<<<dim3((unsigned)(B * H)), width * PARTS, lds, st>>>((const T *)proj, ld, q_col, k_col, v_col, g_col, seq, H, D, Dv, \
                                                                                                rot_dims, cos_t, sin_t, table_len, decay, eps, state, (T *)out, mode)
     if (parts == 4) RET_LAUNCH(4, 512);
     else if (parts == 2) RET_LAUNCH(2, 512);

@@ -103,3 +103,32 @@ def test_portions_of_both_kinds(H, D, counts, least):
     assert torch.equal(outs[0][short], outs[1][short])
     # sums of 32-bit products in another order, normed: as in test_pieces
     assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[1].norm() and (states[0] - states[1]).norm() <= 4e-6 * states[1].norm()
+
+
+@pytest.mark.parametrize("D,Dv", [(96, 64), (20, 100), (130, 200), (33, 300), (128, 128)])
+def test_short_portions_with_infinities(D, Dv):
+    """Sums of a column that are infinite (keys and queries of one sign) stay infinite where the kernel's rows are more than D: the other columns of the head come to zero under their norm."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, counts, starts = "cuda", 2, [3, 1, 5], [0, 4, 2]
+    g, n = torch.Generator(device=dev).manual_seed(D), sum(counts)
+    cols = (0, H * D, 2 * H * D, 2 * H * D + H * Dv)
+    proj = torch.randn(n, cols[3] + H * Dv, generator=g, device=dev)
+    proj[:, :cols[2]].abs_()
+    start, decay = torch.rand(3, H, D, Dv, generator=g, device=dev), torch.tensor([0.9, 0.5], device=dev)
+    proj[1, cols[2] + 7], proj[3, cols[2] + Dv + 9], proj[6, cols[2] + Dv - 1] = float("inf"), float("inf"), float("-inf")
+    batch, state = LO.RaggedBatch.build(counts, starts, [0, 1, 2], [[0], [1], [2]], 64, dev), start.clone()
+    got = LO.retention(proj, cols, batch, H, D, Dv, 0, None, None, decay, 1e-5, state).view(n, H, Dv)
+    assert not any(isinstance(k, tuple) and k[0] in ("pieces", "long") for k in batch._tiles)
+    p, r0 = proj.double(), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        S = start[b].double() if s else torch.zeros(H, D, Dv, dtype=torch.float64, device=dev)
+        for t in range(r0, r0 + c):
+            q, k = (p[t, x:x + H * D].view(H, D) for x in cols[:2])
+            v, gate = (p[t, x:x + H * Dv].view(H, Dv) for x in cols[2:])
+            S = decay.double().view(H, 1, 1) * S + (k * D ** -0.5).unsqueeze(-1) * v.unsqueeze(-2)
+            o = (q.unsqueeze(-1) * S).sum(-2)
+            o = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * torch.nn.functional.silu(gate)
+            ok = o.isfinite()
+            assert torch.equal(got[t].isfinite(), ok) and torch.allclose(got[t][ok].double(), o[ok], rtol=2e-5, atol=2e-5), (b, t)
+        assert torch.equal(state[b].isfinite(), S.isfinite())
+        r0 += c
