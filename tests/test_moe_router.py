@@ -97,3 +97,24 @@ def test_choices_among_values_that_are_not_numbers(monkeypatch, route, E, correc
     if route == "top_softmax" or (route == "sigmoid" and not correct):
         assert all(want[1][2 + i, :len(f)].tolist() == f for i, f in enumerate(first))
     assert all(len(set(row)) == 3 for row in want[1].tolist())
+
+
+@pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K,E", [(1, 1024, 16), (32, 2048, 33), (70, 520, 64), (2000, 200, 9)])
+def test_weights_of_random_operands(monkeypatch, x_dtype, N, K, E):
+    """The product's operands and sums keep 32 bits: every output's weight against 64 bits.  A rounding (2 ** -24) of each product and of its sums comes to less than 1e-6 of a logit of size one; a
+    weight rounded to 16 bits would be off by 2 ** -9, which is 3e-4 in a sigmoid."""
+    from jacobiforcing_amd import layer_ops as LO
+    for limit in ("ROUTER_DEPTH", "ROUTER_DEPTH_FEW"):
+        monkeypatch.setattr(LO, limit, 1 << 30)
+    g = torch.Generator(device="cuda").manual_seed(N + E)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, w, b, corr = rnd(N, K).to(x_dtype), rnd(E, K) * K ** -0.5, rnd(E), rnd(E)
+    h, up, down = rnd(N, 64).bfloat16(), rnd(E - 1, 32, 64).bfloat16(), rnd(E - 1, 64, 32).bfloat16()
+    assert LO._router_in_one(x, w, b)
+    z = x.double() @ w.double().T + b.double()
+    for route, want in (("sigmoid", z.sigmoid()), ("softmax_renorm", z.softmax(1)), ("top_softmax", z.softmax(1))):
+        _, ids, weights = LO.moe_experts(h, None, corr, E, 1.0, up, down, route=route, identity=1, router=(x, w, b))
+        assert torch.equal(ids.sort(1).values, torch.arange(E, device="cuda", dtype=torch.int32).expand(N, E))
+        got = torch.zeros_like(z).scatter_(1, ids.long(), weights.double())
+        assert float((got - want).abs().max()) < 2e-6, route

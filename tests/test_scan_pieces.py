@@ -135,3 +135,30 @@ def test_what_is_not_finite_reaches_later_tokens_only(monkeypatch, H, G, D, Dv, 
         off[t:t + 1 if what == "q" else n, h if what in ("v", "dt") else slice(H - per, H), c if what == "v" else slice(0, Dv)] = True
         assert torch.equal(~got.isfinite(), off) and torch.equal(got[~off], want[~off]), t
         assert torch.equal(got.isfinite(), scan.isfinite()) and torch.equal(state.isfinite(), scan_state.isfinite()) and torch.equal(state[state.isfinite()], clean[state.isfinite()]), t
+
+
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("H,G,D,Dv", [(6, 2, 64, 40), (4, 4, 128, 128), (8, 1, 96, 64)])
+@pytest.mark.parametrize("whole", [True, False])
+def test_operands_keep_their_24_bits(monkeypatch, H, G, D, Dv, fixed, whole):
+    """Memories of hundreds of tokens, against 64 bits: a rounding (2 ** -24) of each of the float sums' few halvings and of the operands, 5e-7 at most here; with two bfloat16 terms per operand instead of
+    three they would be off by 2 ** -17 each, 8e-6 in the outputs."""
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "scan_piece_groups", lambda counts, waves: -(-max(counts) // 64) if whole else 1)
+    g, n = torch.Generator(device="cuda").manual_seed(H * D), 500
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, start = rnd(n, 2 * G * D + H * Dv).bfloat16(), rnd(1, H, D, Dv)
+    kw = dict(decay=1 - 2.0 ** -torch.linspace(5, 9, H, device="cuda")) if fixed else dict(dt=rnd(n, H).bfloat16(), a_log=rnd(H) - 5, dt_bias=rnd(H), skip=rnd(H))
+    batch, st = LO.RaggedBatch.build([n], [1], [0], [list(range(8))], 64, "cuda"), start.clone()
+    got = LO.linear_scan(x, (0, G * D, 2 * G * D), batch, H, G, D, Dv, st, **kw).double().view(n, H, Dv)
+    q, k = (x[:, c:c + G * D].double().view(n, G, D).repeat_interleave(H // G, 1) for c in (0, G * D))
+    v, S, o = x[:, 2 * G * D:].double().view(n, H, Dv), start[0].double(), []
+    d = {key: t.double() for key, t in kw.items()}
+    for t in range(n):
+        u = torch.ones(H, dtype=torch.float64, device="cuda") if fixed else torch.nn.functional.softplus(d["dt"][t] + d["dt_bias"])
+        a = d["decay"] if fixed else torch.exp(-torch.exp(d["a_log"]) * u)
+        S = a.view(H, 1, 1) * S + k[t].unsqueeze(2) * (u.view(H, 1) * v[t]).unsqueeze(1)
+        o.append((S * q[t].unsqueeze(2)).sum(1) + (0 if fixed else d["skip"].view(H, 1) * v[t]))
+    o = torch.stack(o)
+    errors = float((got - o).norm() / o.norm()), float((st[0].double() - S).norm() / S.norm())
+    assert max(errors) < 1e-6, errors

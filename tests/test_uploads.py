@@ -47,13 +47,16 @@ def test_tables_do_not_wait_and_last():
     x = torch.randn(8192, 8192, device="cuda").bfloat16()
     x @ x
     torch.cuda.synchronize()
-    done = torch.cuda.Event()
-    for _ in range(60):                                      # tens of milliseconds
+    queued = torch.cuda.Event()
+    for _ in range(300):                                     # hundreds of milliseconds
         y = x @ x
+    queued.record()
+    first = LO.RaggedBatch.build([40], [0], [0], [list(range(8))], 64, "cuda")
+    assert not queued.query(), "the tables waited for the queue"
     got = torch.empty(200, 40, dtype=torch.int64, device="cuda")
     other = torch.cuda.Stream()
     for i in range(200):
-        b = LO.RaggedBatch.build([40], [i], [0], [list(range(i, i + 8))], 64, "cuda")
+        b = LO.RaggedBatch.build([40], [i], [0], [list(range(i, i + 8))], 64, "cuda") if i else first
         if i % 50 == 0:
             with torch.cuda.stream(other):
                 seen = b.kv_slot.clone()
@@ -61,8 +64,6 @@ def test_tables_do_not_wait_and_last():
             assert seen.tolist() == tables([40], [i], [0], [list(range(i, i + 8))], 64)[1]
         got[i].copy_(b.kv_slot)
         del b
-    done.record()
-    assert not done.query(), "the tables waited for the queue"
     torch.cuda.synchronize()
     assert got.tolist() == [tables([40], [i], [0], [list(range(i, i + 8))], 64)[1] for i in range(200)] and bool(y.isfinite().all())
 
