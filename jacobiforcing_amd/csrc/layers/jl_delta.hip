@@ -287,7 +287,7 @@ int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int 
     return JL_OK;
 }
 
-// ---- long portions on the float matrix instructions: 64 tokens at a time ------------------------------------------------------------------------
+// ---- long portions on the matrix instructions, of floats and (the chain) of bfloat16 terms: 64 tokens at a time ------------------------------------------------------------------------
 // With c_t = the running sum of ln g within a chunk of 64 tokens, S the state the chunk starts from, and u_t the corrections, the recurrence is
 //   (I + A) U = diag(beta) V - diag(beta e^c) K S,   A_tj = beta_t e^(c_t - c_j) (k_t . k_j) for j < t        (unit lower triangular)
 //   o_t = e^(c_t) S^T q_t + sum_{j <= t} e^(c_t - c_j) (q_t . k_j) u_j,        S <- e^(c_63) S + sum_j e^(c_63 - c_j) k_j u_j^T

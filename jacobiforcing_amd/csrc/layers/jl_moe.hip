@@ -176,9 +176,9 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *__restri
 
 // Rows of a tile.  High tiles read the weights less often and do more per byte of LDS, low ones pad less, give more workgroups and overlap their starts and ends.
 // 128 rows need both products to fill the chip and about a tile of rows per expert; 64 need as many blocks as the chip takes at once.  Measured, experts alone, gated,
-// bfloat16, us at 32 / 64 / 128 rows: 8192 tokens x 4 of 32 (2048 x 1024) 1059 / 790 / 623, 1024 tokens 213 / 171 / 160, 512 tokens 147 / 140 / 155, 256 tokens 121 / 124 / 142;
-// 4096 x 4 of 16 (1024 x 512) 180 / 135 / 123, 1024 tokens 75 / 66 / 79, 512 tokens 51 / 57 / 77; 4096 x 4 of 12 (768 x 512) 151 / 117 / 104, 2048 tokens 95 / 77 / 80;
-// float, 2048 x 4 of 16 (1024 x 512): 341 / 311 / 401.  (The tiles of 32 rows have become faster since, by 7 % at 256 tokens of the first.)
+// bfloat16, us at 32 / 64 / 128 rows, choice and grouping included: 8192 tokens x 4 of 32 (2048 x 1024) 1046 / 716 / 539, 1024 tokens 195 / 168 / 159, 512 tokens 136 / 132 / 143, 256 tokens
+// 111 / 117 / 140; 4096 x 4 of 16 (1024 x 512) 175 / 122 / 110, 1024 tokens 64 / 57 / 73, 512 tokens 47 / 51 / 69; 4096 x 4 of 12 (768 x 512) 147 / 105 / 91, 2048 tokens 85 / 66 / 70;
+// float, 2048 x 4 of 16 (1024 x 512), 32 / 64 rows: 356 / 318.
 // Sizes the matrix-core product does not take (rows that do not start at 16-byte borders) go in tiles of MOE_TM.
 static bool moe_mm_sizes(int dtype, int64_t K) { return (dtype == JL_BF16 && K % 8 == 0) || (dtype == JL_F32 && K % 4 == 0); }
 extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff) {
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const T *__restrict__ X, 
 // Loads carry no branch and no 64-bit address arithmetic of their own: offsets of 32 bits from a base (of the tile where its rows lie together; FAR: rows gathered from more than
 // 4 GiB have 64-bit addresses), rows that do not exist repeat another, stages behind the last repeat the
 // first, depths beyond the last whole stage come after the loop (a condition per load had cost six vector instructions per product: 431 us instead of 406 for the gated product
-// above; us for up and down at 32 rows x 4 of 16 of 1024 x 512: 49 -> 41, float 16 rows 100 -> 79, 400 rows 53 -> 45).
+// above).
 struct MoeMM {
     const void *X, *Wt;
     const int32_t *perm, *offsets, *tile_expert, *tile_row0;

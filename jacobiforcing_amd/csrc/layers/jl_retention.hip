@@ -9,8 +9,7 @@
 // four take 12.7; a step of 32 decoding requests 516 -> 503 us, which then waits for the host.
 constexpr int RET_TT = 8;
 
-// MAXT: the largest workgroup the instantiation is launched with.  With 256 the state's DMAX rows stay in registers up to
-// DMAX = 128 (the default bound of 1 024 threads leaves 128 registers per lane and spills them).
+// MAXT: the largest workgroup the instantiation is launched with (1 024 threads leave 128 registers per lane: one thread per column keeps up to 64 rows in them).
 // WHOLE: D is DMAX.  Else rows beyond D, zeros times a v that may not be finite, stay out of the sums: a branch per RB rows (fewer rows where a part has few; 32 tokens of 8 heads of 96: 9.8 -> 8.5 us, with its
 // bound of registers; 300 of 4 heads of 192 in chunks 276 -> 393).
 template <typename T, int DMAX, int PARTS, int MAXT, bool WHOLE>

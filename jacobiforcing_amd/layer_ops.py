@@ -37,10 +37,10 @@ SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep atten
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
 RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
-SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us of the launches,
-                                            # 4 x 2048 tokens of 16 heads of 128, at 1024 / 2048 / 4096: 149 / 128 / 168)
+SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us at
+                                            # 1024 / 2048 / 4096: 4 x 2048 tokens of 16 heads of 128 141 / 125 / 151, one of 8192 144 / 127 / 156; 2 x 2048 of 8 heads 59 / 63 / 63, 5 x 1500 of 6 heads of 64 44 / 44 / 44)
 DELTA_COLUMNS_FROM = 32       # delta rule: from this many tokens in a request's portion on, the state's columns are shared out over wavefronts
-DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (alone in its step; else delta_chunks_from.  us at 16 heads of 128, chunks / columns: 32 tokens 38 / 27, 64 41 / 44, 8 x 64 61 / 66)
+DELTA_CHUNKS_FROM = 64        # ... from here on its chunks of 64 tokens go to the matrix instructions (alone in its step; else delta_chunks_from.  us at 16 heads of 128, chunks / columns: 32 tokens 35 / 26, 40 35 / 31, 64 37 / 45, 8 x 64 49 / 67)
 DELTA_SCRATCH_FLOATS = 256 << 20     # scratch of those chunks at most (1 GiB: more heads than it holds take turns), as long as it holds one key head's
 
 
@@ -655,17 +655,17 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
 
 
 def retention_pieces_from(counts: Sequence[int], H: int, D: int) -> int:
-    """From how many tokens on the requests of a step run in pieces, the others in the scan behind them (0: all in the scan).  A round of pieces (one workgroup per CU) takes 37 us at
-    128 x 128, 18 at 64 x 64, however few tokens they hold; the scan 8.5 and 5.3 us per token of its longest portion, up to 1024 or 4096 (request, head) pairs at a time, and the more
-    requests it has besides, the less a longer portion shows.  us, scan of all / all in pieces / this rule: 8 heads of 128, 8 tokens and 250 x 1 101 / 319 / 101, 777 + 300 and 30 x 1
-    1063 / 101 / 93, 100 x 8 96 / 151 / 96, 100 x 16 165 / 158 / 158; 32 heads, 8 and 30 x 1 95 / 163 / 71, 40 + 10 and 60 x 1 360 / 323 / 113, 10 x 10 and 60 x 1 116 / 359 / 116; 16 heads
-    of 64, 200 x 20 153 / 255 / 153, 700, 40 x 10 and 40 x 1 746 / 130 / 112."""
+    """From how many tokens on the requests of a step run in pieces, the others in the scan behind them (0: all in the scan).  A round of pieces (one workgroup per CU) takes 27 us at
+    128 x 128, 19 at 64 x 64, however few tokens they hold, and with single tokens beside them about twice that; the scan 9 and 0.75 us per token of its longest portion.  The line was drawn when
+    the scan's threads kept whole columns (8.5 and 5.3 us per token): it is right where portions are long or all are short, and lies low for portions of 8 to 30 tokens.  us, scan of all / all in
+    pieces / this rule: 8 heads of 128, 8 tokens 13 / 27 / 27, 32 32 / 30 / 30, 8 and 250 x 1 41 / 323 / 41, 777 + 300 and 30 x 1 166 / 100 / 70, 100 x 8 36 / 153 / 36, 100 x 16 53 / 158 / 158;
+    32 heads, 8 and 30 x 1 23 / 163 / 52, 40 + 10 and 60 x 1 52 / 322 / 73, 10 x 10 and 60 x 1 50 / 356 / 50; 16 heads of 64, 200 x 20 70 / 253 / 70, 700, 40 x 10 and 40 x 1 118 / 129 / 100."""
     long = sum(c >= RETENTION_PIECES_FROM for c in counts)
     rounds = -(-long * H // 256)
     least = max(RETENTION_PIECES_FROM, min(4 * rounds, 16) if D > 64 else min(3 * rounds, 48), 3 + (len(counts) - long) * H // 230)
     if max(counts) < least:
         return 0
-    return 1 if len(counts) * H < 256 else least                     # single tokens beside them where CUs are free: a launch less (8 heads, 8 and 30 x 1 53 / 62 us)
+    return 1 if len(counts) * H < 256 else least                     # single tokens beside them where CUs are free: a launch less
 
 
 def retention(proj: torch.Tensor, cols: Tuple[int, int, int, int], batch: RaggedBatch, H: int, D: int, Dv: int, rot_dims: int,
@@ -1328,8 +1328,8 @@ def delta_chunks_from(counts: Sequence[int], H: int, D: int) -> int:
     """From how many tokens on the requests of a step go through the delta rule in chunks, the others behind them in the forms for short portions (0: none of them).  Portions of
     DELTA_CHUNKS_FROM tokens on are worth it alone; beside other requests the times of both ways are estimated, us per chunk of the longest, chunk and head, token of the columns' longest, token
     and head, request and head, token of the others' longest.  At widths of 64 the columns' walk is the faster one as soon as it fills the chip.  us, columns / chunks from 64 tokens on /
-    this rule: 16 heads of 64, 100 x 100 214 / 404 / 214, 30 x 200 164 / 227 / 164; 8 heads of 128, 70 and 10 x 31 56 / 140 / 56, 300 + 63 174 / 104 / 65, 64 and 200 x 1 131 / 117 / 117,
-    100 x 64 333 / 225 / 225."""
+    this rule: 16 heads of 64, 100 x 100 233 / 288 / 231, 30 x 200 175 / 170 / 177; 8 heads of 128, 70 and 10 x 31 57 / 135 / 57, 300 + 63 178 / 93 / 51, 64 and 200 x 1 110 / 89 / 90,
+    100 x 64 356 / 178 / 177.  (The times per chunk are those of a chain and chunks that took half as long again: the rule still finds the better way in these, by less.)"""
     if max(counts) < DELTA_CHUNKS_FROM or len(counts) == 1:
         return DELTA_CHUNKS_FROM if max(counts) >= DELTA_CHUNKS_FROM else 0
     first, chain, chunk, step, token, request, alone, single = (30, 6.7, 0.28, 0.6, 5.5e-3, 0.05, 2.7, 0.045) if D > 64 else (24, 4.9, 0.145, 0.49, 1.34e-3, 6e-3, 1.4, 0.012)
