@@ -10,6 +10,7 @@ import ctypes as C
 import itertools
 import operator
 import os
+import threading
 from collections import deque
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence, Tuple
@@ -74,13 +75,37 @@ def _dev(t: torch.Tensor) -> None:
 
 
 _UPLOADS: dict = {}                                  # device index -> the stream its tables are copied on, and a block of its pool
-_GONE: dict = {}                                     # a stream's id -> the stream, and the tables uploaded from it whose batch is gone
+_GONE: dict = {}                                     # a stream's id -> _Gone
+GONE_AT_ONCE = 64                                    # tables (of some KB each; built keys' rows of a long step up to a MB) that wait for an event together
+
+
+class _Gone:
+    """Tables uploaded from one stream whose batch is gone.  They are let go, GONE_AT_ONCE at a time, once the stream is done with what lies in front of an upload behind their batch's end.  One
+    event says so for all of them: an event takes the host 15 to 20 us (one portion of 200 tokens, us a pass: one per table or per upload 695, this 665, tables on the kernels' stream 655)."""
+
+    def __init__(self, stream: torch.cuda.Stream):
+        self.stream, self.tables, self.waiting, self.lock = stream, deque(), deque(), threading.Lock()
+
+    def sweep(self) -> None:
+        if len(self.tables) < GONE_AT_ONCE:
+            return
+        with self.lock:
+            while self.waiting and self.waiting[0][0].query():
+                for t in self.waiting.popleft()[1]:
+                    if torch._C._storage_Use_Count(t.untyped_storage()._cdata) > 2:      # more than this tensor and its storage's object: somebody kept a part of the tables
+                        t.record_stream(self.stream)
+            left = []
+            while self.tables:
+                left.append(self.tables.popleft())
+            event = torch.cuda.Event()
+            event.record(self.stream)
+            self.waiting.append((event, left))
 
 
 def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
     """``host`` on ``device``, there for every stream when this returns.  A copy from ordinary host memory waits for its stream: on one of its own it waits for itself and not for the kernels
     queued so far.  That shows where passes queue behind one another (us a pass, tables on the kernels' stream / on this one: 32 decoding requests of Mikipel 860 / 796, 4 prompts of 2048 of Lokizen
-    2402 / 2301); on an idle stream an upload costs about 10 us more (one token of Safisun 619 / 637).
+    2402 / 2301).
     The tensor joins ``held``, the batch's list.  Its memory goes back to the copies' stream once the stream that asked for it is done with what lies in front of its first upload behind the batch's
     end: what a caller makes that stream wait for until then (kernels of another stream that read the tables) comes first, as it did when the memory was that stream's own."""
     device = torch.device(device)
@@ -97,13 +122,9 @@ def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
             _UPLOADS.setdefault(index, (side, torch.empty(1, dtype=torch.int32, device=device)))
     side, user = _UPLOADS[index][0], torch._C._cuda_getCurrentStream(index)      # (the stream's id, not an object for every upload)
     if user not in _GONE:
-        _GONE.setdefault(user, (torch.cuda.current_stream(index), deque()))
-    stream, gone = _GONE[user]
-    while gone:
-        try:
-            gone.popleft().record_stream(stream)
-        except IndexError:                               # another thread took the last one
-            break
+        _GONE.setdefault(user, _Gone(torch.cuda.current_stream(index)))
+    gone = _GONE[user]
+    gone.sweep()
     if index == here:                                    # a fifth of what the context below takes
         torch._C._cuda_setStream(stream_id=side.stream_id, device_index=side.device_index, device_type=side.device_type)
         try:
@@ -113,8 +134,7 @@ def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
     else:
         with torch.cuda.stream(side):
             up = t.to(device)
-    up.record_stream(stream)                             # (views of it may outlive the batch)
-    held.append((gone, up))
+    held.append((gone.tables, up))
     return up
 
 
@@ -139,7 +159,8 @@ class RaggedBatch:
     slots: List[int]
     _tiles: dict
     _host_tables: Optional[np.ndarray] = None         # tables on the host, for key_rows and part (None: read back when they need it)
-    _whole: Optional[Tuple[int, torch.Tensor]] = None  # the largest portion, and a tile per request (None: a request without tokens)
+    # the largest portion, and where a tile per request lies in the upload, and behind it, for portions of SCAN_PIECES_FROM tokens on (else 0), a piece per request and the requests' records of them
+    _whole: Optional[Tuple[int, torch.Tensor, int, int]] = None      # (None: a request without tokens)
     _held: list = field(default_factory=list, repr=False, compare=False)      # what was uploaded for it, with the list it joins behind the batch's end
 
     def __del__(self):
@@ -162,15 +183,21 @@ class RaggedBatch:
             raise ValueError("a request of fewer than no tokens")
         row0 = list(itertools.accumulate(counts, initial=0))
         N_ = row0[B]
-        # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on; `whole`: tiles() of steps whose requests are one tile each
+        # one upload: the pool tokens (64 bits), then the 32-bit tables, each from a 16-byte border on; `whole`: tiles() and pieces() of steps whose requests are one tile, one piece each (on
+        # an idle stream a second upload costs a step of 40 tokens 25 us)
         seq = [x for r in zip(row0, counts, starts, slots) for x in r]
         whole = [x for r in zip(range(B), starts, counts, row0) for x in r]
-        sizes = (4 * B, B * C_, N_, N_, 4 * B)
+        longest, pieced = max(counts), 0
+        if longest >= SCAN_PIECES_FROM and min(counts) > 0:
+            pieced = 4 * B
+            whole += [x for r, c, sl in zip(row0, counts, slots) for x in (r, c, sl, 1)]
+            whole += [x for b, s, sl in zip(range(B), starts, slots) for x in (b, 1, s, sl)]
+        sizes = (4 * B, B * C_, N_, N_, 4 * B, pieced, pieced)
         at = list(itertools.accumulate(((n + 3) // 4 * 4 for n in sizes), initial=2 * (N_ + N_ % 2)))
         host = np.empty(at[-1] // 2, dtype=np.int64)
         words = host.view(np.int32)
         a_seq, a_bt, a_req, a_pos, a_whole = at[:5]
-        words[a_seq:a_seq + 4 * B], words[a_whole:a_whole + 4 * B] = seq, whole
+        words[a_seq:a_seq + 4 * B], words[a_whole:a_whole + 4 * B + 2 * pieced] = seq, whole
         bt = words[a_bt:a_bt + B * C_].reshape(B, C_)
         pages = np.fromiter(itertools.chain.from_iterable(block_tables), dtype=np.int64, count=sum(held))
         if min(held) == C_:
@@ -182,17 +209,22 @@ class RaggedBatch:
             words[a_req:a_req + N_], words[a_pos:a_pos + N_] = range(B), starts
             host[:N_] = [int(t[s // page_size]) * page_size + s % page_size for t, s in zip(block_tables, starts)]
         elif N_:
-            c = np.asarray(counts)
-            pos = np.arange(N_, dtype=np.int64) + np.repeat(np.asarray(starts) - row0[:B], c)
-            words[a_req:a_req + N_], words[a_pos:a_pos + N_] = np.repeat(np.arange(B, dtype=np.int32), c), pos
-            host[:N_] = pages[np.repeat(np.cumsum(held) - held, c) + pos // page_size] * page_size + pos % page_size
+            if B == 1:
+                rows, pos, first = 0, np.arange(starts[0], starts[0] + N_), 0
+            else:
+                rows = np.repeat(np.arange(B), counts)
+                pos = np.arange(N_) + np.asarray(starts)[rows] - np.asarray(row0)[rows]
+                first = np.asarray(list(itertools.accumulate(held, initial=0)))[rows]
+            page = pos // page_size
+            words[a_req:a_req + N_], words[a_pos:a_pos + N_] = rows, pos
+            host[:N_] = pages[first + page] * page_size + (pos - page * page_size)
         held_by = []
         up = _upload(host, device, held_by)
         w32 = up.view(torch.int32)
-        d_seq, d_bt, d_req, d_pos, d_whole = (w32[a:a + n] for n, a in zip(sizes, at))
-        return cls(B=B, N=N_, counts=counts, starts=starts, seq=d_seq.view(B, 4), kv_slot=up[:N_], tables=d_bt.view(B, C_), row_req=d_req, pos=d_pos, page_size=int(page_size),
+        return cls(B=B, N=N_, counts=counts, starts=starts, seq=w32.as_strided((B, 4), (4, 1), a_seq), kv_slot=up[:N_], tables=w32.as_strided((B, C_), (C_, 1), a_bt),
+                   row_req=w32[a_req:a_req + N_], pos=w32[a_pos:a_pos + N_], page_size=int(page_size),
                    max_pos=max(s + c for s, c in zip(starts, counts)), max_page=int(bt.max()), max_slot=max(slots), slots=slots, _tiles={}, _host_tables=bt,
-                   _whole=(max(counts), d_whole.view(B, 4)) if min(counts) > 0 else None, _held=held_by)
+                   _whole=(longest, w32, a_whole, pieced) if min(counts) > 0 else None, _held=held_by)
 
     def chunks(self, size: int):
         """A portion of at least two chunks is cut into chunks of ``size`` tokens that the recurrent layers run side by side.
@@ -219,6 +251,9 @@ class RaggedBatch:
         last piece}, request records [requests with tokens, 4] int32 {first piece, pieces, pos0, slot}), on the device.  A request without tokens has
         no record: more pieces than records means that some request has several."""
         key = ("pieces", size)
+        if key not in self._tiles and self._whole is not None and self._whole[0] <= size and self._whole[3]:
+            _, words, at, n = self._whole                # came with the batch's own upload
+            self._tiles[key] = tuple(words.as_strided((self.B, 4), (4, 1), at + x * n) for x in (1, 2))
         if key not in self._tiles:
             rec, req, r0 = [], [], 0
             for c, s, sl in zip(self.counts, self.starts, self.slots):
@@ -291,7 +326,7 @@ class RaggedBatch:
         key = ("longest first" if longest_first else "in order", tq, None if requests is None else tuple(requests)) if longest_first or requests is not None else tq
         t = self._tiles.get(key)
         if t is None and key == tq and self._whole is not None and self._whole[0] <= tq:
-            t = self._tiles[key] = self._whole[1]        # came with the batch's own upload
+            t = self._tiles[key] = self._whole[1].as_strided((self.B, 4), (4, 1), self._whole[2])      # came with the batch's own upload
         if t is None:
             rows, r0 = [], 0
             for b, (c, s) in enumerate(zip(self.counts, self.starts)):

@@ -98,6 +98,18 @@ def test_requests_without_tokens_have_no_record_of_pieces():
     assert rec.tolist() == [[0, 64, 1, 0], [64, 64, 1, 1], [128, 5, 3, 1]] and req.tolist() == [[0, 2, 0, 1], [2, 1, 64, 3]]
 
 
+@pytest.mark.parametrize("counts", [[40, 7, 1], [31, 7], [100], [64, 65], [200, 1, 90]])
+def test_pieces_that_come_with_the_tables(counts):
+    """Portions that are one piece each have their records in the batch's own upload; the same as made on their own."""
+    import dataclasses
+    b = batch(counts, [3, 0, 70][:len(counts)])
+    bare = dataclasses.replace(b, _tiles={}, _whole=None)
+    for size in (64, 128, 256):
+        got, want = b.pieces(size), bare.pieces(size)
+        assert [t.tolist() for t in got] == [t.tolist() for t in want] and all(t.dtype == torch.int32 and t.is_contiguous() for t in got)
+        assert (got[0].untyped_storage().data_ptr() == b.seq.untyped_storage().data_ptr()) == (32 <= max(counts) <= size)
+
+
 def test_what_a_batch_is_built_of():
     """Page tables beyond the requests' are left out, but for the tables' width; lists of other lengths, positions that are not whole and counts below zero are refused."""
     build = lambda counts=[1, 70], starts=[2, 0], slots=[0, 1], tables=[[1], [2, 3], [4, 5, 6]]: LO.RaggedBatch.build(counts, starts, slots, tables, 64, "cpu")

@@ -88,6 +88,7 @@ def test_tables_that_another_stream_reads():
 
 
 @pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
 def test_tables_are_refused_in_a_capture():
     """... before anything that would leave an error behind."""
     build = lambda: LO.RaggedBatch.build([3, 1], [0, 5], [0, 1], [[0], [1]], 64, "cuda")
@@ -98,3 +99,23 @@ def test_tables_are_refused_in_a_capture():
         b.pieces(64)
     torch.cuda.synchronize()
     assert build().pos.tolist() == [0, 1, 2, 5] and b.pieces(64)[1].tolist() == [[0, 1, 0, 0], [1, 1, 5, 1]]
+
+
+@pytest.mark.gpu
+def test_what_is_kept_is_given_back(monkeypatch):
+    """Tables of batches that are gone wait for one event at a time and then go, but for those that somebody kept a part of, which stay whole."""
+    monkeypatch.setattr(LO, "GONE_AT_ONCE", 8)
+    build = lambda i: LO.RaggedBatch.build([40], [i], [0], [list(range(i, i + 8))], 64, "cuda")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        kept = [build(i).kv_slot[3:] for i in range(20)]
+        for i in range(300):
+            b = build(i % 100)
+            b.pieces(64)
+        torch.cuda.synchronize()
+        gone = next(g for g in LO._GONE.values() if g.stream == stream)
+        for i in range(2 * LO.GONE_AT_ONCE):                     # two sweeps more: the first finds all events passed
+            b = build(i)
+        assert len(gone.tables) <= LO.GONE_AT_ONCE and sum(len(left) for _, left in gone.waiting) <= 3 * LO.GONE_AT_ONCE
+        torch.cuda.synchronize()
+        assert all(t.tolist() == tables([40], [i], [0], [list(range(i, i + 8))], 64)[1][3:] for i, t in enumerate(kept))
