@@ -142,7 +142,8 @@ def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
 class RaggedBatch:
     """What one step runs: requests b = 0..B-1 with ``counts[b]`` new tokens from position ``starts[b]``, state slot ``slots[b]``
     and pages ``block_tables[b]``.  Device tensors: ``seq`` [B, 4] int32 {row0, count, pos0, slot}, ``kv_slot`` [N] int64 (pool
-    token of every new row), ``tables`` [B, C] int32, ``row_req`` / ``pos`` [N] int32 (request and position of every row)."""
+    token of every new row), ``tables`` [B, C] int32, ``row_req`` / ``pos`` [N] int32 (request and position of every row).  They are there for every stream when ``build`` returns; a stream
+    other than the one that was current then may read them for as long as that one is made to wait for it before it builds its next batch."""
     B: int
     N: int
     counts: List[int]
