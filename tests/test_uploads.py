@@ -69,8 +69,9 @@ def test_tables_do_not_wait_and_last():
 
 
 @pytest.mark.gpu
-def test_tables_that_another_stream_reads():
+def test_tables_that_another_stream_reads(monkeypatch):
     """A batch built on one stream, read behind a queue on another and dropped: its memory is not written before the first stream, which waits for the other, is through."""
+    monkeypatch.setattr(LO, "GONE_AT_ONCE", 1)
     x, other, here = torch.randn(8192, 8192, device="cuda").bfloat16(), torch.cuda.Stream(), torch.cuda.current_stream()
     for start in (7, 3):
         b = LO.RaggedBatch.build([40], [start], [0], [[5, 9, 2]], 64, "cuda")
