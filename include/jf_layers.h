@@ -215,6 +215,10 @@ JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, co
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                          void *stream);
 
+/* The same for float rows of any number (x [N, x_ld], W [O, K], rows at 16-byte borders, out rows out_ld floats apart), on the bfloat16 matrix instructions in three terms per operand: sums at
+ * least as close to 64 bits as the float instructions' (products below 2^-110 aside). */
+JL_API int jl_linear_split(const float *x, int64_t N, int64_t x_ld, const float *w, int32_t K, int32_t O, const float *bias, float *out, int64_t out_ld, void *stream);
+
 /* z <- cap * tanh(z / cap) in place over `total` floats (soft cap of the logits). */
 JL_API int jl_softcap(float *z, int64_t total, float cap, void *stream);
 /* the same of z (`dtype`) into out */
@@ -445,6 +449,8 @@ JL_API int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, i
 JL_API int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff);
 /* 1: bfloat16 tiles of 128 rows are better grouped in pairs (tile_rows 256 for jl_moe_group and the products) */
 JL_API int jl_moe_tile_pairs(int64_t rows, int32_t E, int32_t W, int32_t ff, int32_t gated);
+/* 64, or 256 where float tiles of 64 rows are better grouped in fours */
+JL_API int jl_moe_float_tiles(int64_t rows, int32_t E, int32_t W, int32_t ff);
 
 /* Router product, choice and grouping of a step of up to 32 * JL_MOE_ROUTER_BLOCKS tokens in one call: logits = x W^T (+ bias) in float (x [N, K] of x_dtype with rows x_ld apart, W [E, K] and bias float),
  * then what jl_moe_route gives for them (`E` outputs, kind, correction) and what jl_moe_group gives for the `experts` of them that have weights.  E <= 64, K a multiple of 4, rows of x and W at

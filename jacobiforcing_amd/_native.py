@@ -345,6 +345,7 @@ _LAYER_SIGNATURES = {
     "jl_delta_rule": (C.c_int, [_vp, C.c_int, _i64, _i32, _i32, _i32, _vp, C.c_int, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                 _i32, _i32, _f32, _f32, _f32, _vp, _vp, _vp, _vp]),
     "jl_linear_mid": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _i64, _i32, _vp]),
+    "jl_linear_split": (C.c_int, [_vp, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _i64, _vp]),
     "jl_linear_small": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, C.c_int, _i32, _i32, _vp, _vp, _i64, _i32, _vp]),
     "jl_heads_gate": (C.c_int, [_vp, _vp, _i64, C.c_int, _i64, _i32, _i32, _vp, _vp]),
     "jl_retention": (C.c_int, [_vp, C.c_int, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp, _f32,
@@ -356,6 +357,7 @@ _LAYER_SIGNATURES = {
     "jl_moe_group": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _vp]),
     "jl_moe_tile_rows": (C.c_int, [C.c_int, _i64, _i32, _i32, _i32]),
     "jl_moe_tile_pairs": (C.c_int, [_i64, _i32, _i32, _i32, _i32]),
+    "jl_moe_float_tiles": (C.c_int, [_i64, _i32, _i32, _i32]),
     "jl_moe_router_blocks": (C.c_int, [_i64]),
     "jl_moe_router_run": (C.c_int, [C.POINTER(MoeRouter), _vp]),
     "jl_moe_gemm": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
@@ -363,7 +365,7 @@ _LAYER_SIGNATURES = {
 }
 LAYER_SYMBOLS = tuple(_LAYER_SIGNATURES)
 # which library a symbol lives in (jacobiforcing_amd/_build.py: LAYER_GROUPS); both carry their own jl_version / jl_last_error
-_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_router_blocks", "jl_moe_router_run", "jl_moe_gemm", "jl_moe_gemm_gated")
+_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_float_tiles", "jl_moe_router_blocks", "jl_moe_router_run", "jl_moe_gemm", "jl_moe_gemm_gated")
 
 
 class _LayerLibs:

@@ -1,5 +1,6 @@
 // jl_linear.hip — dense products of a few rows (decoding): out[n] = W x[n] (+ bias), W [O, K] read once.
 #include "jl_small.h"
+#include "jl_split.h"
 
 // What bounds such a product is W's bytes when W is large and the way there when it is small (a launch alone is 3 us, a trip to memory 2 us).  So a workgroup's NW wavefronts
 // share the depth of 16 * OT rows of W, every lane has LS_AHEAD pairs of 16-byte units of each of its rows of W and x (which comes from L2) on the way at once, straight into the
@@ -170,6 +171,57 @@ extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, 
     linear_mid_kernel<<<dim3((unsigned)groups), 256, 0, (hipStream_t)stream>>>((const bf16_t *)x, x_ld, (const bf16_t *)w, (const bf16_t *)bias, out, out_ld, (int)N, K, O, out_mode,
                                                                               row_tiles);
     return jl_check_launch("linear_mid_kernel");
+}
+
+// ---- float products of many rows: TM of x by 128 of W per workgroup, on the bfloat16 matrix instructions in three terms per operand (jl_split.h) -----
+// Eight wavefronts, so that two share a SIMD where a CU has one tile only: one wavefront issues vector instructions at half their rate and makes its terms while nobody multiplies (64 rows, one tile per
+// CU, 1024 depths: 36 us with four, 27 with eight).  Large products reach 184 TFLOP/s, 1100 of the bfloat16 instructions, which is what a large bfloat16 product reaches here; smaller ones
+// wait for their stages.  Error against 64 bits of 2553 x 1024 by 1024, 2-norm: 4.9e-7, the library's on the float instructions 5.7e-7 (of 4096 x 4096 by 4096 1.0e-6 / 1.15e-6).
+template <int TM, int NW, int WM, int TKU>
+__global__ __launch_bounds__(64 * NW, NW / 2) void linear_split_kernel(const float *__restrict__ x, int64_t x_ld, const float *__restrict__ w, const float *__restrict__ bias, float *__restrict__ out,
+                                                              int64_t out_ld, int64_t N, int K, int O, int row_tiles, int tiles) {
+    constexpr int WR = 128, XT = TM / WM / 32, WN = NW / WM, NT = WR / WN / 32;
+    __shared__ uint4 smem[split_units(TM, WR, TKU)];
+    // workgroups with the same remainder by 8 share an XCD: neighbouring tiles, which share W's rows
+    const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5, wm = wave / WN, wn = wave % WN;
+    const int64_t n0 = (int64_t)(tile % row_tiles) * TM;
+    const int o0 = tile / row_tiles * WR;
+    auto x_at = [&](int m) { return x + (n0 + m < N ? n0 + m : N - 1) * x_ld; };
+    auto w_at = [&](int j) { return w + (int64_t)(o0 + j < O ? o0 + j : O - 1) * K; };
+    auto x_row = [&](int t) { return wm * (TM / WM) + 32 * t; };
+    auto w_row = [&](int t) { return wn * (WR / WN) + 32 * t; };
+    sp_f32x16 acc[XT][NT];
+    split_products<TM, WR, NW, WM, TKU>(acc, smem, K, x_at, w_at, x_row, w_row);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int o = o0 + w_row(t) + l32;
+        if (o >= O) continue;
+        const float add = bias ? bias[o] : 0.f;
+#pragma unroll
+        for (int xt = 0; xt < XT; ++xt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t n = n0 + x_row(xt) + 8 * (r >> 2) + 4 * hi + (r & 3);
+                if (n < N) out[n * out_ld + o] = acc[xt][t][r] + add;
+            }
+    }
+}
+
+extern "C" int jl_linear_split(const float *x, int64_t N, int64_t x_ld, const float *w, int32_t K, int32_t O, const float *bias, float *out, int64_t out_ld, void *stream) {
+    if (N <= 0 || O <= 0) return JL_OK;
+    if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < O) return jl_fail(JL_E_INVALID, "jl_linear_split: null pointer or bad sizes");
+    if (K % 4 || x_ld % 4 || (((uintptr_t)x | (uintptr_t)w) & 15)) return jl_fail(JL_E_INVALID, "jl_linear_split: rows of x and W at 16-byte borders");
+    const int64_t cols = ((int64_t)O + 127) / 128;
+    // 128 rows per tile as soon as they give about half of the CUs one each.  us, 128 / 64 rows: 2553 x 1024 by 1100 (180 tiles of 128) 47 / 52, by 4096 139 / 150, 1500 x 768 by 1536 (144) 36 / 39;
+    // below, 512 x 1024 by 4096 (128) 51 / 36, 2553 x 512 by 768 (120) 26 / 18
+    const bool low = (N + 127) / 128 * cols < 140;
+    const int64_t row_tiles = low ? (N + 63) / 64 : (N + 127) / 128, tiles = row_tiles * cols;
+    if (tiles > INT32_MAX / 512) return jl_fail(JL_E_INVALID, "jl_linear_split: too many tiles");
+    (low ? linear_split_kernel<64, 8, 2, 8> : linear_split_kernel<128, 8, 2, 4>)<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 512, 0, (hipStream_t)stream>>>(x, x_ld, w, bias, out, out_ld, N, K, O,
+                                                                                                                                                       (int)row_tiles, (int)tiles);
+    return jl_check_launch("linear_split_kernel");
 }
 
 extern "C" int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,

@@ -2,6 +2,7 @@
 // a correction, or a softmax over the chosen logits alone), the rows grouped by expert (a choice of an expert without weights has none), and
 // the grouped products: up with relu^2, plain, or with the gated unit in its epilogue, down with the routing weights.
 #include "jl_small.h"
+#include "jl_split.h"
 #include <stdlib.h>
 #include <type_traits>
 constexpr int MOE_MAX_E = 4096;   // experts (router outputs) at most
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *__restri
 // 128 rows need both products to fill the chip and about a tile of rows per expert; 64 need as many blocks as the chip takes at once.  Measured, experts alone, gated,
 // bfloat16, us at 32 / 64 / 128 rows, choice and grouping included: 8192 tokens x 4 of 32 (2048 x 1024) 1046 / 716 / 539, 1024 tokens 195 / 168 / 159, 512 tokens 136 / 132 / 143, 256 tokens
 // 111 / 117 / 140; 4096 x 4 of 16 (1024 x 512) 175 / 122 / 110, 1024 tokens 64 / 57 / 73, 512 tokens 47 / 51 / 69; 4096 x 4 of 12 (768 x 512) 147 / 105 / 91, 2048 tokens 85 / 66 / 70;
-// float, 2048 x 4 of 16 (1024 x 512), 32 / 64 rows: 356 / 318.
+// float, 2048 x 4 of 16 (1024 x 512), 32 / 64 rows: 356 / 318 (64 on the float instructions).
 // Sizes the matrix-core product does not take (rows that do not start at 16-byte borders) go in tiles of MOE_TM.
 static bool moe_mm_sizes(int dtype, int64_t K) { return (dtype == JL_BF16 && K % 8 == 0) || (dtype == JL_F32 && K % 4 == 0); }
 extern "C" int jl_moe_tile_rows(int dtype, int64_t rows, int32_t E, int32_t W, int32_t ff) {
@@ -196,6 +197,12 @@ static bool moe_big_sizes(int64_t K, int64_t rows) { return K % 64 == 0 && rows 
 extern "C" int jl_moe_tile_pairs(int64_t rows, int32_t E, int32_t W, int32_t ff, int32_t gated) {
     const int cols = gated ? 128 : 256;
     return E > 0 && rows >= (int64_t)256 * E && (rows / 256 + E / 2) * ((ff + cols - 1) / cols) >= 640 && moe_big_sizes(W, rows + (int64_t)256 * E);
+}
+
+// Float tiles of 64 rows in fours, which the products walk in parts of 128 rows (moe_split_kernel), where experts fill them.  us, experts alone, gated, 64 / 128: 638 rows per expert (2553 x 4 of 16 of
+// 1024 x 512) 276 / 248, 383 170 / 158, 340 (2042 x 4 of 24 of 768 x 320) 124 / 116; below the line 311 (700 x 4 of 9 of 1024 x 1024) 167 / 220, 263 (2042 x 4 of 31 of 960 x 704) 304 / 330, 255 167 / 147 and 137 / 156.
+extern "C" int jl_moe_float_tiles(int64_t rows, int32_t E, int32_t W, int32_t ff) {
+    return E > 0 && rows >= (int64_t)320 * E && moe_mm_sizes(JL_F32, W) && moe_mm_sizes(JL_F32, ff) ? 256 : 64;
 }
 
 extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t E, int32_t tile_rows, int32_t *perm, int32_t *offsets,
@@ -981,6 +988,41 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(MoeMM a) {
     while (half ? walk(std::integral_constant<int, XT / 2>()) : walk(std::integral_constant<int, XT>())) {}
 }
 
+// ---- the same product of floats for experts with many rows, on the bfloat16 matrix instructions in three terms per operand (jl_split.h) -----------------------------------------------
+// 64 rows by 256 weight rows (four wavefronts), 128 by 128 (eight) where experts fill them (jl_moe_float_tiles).  us of the experts on the float instructions (64 x 256) / so: 2553 x 4 of 16 of 1024 x 512
+// gated 348 / 248, plain 258 / 182, 1021 x 3 of 24 of 1024 x 1024 254 / 210, 2042 x 2 of 16 of 1024 x 512 221 / 167; error against 64 bits 9.7e-7 / 8.3e-7.
+template <int TM, int WR, int NW, int WM, int TKU, bool GATED>
+__global__ __launch_bounds__(64 * NW, NW / 2) void moe_split_kernel(MoeMM a) {
+    constexpr int WN = NW / WM, XT = TM / WM / 32, NT = WR / WN / 32, TN = GATED ? WR / 2 : WR;
+    __shared__ uint4 smem[split_units(TM, WR, TKU)];
+    __shared__ int rows_out[TM];                                    // way down: the flat indices and weights of the tile's rows
+    __shared__ float rows_weight[TM];
+    // workgroups with the same remainder by 8 share an XCD
+    const int per_xcd = (a.offsets[a.E + 1] + 7) / 8, xcd = blockIdx.x & 7, s = blockIdx.x >> 3;
+    if (s >= per_xcd * a.col_blocks * a.parts) return;
+    const int tile = xcd * per_xcd + s / (a.col_blocks * a.parts), part = s / a.col_blocks % a.parts, col = s % a.col_blocks;
+    if (tile >= a.max_tiles) return;
+    const int e = a.tile_expert[tile];
+    if (e < 0) return;
+    const int r0 = a.tile_row0[tile] + part * TM, K = a.K, n_out = a.n_out, n0 = col * TN, left = a.offsets[e + 1] - r0, nr = left < TM ? left : TM;
+    if (nr <= 0) return;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wm = wave / WN, wn = wave % WN;
+    if (!GATED && a.mode == 1 && tid < nr) {
+        const int p = a.perm[r0 + tid];
+        rows_out[tid] = p;
+        rows_weight[tid] = a.weights[p];
+    }
+    const float *W = (const float *)a.Wt + (int64_t)e * (GATED ? 2 : 1) * n_out * K;
+    // the first half of a gated tile's rows are the gate's, the others the linear branch's, n_out further on; rows that do not exist repeat others and are not stored
+    auto x_at = [&](int m) { const int row = m < nr ? m : 0; return (const float *)a.X + (int64_t)(a.mode != 1 ? a.perm[r0 + row] / a.top : r0 + row) * K; };
+    auto w_at = [&](int j) { const int c = n0 + (GATED ? j % TN : j); return W + ((c < n_out ? c : n_out - 1) + (int64_t)(GATED && j >= TN ? n_out : 0)) * K; };
+    auto x_row = [&](int x) { return wm * (TM / WM) + 32 * x; };
+    auto w_row = [&](int t) { return GATED ? (t < NT / 2 ? 0 : TN) + wn * (TN / WN) + 32 * (t % (NT / 2 > 0 ? NT / 2 : 1)) : wn * (WR / WN) + 32 * t; };
+    mm_f32x16 acc[XT][NT];
+    split_products<TM, WR, NW, WM, TKU>(acc, smem, K, x_at, w_at, x_row, w_row);
+    moe_store<float, XT, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int x, int k, int &p, float &w) { const int m = x_row(x) + k; p = rows_out[m]; w = rows_weight[m]; }, x_row, w_row, lane);
+}
+
 template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(MoeMM &a, bool gated, hipStream_t st) {
     const int tn = gated ? WR / 2 : WR;
     a.col_blocks = (a.n_out + tn - 1) / tn;
@@ -1004,8 +1046,18 @@ template <typename T> static int moe_mm_rows(MoeMM &a, int tile_rows, bool gated
             return jl_check_launch("moe_big_kernel");
         }
         if (tile_rows == 128) return moe_mm_launch<T, 128, 4, 256, 4>(a, gated, st);
-    } else if (tile_rows >= 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32 or 64 rows");
-    if (tile_rows == 64) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
+    } else if (tile_rows == 128) return jl_fail(JL_E_INVALID, "jl_moe_gemm: float tiles have 32, 64 or 256 rows");
+    if (tile_rows == 64 || tile_rows == 256) {
+        if constexpr (sizeof(T) == 2) return moe_mm_launch<T, 64, 4, 256, 4>(a, gated, st);
+        const int tm = tile_rows == 256 ? 128 : 64, tn = (tile_rows == 256 ? 128 : 256) / (gated ? 2 : 1);
+        a.parts = tile_rows / tm;
+        a.col_blocks = (a.n_out + tn - 1) / tn;
+        const int64_t groups = (int64_t)(a.max_tiles + 7) / 8 * 8 * a.col_blocks * a.parts;
+        if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");
+        if (tm == 128) (gated ? moe_split_kernel<128, 128, 8, 4, 4, true> : moe_split_kernel<128, 128, 8, 4, 4, false>)<<<dim3((unsigned)groups), 512, 0, st>>>(a);
+        else (gated ? moe_split_kernel<64, 256, 4, 1, 4, true> : moe_split_kernel<64, 256, 4, 1, 4, false>)<<<dim3((unsigned)groups), 256, 0, st>>>(a);
+        return jl_check_launch("moe_split_kernel");
+    }
     a.col_blocks = (a.n_out + (gated ? 31 : 63)) / (gated ? 32 : 64);
     const int64_t groups = (int64_t)a.max_tiles * a.col_blocks;
     if (groups > 0x7fffffff) return jl_fail(JL_E_INVALID, "jl_moe_gemm: too many tiles");

@@ -363,9 +363,17 @@ def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
     return dtype == torch.bfloat16 and n > 0 and (k <= 1024 and tiles <= 512 or k <= 2048 and tiles <= 256)
 
 
+def linear_split(n: int, k: int, o: int) -> bool:
+    """Whether ``linear`` takes n float rows of k values times [o, k] to the bfloat16 matrix instructions in three terms per operand: from 192 tiles of 64 rows by 128 of W on.  us of GPU time, library /
+    own: 2553 rows of 1024 by 1024 57 / 54, by 3072 140 / 100, by 4096 178 / 139, 4096 of 4096 by 4096 948 / 747 (184 TFLOP/s; the library's product on the float instructions 145), 512 of 1024 by
+    4096 39.6 / 36.1, 1021 of 256 by 2048 19.2 / 12.0, at the line (1021 of 1024 by 1536) 31.0 / 29.6; below it 2553 of 1024 by 512 (160 tiles) 26.0 / 29.6, 256 of 1024 by 4096 (128) 21.5 / 27.5:
+    a tile's way through its stages alone takes 27."""
+    return k > 0 and -(-n // 64) * -(-o // 128) >= 192
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:
-    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``) and a few hundred (``linear_mid``), the library's product
-    for more.  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
+    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``), a few hundred (``linear_mid``) and many float ones
+    (``linear_split``), the library's product for the others.  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
     n, k = x.shape
@@ -373,7 +381,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     same = wt == dt
     _need(same or (wt == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
     small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
-    if small or (same and linear_mid(n, k, o, dt)):
+    split = not small and wt == torch.float32 and linear_split(n, k, o)
+    if small or split or (same and linear_mid(n, k, o, dt)):
         size = w.element_size()
         if (w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and
                 (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == wt and bias.shape == (o,) and bias.is_contiguous())) and dt in _LINEAR_TYPES and k > 0 and
@@ -384,6 +393,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
                 out = torch.empty((n, o), dtype=dt if float_out is None else torch.float32, device=x.device)
                 N.check_layers(N.layers().jl_linear_small(x.data_ptr(), _code(dt), n, x.stride(0), w.data_ptr(), _code(wt), k, o, _ptr(bias), out.data_ptr(), o, mode,
                                                          _stream(x.device)), "jl_linear_small")
+                return out
+            if split:
+                x = x.float()
+                out = torch.empty((n, o), dtype=torch.float32, device=x.device)
+                N.check_layers(N.layers().jl_linear_split(x.data_ptr(), n, x.stride(0), w.data_ptr(), k, o, _ptr(bias), out.data_ptr(), o, _stream(x.device)), "jl_linear_split")
                 return out
             if n * x.stride(0) * size < 1 << 32:
                 out = torch.empty((n, o), dtype=dt if float_out is None else torch.float32, device=x.device)
@@ -820,6 +834,8 @@ def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correcti
     tm = int(L.jl_moe_tile_rows(_code(dt), rows, E, W, ff))
     if tm == 128 and L.jl_moe_tile_pairs(rows, E, W, ff, int(gated is not None)):
         tm = 256
+    elif tm == 64 and dt == torch.float32:
+        tm = int(L.jl_moe_float_tiles(rows, E, W, ff))
     max_tiles = rows // tm + E
     from_logits = not in_one and 0 < n <= ROUTER_TOKENS and Er <= ROUTER_OUTPUTS
     blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
@@ -1223,7 +1239,7 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
         out.index_copy_(0, rows, over_latent(q.index_select(0, rows), rest, None if gate is None else gate.index_select(0, rows)))
     keys, base = batch.key_rows(built, window)
     lat = pool.index_select(0, keys)
-    kv = F.linear(lat[:, :R], w_ukv)
+    kv = linear(lat[:, :R], w_ukv) if lat.dtype == torch.float32 else F.linear(lat[:, :R], w_ukv)
     tl = _angle_tables(rot_dims, cos, sin, batch, "latent_attention")
     st = _stream(q.device)
     N.check_layers(N.layers().jl_rotate_heads(_ptr(q), _code(dt), n, q.stride(0), H, D, rd, rot_dims, _ptr(batch.pos), _ptr(cos), _ptr(sin), tl, int(pairing), st), "jl_rotate_heads")
