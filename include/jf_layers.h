@@ -462,8 +462,11 @@ typedef struct {
     int64_t N, x_ld;
     int32_t x_dtype, K, E, experts, top, kind, tile_rows, max_tiles;
     float scale, renorm_eps;
+    float *parts; int32_t slices;
 } jl_moe_router;
 JL_API int jl_moe_router_blocks(int64_t N);
+/* in how many slices of the depth the product is better formed (1: whole): `slices`, with slices * N * E floats of scratch in `parts` when it is more than one */
+JL_API int jl_moe_router_slices(int64_t N, int32_t E, int32_t K);
 JL_API int jl_moe_router_run(const jl_moe_router *a, void *stream);
 
 /* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].

@@ -261,7 +261,7 @@ class ScanArgs(C.Structure):
 class MoeRouter(C.Structure):
     """jl_moe_router (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("x", "w", "bias", "correction", "ids", "weights", "perm", "offsets", "tile_expert", "tile_row0", "counts")] + [("N", _i64), ("x_ld", _i64)] + \
-               [(k, _i32) for k in ("x_dtype", "K", "E", "experts", "top", "kind", "tile_rows", "max_tiles")] + [("scale", _f32), ("renorm_eps", _f32)]
+               [(k, _i32) for k in ("x_dtype", "K", "E", "experts", "top", "kind", "tile_rows", "max_tiles")] + [("scale", _f32), ("renorm_eps", _f32), ("parts", _vp), ("slices", _i32)]
 
 
 class RetentionPieces(C.Structure):
@@ -359,13 +359,14 @@ _LAYER_SIGNATURES = {
     "jl_moe_tile_pairs": (C.c_int, [_i64, _i32, _i32, _i32, _i32]),
     "jl_moe_float_tiles": (C.c_int, [_i64, _i32, _i32, _i32]),
     "jl_moe_router_blocks": (C.c_int, [_i64]),
+    "jl_moe_router_slices": (C.c_int, [_i64, _i32, _i32]),
     "jl_moe_router_run": (C.c_int, [C.POINTER(MoeRouter), _vp]),
     "jl_moe_gemm": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
     "jl_moe_gemm_gated": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _vp, _vp]),
 }
 LAYER_SYMBOLS = tuple(_LAYER_SIGNATURES)
 # which library a symbol lives in (jacobiforcing_amd/_build.py: LAYER_GROUPS); both carry their own jl_version / jl_last_error
-_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_float_tiles", "jl_moe_router_blocks", "jl_moe_router_run", "jl_moe_gemm", "jl_moe_gemm_gated")
+_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_float_tiles", "jl_moe_router_blocks", "jl_moe_router_slices", "jl_moe_router_run", "jl_moe_gemm", "jl_moe_gemm_gated")
 
 
 class _LayerLibs:

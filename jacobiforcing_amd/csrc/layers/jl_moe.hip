@@ -220,7 +220,7 @@ extern "C" int jl_moe_group(const int32_t *ids, int64_t N, int32_t top, int32_t 
 // them (LOGITS), chooses per token from LDS and counts its choices per expert; with one workgroup it groups them too.  With more, a second launch of as many workgroups adds the counts up to where each
 // one's rows go: no workgroup walks all rows.  What bounds them: what one CU takes in, 26 GB/s of x and W (more of them on the way, or the products on the bfloat16 instructions in three terms, change
 // nothing), then the table of counts.  us, product + choice + grouping in launches of their own / in these (from logits): 8192 x 1024 bfloat16 by 16 outputs 57 / 17 (9), 8192 x 2048 float by 32
-// 51 / 32 (13), by 40 56 / 45 (19), 32 x 1024 by 16 24 / 11 in one launch instead of three, 32 x 2048 float by 32 27 / 21, 2246 x 1024 float by 16 28 / 13.
+// 51 / 32 (13), by 40 56 / 45 (19), 32 x 1024 by 16 24 / 11 in one launch instead of three, 32 x 2048 float by 32 27 / 21 (in slices of the depth, jl_moe_router_slices: 13), 2246 x 1024 float by 16 28 / 13.
 constexpr int MR_MAX_E = 64, MR_NW = 8;
 
 // lane e of the first wavefront: where expert e's rows and tiles start; offsets and the list of tiles (the first workgroup's to write)
@@ -312,6 +312,33 @@ __device__ __forceinline__ void moe_route_rows(const float *const (&z)[R], const
         if (turn[r] >= 0) each(r, turn[r], e, sc[r] / (kind == JL_ROUTE_SIGMOID ? 1.0f : kind == JL_ROUTE_SOFTMAX_RENORM ? chosen[r] + renorm_eps : chosen[r]) * scale);
 }
 
+// a slice of the depth of a block's logits: [slices][N][E] in a.parts, for moe_router_kernel to add up
+template <typename TX, int NT, int OT>
+__global__ __launch_bounds__(64 * MR_NW) void moe_router_part_kernel(jl_moe_router a) {
+    constexpr int ROWS = 16 * NT;
+    __shared__ ls_f32x4 part[MR_NW][OT][NT][64];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, k0 = (int)((int64_t)a.K * blockIdx.y / a.slices) & ~31, k1 = blockIdx.y + 1 == (unsigned)a.slices ? a.K : (int)((int64_t)a.K * (blockIdx.y + 1) / a.slices) & ~31;
+    const int64_t n0 = (int64_t)blockIdx.x * ROWS;
+    const int rows = a.N - n0 < ROWS ? (int)(a.N - n0) : ROWS;
+    ls_f32x4 acc[OT][NT];
+    ls_products<TX, float, NT, OT, MR_NW, 1>(acc, (const TX *)a.x + n0 * a.x_ld + k0, a.x_ld, a.w + k0, rows, k1 - k0, 0, a.E, wave, lane, a.K);
+#pragma unroll
+    for (int o = 0; o < OT; ++o)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) part[wave][o][t][lane] = acc[o][t];
+    __syncthreads();
+    float *to = a.parts + ((int64_t)blockIdx.y * a.N + n0) * a.E;
+    for (int e = tid; e < OT * NT * 64; e += 64 * MR_NW) {
+        const int l = e & 63, t = (e >> 6) % NT, ot = (e >> 6) / NT, o = 16 * ot + 4 * (l >> 4), n = 16 * t + (l & 15);
+        ls_f32x4 s = part[0][ot][t][l];
+#pragma unroll
+        for (int i = 1; i < MR_NW; ++i) s += part[i][ot][t][l];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n < rows && o + i < a.E) to[n * a.E + o + i] = s[i];
+    }
+}
+
 template <typename TX, int NT, int OT, bool LOGITS>
 __global__ __launch_bounds__(64 * MR_NW) void moe_router_kernel(jl_moe_router a) {
     constexpr int ROWS = 16 * NT;
@@ -323,8 +350,13 @@ __global__ __launch_bounds__(64 * MR_NW) void moe_router_kernel(jl_moe_router a)
     const int rows = a.N - n0 < ROWS ? (int)(a.N - n0) : ROWS;
     if (tid < MR_MAX_E) count[tid] = 0;
     if constexpr (LOGITS) {
-        const float *from = (const float *)a.x + n0 * a.E;
-        for (int i = tid; i < rows * a.E; i += 64 * MR_NW) z[i / a.E][i % a.E] = from[i];
+        const float *from = (a.slices > 1 ? a.parts : (const float *)a.x) + n0 * a.E;
+        for (int i = tid; i < rows * a.E; i += 64 * MR_NW) {
+            float sum = from[i];
+#pragma unroll 8
+            for (int p = 1; p < a.slices; ++p) sum += from[p * a.N * a.E + i];
+            z[i / a.E][i % a.E] = a.bias ? sum + a.bias[i % a.E] : sum;
+        }
     } else {
         ls_f32x4 acc[OT][NT];
         ls_products<TX, float, NT, OT, MR_NW, 1, true>(acc, (const TX *)a.x + n0 * a.x_ld, a.x_ld, a.w, rows, a.K, 0, a.E, wave, lane);
@@ -413,12 +445,16 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(jl_moe_router a, int ro
 }
 
 extern "C" int jl_moe_router_blocks(int64_t N) { return (int)(N <= 16 ? 1 : (N + 31) / 32 < 0x7fffffff ? (N + 31) / 32 : 0x7fffffff); }
+// The product in four slices of the depth, in front of the choice, where a workgroup would take in half a MB of x and W by itself.  us of product, choice and grouping, one / four slices: 32 x 2048 float
+// by 32 outputs 20.6 / 12.9 (two 15.9, eight 13.1), by 40 27.7 / 17.0, 128 by 32 23.1 / 15.1, 1 by 32 12.7 / 8.7, 48 x 2048 bfloat16 by 32 24.7 / 15.9, 1400 x 1024 float by 20 15.4 / 13.5; below the
+// line it saves less than a launch costs: 32 x 1024 bfloat16 by 16 10.3 / 8.7, 1 token 6.6 / 6.8.
+extern "C" int jl_moe_router_slices(int64_t N, int32_t E, int32_t K) { return jl_moe_router_blocks(N) <= 64 && (int64_t)K * ((E + 15) / 16) >= 2048 ? 4 : 1; }
 extern "C" int jl_moe_router_run(const jl_moe_router *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_moe_router_run: null arguments");
     const jl_moe_router &a = *ap;
     if (a.N <= 0) return JL_OK;
     const int blocks = jl_moe_router_blocks(a.N);
-    const bool logits = !a.w;
+    bool logits = !a.w;
     if (!a.x || !a.ids || !a.weights || !a.perm || !a.offsets || !a.tile_expert || !a.tile_row0 || (blocks > 1 && !a.counts)) return jl_fail(JL_E_INVALID, "jl_moe_router_run: null pointer");
     if (a.E <= 0 || a.E > MR_MAX_E || a.experts <= 0 || a.experts > a.E || a.top <= 0 || a.top > a.E || a.kind < JL_ROUTE_SIGMOID || a.kind > JL_ROUTE_TOP_SOFTMAX)
         return jl_fail(JL_E_INVALID, "jl_moe_router_run: up to %d router outputs, experts and choices among them", MR_MAX_E);
@@ -435,6 +471,14 @@ extern "C" int jl_moe_router_run(const jl_moe_router *ap, void *stream) {
         else JL_DISPATCH(a.x_dtype, moe_router_kernel<T, NT, OT, false><<<dim3((unsigned)blocks), 64 * MR_NW, 0, st>>>(a));        \
     } while (0)
     const int ot = (a.E + 15) / 16;
+    if (a.slices > 1) {
+        if (logits || !a.parts) return jl_fail(JL_E_INVALID, "jl_moe_router_run: slices of a product, and room for them");
+#define MR_PART(NT, OT) JL_DISPATCH(a.x_dtype, moe_router_part_kernel<T, NT, OT><<<dim3((unsigned)blocks, (unsigned)a.slices), 64 * MR_NW, 0, st>>>(a))
+        if (a.N <= 16) { if (ot == 1) MR_PART(1, 1); else if (ot == 2) MR_PART(1, 2); else if (ot == 3) MR_PART(1, 3); else MR_PART(1, 4); }
+        else { if (ot == 1) MR_PART(2, 1); else if (ot == 2) MR_PART(2, 2); else if (ot == 3) MR_PART(2, 3); else MR_PART(2, 4); }
+#undef MR_PART
+        logits = true;
+    }
     if (a.N <= 16) { if (ot == 1) MR_CASE(1, 1); else if (ot == 2) MR_CASE(1, 2); else if (ot == 3) MR_CASE(1, 3); else MR_CASE(1, 4); }
     else { if (ot == 1) MR_CASE(2, 1); else if (ot == 2) MR_CASE(2, 2); else if (ot == 3) MR_CASE(2, 3); else MR_CASE(2, 4); }
 #undef MR_CASE

@@ -26,9 +26,9 @@ __device__ __forceinline__ uint4 ls_unit(const bf16_t *p, const float *) {      
 }
 
 // acc[o][t]: rows o0 + 16 o .. of W (first operand) by rows 16 t .. of x, summed over this wavefront's share of the depth (NW wavefronts share it); rows that do not exist repeat the last
-// AHEAD steps' units are on their way at once; TURNS: and as many more while those are multiplied
+// (w_ld: how far W's rows lie apart, if not K).  AHEAD steps' units are on their way at once; TURNS: and as many more while those are multiplied
 template <typename TX, typename T, int NT, int OT, int NW, int AHEAD = LS_AHEAD, bool TURNS = false>
-__device__ __forceinline__ void ls_products(ls_f32x4 (&acc)[OT][NT], const TX *__restrict__ x, int64_t x_ld, const T *__restrict__ w, int N, int K, int o0, int O, int wave, int lane) {
+__device__ __forceinline__ void ls_products(ls_f32x4 (&acc)[OT][NT], const TX *__restrict__ x, int64_t x_ld, const T *__restrict__ w, int N, int K, int o0, int O, int wave, int lane, int w_ld = 0) {
     constexpr int UNIT = 16 / sizeof(T), LINE = 8 * UNIT;           // elements of a unit, of the 128 bytes that a step takes from every row
     const int r16 = lane & 15, g = lane >> 4;
     const int k_lane = UNIT * g;
@@ -37,7 +37,7 @@ __device__ __forceinline__ void ls_products(ls_f32x4 (&acc)[OT][NT], const TX *_
 #pragma unroll
     for (int o = 0; o < OT; ++o) {
         const int r = o0 + 16 * o + r16;
-        wp[o] = w + (int64_t)(r < O ? r : O - 1) * K + k_lane;      // rows and columns that do not exist repeat the last one and are not stored
+        wp[o] = w + (int64_t)(r < O ? r : O - 1) * (w_ld ? w_ld : K) + k_lane;      // rows and columns that do not exist repeat the last one and are not stored
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[o][t] = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
     }

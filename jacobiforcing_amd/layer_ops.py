@@ -839,7 +839,8 @@ def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correcti
     max_tiles = rows // tm + E
     from_logits = not in_one and 0 < n <= ROUTER_TOKENS and Er <= ROUTER_OUTPUTS
     blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
-    lists = torch.empty((rows + E + 2 + 2 * max_tiles + blocks * E,), dtype=torch.int32, device=dev)       # the grouping's lists, one behind the other
+    slices = int(L.jl_moe_router_slices(n, Er, router[0].shape[1])) if in_one else 1
+    lists = torch.empty((rows + E + 2 + 2 * max_tiles + blocks * E + (slices * n * Er if slices > 1 else 0),), dtype=torch.int32, device=dev)       # the grouping's lists, one behind the other, the product's slices
     perm = lists.data_ptr()
     offsets = perm + 4 * rows
     tile_e = offsets + 4 * (E + 2)
@@ -849,7 +850,7 @@ def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correcti
     if in_one or from_logits:
         a = N.MoeRouter(x=x.data_ptr(), w=_ptr(rw), bias=_ptr(rb), correction=_ptr(correction), ids=ids.data_ptr(), weights=wts.data_ptr(), perm=perm, offsets=offsets, tile_expert=tile_e,
                         tile_row0=tile_r, counts=tile_r + 4 * max_tiles, N=n, x_ld=x.stride(0), x_dtype=_code(x.dtype), K=x.shape[1], E=Er, experts=E, top=top, kind=_ROUTES[route],
-                        tile_rows=tm, max_tiles=max_tiles, scale=float(scale), renorm_eps=float(renorm_eps))
+                        tile_rows=tm, max_tiles=max_tiles, scale=float(scale), renorm_eps=float(renorm_eps), parts=tile_r + 4 * (max_tiles + blocks * E), slices=slices)
         N.check_layers(L.jl_moe_router_run(C.byref(a), st), "jl_moe_router_run")
     else:
         N.check_layers(L.jl_moe_route(_ptr(router_logits), _ptr(correction), n, Er, top, float(scale), _ptr(ids), _ptr(wts),

@@ -45,6 +45,16 @@ def test_the_same_as_from_logits(monkeypatch, x_dtype, N, K, E, identity, top, b
     assert run(monkeypatch, N, K, E, identity, top, x_dtype, bias, route, pad), "the launches did not run"
 
 
+@pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K,E,identity,top,bias,route,pad", [(1, 2048, 16, 0, 4, True, "sigmoid", 0), (16, 516, 60, 4, 3, False, "top_softmax", 4), (17, 2052, 17, 0, 2, True, "softmax_renorm", 12),
+                                                               (65, 1028, 30, 9, 4, True, "sigmoid", 12), (2048, 1032, 20, 0, 4, False, "softmax_renorm", 0), (2049, 1024, 32, 0, 4, False, "sigmoid", 0)])
+def test_products_in_slices_of_the_depth(monkeypatch, x_dtype, N, K, E, identity, top, bias, route, pad):
+    """The smallest products that are sliced, depths whose slices end beside whole lines, one workgroup and the most (one more: whole)."""
+    from jacobiforcing_amd import _native as N_
+    assert N_.layers().jl_moe_router_slices(N, E + identity, K) == (4 if N <= 2048 else 1)
+    assert run(monkeypatch, N, K, E, identity, top, x_dtype, bias, route, pad), "the launches did not run"
+
+
 @pytest.mark.parametrize("N,K,E", [(16385, 16, 4), (20, 30, 8), (50, 64, 65)])
 def test_what_the_launches_do_not_take(monkeypatch, N, K, E):
     """More tokens, depths beside 16-byte borders, more outputs: the product, the choice and the grouping one after the other."""
