@@ -26,6 +26,31 @@ LAYER_GROUPS = {
 LAYERS_HEADERS = [CSRC / "layers" / "jl_common.h", CSRC / "layers" / "jl_attn.h", CSRC / "layers" / "jl_small.h", ROOT / "include" / "jf_layers.h"]
 
 
+# the wrappers' host side (a CPython module on torch's C++ interface), beside the libraries that it calls
+HOST_SOURCE, HOST_LIB = CSRC / "layers" / "jl_host.cpp", LIB_DIR / "_jl_host.so"
+
+
+def build_host(force: bool = False) -> Path:
+    """``lib/_jl_host.so`` with the compiler of the host; nothing of it runs on the GPU."""
+    if not force and not stale(HOST_LIB, [HOST_SOURCE, ROOT / "include" / "jf_layers.h"]):
+        return HOST_LIB
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    LIB_DIR.mkdir(parents=True, exist_ok=True)
+    include = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"], str(ROOT / "include")]
+    with tempfile.TemporaryDirectory(dir=LIB_DIR) as tmp:
+        out = f"{tmp}/_jl_host.so"
+        done = subprocess.run([shutil.which("g++") or hipcc(), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-deprecated-declarations", *[f"-I{i}" for i in include], str(HOST_SOURCE),
+                               f"-L{cpp_extension.library_paths()[0]}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-o", out], stderr=subprocess.PIPE, text=True)
+        if done.returncode:
+            raise RuntimeError(f"the compiler failed on jl_host.cpp:\n{done.stderr[-4000:]}")
+        os.replace(out, HOST_LIB)
+    return HOST_LIB
+
+
 def layer_lib(group: str) -> Path:
     return LIB_DIR / f"libjf_{group}.so"
 

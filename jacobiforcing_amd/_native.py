@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 136                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 137                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -428,6 +428,31 @@ def layers():
     if "layers" not in _LAYERS._libs:               # the attention / norm library is what every ragged family needs: load (or build) it now
         _LAYERS._load("layers")
     return _LAYERS
+
+
+def host(*rules):
+    """The host's side of the small launches (csrc/layers/jl_host.cpp), bound to both kernel libraries; built when there is none.  ``rules``: the numbers that ``linear``'s rules go by."""
+    import importlib.machinery
+    import importlib.util
+    from . import _build
+    if not _build.HOST_LIB.exists():
+        try:
+            _build.build_host()
+        except Exception as e:
+            raise NativeLibraryError(f"cannot build {_build.HOST_LIB}: {e}") from e
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_jl_host", str(_build.HOST_LIB))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_jl_host", loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        raise NativeLibraryError(f"cannot load {_build.HOST_LIB}: {e}") from e
+    if module.version != JL_VERSION:
+        raise NativeLibraryError(f"{_build.HOST_LIB} has version {module.version}, this package calls version {JL_VERSION}: build it again (python -c 'import __graft_entry__ as g; g.build()')")
+    L, address = layers(), lambda fn: C.cast(fn, C.c_void_p).value
+    symbols = {name: address(getattr(L, name)) for name in module.symbols()}
+    symbols["jl_last_error"], symbols["jl_last_error of the recurrences"] = (address(L._library(name).jl_last_error) for name in ("jl_linear_small", "jl_linear_scan"))
+    module.bind(symbols, *rules)
+    return module
 
 
 def check_layers(rc: int, what: str = ""):

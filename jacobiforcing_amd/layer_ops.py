@@ -74,6 +74,16 @@ def _dev(t: torch.Tensor) -> None:
         raise N.NativeLibraryError("the layer kernels run on the GPU only (no CPU fallback)")
 
 
+_H = None                                            # the wrappers' host side in native code: what it does not take comes back as NotImplemented, and the wrapper goes on
+
+
+def _host():
+    global _H
+    if _H is None:
+        _H = N.host(LINEAR_SMALL_ROWS, LINEAR_ONE_TILE, LINEAR_X_BYTES)
+    return _H
+
+
 _UPLOADS: dict = {}                                  # device index -> the stream its tables are copied on, and a block of its pool
 _GONE: dict = {}                                     # a stream's id -> _Gone
 GONE_AT_ONCE = 64                                    # tables (of some KB each; built keys' rows of a long step up to a MB) that wait for an event together
@@ -376,6 +386,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     (``linear_split``), the library's product for the others.  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
+    r = (_H or _host()).linear(x, w, bias, float_out)
+    if r is not NotImplemented:
+        return r
     n, k = x.shape
     o, dt, wt = w.shape[0], x.dtype, w.dtype
     same = wt == dt
@@ -421,6 +434,9 @@ def embed_scale(embed: torch.Tensor, ids: torch.Tensor, scale: float, want_copy:
     """Rows ``ids`` of ``embed`` times ``scale`` as float [N, W] (written into ``out`` when given), and a second copy with ``want_copy``
     (float, or rounded to bfloat16 with ``copy_dtype``)."""
     _dev(embed)
+    r = (_H or _host()).embed_scale(embed, ids, scale, want_copy, out, copy_dtype)
+    if r is not NotImplemented:
+        return r
     _need(embed.dim() == 2 and embed.is_contiguous() and ids.dtype == torch.int64 and ids.is_contiguous(), "embed_scale: embed [V, W], ids int64 [N]")
     n, W = ids.numel(), embed.shape[1]
     if out is not None:
@@ -439,6 +455,9 @@ def add_rmsnorm(x: torch.Tensor, y: Optional[torch.Tensor], x0: Optional[torch.T
     """x (float [N, W], in place) += y summed over its middle axis ([N, W] or [N, S, W], float or bf16) + x0; returns
     rms_norm(x) * w in ``out_dtype`` (None: the update only)."""
     _dev(x)
+    r = (_H or _host()).add_rmsnorm(x, y, x0, w, eps, out_dtype)
+    if r is not NotImplemented:
+        return r
     n, W = x.shape
     _need(x.dtype == torch.float32 and x.is_contiguous(), "add_rmsnorm: x must be contiguous float32 [N, W]")
     cnt = 0
@@ -463,6 +482,10 @@ def qk_norm_append(proj: torch.Tensor, cols: Tuple[int, int, int], H: int, G: in
     """RMS norm of q over all its heads together (and of k over its), with ``rot_dims`` the rotation of both by position behind it (needs
     ``batch`` and its angle tables), keys / values appended to the pools.  Returns q [N, H*D]."""
     _dev(proj)
+    r = (_H or _host()).qk_norm_append(proj, *cols, H, G, D, Dv, wq, wk, eps, k_cache, v_cache, kv_slot, rot_dims, pairing, batch.N if batch is not None else 0,
+                                       batch.max_pos if batch is not None else 0, batch.pos if batch is not None else None, cos, sin)
+    if r is not NotImplemented:
+        return r
     n, ld = proj.shape
     dt = proj.dtype
     _need(proj.is_contiguous() and kv_slot.dtype == torch.int64 and kv_slot.numel() == n, "qk_norm_append: proj [N, ld], one pool token per row")
@@ -507,6 +530,20 @@ def attn_tile_rows(dtype: torch.dtype, H: int, G: int, D: int, Dv: int, k_ld: in
     return tq
 
 
+def _attn_args(q, k_cache, v_cache, out, batch: RaggedBatch, tiles, gate, sink, rel, lut, talk, scratch, q_pack, scale, softcap, out_scale, H, G, Gv, D, Dv, window, keep_first, chunk, tq, splits,
+               out_dtype, gate_heads) -> N.AttnArgs:
+    """The arguments of an attention launch whose operands the caller has checked."""
+    a, numbers = N.AttnArgs(), (batch.page_size, H, G, Gv, D, Dv, int(window), int(keep_first), int(chunk), tq, splits, out_dtype, int(gate_heads))
+    if (_H or _host()).attention_args(C.addressof(a), q, k_cache, v_cache, out, batch.tables, tiles, gate, sink, rel, lut, talk, scratch, q_pack, float(scale), float(softcap), float(out_scale),
+                                      *numbers) is not NotImplemented:
+        return a
+    return N.AttnArgs(q=_ptr(q), k_cache=_ptr(k_cache), v_cache=_ptr(v_cache), out=_ptr(out), block_tables=_ptr(batch.tables), tiles=_ptr(tiles), gate=_ptr(gate),
+                      gate_ld=gate.stride(0) if gate is not None else 0, sink=_ptr(sink), rel=_ptr(rel), lut=_ptr(lut), talk=_ptr(talk), scratch=_ptr(scratch), q_pack=_ptr(q_pack),
+                      lut_len=(lut.numel() if lut is not None else rel.shape[0]) if rel is not None else 0, scale=float(scale), softcap=float(softcap), out_scale=float(out_scale),
+                      bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0], n_rows=q.shape[0], k_ld=k_cache.stride(0), v_ld=v_cache.stride(0), out_ld=out.stride(0), dtype=_code(q.dtype),
+                      **dict(zip(("page_size", "H", "G", "Gv", "D", "Dv", "window", "keep_first", "chunk", "TQ", "splits", "out_dtype", "gate_heads"), numbers)))
+
+
 def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: torch.Tensor, batch: RaggedBatch,
                 H: int, G: int, D: int, Dv: int, scale: float, window: int, keep_first: int, rel: Optional[torch.Tensor],
                 lut: Optional[torch.Tensor], talk: Optional[torch.Tensor], value_heads: int = 0, float_out: bool = False,
@@ -548,12 +585,8 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
         per_tile = int(N.layers().jl_attn_talk_scratch_floats(1, tq, H, G, Dv, splits))
         pass_tiles = min(tiles.shape[0], max(1, TALK_SCRATCH_FLOATS // per_tile))
         scratch = torch.empty((per_tile * pass_tiles,), dtype=torch.float32, device=q.device)
-        a = N.AttnArgs(q=q.data_ptr(), gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0, k_cache=k_cache.data_ptr(),
-                       v_cache=v_cache.data_ptr(), out=out.data_ptr(), block_tables=batch.tables.data_ptr(), tiles=tiles.data_ptr(), rel=rel.data_ptr() if rel is not None else None,
-                       lut=lut.data_ptr() if lut is not None else None, talk=talk.data_ptr(), bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0],
-                       lut_len=(lut.numel() if lut is not None else rel.shape[0]) if rel is not None else 0, page_size=batch.page_size, H=H, G=G, D=D, Dv=Dv, window=int(window),
-                       keep_first=max(0, int(keep_first)), TQ=tq, dtype=_code(dt), scale=float(scale), splits=splits, n_rows=n, scratch=scratch.data_ptr(), k_ld=k_ld, v_ld=v_ld, Gv=Gv,
-                       out_dtype=N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME, gate_heads=int(gate_per_head), out_scale=float(out_scale), out_ld=out.stride(0))
+        a = _attn_args(q, k_cache, v_cache, out, batch, tiles, gate, None, rel, lut, talk, scratch, None, scale, 0.0, out_scale, H, G, Gv, D, Dv, window, max(0, int(keep_first)), 0, tq, splits,
+                       N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME, gate_per_head)
         N.check_layers(N.layers().jl_attn_talk(C.byref(a), int(wide), pass_tiles, _stream(q.device)), "jl_attn_talk")
         return out
     tq = attn_tile_rows(dt, H, G, D, Dv, k_ld, v_ld)
@@ -566,17 +599,8 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
         if splits > 1:
             scratch = torch.empty((int(N.layers().jl_attn_scratch_floats(tiles.shape[0], n, H, Dv, splits)),), dtype=torch.float32, device=q.device)
     q_pack = torch.empty((tiles.shape[0] * 32 * H * D,), dtype=dt, device=q.device) if tq == 32 else None
-    a = N.AttnArgs(q=q.data_ptr(), gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0,
-                   k_cache=k_cache.data_ptr(), v_cache=v_cache.data_ptr(), out=out.data_ptr(), block_tables=batch.tables.data_ptr(),
-                   tiles=tiles.data_ptr(), rel=rel.data_ptr() if rel is not None else None, lut=lut.data_ptr() if lut is not None else None,
-                   talk=talk.data_ptr() if talk is not None else None, bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0],
-                   lut_len=(lut.numel() if lut is not None else rel.shape[0]) if rel is not None else 0, page_size=batch.page_size, H=H, G=G, D=D, Dv=Dv, window=int(window),
-                   keep_first=int(keep_first), TQ=tq, dtype=_code(dt), scale=float(scale), splits=splits, n_rows=n,
-                   scratch=scratch.data_ptr() if scratch is not None else None,
-                   q_pack=q_pack.data_ptr() if q_pack is not None else None, k_ld=k_ld, v_ld=v_ld, Gv=Gv,
-                   out_dtype=N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME,
-                   sink=sink.data_ptr() if sink is not None else None, gate_heads=int(gate_per_head), chunk=int(chunk), softcap=float(softcap),
-                   out_scale=float(out_scale), out_ld=out.stride(0))
+    a = _attn_args(q, k_cache, v_cache, out, batch, tiles, gate, sink, rel, lut, talk, scratch, q_pack, scale, softcap, out_scale, H, G, Gv, D, Dv, window, keep_first, chunk, tq, splits,
+                   N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME, gate_per_head)
     N.check_layers(N.layers().jl_attn_window(C.byref(a), _stream(q.device)), "jl_attn_window")
     return out
 
@@ -690,13 +714,8 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
         if splits > 1:
             scratch = torch.empty((int(N.layers().jl_attn_sweep_scratch_floats(tiles.shape[0], H, G, Dv, splits)),), dtype=torch.float32, device=q.device)
     tiles = batch.tiles(tq) if tiles is None else tiles
-    a = N.AttnArgs(q=q.data_ptr(), k_cache=k_cache.data_ptr(), v_cache=v_cache.data_ptr(), out=out.data_ptr(), block_tables=batch.tables.data_ptr(),
-                   tiles=tiles.data_ptr(), bt_stride=batch.tables.shape[1], n_tiles=tiles.shape[0], page_size=batch.page_size, H=H, G=G, D=D, Dv=Dv,
-                   window=int(window), TQ=tq, dtype=_code(q.dtype), scale=float(scale), n_rows=n, k_ld=k_cache.stride(0), v_ld=v_cache.stride(0), Gv=Gv,
-                   splits=splits, scratch=scratch.data_ptr() if scratch is not None else None,
-                   out_dtype=N.JL_OUT_F32 if float_out else N.JL_OUT_SAME, sink=sink.data_ptr() if sink is not None else None,
-                   gate=gate.data_ptr() if gate is not None else None, gate_ld=gate.stride(0) if gate is not None else 0, gate_heads=int(gate_per_head),
-                   chunk=int(chunk), softcap=float(softcap), out_scale=float(out_scale), out_ld=out.stride(0))
+    a = _attn_args(q, k_cache, v_cache, out, batch, tiles, gate, sink, None, None, None, scratch, None, scale, softcap, out_scale, H, G, Gv, D, Dv, window, 0, chunk, tq, splits,
+                   N.JL_OUT_F32 if float_out else N.JL_OUT_SAME, gate_per_head)
     if narrow:
         N.check_layers(N.layers().jl_attn_narrow(C.byref(a), _stream(q.device)), "jl_attn_narrow")
         return out
@@ -828,18 +847,22 @@ def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correcti
     if correction is not None:
         _need(correction.dtype == torch.float32 and correction.numel() == Er, "moe_experts: correction float, one per router output")
     L, st = N.layers(), _stream(dev)
-    ids = torch.empty((n, top), dtype=torch.int32, device=dev)
-    wts = torch.empty((n, top), dtype=torch.float32, device=dev)
     rows = n * top
     tm = int(L.jl_moe_tile_rows(_code(dt), rows, E, W, ff))
     if tm == 128 and L.jl_moe_tile_pairs(rows, E, W, ff, int(gated is not None)):
         tm = 256
     elif tm == 64 and dt == torch.float32:
         tm = int(L.jl_moe_float_tiles(rows, E, W, ff))
-    max_tiles = rows // tm + E
     from_logits = not in_one and 0 < n <= ROUTER_TOKENS and Er <= ROUTER_OUTPUTS
-    blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
     slices = int(L.jl_moe_router_slices(n, Er, router[0].shape[1])) if in_one else 1
+    if (in_one or from_logits) and not os.environ.get("JL_MOE_UNFUSED_ACT"):
+        r = (_H or _host()).moe_experts(h, *(router if in_one else (router_logits, None, None)), correction, top, scale, w_up, w_down, _ROUTES[route], renorm_eps, gated, identity, tm, slices)
+        if r is not NotImplemented:
+            return r
+    ids = torch.empty((n, top), dtype=torch.int32, device=dev)
+    wts = torch.empty((n, top), dtype=torch.float32, device=dev)
+    max_tiles = rows // tm + E
+    blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
     lists = torch.empty((rows + E + 2 + 2 * max_tiles + blocks * E + (slices * n * Er if slices > 1 else 0),), dtype=torch.int32, device=dev)       # the grouping's lists, one behind the other, the product's slices
     perm = lists.data_ptr()
     offsets = perm + 4 * rows
@@ -883,6 +906,9 @@ def gated_act(z: torch.Tensor, g_col: int, u_col: int, F_: int, kind: int, limit
     shift).  ACT_SILU: g sigmoid(g) * u.  ACT_GELU_ERF: 0.5 g (1 + erf(g / sqrt 2)) * u.  ``u_col`` < 0: no linear branch (a plain
     activation of the F_ columns at g_col).  ``row_gate`` [N] or [N, 1] view (row stride free): the row is further multiplied by sigmoid(row_gate).  Returns [N, F_]."""
     _dev(z)
+    r = (_H or _host()).gated_act(z, g_col, u_col, F_, kind, limit, alpha, shift, row_gate)
+    if r is not NotImplemented:
+        return r
     u_col = -1 if u_col < 0 else u_col
     _need(z.dim() == 2 and z.stride(1) == 1 and 0 <= g_col and g_col + F_ <= z.shape[1] and u_col + F_ <= z.shape[1], "gated_act: z [N, ld] with both column ranges inside")
     n = z.shape[0]
@@ -951,6 +977,9 @@ def output_norm(x: torch.Tensor, addends: Sequence[Tuple[torch.Tensor, Optional[
     ``choices`` = (ids, weights, E): the first addend is what ``moe_experts`` returned with identity experts; choices >= E stand for
     weight * x (x before the update)."""
     _dev(x)
+    r = (_H or _host()).output_norm(x, addends, w, eps, kind, mult, w_next, out_dtype, choices)
+    if r is not NotImplemented:
+        return r
     n, W = x.shape
     _need(x.dtype == torch.float32 and x.is_contiguous() and len(addends) <= 3, "output_norm: x contiguous float32 [N, W], at most 3 addends")
     arr = _addends(addends, n, W, "output_norm")
@@ -982,6 +1011,9 @@ def sandwich_norm(x_in: torch.Tensor, y: Optional[torch.Tensor], w_post: Optiona
     returns rms_norm(x_in) * w_next — or x_in itself with ``plain`` — in ``out_dtype`` or in ``out`` (a column range of wider rows); None with
     neither."""
     _dev(x_in)
+    r = (_H or _host()).sandwich_norm(x_in, y, w_post, eps, w_next, out_dtype, add_row, out, plain)
+    if r is not NotImplemented:
+        return r
     n, W = x_in.shape
     _need(x_in.dtype == torch.float32 and x_in.is_contiguous(), "sandwich_norm: x contiguous float32 [N, W]")
     _need(y is None or (tuple(y.shape) == (n, W) and y.is_contiguous() and w_post is not None), "sandwich_norm: y [N, W] with its norm weight")
@@ -1004,6 +1036,9 @@ def gated_norm(raw: torch.Tensor, gate: torch.Tensor, w: torch.Tensor, eps: floa
     raw * act(gate) (``gate_first``), or of raw with act(gate) on the result; times w (float [C]) and ``scale``.  [N, C] of gate's dtype, in
     ``out`` (a column range of wider rows) when given."""
     _dev(raw)
+    r = (_H or _host()).gated_norm(raw, gate, w, eps, act, gate_first, parts, scale, out)
+    if r is not NotImplemented:
+        return r
     n, C_ = raw.shape
     _need(raw.dtype == torch.float32 and raw.is_contiguous() and tuple(gate.shape) == (n, C_) and gate.stride(1) == 1, "gated_norm: raw float [N, C], gate [N, C]")
     _need(w.dtype == torch.float32 and w.numel() == C_ and w.is_contiguous() and parts >= 1 and C_ % parts == 0, "gated_norm: w float [C], parts that divide C")
@@ -1099,6 +1134,9 @@ def latent_prep(proj: torch.Tensor, q_col: int, Rq: int, kv_col: int, R: int, rd
     """Normalised query latent [N, Rq] (None with Rq = 0: a model without one); the pool row of every token becomes [normalised key/value
     latent | rotated shared key].  ``pool`` None: the query latent alone (a layer that attends over another layer's pool)."""
     _dev(proj)
+    r = (_H or _host()).latent_prep(proj, q_col, Rq, kv_col, R, rd, rot_dims, wq, wkv, eps, batch.N, batch.max_pos, batch.pos, batch.kv_slot, cos, sin, pool, pairing)
+    if r is not NotImplemented:
+        return r
     n, ld = proj.shape
     dt = proj.dtype
     _need(proj.is_contiguous() and n == batch.N and (Rq == 0 or (wq is not None and wq.numel() == Rq and wq.dtype == dt)) and
@@ -1121,6 +1159,9 @@ def latent_q_pack(qa: torch.Tensor, q: torch.Tensor, H: int, D: int, R: int, rd:
     """qa [H, N, R] (queries times the key up-projection), q [N, H*(D + rd)] (row stride free: a column range of a wider product) ->
     [N, H*(R + rd)] with the rotary part rotated."""
     _dev(q)
+    r = (_H or _host()).latent_q_pack(qa, q, H, D, R, rd, rot_dims, batch.N, batch.max_pos, batch.pos, cos, sin, pairing)
+    if r is not NotImplemented:
+        return r
     n = q.shape[0]
     _need(q.stride(1) == 1 and qa.is_contiguous() and tuple(qa.shape) == (H, n, R) and q.shape[1] == H * (D + rd) and qa.dtype == q.dtype and n == batch.N,
           "latent_q_pack: qa [H, N, R], q [N, H*(D + rd)]")
@@ -1258,6 +1299,9 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
 def heads_gate(ov: torch.Tensor, gate: Optional[torch.Tensor]) -> torch.Tensor:
     """ov [H, N, Dv] -> [N, H*Dv], times sigmoid(gate) (a [N, H*Dv] view, row stride free)."""
     _dev(ov)
+    r = (_H or _host()).heads_gate(ov, gate)
+    if r is not NotImplemented:
+        return r
     H, n, Dv = ov.shape
     _need(ov.is_contiguous(), "heads_gate: ov [H, N, Dv] contiguous")
     if gate is not None:
@@ -1289,6 +1333,10 @@ def depth_mix_norm(x_in: torch.Tensor, addends: Sequence[Tuple[torch.Tensor, Opt
     ``shift`` = (mu float [W], batch, tail float [slots, 1, W]): for a step in which every request brings ONE row, ``token_shift`` of the
     unrounded norm in the same launch; its result (``out_dtype``) is appended to what is returned."""
     _dev(x_in)
+    if shift is None or (x_in.dim() == 2 and shift[1].N == shift[1].B == x_in.shape[0] and max(shift[1].counts) == 1):
+        r = (_H or _host()).depth_mix_norm(x_in, addends, mult, streams, depth, mix, x_out, w, eps, out_dtype, want_float, None if shift is None else (shift[0], shift[2], shift[1].seq, shift[1].max_slot))
+        if r is not NotImplemented:
+            return r
     n, W = x_in.shape
     _need(x_in.dtype == torch.float32 and x_in.is_contiguous() and len(addends) <= 3, "depth_mix_norm: x_in contiguous float32 [N, W], at most 3 addends")
     arr = _addends(addends, n, W, "depth_mix_norm")
@@ -1327,6 +1375,9 @@ def token_shift(h: torch.Tensor, mu: torch.Tensor, batch: RaggedBatch, tail: tor
     """h + (h of the previous token - h) * mu: h float [N, W], mu float [W]; ``tail`` float [slots, 1, W] carries every request's last h
     from step to step (updated here; never read by a request that starts at position 0)."""
     _dev(h)
+    r = (_H or _host()).token_shift(h, mu, batch.N, batch.max_slot, batch.row_req, batch.seq, tail, out_dtype)
+    if r is not NotImplemented:
+        return r
     n, W = h.shape
     _need(h.dtype == torch.float32 and h.is_contiguous() and n == batch.N and mu.dtype == torch.float32 and mu.numel() == W and mu.is_contiguous(),
           "token_shift: h float [N, W] of the batch, mu float [W]")
@@ -1362,6 +1413,12 @@ def short_conv(x: torch.Tensor, col: int, C_: int, w: torch.Tensor, batch: Ragge
     """act(bias + causal depthwise convolution over time, per request) of the columns col .. col + C_ of x [N, ld], with w [C_, taps]; [N, C_]
     of ``out_dtype`` (float, or x's).  ``tail`` float [slots, taps - 1, C_] carries every request's last inputs from step to step (updated here)."""
     _dev(x)
+    longest = batch._tiles.get("continued")
+    if longest is None:                                  # the longest portion of a request that has a tail
+        longest = batch._tiles["continued"] = max([c for c, s in zip(batch.counts, batch.starts) if s > 0], default=1)
+    r = (_H or _host()).short_conv(x, col, C_, w, batch.N, batch.B, batch.max_slot, longest, batch.row_req, batch.seq, tail, act, bias, out_dtype)
+    if r is not NotImplemented:
+        return r
     n, ld = x.shape
     taps = w.shape[1]
     _need(x.is_contiguous() and n == batch.N and w.is_contiguous() and w.shape[0] == C_ and w.dtype == x.dtype and 0 <= col and col + C_ <= ld and 1 <= taps <= 8,
@@ -1373,7 +1430,7 @@ def short_conv(x: torch.Tensor, col: int, C_: int, w: torch.Tensor, batch: Ragge
     _need(out_dtype in (torch.float32, x.dtype), "short_conv: the output is float or of x's dtype")
     out = torch.empty((n, C_), dtype=out_dtype, device=x.device)
     N.check_layers(N.layers().jl_short_conv(_ptr(x), _code(x.dtype), ld, col, _ptr(w), _ptr(bias), _ptr(batch.row_req), _ptr(batch.seq), batch.B,
-                                           max([c for c, s in zip(batch.counts, batch.starts) if s > 0], default=1), _ptr(tail), n, C_, taps, int(act), _ptr(out), _code(out_dtype), _stream(x.device)), "jl_short_conv")
+                                           longest, _ptr(tail), n, C_, taps, int(act), _ptr(out), _code(out_dtype), _stream(x.device)), "jl_short_conv")
     return out
 
 
@@ -1470,6 +1527,10 @@ def linear_scan(src: torch.Tensor, cols: Tuple[int, int, int], batch: RaggedBatc
     stride free, src's dtype), a_log / dt_bias float [H].  skip float [H] or None.  state [slots, H, D, Dv] float, updated in place.  Returns
     float [N, H*Dv]."""
     _dev(src)
+    if max(batch.counts) < SCAN_PIECES_FROM:
+        r = (_H or _host()).linear_scan(src, *cols, batch.N, batch.B, batch.max_slot, batch.seq, H, G, D, Dv, state, act, decay, dt, a_log, dt_bias, skip)
+        if r is not NotImplemented:
+            return r
     n, ld = src.shape
     _need(src.stride(1) == 1 and n == batch.N and H % G == 0 and max(cols[0], cols[1]) + G * D <= ld and cols[2] + H * Dv <= ld, "linear_scan: columns of the batch's rows")
     _need(state.dtype == torch.float32 and state.is_contiguous() and tuple(state.shape[1:]) == (H, D, Dv) and batch.max_slot < state.shape[0],

@@ -1,0 +1,133 @@
+"""The wrappers' native host side: what it takes gives what the wrappers' own way gives, bit for bit, and what it does not take it leaves alone."""
+import pytest
+import torch
+
+
+@pytest.fixture
+def both(monkeypatch):
+    """run(f): f() with the native calls and without them."""
+    from jacobiforcing_amd import layer_ops as LO
+
+    class Nothing:
+        def __getattr__(self, name):
+            return lambda *a: NotImplemented
+
+    def run(f):
+        got = f()
+        with monkeypatch.context() as m:
+            m.setattr(LO, "_H", Nothing())
+            return got, f()
+    return run
+
+
+def test_the_rules_of_linear():
+    """The product that the native call takes is the one that the wrapper's rules name, at their lines and around them."""
+    from jacobiforcing_amd import layer_ops as LO
+    H = LO._host()
+    for n in (1, 2, 16, 17, 63, 64, 65, 127, 191, 193, 512, 1021, 2553, 9000):
+        for k in (4, 64, 512, 1020, 1024, 1028, 2048, 2052, 4096):
+            for o in (1, 16, 96, 1024, 4096, 4097, 8192, 16384, 16385, 32000):
+                for size in (2, 4):
+                    small = n <= LO.LINEAR_SMALL_ROWS and LO.linear_small(n, k, o, size)
+                    want = 1 if small else (2 if LO.linear_split(n, k, o) else 0) if size == 4 else 3 if LO.linear_mid(n, k, o, torch.bfloat16) else 0
+                    assert H.linear_rule(n, k, o, size) == want, (n, k, o, size)
+
+
+def test_what_it_does_not_take():
+    """Host tensors, other numbers of arguments, other kinds of values: handed back, nothing raised."""
+    from jacobiforcing_amd import layer_ops as LO
+    H, x = LO._host(), torch.randn(4, 64)
+    assert H.linear(x, x, None, None) is NotImplemented and H.linear(x, x) is NotImplemented and H.linear(None, 1, "x", 2.0) is NotImplemented
+    assert H.add_rmsnorm(x, None, None, None, "eps", None) is NotImplemented and H.sandwich_norm(x, None, None, 1e-5, None, torch.float16, None, None, False) is NotImplemented
+    assert H.moe_experts(*[None] * 15) is NotImplemented and H.attention_args(*[7] * 30) is NotImplemented and H.linear_scan(*[x] * 19) is NotImplemented
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 5, 130])
+def test_the_same_as_the_wrappers(both, dtype, n):
+    from jacobiforcing_amd import _native as N, layer_ops as LO
+    dev, W, H, D = "cuda", 64, 2, 32
+    g = torch.Generator(device=dev).manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, y, y3, w, row, wide = rnd(n, W), rnd(n, W).to(dtype), rnd(n, 3, W), rnd(W), rnd(W), rnd(n, 6 * W).to(dtype)
+    mat, bias = rnd(96, W).to(dtype), rnd(96).to(dtype)
+    counts, starts = ([1] * n, [3] * n) if n < 100 else ([60, 70], [0, 9])
+    batch = LO.RaggedBatch.build(counts, starts, list(range(len(counts))), [list(range(2 * b, 2 * b + 2)) for b in range(len(counts))], 64, dev)
+    B, cos, sin = len(counts), rnd(200, 8), rnd(200, 8)
+    pool, pool_v = (torch.zeros(B * 128, H * D, dtype=dtype, device=dev) for _ in range(2))
+    calls = dict(
+        linear=lambda s: [LO.linear(y, mat, b, f) for b in (None, bias) for f in (None, True, False)] + [LO.linear(wide[:, W:2 * W], mat)],
+        add_rmsnorm=lambda s: [LO.add_rmsnorm(s["x"], v, u, k, 1e-5, t) for v, u, k, t in ((y, None, w.to(dtype), dtype), (y3, x, None, torch.float32), (None, None, None, None))] + [s["x"]],
+        sandwich_norm=lambda s: [LO.sandwich_norm(s["x"], y, w, 1e-5, row, dtype), LO.sandwich_norm(s["x"], None, None, 1e-5, None, torch.float32, add_row=row, plain=True),
+                                 LO.sandwich_norm(s["x"], y, w, 1e-5, w, None, out=s["wide"][:, W:2 * W]), s["x"], s["wide"]],
+        output_norm=lambda s: [LO.output_norm(s["x"], [(y, None), (y3, row)], w, 1e-5, kind, 0.5, row, dtype) for kind in (LO.NORM_RMS, LO.NORM_LAYER)] + [LO.output_norm(s["x"], [], None, 1e-5, 0, out_dtype=dtype)],
+        gated_norm=lambda s: [LO.gated_norm(x, wide[:, :W], w, 1e-5, N.JL_ACT_SILU, True, 2, 0.5), LO.gated_norm(x, wide[:, :W], w, 1e-5, N.JL_ACT_SIGMOID, False, out=s["wide"][:, 2 * W:3 * W]), s["wide"]],
+        gated_act=lambda s: [LO.gated_act(wide, 0, W, W, LO.ACT_SILU), LO.gated_act(wide, W, -1, 2 * W, LO.ACT_GELU_ERF, row_gate=wide[:, 5])],
+        heads_gate=lambda s: [LO.heads_gate(wide.view(H, n, 3 * W), None), LO.heads_gate(wide[:, :2 * W].contiguous().view(H, n, W), wide[:, 2 * W:4 * W])],
+        embed_scale=lambda s: [v for v in LO.embed_scale(mat, torch.arange(n, device=dev) % 96, 1.5, True, copy_dtype=torch.bfloat16) + LO.embed_scale(mat, torch.arange(n, device=dev) % 96, 2.0, False, s["x"])],
+        token_shift=lambda s: [LO.token_shift(x, w, batch, s["tail"], dtype), s["tail"]],
+        short_conv=lambda s: [LO.short_conv(wide, W, W, rnd(W, 4).to(dtype).zero_() + 0.5, batch, s["tail3"], bias=mat[0], out_dtype=dtype), s["tail3"]],
+        depth_mix_norm=lambda s: [v for v in LO.depth_mix_norm(x, [(y, row)], 0.7, s["streams"], 1, w, s["x"], w, 1e-5, dtype, True, (row, batch, s["tail"]) if n < 100 else None)] + [s["streams"][1], s["tail"]],
+        linear_scan=lambda s: [LO.linear_scan(wide, (0, 64, 128), batch, H, H, 32, 32, s["state"], act=N.JL_ACT_SILU, decay=torch.full((H,), 0.9, device=dev), skip=row[:H].contiguous()), s["state"]],
+        qk_norm_append=lambda s: [LO.qk_norm_append(wide, (0, 64, 128), H, H, D, D, w.to(dtype), row.to(dtype), 1e-5, s["k"], s["v"], batch.kv_slot, 16, batch=batch, cos=cos, sin=sin), s["k"], s["v"]],
+        latent_prep=lambda s: [LO.latent_prep(wide, 0, 64, 64, 48, 16, 16, w.to(dtype), w[:48].to(dtype), 1e-5, batch, cos, sin, s["k"]), s["k"]],
+        latent_q_pack=lambda s: [LO.latent_q_pack(wide.view(H, n, 3 * W)[:, :, :48].contiguous(), wide[:, :H * (D + 16)], H, D, 48, 16, 16, batch, cos, sin)],
+        moe_experts=lambda s: [v for route, identity in (("sigmoid", 0), ("top_softmax", 2)) for kw in (dict(router_logits=rnd_logits[:, :4 + identity].contiguous(), router=None),
+                               dict(router_logits=None, router=(x, rnd_w[:4 + identity].contiguous(), None)))
+                               for r in [LO.moe_experts(y, kw["router_logits"], row[:4 + identity].contiguous(), 2, 0.5, up, down, route=route, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0), identity=identity, router=kw["router"])]
+                               for v in ((r,) if torch.is_tensor(r) else r[1:])],
+        attention_args=lambda s: [LO.attn_window(wide[:, :H * D].contiguous(), wide[:, 64:128], pool + 0.5, pool_v + 0.25, batch, H, H, D, D, 0.2, 0, 0, None, None, None, sink=row[:H].contiguous()),
+                             LO.attn_sweep(wide[:, :H * D].contiguous(), pool + 0.5, pool_v + 0.25, batch, H, H, D, D, 0.2, 16, gate=wide[:, :H], gate_per_head=True)],
+    )
+    rnd_logits, rnd_w, up, down = rnd(n, 6), rnd(6, W), rnd(4, 2 * 32, W).to(dtype), rnd(4, W, 32).to(dtype)
+    slots = B
+    fresh = lambda: dict(x=x.clone(), wide=wide.clone(), tail=torch.ones(slots, 1, W, device=dev), tail3=torch.ones(slots, 3, W, device=dev), streams=torch.ones(2, n, W, device=dev),
+                         state=torch.ones(slots, H, 32, 32, device=dev), k=pool.clone(), v=pool_v.clone())
+    taken = []
+    from unittest import mock
+    host = LO._host()
+
+    class Watched:
+        def __getattr__(self, name):
+            def call(*a):
+                r = getattr(host, name)(*a)
+                if r is not NotImplemented:
+                    taken.append(name)
+                return r
+            return call
+    with mock.patch.object(LO, "_H", Watched()):
+        for name, f in calls.items():
+            got, want = both(lambda: f(fresh()))
+            assert len(got) == len(want) and all((a is None) == (b is None) and (a is None or (a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b))) for a, b in zip(got, want)), name
+    left = set(calls) - set(taken)
+    assert left == (set() if n < 100 else {"linear_scan"} | ({"linear"} if dtype == torch.float32 else set())), left      # portions of 32 tokens and more go in pieces; 130 float rows to the library
+
+
+@pytest.mark.gpu
+def test_refused_as_before():
+    """Wrong shapes, types, devices and streams' tensors raise what the wrappers raise; gradients go where they went."""
+    from jacobiforcing_amd import _native as N, layer_ops as LO
+    dev = "cuda"
+    x, w = torch.randn(4, 64, device=dev), torch.randn(64, device=dev)
+    for call in (lambda: LO.add_rmsnorm(x.bfloat16(), None, None, None, 1e-5, torch.float32), lambda: LO.add_rmsnorm(x, x[:3], None, None, 1e-5, torch.float32),
+                 lambda: LO.sandwich_norm(x, None, None, 1e-5, None, torch.float32), lambda: LO.gated_act(x, 60, -1, 8, LO.ACT_SILU), lambda: LO.add_rmsnorm(x, None, None, w, 1e-5, torch.float16),
+                 lambda: LO.output_norm(x, [(x, None)] * 4, w, 1e-5, 0), lambda: LO.output_norm(x, [(x, None)], w, 1e-5, 9), lambda: LO.heads_gate(x.view(2, 2, 64).half(), None)):
+        with pytest.raises(ValueError):
+            call()
+    with pytest.raises(N.NativeLibraryError):
+        LO.add_rmsnorm(x.cpu(), None, None, None, 1e-5, torch.float32)
+    leaf = torch.randn(16, 64, device=dev, requires_grad=True)
+    LO.linear(x, leaf).sum().backward()
+    assert leaf.grad is not None
+    with torch.no_grad():
+        assert not LO.linear(x, leaf).requires_grad
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        LO.add_rmsnorm(x.clone(), None, None, w, 1e-5, torch.float32)
+    assert torch.empty in seen                                                               # a mode that watches calls still sees the wrapper's
