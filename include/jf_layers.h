@@ -322,6 +322,15 @@ JL_API int jl_latent_prep(const void *proj, int dtype, int64_t N, int64_t ld, in
 JL_API int jl_latent_q_pack(const void *qa, const void *q, int64_t q_ld, int dtype, int64_t N, int32_t H, int32_t D, int32_t R, int32_t rd,
                             int32_t rot_dims, const int32_t *pos, const float *cos_t, const float *sin_t, int64_t table_len, void *q_out,
                             int32_t pairing, void *stream);
+/* Per-head products of a few tokens, bfloat16: out[n, h, :O] = x[n, h, :K] . w[h] with w [H, K, O]; x rows x_ld and heads x_head elements apart, out likewise.  gate (or null; [N, H*O], rows gate_ld apart):
+ * times its sigmoid.  rd > 0: out[n, h, O : O + rd] = rotate(x[n, h, K : K + rd], pos[n]).  Rows and heads of x, and w, at 16-byte borders, K and O multiples of 8. */
+typedef struct {
+    const void *x; const void *w; void *out; const void *gate;
+    const int32_t *pos; const float *cos_t; const float *sin_t;
+    int64_t N, x_ld, out_ld, gate_ld;
+    int32_t H, K, O, x_head, out_head, rd, rot_dims, pairing;
+} jl_latent_heads;
+JL_API int jl_latent_heads_run(const jl_latent_heads *a, void *stream);
 /* out[n, h*Dv + d] = ov[h, n, d] * sigmoid(gate[n * gate_ld + h*Dv + d]) (gate null: no gate). */
 JL_API int jl_heads_gate(const void *ov, const void *gate, int64_t gate_ld, int dtype, int64_t N, int32_t H, int32_t Dv, void *out,
                          void *stream);

@@ -264,6 +264,12 @@ class MoeRouter(C.Structure):
                [(k, _i32) for k in ("x_dtype", "K", "E", "experts", "top", "kind", "tile_rows", "max_tiles")] + [("scale", _f32), ("renorm_eps", _f32), ("parts", _vp), ("slices", _i32)]
 
 
+class LatentHeads(C.Structure):
+    """jl_latent_heads (include/jf_layers.h)."""
+    _fields_ = [(k, _vp) for k in ("x", "w", "out", "gate", "pos", "cos_t", "sin_t")] + [(k, _i64) for k in ("N", "x_ld", "out_ld", "gate_ld")] + \
+               [(k, _i32) for k in ("H", "K", "O", "x_head", "out_head", "rd", "rot_dims", "pairing")]
+
+
 class RetentionPieces(C.Structure):
     """jl_retention_pieces (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("proj", "piece_rec", "req", "pos", "cos_t", "sin_t", "decay", "state", "scratch", "out", "raw")] + [("ld", _i64), ("table_len", _i64), ("N", _i64)] + \
@@ -344,6 +350,7 @@ _LAYER_SIGNATURES = {
     "jl_delta_chunks_run": (C.c_int, [_vp, _vp]),
     "jl_delta_rule": (C.c_int, [_vp, C.c_int, _i64, _i32, _i32, _i32, _vp, C.c_int, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                 _i32, _i32, _f32, _f32, _f32, _vp, _vp, _vp, _vp]),
+    "jl_latent_heads_run": (C.c_int, [C.POINTER(LatentHeads), _vp]),
     "jl_linear_mid": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _i64, _i32, _vp]),
     "jl_linear_split": (C.c_int, [_vp, _i64, _i64, _vp, _i32, _i32, _vp, _vp, _i64, _vp]),
     "jl_linear_small": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, C.c_int, _i32, _i32, _vp, _vp, _i64, _i32, _vp]),

@@ -21,7 +21,7 @@ namespace {
 
 #define JL_HOST_CALLS(X)                                                                                                                              \
     X(jl_linear_small) X(jl_linear_mid) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
-    X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) \
+    X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) X(jl_latent_heads_run) \
     X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
 #define DECLARE(name) decltype(&name) p_##name;
 JL_HOST_CALLS(DECLARE)
@@ -326,6 +326,29 @@ CALL(latent_q_pack, 13)
     return wrap(out);
 END_CALL
 
+// x (heads of x_head columns), w [H, K, O], x_head, rd, gate, rot_dims, N, max_pos, pos, cos, sin, pairing: the products of latent attention's heads, [N, H * (O + rd)]
+CALL(latent_heads, 12)
+    const Tensor *x, *w, *gate, *pos, *cos, *sin;
+    int32_t x_head, rd, rot_dims, pairing;
+    int64_t n, max_pos, length;
+    NEED(take(arg[0], x) && take(arg[1], w) && take(arg[2], x_head) && take(arg[3], rd) && take_maybe(arg[4], gate) && take(arg[5], rot_dims) && take(arg[6], n) && take(arg[7], max_pos) &&
+         take(arg[8], pos) && take_maybe(arg[9], cos) && take_maybe(arg[10], sin) && take(arg[11], pairing));
+    NEED(x->dim() == 2 && x->scalar_type() == at::kBFloat16 && x->stride(1) == 1 && x->size(0) == n && n > 0 && w->dim() == 3 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && rd >= 0);
+    const int64_t H = w->size(0), K = w->size(1), O = w->size(2);
+    NEED(H > 0 && K > 0 && O > 0 && H * (O + rd) <= INT32_MAX && x_head >= K + rd && x->size(1) == H * x_head && w->device() == x->device());
+    NEED(!gate || (rows(*gate, n, H * O) && gate->stride(1) == 1 && gate->scalar_type() == at::kBFloat16 && rd == 0));
+    NEED(angles(rot_dims, cos, sin, max_pos, length));
+    NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())));
+    Tensor out = make({n, H * (O + rd)}, at::kBFloat16, *x);
+    jl_latent_heads a = {};
+    a.x = x->data_ptr(); a.w = w->data_ptr(); a.out = out.data_ptr(); a.gate = at_(gate); a.gate_ld = gate ? gate->stride(0) : 0;
+    a.pos = (const int32_t *)pos->data_ptr(); a.cos_t = (const float *)at_(cos); a.sin_t = (const float *)at_(sin);
+    a.N = n; a.x_ld = x->stride(0); a.out_ld = H * (O + rd); a.H = (int32_t)H; a.K = (int32_t)K; a.O = (int32_t)O; a.x_head = x_head; a.out_head = (int32_t)(O + rd); a.rd = rd;
+    a.rot_dims = rot_dims; a.pairing = pairing;
+    RUN(jl_latent_heads_run, &a, stream_of(*x));
+    return wrap(out);
+END_CALL
+
 // float [slots, ..] with `per` values per slot and the batch's slots
 bool carries(const Tensor *tail, int64_t per, int64_t max_slot) {
     return tail && is_float(*tail) && tail->is_contiguous() && tail->dim() > 0 && tail->numel() == tail->size(0) * per && max_slot < tail->size(0);
@@ -576,7 +599,7 @@ PyObject *symbols(PyObject *, PyObject *) {
 }
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack),
+PyMethodDef methods[] = {FAST(linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
                          FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), {"bind", bind, METH_VARARGS, nullptr},
                          {"linear_rule", linear_rule, METH_VARARGS, nullptr}, {"symbols", symbols, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_jl_host", nullptr, -1, methods};

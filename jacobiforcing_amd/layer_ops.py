@@ -1247,6 +1247,16 @@ def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, 
     return chosen
 
 
+LATENT_HEADS = 8 << 20                # rows x heads x latent up to which the package forms the products of latent attention's heads
+
+
+def latent_heads(n: int, H: int, D: int, R: int, Dv: int, dtype: torch.dtype) -> bool:
+    """Whether the heads' products on both sides of attention over a latent are the package's launches, for n tokens.  us of GPU time, queries + outputs, library's products and their packing / own: 32
+    tokens of 16 heads of 128, latent 512, 14.7 + 13.9 / 7.7 + 5.7, 1 token 13.1 + 14.4 / 4.1 + 5.0, 256 17.3 + 19.5 / 10.0 + 7.3, 512 22.1 + 15.4 / 15.5 + 14.8, 2000 of 8 heads, latent 256, 22.0 + 14.5 /
+    15.6 + 10.3; at the line 1000 of 16 heads, latent 512, 34.3 + 18.6 / 30.4 + 22.2.  And 50 us less of the host."""
+    return dtype == torch.bfloat16 and 0 < n * H * R <= LATENT_HEADS and D % 8 == 0 and R % 8 == 0 and Dv % 8 == 0
+
+
 def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w_uk: torch.Tensor, w_uv: torch.Tensor, batch: RaggedBatch, H: int, D: int, R: int, rd: int, Dv: int, rot_dims: int,
                      cos, sin, pairing: int, scale: float, window: int, sink: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
                      gate_per_head: bool = False) -> torch.Tensor:
@@ -1255,7 +1265,8 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
     w_uk [H, D, R] and w_uv [H, R, Dv] the same per head, the latter turned.  ``window`` 0: plain causal; ``sink`` float [H]; ``gate`` a [N, H*Dv] view, or [N, H] with
     ``gate_per_head``: sigmoid gates on the outputs.
     Decoded tokens and short portions bring their queries to the latent (``latent_q_pack``, ``latent_attend``); for long portions in bfloat16 keys and values
-    are built per head (``_latent_built_requests``) and attended on the 128-row tiles; a step may hold both."""
+    are built per head (``_latent_built_requests``) and attended on the 128-row tiles; a step may hold both.  Few tokens over the latent: the heads' products in launches of the package's own
+    (``latent_heads``)."""
     _dev(q)
     n, dt = q.shape[0], q.dtype
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] == H * (D + rd) and n == batch.N, "latent_attention: q [N, H*(D + rd)] of the batch")
@@ -1265,6 +1276,13 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
 
     def over_latent(q, batch, gate):
         m = q.shape[0]
+        if latent_heads(m, H, D, R, Dv, dt) and attn_sweep_tile_rows(dt, H, 1, R + rd, R, pool, pool[:, :R]):
+            qf = (_H or _host()).latent_heads(q, w_uk, D + rd, rd, None, rot_dims, batch.N, batch.max_pos, batch.pos, cos, sin, pairing)
+            if qf is not NotImplemented:
+                o = attn_sweep(qf, pool, pool[:, :R], batch, H, 1, R + rd, R, scale, window, sink=sink, gate=gate if gate_per_head else None, gate_per_head=gate_per_head)
+                r = (_H or _host()).latent_heads(o, w_uv, R, 0, None if gate_per_head else gate, 0, batch.N, batch.max_pos, batch.pos, None, None, pairing)
+                if r is not NotImplemented:
+                    return r
         qa = torch.bmm(q.view(m, H, D + rd)[:, :, :D].transpose(0, 1), w_uk)      # [H, N, R]: query . (W_uk c) = (W_uk^T query) . c
         qf = latent_q_pack(qa, q, H, D, R, rd, rot_dims, batch, cos, sin, pairing=pairing)
         return heads_gate(latent_attend(qf, pool, w_uv, batch, H, R, rd, scale, window, sink=sink, gate=gate if gate_per_head else None), None if gate_per_head else gate)
