@@ -207,40 +207,47 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
     return jl_check_launch("retention_join_kernel");
 }
 
-// ---- long portions on the float matrix instructions: pieces side by side, 64 tokens at a time -------------------------------------------------
+// ---- long portions in pieces side by side, 32 tokens at a time on the bfloat16 matrix instructions ----------------------------------------------
 // With g = the head's decay, a group of n tokens is three products on the state S the group starts from:
 //   o_i = g^(i+1) S^T q_i + sum_{j <= i} g^(i-j) (q_i . k_j) v_j,          S <- g^n S + sum_j g^(n-1-j) k_j v_j^T.
 // A portion is cut into pieces (whole groups, except the last) that run side by side: every piece's own contribution to the state (RM_LOCAL, not for a
 // request's last piece), the state every piece starts from (retention_pieces_join_kernel), outputs (RM_OUT; the last piece leaves the final state in its slot).
-// A workgroup owns one head of one piece; wavefront w holds columns 32 w .. + 31 of S [D, Dv] in accumulators.  v_mfma_f32_32x32x2_f32: lane l supplies
-// row (A) or column (B) l % 32 at depth l / 32, accumulator r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 — so the state's accumulators are the B operand of
-// S^T q as they are (register r against the query's element of the same row), and never cross LDS.  Everything is a 32-bit number from the projection on, as in
-// the scan: no operand is split or rounded.  q, k (rotated, scaled), v and the pairs' weights of the group lie in LDS as floats; the next group's rows
-// are on their way meanwhile.
-// What bounds it: 368 matrix instructions of 64 cycles per wavefront and group of 64 tokens at 128 x 128, and the phases of a group at one workgroup per CU.
-// Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups (a second pass over a group that holds one).
-// Outputs leave as floats and are normed and gated by rows in a launch of their own: in this one, a wavefront's sums over its 32 columns cost 160 exchanges per group and the gates
-// came two bytes at a time, four on their way (outputs 211 us then, 119 and 18 now).
-// Measured at 8 heads of 128 x 128, bfloat16, against the scan (chunks of 64 tokens side by side): 4 x 2048 tokens 1157 -> 182 us, one prompt of 128
-// 985 -> 53, 8 x 8 tokens 84 -> 34; float, 1021 + 851 + 681 tokens: 1091 -> 105.
-constexpr int RM_T = 64, RM_OUT = 0, RM_LOCAL = 1;
+// q and k are 32-bit numbers behind their rotation, as are the state, the pairs' weights and the decayed values: each enters the products as the sum of three bfloat16 numbers, of whose nine products six are
+// formed (jl_split8; bfloat16 values are one number).  The terms of q and k are made once per group, on the way into LDS, the others in the registers that hold them: a workgroup owns one head of one
+// piece, wavefront w columns 32 w .. + 31 of S [D, Dv] in accumulators.  Accumulator r of lane l of a 32 x 32 product is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32, so registers 8s .. 8s + 7 are an operand
+// over the depths 16s + 4 (l / 32) + {0 .. 3, 8 .. 11} as they are: the state as B of S^T q, the weights of the pairs (formed turned, K Q^T, by every wavefront for itself) as A of the sum over values.
+// q and k rows are read in that order as two 8-byte halves; k (for the state) and v are turned by ds_read_b64_tr_b16.  Two barriers per group.
+// What bounds it: issue and latency at two workgroups per CU; 150 products of 32 cycles per group and wavefront (4 800 cycles) beside splits, rotations and
+// LDS reads, where a group takes 14 us with all of them.
+// Before, 64 tokens at a time on the float matrix instructions (368 products of 64 cycles per wavefront, rotated in LDS behind a barrier of their own, the pairs' weights through LDS, one workgroup per CU).
+// us, 8 heads of 128 x 128, bfloat16, 4 x 2048 tokens, outputs / contributions: 121 / 54 then, 58 / 26 now; the whole layer 188 / 117, one portion of 128 51 / 36, of 1000 60 / 47, 8 of 8 33 / 24; 8 heads of 64 109 / 70;
+// float, 1021 + 851 + 681 tokens 105 / 80.  Error of the states against 64 bits 2.1e-7 then, 1.7e-7 now.
+// Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups: they are left out of them, and their columns' outputs and state set behind.
+// Outputs leave as floats and are normed and gated by rows in a launch of their own.
+constexpr int RM_T = 64, RC_T = 32, RM_OUT = 0, RM_LOCAL = 1, RC_VROW = 128 + 16;      // RM_T: pieces come in multiples of it
 typedef float rm_f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ rm_f32x16 rm_mma(float a, float b, rm_f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-static constexpr size_t rm_lds_bytes(int DP, bool out) { return ((size_t)RM_T * DP * (out ? 2 : 1) + RM_T * 128 + (out ? RM_T * RM_T : 0) + 2 * RM_T) * 4; }
+typedef float rm_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 rm_bf16x4 __attribute__((ext_vector_type(4)));
+typedef short rm_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) rm_s16x4 rm_lds_s16x4;
+constexpr int RM_TERMS = JL_SPLIT_TERMS;
+template <typename T> static constexpr size_t rm_lds_bytes(int DP, bool out) {
+    return 2 * RC_T * ((out ? 2 : 1) * (size_t)RM_TERMS * (DP + 8) + (sizeof(T) == 4 ? RM_TERMS : 1) * RC_VROW) + (RC_T + 2 * RC_T + 4 * RC_T + 4) * 4;
+}
 
 template <typename T, int DP, int MODE>
-__global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_pieces a) {
+__global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retention_pieces_kernel(jl_retention_pieces a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr bool OUT = MODE == RM_OUT;
-    constexpr int U = DP / 4, KPF = RM_T * U / 256, VPF = RM_T * 32 / 256, NS = DP / 32;
+    constexpr int QROW = DP + 8, SLOTS = DP / 8, QIT = RC_T * SLOTS / 256, VIT = RC_T * 32 / 256, NS = DP / 32, VT = sizeof(T) == 4 ? RM_TERMS : 1;
     const int piece = blockIdx.x, h = blockIdx.y, H = a.H, D = a.D, Dv = a.Dv;
     const int row0 = a.piece_rec[4 * piece], cnt = a.piece_rec[4 * piece + 1], slot = a.piece_rec[4 * piece + 2], last = a.piece_rec[4 * piece + 3];
     if (cnt <= 0 || (!OUT && last)) return;
-    float4 *Ks = (float4 *)smem, *Qs = Ks + RM_T * U;               // [64][D], 16-byte units permuted by the row
-    float *Vs = (float *)(OUT ? Qs + RM_T * U : Qs);                // [64][128]
-    float4 *Ps = (float4 *)(Vs + RM_T * 128);                       // [64][64] decayed q . k of the pairs, permuted likewise
-    float *gp = (float *)Ps + (OUT ? RM_T * RM_T : 0);              // g^0 .. g^64
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, nw = (Dv + 31) / 32, col = 32 * wave + l32;
+    bf16_t *Ks = (bf16_t *)smem, *Vs = Ks + RM_TERMS * RC_T * QROW, *Qs = Vs + VT * RC_T * RC_VROW;      // [terms][32][..]
+    float *g1 = (float *)(Qs + (OUT ? RM_TERMS * RC_T * QROW : 0)), *dec = g1 + RC_T;        // g^(i+1); g^(31-m), none from 32 on
+    int *brokenS = (int *)(dec + 2 * RC_T), *flawS = brokenS + 4 * RC_T;                     // per column: the group's first token whose value is not finite; whether this group, the one before, has one
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * wave + l32;
+    const bool busy = 32 * wave < Dv;
     const float gamma = a.decay[h], kscale = 1.0f / sqrtf((float)D);
     if (wave == 0) {                                                // powers by doubling, which doubles a rounding error too: in 64 bits.  Lane l holds g^(l+1)
         double p = gamma;
@@ -249,211 +256,257 @@ __global__ __launch_bounds__(256, 1) void retention_pieces_kernel(jl_retention_p
             const double y = __shfl_up(p, off, 64);
             if (lane >= off) p *= y;
         }
-        gp[lane + 1] = (float)p;
-        if (lane == 0) gp[0] = 1.0f;
+        if (lane < RC_T) g1[lane] = (float)p;
+        const double q = __shfl(p, lane < 31 ? 30 - lane : 0, 64);
+        dec[lane] = lane < 31 ? (float)q : lane == 31 ? 1.0f : 0.f;
+        if (lane < 4) flawS[lane] = 0;
     }
-    auto at = [](int row, int u) { return u ^ (row & 15); };        // U is a multiple of 16
     const T *src = (const T *)a.proj + (int64_t)row0 * a.ld;
     const int half = a.rot_dims >> 1, hu = half / 4;
+    const int64_t pos0 = half ? a.pos[row0] : 0;                    // a portion's positions follow each other
 
     rm_f32x16 S[NS];
     float *sp = a.scratch + ((int64_t)piece * H + h) * D * Dv;
+    // f(row of the state, byte offset in it, register): one address that moves on, not sixty-four in registers
+    auto each_state = [&](auto &&f) {
+        uint32_t off = (uint32_t)(4 * hi * Dv + col) * 4;
 #pragma unroll
-    for (int t = 0; t < NS; ++t)
+        for (int t = 0; t < NS; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d = 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
-            S[t][r] = (OUT && d < D && col < Dv) ? sp[(int64_t)d * Dv + col] : 0.f;
-        }
-    // a group's rows on their way: four elements of a row per unit
-    typedef typename std::conditional<sizeof(T) == 2, uint2, float4>::type unit_t;
-    unit_t rq[KPF], rk[KPF], rv[VPF];
-    auto to_float = [](const unit_t &w) -> float4 {
-        float v[4];
-        ld4_f((const T *)&w, v);
-        return make_float4(v[0], v[1], v[2], v[3]);
+            for (int r = 0; r < 16; ++r) {
+                asm volatile("" : "+v"(off));
+                S[t][r] = f(32 * t + 8 * (r >> 2) + 4 * hi + (r & 3), off, S[t][r]);
+                off += ((r & 3) == 3 ? 5 : 1) * Dv * 4;
+            }
     };
+    each_state([&](int d, uint32_t off, float) { return (OUT && d < D && col < Dv) ? *(const float *)((const char *)sp + off) : 0.f; });
+    // a group's rows on their way.  A thread's share of q and k: pairs of units of four dimensions that are rotated together (or two that are not)
+    typedef typename std::conditional<sizeof(T) == 2, uint2, rm_f32x4>::type unit_t;
+    unit_t rq[QIT][2], rk[QIT][2], rv[VIT];
+    rm_f32x4 rc[QIT], rs[QIT];
+    const int pair = tid % SLOTS, ua = pair < hu ? pair : 2 * pair, ub = pair < hu ? pair + hu : 2 * pair + 1;
+    const bool turns = pair < hu, in_a = 4 * ua < D, in_b = 4 * ub < D;
     auto fetch = [&](int t0) {
         const int nt = cnt - t0;
         const T *base = src + (int64_t)t0 * a.ld;
         const unit_t zero = {};
 #pragma unroll
-        for (int it = 0; it < KPF; ++it) {
-            const int e = tid + it * 256, tt = e / U, u = e % U;
-            rk[it] = rq[it] = zero;
-            if (tt < nt && 4 * u < D) {
-                const T *row = base + (int64_t)tt * a.ld + h * D + 4 * u;
-                rk[it] = *(const unit_t *)(row + a.k_col);
-                if (OUT) rq[it] = *(const unit_t *)(row + a.q_col);
+        for (int it = 0; it < QIT; ++it) {
+            const int tt = tid / SLOTS + it * (256 / SLOTS);
+            rk[it][0] = rk[it][1] = rq[it][0] = rq[it][1] = zero;
+            if (tt < nt) {
+                const T *k = base + (int64_t)tt * a.ld + h * D + a.k_col, *q = base + (int64_t)tt * a.ld + h * D + a.q_col;
+                if (in_a) rk[it][0] = *(const unit_t *)(k + 4 * ua);
+                if (in_b) rk[it][1] = *(const unit_t *)(k + 4 * ub);
+                if (OUT && in_a) rq[it][0] = *(const unit_t *)(q + 4 * ua);
+                if (OUT && in_b) rq[it][1] = *(const unit_t *)(q + 4 * ub);
+                if (turns) {
+                    const int64_t p = pos0 + t0 + tt < a.table_len ? pos0 + t0 + tt : a.table_len - 1;
+                    rc[it] = *(const rm_f32x4 *)(a.cos_t + p * half + 4 * ua);
+                    rs[it] = *(const rm_f32x4 *)(a.sin_t + p * half + 4 * ua);
+                }
             }
         }
 #pragma unroll
-        for (int it = 0; it < VPF; ++it) {
+        for (int it = 0; it < VIT; ++it) {
             const int e = tid + it * 256, tt = e >> 5, u = e & 31;
             rv[it] = zero;
             if (tt < nt && 4 * u < Dv) rv[it] = *(const unit_t *)(base + (int64_t)tt * a.ld + a.v_col + h * Dv + 4 * u);
         }
     };
+    auto to_float = [](const unit_t &w, const unit_t &x) {
+        float v[4], u[4];
+        ld4_f((const T *)&w, v);
+        ld4_f((const T *)&x, u);
+        return jl_f32x8{v[0], v[1], v[2], v[3], u[0], u[1], u[2], u[3]};
+    };
+    auto put = [](bf16_t *to, const jl_bf16x8 &v, int part) {       // four of the eight
+        *(rm_bf16x4 *)to = part ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
+    };
+    // turned operands: column (or row) l % 32 of 32 columns from c on, tokens 16 s + 4 hi + {0 .. 3, 8 .. 11}
+    const int tr_row = 4 * hi + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    auto turned = [&](const bf16_t *tile, int row_len, int c, int s) {
+        rm_s16x4 part[2];
+#pragma unroll
+        for (int y = 0; y < 2; ++y) part[y] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rm_lds_s16x4 *)(tile + (16 * s + 8 * y + tr_row) * row_len + c + tr_col));
+        return __builtin_bit_cast(jl_bf16x8, __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    auto row_of = [&](const bf16_t *tile, int s) {                  // row l % 32, depths 16 s + 4 hi + {0 .. 3, 8 .. 11}
+        const rm_bf16x4 x = *(const rm_bf16x4 *)(tile + l32 * QROW + 16 * s + 4 * hi), y = *(const rm_bf16x4 *)(tile + l32 * QROW + 16 * s + 8 + 4 * hi);
+        return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto acc8 = [](const rm_f32x16 &v, int s) {
+        jl_f32x8 f;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) f[x] = v[8 * s + x];
+        return f;
+    };
     fetch(0);
-    for (int t0 = 0; t0 < cnt; t0 += RM_T) {
-        const int nt = cnt - t0 < RM_T ? cnt - t0 : RM_T;
+    for (int t0 = 0; t0 < cnt; t0 += RC_T) {
+        const int nt = cnt - t0 < RC_T ? cnt - t0 : RC_T;
         __syncthreads();                                            // the group before has been read
 #pragma unroll
-        for (int it = 0; it < KPF; ++it) {
-            const int e = tid + it * 256, tt = e / U, u = e % U;
-            const float4 k = to_float(rk[it]);
-            Ks[tt * U + at(tt, u)] = make_float4(k.x * kscale, k.y * kscale, k.z * kscale, k.w * kscale);
-            if (OUT) Qs[tt * U + at(tt, u)] = to_float(rq[it]);
-        }
+        for (int it = 0; it < QIT; ++it) {
+            const int tt = tid / SLOTS + it * (256 / SLOTS);
+            auto stage = [&](bf16_t *rows, jl_f32x8 v) {
+                if (turns && tt < nt) {
+                    const jl_f32x8 w = v;
 #pragma unroll
-        for (int it = 0; it < VPF; ++it) {
-            const int e = tid + it * 256;
-            ((float4 *)Vs)[e] = to_float(rv[it]);                   // rows of 128 columns, those beyond Dv and tokens beyond the portion zero
-        }
-        __syncthreads();
-        int broken = RM_T;                                          // the group's first token whose value in this lane's column is not finite
-        if (t0 + RM_T < cnt) fetch(t0 + RM_T);                      // in flight while this group is multiplied
-        for (int e = tid; e < nt * hu; e += 256) {                  // rotation in place: units u and u + half / 4 of a row
-            const int tt = e / hu, u = e - tt * hu;
-            int64_t p = a.pos[row0 + t0 + tt];
-            if (p >= a.table_len) p = a.table_len - 1;
-            const float4 c = *(const float4 *)(a.cos_t + p * half + 4 * u), s = *(const float4 *)(a.sin_t + p * half + 4 * u);
-            auto turn = [&](float4 *rows) {
-                float4 *x = rows + tt * U + at(tt, u), *y = rows + tt * U + at(tt, u + hu);
-                const float4 v = *x, w = *y;
-                *x = make_float4(v.x * c.x - w.x * s.x, v.y * c.y - w.y * s.y, v.z * c.z - w.z * s.z, v.w * c.w - w.w * s.w);
-                *y = make_float4(w.x * c.x + v.x * s.x, w.y * c.y + v.y * s.y, w.z * c.z + v.z * s.z, w.w * c.w + v.w * s.w);
+                    for (int i = 0; i < 4; ++i) { v[i] = w[i] * rc[it][i] - w[4 + i] * rs[it][i]; v[4 + i] = w[4 + i] * rc[it][i] + w[i] * rs[it][i]; }
+                }
+                jl_bf16x8 part[RM_TERMS];
+                jl_split8(v, part);
+#pragma unroll
+                for (int x = 0; x < RM_TERMS; ++x) {
+                    put(rows + (x * RC_T + tt) * QROW + 4 * ua, part[x], 0);
+                    put(rows + (x * RC_T + tt) * QROW + 4 * ub, part[x], 1);
+                }
             };
-            turn(Ks);
-            if (OUT) turn(Qs);
+            stage(Ks, to_float(rk[it][0], rk[it][1]) * kscale);
+            if (OUT) stage(Qs, to_float(rq[it][0], rq[it][1]));
         }
+        float zero = 0.f;                                           // not a number with a value that is not finite
+#pragma unroll
+        for (int it = 0; it < VIT; it += 2) {                       // rows of 128 columns, those beyond Dv and tokens beyond the portion zero
+            const jl_f32x8 v = to_float(rv[it], rv[it + 1]);
+            if (OUT)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) zero = __builtin_fmaf(v[i], 0.f, zero);
+            jl_bf16x8 part[RM_TERMS];
+            if (VT > 1) jl_split8(v, part);
+            else part[0] = __builtin_convertvector(v, jl_bf16x8);
+#pragma unroll
+            for (int x = 0; x < VT; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) {
+                    const int e = tid + (it + y) * 256;
+                    put(Vs + (x * RC_T + (e >> 5)) * RC_VROW + 4 * (e & 31), part[x], y);
+                }
+        }
+        if (OUT && zero != 0.f) flawS[t0 / RC_T & 1] = 1;
         __syncthreads();
+        bool flawed = false;
         if (OUT) {
-            for (int part = wave; part < 3; part += 4) {            // quadrants (queries, keys) of the pairs: (0, 0), (1, 0), (1, 1)
-                const int qi = part > 0, qj = part > 1;
-                rm_f32x16 s;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = 0.f;
-                const int ki = 32 * qj + l32, ii = 32 * qi + l32;
-#pragma unroll 4
-                for (int x = 0; x < U / 2; ++x) {
-                    const float4 k = Ks[ki * U + at(ki, 2 * x + hi)], q = Qs[ii * U + at(ii, 2 * x + hi)];
-                    s = rm_mma(k.x, q.x, s);
-                    s = rm_mma(k.y, q.y, s);
-                    s = rm_mma(k.z, q.z, s);
-                    s = rm_mma(k.w, q.w, s);
+            flawed = __builtin_amdgcn_readfirstlane(flawS[t0 / RC_T & 1]);
+            if (tid == 0) flawS[~(t0 / RC_T) & 1] = 0;
+            if (flawed && busy) {                                   // such values are left out of the products; what they reach is set behind them
+                int broken = RC_T;
+                for (int t = 16 * hi; t < 16 * hi + 16; ++t) {
+                    float v = 0.f;
+                    for (int x = 0; x < VT; ++x) v += ld_f(Vs + (x * RC_T + t) * RC_VROW + col);
+                    if (__builtin_isfinite(v)) continue;
+                    broken = min(broken, t);
+                    for (int x = 0; x < VT; ++x) Vs[(x * RC_T + t) * RC_VROW + col] = 0;
                 }
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int j0 = 32 * qj + 8 * g + 4 * hi;
-                    float v[4];
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = j0 + x <= ii ? s[4 * g + x] * gp[ii - j0 - x > 0 ? ii - j0 - x : 0] : 0.f;
-                    Ps[ii * 16 + at(ii, j0 >> 2)] = make_float4(v[0], v[1], v[2], v[3]);
-                }
+                broken = min(broken, __shfl_xor(broken, 32, 64));
+                brokenS[32 * wave + l32] = broken;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
-            __syncthreads();
-            rm_f32x16 o[2];
-            if (wave < nw) {
-                for (bool first_time = true;; first_time = false) {
+        }
+        if (t0 + RC_T < cnt) fetch(t0 + RC_T);                      // in flight while this group is multiplied
+        if (!busy) continue;
+        jl_bf16x8 vf[VT][2];
 #pragma unroll
-                    for (int rt = 0; rt < 2; ++rt) {
+        for (int x = 0; x < VT; ++x)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) o[rt][r] = 0.f;
+            for (int s = 0; s < 2; ++s) vf[x][s] = turned(Vs + x * RC_T * RC_VROW, RC_VROW, 32 * wave, s);
+        if (OUT) {
+            rm_f32x16 o, p;                                         // outputs; weights of the pairs, turned
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[r] = p[r] = 0.f;
+#pragma unroll
+            for (int s = 0; s < DP / 16; ++s) {
+                jl_bf16x8 qf[RM_TERMS], kf[RM_TERMS], sf[RM_TERMS];
+#pragma unroll
+                for (int x = 0; x < RM_TERMS; ++x) { qf[x] = row_of(Qs + x * RC_T * QROW, s); kf[x] = row_of(Ks + x * RC_T * QROW, s); }
+                jl_split8(acc8(S[s >> 1], s & 1), sf);
+#pragma unroll
+                for (int d = RM_TERMS - 1; d >= 0; --d)             // the terms whose numbers add up to d
+#pragma unroll
+                    for (int x = 0; x <= d; ++x) {
+                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[x], qf[d - x], p, 0, 0, 0);
+                        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[x], sf[d - x], o, 0, 0, 0);
                     }
+                __builtin_amdgcn_sched_barrier(0);       // all operands at once would not fit the registers
+            }
 #pragma unroll
-                    for (int x = 0; x < U / 2; ++x) {
-                        if (x % 2 == 0) __builtin_amdgcn_sched_barrier(0);      // all operands at once would not fit the registers
+            for (int x = 0; x < 4; ++x) {
+                const rm_f32x4 g4 = *(const rm_f32x4 *)(g1 + 8 * x + 4 * hi);
 #pragma unroll
-                        for (int rt = 0; rt < 2; ++rt) {
-                            const int i = 32 * rt + l32;
-                            const float4 q = Qs[i * U + at(i, 2 * x + hi)];
-                            o[rt] = rm_mma(q.x, S[x >> 2][4 * (x & 3)], o[rt]);
-                            o[rt] = rm_mma(q.y, S[x >> 2][4 * (x & 3) + 1], o[rt]);
-                            o[rt] = rm_mma(q.z, S[x >> 2][4 * (x & 3) + 2], o[rt]);
-                            o[rt] = rm_mma(q.w, S[x >> 2][4 * (x & 3) + 3], o[rt]);
-                        }
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int i = 0; i < 4; ++i) o[4 * x + i] *= g4[i];
+            }
 #pragma unroll
-                    for (int rt = 0; rt < 2; ++rt)
+            for (int s = 0; s < 2; ++s) {
+                jl_f32x8 w = acc8(p, s);
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) o[rt][r] *= gp[32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3) + 1];
-                    auto pairs = [&](int x, int first) {                // eight keys; no key of the second half is visible to the first half's queries
-                        float v[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) v[i] = Vs[(8 * x + 4 * hi + i) * 128 + col];
-#pragma unroll
-                        for (int rt = 0; rt < 2; ++rt) {
-                            if (rt < first) continue;
-                            const int i = 32 * rt + l32;
-                            const float4 p = Ps[i * 16 + at(i, 2 * x + hi)];
-                            o[rt] = rm_mma(p.x, v[0], o[rt]);
-                            o[rt] = rm_mma(p.y, v[1], o[rt]);
-                            o[rt] = rm_mma(p.z, v[2], o[rt]);
-                            o[rt] = rm_mma(p.w, v[3], o[rt]);
-                        }
-                    };
-#pragma unroll 2
-                    for (int x = 0; x < 4; ++x) pairs(x, 0);
-#pragma unroll 2
-                    for (int x = 4; x < 8; ++x) pairs(x, 1);
-                    // A value that is not finite makes every sum of its column none, through weights of zero also those of tokens in front of it.  Then, once more without it: what it
-                    // reaches is set below.  (All keys enter a row of the second half.)
-                    if (!first_time || !__any(!__builtin_isfinite(o[1][0]))) break;
-                    for (int j = RM_T - 1; j >= 0; --j)
-                        if (!__builtin_isfinite(Vs[j * 128 + col])) {
-                            broken = j;
-                            if (hi) Vs[j * 128 + col] = 0.f;        // the column's other lane looks at it in the same instruction
-                        }
-                    if (!__any(broken < RM_T)) break;
+                for (int i = 0; i < 8; ++i) {
+                    const int j = 16 * s + 4 * hi + (i & 3) + 8 * (i >> 2);
+                    const float f = w[i] * dec[31 - l32 + j];
+                    w[i] = j <= l32 ? f : 0.f;
                 }
-                if (col < Dv) {                                     // as they are: the norm over a head's Dv columns spans wavefronts, and a gate's bytes are better read in rows
+                jl_bf16x8 wf[RM_TERMS];
+                jl_split8(w, wf);
 #pragma unroll
-                    for (int rt = 0; rt < 2; ++rt)
+                for (int d = RM_TERMS - 1; d >= 0; --d)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int i = 32 * rt + 8 * (r >> 2) + 4 * hi + (r & 3);
-                            if (i < nt) a.raw[(int64_t)(row0 + t0 + i) * ((int64_t)H * Dv) + h * Dv + col] = i < broken ? o[rt][r] : NAN;
-                        }
+                    for (int x = 0; x <= d; ++x)
+                        if (d - x < VT) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[x], vf[d - x < VT ? d - x : 0][s], o, 0, 0, 0);
+            }
+            const int broken = flawed ? brokenS[32 * wave + l32] : RC_T;
+            if (col < Dv) {                                         // as they are: the norm over a head's Dv columns spans wavefronts, and a gate's bytes are better read in rows
+                const uint32_t o_row = (uint32_t)(H * Dv) * 4;
+                char *to = (char *)(a.raw + (int64_t)(row0 + t0) * ((int64_t)H * Dv) + h * Dv);
+                uint32_t off = 4 * hi * o_row + 4 * col;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    asm volatile("" : "+v"(off));
+                    const int i = 8 * (r >> 2) + 4 * hi + (r & 3);
+                    if (i < nt) *(float *)(to + off) = i < broken ? o[r] : NAN;
+                    off += (r & 3) == 3 ? 5 * o_row : o_row;
                 }
             }
         }
-        if (wave < nw && (!OUT || last || t0 + RM_T < cnt)) {       // the state behind the group
-            const float gn = gp[nt];
+        if (!OUT || last || t0 + RC_T < cnt) {                      // the state behind the group
+            const float gn = g1[nt - 1];
 #pragma unroll
             for (int t = 0; t < NS; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) S[t][r] *= gn;
-#pragma unroll 1
-            for (int x = 0; 8 * x < nt; ++x) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int j = 8 * x + 4 * hi + i;
-                    const float v = Vs[j * 128 + col] * gp[nt - 1 - j > 0 ? nt - 1 - j : 0];
+            for (int s = 0; s < 2; ++s) {
+                jl_f32x8 v;
 #pragma unroll
-                    for (int t = 0; t < NS; ++t) {
-                        const int d = 32 * t + l32;
-                        S[t] = rm_mma(((const float *)(Ks + j * U + at(j, d >> 2)))[d & 3], v, S[t]);
-                    }
+                for (int i = 0; i < 8; ++i) {
+                    const int j = 16 * s + 4 * hi + (i & 3) + 8 * (i >> 2);
+                    float f = (float)vf[VT - 1][s][i];
+#pragma unroll
+                    for (int x = VT - 2; x >= 0; --x) f += (float)vf[x][s][i];
+                    v[i] = f * dec[RC_T - nt + j];
+                }
+                jl_bf16x8 vd[RM_TERMS];
+                jl_split8(v, vd);
+#pragma unroll
+                for (int t = 0; t < NS; ++t) {
+                    jl_bf16x8 kf[RM_TERMS];
+#pragma unroll
+                    for (int x = 0; x < RM_TERMS; ++x) kf[x] = turned(Ks + x * RC_T * QROW, QROW, 32 * t, s);
+#pragma unroll
+                    for (int d = RM_TERMS - 1; d >= 0; --d)
+#pragma unroll
+                        for (int x = 0; x <= d; ++x) S[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[x], vd[d - x], S[t], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            if (OUT && broken < RM_T)
+            if (OUT && flawed && brokenS[32 * wave + l32] < RC_T)
 #pragma unroll
                 for (int t = 0; t < NS; ++t)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) S[t][r] = NAN;
         }
     }
-    float *dst = OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : sp;
-    if (col < Dv && (!OUT || last))
-#pragma unroll
-        for (int t = 0; t < NS; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int d = 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
-                if (d < D) dst[(int64_t)d * Dv + col] = S[t][r];
-            }
+    char *dst = (char *)(OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : sp);
+    if (col < Dv && (!OUT || last)) each_state([&](int d, uint32_t off, float v) { if (d < D) *(float *)(dst + off) = v; return v; });
 }
 
 // The state every piece of a request starts from, in place of the piece's own contribution: S = the slot's state (zero at position 0), then for every piece but
@@ -489,7 +542,7 @@ extern "C" int jl_retention_pieces_ok(int dtype, int32_t D, int32_t Dv, int32_t 
 template <typename T, int DP> static int rm_launch(const jl_retention_pieces &a, hipStream_t st) {
     auto local = retention_pieces_kernel<T, DP, RM_LOCAL>;
     auto outs = retention_pieces_kernel<T, DP, RM_OUT>;
-    constexpr size_t l0 = rm_lds_bytes(DP, false), l1 = rm_lds_bytes(DP, true);
+    constexpr size_t l0 = rm_lds_bytes<T>(DP, false), l1 = rm_lds_bytes<T>(DP, true);
     hipError_t e = hipFuncSetAttribute((const void *)local, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l0);
     if (e == hipSuccess) e = hipFuncSetAttribute((const void *)outs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l1);
     if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_retention_pieces_run: cannot get %zu bytes of LDS: %s", l1, hipGetErrorString(e));

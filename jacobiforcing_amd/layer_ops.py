@@ -36,7 +36,7 @@ NARROW_WHOLE = 128                    # ... up to this many keys never: one laun
 BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
-RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 256     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at
+RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 512     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at (us at 256 / 512: 8 heads of 128, 4 x 2048 tokens 126 / 117, of 64 78 / 70; one of 1000 47 / 47)
 RETENTION_CHUNK = 64          # tokens per chunk when a long portion's recurrence is cut into chunks that run side by side
 SCAN_PIECES_FROM, SCAN_WAVES = 32, 2048     # linear recurrence: portions from this many tokens on run in pieces on the matrix cores; wavefronts of 32 columns to aim at (us at
                                             # 1024 / 2048 / 4096: 4 x 2048 tokens of 16 heads of 128 141 / 125 / 151, one of 8192 144 / 127 / 156; 2 x 2048 of 8 heads 59 / 63 / 63, 5 x 1500 of 6 heads of 64 44 / 44 / 44)
