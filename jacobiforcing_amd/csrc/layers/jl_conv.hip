@@ -141,7 +141,7 @@ extern "C" int jl_causal_conv_carry(const float *x, const int32_t *seq, int32_t 
 
 // ---- short causal convolution of a column range of a projection, with an optional bias and an activation, no residual -----------------------
 //   out[t, c] = act(bias[c] + sum_{j < taps} w[c, j] * x[t - taps + 1 + j, col + c])        (zeros before the sequence's start)
-// A workgroup walks CONV_ROWS consecutive rows, a thread owns VC channels (one, or four with 8- or 16-byte loads) and keeps the last taps - 1
+// A workgroup walks ROWS consecutive rows, a thread owns VC channels (one, or four with 8- or 16-byte loads) and keeps the last taps - 1
 // inputs in registers.  The tail (float [slots, taps - 1, C]) is read for the inputs before the step and moved on here by requests with
 // ONE row and by those that start at position 0 (nobody reads their tail); the others leave that to short_conv_carry_kernel, enqueued after
 // every row has read.
@@ -153,7 +153,7 @@ template <int VC, typename P> __device__ __forceinline__ void conv_st(P *p, cons
     if constexpr (VC == 4) st4_f(p, v);
     else st_f(p, v[0]);
 }
-template <typename T, typename TO, int TAPS, int VC>
+template <typename T, typename TO, int TAPS, int VC, int ROWS>
 __global__ __launch_bounds__(256) void short_conv_kernel(const T *__restrict__ x, int64_t ld, int col, const T *__restrict__ w, const T *__restrict__ bias,
                                                           const int32_t *__restrict__ row_req, const int32_t *__restrict__ seq, float *tail, int64_t N, int C, int act,
                                                           TO *__restrict__ out) {
@@ -168,8 +168,8 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T *__restrict__ x
 #pragma unroll
     for (int e = 0; e < VC; ++e) bv[e] = bias ? ld_f(bias + c + e) : 0.f;
     int prev_req = -1;
-    const int64_t n0 = (int64_t)blockIdx.x * CONV_ROWS;
-    for (int r = 0; r < CONV_ROWS && n0 + r < N; ++r) {
+    const int64_t n0 = (int64_t)blockIdx.x * ROWS;
+    for (int r = 0; r < ROWS && n0 + r < N; ++r) {
         const int64_t n = n0 + r;
         const int req = row_req[n];
         const int32_t *rec = seq + 4 * (int64_t)req;
@@ -229,17 +229,24 @@ __global__ __launch_bounds__(256) void short_conv_carry_kernel(const T *__restri
         if (s < keep) tail[((int64_t)slot * keep + s) * C + c] = v[s];
 }
 
+// A row per workgroup where a step's rows are few: they leave the chip room, and eight rows of one thread wait for one another, above all where each is a request of its own whose window comes from its tail.
+// us, bfloat16, eight rows / one per workgroup: 32 requests of one row x 3072 channels 9.4 / 3.0; 8 of 16 rows 9.7 / 5.9; 1207 rows x 1536 12.8 / 8.3; 1024 rows x 3072 11.9 / 11.9 (the border); 2048 rows
+// 16.8 / 18.1; 8192 rows 32.4 / 46.2, whose windows are then read four times.
+constexpr int64_t CONV_FEW = 3 << 20;                                // rows x channels
 template <typename T, typename TO, int TAPS>
-static void short_conv_launch(const void *x, int64_t ld, int col, const void *w, const void *bias, const int32_t *row_req, const int32_t *seq, float *tail, int64_t N,
-                              int C, int act, void *out, hipStream_t st) {
-    const unsigned gx = (unsigned)((N + CONV_ROWS - 1) / CONV_ROWS);
+static void short_conv_launch(const void *x, int64_t ld, int col, const void *w, const void *bias, const int32_t *row_req, const int32_t *seq, float *tail, int64_t N, int C,
+                              int act, void *out, hipStream_t st) {
+    const bool few = N * C <= CONV_FEW;
+    const unsigned gx = (unsigned)(few ? N : (N + CONV_ROWS - 1) / CONV_ROWS);
     auto al = [](const void *q, uintptr_t a) { return ((uintptr_t)q % a) == 0; };
-    if (C % 4 == 0 && col % 4 == 0 && ld % 4 == 0 && al(x, 4 * sizeof(T)) && al(out, 4 * sizeof(TO)) && al(tail, 16))
-        short_conv_kernel<T, TO, TAPS, 4><<<dim3(gx, (unsigned)((C / 4 + 255) / 256)), 256, 0, st>>>((const T *)x, ld, col, (const T *)w, (const T *)bias, row_req, seq,
-                                                                                                     tail, N, C, act, (TO *)out);
-    else
-        short_conv_kernel<T, TO, TAPS, 1><<<dim3(gx, (unsigned)((C + 255) / 256)), 256, 0, st>>>((const T *)x, ld, col, (const T *)w, (const T *)bias, row_req, seq, tail,
-                                                                                                 N, C, act, (TO *)out);
+#define CONV_KERNEL(VC, ROWS) \
+    short_conv_kernel<T, TO, TAPS, VC, ROWS><<<dim3(gx, (unsigned)((C / VC + 255) / 256)), 256, 0, st>>>((const T *)x, ld, col, (const T *)w, (const T *)bias, row_req, seq, tail, N, C, act, (TO *)out)
+    if (C % 4 == 0 && col % 4 == 0 && ld % 4 == 0 && al(x, 4 * sizeof(T)) && al(out, 4 * sizeof(TO)) && al(tail, 16)) {
+        if (few) CONV_KERNEL(4, 1);
+        else CONV_KERNEL(4, CONV_ROWS);
+    } else if (few) CONV_KERNEL(1, 1);
+    else CONV_KERNEL(1, CONV_ROWS);
+#undef CONV_KERNEL
 }
 
 extern "C" int jl_short_conv(const void *x, int dtype, int64_t ld, int32_t col, const void *w, const void *bias, const int32_t *row_req, const int32_t *seq, int32_t B,

@@ -1,4 +1,4 @@
-"""Launches of a row per workgroup in their forms of four values and of one: widths around the borders of the forms, against 64 bits."""
+"""Launches of a row (or a few) per workgroup in their forms of four values and of one, and with few and with many rows: widths around the borders of the forms, against 64 bits."""
 import pytest
 import torch
 
@@ -90,3 +90,28 @@ def test_latents_and_heads(Rq, R, rd, by, pairing, dtype):
         parts = lambda t: t[:, :H * (D + rd)].view(n, H, D + rd)
         want, size = turned(parts(before)[..., D:])
         assert close(parts(q)[..., D:], want, size, 3, dtype) and torch.equal(parts(q)[..., :D], parts(before)[..., :D]) and torch.equal(q[:, H * (D + rd):], before[:, H * (D + rd):])
+
+
+@pytest.mark.parametrize("C,long", [(3072, 1), (3072, 1018), (3072, 1019), (3071, 1021)])
+@pytest.mark.parametrize("taps", [2, 4])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_short_convolution(C, long, taps, dtype):
+    """Requests of one row, of two and of many, from the start and continued, with few and with many rows in the step."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(long)
+    counts, starts = [1, long, 2, 1, 2], [3, 4, 0, 0, 9]
+    b, n = batch(counts, starts), sum(counts)
+    x, w = torch.randn(n, C + 4, generator=g, device="cuda").to(dtype), torch.randn(C, taps, generator=g, device="cuda").to(dtype)
+    bias, tail = torch.randn(C, generator=g, device="cuda").to(dtype), torch.randn(5, taps - 1, C, generator=g, device="cuda").to(dtype).float()
+    want, size, ends, row = [], [], tail.clone(), 0
+    for i, (cnt, start) in enumerate(zip(counts, starts)):
+        past = tail[4 - i].double() if start else torch.zeros_like(tail[0], dtype=torch.float64)
+        seq = torch.cat([past, x[row:row + cnt, 4:].double()])
+        parts = torch.stack([seq[j:j + cnt] * w[:, j].double() for j in range(taps)])
+        want.append(parts.sum(0) + bias.double())
+        size.append(parts.abs().sum(0) + bias.double().abs())
+        ends[4 - i], row = seq[-(taps - 1):].float(), row + cnt
+    for odt in {torch.float32, dtype}:
+        t = tail.clone()
+        y = LO.short_conv(x, 4, C, w, b, t, LO.ACT_NONE, bias=bias, out_dtype=odt)
+        assert close(y, torch.cat(want), torch.cat(size), taps + 1, odt) and torch.equal(t, ends)
