@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 137
+#define JL_VERSION 138
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -149,7 +149,7 @@ JL_API int64_t jl_attn_talk_scratch_floats(int32_t tiles, int32_t TQ, int32_t H,
  * 0 .. kv_len[r] + min(t + 1, row_len[r]) - 1 of the row, at most max_keys: of cache row row_prompt[r] (tables null; page_size the cache's row length) or of the blocks
  * tables[r * table_ld ..] in order (table_cols of them; a negative one counts as block 0).  With cand_rows > 0 a row whose row_cand is not negative has its keys from kv_len on in
  * ck / cv [cand_rows, nkv, cand_max, D].  out [R * T, nkv * G * D].  Indexes beyond their tables are clamped.  Keys shared out over `splits` workgroups
- * (scratch of jl_attn_block_scratch_floats). */
+ * (scratch of jl_attn_block_scratch_floats).  grouped: tiles of 64 (head, token) rows whose keys a workgroup's wavefronts take in groups, else of 128. */
 typedef struct jl_block_args {
     const void *q, *k, *v, *ck, *cv;
     const int32_t *kv_len, *row_len, *row_prompt, *row_cand, *tables;
@@ -158,7 +158,7 @@ typedef struct jl_block_args {
     int64_t table_ld;
     int32_t R, T, nkv, G, D, blocks, page_size, table_cols, cand_rows, cand_max, max_keys, splits;
     float scale;
-    int32_t reserved;
+    int32_t grouped;
 } jl_block_args;
 JL_API int jl_attn_block(const jl_block_args *a, void *stream);
 /* Cache slots of the block's tokens, [R * T] int64: row_prompt * S_max + position where row_cand is negative and the token is one of the row's row_len, else -1; slot_cand (may be

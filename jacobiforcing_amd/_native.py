@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 137                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 138                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -279,7 +279,7 @@ class RetentionPieces(C.Structure):
 class BlockArgs(C.Structure):
     """jl_block_args (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("q", "k", "v", "ck", "cv", "kv_len", "row_len", "row_prompt", "row_cand", "tables", "out", "scratch")] + [("table_ld", _i64)] + \
-               [(k, _i32) for k in ("R", "T", "nkv", "G", "D", "blocks", "page_size", "table_cols", "cand_rows", "cand_max", "max_keys", "splits")] + [("scale", _f32), ("reserved", _i32)]
+               [(k, _i32) for k in ("R", "T", "nkv", "G", "D", "blocks", "page_size", "table_cols", "cand_rows", "cand_max", "max_keys", "splits")] + [("scale", _f32), ("grouped", _i32)]
 
 
 class DeltaChunks(C.Structure):

@@ -2,25 +2,30 @@
 // the block up to itself; a candidate row's block lies in a scratch of its own.
 // The structure is jl_attn_rows.hip's (32 (head, token) rows per wavefront, S^T = K Q^T, weights straight into the second product, V^T through ds_read_b64_tr_b16).  Lengths, cache
 // rows, pages and scratch rows are read by the kernel, so the host builds no mask and gathers no prefix, and the outputs leave token by token as the next product reads them.
-// A key head's rows (heads of a group times tokens) go in tiles of 128; keys are shared out over `splits` workgroups where there are fewer of them than CUs, and a second launch
-// joins the shares (384 workgroups to aim at: one row of 32 tokens, 8 heads over 2, context 512, 28 us whole, 17 shared out; 64 rows 32 and 30).
-// What bounds it: the keys' way through LDS and the softmax's issue at two workgroups per CU, and launches below 20 us.  us against the library's attention with a mask tensor and the
-// copy that its output needs (bfloat16): 64 rows of 32 tokens, 8 heads of 128 over 2, context 512 47 -> 30; one row 40 -> 17; 64 rows of 64, 16 over 2, context 1500 182 -> 96;
-// 32 rows, 14 heads of 64 over 2, context 1000 89 -> 27; 64 rows, 28 heads of 128 over 4, context 1000 199 -> 68.
+// Two forms.  Many rows: tiles of 128 (head, token) rows, four wavefronts that share every tile of 64 keys, two workgroups per CU.  Few (layer_ops._block_plan draws the line): tiles of 64 rows, and a
+// workgroup of eight wavefronts takes four tiles of 32 keys at a time, a pair of wavefronts each; the four groups' sums meet in LDS.  The chip is full with a quarter of the rows, nothing leaves for
+// memory between the shares, and no launch joins them.  Where even that leaves CUs idle, keys are shared out over `splits` workgroups too, and a second launch joins the shares.
+// What bounds it: the keys' way through LDS, the softmax's issue and the matrix instructions, about as long each; few rows: latency of launch, loads and barriers (15 us with one round of keys and with five;
+// loads two rounds ahead changed nothing).  us, bfloat16, 32 tokens, 8 heads of 128 over 2, context 512, before (tiles of 128 rows, keys shared out over up to three workgroups) / now: 64 rows
+// 30.2 / 20.0, 32 27.1 / 18.5, 16 23.8 / 17.5, one 16.7 / 16.0; context 4000, one row 42.7 / 24.6, 8 rows 45.4 / 30.3; 32 rows, 14 heads of 64 over 2, context 1000 27.7 / 17.7.  Many rows (sums scaled
+// seldom, scores scaled in the exponent's own instruction): 128 rows 35.4 / 28.7; 64 rows of 64, 16 heads over 2, context 1500 111.8 / 88.6; 64 rows, 28 heads of 128 over 4, context 1000 79.6 / 65.7.
+// The library's attention with a mask tensor and the copy that its output needs: the first 47, the one row 40, the 14 heads 89, the last two 182 and 199.
 #include "jl_attn.h"
 
-constexpr int AB_THREADS = 256, AB_KT = 64;
-constexpr size_t ab_lds_bytes(int KU) { return 2 * ((size_t)2 * AB_KT * KU * 16 + AB_KT * 4); }
+// two tiles of KT keys and values per key group and their rows; the groups' sums are joined in the same place
+constexpr size_t ab_lds_bytes(int KU, int WM, int KG, int KT) { return (size_t)KG * (2 * 2 * KT * KU * 16 + (KG > 1 && 32 * WM > KT ? 32 * WM : KT) * 8); }
 
-template <int KU>                                                                       // D <= 8 * KU
-__global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args a, int row_tiles) {
+template <int KU, int WM, int KG, int KT>                           // D <= 8 * KU; WM wavefronts of 32 rows, KG groups of them that take every KG-th tile of KT keys
+__global__ __launch_bounds__(64 * WM * KG, KG == 1 ? 2 : 1) void attn_block_kernel(jl_block_args a, int row_tiles) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int KT = AB_KT, NDV = KU / 4, BUF = 2 * KT * KU, PF = KT * KU / AB_THREADS;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+    constexpr int THREADS = 64 * WM, NHF = KT / 32, NDV = KU / 4, BUF = 2 * KT * KU, PF = KT * KU / THREADS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, kg = wave / WM, tid = threadIdx.x - kg * THREADS, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
     const int D = a.D, T = a.T, GT = a.G * T, S = a.splits;
-    const int c = blockIdx.x % a.nkv, split = blockIdx.x / a.nkv % S, rt = blockIdx.x / (a.nkv * S) % row_tiles, r = blockIdx.x / (a.nkv * S * row_tiles);
-    uint4 *buf0 = (uint4 *)smem;
-    int *tokS = (int *)(buf0 + 2 * BUF);                            // [2][KT] rows of D elements in the cache, or ~ rows in the scratch
+    // workgroups that read the same keys lie eight apart, on one XCD
+    const int rt = blockIdx.x / 8 % row_tiles, unit = blockIdx.x / (8 * row_tiles) * 8 + blockIdx.x % 8, c = unit % a.nkv, split = unit / a.nkv % S, r = unit / (a.nkv * S);
+    if (r >= a.R) return;
+    uint4 *buf0 = (uint4 *)smem + kg * 2 * BUF;
+    int *tokS = (int *)((uint4 *)smem + KG * 2 * BUF) + kg * 2 * KT;      // [2][KT] rows of D elements in the cache, or ~ rows in the scratch
     const int cand = a.cand_rows > 0 ? a.row_cand[r] : -1, page_size = a.page_size;
     int kv = a.kv_len[r], len = a.row_len[r];
     kv = kv < 0 ? 0 : kv < a.max_keys ? kv : a.max_keys;
@@ -34,9 +39,8 @@ __global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args
     }
     const int cand_row = cand < a.cand_rows ? cand : a.cand_rows - 1;
     const bf16_t *K = (const bf16_t *)a.k, *V = (const bf16_t *)a.v, *CK = (const bf16_t *)a.ck, *CV = (const bf16_t *)a.cv;
-    for (int e = tid; e < 2 * BUF; e += AB_THREADS) buf0[e] = make_uint4(0, 0, 0, 0);      // columns beyond D and rows beyond the last key stay zero or finite
 
-    const int R = 128 * rt + 32 * wave + l32, t = R % T;            // this lane's row: head R / T of the group, token t; both half-wavefronts hold it
+    const int R = 32 * WM * rt + 32 * wm + l32, t = R % T;            // this lane's row: head R / T of the group, token t; both half-wavefronts hold it
     const bool ok = R < GT;
     const int last = kv + (t + 1 < len ? t + 1 : len) - 1 < n_keys - 1 ? kv + (t + 1 < len ? t + 1 : len) - 1 : n_keys - 1;      // its last key
     ar_bf16x8 qf[KU / 2];
@@ -44,17 +48,18 @@ __global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args
     for (int x = 0; x < KU / 2; ++x) {
         ar_s16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
         if (ok && 16 * x + 8 * hi < D) w = *(const ar_s16x8 *)((const bf16_t *)a.q + (((int64_t)r * a.nkv + c) * GT + R) * D + 16 * x + 8 * hi);
+        if (a.scale < 0.f) w ^= (short)0x8000;                      // scores are scaled behind their maximum: by a factor above zero
         qf[x] = __builtin_bit_cast(ar_bf16x8, w);
     }
     constexpr float LOG2E = 1.44269504088896341f;
-    const float c2 = a.scale * LOG2E;
+    const float c2 = fmaxf(fabsf(a.scale * LOG2E), 1e-30f);
     float m_run = -INFINITY, l_run = 0.f;
     ar_f32x16 acc[NDV];
 #pragma unroll
     for (int y = 0; y < NDV; ++y)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[y][i] = 0.f;
-    const bool wave_live = 128 * rt + 32 * wave < GT, wave_full = 128 * rt + 32 * wave + 31 < GT;
+    const bool wave_live = 32 * (WM * rt + wm) < GT, wave_full = 32 * (WM * rt + wm) + 31 < GT;
 
     ar_s16x8 kreg[PF], vreg[PF];
     int tok_next = 0;
@@ -76,7 +81,7 @@ __global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args
         const int nk = n_keys - kt * KT < KT ? n_keys - kt * KT : KT;
 #pragma unroll
         for (int it = 0; it < PF; ++it) {
-            const int e = tid + it * AB_THREADS, jj = e / KU, u = e % KU;
+            const int e = tid + it * THREADS, jj = e / KU, u = e % KU;
             if (jj < nk && 8 * u < D) {
                 const int x = tok[jj];
                 const int64_t at = (int64_t)(x < 0 ? ~x : x) * D + 8 * u;
@@ -85,79 +90,80 @@ __global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args
             }
         }
     };
-    auto stash = [&](int kt, uint4 *Ks) {
+    auto stash = [&](int kt, uint4 *Ks) {                           // columns beyond D and rows beyond the last key as zeros
         const int nk = n_keys - kt * KT < KT ? n_keys - kt * KT : KT;
+        const ar_s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int it = 0; it < PF; ++it) {
-            const int e = tid + it * AB_THREADS, jj = e / KU, u = e % KU;
-            if (jj < nk && 8 * u < D) {
-                Ks[jj * KU + ar_key_unit<KU>(jj, u)] = __builtin_bit_cast(uint4, kreg[it]);
-                Ks[KT * KU + jj * KU + ar_value_unit<KU>(jj, u)] = __builtin_bit_cast(uint4, vreg[it]);
-            }
+            const int e = tid + it * THREADS, jj = e / KU, u = e % KU;
+            const bool in = jj < nk && 8 * u < D;
+            Ks[jj * KU + ar_key_unit<KU>(jj, u)] = __builtin_bit_cast(uint4, in ? kreg[it] : zero);
+            Ks[KT * KU + jj * KU + ar_value_unit<KU>(jj, u)] = __builtin_bit_cast(uint4, in ? vreg[it] : zero);
         }
     };
-    look_up(t_lo);
+    const int first = t_lo + kg;                                    // this group's first tile
+    look_up(first);
     tokens_out(0);
-    look_up(t_lo + 1);
+    look_up(first + KG);
     tokens_out(1);
     __syncthreads();
-    if (t_lo < t_hi) {
-        fetch(t_lo, tokS);
-        stash(t_lo, buf0);
+    if (first < t_hi) {
+        fetch(first, tokS);
+        stash(first, buf0);
     }
     __syncthreads();
-    for (int kt = t_lo, sel = 0; kt < t_hi; ++kt, sel ^= 1) {
-        if (kt + 1 < t_hi) fetch(kt + 1, tokS + (sel ^ 1) * KT);
-        look_up(kt + 2);
+    for (int kt = first, sel = 0; kt - kg < t_hi; kt += KG, sel ^= 1) {      // as many rounds for every group
+        if (kt + KG < t_hi) fetch(kt + KG, tokS + (sel ^ 1) * KT);
+        look_up(kt + 2 * KG);
         const uint4 *Ks = buf0 + sel * BUF;
         const int j0 = kt * KT;
-        if (wave_live) {
-            ar_f32x16 sc[2];
+        if (wave_live && kt < t_hi) {
+            ar_f32x16 sc[NHF];
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+            for (int hf = 0; hf < NHF; ++hf)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) sc[hf][i] = 0.f;
 #pragma unroll
             for (int x = 0; x < KU / 2; ++x)
 #pragma unroll
-                for (int hf = 0; hf < 2; ++hf) {
+                for (int hf = 0; hf < NHF; ++hf) {
                     const int row = 32 * hf + l32;
                     sc[hf] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ar_bf16x8, Ks[row * KU + ar_key_unit<KU>(row, 2 * x + hi)]), qf[x], sc[hf], 0, 0, 0);
                 }
-            const bool inside = wave_full && j0 + KT <= kv;         // committed keys only: every row sees them
-            const int upto = ok ? last - j0 : -1;
+            if (!wave_full || j0 + KT > kv) {                       // not committed keys only, which every row sees
+                const int upto = ok ? last - j0 : -1;
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+                for (int hf = 0; hf < NHF; ++hf)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float s = sc[hf][i] * c2;
-                    sc[hf][i] = inside || 32 * hf + 8 * (i >> 2) + 4 * hi + (i & 3) <= upto ? s : -INFINITY;
-                }
+                    for (int i = 0; i < 16; ++i) sc[hf][i] = 32 * hf + 8 * (i >> 2) + 4 * hi + (i & 3) <= upto ? sc[hf][i] : -INFINITY;
+            }
             float mx = sc[0][0];
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+            for (int hf = 0; hf < NHF; ++hf)
 #pragma unroll
                 for (int i = hf == 0 ? 1 : 0; i < 16; ++i) mx = fmaxf(mx, sc[hf][i]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run, mx), m_sub = m_new > -INFINITY ? m_new : 0.f;
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);
-            float sum = 0.f;
-#pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) { sc[hf][i] = __builtin_amdgcn_exp2f(sc[hf][i] - m_sub); sum += sc[hf][i]; }
-            l_run = l_run * alpha + sum;
-            m_run = m_new;
-            if (__any(alpha != 1.0f)) {
+            const float m_new = fmaxf(m_run, mx * c2);
+            if (__any(m_new - m_run > AR_SLACK)) {                  // seldom after the first tiles
+                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));
+                m_run = m_new;
+                l_run *= alpha;
 #pragma unroll
                 for (int y = 0; y < NDV; ++y)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) acc[y][i] *= alpha;
             }
+            const float m_sub = m_run > -INFINITY ? m_run : 0.f;
+            float sum = 0.f;
+#pragma unroll
+            for (int hf = 0; hf < NHF; ++hf)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) { sc[hf][i] = __builtin_amdgcn_exp2f(fmaf(sc[hf][i], c2, -m_sub)); sum += sc[hf][i]; }
+            l_run += sum;
             const char *Vs = (const char *)(Ks + KT * KU);
             const int vk = 4 * hi + ((lane & 15) >> 2), vc8 = 8 * (lane & 1), vu = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);      // this lane's key, half unit and unit of a turned block
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+            for (int hf = 0; hf < NHF; ++hf)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
                     ar_f32x8 pf;
@@ -177,26 +183,71 @@ __global__ __launch_bounds__(AB_THREADS, 2) void attn_block_kernel(jl_block_args
                     }
                 }
         }
-        if (kt + 1 < t_hi) stash(kt + 1, buf0 + (sel ^ 1) * BUF);
+        if (kt + KG < t_hi) stash(kt + KG, buf0 + (sel ^ 1) * BUF);
         tokens_out(sel);
         __syncthreads();
     }
     l_run += __shfl_xor(l_run, 32, 64);
+    if constexpr (KG > 1) {                                         // the groups' sums meet in LDS: a wavefront joins its rows' columns 32 kg .. 32 kg + 31
+        ar_f32x4 *sums = (ar_f32x4 *)smem;                          // [KG][WM][NDV][4][64]
+        float *ml = (float *)((uint4 *)smem + KG * 2 * BUF);        // [KG][WM][32] greatest exponents, then the weights' sums
+        static_assert(KG * WM * NDV * 4 * 64 <= KG * 2 * BUF && NDV <= KG);
+        const int mine = kg * WM + wm;
+#pragma unroll
+        for (int y = 0; y < NDV; ++y)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ar_f32x4 v;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[x] = acc[y][4 * g + x];
+                sums[((mine * NDV + y) * 4 + g) * 64 + lane] = v;
+            }
+        if (hi == 0) {
+            ml[mine * 32 + l32] = m_run;
+            ml[(KG * WM + mine) * 32 + l32] = l_run;
+        }
+        __syncthreads();
+        float w[KG];
+        bool any[KG];
+        m_run = -INFINITY;
+        l_run = 0.f;
+#pragma unroll
+        for (int g = 0; g < KG; ++g) m_run = fmaxf(m_run, ml[(g * WM + wm) * 32 + l32]);
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+            const float l = ml[(KG * WM + g * WM + wm) * 32 + l32];
+            any[g] = l != 0.f;                                      // an empty share's sums are not read
+            w[g] = any[g] ? __builtin_amdgcn_exp2f(ml[(g * WM + wm) * 32 + l32] - m_run) : 0.f;
+            l_run += w[g] * l;
+        }
+        if (kg >= NDV) return;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            ar_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                const ar_f32x4 x = sums[(((g * WM + wm) * NDV + kg) * 4 + q) * 64 + lane];
+                if (any[g]) v += w[g] * x;
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x) acc[0][4 * q + x] = v[x];
+        }
+    }
     if (!ok) return;
     const float inv = l_run != 0.f ? 1.0f / l_run : 0.f;
     const int64_t width = (int64_t)a.nkv * a.G * D, row = ((int64_t)r * T + t) * width + (int64_t)(c * a.G + R / T) * D;
     const int64_t rows = (int64_t)a.R * T * a.nkv * a.G;            // a split's (token, head) rows
-    if (S > 1 && hi == 0) {
+    if (S > 1 && hi == 0 && (KG == 1 || kg == 0)) {
         float *ml = a.scratch + S * rows * D + (split * rows + row / D) * 2;
         ml[0] = m_run;
         ml[1] = l_run;
     }
     if (S > 1 && l_run == 0.f) return;                             // an empty share is not read
 #pragma unroll
-    for (int y = 0; y < NDV; ++y)
+    for (int y = 0; y < (KG > 1 ? 1 : NDV); ++y)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int col = 32 * y + 8 * g + 4 * hi;                // registers 4g .. 4g + 3: four consecutive columns
+            const int col = 32 * (KG > 1 ? kg : y) + 8 * g + 4 * hi;      // registers 4g .. 4g + 3: four consecutive columns
             if (col >= D) continue;
             float v[4];
 #pragma unroll
@@ -255,15 +306,17 @@ extern "C" int jl_block_slots(const int32_t *positions, const int32_t *row_promp
 extern "C" int jl_attn_block_ok(int dtype, int32_t D) { return dtype == JL_BF16 && D > 0 && D % 8 == 0 && D <= 128; }
 extern "C" int64_t jl_attn_block_scratch_floats(int64_t R, int32_t T, int32_t nkv, int32_t G, int32_t D, int32_t splits) { return splits > 1 ? splits * R * T * nkv * G * (D + 2) : 0; }
 
-template <int KU> static int ab_launch(const jl_block_args &a, hipStream_t st) {
-    constexpr size_t lds = ab_lds_bytes(KU);
-    auto kern = attn_block_kernel<KU>;
+template <int KU, int WM, int KG, int KT> static int ab_launch(const jl_block_args &a, hipStream_t st) {
+    constexpr size_t lds = ab_lds_bytes(KU, WM, KG, KT);
+    auto kern = attn_block_kernel<KU, WM, KG, KT>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_attn_block: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     }
-    const int row_tiles = (a.G * a.T + 127) / 128;
-    kern<<<dim3((unsigned)(a.R * row_tiles * a.splits * a.nkv)), AB_THREADS, lds, st>>>(a, row_tiles);
+    const int row_tiles = (a.G * a.T + 32 * WM - 1) / (32 * WM);
+    const int64_t units = ((int64_t)a.R * a.nkv * a.splits + 7) / 8 * 8;
+    if (units * row_tiles > INT32_MAX) return jl_fail(JL_E_INVALID, "jl_attn_block: more rows than 32 bits count");
+    kern<<<dim3((unsigned)(units * row_tiles)), 64 * WM * KG, lds, st>>>(a, row_tiles);
     if (a.splits > 1) {
         const int64_t rows = (int64_t)a.R * a.T * a.nkv * a.G;
         attn_block_join_kernel<<<dim3((unsigned)((rows + 7) / 8)), 256, 0, st>>>(a, rows);
@@ -281,8 +334,10 @@ extern "C" int jl_attn_block(const jl_block_args *ap, void *stream) {
         (a.tables ? a.table_cols <= 0 || a.table_ld < a.table_cols : a.max_keys > a.page_size) ||
         (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.ck | (uintptr_t)a.cv | (uintptr_t)a.out | (uintptr_t)a.scratch) & 15))
         return jl_fail(JL_E_INVALID, "jl_attn_block: sizes or alignment (ask jl_attn_block_ok)");
-    if ((int64_t)a.blocks * a.nkv * a.page_size > INT32_MAX || (int64_t)(a.cand_rows > 0 ? a.cand_rows : 0) * a.nkv * a.cand_max > INT32_MAX ||
-        (int64_t)a.R * ((a.G * (int64_t)a.T + 127) / 128) * a.splits * a.nkv > INT32_MAX)
+    if ((int64_t)a.blocks * a.nkv * a.page_size > INT32_MAX || (int64_t)(a.cand_rows > 0 ? a.cand_rows : 0) * a.nkv * a.cand_max > INT32_MAX || a.G * (int64_t)a.T > INT32_MAX - 128 ||
+        (int64_t)a.R * a.splits * a.nkv > INT32_MAX)
         return jl_fail(JL_E_INVALID, "jl_attn_block: more rows than 32 bits count");
-    return a.D <= 64 ? ab_launch<8>(a, (hipStream_t)stream) : ab_launch<16>(a, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (a.grouped) return a.D <= 64 ? ab_launch<8, 2, 4, 32>(a, st) : ab_launch<16, 2, 4, 32>(a, st);
+    return a.D <= 64 ? ab_launch<8, 4, 1, 64>(a, st) : ab_launch<16, 4, 1, 64>(a, st);
 }

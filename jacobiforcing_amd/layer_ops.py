@@ -8,6 +8,7 @@ from __future__ import annotations
 import bisect
 import ctypes as C
 import itertools
+import math
 import operator
 import os
 import threading
@@ -33,7 +34,7 @@ NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, a
                                       # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
 NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
                                       # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
-BLOCK_WORKGROUPS = 384               # a draft block's attention: workgroups to aim at when keys are shared out
+BLOCK_WORKGROUPS = 384               # a draft block's attention without key groups: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
 RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 512     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at (us at 256 / 512: 8 heads of 128, 4 x 2048 tokens 126 / 117, of 64 78 / 70; one of 1000 47 / 47)
@@ -622,6 +623,17 @@ def block_slots(positions: torch.Tensor, T: int, row_prompt: torch.Tensor, row_c
     return out[0], out[1] if candidates else None
 
 
+def _block_plan(heads: int, GT: int, max_keys: int):
+    """(shares of the keys, whether a workgroup's wavefronts take keys in groups) for ``heads`` (row, key head) pairs of GT (head, token) rows.  Groups, one workgroup of 64 rows per CU, where
+    those fit the chip at once; us with / without, 8 heads of 128 over 2, 32 tokens, context 512: 64 rows (256 workgroups) 20.0 / 27.1, 96 rows 35.8 / 27.6.  A share more costs its sums' way
+    through memory, by the rows, and a launch: one row, context 500 / 1000 / 4000 / 16000: 2, 4, 8 and 16 shares are the fastest; 32 rows, context 512: one 18.5, two 21.6, context 2000: 43.0
+    and 32.9.  Without groups, 96 rows: one share / two at context 512 27.6 / 32.2, 1000 50.0 / 50.6, 2000 79.8 / 69.9."""
+    units = max(1, heads * -(-GT // 64))
+    if units <= 256:
+        return max(1, min(256 // units, math.isqrt(max_keys // (64 + 2 * units)))), 1
+    return max(1, min(BLOCK_WORKGROUPS // (heads * -(-GT // 128)), max_keys // 768)), 0
+
+
 def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len: torch.Tensor, row_len: torch.Tensor, max_keys: int, row_prompt: Optional[torch.Tensor] = None,
                tables: Optional[torch.Tensor] = None, row_cand: Optional[torch.Tensor] = None, ck: Optional[torch.Tensor] = None, cv: Optional[torch.Tensor] = None,
                scale: Optional[float] = None) -> torch.Tensor:
@@ -640,8 +652,7 @@ def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len
           (ck is None or (ck.shape == cv.shape and ck.shape[2] >= T)), "attn_block: shapes")
     out = torch.empty((R * T, nkv * G * D), dtype=q.dtype, device=q.device)
     max_keys = min(int(max_keys), k.shape[2] * (1 if tables is None else tables.shape[1]))
-    groups = R * nkv * -(-GT // 128)
-    splits = max(1, min(BLOCK_WORKGROUPS // max(1, groups), -(-max_keys // 128), 32))
+    splits, grouped = _block_plan(R * nkv, GT, max_keys)
     scratch = None
     if splits > 1:
         scratch = torch.empty((int(N.layers().jl_attn_block_scratch_floats(R, T, nkv, G, D, splits)),), dtype=torch.float32, device=q.device)
@@ -649,7 +660,7 @@ def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len
                     row_prompt=row_prompt.data_ptr() if tables is None else None, row_cand=row_cand.data_ptr() if ck is not None else None, tables=_ptr(tables), out=out.data_ptr(),
                     scratch=_ptr(scratch), table_ld=tables.stride(0) if tables is not None else 0, R=R, T=T, nkv=nkv, G=G, D=D, blocks=k.shape[0], page_size=k.shape[2],
                     table_cols=tables.shape[1] if tables is not None else 0, cand_rows=ck.shape[0] if ck is not None else 0, cand_max=ck.shape[2] if ck is not None else 0,
-                    max_keys=max_keys, splits=splits, scale=D ** -0.5 if scale is None else float(scale))
+                    max_keys=max_keys, splits=splits, grouped=grouped, scale=D ** -0.5 if scale is None else float(scale))
     N.check_layers(N.layers().jl_attn_block(C.byref(a), _stream(q.device)), "jl_attn_block")
     return out
 

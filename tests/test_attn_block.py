@@ -54,6 +54,38 @@ def test_block(monkeypatch, R, T, nkv, G, D, kv, lens, kind, wgs):
         assert err <= 4 * 2.0 ** -8 * max(1.0, want.abs().max().item() / 4), (r, err)
 
 
+@pytest.mark.parametrize("plan", [(1, 0), (3, 0), (1, 1), (2, 1), (5, 1)])      # shares of the keys, whether wavefronts take keys in groups
+@pytest.mark.parametrize("T,G,D,kv,scale,climb", [
+    (32, 2, 128, [0, 31, 32, 33, 95, 96, 97, 127, 128, 129, 640], None, 0.), (21, 3, 64, [5, 107, 108, 235, 236], None, 0.), (65, 1, 8, [0, 63, 700], None, 0.), (7, 18, 72, [300, 1, 511], -0.1, 0.),
+    (16, 4, 128, [64, 400], 0., 0.), (32, 2, 128, [900, 64, 33], None, 0.1), (32, 4, 64, [700, 257], None, -0.1),
+])
+def test_shares_and_groups(monkeypatch, plan, T, G, D, kv, scale, climb):
+    """Every form at the borders of tiles (32 and 64 keys, 64 and 128 rows) and of rounds (128 keys); scores that climb from key to key (or fall) pass every greatest one before them by a little."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, nkv, R = "cuda", 2, len(kv)
+    monkeypatch.setattr(LO, "_block_plan", lambda *a: plan)
+    g = torch.Generator(device=dev).manual_seed(T * D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    longest = max(kv) + T
+    q, k, v = rnd(R, nkv, G * T, D), rnd(R, nkv, longest, D), rnd(R, nkv, longest, D)
+    if climb:
+        q[..., 0], k[..., 0] = 16., (torch.arange(longest, device=dev) * climb).bfloat16() * D ** 0.5 / 16
+    lens = [T - r % 2 * (T // 3) for r in range(R)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    out = LO.attn_block(q, T, k, v, i32(kv), i32(lens), longest, i32(list(range(R))), scale=scale).double().view(R, T, nkv, G, D)
+    t, f = torch.arange(T, device=dev).view(T, 1), D ** -0.5 if scale is None else scale
+    for r in range(R):
+        n = kv[r] + lens[r]
+        kk, vv, j = k[r].double()[:, :n], v[r].double()[:, :n], torch.arange(n, device=dev).view(1, n)
+        s = (q[r].double() @ kk.transpose(1, 2).contiguous() * f).view(nkv, G, T, n)
+        p = torch.softmax(s.masked_fill((j >= kv[r]) & (j - kv[r] > t), float("-inf")), -1).view(nkv, G * T, n)
+        want, size = (x.view(nkv, G, T, D).permute(2, 0, 1, 3) for x in (p @ vv, p @ vv.abs()))
+        # weights are rounded to bfloat16 (half of a last place, 2^-7 of the number at most: 2^-8 of each; their sum is of the unrounded ones), the result once more; a score is off by a few
+        # 2^-24 of the greatest sum of its products
+        tol = 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 2.0 ** -18 * size * (1 + float(s.abs().max())) + 2.0 ** -16 * size
+        assert bool(((out[r] - want).abs() <= tol).all()), (r, float(((out[r] - want).abs() / tol).max()))
+
+
 @pytest.mark.parametrize("R,T,candidates", [(1, 1, False), (5, 33, True), (64, 32, True), (3, 200, False)])
 def test_slots(R, T, candidates):
     from jacobiforcing_amd import layer_ops as LO
