@@ -62,14 +62,16 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     const int R = 32 * wave + l32, ii = R / HF, hh = h0 + R % HF;
     const bool ok = R < TQ * HF && ii < cnt && hh < h_end;
     const int qi = i0 + ii, q_lo = chunk > 0 ? qi - qi % chunk : qi - window + 1;                 // the row's keys: q_lo .. qi
+    const bool capped = a.softcap > 0.f;
     ar_bf16x8 qf[KU / 2];
     {
+        const uint32_t sign = !capped && a.scale < 0.f ? 0x80008000u : 0u;      // scores are scaled behind their maximum: by a factor above zero
         const bf16_t *qp = (const bf16_t *)a.q + (int64_t)(row0 + ii) * a.q_ld + hh * D + 8 * hi;
 #pragma unroll
         for (int x = 0; x < KU / 2; ++x) {
             uint2 w[2] = {make_uint2(0, 0), make_uint2(0, 0)};
             if (ok && 16 * x + 8 * hi < D) { w[0] = *(const uint2 *)(qp + 16 * x); w[1] = *(const uint2 *)(qp + 16 * x + 4); }
-            qf[x] = __builtin_bit_cast(ar_bf16x8, make_uint4(w[0].x, w[0].y, w[1].x, w[1].y));
+            qf[x] = __builtin_bit_cast(ar_bf16x8, make_uint4(w[0].x ^ sign, w[0].y ^ sign, w[1].x ^ sign, w[1].y ^ sign));
         }
     }
     // scores are kept times log2(e): weights are 2 ** (s - max)
@@ -77,8 +79,7 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     float m_run = -INFINITY, l_run = 0.f;
     if (a.sink && ok) { m_run = a.sink[hh] * LOG2E; l_run = 1.f; }   // the sink: an extra score that attends to nothing
     if (hi) l_run = 0.f;                                            // each half-wavefront sums its own keys; the halves meet at the end
-    const bool capped = a.softcap > 0.f;
-    const float c2 = capped ? LOG2E : a.scale * LOG2E;
+    const float c2 = capped ? LOG2E : fmaxf(fabsf(a.scale * LOG2E), 1e-30f);
     ar_f32x16 acc[NDV];
 #pragma unroll
     for (int t = 0; t < NDV; ++t)
@@ -198,14 +199,8 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int kk = 32 * hf + 8 * (r >> 2) + 4 * hi + (r & 3);
-                        const float x = sc[hf][r] * c2;
-                        sc[hf][r] = kk >= first && kk <= last ? x : -INFINITY;
+                        sc[hf][r] = kk >= first && kk <= last ? sc[hf][r] : -INFINITY;
                     }
-            } else {
-#pragma unroll
-                for (int hf = 0; hf < HALVES; ++hf)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) sc[hf][r] *= c2;
             }
             float mx = sc[0][0];
 #pragma unroll
@@ -213,22 +208,23 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
 #pragma unroll
                 for (int r = hf == 0 ? 1 : 0; r < 16; ++r) mx = fmaxf(mx, sc[hf][r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run, mx);
-            const float m_sub = m_new > -INFINITY ? m_new : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);      // m_run = -inf: 0, and nothing has been accumulated yet
-            float sum = 0.f;
-#pragma unroll
-            for (int hf = 0; hf < HALVES; ++hf)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) { sc[hf][r] = __builtin_amdgcn_exp2f(sc[hf][r] - m_sub); sum += sc[hf][r]; }
-            l_run = l_run * alpha + sum;
-            m_run = m_new;
-            if (__any(alpha != 1.0f)) {                             // after the first tiles a row's maximum seldom moves
+            const float m_new = fmaxf(m_run, mx * c2);
+            if (__any(m_new - m_run > AR_SLACK)) {                  // seldom after the first tiles
+                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));      // m_run = -inf: 0, and nothing has been accumulated yet
+                m_run = m_new;
+                l_run *= alpha;
 #pragma unroll
                 for (int t = 0; t < NDV; ++t)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
             }
+            const float m_sub = m_run > -INFINITY ? m_run : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
+            float sum = 0.f;
+#pragma unroll
+            for (int hf = 0; hf < HALVES; ++hf)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { sc[hf][r] = __builtin_amdgcn_exp2f(fmaf(sc[hf][r], c2, -m_sub)); sum += sc[hf][r]; }
+            l_run += sum;
             const char *Vs = (const char *)(V_IN_K ? Ks : Ks + KT * KU);
             const int vk = 4 * hi + ((lane & 15) >> 2), vc8 = 8 * (lane & 1), vu = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);      // this lane's key, half unit and unit of a turned block
 #pragma unroll
