@@ -23,7 +23,7 @@ LAYER_GROUPS = {
     "layers": ["jl_error", "jl_norm", "jl_conv", "jl_headnorm", "jl_latent", "jl_attn_sweep", "jl_attn_rows", "jl_attn_f32", "jl_attn_talk", "jl_attn_block", "jl_attn", "jl_linear"],
     "layers_seq": ["jl_error", "jl_retention", "jl_delta", "jl_scan", "jl_moe"],
 }
-LAYERS_HEADERS = [CSRC / "layers" / "jl_common.h", CSRC / "layers" / "jl_attn.h", CSRC / "layers" / "jl_small.h", ROOT / "include" / "jf_layers.h"]
+LAYERS_HEADERS = [CSRC / "layers" / "jl_common.h", CSRC / "layers" / "jl_attn.h", CSRC / "layers" / "jl_small.h", CSRC / "layers" / "jl_split.h", ROOT / "include" / "jf_layers.h"]
 
 
 # the wrappers' host side (a CPython module on torch's C++ interface), beside the libraries that it calls

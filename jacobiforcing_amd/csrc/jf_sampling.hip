@@ -1180,6 +1180,9 @@ __device__ __forceinline__ uint32_t zn_pk_sub(uint32_t a, uint32_t b) {      // 
 __device__ __forceinline__ uint32_t zn_pk_min(uint32_t a, uint32_t b) {      // v_pk_min_u16
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(zn_u16x2, a), __builtin_bit_cast(zn_u16x2, b)));
 }
+__device__ __forceinline__ uint32_t zn_pk_max(uint32_t a, uint32_t b) {      // v_pk_max_i16: patterns of values from +0 on in the values' order, those below under all of them
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(zn_s16x2, a), __builtin_bit_cast(zn_s16x2, b)));
+}
 __device__ __forceinline__ uint32_t zn_pk_rotl1(uint32_t a) {                // each half rotated left by one: magnitude << 1 | sign
     const zn_u16x2 v = __builtin_bit_cast(zn_u16x2, a);
     return __builtin_bit_cast(uint32_t, (zn_u16x2)((v << (zn_u16x2){1, 1}) | (v >> (zn_u16x2){15, 15})));
@@ -1211,11 +1214,12 @@ __device__ __forceinline__ void rs_scaled_pk_from_vec(const RsRow &r, const u32x
 // What top-k / top-p make of the row, from its pattern counts.  FAST: the occupied patterns as a compact list in LDS, largest value
 // first — item i = occ[i] = key << 16 | count, its probability's bf16 bits in pc[i]; a thread owns `ipt` consecutive items.  !FAST:
 // the counters themselves, a thread owns 64 consecutive patterns (rows with more than FH_ITEMS occupied patterns, or a pattern that
-// occurs more than 65 535 times).  The stages are written once over "this thread's items" (any order) and "this thread's items,
+// occurs more than 65 535 times).  tops: the greatest pattern of every thread's eight tiles, or null (the tie pass then reads the row).  The stages are written once over "this thread's items" (any order) and "this thread's items,
 // largest value first".
+constexpr int ZN_MEMBERS = 256, ZN_SLOT_TILES = 8, ZN_SPARSE = 128;                            // tiles whose greatest value a thread keeps as one; threads that may read their vectors again alone
 template <bool FAST>
 __device__ __forceinline__ float fh_solve(FhShared &sh, const uint32_t *hist, const uint32_t *occ, uint16_t *pc, int n_occ, const RsRow &row, int64_t r,
-                                          int64_t V, const int64_t *draft_next, int top_k, double top_p, bool k_on, bool p_on, jf_rs_filter_row &rec) {
+                                          int64_t V, const int64_t *draft_next, int top_k, double top_p, bool k_on, bool p_on, jf_rs_filter_row &rec, const int16_t *tops) {
     constexpr int EPV = 8;
     const int tid = threadIdx.x;
     const float M = row.M;
@@ -1391,7 +1395,10 @@ __device__ __forceinline__ float fh_solve(FhShared &sh, const uint32_t *hist, co
         const int64_t ntiles = (V + TILE - 1) / TILE;
         __syncthreads();
         if (tid < FH_MAX_TILES) { sh.tileA[tid] = 0; sh.tileB[tid] = 0; }
+        if (tid < 2) sh.bi[2 + tid] = 0;
         __syncthreads();
+        bool sparse = false;                                                 // few threads hold members: their ids are in `members` (which takes the items' place), class A's, then class B's
+        int *members = FAST ? (int *)const_cast<uint32_t *>(occ) : nullptr;
         // class A: keys of the top-k cut group; class B: keys above the top-k cut whose y equals the top-p cut (a key range: y is monotone)
         const int a_lo = ka1, a_hi = kb1, b_lo = ka2, b_hi = kb2;
         auto classes = [&](const u32x4 vv, int64_t e0, uint32_t &ma, uint32_t &mb) {
@@ -1423,8 +1430,55 @@ __device__ __forceinline__ float fh_solve(FhShared &sh, const uint32_t *hist, co
 #pragma unroll
                 for (int k = 0; k < NB; ++k) { const int64_t e0 = (tb + k) * TILE + (int64_t)tid * EPV; if (tb + k < ntiles && e0 < V) dst[k] = rs_load_vec<JF_BF16>(row, e0); }
             };
-            if constexpr (FAST) load_batch(0, v);
-            for (int64_t t0 = 0; t0 < ntiles; t0 += NB) {
+            auto any_member = [&](const u32x4 vec) {
+                uint32_t pk[4], hit = 0u;
+                rs_scaled_pk_from_vec(row, vec, pk);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t key2 = zn_pk_key(pk[j]);
+                    if (rangeA) { const uint32_t d = zn_pk_sub(key2, aLo2); hit |= zn_pk_has_zero(zn_pk_min(d, aSp2) ^ d); }
+                    if (rangeB) { const uint32_t d = zn_pk_sub(key2, bLo2); hit |= zn_pk_has_zero(zn_pk_min(d, bSp2) ^ d); }
+                }
+                return hit != 0u;
+            };
+            // Members are values at or above the lower cut; where that is zero or more and few threads have one so large (the count pass kept the greatest of each thread's eight tiles),
+            // those threads read their eight vectors again and nobody else does.
+            int from = 0x10000;
+            if (rangeA && a_lo < from) from = a_lo;
+            if (rangeB && b_lo < from) from = b_lo;
+            uint32_t slots = 0u;
+            if constexpr (FAST) {
+                if (tops && from >= 0x8000) {                                // (workgroup-uniform; the key of a pattern without sign is the pattern + 0x8000)
+                    for (int sl = 0; sl * ZN_SLOT_TILES < (int)ntiles; ++sl) slots |= (int)tops[sl * TPB + tid] >= from - 0x8000 ? 1u << sl : 0u;
+                    sparse = __syncthreads_count(slots != 0u) <= ZN_SPARSE;
+                }
+                if (sparse)
+                    for (; slots; slots &= slots - 1u) {
+                        const int64_t t0 = (int64_t)(__ffs((int)slots) - 1) * ZN_SLOT_TILES;
+                        uint32_t held = 0u;
+#pragma unroll
+                        for (int half = 0; half < ZN_SLOT_TILES; half += NB) {
+                            load_batch(t0 + half, v);
+#pragma unroll
+                            for (int k = 0; k < NB; ++k) held |= t0 + half + k < ntiles && (t0 + half + k) * TILE + (int64_t)tid * EPV < V && any_member(v[k]) ? 1u << (half + k) : 0u;
+                        }
+                        for (; held; held &= held - 1u) {
+                            const int64_t tile = t0 + __ffs((int)held) - 1, e0 = tile * TILE + (int64_t)tid * EPV;
+                            uint32_t ma = 0u, mb = 0u;
+                            classes(rs_load_vec<JF_BF16>(row, e0), e0, ma, mb);
+                            if (!wantA) ma = 0u;
+                            if (!wantB) mb = 0u;
+                            if (ma) atomicAdd(&sh.tileA[tile], __popc(ma));
+                            if (mb) atomicAdd(&sh.tileB[tile], __popc(mb));
+                            for (uint32_t both = ma | mb; both; both &= both - 1u) {
+                                const int j = __ffs((int)both) - 1, of = ma >> j & 1u ? 0 : 1, at = atomicAdd(&sh.bi[2 + of], 1);
+                                if (at < ZN_MEMBERS) members[of * ZN_MEMBERS + at] = (int)e0 + j;
+                            }
+                        }
+                    }
+                else load_batch(0, v);
+            }
+            for (int64_t t0 = sparse ? ntiles : 0; t0 < ntiles; t0 += NB) {
                 if constexpr (FAST) {                                        // the next batch's loads, in front of this batch's arithmetic and its barrier
 #pragma unroll
                     for (int k = 0; k < NB; ++k) {
@@ -1437,15 +1491,7 @@ __device__ __forceinline__ float fh_solve(FhShared &sh, const uint32_t *hist, co
                     if (t0 + k >= ntiles) continue;                          // (workgroup-uniform)
                     const int64_t e0 = (t0 + k) * TILE + (int64_t)tid * EPV;
                     if (e0 >= V) continue;
-                    uint32_t pk[4], hit = 0u;
-                    rs_scaled_pk_from_vec(row, v[k], pk);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint32_t key2 = zn_pk_key(pk[j]);
-                        if (rangeA) { const uint32_t d = zn_pk_sub(key2, aLo2); hit |= zn_pk_has_zero(zn_pk_min(d, aSp2) ^ d); }
-                        if (rangeB) { const uint32_t d = zn_pk_sub(key2, bLo2); hit |= zn_pk_has_zero(zn_pk_min(d, bSp2) ^ d); }
-                    }
-                    if (__builtin_expect(hit != 0u, 0)) {
+                    if (__builtin_expect(any_member(v[k]), 0)) {
                         uint32_t ma = 0u, mb = 0u;
                         classes(v[k], e0, ma, mb);
                         if (ma && wantA) atomicAdd(&sh.tileA[t0 + k], __popc(ma));     // (members of a cut group are few: an add per lane that holds one)
@@ -1468,20 +1514,43 @@ __device__ __forceinline__ float fh_solve(FhShared &sh, const uint32_t *hist, co
         FH_STAMP(6);
         // the id of the c-th (1-based) member, in id order, of: class A ids (use_a, up to id a_max) and class B ids (use_b)
         auto nth = [&](long long c, bool use_a, int64_t a_max, bool use_b) -> int64_t {
-            if (tid == 0) {
-                long long before = 0;
-                sh.bi[1] = -1;
-                for (int tl = 0; tl < (int)ntiles; ++tl) {
-                    long long n = use_b ? sh.tileB[tl] : 0;
+            if constexpr (FAST) {
+                const int n_a = sh.bi[2], n_b = sh.bi[3];
+                if (sparse && n_a <= ZN_MEMBERS && n_b <= ZN_MEMBERS) {      // (workgroup-uniform) a member per thread: its place among the others
+                    const int i_a = use_a ? n_a : 0, i_b = use_b ? n_b : 0;
+                    if (tid == 0) sh.bl[1] = V - 1;
+                    __syncthreads();
+                    if (tid < i_a + i_b) {
+                        const int id = tid < i_a ? members[tid] : members[ZN_MEMBERS + tid - i_a];
+                        long long place = 1;
+                        for (int j = 0; j < i_a; ++j) place += members[j] < id && members[j] <= a_max ? 1 : 0;
+                        for (int j = 0; j < i_b; ++j) place += members[ZN_MEMBERS + j] < id ? 1 : 0;
+                        if (place == c && (tid >= i_a || id <= a_max)) sh.bl[1] = id;
+                    }
+                    __syncthreads();
+                    const int64_t hit = sh.bl[1];
+                    __syncthreads();
+                    return hit;
+                }
+            }
+            if (tid < 64) {                                                  // a tile per lane (FH_MAX_TILES of them at most)
+                int n = 0;
+                if (tid < (int)ntiles) {
+                    if (use_b) n = sh.tileB[tid];
                     if (use_a) {
-                        const int64_t t_lo = (int64_t)tl * TILE;
+                        const int64_t t_lo = (int64_t)tid * TILE;
                         int64_t t_hi = t_lo + TILE - 1;
                         if (t_hi > V - 1) t_hi = V - 1;
-                        n += a_max >= t_hi ? sh.tileA[tl] : a_max >= t_lo ? sh.bl[2] : 0;
+                        n += a_max >= t_hi ? sh.tileA[tid] : a_max >= t_lo ? (int)sh.bl[2] : 0;
                     }
-                    if (before < c && c <= before + n) { sh.bi[1] = tl; sh.bl[0] = c - before; break; }
-                    before += n;
                 }
+                int upto = n;
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) { const int o = __shfl_up(upto, off, 64); if (tid >= off) upto += o; }
+                const bool here = upto - n < c && c <= upto;
+                const unsigned long long found = __ballot(here);
+                if (here) sh.bl[0] = c - (upto - n);
+                if (tid == 0) sh.bi[1] = found ? __ffsll(found) - 1 : -1;
             }
             __syncthreads();
             const int tl = sh.bi[1];
@@ -1604,7 +1673,7 @@ __device__ __forceinline__ void fh_hist_row(FhShared &sh, unsigned char *fh_dyn,
             if (w >> 16) occ[(int)ce + __popcll(b0 + 2u < 64u ? occ_mask >> (b0 + 2u) : 0ull)] = ((kbase + b0 + 1u) << 16) | (w >> 16);
         }
         __syncthreads();
-        pd = fh_solve<true>(sh, hist, occ, pc, (int)n_occ, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec);
+        pd = fh_solve<true>(sh, hist, occ, pc, (int)n_occ, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec, nullptr);
     } else {
         if (wrapped) {                                                       // count again, noticing the wraps; then once more with side counters for those patterns
             for (int w = tid; w < FH_WORDS; w += FH_TPB) hist[w] = 0u;
@@ -1619,7 +1688,7 @@ __device__ __forceinline__ void fh_hist_row(FhShared &sh, unsigned char *fh_dyn,
             __syncthreads();
             fh_count_row<true>(sh, hist, row);
         }
-        pd = fh_solve<false>(sh, hist, occ, pc, 0, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec);
+        pd = fh_solve<false>(sh, hist, occ, pc, 0, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec, nullptr);
     }
     finish(pd);
 }
@@ -1639,8 +1708,8 @@ __global__ __launch_bounds__(FH_TPB, 1) void rs_filter_hist_kernel(const void *l
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same record from 32 KB of counters instead of 128 KB, so that a CU holds THREE rows at once and one row's solving overlaps
-// the others' streaming.  Between M - 104 and M the scaled logits of a row span ~34 000 bf16 patterns, but nearly all of those are
+// The same record from 32 KB of counters instead of 128 KB, so that a CU holds several rows at once and one row's solving overlaps
+// another's streaming.  Between M - 104 and M the scaled logits of a row span ~34 000 bf16 patterns, but nearly all of those are
 // the patterns of magnitudes below 2^-16 on either side of zero, which a row of 152 064 logits visits a handful of times: the table
 // holds the patterns with 2^-16 <= |x| < 2^16 (32 binades x 128 x 2 signs = 8 192 32-bit counters, the two signs of a magnitude
 // side by side), a row's smaller magnitudes go to a list of 64 keys (sorted and counted by 64 threads), and a row that does not
@@ -1655,18 +1724,20 @@ __global__ __launch_bounds__(FH_TPB, 1) void rs_filter_hist_kernel(const void *l
 // with an id outside the table (one in ~10^4) takes the slow path per element, every other one is eight plain LDS adds.  Nothing is
 // compared with M - 104 per element: patterns below it are dropped when the list is built (the slot's value says so), and since the
 // counters are 32 bits wide there is no checksum for wrapped counters either.
+//
+// What bounds it: up to 512 rows the chain of one row (35 us of counting at 496 rows, whose bytes take 29, then 20 of reductions, one after another, then the tie pass), beyond them HBM.  The tie pass read
+// the row again, on average half of it.  Now the count pass keeps the greatest pattern of every thread's eight tiles (one packed maximum per word), and only threads that hold a value at or above the
+// lower cut read their eight vectors again and write their members' ids to a list.  Two rows per CU: the 85 registers of three spilled 193, which cost more than the third row gave.  us per call, rows of
+// 152 064, top-k 50 and top-p 0.9, before / now: 31 rows 74 / 59, 124 81 / 62, 496 104 / 81, 620 117 / 113, 992 163 / 142, 1984 279 / 250; top-p alone 98 / 77, 496 rows 133 / 106, 1984 367 / 326.
 // ------------------------------------------------------------------------------------------------
-#ifndef JF_ZN_WAVES
-#define JF_ZN_WAVES 6                       // waves per SIMD asked of the compiler: 6 = three rows per CU (<= 85 VGPRs), 4 = two
-#endif
 constexpr int ZN_TPB = 512, ZN_SLOTS = 8192, ZN_TINY = 64, ZN_EXP_LO = 111, ZN_EXP_HI = 142;
 constexpr uint32_t ZN_LO16 = (uint32_t)ZN_EXP_LO << 7;                       // first magnitude pattern of the table
-constexpr unsigned ZN_LDS = (ZN_SLOTS + 4) * 4;                               // the counters; the list of occupied patterns and their probabilities re-use them
+constexpr unsigned ZN_LDS = (ZN_SLOTS + 4) * 4 + FH_MAX_TILES / ZN_SLOT_TILES * ZN_TPB * 2;      // the counters (the list of occupied patterns and their probabilities re-use them); the threads' greatest patterns
 static_assert(FH_ITEMS * 4 + FH_ITEMS * 2 <= ZN_SLOTS * 4, "occ + pc must fit the counters they replace");
-__global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(const void *logits, int64_t R, int64_t V, int64_t row_stride, const int64_t *draft_next,
+__global__ __launch_bounds__(ZN_TPB, 4) void rs_filter_zone_kernel(const void *logits, int64_t R, int64_t V, int64_t row_stride, const int64_t *draft_next,
                                                                     float t, int top_k, double top_p, jf_rs_filter_row *filt, float *p_draft,
                                                                     float *row_max, float *row_sumexp) {
-    constexpr int EPV = 8, NB = 4;                                          // (four loads in flight per thread x three workgroups per CU)
+    constexpr int EPV = 8, NB = 4;                                          // (four loads in flight per thread x two workgroups per CU)
     __shared__ FhShared sh;
     __shared__ uint32_t s_tiny[ZN_TINY];
     __shared__ int s_ntiny, s_retry, s_ndist;
@@ -1674,6 +1745,7 @@ __global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(con
     uint32_t *table = (uint32_t *)zn_dyn;                                   // [ZN_SLOTS] counter of magnitude LO16 + (i >> 1), sign i & 1
     uint32_t *occ = table;                                                   // [FH_ITEMS] the list, once every counter has been read
     uint16_t *pc = (uint16_t *)(occ + FH_ITEMS);
+    int16_t *tops = (int16_t *)(table + ZN_SLOTS + 4);                       // [8][512] the greatest pattern of a thread's eight tiles (zn_pk_max)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t r = blockIdx.x;
     const float M = row_max[r];
@@ -1699,7 +1771,10 @@ __global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(con
         u32x4 v[NB], vn[NB];
 #pragma unroll
         for (int k = 0; k < NB; ++k) { const int64_t e0 = (int64_t)tid * EPV + (int64_t)k * ZN_TPB * EPV; if (e0 < V) v[k] = rs_load_vec<JF_BF16>(row, e0); }
-        for (int64_t b0 = (int64_t)tid * EPV; b0 < V; b0 += step) {
+        static_assert(ZN_SLOT_TILES == 2 * NB, "a slot is two rounds");
+        uint32_t top = 0x80008000u;
+        int round = 0;
+        for (int64_t b0 = (int64_t)tid * EPV; b0 < V; b0 += step, ++round) {
 #pragma unroll
             for (int k = 0; k < NB; ++k) { const int64_t e0 = b0 + step + (int64_t)k * ZN_TPB * EPV; if (e0 < V) vn[k] = rs_load_vec<JF_BF16>(row, e0); }   // the next round's loads, in front of this round's arithmetic
 #pragma unroll
@@ -1708,6 +1783,7 @@ __global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(con
                 if (e0 >= V) continue;
                 uint32_t pk[4], d[4];
                 rs_scaled_pk_from_vec(row, v[k], pk);
+                top = zn_pk_max(zn_pk_max(top, zn_pk_max(pk[0], pk[1])), zn_pk_max(pk[2], pk[3]));
 #pragma unroll
                 for (int j = 0; j < 4; ++j) d[j] = zn_pk_sub(zn_pk_rotl1(pk[j]), (2u * ZN_LO16) * 0x00010001u);
                 if (__builtin_expect(((d[0] | d[1] | d[2] | d[3]) & 0xE000E000u) == 0u, 1)) {      // all eight ids inside the table
@@ -1728,7 +1804,11 @@ __global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(con
             }
 #pragma unroll
             for (int k = 0; k < NB; ++k) v[k] = vn[k];
+            const int16_t t_lo = (int16_t)(top & 0xFFFFu), t_hi = (int16_t)(top >> 16);
+            tops[(round >> 1) * ZN_TPB + tid] = t_lo > t_hi ? t_lo : t_hi;
+            if (round & 1) top = 0x80008000u;
         }
+        for (int sl = (round + 1) >> 1; sl < FH_MAX_TILES / ZN_SLOT_TILES; ++sl) tops[sl * ZN_TPB + tid] = -0x8000;
     }
     __syncthreads();
     FH_STAMP(10);
@@ -1797,7 +1877,7 @@ __global__ __launch_bounds__(ZN_TPB, JF_ZN_WAVES) void rs_filter_zone_kernel(con
     if (my_pos >= 0) occ[n_pos + my_pos] = (my_tiny << 16) | my_cnt;
     __syncthreads();
     FH_STAMP(11);
-    const float pd = fh_solve<true>(sh, nullptr, occ, pc, n_occ, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec);
+    const float pd = fh_solve<true>(sh, nullptr, occ, pc, n_occ, row, r, V, draft_next, top_k, top_p, k_on, p_on, rec, tops);
     if (tid == 0) { filt[r] = rec; p_draft[r] = pd; row_max[r] = INFINITY; row_sumexp[r] = RS_PROB_ROW; }
 }
 

@@ -798,6 +798,25 @@ def test_rs_filter_bf16_rows_that_leave_the_fast_path(shape, top_k, top_p):
 
 
 @GPU
+@pytest.mark.parametrize("V", [152064, 8191, 33000])
+@pytest.mark.parametrize("top_k,top_p,members,stride,above", [(7, 0.0, 9, 4096, 3.0), (3, 0.9, 40, 513, 0.0), (100, 0.0, 128, 8, 3.0), (100, 0.0, 129, 8, 3.0), (200, 0.3, 256, 1, 3.0), (250, 0.99, 257, 1, 3.0),
+                                                              (64, 0.9, 300, 3, 0.0), (5, 0.0, 8, 1000, -9.0), (0, 0.5, 600, 4, 3.0), (0, 0.2, 30, 32768, 3.0)])
+def test_rs_filter_members_of_a_cut_group_in_few_threads(V, top_k, top_p, members, stride, above):
+    """Ids of one value at the cut, a vector of eight, a tile of 4 096 or eight tiles apart: the threads that hold them list them (up to 128 threads, 256 ids of a class), more of them are counted by
+    tiles; with values above them or none (then the top-k group's kept ids are the top-p group's), and cuts below zero.  Bit for bit against the oracle, T = 0.8."""
+    g = torch.Generator().manual_seed(V + members)
+    x = torch.randn(2, V, generator=g) - 14.0
+    at = (torch.arange(members) * stride + 5) % V
+    x[0, at], x[1, V - 1 - at] = above, above
+    if above > 0:
+        x[:, torch.randperm(V, generator=g)[:3]] = above + 0.5
+    x = x.to(torch.bfloat16)
+    got = _filter_rows(x.cuda(), 0.8, top_k, top_p)
+    want = O.target_probs(x.float().numpy(), 0.8, "bf16", top_k or None, top_p or None)
+    assert np.array_equal(got, want), [(np.flatnonzero(got[r] != want[r])[:5].tolist(), int((got[r] > 0).sum()), int((want[r] > 0).sum())) for r in range(2)]
+
+
+@GPU
 @pytest.mark.parametrize("top_k,top_p", [(50, 0.0), (0, 0.9), (40, 0.95)], ids=["k50", "p09", "k40_p095"])
 @pytest.mark.parametrize("shape", ["below_the_exp_cut", "partly_below_the_exp_cut", "tiny_magnitudes", "zeros_of_both_signs", "huge_without_mass",
                                    "huge_with_mass", "ragged_unaligned"])
