@@ -735,15 +735,15 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
 
 
 def retention_pieces_from(counts: Sequence[int], H: int, D: int) -> int:
-    """From how many tokens on the requests of a step run in pieces, the others in the scan behind them (0: all in the scan).  A round of pieces (one workgroup per CU) takes 27 us at
-    128 x 128, 19 at 64 x 64, however few tokens they hold, and with single tokens beside them about twice that; the scan 9 and 0.75 us per token of its longest portion.  The line was drawn when
-    the scan's threads kept whole columns (8.5 and 5.3 us per token): it is right where portions are long or all are short, and lies low for portions of 8 to 30 tokens.  us, scan of all / all in
-    pieces / this rule: 8 heads of 128, 8 tokens 13 / 27 / 27, 32 32 / 30 / 30, 8 and 250 x 1 41 / 323 / 41, 777 + 300 and 30 x 1 166 / 100 / 70, 100 x 8 36 / 153 / 36, 100 x 16 53 / 158 / 158;
-    32 heads, 8 and 30 x 1 23 / 163 / 52, 40 + 10 and 60 x 1 52 / 322 / 73, 10 x 10 and 60 x 1 50 / 356 / 50; 16 heads of 64, 200 x 20 70 / 253 / 70, 700, 40 x 10 and 40 x 1 118 / 129 / 100."""
+    """From how many tokens on the requests of a step run in pieces, the others in the scan behind them (0: all in the scan).  Pieces of up to 32 tokens take 17 us at 128 x 128 and 30 for each
+    256 heads of portions, the scan 6 and 0.75 per token of its longest portion, with more than 256 heads as much more; so all go to the scan where the longest portion is below a line that rises
+    with the heads.  us, scan / pieces, 8 heads of 128: 8 tokens 12 / 17, 16 19 / 17, 8 x 16 19 / 23, 8 x 24 25 / 24, 16 x 24 26 / 32, 16 x 32 32 / 33, 32 x 32 37 / 45, 32 x 48 52 / 52, 64 x 48
+    67 / 83, 128 x 64 159 / 157; 8 heads of 64: 16 14 / 13, 32 x 16 15 / 20, 32 x 32 25 / 21, 128 x 32 34 / 54, 128 x 64 68 / 74.  With single tokens beside, scan / pieces / both: 8 heads of 128,
+    777 + 300 and 30 x 1 167 / 73 / 56, 8 x 16 and 32 x 1 24 / 53 / 34, 32 x 64 and 32 x 1 72 / 84 / 63; 16 heads of 64, 700, 40 x 10 and 40 x 1 121 / 78 / 69."""
     long = sum(c >= RETENTION_PIECES_FROM for c in counts)
     rounds = -(-long * H // 256)
     least = max(RETENTION_PIECES_FROM, min(4 * rounds, 16) if D > 64 else min(3 * rounds, 48), 3 + (len(counts) - long) * H // 230)
-    if max(counts) < least:
+    if max(counts) < max(least, min(10 + long * H // 6, 64) if D > 64 else min(14 + long * H // 20, 72)):
         return 0
     return 1 if len(counts) * H < 256 else least                     # single tokens beside them where CUs are free: a launch less
 
