@@ -17,9 +17,6 @@ typedef __attribute__((address_space(3))) ar_s16x4 ar_lds_s16x4;
 template <int U> __device__ __forceinline__ int ar_key_unit(int r, int u) { return U % 16 == 0 ? u ^ (r & 15) : u ^ ((r >> 1) & 7); }
 template <int U> __device__ __forceinline__ int ar_value_unit(int r, int u) { return U == 16 ? u ^ ((r & 3) << 2) : u ^ ((r & 2) << 1); }
 
-// The sums so far are scaled when a row's maximum has grown by more than this power of two since the last time, not whenever it has grown: of 32 rows one has in nearly every tile.  Weights then reach
-// 2 ** 8 instead of 1, with as many digits, and what is divided by their sum is the same.
-constexpr float AR_SLACK = 8.f;
 constexpr int AR_ROWS = 128;          // (query, head) rows of a tile of the wide form
 
 // tiles and groups (``hb`` per key head) lie along one axis of the grid: up to 2 ** 32 threads of workgroups of 256

@@ -22,6 +22,7 @@ constexpr int AR_THREADS = 256;
 //   1 x 8192 tokens, the same heads                        1728 -> 434 us (633 TFLOP/s)
 //   4 x 2048 tokens, 16 heads of 192 / 128 apart           806 -> 180 us (479 TFLOP/s)
 //   4 x 2048 tokens, 8 heads of 128 over 2, window 1024    180 -> 66 us
+// Scores scaled in the exponent's multiply-add behind their maximum (queries take a negative scale's sign) instead of one by one: the first 129 -> 124, the second 393 -> 383.
 
 constexpr int ar_tile_keys(int KU) { return KU <= 16 ? 64 : 32; }
 constexpr size_t ar_lds_bytes(int KU, int VU) { return 2 * (size_t)ar_tile_keys(KU) * (KU + VU) * 16 + 2 * ar_tile_keys(KU) * 4; }
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
                 for (int r = hf == 0 ? 1 : 0; r < 16; ++r) mx = fmaxf(mx, sc[hf][r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = fmaxf(m_run, mx * c2);
-            if (__any(m_new - m_run > AR_SLACK)) {                  // seldom after the first tiles
+            if (__any(m_new > m_run)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
                 const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));      // m_run = -inf: 0, and nothing has been accumulated yet
                 m_run = m_new;
                 l_run *= alpha;

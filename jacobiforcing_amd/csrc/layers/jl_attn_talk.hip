@@ -199,21 +199,19 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
 #pragma unroll
             for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run, mx);
-            if (__any(m_new - m_run > AR_SLACK)) {                  // seldom after the first tiles
-                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));      // m_run = -inf: 0, and nothing has been accumulated yet
-                m_run = m_new;
-                l_run *= alpha;
+            const float m_new = fmaxf(m_run, mx), m_sub = m_new > -INFINITY ? m_new : 0.f;      // a row that has seen no key yet: all weights are 2 ** -inf
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { sc[r] = __builtin_amdgcn_exp2f(sc[r] - m_sub); sum += sc[r]; }
+            l_run = l_run * alpha + sum;
+            m_run = m_new;
+            if (__any(alpha != 1.0f)) {                             // after the first tiles a row's maximum seldom moves
 #pragma unroll
                 for (int y = 0; y < NDV; ++y)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[y][r] *= alpha;
             }
-            const float m_sub = m_run > -INFINITY ? m_run : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
-            float sum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) { sc[r] = __builtin_amdgcn_exp2f(sc[r] - m_sub); sum += sc[r]; }
-            l_run += sum;
             const char *Vs = (const char *)(Ks + KT * KU);
             const int vk = 4 * hi + ((lane & 15) >> 2), vc8 = 8 * (lane & 1), vu = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);      // this lane's key, half unit and unit of a turned block
 #pragma unroll

@@ -625,9 +625,9 @@ def block_slots(positions: torch.Tensor, T: int, row_prompt: torch.Tensor, row_c
 
 def _block_plan(heads: int, GT: int, max_keys: int):
     """(shares of the keys, whether a workgroup's wavefronts take keys in groups) for ``heads`` (row, key head) pairs of GT (head, token) rows.  Groups, one workgroup of 64 rows per CU, where
-    those fit the chip at once; us with / without, 8 heads of 128 over 2, 32 tokens, context 512: 64 rows (256 workgroups) 20.0 / 27.1, 96 rows 35.8 / 27.6.  A share more costs its sums' way
-    through memory, by the rows, and a launch: one row, context 500 / 1000 / 4000 / 16000: 2, 4, 8 and 16 shares are the fastest; 32 rows, context 512: one 18.5, two 21.6, context 2000: 43.0
-    and 32.9.  Without groups, 96 rows: one share / two at context 512 27.6 / 32.2, 1000 50.0 / 50.6, 2000 79.8 / 69.9."""
+    those fit the chip at once; us with / without, 8 heads of 128 over 2, 32 tokens, context 512: 64 rows (256 workgroups) 20.6 / 27.4, 96 rows 37.1 / 28.9.  A share more costs its sums' way
+    through memory, by the rows, and a launch: one row, context 500 / 1000 / 4000 / 16000: 2, 4, 8 and 16 shares are the fastest; 32 rows, context 512: one 19.0, two 21.6, context 2000: 44.1
+    and 33.9.  Without groups, 96 rows: one share / two at context 512 28.9 / 33.3, 1000 50.1 / 52.3, 2000 83.6 / 71.1."""
     units = max(1, heads * -(-GT // 64))
     if units <= 256:
         return max(1, min(256 // units, math.isqrt(max_keys // (64 + 2 * units)))), 1
