@@ -1287,7 +1287,7 @@ def latent_attention(q: torch.Tensor, pool: torch.Tensor, w_ukv: torch.Tensor, w
 
     def over_latent(q, batch, gate):
         m = q.shape[0]
-        if latent_heads(m, H, D, R, Dv, dt) and attn_sweep_tile_rows(dt, H, 1, R + rd, R, pool, pool[:, :R]):
+        if latent_heads(m, H, D, R, Dv, dt) and w_uk.shape == (H, D, R) and w_uv.shape == (H, R, Dv) and attn_sweep_tile_rows(dt, H, 1, R + rd, R, pool, pool[:, :R]):
             qf = (_H or _host()).latent_heads(q, w_uk, D + rd, rd, None, rot_dims, batch.N, batch.max_pos, batch.pos, cos, sin, pairing)
             if qf is not NotImplemented:
                 o = attn_sweep(qf, pool, pool[:, :R], batch, H, 1, R + rd, R, scale, window, sink=sink, gate=gate if gate_per_head else None, gate_per_head=gate_per_head)

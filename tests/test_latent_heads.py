@@ -76,3 +76,17 @@ def test_attention_takes_them_and_agrees(monkeypatch):
         assert got.shape == want.shape and (got.double() - want.double()).abs().max() <= 3 * 2.0 ** -8 * want.double().abs().max()
     with pytest.raises(ValueError):
         run(rnd(5, H * Dv + 1).bfloat16())
+
+
+@pytest.mark.parametrize("uk,uv", [((4, 56, 128), (4, 128, 64)), ((4, 8, 128), (4, 128, 64)), ((4, 72, 128), (4, 128, 64)), ((4, 64, 128), (4, 120, 64)), ((4, 64, 128), (4, 136, 64)),
+                                   ((4, 64, 120), (4, 128, 64)), ((3, 64, 128), (4, 128, 64))])
+def test_up_projections_of_other_sizes_are_refused(uk, uv):
+    """Up-projections whose depths are not the heads' are an error, also where they would fit the heads' columns, and whichever products the rule names."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, D, R, rd, Dv = "cuda", 4, 64, 128, 32, 64
+    assert LO.latent_heads(3, H, D, R, Dv, torch.bfloat16)
+    batch = LO.RaggedBatch.build([1, 1, 1], [70, 20, 0], [0, 1, 2], [[0, 1], [2], [3]], 64, dev)
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    cos = torch.zeros(80, rd // 2, device=dev)
+    with pytest.raises((RuntimeError, ValueError)):
+        LO.latent_attention(z(3, H * (D + rd)), z(256, R + rd), z(H * (D + Dv), R), z(*uk), z(*uv), batch, H, D, R, rd, Dv, rd, cos, cos, 0, 0.1, 0)
