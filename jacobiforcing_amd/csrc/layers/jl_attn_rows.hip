@@ -210,16 +210,16 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
                 for (int r = hf == 0 ? 1 : 0; r < 16; ++r) mx = fmaxf(mx, sc[hf][r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = fmaxf(m_run, mx * c2);
-            if (__any(m_new > m_run)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
-                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));      // m_run = -inf: 0, and nothing has been accumulated yet
-                m_run = m_new;
+            const float m_sub = m_new > -INFINITY ? m_new : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);      // m_run = -inf: 0, and nothing has been accumulated yet; none where the sink is NaN or infinite, and so the row
+            m_run = m_new;
+            if (__any(alpha != 1.0f)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
                 l_run *= alpha;
 #pragma unroll
                 for (int t = 0; t < NDV; ++t)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
             }
-            const float m_sub = m_run > -INFINITY ? m_run : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
             float sum = 0.f;
 #pragma unroll
             for (int hf = 0; hf < HALVES; ++hf)

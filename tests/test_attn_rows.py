@@ -172,3 +172,36 @@ def test_more_tiles_than_a_short_grid_axis_holds(dtype, single):
         return out
 
     assert torch.equal(run(0, n), torch.cat([run(0, half), run(half, n)]))
+
+
+@pytest.mark.parametrize("built", [False, True])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+def test_sinks_that_are_not_finite(monkeypatch, built, value):
+    """A sink that is not a number, or infinite, leaves its head's outputs none; one at minus infinity takes nothing; other heads' outputs are what they were, bit for bit.  On built keys a
+    wavefront's rows are all of one head, on the pools' of several."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, G, D, R, rd = "cuda", 16, 4, 64, 128, 32
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    counts, starts, pages = [1100, 131], [0, 37], [list(range(18)), list(range(18, 21))]
+    batch = LO.RaggedBatch.build(counts, starts, [0, 1], pages, 64, dev)
+    q, pool, n = rnd(1231, H * (D + (rd if built else 0))), rnd(21 * 64, R + rd if built else G * D), 1231
+    v, uk, uv = rnd(21 * 64, G * D), rnd(H, D, R), rnd(H, R, D)
+    monkeypatch.setattr(LO, "_latent_built_requests", lambda *a: [0, 1])
+
+    def run(sink):
+        if built:
+            return LO.latent_attention(q.clone(), pool, torch.cat([uk.reshape(H * D, R), uv.transpose(1, 2).reshape(H * D, R)]).contiguous(), uk, uv, batch, H, D, R, rd, D, 0, None, None, 0, 0.02, 0, sink=sink)
+        out = LO.attn_sweep(q, pool, v, batch, H, G, D, D, 0.125, 0, sink=sink)
+        assert ("longest first", 32, None) in batch._tiles, "the 128-row form did not run"
+        return out
+    sink = torch.randn(H, generator=g, device=dev)
+    want, sink[5] = run(sink).view(n, H, D), value
+    got = run(sink).view(n, H, D)
+    if value == float("-inf"):
+        sink[5] = -1e30
+        assert torch.equal(got[:, 5], run(sink).view(n, H, D)[:, 5]) and bool(got.isfinite().all())
+    else:
+        assert bool(got[:, 5].isnan().all())
+    got[:, 5] = want[:, 5]
+    assert torch.equal(got, want)
