@@ -163,6 +163,7 @@ CALL(linear, 4)
          starts16(*w) && w->device() == x->device());
     NEED(!bias || (bias->scalar_type() == w->scalar_type() && bias->dim() == 1 && bias->size(0) == o && bias->is_contiguous() && bias->device() == x->device()));
     NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad() || (bias && bias->requires_grad()))));
+    NEED(!x->_fw_grad(0).defined() && !w->_fw_grad(0).defined() && !(bias && bias->_fw_grad(0).defined()));      // forward-mode tangents
     NEED(small || split || n * ld * size < (int64_t)1 << 32);
     const int mode = typed ? JL_LINEAR_SAME : as_float ? JL_LINEAR_FLOAT : JL_LINEAR_ROUNDED_FLOAT;
     Tensor out = make({n, o}, typed ? x->scalar_type() : at::kFloat, *x);

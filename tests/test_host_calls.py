@@ -131,3 +131,70 @@ def test_refused_as_before():
     with Mode():
         LO.add_rmsnorm(x.clone(), None, None, w, 1e-5, torch.float32)
     assert torch.empty in seen                                                               # a mode that watches calls still sees the wrapper's
+
+
+@pytest.mark.parametrize("n", [4, 200, 640])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_linear_of_tensors_without_memory(n, dtype):
+    """Fake tensors are answered by their shape, whatever launch the sizes would go to."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from jacobiforcing_amd import layer_ops as LO
+    with FakeTensorMode():
+        x, w, b = (torch.empty(*s, dtype=dtype, device="cuda") for s in ((n, 64), (2500, 64), (2500,)))
+        for bias in (None, b):
+            for float_out in (None, True, False):
+                if float_out and dtype != torch.float32:
+                    continue                                                                  # torch's product with a type of its own for the result has no fake form on every version
+                y = LO.linear(x, w, bias, float_out)
+                assert y.shape == (n, 2500) and y.dtype == (dtype if float_out is None else torch.float32) and y.is_cuda
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [4, 640])
+def test_linear_lets_transforms_and_modes_pass(n):
+    """Forward-mode tangents, vmap, and modes and subclasses that see the library's call: as they were without launches; a default device changes nothing."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from jacobiforcing_amd import layer_ops as LO
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, w, b, t, u = rnd(n, 64), rnd(2500, 64), rnd(2500), rnd(n, 64), rnd(2500, 64)
+    assert LO.linear_split(n, 64, 2500) == (n == 640) and LO.linear_small(n, 64, 2500, 4) == (n == 4)
+    close = lambda a, c: torch.allclose(a, c, rtol=1e-4, atol=1e-4)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        for args, want in (((torch.autograd.forward_ad.make_dual(x, t), w, b), t @ w.T), ((x, torch.autograd.forward_ad.make_dual(w, u), b), x @ u.T)):
+            y, tangent = torch.autograd.forward_ad.unpack_dual(LO.linear(*args))
+            assert tangent is not None and close(tangent, want) and close(y, x @ w.T + b)
+    many = rnd(3, n, 64)
+    assert close(torch.vmap(lambda r: LO.linear(r, w, b))(many), many @ w.T + b)
+    seen = []
+
+    class Functions(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Operations(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Kind(torch.Tensor):
+        pass
+    with Functions():
+        LO.linear(x, w, b)
+    assert torch.nn.functional.linear in seen
+    seen.clear()
+    with Operations():
+        LO.linear(x, w, b)
+    assert any("addmm" in str(f) or "linear" in str(f) for f in seen)
+    assert type(LO.linear(x.as_subclass(Kind), w, b)) is Kind
+    want = LO.linear(x, w, b)
+    with torch.device(dev):
+        assert torch.equal(LO.linear(x, w, b), want)                                          # the same launch
+    calls = []
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(LO.F, "linear", lambda *a: calls.append(a))
+        with torch.device(dev):
+            LO.linear(x, w, b)
+    assert not calls
