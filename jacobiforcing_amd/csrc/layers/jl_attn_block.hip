@@ -44,17 +44,17 @@ __global__ __launch_bounds__(64 * WM * KG, KG == 1 ? 2 : 1) void attn_block_kern
     const int R = 32 * WM * rt + 32 * wm + l32, t = R % T;            // this lane's row: head R / T of the group, token t; both half-wavefronts hold it
     const bool ok = R < GT;
     const int last = kv + (t + 1 < len ? t + 1 : len) - 1 < n_keys - 1 ? kv + (t + 1 < len ? t + 1 : len) - 1 : n_keys - 1;      // its last key
+    const bool scaled = !ar_one_by_one(a.scale);
     ar_bf16x8 qf[KU / 2];
 #pragma unroll
     for (int x = 0; x < KU / 2; ++x) {
         ar_s16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
         if (ok && 16 * x + 8 * hi < D) w = *(const ar_s16x8 *)((const bf16_t *)a.q + (((int64_t)r * a.nkv + c) * GT + R) * D + 16 * x + 8 * hi);
-        if (a.scale < 0.f) w ^= (short)0x8000;                      // scores are scaled behind their maximum: by a factor above zero
+        if (scaled && a.scale < 0.f) w ^= (short)0x8000;
         qf[x] = __builtin_bit_cast(ar_bf16x8, w);
     }
-    constexpr float LOG2E = 1.44269504088896341f;
-    const float c2 = fmaxf(fabsf(a.scale * LOG2E), 1e-30f);
-    float m_run = -INFINITY, l_run = 0.f;
+    const float c2 = scaled ? fabsf(a.scale * AR_LOG2E) : AR_LOG2E;
+    float m_run = -INFINITY, l_run = 0.f, entry = -INFINITY;
     ar_f32x16 acc[NDV];
 #pragma unroll
     for (int y = 0; y < NDV; ++y)
@@ -131,6 +131,11 @@ __global__ __launch_bounds__(64 * WM * KG, KG == 1 ? 2 : 1) void attn_block_kern
                     const int row = 32 * hf + l32;
                     sc[hf] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ar_bf16x8, Ks[row * KU + ar_key_unit<KU>(row, 2 * x + hi)]), qf[x], sc[hf], 0, 0, 0);
                 }
+            if (!scaled)
+#pragma unroll
+                for (int hf = 0; hf < NHF; ++hf)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sc[hf][i] *= a.scale;
             if (!wave_full || j0 + KT > kv) {                       // not committed keys only, which every row sees
                 const int upto = ok ? last - j0 : -1;
 #pragma unroll
@@ -145,9 +150,12 @@ __global__ __launch_bounds__(64 * WM * KG, KG == 1 ? 2 : 1) void attn_block_kern
                 for (int i = hf == 0 ? 1 : 0; i < 16; ++i) mx = fmaxf(mx, sc[hf][i]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = fmaxf(m_run, mx * c2);
-            if (__any(m_new > m_run)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
+            float factor = c2;
+            if (__any(m_new > entry)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
                 const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));
                 m_run = m_new;
+                entry = ar_entry(m_run);
+                factor = ar_factor(sc, c2, m_run);
                 l_run *= alpha;
 #pragma unroll
                 for (int y = 0; y < NDV; ++y)
@@ -159,7 +167,7 @@ __global__ __launch_bounds__(64 * WM * KG, KG == 1 ? 2 : 1) void attn_block_kern
 #pragma unroll
             for (int hf = 0; hf < NHF; ++hf)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) { sc[hf][i] = __builtin_amdgcn_exp2f(fmaf(sc[hf][i], c2, -m_sub)); sum += sc[hf][i]; }
+                for (int i = 0; i < 16; ++i) { sc[hf][i] = __builtin_amdgcn_exp2f(fmaf(sc[hf][i], factor, -m_sub)); sum += sc[hf][i]; }
             l_run += sum;
             const char *Vs = (const char *)(Ks + KT * KU);
             const int vk = 4 * hi + ((lane & 15) >> 2), vc8 = 8 * (lane & 1), vu = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);      // this lane's key, half unit and unit of a turned block

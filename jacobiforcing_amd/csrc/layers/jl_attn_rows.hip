@@ -76,11 +76,12 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
         }
     }
     // scores are kept times log2(e): weights are 2 ** (s - max)
-    constexpr float LOG2E = 1.44269504088896341f;
     float m_run = -INFINITY, l_run = 0.f;
-    if (a.sink && ok) { m_run = a.sink[hh] * LOG2E; l_run = 1.f; }   // the sink: an extra score that attends to nothing
+    if (a.sink && ok) { m_run = a.sink[hh] * AR_LOG2E; l_run = 1.f; }   // the sink: an extra score that attends to nothing
+    if (m_run == INFINITY) m_run = NAN;                             // such a row is none: its first tile scales its sums by NaN
+    float entry = ar_entry(m_run);
     if (hi) l_run = 0.f;                                            // each half-wavefront sums its own keys; the halves meet at the end
-    const float c2 = capped ? LOG2E : fmaxf(fabsf(a.scale * LOG2E), 1e-30f);
+    const float c2 = capped ? AR_LOG2E : fabsf(a.scale * AR_LOG2E);
     ar_f32x16 acc[NDV];
 #pragma unroll
     for (int t = 0; t < NDV; ++t)
@@ -210,21 +211,24 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
                 for (int r = hf == 0 ? 1 : 0; r < 16; ++r) mx = fmaxf(mx, sc[hf][r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float m_new = fmaxf(m_run, mx * c2);
-            const float m_sub = m_new > -INFINITY ? m_new : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);      // m_run = -inf: 0, and nothing has been accumulated yet; none where the sink is NaN or infinite, and so the row
-            m_run = m_new;
-            if (__any(alpha != 1.0f)) {                             // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
+            float factor = c2;
+            if (__any(!(m_new <= entry))) {                         // after the first tiles a row's maximum seldom moves (a stale one would leave the greatest weight inexact)
+                const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new > -INFINITY ? m_new : 0.f));      // m_run = -inf: 0, and nothing has been accumulated yet
+                m_run = m_new;
+                entry = ar_entry(m_run);
+                factor = ar_factor(sc, c2, m_run);
                 l_run *= alpha;
 #pragma unroll
                 for (int t = 0; t < NDV; ++t)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[t][r] *= alpha;
             }
+            const float m_sub = m_run > -INFINITY ? m_run : 0.f;   // a row that has seen no key yet: all weights are 2 ** -inf
             float sum = 0.f;
 #pragma unroll
             for (int hf = 0; hf < HALVES; ++hf)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) { sc[hf][r] = __builtin_amdgcn_exp2f(fmaf(sc[hf][r], c2, -m_sub)); sum += sc[hf][r]; }
+                for (int r = 0; r < 16; ++r) { sc[hf][r] = __builtin_amdgcn_exp2f(fmaf(sc[hf][r], factor, -m_sub)); sum += sc[hf][r]; }
             l_run += sum;
             const char *Vs = (const char *)(V_IN_K ? Ks : Ks + KT * KU);
             const int vk = 4 * hi + ((lane & 15) >> 2), vc8 = 8 * (lane & 1), vu = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);      // this lane's key, half unit and unit of a turned block
@@ -280,7 +284,9 @@ __global__ __launch_bounds__(AR_THREADS, 2) void attn_rows_kernel(jl_attn_args a
     }
 }
 
-template <int KU, int VU, int SRC> static int ar_launch(const jl_attn_args &a, int hf, int hb, hipStream_t st) {
+template <int KU, int VU, int SRC> static int ar_launch(const jl_attn_args &args, int hf, int hb, hipStream_t st) {
+    jl_attn_args a = args;
+    if (!(a.softcap > 0.f) && ar_one_by_one(a.scale)) a.softcap = INFINITY;      // a cap's scores are multiplied one by one, and come out of an infinite one as they are
     constexpr size_t lds = ar_lds_bytes(KU, VU);
     auto kern = attn_rows_kernel<KU, VU, SRC>;
     if (lds > 64 * 1024) {

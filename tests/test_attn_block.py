@@ -117,3 +117,25 @@ def test_operands_in_host_memory_are_refused():
         with pytest.raises(ValueError):
             LO.block_slots(args[0], T, *args[1:], 32, T, True)
     assert LO.attn_block(q, T, max_keys=32, **good).shape == (R * T, 6 * D)
+
+
+@pytest.mark.parametrize("plan", [(1, 0), (3, 0), (1, 1), (2, 1)])
+@pytest.mark.parametrize("up,scale", [(20, 2.0 ** -3), (30, -2.0 ** -3), (50, 2.0 ** -40), (53, 2.0 ** -108), (53, -2.0 ** -108), (53, 0.0), (0, float("nan"))])
+def test_scores_and_scales_of_any_size(monkeypatch, plan, up, scale):
+    """Sums of products of small whole numbers, exact in 32 bits, times 2 ** (2 * up): scores of any size that tie or lie apart by one unit of theirs."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, R, T, nkv, G, D, n = "cuda", 2, 32, 2, 2, 64, 400
+    monkeypatch.setattr(LO, "_block_plan", lambda *a: plan)
+    g = torch.Generator(device=dev).manual_seed(4)
+    whole = lambda *s: torch.randint(-2, 3, s, generator=g, device=dev).bfloat16() * 2.0 ** up
+    q, k, v = whole(R, nkv, G * T, D), whole(R, nkv, n, D), torch.randn(R, nkv, n, D, generator=g, device=dev).bfloat16()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    got = LO.attn_block(q, T, k, v, i32([n - T] * R), i32([T] * R), n, i32([0, 1]), scale=scale).double().view(R, T, nkv, G, D)
+    if scale != scale:
+        assert bool(got.isnan().all())
+        return
+    t, j = torch.arange(T, device=dev).view(T, 1), torch.arange(n, device=dev).view(1, n)
+    s = (q.double() @ k.double().transpose(2, 3).contiguous() * scale).view(R, nkv, G, T, n).masked_fill(j - (n - T) > t, float("-inf"))
+    want = (torch.softmax(s, -1).view(R, nkv, G * T, n) @ v.double()).view(R, nkv, G, T, D).permute(0, 3, 1, 2, 4)
+    err = (got - want).abs()               # weights and outputs are rounded to bfloat16, as in test_block
+    assert bool(got.isfinite().all()) and float(err.max()) <= 4 * 2.0 ** -8 * max(1.0, float(want.abs().max()) / 4)

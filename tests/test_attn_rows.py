@@ -205,3 +205,23 @@ def test_sinks_that_are_not_finite(monkeypatch, built, value):
         assert bool(got[:, 5].isnan().all())
     got[:, 5] = want[:, 5]
     assert torch.equal(got, want)
+
+
+# sums of products of small whole numbers, exact in 32 bits, times 2 ** (2 * up): scores of any size that tie or lie apart by one unit of theirs
+@pytest.mark.parametrize("up,scale", [(20, 2.0 ** -3), (30, -2.0 ** -3), (50, 2.0 ** -40), (53, 2.0 ** -108), (53, -2.0 ** -108), (53, 0.0), (0, float("nan"))])
+def test_scores_and_scales_of_any_size(up, scale):
+    from jacobiforcing_amd import layer_ops as LO
+    dev, H, G, D = "cuda", 16, 4, 64
+    g = torch.Generator(device=dev).manual_seed(4)
+    whole = lambda *s: torch.randint(-2, 3, s, generator=g, device=dev).bfloat16() * 2.0 ** up
+    counts, starts, pages = [1100, 131], [0, 37], [list(range(18)), list(range(18, 21))]
+    q, k, v = whole(1231, H * D), whole(21 * 64, G * D), torch.randn(21 * 64, G * D, generator=g, device=dev).bfloat16()
+    batch = LO.RaggedBatch.build(counts, starts, [0, 1], pages, 64, dev)
+    got = LO.attn_sweep(q, k, v, batch, H, G, D, D, scale, 0, float_out=True)
+    assert ("longest first", 32, None) in batch._tiles, "the 128-row form did not run"
+    if scale != scale:
+        assert bool(got.isnan().all())
+        return
+    want = reference(q, k, v, starts, counts, pages, 64, H, G, G, D, D, scale, 0, 0, 0.0, None)
+    err = (got.double() - want).abs()      # weights are rounded to bfloat16 once, as in test_wide_tiles
+    assert bool(got.isfinite().all()) and err.max() < 2.0 ** -7 * want.abs().max() and err.norm() < 2.0 ** -8 * want.norm()
