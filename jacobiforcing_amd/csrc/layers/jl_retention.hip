@@ -223,6 +223,9 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // us, 8 heads of 128 x 128, bfloat16, 4 x 2048 tokens, outputs / contributions: 121 / 54 then, 58 / 26 now; the whole layer 188 / 117, one portion of 128 51 / 36, of 1000 60 / 47, 8 of 8 33 / 24; 8 heads of 64 109 / 70;
 // float, 1021 + 851 + 681 tokens 105 / 80.  Error of the states against 64 bits 2.1e-7 then, 1.7e-7 now.
 // Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups: they are left out of them, and their columns' outputs and state set behind.
+// Numbers that no bfloat16 number comes near (infinities, and floats between the two types' ends) have no terms: groups whose outputs are not all finite, and contributions of keys or values like that, are
+// formed on the float instructions from the numbers themselves, so that sums of one sign stay infinite and finite ones finite (looking for them takes 2 %: 4 x 2048 tokens 104 / 106 us).  Numbers below
+// 2^-110 lose the bits of their terms that lie below bfloat16's last place, 2^-133.
 // Outputs leave as floats and are normed and gated by rows in a launch of their own.
 constexpr int RM_T = 64, RC_T = 32, RM_OUT = 0, RM_LOCAL = 1, RC_VROW = 128 + 16;      // RM_T: pieces come in multiples of it
 typedef float rm_f32x16 __attribute__((ext_vector_type(16)));
@@ -231,6 +234,7 @@ typedef __bf16 rm_bf16x4 __attribute__((ext_vector_type(4)));
 typedef short rm_s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) rm_s16x4 rm_lds_s16x4;
 constexpr int RM_TERMS = JL_SPLIT_TERMS;
+constexpr float RM_BEYOND = 3.395e38f;                               // bfloat16 ends at 3.3895e38; from 3.3953e38 on a float is rounded to infinity
 template <typename T> static constexpr size_t rm_lds_bytes(int DP, bool out) {
     return 2 * RC_T * ((out ? 2 : 1) * (size_t)RM_TERMS * (DP + 8) + (sizeof(T) == 4 ? RM_TERMS : 1) * RC_VROW) + (RC_T + 2 * RC_T + 4 * RC_T + 4) * 4;
 }
@@ -246,6 +250,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
     bf16_t *Ks = (bf16_t *)smem, *Vs = Ks + RM_TERMS * RC_T * QROW, *Qs = Vs + VT * RC_T * RC_VROW;      // [terms][32][..]
     float *g1 = (float *)(Qs + (OUT ? RM_TERMS * RC_T * QROW : 0)), *dec = g1 + RC_T;        // g^(i+1); g^(31-m), none from 32 on
     int *brokenS = (int *)(dec + 2 * RC_T), *flawS = brokenS + 4 * RC_T;                     // per column: the group's first token whose value is not finite; whether this group, the one before, has one
+    int *beyondS = flawS + 2;                                                                // RM_LOCAL: whether this group, the one before, has a key or value that no bfloat16 number comes near
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * wave + l32;
     const bool busy = 32 * wave < Dv;
     const float gamma = a.decay[h], kscale = 1.0f / sqrtf((float)D);
@@ -341,19 +346,39 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
         for (int x = 0; x < 8; ++x) f[x] = v[8 * s + x];
         return f;
     };
+    // what the terms stand for, from memory: the value of token t of a group at depth d of q or k, turned and scaled, and of v at this lane's column
+    auto whole = [&](int from, float scale, int t0, int nt, int t, int d) {
+        asm volatile("" : "+v"(t), "+v"(d));                        // nothing of it is worth a register in the loop around
+        if (t >= nt || d >= D) return 0.f;
+        const T *x = src + (int64_t)(t0 + t) * a.ld + h * D + from;
+        const float u = ld_f(x + d) * scale;
+        if (d >= 2 * half) return u;
+        const int64_t p = (pos0 + t0 + t < a.table_len ? pos0 + t0 + t : a.table_len - 1) * half + (d < half ? d : d - half);
+        const float w = ld_f(x + (d < half ? d + half : d - half)) * scale, c = a.cos_t[p], s = a.sin_t[p];
+        return d < half ? u * c - w * s : u * c + w * s;
+    };
+    auto value = [&](int t0, int nt, int t) {                       // (one that is not finite is left out of outputs and set behind them, as in the terms)
+        asm volatile("" : "+v"(t));
+        const float v = t < nt && col < Dv ? ld_f(src + (int64_t)(t0 + t) * a.ld + a.v_col + h * Dv + col) : 0.f;
+        return OUT && !__builtin_isfinite(v) ? 0.f : v;
+    };
     fetch(0);
     for (int t0 = 0; t0 < cnt; t0 += RC_T) {
         const int nt = cnt - t0 < RC_T ? cnt - t0 : RC_T;
         __syncthreads();                                            // the group before has been read
+        float big = 0.f;                                            // of keys and values, where no outputs tell (NaN passes: it reaches the same sums either way)
 #pragma unroll
         for (int it = 0; it < QIT; ++it) {
             const int tt = tid / SLOTS + it * (256 / SLOTS);
-            auto stage = [&](bf16_t *rows, jl_f32x8 v) {
+            auto stage = [&](bf16_t *rows, jl_f32x8 v, bool key) {
                 if (turns && tt < nt) {
                     const jl_f32x8 w = v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) { v[i] = w[i] * rc[it][i] - w[4 + i] * rs[it][i]; v[4 + i] = w[4 + i] * rc[it][i] + w[i] * rs[it][i]; }
                 }
+                if (!OUT && key)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) big = fmaxf(big, fabsf(v[i]));
                 jl_bf16x8 part[RM_TERMS];
                 jl_split8(v, part);
 #pragma unroll
@@ -362,8 +387,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                     put(rows + (x * RC_T + tt) * QROW + 4 * ub, part[x], 1);
                 }
             };
-            stage(Ks, to_float(rk[it][0], rk[it][1]) * kscale);
-            if (OUT) stage(Qs, to_float(rq[it][0], rq[it][1]));
+            stage(Ks, to_float(rk[it][0], rk[it][1]) * kscale, true);
+            if (OUT) stage(Qs, to_float(rq[it][0], rq[it][1]), false);
         }
         float zero = 0.f;                                           // not a number with a value that is not finite
 #pragma unroll
@@ -372,6 +397,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
             if (OUT)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) zero = __builtin_fmaf(v[i], 0.f, zero);
+            if (!OUT)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) big = fmaxf(big, fabsf(v[i]));
             jl_bf16x8 part[RM_TERMS];
             if (VT > 1) jl_split8(v, part);
             else part[0] = __builtin_convertvector(v, jl_bf16x8);
@@ -384,7 +412,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                 }
         }
         if (OUT && zero != 0.f) flawS[t0 / RC_T & 1] = 1;
+        if (!OUT && big >= RM_BEYOND) beyondS[t0 / RC_T & 1] = 1;
         __syncthreads();
+        bool beyond = false;                                        // the group takes the float instructions
+        if (!OUT) {
+            beyond = __builtin_amdgcn_readfirstlane(beyondS[t0 / RC_T & 1]);
+            if (tid == 0) beyondS[~(t0 / RC_T) & 1] = 0;
+        }
         bool flawed = false;
         if (OUT) {
             flawed = __builtin_amdgcn_readfirstlane(flawS[t0 / RC_T & 1]);
@@ -453,6 +487,30 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                     for (int x = 0; x <= d; ++x)
                         if (d - x < VT) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[x], vf[d - x < VT ? d - x : 0][s], o, 0, 0, 0);
             }
+            float odd = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) odd = __builtin_fmaf(o[r], 0.f, odd);
+            beyond = __ballot(odd != 0.f) != 0;                     // not a number in some lane (a key or value like that is in its own token's output)
+            if (beyond) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[r] = p[r] = 0.f;
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll 1
+                    for (int r = 0; r < 16; ++r) {
+                        const int d = 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
+                        const float q = whole(a.q_col, 1.0f, t0, nt, l32, d), k = whole(a.k_col, kscale, t0, nt, l32, d);
+                        p = __builtin_amdgcn_mfma_f32_32x32x2f32(k, q, p, 0, 0, 0);
+                        o = __builtin_amdgcn_mfma_f32_32x32x2f32(q, S[t][r], o, 0, 0, 0);
+                    }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[r] *= g1[8 * (r >> 2) + 4 * hi + (r & 3)];
+#pragma unroll 1
+                for (int r = 0; r < 16; ++r) {
+                    const int j = 8 * (r >> 2) + 4 * hi + (r & 3);
+                    o = __builtin_amdgcn_mfma_f32_32x32x2f32(j <= l32 ? p[r] * dec[31 - l32 + j] : 0.f, value(t0, nt, j), o, 0, 0, 0);
+                }
+            }
             const int broken = flawed ? brokenS[32 * wave + l32] : RC_T;
             if (col < Dv) {                                         // as they are: the norm over a head's Dv columns spans wavefronts, and a gate's bytes are better read in rows
                 const uint32_t o_row = (uint32_t)(H * Dv) * 4;
@@ -473,6 +531,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
             for (int t = 0; t < NS; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) S[t][r] *= gn;
+            if (beyond) {
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll 1
+                    for (int r = 0; r < 16; ++r) {
+                        const int j = 8 * (r >> 2) + 4 * hi + (r & 3);
+                        S[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(whole(a.k_col, kscale, t0, nt, j, 32 * t + l32), value(t0, nt, j) * dec[RC_T - nt + j], S[t], 0, 0, 0);
+                    }
+            } else
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 jl_f32x8 v;

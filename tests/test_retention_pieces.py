@@ -132,3 +132,64 @@ def test_short_portions_with_infinities(D, Dv):
             assert torch.equal(got[t].isfinite(), ok) and torch.allclose(got[t][ok].double(), o[ok], rtol=2e-5, atol=2e-5), (b, t)
         assert torch.equal(state[b].isfinite(), S.isfinite())
         r0 += c
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("what", ["state", "key", "query", "earlier value", "large value", "large query"])
+def test_infinities_and_numbers_beyond_bfloat16(monkeypatch, what, dtype):
+    """An infinite state column or key, and floats that lie beyond bfloat16's greatest number, give what the scan gives: sums of one sign stay infinite, finite ones finite, and no token in front is
+    reached.  (Values that are not finite spoil their own piece's rows from their token on; those of a later piece see an infinite state.)"""
+    from jacobiforcing_amd import layer_ops as LO
+    if what.startswith("large") and dtype == "bfloat16":
+        pytest.skip("floats alone lie beyond")
+    monkeypatch.setattr(LO, "RETENTION_WORKGROUPS", 1024)
+    dev, dt, H, D, Dv, counts, starts = "cuda", getattr(torch, dtype), 2, 64, 96, [300, 70], [5, 9]
+    g = torch.Generator(device=dev).manual_seed(7)
+    cols, rot = (0, H * D, 2 * H * D, 2 * H * D + H * Dv), 0
+    proj = torch.randn(370, cols[3] + H * Dv, generator=g, device=dev)
+    proj[:, :cols[2]] = proj[:, :cols[2]].abs() * 0.1 + 0.01                                  # queries and keys above zero: an infinity stays one
+    start = torch.rand(2, H, D, Dv, generator=g, device=dev) + 0.1
+    first, rows = 0, [0, 300]                                                                 # the rows from `first` on of the request are the ones reached
+    if what == "state":
+        start[0, 1, 3, 40] = float("inf")
+    elif what == "key":
+        first, proj[150, cols[1] + D + 5] = 150, float("inf")
+    elif what == "query":
+        first, proj[37, cols[0] + D + 5] = 37, float("inf")
+    elif what == "earlier value":
+        first, proj[20, cols[2] + Dv + 11] = 64, float("-inf")
+    elif what == "large value":
+        first, proj[37, cols[2] + Dv + 11] = 37, 3.4e38
+        proj[:, :cols[2]] *= 1e-3
+    else:
+        first, proj[37, cols[0] + D + 5] = 37, 3.4e38
+        start *= 1e-30
+        proj[:, cols[2]:cols[3]] *= 1e-30
+    proj, decay, pages = proj.to(dt), torch.tensor([0.9, 0.97], device=dev), [[0, 1, 2, 3, 4], [5, 6]]
+    outs, states = [], []
+    for scan in (False, True):
+        batch, st = LO.RaggedBatch.build(counts, starts, [0, 1], pages, 64, dev), start.clone()
+        if scan:
+            batch._tiles[("retention", H, D)] = 0
+        outs.append(LO.retention(proj, cols, batch, H, D, Dv, rot, None, None, decay, 1e-5, st).view(370, H, Dv))
+        states.append(st)
+        assert scan or ("pieces", 64) in batch._tiles
+    got, want = outs
+    free = torch.ones(370, H, dtype=torch.bool, device=dev)                                   # what nothing reaches
+    free[first:300, 1] = False
+    assert bool(got[free].isfinite().all()) or what == "earlier value"
+    if what == "earlier value":
+        free[20:64, 1] = False
+        assert bool(got[free].isfinite().all())
+    later = torch.zeros_like(free)
+    later[first:300, 1] = True
+    for a, b in ((got[free], want[free]), (got[later], want[later])):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+        ok = b.isfinite()
+        # sums of 32-bit products in another order, normed; bfloat16 outputs round once more
+        assert (a[ok].double() - b[ok].double()).norm() <= (2.0 ** -7 if dtype == "bfloat16" else 1e-5) * max(1.0, float(b[ok].double().norm()))
+    a, b = states
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()])
+    ok = b.isfinite()
+    assert (a[ok].double() - b[ok].double()).norm() <= 4e-6 * b[ok].double().norm()
+    assert bool(ok.all()) == (what in ("query", "large value", "large query"))
