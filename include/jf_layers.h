@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 138
+#define JL_VERSION 139
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -212,11 +212,13 @@ JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_re
 JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                            int32_t out_mode, void *stream);
 /* The same for more rows (a few hundred), all bfloat16, the result at a 16-byte border, operands of up to 4 GB. */
+JL_API int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O);       /* whether the launch is the better one for these sizes, whatever their type */
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                          void *stream);
 
 /* The same for float rows of any number (x [N, x_ld], W [O, K], rows at 16-byte borders, out rows out_ld floats apart), on the bfloat16 matrix instructions in three terms per operand: sums at
- * least as close to 64 bits as the float instructions' (products below 2^-110 aside). */
+ * least as close to 64 bits as the float instructions' (products below 2^-110 aside).  jl_linear_split_ok: whether that is the better launch for these sizes. */
+JL_API int jl_linear_split_ok(int64_t N, int64_t K, int64_t O);
 JL_API int jl_linear_split(const float *x, int64_t N, int64_t x_ld, const float *w, int32_t K, int32_t O, const float *bias, float *out, int64_t out_ld, void *stream);
 
 /* z <- cap * tanh(z / cap) in place over `total` floats (soft cap of the logits). */

@@ -20,7 +20,7 @@
 namespace {
 
 #define JL_HOST_CALLS(X)                                                                                                                              \
-    X(jl_linear_small) X(jl_linear_mid) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
+    X(jl_linear_small) X(jl_linear_mid_ok) X(jl_linear_mid) X(jl_linear_split_ok) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
     X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) X(jl_latent_heads_run) \
     X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
 #define DECLARE(name) decltype(&name) p_##name;
@@ -135,17 +135,12 @@ decltype(&jl_last_error) p_last_error, p_last_error_seq;
     } while (0)
 #define NEED(...) do { if (!(__VA_ARGS__)) return not_taken(); } while (0)
 
-// LINEAR_SMALL_ROWS, LINEAR_ONE_TILE, LINEAR_X_BYTES of layer_ops.py, whose rules these are (linear_small, linear_mid, linear_split)
+// LINEAR_SMALL_ROWS, LINEAR_ONE_TILE, LINEAR_X_BYTES of layer_ops.py, whose rule this is (linear_small)
 int64_t small_rows, one_tile, x_bytes;
 bool rule_small(int64_t n, int64_t k, int64_t o, int64_t item) {
     const int64_t tile = o <= one_tile || n == 1 ? 16 : o <= 4 * one_tile ? 32 : 64;
     return n > 0 && n <= small_rows && n * k * item * ((o + tile * 256 - 1) / (tile * 256)) <= x_bytes;
 }
-bool rule_mid(int64_t n, int64_t k, int64_t o) {
-    const int64_t tiles = ((n + 63) / 64) * ((o + 63) / 64);
-    return n > 0 && ((k <= 1024 && tiles <= 512) || (k <= 2048 && tiles <= 256));
-}
-bool rule_split(int64_t n, int64_t k, int64_t o) { return k > 0 && ((n + 63) / 64) * ((o + 127) / 128) >= 192; }
 
 // x, w, bias, float_out
 CALL(linear, 4)
@@ -157,7 +152,8 @@ CALL(linear, 4)
     const int64_t n = x->size(0), k = x->size(1), o = w->size(0), ld = x->stride(0), size = w->element_size();
     const bool same = w->scalar_type() == x->scalar_type();
     NEED(same || (is_float(*w) && !typed && as_float));
-    const bool small = rule_small(n, k, o, size), split = !small && same && is_float(*w) && rule_split(n, k, o), mid = !small && !split && same && !is_float(*x) && rule_mid(n, k, o);
+    const bool small = rule_small(n, k, o, size), split = !small && same && is_float(*w) && p_jl_linear_split_ok(n, k, o),
+               mid = !small && !split && same && !is_float(*x) && p_jl_linear_mid_ok(n, k, o);
     NEED(small || split || mid);
     NEED(w->size(1) == k && w->is_contiguous() && x->stride(1) == 1 && ld >= k && k > 0 && o > 0 && o <= INT32_MAX && k * size % 16 == 0 && ld * (int64_t)x->element_size() % 16 == 0 && starts16(*x) &&
          starts16(*w) && w->device() == x->device());
@@ -584,7 +580,7 @@ PyObject *bind(PyObject *, PyObject *args) {
 PyObject *linear_rule(PyObject *, PyObject *args) {
     long long n, k, o, item;
     if (!PyArg_ParseTuple(args, "LLLL", &n, &k, &o, &item)) return nullptr;
-    return PyLong_FromLong(rule_small(n, k, o, item) ? 1 : item == 4 ? (rule_split(n, k, o) ? 2 : 0) : rule_mid(n, k, o) ? 3 : 0);
+    return PyLong_FromLong(rule_small(n, k, o, item) ? 1 : item == 4 ? (p_jl_linear_split_ok(n, k, o) ? 2 : 0) : p_jl_linear_mid_ok(n, k, o) ? 3 : 0);
 }
 PyObject *symbols(PyObject *, PyObject *) {
 #define NAME(name) #name,

@@ -157,6 +157,11 @@ __global__ __launch_bounds__(256) void linear_mid_kernel(const bf16_t *__restric
     }
 }
 
+// Up to two tiles per CU at depths of up to 1024, one at up to 2048 (layer_ops.linear_mid has the figures).
+extern "C" int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O) {
+    const int64_t tiles = ((N + LD_TILE - 1) / LD_TILE) * ((O + LD_TILE - 1) / LD_TILE);
+    return N > 0 && ((K <= 1024 && tiles <= 512) || (K <= 2048 && tiles <= 256));
+}
 extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                              void *stream) {
     if (N <= 0 || O <= 0) return JL_OK;
@@ -209,14 +214,31 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void linear_split_kernel(const flo
     }
 }
 
+// 128 rows per tile as soon as they give about half of the CUs one each.  us, 128 / 64 rows: 2553 x 1024 by 1100 (180 tiles of 128) 47 / 52, by 4096 139 / 150, 1500 x 768 by 1536 (144) 36 / 39;
+// below, 512 x 1024 by 4096 (128) 51 / 36, 2553 x 512 by 768 (120) 26 / 18
+static bool split_low(int64_t N, int64_t O) { return (N + 127) / 128 * ((O + 127) / 128) < 140; }
+
+// The launch's time goes by rounds of 256 tiles, the library's, which has tiles of more heights and splits depths, more nearly by the product's size, so the line lies where a round is full enough: by the
+// product's size in units of 64 x 128 against the tiles it is padded to.  us of GPU time, library / own: 2553 rows of 1024 by 1024 57 / 52, by 3072 135 / 100, 4096 of 4096 by 4096 948 / 747 (184 TFLOP/s; the
+// float instructions reach 145), 2049 of 1028 by 1153 69 / 57, 1700 of 1024 by 1024 38 / 37, 128 of 1024 by 16384 39 / 36.  Beyond the line: padded rows, 96 of 1024 by 16384 30 / 35, 160 by 8192 28 / 33,
+// 650 by 3072 41 / 53; rounds that have just begun, 513 of 1024 by 4096 49 / 52, 1290 by 3072 68 / 86, 2060 by 1024 49 / 54, 4100 of 2048 by 1024 149 / 160; one round of 64 rows at great depths, 1536
+// of 4096 by 1024 111 / 115.  Up to depths of 320 both take 3 us more or less of the GPU, but the library's call 15 more of the host: from 192 tiles of 64 rows on.
+extern "C" int jl_linear_split_ok(int64_t N, int64_t K, int64_t O) {
+    if (N <= 0 || K <= 0 || O <= 0) return 0;
+    const int64_t cols = (O + 127) / 128, tiles = (N + 63) / 64 * cols;
+    if (K < 320) return tiles >= 192;
+    const double size = (double)N * (double)O / (64 * 128);
+    if (split_low(N, O)) return tiles >= 192 && tiles <= 256 && size >= 164 && size >= 0.8 * (double)tiles && (K < 2048 || size >= 200);
+    const int64_t high = (N + 127) / 128 * cols, rounds = (high + 255) / 256;
+    return rounds == 1 ? size > (high <= 200 ? 288 : 340) : size >= 330.0 * (double)rounds;
+}
+
 extern "C" int jl_linear_split(const float *x, int64_t N, int64_t x_ld, const float *w, int32_t K, int32_t O, const float *bias, float *out, int64_t out_ld, void *stream) {
     if (N <= 0 || O <= 0) return JL_OK;
     if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < O) return jl_fail(JL_E_INVALID, "jl_linear_split: null pointer or bad sizes");
     if (K % 4 || x_ld % 4 || (((uintptr_t)x | (uintptr_t)w) & 15)) return jl_fail(JL_E_INVALID, "jl_linear_split: rows of x and W at 16-byte borders");
     const int64_t cols = ((int64_t)O + 127) / 128;
-    // 128 rows per tile as soon as they give about half of the CUs one each.  us, 128 / 64 rows: 2553 x 1024 by 1100 (180 tiles of 128) 47 / 52, by 4096 139 / 150, 1500 x 768 by 1536 (144) 36 / 39;
-    // below, 512 x 1024 by 4096 (128) 51 / 36, 2553 x 512 by 768 (120) 26 / 18
-    const bool low = (N + 127) / 128 * cols < 140;
+    const bool low = split_low(N, O);
     const int64_t row_tiles = low ? (N + 63) / 64 : (N + 127) / 128, tiles = row_tiles * cols;
     if (tiles > INT32_MAX / 512) return jl_fail(JL_E_INVALID, "jl_linear_split: too many tiles");
     (low ? linear_split_kernel<64, 8, 2, 8> : linear_split_kernel<128, 8, 2, 4>)<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 512, 0, (hipStream_t)stream>>>(x, x_ld, w, bias, out, out_ld, N, K, O,

@@ -372,16 +372,13 @@ def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
     and one.  There its GPU time is the library's give or take 3 us (1024 x 1024 by 128 rows 7.6 / 5.4, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 2048 x 2048 by 512 13.3 / 11.2), and the call
     costs 11 us less of the host, which such steps wait for (two portions of 50 beside 16 decoding requests at widths of 2048, us without / with the second line: Mikipel 1180 / 1122,
     Safisun 1050 / 936, Voborax 1400 / 1247)."""
-    tiles = -(-n // 64) * -(-o // 64)
-    return dtype == torch.bfloat16 and n > 0 and (k <= 1024 and tiles <= 512 or k <= 2048 and tiles <= 256)
+    return dtype == torch.bfloat16 and bool(N.layers().jl_linear_mid_ok(n, k, o))
 
 
 def linear_split(n: int, k: int, o: int) -> bool:
-    """Whether ``linear`` takes n float rows of k values times [o, k] to the bfloat16 matrix instructions in three terms per operand: from 192 tiles of 64 rows by 128 of W on.  us of GPU time, library /
-    own: 2553 rows of 1024 by 1024 57 / 54, by 3072 140 / 100, by 4096 178 / 139, 4096 of 4096 by 4096 948 / 747 (184 TFLOP/s; the library's product on the float instructions 145), 512 of 1024 by
-    4096 39.6 / 36.1, 1021 of 256 by 2048 19.2 / 12.0, at the line (1021 of 1024 by 1536) 31.0 / 29.6; below it 2553 of 1024 by 512 (160 tiles) 26.0 / 29.6, 256 of 1024 by 4096 (128) 21.5 / 27.5:
-    a tile's way through its stages alone takes 27."""
-    return k > 0 and -(-n // 64) * -(-o // 128) >= 192
+    """Whether ``linear`` takes n float rows of k values times [o, k] to the bfloat16 matrix instructions in three terms per operand: where their tiles fill the chip well enough (the rule and its
+    figures are the launch's, jl_linear_split_ok)."""
+    return bool(N.layers().jl_linear_split_ok(n, k, o))
 
 
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:

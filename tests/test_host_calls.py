@@ -33,6 +33,17 @@ def test_the_rules_of_linear():
                     assert H.linear_rule(n, k, o, size) == want, (n, k, o, size)
 
 
+@pytest.mark.parametrize("n,k,o,own", [
+    (2553, 1024, 1024, True), (2553, 1024, 3072, True), (4096, 4096, 4096, True), (2049, 1028, 1153, True), (1700, 1024, 1024, True), (128, 1024, 16384, True), (8192, 512, 1024, True), (640, 64, 2500, True),
+    (96, 1024, 16384, False), (160, 1024, 8192, False), (65, 2048, 25000, False), (650, 1024, 3072, False), (513, 1024, 4096, False), (1290, 1024, 3072, False), (2060, 1024, 1024, False),
+    (4100, 2048, 1024, False), (1536, 4096, 1024, False), (640, 512, 1024, False), (1, 1024, 100000, False), (0, 1024, 1024, False),
+])
+def test_linear_leaves_what_fills_tiles_badly_to_the_library(n, k, o, own):
+    """Products that were measured faster one way or the other (jl_linear_split_ok)."""
+    from jacobiforcing_amd import layer_ops as LO
+    assert LO.linear_split(n, k, o) == own
+
+
 def test_what_it_does_not_take():
     """Host tensors, other numbers of arguments, other kinds of values: handed back, nothing raised."""
     from jacobiforcing_amd import layer_ops as LO
