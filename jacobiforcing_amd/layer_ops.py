@@ -36,7 +36,7 @@ NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, a
                                       # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
 NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
                                       # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
-BLOCK_WORKGROUPS = 384               # a draft block's attention without key groups: workgroups to aim at when keys are shared out
+BLOCK_WORKGROUPS = 512               # a draft block's attention without key groups: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
 RETENTION_PIECES_FROM, RETENTION_WORKGROUPS = 8, 512     # retention: portions from this many tokens on (retention_pieces_from) run in pieces on the matrix cores; workgroups to aim at (us at 256 / 512: 8 heads of 128, 4 x 2048 tokens 126 / 117, of 64 78 / 70; one of 1000 47 / 47)
@@ -633,15 +633,20 @@ def block_slots(positions: torch.Tensor, T: int, row_prompt: torch.Tensor, row_c
     return out[0], out[1] if candidates else None
 
 
-def _block_plan(heads: int, GT: int, max_keys: int):
+def _block_plan(heads: int, GT: int, max_keys: int, D: int):
     """(shares of the keys, whether a workgroup's wavefronts take keys in groups) for ``heads`` (row, key head) pairs of GT (head, token) rows.  Groups, one workgroup of 64 rows per CU, where
-    those fit the chip at once; us with / without, 8 heads of 128 over 2, 32 tokens, context 512: 64 rows (256 workgroups) 20.6 / 27.4, 96 rows 37.1 / 28.9.  A share more costs its sums' way
-    through memory, by the rows, and a launch: one row, context 500 / 1000 / 4000 / 16000: 2, 4, 8 and 16 shares are the fastest; 32 rows, context 512: one 19.0, two 21.6, context 2000: 44.1
-    and 33.9.  Without groups, 96 rows: one share / two at context 512 28.9 / 33.3, 1000 50.1 / 52.3, 2000 83.6 / 71.1."""
-    units = max(1, heads * -(-GT // 64))
-    if units <= 256:
-        return max(1, min(256 // units, math.isqrt(max_keys // (64 + 2 * units)))), 1
-    return max(1, min(BLOCK_WORKGROUPS // (heads * -(-GT // 128)), max_keys // 768)), 0
+    those fit the chip at once, unless keys are many and few shares of them fit; us with / without, 8 heads of 128 over 2, 32 tokens, context 512: 64 rows (256 workgroups) 20.6 / 27.4,
+    96 rows 37.1 / 28.9; context 4000: 24 rows 48.9 / 44.7, 48 rows 76.3 / 61.3; 16 tokens, whose 64 rows leave half of the other form's tiles empty, 64 rows, context 4000: 52.2 / 57.1.  A share more
+    costs its sums' way through memory, by the rows, and a launch, which takes the host 3 us: one row, whole / in two, 256 keys 13.2 / 16.2, 512 17.5 / 16.8, heads of 64 512 12.1 / 16.7, 1000
+    16.4 / 16.6; context 500 / 1000 / 4000 / 16000: 2, 4, 8 and 16 shares are the fastest; 32 rows, context 512: one 19.0, two 21.6, context 2000: 44.1 and 33.9.  Without groups two workgroups per CU
+    as far as a share has 500 keys (750 of up to 64 columns): one share / two / three, 80 rows, context 1000 45.2 / 42.6 / 37.9; one / two, 96 rows 512 27.7 / 32.1, 1000 45.3 / 44.0, 1500 60.9 / 52.3,
+    64 rows of 14 heads of 64 over 2 1000 27.1 / 31.0, 2000 48.2 / 43.5."""
+    units = heads * -(-GT // 64)
+    if units <= 256 and (max_keys <= 2500 or units <= 85 or (units <= 128 and (D <= 64 or 8 * GT < 896 * -(-GT // 128)))):
+        if max_keys < (300 if D > 64 else 900) or units > 128 or units == 0:
+            return 1, 1
+        return min(256 // units, math.isqrt(max_keys // (64 + 2 * units))) or 1, 1
+    return max(1, min(BLOCK_WORKGROUPS // (heads * -(-GT // 128)), max_keys // (500 if D > 64 else 750))), 0
 
 
 def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len: torch.Tensor, row_len: torch.Tensor, max_keys: int, row_prompt: Optional[torch.Tensor] = None,
@@ -662,7 +667,7 @@ def attn_block(q: torch.Tensor, T: int, k: torch.Tensor, v: torch.Tensor, kv_len
           (ck is None or (ck.shape == cv.shape and ck.shape[2] >= T)), "attn_block: shapes")
     out = torch.empty((R * T, nkv * G * D), dtype=q.dtype, device=q.device)
     max_keys = min(int(max_keys), k.shape[2] * (1 if tables is None else tables.shape[1]))
-    splits, grouped = _block_plan(R * nkv, GT, max_keys)
+    splits, grouped = _block_plan(R * nkv, GT, max_keys, D)
     scratch = None
     if splits > 1:
         scratch = torch.empty((int(N.layers().jl_attn_block_scratch_floats(R, T, nkv, G, D, splits)),), dtype=torch.float32, device=q.device)

@@ -86,6 +86,15 @@ def test_shares_and_groups(monkeypatch, plan, T, G, D, kv, scale, climb):
         assert bool(((out[r] - want).abs() <= tol).all()), (r, float(((out[r] - want).abs() / tol).max()))
 
 
+@pytest.mark.parametrize("heads,GT,keys,D,plan", [(8, 128, 544, 128, (2, 1)), (128, 128, 544, 128, (1, 1)), (2, 128, 280, 128, (1, 1)), (2, 224, 544, 64, (1, 1)), (40, 128, 4032, 128, (3, 1)), (128, 64, 4032, 128, (2, 1)),
+                                                  (48, 128, 4032, 128, (8, 0)), (96, 128, 4032, 128, (5, 0)), (160, 128, 1532, 128, (3, 0)), (192, 128, 1532, 128, (2, 0)), (192, 128, 544, 128, (1, 0)),
+                                                  (256, 128, 2032, 128, (2, 0)), (128, 224, 1032, 64, (1, 0)), (128, 224, 2032, 64, (2, 0)), (1024, 256, 9000, 128, (1, 0)), (0, 0, 544, 128, (1, 1)), (4, 128, -1, 128, (1, 1))])
+def test_plan(heads, GT, keys, D, plan):
+    """Shares and groups as they were measured the fastest, or nearly; what the launch refuses has a plan too."""
+    from jacobiforcing_amd import layer_ops as LO
+    assert LO._block_plan(heads, GT, keys, D) == plan
+
+
 @pytest.mark.parametrize("R,T,candidates", [(1, 1, False), (5, 33, True), (64, 32, True), (3, 200, False)])
 def test_slots(R, T, candidates):
     from jacobiforcing_amd import layer_ops as LO
