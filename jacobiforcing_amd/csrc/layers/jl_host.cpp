@@ -87,6 +87,12 @@ void *at_(const Tensor *t) { return t ? t->data_ptr() : nullptr; }
 void *at_(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 bool starts16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
 void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+// other threads of the program run from here on, while memory is asked for (which may wait for the device) and launches are queued (which may wait for the queue), until back()
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    void back() { if (state) { PyEval_RestoreThread(state); state = nullptr; } }
+    ~Unlocked() { back(); }
+};
 Tensor make(at::IntArrayRef size, at::ScalarType type, const Tensor &like) { return at::empty(size, at::TensorOptions().dtype(type).device(like.device())); }
 bool overridden() { return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set(); }
 PyObject *wrap(const Tensor &t) { return t.defined() ? THPVariable_Wrap(t) : (Py_INCREF(Py_None), Py_None); }
@@ -125,13 +131,16 @@ bool angles(int32_t rot_dims, const Tensor *cos, const Tensor *sin, int64_t max_
     END_HANDLE_TH_ERRORS                                                                     \
     }
 bool of_sequences(const char *name) { return !strcmp(name, "jl_linear_scan") || !strncmp(name, "jl_moe", 6); }      // in the library of the recurrences and experts
-// a call into the library: refused arguments are the wrapper's to report, a failed launch is raised as it is there
+// a call into the library, with `others` unlocked: refused arguments are the wrapper's to report, a failed launch is raised as it is there
 decltype(&jl_last_error) p_last_error, p_last_error_seq;
 #define RUN(name, ...)                                                                                                                                               \
     do {                                                                                                                                                              \
         const int rc = p_##name(__VA_ARGS__);                                                                                                                        \
-        if (rc == JL_E_INVALID) return not_taken();                                                                                                                  \
-        if (rc != JL_OK) return PyErr_Format(PyExc_RuntimeError, "%s: %s", #name, (of_sequences(#name) ? p_last_error_seq : p_last_error)());                            \
+        if (rc != JL_OK) {                                                                                                                                            \
+            others.back();                                                                                                                                            \
+            if (rc == JL_E_INVALID) return not_taken();                                                                                                               \
+            return PyErr_Format(PyExc_RuntimeError, "%s: %s", #name, (of_sequences(#name) ? p_last_error_seq : p_last_error)());                                      \
+        }                                                                                                                                                             \
     } while (0)
 #define NEED(...) do { if (!(__VA_ARGS__)) return not_taken(); } while (0)
 
@@ -162,11 +171,13 @@ CALL(linear, 4)
     NEED(!x->_fw_grad(0).defined() && !w->_fw_grad(0).defined() && !(bias && bias->_fw_grad(0).defined()));      // forward-mode tangents
     NEED(small || split || n * ld * size < (int64_t)1 << 32);
     const int mode = typed ? JL_LINEAR_SAME : as_float ? JL_LINEAR_FLOAT : JL_LINEAR_ROUNDED_FLOAT;
+    Unlocked others;
     Tensor out = make({n, o}, typed ? x->scalar_type() : at::kFloat, *x);
     void *st = stream_of(*x);
     if (small) RUN(jl_linear_small, x->data_ptr(), code(*x), n, ld, w->data_ptr(), code(*w), (int32_t)k, (int32_t)o, at_(bias), out.data_ptr(), o, mode, st);
     else if (split) RUN(jl_linear_split, (const float *)x->data_ptr(), n, ld, (const float *)w->data_ptr(), (int32_t)k, (int32_t)o, (const float *)at_(bias), (float *)out.data_ptr(), o, st);
     else RUN(jl_linear_mid, x->data_ptr(), code(*x), n, ld, w->data_ptr(), (int32_t)k, (int32_t)o, at_(bias), out.data_ptr(), o, mode, st);
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -183,10 +194,12 @@ CALL(add_rmsnorm, 6)
     NEED(!y || (known(*y) && y->is_contiguous() && (y->dim() == 2 || y->dim() == 3) && y->size(0) == n && y->size(-1) == W && (y->dim() == 2 || y->size(1) > 0)));
     NEED(!x0 || (x0->sizes() == x->sizes() && is_float(*x0) && x0->is_contiguous()));
     NEED(!wanted || !w || (w->scalar_type() == type && w->numel() == W && w->is_contiguous()));
+    Unlocked others;
     Tensor out;
     if (wanted) out = make({n, W}, type, *x);
     RUN(jl_add_rmsnorm, (float *)x->data_ptr(), at_(y), y ? code(*y) : 0, !y ? 0 : y->dim() == 2 ? 1 : (int32_t)y->size(1), (const float *)at_(x0), at_(w), (float)eps, at_(out), code(type), n,
                           (int32_t)W, stream_of(*x));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -203,11 +216,13 @@ CALL(sandwich_norm, 9)
     NEED(n > 0 && W > 0 && (!y || (rows(*y, n, W) && known(*y) && y->is_contiguous() && w_post)) && row_weights(w_post, W) && row_weights(add_row, W) && row_weights(w_next, W));
     NEED(!into || (rows(*into, n, W) && known(*into) && into->stride(1) == 1));
     NEED(!(into || wanted) || plain || w_next);
+    Unlocked others;
     Tensor out;
     if (into) out = *into;
     else if (wanted) out = make({n, W}, type, *x);
     RUN(jl_sandwich_norm, (const float *)x->data_ptr(), (float *)x->data_ptr(), at_(y), y ? code(*y) : 0, (const float *)at_(w_post), (const float *)at_(add_row), (float)eps,
                             (const float *)at_(w_next), at_(out), out.defined() ? code(out) : 0, out.defined() ? out.stride(0) : 0, plain, n, (int32_t)W, stream_of(*x));
+    others.back();
     if (into) { Py_INCREF(arg[7]); return arg[7]; }
     return wrap(out);
 END_CALL
@@ -232,10 +247,12 @@ CALL(output_norm, 9)
         NEED(first && first->dim() == 3 && rows(*ids, n, first->size(1)) && rows(*weights, n, first->size(1)) && ids->scalar_type() == at::kInt && is_float(*weights) && ids->is_contiguous() &&
              weights->is_contiguous());
     }
+    Unlocked others;
     Tensor out;
     if (wanted) out = make({n, W}, type, *x);
     RUN(jl_output_norm, (float *)x->data_ptr(), addends, count, (const int32_t *)at_(ids), (const float *)at_(weights), ids ? (int32_t)ids->size(1) : 0, experts, kind, (const float *)at_(w),
                           (float)mult, (float)eps, (const float *)at_(w_next), at_(out), code(type), n, (int32_t)W, stream_of(*x));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -251,9 +268,11 @@ CALL(gated_norm, 9)
     const int64_t n = raw->size(0), C = raw->size(1);
     NEED(n > 0 && C > 0 && rows(*gate, n, C) && known(*gate) && gate->stride(1) == 1 && row_weights(w, C) && parts >= 1 && C % parts == 0);
     NEED(!into || (rows(*into, n, C) && into->scalar_type() == gate->scalar_type() && into->stride(1) == 1));
+    Unlocked others;
     Tensor out = into ? *into : make({n, C}, gate->scalar_type(), *raw);
     RUN(jl_gated_norm, (const float *)raw->data_ptr(), gate->data_ptr(), code(*gate), gate->stride(0), (const float *)w->data_ptr(), (float)eps, act, gate_first, (float)scale, out.data_ptr(),
                          out.stride(0), n, (int32_t)C, parts, stream_of(*raw));
+    others.back();
     if (into) { Py_INCREF(arg[8]); return arg[8]; }
     return wrap(out);
 END_CALL
@@ -269,9 +288,11 @@ CALL(gated_act, 9)
     NEED(z->dim() == 2 && known(*z) && z->stride(1) == 1 && g_col >= 0 && F > 0 && (int64_t)g_col + F <= z->size(1) && (int64_t)u_col + F <= z->size(1));
     const int64_t n = z->size(0);
     NEED(n > 0 && (!row_gate || (row_gate->scalar_type() == z->scalar_type() && row_gate->dim() > 0 && row_gate->numel() == n && row_gate->size(0) == n)));
+    Unlocked others;
     Tensor out = make({n, F}, z->scalar_type(), *z);
     RUN(jl_gated_act, z->data_ptr(), code(*z), n, z->stride(0), g_col, u_col, F, kind, (float)limit, (float)alpha, (float)shift, at_(row_gate), row_gate ? row_gate->stride(0) : 0, out.data_ptr(),
                         stream_of(*z));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -281,8 +302,10 @@ CALL(heads_gate, 2)
     NEED(take(arg[0], ov) && take_maybe(arg[1], gate) && ov->dim() == 3 && known(*ov) && ov->is_contiguous());
     const int64_t H = ov->size(0), n = ov->size(1), Dv = ov->size(2);
     NEED(H > 0 && n > 0 && Dv > 0 && (!gate || (rows(*gate, n, H * Dv) && gate->stride(1) == 1 && gate->scalar_type() == ov->scalar_type())));
+    Unlocked others;
     Tensor out = make({n, H * Dv}, ov->scalar_type(), *ov);
     RUN(jl_heads_gate, ov->data_ptr(), at_(gate), gate ? gate->stride(0) : 0, code(*ov), n, (int32_t)H, (int32_t)Dv, out.data_ptr(), stream_of(*ov));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -301,10 +324,12 @@ CALL(latent_prep, 18)
                    pool->size(-1) == (int64_t)R + rd));
     if (!pool) R = rd = rot_dims = 0;
     NEED(angles(rot_dims, cos, sin, max_pos, length));
+    Unlocked others;
     Tensor cq;
     if (Rq) cq = make({n, Rq}, proj->scalar_type(), *proj);
     RUN(jl_latent_prep, proj->data_ptr(), code(*proj), n, proj->size(1), q_col, Rq, kv_col, R, rd, rot_dims, Rq ? at_(wq) : nullptr, at_(wkv), (float)eps, (const int32_t *)at_(pos),
                           (const float *)at_(cos), (const float *)at_(sin), length, at_(cq), at_(pool), (const int64_t *)at_(kv_slot), pairing, stream_of(*proj));
+    others.back();
     return wrap(cq);
 END_CALL
 
@@ -317,9 +342,11 @@ CALL(latent_q_pack, 13)
          take(arg[9], pos) && take_maybe(arg[10], cos) && take_maybe(arg[11], sin) && take(arg[12], pairing));
     NEED(n > 0 && rows(*q, n, (int64_t)H * (D + rd)) && known(*q) && q->stride(1) == 1 && qa->is_contiguous() && qa->dim() == 3 && qa->size(0) == H && qa->size(1) == n && qa->size(2) == R &&
          qa->scalar_type() == q->scalar_type() && angles(rot_dims, cos, sin, max_pos, length));
+    Unlocked others;
     Tensor out = make({n, (int64_t)H * (R + rd)}, q->scalar_type(), *q);
     RUN(jl_latent_q_pack, qa->data_ptr(), q->data_ptr(), q->stride(0), code(*q), n, H, D, R, rd, rot_dims, (const int32_t *)at_(pos), (const float *)at_(cos), (const float *)at_(sin), length,
                             out.data_ptr(), pairing, stream_of(*q));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -336,6 +363,7 @@ CALL(latent_heads, 12)
     NEED(!gate || (rows(*gate, n, H * O) && gate->stride(1) == 1 && gate->scalar_type() == at::kBFloat16 && rd == 0));
     NEED(angles(rot_dims, cos, sin, max_pos, length));
     NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())));
+    Unlocked others;
     Tensor out = make({n, H * (O + rd)}, at::kBFloat16, *x);
     jl_latent_heads a = {};
     a.x = x->data_ptr(); a.w = w->data_ptr(); a.out = out.data_ptr(); a.gate = at_(gate); a.gate_ld = gate ? gate->stride(0) : 0;
@@ -343,6 +371,7 @@ CALL(latent_heads, 12)
     a.N = n; a.x_ld = x->stride(0); a.out_ld = H * (O + rd); a.H = (int32_t)H; a.K = (int32_t)K; a.O = (int32_t)O; a.x_head = x_head; a.out_head = (int32_t)(O + rd); a.rd = rd;
     a.rot_dims = rot_dims; a.pairing = pairing;
     RUN(jl_latent_heads_run, &a, stream_of(*x));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -359,9 +388,11 @@ CALL(token_shift, 8)
     bool wanted;
     NEED(take(arg[0], h) && take(arg[1], mu) && take(arg[2], n) && take(arg[3], max_slot) && take(arg[4], row_req) && take(arg[5], seq) && take(arg[6], tail) && take_type(arg[7], type, wanted) && wanted);
     NEED(h->dim() == 2 && is_float(*h) && h->is_contiguous() && h->size(0) == n && n > 0 && row_weights(mu, h->size(1)) && carries(tail, h->size(1), max_slot));
+    Unlocked others;
     Tensor out = make({n, h->size(1)}, type, *h);
     RUN(jl_token_shift, (const float *)h->data_ptr(), (const float *)mu->data_ptr(), (const int32_t *)row_req->data_ptr(), (const int32_t *)seq->data_ptr(), (float *)tail->data_ptr(), n,
                           (int32_t)h->size(1), out.data_ptr(), code(type), stream_of(*h));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -387,6 +418,7 @@ CALL(depth_mix_norm, 12)
     if (arg[11] != Py_None)
         NEED(PyTuple_CheckExact(arg[11]) && PyTuple_GET_SIZE(arg[11]) == 4 && take(PyTuple_GET_ITEM(arg[11], 0), mu) && take(PyTuple_GET_ITEM(arg[11], 1), tail) &&
              take(PyTuple_GET_ITEM(arg[11], 2), seq) && take(PyTuple_GET_ITEM(arg[11], 3), max_slot) && wanted && row_weights(mu, W) && carries(tail, W, max_slot));
+    Unlocked others;
     Tensor out, outf, outs;
     if (wanted) out = make({n, W}, type, *x);
     if (want_float) outf = make({n, W}, at::kFloat, *x);
@@ -394,6 +426,7 @@ CALL(depth_mix_norm, 12)
     RUN(jl_depth_mix_norm, (const float *)x->data_ptr(), addends, count, (float)mult, depth >= 0 ? (float *)at_(streams) : nullptr, depth >= 0 ? n * W : 0, depth,
                              depth >= 0 ? (const float *)at_(mix) : nullptr, written ? (float *)at_(x_out) : nullptr, (const float *)at_(w), (float)eps, at_(out), code(type), (float *)at_(outf), n,
                              (int32_t)W, (const float *)at_(mu), (const int32_t *)at_(seq), (float *)at_(tail), at_(outs), stream_of(*x));
+    others.back();
     if (!want_float && !mu) return wrap(out);
     if (want_float && !mu) return Py_BuildValue("(NN)", wrap(out), wrap(outf));
     if (!want_float) return Py_BuildValue("(NN)", wrap(out), wrap(outs));
@@ -414,9 +447,11 @@ CALL(short_conv, 14)
     const int32_t taps = (int32_t)w->size(1);
     NEED(taps == 1 || (tail && is_float(*tail) && tail->is_contiguous() && tail->dim() == 3 && tail->size(1) == taps - 1 && tail->size(2) == C && max_slot < tail->size(0)));
     NEED((!bias || (bias->scalar_type() == x->scalar_type() && bias->numel() == C && bias->is_contiguous())) && (type == at::kFloat || type == x->scalar_type()));
+    Unlocked others;
     Tensor out = make({n, C}, type, *x);
     RUN(jl_short_conv, x->data_ptr(), code(*x), x->size(1), col, w->data_ptr(), at_(bias), (const int32_t *)row_req->data_ptr(), (const int32_t *)seq->data_ptr(), B, longest, (float *)at_(tail), n, C,
                          taps, act, out.data_ptr(), code(type), stream_of(*x));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -434,12 +469,14 @@ CALL(linear_scan, 19)
     NEED(is_float(*state) && state->is_contiguous() && state->dim() == 4 && state->size(1) == H && state->size(2) == D && state->size(3) == Dv && max_slot < state->size(0));
     NEED((decay || (dt && a_log && dt_bias)) && row_weights(decay, H) && row_weights(a_log, H) && row_weights(dt_bias, H) && row_weights(skip, H));
     NEED(decay || (rows(*dt, n, H) && dt->stride(1) == 1 && dt->scalar_type() == src->scalar_type()));
+    Unlocked others;
     Tensor out = make({n, (int64_t)H * Dv}, at::kFloat, *src);
     jl_scan_args a = {};
     a.src = src->data_ptr(); a.dt = decay ? nullptr : dt->data_ptr(); a.decay = (const float *)at_(decay); a.A_log = (const float *)at_(a_log); a.dt_bias = (const float *)at_(dt_bias);
     a.skip = (const float *)at_(skip); a.seq = (const int32_t *)seq->data_ptr(); a.state = (float *)state->data_ptr(); a.out = (float *)out.data_ptr();
     a.ld = src->stride(0); a.dt_ld = decay ? 0 : dt->stride(0); a.N = n; a.q_col = q_col; a.k_col = k_col; a.v_col = v_col; a.dtype = code(*src); a.act = act; a.B = B; a.H = H; a.G = G; a.D = D; a.Dv = Dv;
     RUN(jl_linear_scan, &a, stream_of(*src));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -453,11 +490,13 @@ CALL(embed_scale, 6)
     NEED(embed->dim() == 2 && known(*embed) && embed->is_contiguous() && ids->scalar_type() == at::kLong && ids->is_contiguous());
     const int64_t n = ids->numel(), W = embed->size(1);
     NEED(n > 0 && W > 0 && (!into || (is_float(*into) && into->is_contiguous() && rows(*into, n, W))));
+    Unlocked others;
     Tensor x = into ? *into : make({n, W}, at::kFloat, *embed), x0;
     if (copy) x0 = make({n, W}, type, *embed);
     const bool wide = type == at::kFloat;
     RUN(jl_embed_scale, embed->data_ptr(), code(*embed), (const int64_t *)ids->data_ptr(), n, (int32_t)W, (float)scale, (float *)x.data_ptr(), wide ? (float *)at_(x0) : nullptr,
                           wide ? nullptr : at_(x0), stream_of(*embed));
+    others.back();
     if (into) { Py_INCREF(arg[4]); return Py_BuildValue("(NN)", arg[4], wrap(x0)); }
     return Py_BuildValue("(NN)", wrap(x), wrap(x0));
 END_CALL
@@ -477,10 +516,12 @@ CALL(qk_norm_append, 21)
     NEED(k->scalar_type() == type && v->scalar_type() == type && k->is_contiguous() && v->is_contiguous() && k->dim() > 0 && v->dim() > 0 && k->size(-1) == (int64_t)G * D &&
          v->size(-1) == (int64_t)G * Dv && k->size(0) == v->size(0));
     NEED(rot_dims == 0 || (pos && n == proj->size(0) && rot_dims > 0 && rot_dims % 2 == 0 && rot_dims <= D && angles(rot_dims, cos, sin, max_pos, length)));
+    Unlocked others;
     Tensor q = make({proj->size(0), (int64_t)H * D}, type, *proj);
     RUN(jl_qk_norm_append, proj->data_ptr(), code(*proj), proj->size(0), proj->size(1), q_col, k_col, v_col, H, G, D, Dv, wq->data_ptr(), wk->data_ptr(), (float)eps, q.data_ptr(), k->data_ptr(),
         v->data_ptr(), (const int64_t *)kv_slot->data_ptr(), rot_dims, pairing, rot_dims ? (const int32_t *)at_(pos) : nullptr, rot_dims ? (const float *)at_(cos) : nullptr,
         rot_dims ? (const float *)at_(sin) : nullptr, stream_of(*proj));
+    others.back();
     return wrap(q);
 END_CALL
 
@@ -507,6 +548,7 @@ CALL(moe_experts, 15)
              w_router->size(0) == Er && w_router->size(1) == x->size(1) && row_weights(bias, Er));
     } else NEED(is_float(*x) && x->is_contiguous() && rows(*x, n, Er) && !bias && slices == 1);
     const int64_t max_tiles = rows_ / tm + E, blocks = p_jl_moe_router_blocks(n), lists = rows_ + E + 2 + 2 * max_tiles + blocks * E;
+    Unlocked others;
     Tensor ids = make({n, top}, at::kInt, *h), weights = make({n, top}, at::kFloat, *h), list = make({lists + (slices > 1 ? slices * n * Er : 0)}, at::kInt, *h);
     int32_t *perm = (int32_t *)list.data_ptr(), *offsets = perm + rows_, *tile_expert = offsets + E + 2, *tile_row0 = tile_expert + max_tiles;
     jl_moe_router a = {};
@@ -524,6 +566,7 @@ CALL(moe_experts, 15)
              act.data_ptr(), st);
     RUN(jl_moe_gemm, act.data_ptr(), w_down->data_ptr(), code(*h), 1, (int32_t)ff, (int32_t)W, top, perm, offsets, tile_expert, tile_row0, (int32_t)max_tiles, (int32_t)E, tm, a.weights, y.data_ptr(),
         st);
+    others.back();
     if (!identity) return wrap(y);
     return Py_BuildValue("(NNN)", wrap(y), wrap(ids), wrap(weights));
 END_CALL

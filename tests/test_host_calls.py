@@ -209,3 +209,37 @@ def test_linear_lets_transforms_and_modes_pass(n):
         with torch.device(dev):
             LO.linear(x, w, b)
     assert not calls
+
+
+@pytest.mark.gpu
+def test_other_threads_run_beside_a_launch(tmp_path):
+    """A launch that waits (for a full queue, here by sleeping) holds no lock that other threads of the program need."""
+    import ctypes as C
+    import importlib.machinery
+    import importlib.util
+    import shutil
+    import subprocess
+    import threading
+    import time
+    from jacobiforcing_amd import _build, _native as N, layer_ops as LO
+    (tmp_path / "wait.c").write_text("#include <unistd.h>\nint wait_in_a_launch() { usleep(500000); return 0; }\n")
+    subprocess.check_call([shutil.which("gcc") or "cc", "-shared", "-fPIC", "-O1", str(tmp_path / "wait.c"), "-o", str(tmp_path / "wait.so")])
+    wait = C.CDLL(str(tmp_path / "wait.so"))
+    own = shutil.copy(_build.HOST_LIB, tmp_path / "own.so")                                   # a module of its own: the package's keeps its launches
+    loader = importlib.machinery.ExtensionFileLoader("_jl_host", str(own))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_jl_host", loader))
+    loader.exec_module(module)
+    L, address = N.layers(), lambda f: C.cast(f, C.c_void_p).value
+    symbols = {name: address(getattr(L, name)) for name in module.symbols()}
+    symbols["jl_last_error"], symbols["jl_last_error of the recurrences"] = (address(L._library(name).jl_last_error) for name in ("jl_linear_small", "jl_linear_scan"))
+    symbols["jl_linear_small"] = address(wait.wait_in_a_launch)
+    module.bind(symbols, LO.LINEAR_SMALL_ROWS, LO.LINEAR_ONE_TILE, LO.LINEAR_X_BYTES)
+    x, w = torch.zeros(4, 64, device="cuda"), torch.zeros(64, 64, device="cuda")
+    taken = []
+    thread = threading.Thread(target=lambda: taken.append(module.linear(x, w, None, None)))
+    last, longest, alive = time.monotonic(), 0.0, True
+    thread.start()
+    while alive:
+        alive, now = thread.is_alive(), time.monotonic()
+        last, longest = now, max(longest, now - last)
+    assert torch.is_tensor(taken[0]) and longest < 0.25, longest
