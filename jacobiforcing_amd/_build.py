@@ -6,6 +6,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 from pathlib import Path
 
@@ -27,15 +28,20 @@ LAYERS_HEADERS = [CSRC / "layers" / "jl_common.h", CSRC / "layers" / "jl_attn.h"
 
 
 # the wrappers' host side (a CPython module on torch's C++ interface), beside the libraries that it calls
-HOST_SOURCE, HOST_LIB = CSRC / "layers" / "jl_host.cpp", LIB_DIR / "_jl_host.so"
+HOST_SOURCE = CSRC / "layers" / "jl_host.cpp"
+
+
+def host_lib() -> Path:
+    """Where the host side for this interpreter and this torch lies: one built for another is not theirs to load."""
+    import torch
+    return LIB_DIR / f"_jl_host.{sysconfig.get_config_var('SOABI')}.torch-{torch.__version__}.so"
 
 
 def build_host(force: bool = False) -> Path:
-    """``lib/_jl_host.so`` with the compiler of the host; nothing of it runs on the GPU."""
-    if not force and not stale(HOST_LIB, [HOST_SOURCE, ROOT / "include" / "jf_layers.h"]):
-        return HOST_LIB
-    import sysconfig
-
+    """``host_lib()`` with the compiler of the host; nothing of it runs on the GPU."""
+    lib = host_lib()
+    if not force and not stale(lib, [HOST_SOURCE, ROOT / "include" / "jf_layers.h"]):
+        return lib
     import torch
     from torch.utils import cpp_extension
     LIB_DIR.mkdir(parents=True, exist_ok=True)
@@ -47,8 +53,8 @@ def build_host(force: bool = False) -> Path:
                                f"-L{cpp_extension.library_paths()[0]}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-o", out], stderr=subprocess.PIPE, text=True)
         if done.returncode:
             raise RuntimeError(f"the compiler failed on jl_host.cpp:\n{done.stderr[-4000:]}")
-        os.replace(out, HOST_LIB)
-    return HOST_LIB
+        os.replace(out, lib)
+    return lib
 
 
 def layer_lib(group: str) -> Path:

@@ -439,24 +439,32 @@ def layers():
     return _LAYERS
 
 
+class _NoHost:
+    """In the place of a host side that could not be had: takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
 def host(*rules):
-    """The host's side of the small launches (csrc/layers/jl_host.cpp), bound to both kernel libraries; built when there is none.  ``rules``: the numbers that ``linear``'s rules go by."""
+    """The host's side of the small launches (csrc/layers/jl_host.cpp), bound to both kernel libraries; built when there is none for this torch.  ``rules``: the numbers that ``linear``'s rules go by.
+    Where it can be neither built nor loaded the wrappers make the same launches by themselves, some us later each, and a warning says so."""
     import importlib.machinery
     import importlib.util
+    import warnings
     from . import _build
-    if not _build.HOST_LIB.exists():
-        try:
-            _build.build_host()
-        except Exception as e:
-            raise NativeLibraryError(f"cannot build {_build.HOST_LIB}: {e}") from e
+    lib = _build.host_lib()
     try:
-        loader = importlib.machinery.ExtensionFileLoader("_jl_host", str(_build.HOST_LIB))
+        if not lib.exists():
+            _build.build_host()
+        loader = importlib.machinery.ExtensionFileLoader("_jl_host", str(lib))
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_jl_host", loader))
         loader.exec_module(module)
-    except ImportError as e:
-        raise NativeLibraryError(f"cannot load {_build.HOST_LIB}: {e}") from e
+    except (ImportError, OSError, RuntimeError) as e:
+        warnings.warn(f"the layer calls take more of the host: {lib.name} could not be built or loaded ({e})", RuntimeWarning, stacklevel=3)
+        return _NoHost()
     if module.version != JL_VERSION:
-        raise NativeLibraryError(f"{_build.HOST_LIB} has version {module.version}, this package calls version {JL_VERSION}: build it again (python -c 'import __graft_entry__ as g; g.build()')")
+        raise NativeLibraryError(f"{lib} has version {module.version}, this package calls version {JL_VERSION}: build it again (python -c 'import __graft_entry__ as g; g.build()')")
     L, address = layers(), lambda fn: C.cast(fn, C.c_void_p).value
     symbols = {name: address(getattr(L, name)) for name in module.symbols()}
     symbols["jl_last_error"], symbols["jl_last_error of the recurrences"] = (address(L._library(name).jl_last_error) for name in ("jl_linear_small", "jl_linear_scan"))

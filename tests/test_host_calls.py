@@ -53,6 +53,25 @@ def test_what_it_does_not_take():
     assert H.moe_experts(*[None] * 15) is NotImplemented and H.attention_args(*[7] * 30) is NotImplemented and H.linear_scan(*[x] * 19) is NotImplemented
 
 
+@pytest.mark.parametrize("broken", ["no compiler", "not a library"])
+def test_without_it(monkeypatch, tmp_path, broken):
+    """Where the module can be neither built nor loaded the wrappers go their own way, with a warning; one built for another torch is not found."""
+    from jacobiforcing_amd import _build, _native as N, layer_ops as LO
+    assert torch.__version__ in _build.host_lib().name
+    monkeypatch.setattr(torch, "__version__", "0.1")
+    assert not _build.host_lib().exists()
+    monkeypatch.setattr(_build, "LIB_DIR", tmp_path)
+    if broken == "no compiler":
+        monkeypatch.setenv("PATH", "/nowhere")
+        monkeypatch.setattr(_build, "hipcc", lambda: "/nowhere/hipcc")
+    else:
+        _build.host_lib().write_text("")
+    with pytest.warns(RuntimeWarning, match="more of the host"):
+        H = N.host(LO.LINEAR_SMALL_ROWS, LO.LINEAR_ONE_TILE, LO.LINEAR_X_BYTES)
+    x = torch.randn(4, 64)
+    assert H.linear(x, x, None, None) is NotImplemented and H.moe_experts() is NotImplemented
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n", [1, 5, 130])
@@ -225,7 +244,7 @@ def test_other_threads_run_beside_a_launch(tmp_path):
     (tmp_path / "wait.c").write_text("#include <unistd.h>\nint wait_in_a_launch() { usleep(500000); return 0; }\n")
     subprocess.check_call([shutil.which("gcc") or "cc", "-shared", "-fPIC", "-O1", str(tmp_path / "wait.c"), "-o", str(tmp_path / "wait.so")])
     wait = C.CDLL(str(tmp_path / "wait.so"))
-    own = shutil.copy(_build.HOST_LIB, tmp_path / "own.so")                                   # a module of its own: the package's keeps its launches
+    own = shutil.copy(_build.host_lib(), tmp_path / "own.so")                                   # a module of its own: the package's keeps its launches
     loader = importlib.machinery.ExtensionFileLoader("_jl_host", str(own))
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_jl_host", loader))
     loader.exec_module(module)
