@@ -348,9 +348,9 @@ __global__ __launch_bounds__(256, 2) void latent_heads_kernel(jl_latent_heads a)
             const int m = e / a.rd, d = e - m * a.rd;
             if (n0 + m >= a.N) break;
             const bf16_t *from = (const bf16_t *)a.x + (n0 + m) * a.x_ld + (int64_t)h * a.x_head + K;
-            const float *cs = a.cos_t + (int64_t)a.pos[n0 + m] * half, *sn = a.sin_t + (int64_t)a.pos[n0 + m] * half;
             float v = ld_f(from + d);
-            if (d < a.rot_dims) {
+            if (d < a.rot_dims) {                                    // (without a rotation there are no positions and no tables)
+                const float *cs = a.cos_t + (int64_t)a.pos[n0 + m] * half, *sn = a.sin_t + (int64_t)a.pos[n0 + m] * half;
                 const bool near = a.pairing == JL_ROT_NEIGHBOURS, second = near ? d & 1 : d >= half;
                 const int i = near ? d >> 1 : second ? d - half : d;
                 const float other = ld_f(from + (near ? d ^ 1 : second ? d - half : d + half));

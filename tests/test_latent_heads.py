@@ -57,6 +57,21 @@ def test_rows_and_heads_that_do_not_meet():
     assert torch.equal(got, clean)
 
 
+def test_a_part_that_is_not_rotated_needs_no_positions():
+    """Through the C interface, where positions and tables may be left out then."""
+    import ctypes as C
+    from jacobiforcing_amd import _native as N, layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x, w = torch.randn(5, 2 * 48, generator=g, device="cuda").bfloat16(), torch.randn(2, 32, 40, generator=g, device="cuda").bfloat16()
+    out = torch.empty(5, 2 * 56, dtype=torch.bfloat16, device="cuda")
+    a = N.LatentHeads(x=x.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), N=5, x_ld=96, out_ld=112, H=2, K=32, O=40, x_head=48, out_head=56, rd=16, rot_dims=0, pairing=0)
+    N.check_layers(N.layers().jl_latent_heads_run(C.byref(a), LO._stream(x.device)), "jl_latent_heads_run")
+    want = x.double().view(5, 2, 48)
+    assert torch.equal(out.view(5, 2, 56)[..., 40:], x.view(5, 2, 48)[..., 32:])
+    want = (want[..., :32].unsqueeze(-2) @ w.double()).squeeze(-2)
+    assert bool(((out.view(5, 2, 56)[..., :40].double() - want).abs() <= 2.0 ** -8 * want.abs() + 64 * 2.0 ** -24 * 32).all())
+
+
 def test_attention_takes_them_and_agrees(monkeypatch):
     """A layer's result with the package's products and with the library's: the same within their roundings, and nothing is refused or accepted that was not."""
     from jacobiforcing_amd import layer_ops as LO
