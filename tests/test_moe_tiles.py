@@ -101,18 +101,32 @@ def test_tile_heights_of_each_type():
     assert lib.jl_moe_gemm(x.data_ptr(), x.data_ptr(), N.JL_F32, N.JL_MOE_UP_PLAIN, 64, 64, 1, i.data_ptr(), i.data_ptr(), i.data_ptr(), i.data_ptr(), 1, 1, 128, None, x.data_ptr(), None) == -1
 
 
-@pytest.mark.parametrize("dtype,tile", [("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128), ("float32", 32), ("float32", 64)])
+@pytest.mark.parametrize("dtype,tile", [("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128), ("float32", 32), ("float32", 64), ("float32", 256)])
 @pytest.mark.parametrize("N,E,top,W,ff,gated,identity,skew", [
     (1, 3, 2, 8, 8, True, 0, 0.0), (130, 3, 2, 24, 32, True, 0, 0.0), (259, 4, 2, 64, 96, True, 1, 0.0), (257, 2, 1, 96, 64, False, 0, 0.0), (300, 5, 2, 72, 264, True, 0, 0.0), (200, 3, 1, 64, 50, True, 0, 0.0),
     (513, 9, 1, 160, 136, False, 0, 9.0), (1100, 2, 1, 520, 264, True, 0, 1.0), (640, 40, 2, 40, 256, True, 4, 3.0), (385, 4, 3, 1024, 520, True, 0, 0.0),
 ])
 def test_every_tile_height(monkeypatch, dtype, tile, N, E, top, W, ff, gated, identity, skew):
     """The same with tiles of one height: depths of one, two, three and more stages, beside and below them, columns beside their fours, experts with few rows, many or none."""
-    from jacobiforcing_amd import _native as N_
-    asked = []
-    monkeypatch.setattr(N_.layers(), "jl_moe_tile_rows", lambda *a: asked.append(a) or tile, raising=False)
+    from jacobiforcing_amd import _native as N_, layer_ops as LO
+    lib, host, launched = N_.layers(), LO._host(), []
+    gemm = lib.jl_moe_gemm
+
+    class Watched:
+        def __getattr__(self, name):
+            def call(*a):
+                r = getattr(host, name)(*a)
+                if name == "moe_experts" and r is not NotImplemented:
+                    launched.append(a[13])
+                return r
+            return call
+    monkeypatch.setattr(lib, "jl_moe_tile_rows", lambda *a: 64 if (dtype, tile) == ("float32", 256) else tile, raising=False)
+    monkeypatch.setattr(lib, "jl_moe_float_tiles", lambda *a: tile, raising=False)
+    monkeypatch.setattr(lib, "jl_moe_tile_pairs", lambda *a: 0, raising=False)
+    monkeypatch.setattr(lib, "jl_moe_gemm", lambda *a: launched.append(a[13]) or gemm(*a), raising=False)
+    monkeypatch.setattr(LO, "_H", Watched())
     test_experts(dtype, N, E, top, W, ff, gated, identity, skew)
-    assert asked
+    assert launched and set(launched) == {tile}, launched
 
 
 @pytest.mark.parametrize("dtype,tile,N,E,W,ff", [("bfloat16", 128, 4096, 16, 1024, 512), ("bfloat16", 64, 3000, 40, 520, 256), ("float32", 64, 2048, 16, 1024, 256)])
