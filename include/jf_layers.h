@@ -217,7 +217,8 @@ JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, cons
                          void *stream);
 
 /* The same for float rows of any number (x [N, x_ld], W [O, K], rows at 16-byte borders, out rows out_ld floats apart), on the bfloat16 matrix instructions in three terms per operand: sums at
- * least as close to 64 bits as the float instructions' (products below 2^-110 aside).  jl_linear_split_ok: whether that is the better launch for these sizes. */
+ * least as close to 64 bits as the float instructions' (measured at depths of 4 to 4096), but for operands below 2^-118, whose digits beyond bfloat16's last place, 2^-133, are lost.  Infinities, NaN
+ * and operands beyond bfloat16's greatest number count as they are.  jl_linear_split_ok: whether that is the better launch for these sizes. */
 JL_API int jl_linear_split_ok(int64_t N, int64_t K, int64_t O);
 JL_API int jl_linear_split(const float *x, int64_t N, int64_t x_ld, const float *w, int32_t K, int32_t O, const float *bias, float *out, int64_t out_ld, void *stream);
 
@@ -363,7 +364,9 @@ JL_API int jl_retention_join(const int32_t *req, int32_t B, const int32_t *chunk
 /* The same for long portions on the matrix cores: every request's portion cut into pieces of piece_tokens (a multiple of 64) tokens, the last of a request
  * what is left, that run side by side (own contributions to the state, the state each starts from, outputs).  piece_rec [pieces, 4] int32 {row0, count, slot,
  * 1 for a request's last piece}; req [B, 4] int32 {first piece, pieces, pos0, slot}, of requests that have rows alone (B counts these records: one of no rows
- * would hide that another has several pieces); pos [N] int32 position of every row; scratch [pieces, H, D, Dv] and raw [N, H * Dv] float.
+ * would hide that another has several pieces); pos [N] int32 position of every row, one behind the other within a piece; scratch [pieces, H, D, Dv] and raw [N, H * Dv] float.
+ * Queries, keys, states, decayed values and the pairs' weights are multiplied in three bfloat16 terms: those below 2^-118 lose digits beyond 2^-133; infinities and floats beyond bfloat16's
+ * greatest number count as they are.
  * Sizes as jl_retention_pieces_ok takes them; ld and columns in multiples of four, rows and tables at the borders of four elements. */
 typedef struct jl_retention_pieces {
     const void *proj;
@@ -484,7 +487,8 @@ JL_API int jl_moe_router_run(const jl_moe_router *a, void *stream);
  *   mode 0 (up):   in(r) = perm[r] / top;  out[r, :] = relu(C)^2, stored in `dtype` ([N*top, n_out], sorted order)
  *   mode 1 (down): in(r) = r;              out[perm[r], :] = C * weights[perm[r]], stored as float ([N*top, n_out])
  *   mode JL_MOE_UP_PLAIN: as mode 0 without the activation (out[r, :] = C): a gated unit stacks its gate and linear branch in W and
- *                  applies jl_gated_act to the result */
+ *                  applies jl_gated_act to the result
+ * Float rows in tiles of 64 and 256 are multiplied in three bfloat16 terms per operand, as jl_linear_split does: operands below 2^-118 lose digits beyond 2^-133. */
 #define JL_MOE_UP_PLAIN 2
 JL_API int jl_moe_gemm(const void *X, const void *Wt, int dtype, int32_t mode, int32_t K, int32_t n_out, int32_t top,
                        const int32_t *perm, const int32_t *offsets, const int32_t *tile_expert, const int32_t *tile_row0,

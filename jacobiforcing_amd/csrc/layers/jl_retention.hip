@@ -225,7 +225,7 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // Values that are not finite reach the tokens from their own on and the state, as in the scan, though products run over whole groups: they are left out of them, and their columns' outputs and state set behind.
 // Numbers that no bfloat16 number comes near (infinities, and floats between the two types' ends) have no terms: groups whose outputs are not all finite, and contributions of keys or values like that, are
 // formed on the float instructions from the numbers themselves, so that sums of one sign stay infinite and finite ones finite (looking for them takes 2 %: 4 x 2048 tokens 104 / 106 us).  Numbers below
-// 2^-110 lose the bits of their terms that lie below bfloat16's last place, 2^-133.
+// 2^-118 lose the digits of their terms that lie below bfloat16's last place, 2^-133.
 // Outputs leave as floats and are normed and gated by rows in a launch of their own.
 constexpr int RM_T = 64, RC_T = 32, RM_OUT = 0, RM_LOCAL = 1, RC_VROW = 128 + 16;      // RM_T: pieces come in multiples of it
 typedef float rm_f32x16 __attribute__((ext_vector_type(16)));

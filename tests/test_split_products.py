@@ -52,6 +52,22 @@ def test_values_that_are_not_finite(N, K, O):
     assert bool(((got - clean).abs()[rest] <= (K + 64) * 2.0 ** -24 * (x.abs() @ w.abs().T)[rest]).all())
 
 
+@pytest.mark.parametrize("low", [-110, -118, -122, -126, -130])
+def test_the_smallest_operands(low):
+    """Operands near float's end, against large ones: their terms end with bfloat16's last place, 2^-133, so half of it is lost of each, and nothing that shows from 2^-118 on."""
+    from jacobiforcing_amd import layer_ops as LO
+    dev, N, K, O = "cuda", 640, 512, 4096
+    assert LO.linear_split(N, K, O)
+    g = torch.Generator(device=dev).manual_seed(1)
+    x, w = (torch.rand(N, K, generator=g, device=dev) + 1) * 2.0 ** low, (torch.rand(O, K, generator=g, device=dev) + 1) * 2.0 ** 90
+    got, want = LO.linear(x, w).double(), x.double() @ w.double().T                           # all of one sign: a product's size is its value
+    lost = 2.0 ** -134 * w.double().sum(1)
+    assert bool(((got - want).abs() <= lost + ((6 * K / 16 + 32) * 2.0 ** -24 + 2.0 ** -22) * want).all())
+    if low >= -118:
+        # (-118: 2^-134 of 2^-118 is 2^-16 of an operand at most, and a mean of K of them, of either sign, 2^-20)
+        assert float((got - want).norm() / want.norm()) <= 2.0 ** -19
+
+
 @pytest.mark.parametrize("n,W,ff,E,top,gated,bad", [(1700, 36, 2052, 10, 2, True, False), (3300, 2060, 100, 4, 1, False, False), (3500, 1024, 520, 6, 1, True, True), (800, 1028, 516, 12, 4, True, True),
                                                      (705, 516, 1028, 6, 4, False, True)])
 def test_experts(n, W, ff, E, top, gated, bad):
