@@ -1728,7 +1728,7 @@ __global__ __launch_bounds__(FH_TPB, 1) void rs_filter_hist_kernel(const void *l
 // What bounds it: up to 512 rows the chain of one row (35 us of counting at 496 rows, whose bytes take 29, then 20 of reductions, one after another, then the tie pass), beyond them HBM.  The tie pass read
 // the row again, on average half of it.  Now the count pass keeps the greatest pattern of every thread's eight tiles (one packed maximum per word), and only threads that hold a value at or above the
 // lower cut read their eight vectors again and write their members' ids to a list.  Two rows per CU: the 85 registers of three spilled 193, which cost more than the third row gave.  us per call, rows of
-// 152 064, top-k 50 and top-p 0.9, before / now: 31 rows 74 / 59, 124 81 / 62, 496 104 / 81, 620 117 / 113, 992 163 / 142, 1984 279 / 250; top-p alone 98 / 77, 496 rows 133 / 106, 1984 367 / 326.
+// 152 064, top-k 50 and top-p 0.9, before / now: 31 rows 80 / 57, 124 88 / 61, 496 114 / 79, 620 131 / 122, 992 187 / 135, 1984 303 / 250; top-p alone 110 / 77, 496 rows 147 / 107, 1984 415 / 332.
 // ------------------------------------------------------------------------------------------------
 constexpr int ZN_TPB = 512, ZN_SLOTS = 8192, ZN_TINY = 64, ZN_EXP_LO = 111, ZN_EXP_HI = 142;
 constexpr uint32_t ZN_LO16 = (uint32_t)ZN_EXP_LO << 7;                       // first magnitude pattern of the table

@@ -8,7 +8,8 @@
 // What bounds it: the keys' way through LDS, the softmax's issue and the matrix instructions, about as long each; few rows: latency of launch, loads and barriers (15 us with one round of keys and with five;
 // loads two rounds ahead changed nothing).  us, bfloat16, 32 tokens, 8 heads of 128 over 2, context 512, before (tiles of 128 rows, keys shared out over up to three workgroups) / now: 64 rows
 // 30.2 / 20.6, 32 27.1 / 19.0, 16 23.8 / 18.1, one 16.7 / 16.1; context 4000, one row 42.7 / 25.4, 8 rows 45.4 / 30.7; 32 rows, 14 heads of 64 over 2, context 1000 27.7 / 18.2.  Many rows (scores scaled
-// in the exponent's own instruction): 128 rows 35.4 / 30.2; 64 rows of 64, 16 heads over 2, context 1500 111.8 / 93.2; 64 rows, 28 heads of 128 over 4, context 1000 79.6 / 67.3.
+// in the exponent's own instruction; rows whose scores are beyond 2^24 apart, ar_factor): 128 rows 35.4 / 30.2; 64 rows of 64, 16 heads over 2, context 1500 111.8 / 93.2; 64 rows, 28 heads of 128 over 4,
+// context 1000 79.6 / 67.3; 96 rows of the first, two shares, context 1500 55 / 52.
 // Sums scaled only when a maximum has grown by 2^8 would give 4 to 7 % more, but the greatest weight is then no longer 1 but a rounded one: errors against 64 bits of peaked rows grew by 12 %.
 // The library's attention with a mask tensor and the copy that its output needs: the first 47, the one row 40, the 14 heads 89, the last two 182 and 199.
 #include "jl_attn.h"

@@ -22,7 +22,8 @@ constexpr int AR_THREADS = 256;
 //   1 x 8192 tokens, the same heads                        1728 -> 434 us (633 TFLOP/s)
 //   4 x 2048 tokens, 16 heads of 192 / 128 apart           806 -> 180 us (479 TFLOP/s)
 //   4 x 2048 tokens, 8 heads of 128 over 2, window 1024    180 -> 66 us
-// Scores scaled in the exponent's multiply-add behind their maximum (queries take a negative scale's sign) instead of one by one: the first 129 -> 124, the second 393 -> 383.
+// Scores scaled in the exponent's multiply-add behind their maximum (queries take a negative scale's sign) instead of one by one: the first 129 -> 124, the second 393 -> 383; rows whose
+// maximum is beyond 2^24, which would go wrong so, are multiplied one by one in the branch that scales the sums (ar_factor; the look at every tile instead: 2 to 5 %).
 
 constexpr int ar_tile_keys(int KU) { return KU <= 16 ? 64 : 32; }
 constexpr size_t ar_lds_bytes(int KU, int VU) { return 2 * (size_t)ar_tile_keys(KU) * (KU + VU) * 16 + 2 * ar_tile_keys(KU) * 4; }

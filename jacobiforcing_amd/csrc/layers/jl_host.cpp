@@ -3,7 +3,8 @@
 //
 // Every function takes the arguments of the wrapper of its name (a batch's fields one by one), looks at everything the wrapper would, allocates the result and launches.  Whatever it does not
 // take in full - other types, shapes, layouts or devices, tensor subclasses, a mode that overrides calls, gradients where the wrapper looks for them, a call that the library refuses - it leaves to the
-// wrapper by returning NotImplemented before anything has happened, and the wrapper takes its general way or raises.  A launch that failed is raised here.  Nothing is kept between calls but the kernel libraries' addresses (bind).
+// wrapper by returning NotImplemented before anything has happened, and the wrapper takes its general way or raises (moe_experts, whose later launches may refuse what the first took, leaves results
+// behind that the wrapper forms again).  A launch that failed is raised here.  Nothing is kept between calls but the kernel libraries' addresses (bind).
 #include <Python.h>
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
