@@ -2,12 +2,13 @@
 // wrappers in Python took 6 more, which bounds steps of a few tokens (one token through Safisun's four layers: 49 launches).
 //
 // Every function takes the arguments of the wrapper of its name (a batch's fields one by one), looks at everything the wrapper would, allocates the result and launches.  Whatever it does not
-// take in full - other types, shapes, layouts or devices, tensor subclasses, a mode that overrides calls, gradients where the wrapper looks for them, a call that the library refuses - it leaves to the
+// take in full - other types, shapes, layouts or devices, tensor subclasses, a mode that overrides calls, a trace, gradients where the wrapper looks for them, a call that the library refuses - it leaves to the
 // wrapper by returning NotImplemented before anything has happened, and the wrapper takes its general way or raises (moe_experts, whose later launches may refuse what the first took, leaves results
 // behind that the wrapper forms again).  A launch that failed is raised here.  Nothing is kept between calls but the kernel libraries' addresses (bind).
 #include <Python.h>
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -95,7 +96,7 @@ struct Unlocked {
     ~Unlocked() { back(); }
 };
 Tensor make(at::IntArrayRef size, at::ScalarType type, const Tensor &like) { return at::empty(size, at::TensorOptions().dtype(type).device(like.device())); }
-bool overridden() { return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+bool overridden() { return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled(); }
 PyObject *wrap(const Tensor &t) { return t.defined() ? THPVariable_Wrap(t) : (Py_INCREF(Py_None), Py_None); }
 
 // the addends of a residual update: a list or tuple of (y [N, W] or [N, S, W], float scale [W] or None)

@@ -383,9 +383,9 @@ def linear_split(n: int, k: int, o: int) -> bool:
 
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
     """Whether a launch on these tensors' memory is all that a library's call on them would be: no subclass (fake tensors among them), transform's wrapper, lazy form, sparse layout or forward-mode
-    tangent, and no mode that is to see the call (one that only names a default device has nothing to see)."""
+    tangent, no trace that records calls, and no mode that is to see the call (one that only names a default device has nothing to see)."""
     modes = torch.overrides._get_current_function_mode_stack() if torch._C._len_torch_function_stack() else ()
-    if torch._C._len_torch_dispatch_stack() or any(type(m) is not DeviceContext for m in modes):
+    if torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() or any(type(m) is not DeviceContext for m in modes):
         return False
     dual = forward_ad._current_level >= 0
     return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout == torch.strided and not torch._C._functorch.is_functorch_wrapped_tensor(t) and not t.is_neg() and
@@ -397,16 +397,18 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     (``linear_split``), the library's product for the others and for what a launch would pass by (``_plain``).  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
-    r = (_H or _host()).linear(x, w, bias, float_out)
-    if r is not NotImplemented:
-        return r
+    launch = not torch.compiler.is_dynamo_compiling()    # (a compiler follows the library's call alone)
+    if launch:
+        r = (_H or _host()).linear(x, w, bias, float_out)
+        if r is not NotImplemented:
+            return r
     n, k = x.shape
     o, dt, wt = w.shape[0], x.dtype, w.dtype
     same = wt == dt
     _need(same or (wt == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
-    small = n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
-    split = not small and wt == torch.float32 and linear_split(n, k, o)
-    if (small or split or (same and linear_mid(n, k, o, dt))) and _plain(x, w, bias):
+    small = launch and n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
+    split = launch and not small and wt == torch.float32 and linear_split(n, k, o)
+    if launch and (small or split or (same and linear_mid(n, k, o, dt))) and _plain(x, w, bias):
         size = w.element_size()
         if (w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and
                 (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == wt and bias.shape == (o,) and bias.is_contiguous())) and dt in _LINEAR_TYPES and k > 0 and

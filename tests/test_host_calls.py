@@ -231,6 +231,21 @@ def test_linear_lets_transforms_and_modes_pass(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [4, 640])
+def test_linear_is_traced_and_compiled(n):
+    """A trace records the library's product, and so does a compiler, which finds no call that it cannot follow."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, y, w, b = (torch.randn(*s, generator=g, device="cuda") for s in ((n, 64), (n, 64), (2500, 64), (2500,)))
+    call, want = lambda v: LO.linear(v, w, b), y @ w.T + b
+    with torch.no_grad():
+        traced = torch.jit.trace(call, (x,), check_trace=False)
+        assert "linear" in str(traced.graph) and torch.allclose(traced(y), want, rtol=1e-4, atol=1e-4)
+        compiled = torch.compile(call, backend="eager", fullgraph=True)
+        assert torch.allclose(compiled(x), x @ w.T + b, rtol=1e-4, atol=1e-4) and torch.allclose(compiled(y), want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.gpu
 def test_other_threads_run_beside_a_launch(tmp_path):
     """A launch that waits (for a full queue, here by sleeping) holds no lock that other threads of the program need."""
     import ctypes as C
