@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -163,7 +164,7 @@ CALL(linear, 4)
     const int64_t n = x->size(0), k = x->size(1), o = w->size(0), ld = x->stride(0), size = w->element_size();
     const bool same = w->scalar_type() == x->scalar_type();
     NEED(same || (is_float(*w) && !typed && as_float));
-    const bool small = rule_small(n, k, o, size), split = !small && same && is_float(*w) && p_jl_linear_split_ok(n, k, o),
+    const bool small = rule_small(n, k, o, size), split = !small && same && is_float(*w) && p_jl_linear_split_ok(n, k, o) && !at::autocast::is_autocast_enabled(at::kCUDA),
                mid = !small && !split && same && !is_float(*x) && p_jl_linear_mid_ok(n, k, o);
     NEED(small || split || mid);
     NEED(w->size(1) == k && w->is_contiguous() && x->stride(1) == 1 && ld >= k && k > 0 && o > 0 && o <= INT32_MAX && k * size % 16 == 0 && ld * (int64_t)x->element_size() % 16 == 0 && starts16(*x) &&

@@ -407,7 +407,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     same = wt == dt
     _need(same or (wt == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
     small = launch and n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
-    split = launch and not small and wt == torch.float32 and linear_split(n, k, o)
+    split = launch and not small and wt == torch.float32 and linear_split(n, k, o) and not torch.is_autocast_enabled("cuda")
     if launch and (small or split or (same and linear_mid(n, k, o, dt))) and _plain(x, w, bias):
         size = w.element_size()
         if (w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and

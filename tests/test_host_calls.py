@@ -246,6 +246,17 @@ def test_linear_is_traced_and_compiled(n):
 
 
 @pytest.mark.gpu
+def test_linear_of_many_rows_under_autocast():
+    """Float products of many rows are the library's to round there."""
+    from jacobiforcing_amd import layer_ops as LO
+    x, w = torch.randn(640, 64, device="cuda"), torch.randn(2500, 64, device="cuda")
+    assert LO.linear_split(640, 64, 2500)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y, want = LO.linear(x, w), torch.nn.functional.linear(x, w)
+    assert y.dtype == want.dtype == torch.bfloat16 and torch.equal(y, want) and LO.linear(x, w).dtype == torch.float32
+
+
+@pytest.mark.gpu
 def test_other_threads_run_beside_a_launch(tmp_path):
     """A launch that waits (for a full queue, here by sleeping) holds no lock that other threads of the program need."""
     import ctypes as C
