@@ -20,6 +20,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.compiler import is_dynamo_compiling
 from torch.utils._device import DeviceContext
 
 from . import _native as N
@@ -397,7 +398,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     (``linear_split``), the library's product for the others and for what a launch would pass by (``_plain``).  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
-    launch = not torch.compiler.is_dynamo_compiling()    # (a compiler follows the library's call alone)
+    launch = not is_dynamo_compiling()    # (a compiler follows the library's call alone)
     if launch:
         r = (_H or _host()).linear(x, w, bias, float_out)
         if r is not NotImplemented:
