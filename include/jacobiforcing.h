@@ -504,8 +504,8 @@ JF_API int jf_rs_probs(const void *logits, int dtype, int64_t R, int64_t V, int6
  *                  the rows' statistics from here on (row_max, sum).
  *   workspace      jf_rs_filter_workspace_bytes(dtype, R, V) bytes, 16-byte aligned: none for bf16 rows of up to 524 288 ids (a
  *                  workgroup per row keeps the COUNT of every bf16 pattern of the row's scaled logits in LDS — the probability is a
- *                  monotone function of the pattern, so cuts, sums and tie groups are sums over <= 65 536 counters — and reads the
- *                  row a second time only to find the last kept id of a tie group); float32 rows use R x V x 4 bytes of scratch.
+ *                  monotone function of the pattern, so cuts, sums and tie groups are sums over <= 65 536 counters — and reads a
+ *                  second time only what may hold the last kept id of a tie group); float32 rows use R x V x 4 bytes of scratch.
  * top_k <= 0 or >= V, top_p <= 0 or >= 1: that stage is off (JDN:75, 95-96); top_p is compared AS GIVEN (a double): a value that
  * a float would round to 0 or 1 keeps its stage on.  packed / the greedy next-draft tail of jf_rs_probs are untouched (argmax
  * of the LOGITS, JDN:446).

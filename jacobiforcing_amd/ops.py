@@ -1021,7 +1021,7 @@ class RowFilter:
             need = self._need[(dt, R, V)] = int(lib.jf_rs_filter_workspace_bytes(dt, R, V))
         self.ws = _grown(self.ws, need)
         self.records = _grown(self.records, R * N.RS_FILTER_ROW_BYTES)
-        done = _stage("rs_filter", 2 * R * V * flat.element_size())          # the logits twice (pattern counts, tie ids): no tensor is written
+        done = _stage("rs_filter", R * V * flat.element_size())              # the logits once: no tensor is written, and most of a row is not read again for its tie ids
         N.check(lib.jf_rs_filter(_ptr(flat), dt, R, V, flat.stride(0) if R > 1 else V, _ptr(draft_next), float(temperature), int(top_k),
                                  float(top_p), _ptr(self.records), _ptr(p_draft), _ptr(row_max), _ptr(row_sumexp),
                                  _ptr(self.ws) if need else None, self.ws.numel() if need else 0, _stream(self.device)), "jf_rs_filter")
