@@ -68,6 +68,40 @@ def test_the_smallest_operands(low):
         assert float((got - want).norm() / want.norm()) <= 2.0 ** -19
 
 
+def _lean(got, want):
+    """The mean error against the values' root mean square, and what chance makes of it."""
+    e = (got.double() - want) / want.pow(2).mean().sqrt()
+    return float(e.mean().abs()), 5 * float(e.std()) / e.numel() ** 0.5
+
+
+# the instructions cut sums towards minus infinity: by 2^-27 of them at a depth of 96, 2^-22 at 4096, were they not held with either sign in turn, which leaves a step's cut against its neighbour's
+@pytest.mark.parametrize("N,K,O", [(4096, 96, 4096), (4096, 320, 4096), (6000, 832, 608), (2553, 2048, 3072), (4096, 4096, 4096), (640, 1100, 4096)])
+def test_sums_lean_neither_way(N, K, O):
+    from jacobiforcing_amd import layer_ops as LO
+    assert LO.linear_split(N, K, O)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, w = torch.randn(N, K, generator=g, device="cuda"), torch.randn(O, K, generator=g, device="cuda")
+    lean, chance = _lean(LO.linear(x, w), x.double() @ w.double().T)
+    assert lean <= 2.0 ** -28 + chance, lean
+
+
+@pytest.mark.parametrize("n,W,ff,E", [(4000, 1024, 1024, 4), (3200, 1028, 516, 12)])
+def test_experts_sums_lean_neither_way(n, W, ff, E):
+    """The way down, in parts of 128 rows and tiles of 64 (what the way up leans by meets weights of either sign)."""
+    from jacobiforcing_amd import _native as N, layer_ops as LO
+    assert N.layers().jl_moe_float_tiles(n, E, W, ff) == (256 if n >= 320 * E else 64) and N.layers().jl_moe_tile_rows(N.JL_F32, n, E, W, ff) == 64
+    g = torch.Generator(device="cuda").manual_seed(ff)
+    h, logits = torch.randn(n, W, generator=g, device="cuda"), torch.randn(n, E, generator=g, device="cuda")
+    up, down = torch.randn(E, ff, W, generator=g, device="cuda") * W ** -0.5, torch.randn(E, W, ff, generator=g, device="cuda") * ff ** -0.5
+    got, want = LO.moe_experts(h, logits, None, 1, 1.0, up, down, route="top_softmax")[:, 0], torch.zeros(n, W, dtype=torch.float64, device="cuda")
+    ids = logits.argmax(-1)
+    for e in range(E):
+        r = (ids == e).nonzero()[:, 0]
+        want[r] = torch.relu(h[r].double() @ up[e].double().T) ** 2 @ down[e].double().T
+    lean, chance = _lean(got, want)
+    assert lean <= 2.0 ** -28 + chance, lean
+
+
 @pytest.mark.parametrize("n,W,ff,E,top,gated,bad", [(1700, 36, 2052, 10, 2, True, False), (3300, 2060, 100, 4, 1, False, False), (3500, 1024, 520, 6, 1, True, True), (800, 1028, 516, 12, 4, True, True),
                                                      (705, 516, 1028, 6, 4, False, True)])
 def test_experts(n, W, ff, E, top, gated, bad):
