@@ -226,6 +226,9 @@ extern "C" int jl_retention_join(const int32_t *req, int32_t B, const int32_t *c
 // Numbers that no bfloat16 number comes near (infinities, and floats between the two types' ends) have no terms: groups whose outputs are not all finite, and contributions of keys or values like that, are
 // formed on the float instructions from the numbers themselves, so that sums of one sign stay infinite and finite ones finite (looking for them takes 2 %: 4 x 2048 tokens 104 / 106 us).  Numbers below
 // 2^-118 lose the digits of their terms that lie below bfloat16's last place, 2^-133.
+// The instructions cut what they add to a sum towards minus infinity, which would make all states and outputs lean one way (states by 0.1e-7 of their root mean square at decays of 0.97, 0.4e-7 at 0.9998, and
+// with them all tokens to come); so states and queries have a minus sign in half of the groups, which leaves 0.01e-7 and 0.09e-7.  us of the whole layer, without / with: 4 x 2048 tokens 100.6 / 103.8, of 64 62.9 / 65.0,
+// the float ones 77.1 / 79.6, one portion of 128 33.9 / 35.6.
 // Outputs leave as floats and are normed and gated by rows in a launch of their own.
 constexpr int RM_T = 64, RC_T = 32, RM_OUT = 0, RM_LOCAL = 1, RC_VROW = 128 + 16;      // RM_T: pieces come in multiples of it
 typedef float rm_f32x16 __attribute__((ext_vector_type(16)));
@@ -234,9 +237,10 @@ typedef __bf16 rm_bf16x4 __attribute__((ext_vector_type(4)));
 typedef short rm_s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) rm_s16x4 rm_lds_s16x4;
 constexpr int RM_TERMS = JL_SPLIT_TERMS;
+__device__ __forceinline__ float rm_signed(float v, uint32_t sign) { return __uint_as_float(__float_as_uint(v) ^ sign); }
 constexpr float RM_BEYOND = 3.395e38f;                               // bfloat16 ends at 3.3895e38; from 3.3953e38 on a float is rounded to infinity
 template <typename T> static constexpr size_t rm_lds_bytes(int DP, bool out) {
-    return 2 * RC_T * ((out ? 2 : 1) * (size_t)RM_TERMS * (DP + 8) + (sizeof(T) == 4 ? RM_TERMS : 1) * RC_VROW) + (RC_T + 2 * RC_T + 4 * RC_T + 4) * 4;
+    return 2 * RC_T * ((out ? 2 : 1) * (size_t)RM_TERMS * (DP + 8) + (sizeof(T) == 4 ? RM_TERMS : 1) * RC_VROW) + (RC_T + 4 * RC_T + 4 * RC_T + 4) * 4;
 }
 
 template <typename T, int DP, int MODE>
@@ -248,8 +252,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
     const int row0 = a.piece_rec[4 * piece], cnt = a.piece_rec[4 * piece + 1], slot = a.piece_rec[4 * piece + 2], last = a.piece_rec[4 * piece + 3];
     if (cnt <= 0 || (!OUT && last)) return;
     bf16_t *Ks = (bf16_t *)smem, *Vs = Ks + RM_TERMS * RC_T * QROW, *Qs = Vs + VT * RC_T * RC_VROW;      // [terms][32][..]
-    float *g1 = (float *)(Qs + (OUT ? RM_TERMS * RC_T * QROW : 0)), *dec = g1 + RC_T;        // g^(i+1); g^(31-m), none from 32 on
-    int *brokenS = (int *)(dec + 2 * RC_T), *flawS = brokenS + 4 * RC_T;                     // per column: the group's first token whose value is not finite; whether this group, the one before, has one
+    float *g1 = (float *)(Qs + (OUT ? RM_TERMS * RC_T * QROW : 0)), *powers = g1 + RC_T;     // g^(i+1); g^(31-m), none from 32 on, and all that with a minus sign
+    int *brokenS = (int *)(powers + 4 * RC_T), *flawS = brokenS + 4 * RC_T;                     // per column: the group's first token whose value is not finite; whether this group, the one before, has one
     int *beyondS = flawS + 2;                                                                // RM_LOCAL: whether this group, the one before, has a key or value that no bfloat16 number comes near
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hi = lane >> 5, col = 32 * wave + l32;
     const bool busy = 32 * wave < Dv;
@@ -263,7 +267,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
         }
         if (lane < RC_T) g1[lane] = (float)p;
         const double q = __shfl(p, lane < 31 ? 30 - lane : 0, 64);
-        dec[lane] = lane < 31 ? (float)q : lane == 31 ? 1.0f : 0.f;
+        const float d = lane < 31 ? (float)q : lane == 31 ? 1.0f : 0.f;
+        powers[lane] = d;
+        powers[2 * RC_T + lane] = -d;
         if (lane < 4) flawS[lane] = 0;
     }
     const T *src = (const T *)a.proj + (int64_t)row0 * a.ld;
@@ -363,14 +369,19 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
         return OUT && !__builtin_isfinite(v) ? 0.f : v;
     };
     fetch(0);
+    uint32_t held = 0u;
     for (int t0 = 0; t0 < cnt; t0 += RC_T) {
         const int nt = cnt - t0 < RC_T ? cnt - t0 : RC_T;
+        // the signs that this group's queries have (+ - + -) and the state behind it is held with (+ - - +), a group whose products go with either in turn
+        const uint32_t asked = (uint32_t)(t0 / RC_T) << 31, next = (uint32_t)((t0 / RC_T + 1) >> 1) << 31;
+        const float *dec = powers + (held ? 2 * RC_T : 0);
+        uint32_t given = asked ^ held;                              // and its outputs
         __syncthreads();                                            // the group before has been read
         float big = 0.f;                                            // of keys and values, where no outputs tell (NaN passes: it reaches the same sums either way)
 #pragma unroll
         for (int it = 0; it < QIT; ++it) {
             const int tt = tid / SLOTS + it * (256 / SLOTS);
-            auto stage = [&](bf16_t *rows, jl_f32x8 v, bool key) {
+            auto stage = [&](bf16_t *rows, jl_f32x8 v, bool key, uint32_t sign) {
                 if (turns && tt < nt) {
                     const jl_f32x8 w = v;
 #pragma unroll
@@ -379,6 +390,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                 if (!OUT && key)
 #pragma unroll
                     for (int i = 0; i < 8; ++i) big = fmaxf(big, fabsf(v[i]));
+                if (!key)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = rm_signed(v[i], sign);
                 jl_bf16x8 part[RM_TERMS];
                 jl_split8(v, part);
 #pragma unroll
@@ -387,8 +401,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                     put(rows + (x * RC_T + tt) * QROW + 4 * ub, part[x], 1);
                 }
             };
-            stage(Ks, to_float(rk[it][0], rk[it][1]) * kscale, true);
-            if (OUT) stage(Qs, to_float(rq[it][0], rq[it][1]), false);
+            stage(Ks, to_float(rk[it][0], rk[it][1]) * kscale, true, 0u);
+            if (OUT) stage(Qs, to_float(rq[it][0], rq[it][1]), false, asked);
         }
         float zero = 0.f;                                           // not a number with a value that is not finite
 #pragma unroll
@@ -504,11 +518,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                         o = __builtin_amdgcn_mfma_f32_32x32x2f32(q, S[t][r], o, 0, 0, 0);
                     }
 #pragma unroll
-                for (int r = 0; r < 16; ++r) o[r] *= g1[8 * (r >> 2) + 4 * hi + (r & 3)];
+                for (int r = 0; r < 16; ++r) o[r] *= rm_signed(g1[8 * (r >> 2) + 4 * hi + (r & 3)], held);
+                given = 0u;
 #pragma unroll 1
                 for (int r = 0; r < 16; ++r) {
                     const int j = 8 * (r >> 2) + 4 * hi + (r & 3);
-                    o = __builtin_amdgcn_mfma_f32_32x32x2f32(j <= l32 ? p[r] * dec[31 - l32 + j] : 0.f, value(t0, nt, j), o, 0, 0, 0);
+                    o = __builtin_amdgcn_mfma_f32_32x32x2f32(j <= l32 ? p[r] * powers[31 - l32 + j] : 0.f, value(t0, nt, j), o, 0, 0, 0);
                 }
             }
             const int broken = flawed ? brokenS[32 * wave + l32] : RC_T;
@@ -520,13 +535,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
                 for (int r = 0; r < 16; ++r) {
                     asm volatile("" : "+v"(off));
                     const int i = 8 * (r >> 2) + 4 * hi + (r & 3);
-                    if (i < nt) *(float *)(to + off) = i < broken ? o[r] : NAN;
+                    if (i < nt) *(float *)(to + off) = i < broken ? rm_signed(o[r], given) : NAN;
                     off += (r & 3) == 3 ? 5 * o_row : o_row;
                 }
             }
         }
         if (!OUT || last || t0 + RC_T < cnt) {                      // the state behind the group
-            const float gn = g1[nt - 1];
+            const float gn = rm_signed(g1[nt - 1], held ^ next);
+            held = next;
+            dec = powers + (held ? 2 * RC_T : 0);
 #pragma unroll
             for (int t = 0; t < NS; ++t)
 #pragma unroll
@@ -573,7 +590,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && DP > 64 ? 1 : 2) void retent
         }
     }
     char *dst = (char *)(OUT ? a.state + ((int64_t)slot * H + h) * D * Dv : sp);
-    if (col < Dv && (!OUT || last)) each_state([&](int d, uint32_t off, float v) { if (d < D) *(float *)(dst + off) = v; return v; });
+    if (col < Dv && (!OUT || last)) each_state([&](int d, uint32_t off, float v) { if (d < D) *(float *)(dst + off) = rm_signed(v, held); return v; });
 }
 
 // The state every piece of a request starts from, in place of the piece's own contribution: S = the slot's state (zero at position 0), then for every piece but
