@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 139
+#define JL_VERSION 140
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -106,7 +106,7 @@ typedef struct {
     const void *k_tail;           /* the last k_tail_cols columns of every key head, shared by the heads: row stride k_tail_ld         */
     int64_t k_tail_ld, q_ld;      /* q_ld: row stride of q                                                                            */
     int32_t k_tail_cols;
-    int32_t reserved;
+    int32_t longest;              /* jl_attn_talk, jl_attn_narrow, jl_attn_sweep: no tile has more queries than this (0: no more than TQ is known) */
 } jl_attn_args;
 #define JL_OUT_SAME 0
 #define JL_OUT_F32 2

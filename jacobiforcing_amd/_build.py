@@ -21,7 +21,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibilit
 # The layer kernels come in two libraries, so that a model compiles (at the first call of a fresh checkout) only what it launches:
 # "layers" = norms, convolution, attention and its input / output stages; "layers_seq" = the recurrent mixers and the routed experts.
 LAYER_GROUPS = {
-    "layers": ["jl_error", "jl_norm", "jl_conv", "jl_headnorm", "jl_latent", "jl_attn_sweep", "jl_attn_rows", "jl_attn_f32", "jl_attn_talk", "jl_attn_block", "jl_attn", "jl_linear"],
+    "layers": ["jl_error", "jl_norm", "jl_conv", "jl_headnorm", "jl_latent", "jl_attn_sweep", "jl_attn_rows", "jl_attn_f32", "jl_attn_talk", "jl_attn_token", "jl_attn_block", "jl_attn", "jl_linear"],
     "layers_seq": ["jl_error", "jl_retention", "jl_delta", "jl_scan", "jl_moe"],
 }
 LAYERS_HEADERS = [CSRC / "layers" / "jl_common.h", CSRC / "layers" / "jl_attn.h", CSRC / "layers" / "jl_small.h", CSRC / "layers" / "jl_split.h", ROOT / "include" / "jf_layers.h"]

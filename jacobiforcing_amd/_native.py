@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 139                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 140                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -248,7 +248,7 @@ class AttnArgs(C.Structure):
                 ("Dv", _i32), ("window", _i32), ("keep_first", _i32), ("TQ", _i32), ("dtype", _i32), ("scale", _f32),
                 ("splits", _i32), ("n_rows", _i32), ("scratch", _vp), ("q_pack", _vp), ("k_ld", _i64), ("v_ld", _i64), ("Gv", _i32),
                 ("out_dtype", _i32), ("sink", _vp), ("gate_heads", _i32), ("chunk", _i32), ("softcap", _f32), ("out_scale", _f32), ("out_ld", _i64),
-                ("key_base", _vp), ("k_tail", _vp), ("k_tail_ld", _i64), ("q_ld", _i64), ("k_tail_cols", _i32), ("reserved", _i32)]
+                ("key_base", _vp), ("k_tail", _vp), ("k_tail_ld", _i64), ("q_ld", _i64), ("k_tail_cols", _i32), ("longest", _i32)]
 
 
 class ScanArgs(C.Structure):

@@ -44,6 +44,10 @@ static inline bool jl_attn_grid_fits(const jl_attn_args &a, int hb) { return (in
 // the wide form's launch (jl_attn_rows.hip); sizes as jl_attn_sweep has checked them, ``hf`` heads of a.TQ queries per tile, ``hb`` tiles per group
 int jl_attn_rows_launch(const jl_attn_args &a, int hf, int hb, bool v_in_k, hipStream_t st);
 
+// Portions of a few tokens (jl_attn_token.hip), at most a.longest per tile: a.Gv, strides, checks and tiles as in the forms they are called from (jl_attn_talk, jl_attn_narrow, jl_attn_sweep)
+bool jl_attn_token_fits(const jl_attn_args &a, bool v_in_k);
+int jl_attn_token_launch(const jl_attn_args &a, bool v_in_k, hipStream_t st);
+
 // where keys and values come from: pages of pools, pages whose key rows hold the values in their first columns, or contiguous rows per request whose heads
 // share their last columns (keys and values built for this step)
 enum { AR_PAGED, AR_V_IN_K, AR_BUILT };

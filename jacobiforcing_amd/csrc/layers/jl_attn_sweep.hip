@@ -15,7 +15,7 @@
 // Few tiles with many keys (decoding): the key tiles of a row tile are shared out over blockIdx.z; every share leaves its
 // unnormalised outputs with its maximum and sum in a scratch, and attn_sweep_join_kernel combines them.
 // The next tile's rows travel in registers (16 bytes per lane, all at once) while this one is computed, its pool tokens were looked up a tile before.  What bounds it now: three
-// barriers per 32 keys at two or three workgroups per CU.  us before (rows fetched 8 bytes at a time between two barriers, each behind its page number) and after: 32 tokens at 2048 over
+// barriers per 32 keys at two or three workgroups per CU; what jl_attn_token.hip takes goes there.  us before (rows fetched 8 bytes at a time between two barriers, each behind its page number) and after: 32 tokens at 2048 over
 // latents of 512 + 64, 16 heads 83 -> 49; 4 x 200 tokens at 500 over them 246 -> 149; 777 + 300 tokens beside 30 single ones over 128 + 32, 8 heads 91 -> 69; 32 tokens at 2048, 16 heads
 // of 192 / 128 over 4 119 -> 61.
 // Accumulator r of lane l of a 32 x 32 MFMA is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32; lane l supplies row (A) or
@@ -365,6 +365,10 @@ extern "C" int jl_attn_sweep(const jl_attn_args *ap, void *stream) {
             return jl_attn_f32_launch(a, hf, hb, v_in_k ? AR_V_IN_K : AR_PAGED, true, st);
         }
         return jl_attn_rows_launch(a, hf, hb, v_in_k, st);
+    }
+    if (v_in_k && a.longest > 0 && a.TQ <= tq && (a.splits <= 1 || (a.scratch && a.splits <= 64)) && jl_attn_token_fits(a, true)) {      // also in tiles of fewer queries
+        a.splits = a.splits > 1 ? a.splits : 1;
+        return jl_attn_token_launch(a, true, (hipStream_t)stream);
     }
     if (a.TQ != tq) return jl_fail(JL_E_INVALID, "jl_attn_sweep: tiles of %d queries wanted (ask jl_attn_sweep_tile_rows)", tq);
     if (a.splits > 1 && (!a.scratch || a.splits > 64)) return jl_fail(JL_E_INVALID, "jl_attn_sweep: 2 .. 64 shares of the keys need a scratch");

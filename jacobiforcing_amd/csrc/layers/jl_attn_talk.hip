@@ -6,13 +6,13 @@
 // of mantissa; the mixed weights were rounded to 8 before), two products each.
 // Rows of the products are (query, head) pairs of one key head, as in jl_attn_rows.hip: a wavefront forms S^T = K Q^T for its 32 rows, a lane holds keys of ONE row, the
 // weights are the next product's operand as they are, and V^T is read by ds_read_b64_tr_b16.  A workgroup has 4 wavefronts (128 rows) over the same keys, or one
-// (32 rows: decoding, where keys are shared out over workgroups until the chip is full).  Keys go in tiles of 32 consecutive positions, the kept first ones before the window's; the next
+// (32 rows: portions of a few tokens, where keys are shared out over workgroups until the chip is full; single tokens of up to 16 heads go to jl_attn_token.hip).  Keys go in tiles of 32 consecutive positions, the kept first ones before the window's; the next
 // tile's rows and biases travel while this one is multiplied (one wavefront: other workgroups of the CU fill the wait).  A workgroup collects one value head: two at a time would form
 // the scores once instead of twice, but their 128 accumulators leave the tiles' rows no registers (8 heads over 2: 340 us instead of 200).
 // What bounds it: issue and latency at two wavefronts per SIMD; G (1 + 2) products of D or Dv per score, a third of the matrix rate at 4 x 2048 tokens.
 // Measured against two sweeps with every weight exchanged through LDS (us, norms and gates included, bfloat16, 8 heads over 2 of 128, window 1024, 4 kept):
 //   4 x 2048 tokens 797 -> 195 (173 and 22 for the mixture)    777 + 300 tokens beside 30 single ones 258 -> 79    200 tokens 73 -> 23
-//   32 single tokens at 2048: 137 -> 60 (40 and 20)            one at 700: 63 -> 29        16 heads over 4, 4 x 2048, window 2048: 3000 -> 730; 32 single tokens 402 -> 175
+//   16 heads over 4, 4 x 2048, window 2048: 3000 -> 730
 #include "jl_attn.h"
 
 constexpr int AT_KT = 32;
@@ -27,7 +27,7 @@ __device__ __forceinline__ float at_log2_bias(float b) {
 static __host__ __device__ inline int at_bias_row(int TQ, int HF) { return (TQ + AT_KT - 1 + 31) / 32 * 32 + (HF < 32 ? 32 / HF : 1); }   // heads of a query meet different banks
 static size_t at_lds_bytes(int KU, int VU, int TQ, int HF, int NW) { return (NW > 1 ? 2 : 1) * ((size_t)AT_KT * (KU + VU) * 16 + AT_KT * 4 + (size_t)HF * at_bias_row(TQ, HF) * 4); }
 
-template <int KU, int VU, int NW, bool MIX>                                            // D <= 8 * KU, Dv <= 8 * VU, wavefronts; MIX: products with all value heads
+template <int KU, int VU, int NW>                                                     // D <= 8 * KU, Dv <= 8 * VU, wavefronts
 __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, int HF, int tile0, int n_tiles) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int THREADS = 64 * NW, BUFS = NW > 1 ? 2 : 1, KT = AT_KT, NDV = VU / 4, BUF = KT * (KU + VU);
@@ -35,7 +35,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     const int H = a.H, G = a.G, D = a.D, Dv = a.Dv, TQ = a.TQ, S = a.splits;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
     // key heads (and the value heads' groups) side by side: neighbouring workgroups go to different XCDs, so each keeps few heads' keys in its L2
-    const int sides = MIX ? G * G : G, side = blockIdx.x % sides, rest = blockIdx.x / sides, split = rest % S, ti = rest / S, c = MIX ? side / G : side, g = MIX ? side - c * G : c % a.Gv;
+    const int sides = G * G, side = blockIdx.x % sides, rest = blockIdx.x / sides, split = rest % S, ti = rest / S, c = side / G, g = side - c * G;
     const int *tile = a.tiles + 4 * (int64_t)(tile0 + ti);
     const int b = tile[0], i0 = tile[1], cnt = tile[2], row0 = tile[3], h0 = c * HF;
     if (b < 0 || cnt <= 0) return;
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     const int BR = at_bias_row(TQ, HF);
     const int window = a.window > 0 ? a.window : 0x3fffffff;
     const int i_max = i0 + cnt - 1;
-    const int chunk = MIX ? 0 : a.chunk, keep_first = MIX ? a.keep_first : 0;
-    auto lowest = [&](int i) { return chunk > 0 ? i - i % chunk : i - window + 1; };        // first key that query i sees
+    const int keep_first = a.keep_first;
+    auto lowest = [&](int i) { return i - window + 1; };        // first key that query i sees
     const int lo = lowest(i0) > 0 ? lowest(i0) : 0;                 // of the first row's
     const int kept = keep_first < lo ? keep_first : lo;             // kept first tokens in front of them
     const int kept_tiles = (kept + KT - 1) / KT, n_kt = kept_tiles + (i_max + 1 - lo + KT - 1) / KT;
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
             const int e = tid + it * THREADS, jj = e / VU, u = e % VU;
             if (jj < nk && 8 * u < Dv) vreg[it] = load16(vc + (int64_t)tok[jj] * a.v_ld + 8 * u);
         }
-        if (MIX && NW > 1 && a.rel)
+        if (NW > 1 && a.rel)
 #pragma unroll
             for (int it = 0; it < AT_BIAS; ++it) {
                 const int e = tid + it * THREADS;
@@ -132,13 +132,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
             const int e = tid + it * THREADS, jj = e / VU, u = e % VU;
             if (jj < nk && 8 * u < Dv) Ks[KT * KU + jj * VU + ar_value_unit<VU>(jj, u)] = vreg[it];
         }
-        if (MIX && NW > 1 && a.rel)
+        if (NW > 1 && a.rel)
 #pragma unroll
             for (int it = 0; it < AT_BIAS; ++it) {
                 const int e = tid + it * THREADS;
                 if (e < n_bias) { const int y = e / HF; bias[(e - y * HF) * BR + y] = at_log2_bias(breg[it]); }
             }
-        if (MIX && NW == 1 && a.rel) {
+        if (NW == 1 && a.rel) {
             const int j0 = first_of(t);
 #pragma unroll 4
             for (int e = tid; e < n_bias; e += THREADS) { const int y = e / HF; bias[(e - y * HF) * BR + y] = at_log2_bias(bias_of(e, j0)); }
@@ -175,10 +175,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
 #pragma unroll
             for (int x = 0; x < KU / 2; ++x)
                 sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ar_bf16x8, Ks[l32 * KU + ar_key_unit<KU>(l32, 2 * x + hi)]), qf[x], sc, 0, 0, 0);
-            if (!MIX && a.softcap > 0.f) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sc[r] = soft_cap_fast(sc[r] * a.scale, a.softcap) * LOG2E;
-            } else if (MIX && a.rel) {
+            if (a.rel) {
                 const float *bias = biasS + sel * HF * BR + hl * BR + (ok ? ii : 0) + KT - 1 - 4 * hi;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sc[r] = fmaf(sc[r], c2, bias[-(8 * (r >> 2) + (r & 3))]);
@@ -231,7 +228,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
                     }
                     const ar_bf16x8 va = __builtin_bit_cast(ar_bf16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
                     acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, acc[y], 0, 0, 0);
-                    if (MIX) acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[y], 0, 0, 0);
+                    acc[y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, acc[y], 0, 0, 0);
                 }
             }
         }
@@ -243,36 +240,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_talk_kernel(jl_attn_args a, i
     }
     l_run += __shfl_xor(l_run, 32, 64);
     if (!ok) return;
-    if (!MIX && S == 1) {                                           // keys not shared out: what attn_narrow_join_kernel does with one share, without the way through the scratch
-        const int h = h0 + hl;
-        const float sink = a.sink ? a.sink[h] * LOG2E : -INFINITY, M = fmaxf(sink, m_run), w = m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - M) : 0.f;
-        const float L = (a.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f) + w * l_run, inv = L != 0.f ? a.out_scale / L : 0.f;
-        const int64_t n = row0 + ii;
-        const bf16_t *gate = (const bf16_t *)a.gate;
-#pragma unroll
-        for (int y = 0; y < NDV; ++y)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int col = 32 * y + 8 * q + 4 * hi;
-                if (col >= Dv) continue;
-                float v[4];
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    v[x] = (m_run > -INFINITY ? w * acc[y][4 * q + x] : 0.f) * inv;
-                    if (gate) v[x] *= 1.0f / (1.0f + __expf(-ld_f(gate + n * a.gate_ld + (a.gate_heads ? h : h * Dv + col + x))));
-                }
-                if (a.out_dtype == JL_OUT_F32) st4_f((float *)a.out + n * a.out_ld + h * Dv + col, v);
-                else st4_f((bf16_t *)a.out + n * a.out_ld + h * Dv + col, v);
-            }
-        return;
-    }
     // shares of the pass's rows: [tile, query][split][head][value head][Dv], and their maxima and sums [..][head][2] behind all of them
     const int64_t row = ((int64_t)ti * TQ + ii) * S + split;
-    const int GW = MIX ? G : 1;
-    float *ml = a.scratch + (int64_t)n_tiles * TQ * S * H * GW * Dv + (row * H + h0 + hl) * 2;
-    if ((!MIX || g == 0) && hi == 0) { ml[0] = m_run; ml[1] = l_run; }
+    float *ml = a.scratch + (int64_t)n_tiles * TQ * S * H * G * Dv + (row * H + h0 + hl) * 2;
+    if (g == 0 && hi == 0) { ml[0] = m_run; ml[1] = l_run; }
     if (!(l_run > 0.f) && m_run == -INFINITY) return;               // nothing seen: the share counts for nothing (or, all shares like it, the row is not a number)
-    float *o = a.scratch + ((row * H + h0 + hl) * GW + (MIX ? g : 0)) * Dv;
+    float *o = a.scratch + ((row * H + h0 + hl) * G + g) * Dv;
 #pragma unroll
     for (int y = 0; y < NDV; ++y)
 #pragma unroll
@@ -381,7 +354,7 @@ template <int KU, int VU, int NW> static int at_launch(const jl_attn_args &a, in
     const bool spread = a.splits > 1;
     const size_t lds = at_lds_bytes(KU, VU, a.TQ, HF, NW), mix = (size_t)((spread ? a.H * (a.G * a.Dv > 2 * a.splits ? a.G * a.Dv : 2 * a.splits) + a.splits * a.H : 4 * a.H) + a.H * a.H) * 4;
     if (NW > 1 && HF * (a.TQ + AT_KT - 1) > AT_BIAS * 64 * NW) return jl_fail(JL_E_INVALID, "jl_attn_talk: too many biases per tile");
-    auto kern = attn_talk_kernel<KU, VU, NW, true>;
+    auto kern = attn_talk_kernel<KU, VU, NW>;
     auto join = spread ? attn_talk_mix_kernel<true> : attn_talk_mix_kernel<false>;
     hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess && mix > 64 * 1024) e = hipFuncSetAttribute((const void *)join, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix);
@@ -410,6 +383,7 @@ extern "C" int jl_attn_talk(const jl_attn_args *ap, int32_t wide, int32_t pass_t
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_talk: unknown out_dtype");
     if ((uintptr_t)a.out & (a.out_dtype == JL_OUT_F32 ? 15 : 7)) return jl_fail(JL_E_INVALID, "jl_attn_talk: output rows start at the borders of four values");
     hipStream_t st = (hipStream_t)stream;
+    if (!wide && pass_tiles >= a.n_tiles && jl_attn_token_fits(a, false)) return jl_attn_token_launch(a, false, st);
     const int ku = a.D <= 64 ? 8 : 16, vu = a.Dv <= 64 ? 8 : 16;
 #define AT_CASE(K, V) if (ku == K && vu == V) return wide ? at_launch<K, V, 4>(a, pass_tiles, st) : at_launch<K, V, 1>(a, pass_tiles, st)
     AT_CASE(8, 8); AT_CASE(8, 16); AT_CASE(16, 8); AT_CASE(16, 16);
@@ -417,68 +391,14 @@ extern "C" int jl_attn_talk(const jl_attn_args *ap, int32_t wide, int32_t pass_t
     return jl_fail(JL_E_INVALID, "jl_attn_talk: unsupported size");
 }
 
-// ---- the same for single tokens without mixed heads: a wavefront's keys once, one product with the values -----------------------------------------
-// Decoding's attention is bound by the way to its keys: four wavefronts that meet at three barriers per 32 keys and fetch each tile's rows behind its page numbers (jl_attn_sweep.hip)
-// read keys and values at 1.3 TB/s; single wavefronts, eight to a CU, that keep their rows to themselves at 3.1.  us for both launches, sweep / this (20 and less are the host's): 32 tokens at 2048,
-// 16 heads of 128 over 4 100 / 43, 8 over 2 68 / 32; 200 tokens at 1000, 16 over 4 538 / 103; 48 at 500 40 / 25; 30 portions of 10 at 1000, 8 over 2 63 / 30; 512 tokens 50 / 31.  Few keys are not shared out (layer_ops.NARROW_WHOLE): their
-// rows leave finished, in one launch.
-// A (token, head) row's shares joined: w = 2 ** (m - M) / L with the sink as one more share that holds nothing, times the gate
-__global__ __launch_bounds__(256) void attn_narrow_join_kernel(jl_attn_args a, int64_t groups) {
-    const int64_t r = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-    if (r >= groups) return;
-    const int H = a.H, Dv = a.Dv, S = a.splits, lane = threadIdx.x & 31, h = (int)(r % H);
-    const int64_t rt = r / H;
-    const int ti = (int)(rt / a.TQ), ii = (int)(rt - (int64_t)ti * a.TQ);
-    const int *tile = a.tiles + 4 * (int64_t)ti;
-    if (tile[0] < 0 || ii >= tile[2]) return;
-    const int64_t n = tile[3] + ii;
-    const float *ml = a.scratch + (int64_t)a.n_tiles * a.TQ * S * H * Dv + (rt * S * H + h) * 2, *po = a.scratch + (rt * S * H + h) * Dv + 4 * lane;
-    constexpr float LOG2E = 1.44269504088896341f;
-    const float sink = a.sink ? a.sink[h] * LOG2E : -INFINITY;
-    float M = sink;
-    for (int s = 0; s < S; ++s) M = fmaxf(M, ml[s * H * 2]);
-    float L = a.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
-    const bool in = 4 * lane < Dv;
-#pragma unroll 4
-    for (int s = 0; s < S; ++s) {
-        const float m = ml[s * H * 2], l = ml[s * H * 2 + 1], w = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.f;
-        const float4 p = in ? *(const float4 *)(po + (int64_t)s * H * Dv) : make_float4(0.f, 0.f, 0.f, 0.f);
-        L += w * l;                                                 // an empty share (m = -inf) holds nothing and is not looked at
-        v[0] = m > -INFINITY ? fmaf(w, p.x, v[0]) : v[0];
-        v[1] = m > -INFINITY ? fmaf(w, p.y, v[1]) : v[1];
-        v[2] = m > -INFINITY ? fmaf(w, p.z, v[2]) : v[2];
-        v[3] = m > -INFINITY ? fmaf(w, p.w, v[3]) : v[3];
-    }
-    if (!in) return;
-    const float inv = L != 0.f ? a.out_scale / L : 0.f;             // a sum that is not a number reaches the outputs
-    const bf16_t *gate = (const bf16_t *)a.gate;
-    const int col = h * Dv + 4 * lane;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[i] *= inv;
-        if (gate) v[i] *= 1.0f / (1.0f + __expf(-ld_f(gate + n * a.gate_ld + (a.gate_heads ? h : col + i))));
-    }
-    if (a.out_dtype == JL_OUT_F32) st4_f((float *)a.out + n * a.out_ld + col, v);
-    else st4_f((bf16_t *)a.out + n * a.out_ld + col, v);
-}
-
+// ---- without mixed heads: tiles of up to 32 rows, each wavefront with keys of its own (jl_attn_token.hip) -----------------------------------------
 extern "C" int jl_attn_narrow_ok(int dtype, int32_t H, int32_t G, int32_t Gv, int32_t D, int32_t Dv, int64_t k_ld, int64_t v_ld) {
     return jl_attn_talk_ok(dtype, H, G, D, Dv, k_ld, v_ld) && Gv > 0 && G % Gv == 0;
 }
 
-template <int KU, int VU> static int an_launch(const jl_attn_args &a, hipStream_t st) {
-    const size_t lds = at_lds_bytes(KU, VU, a.TQ, a.H / a.G, 1);
-    auto kern = attn_talk_kernel<KU, VU, 1, false>;
-    kern<<<dim3((unsigned)(a.n_tiles * a.splits * a.G)), 64, lds, st>>>(a, a.H / a.G, 0, a.n_tiles);
-    if (a.splits == 1) return jl_check_launch("attn_talk_kernel (single tokens)");
-    const int64_t groups = (int64_t)a.n_tiles * a.TQ * a.H;
-    attn_narrow_join_kernel<<<dim3((unsigned)((groups + 7) / 8)), 256, 0, st>>>(a, groups);
-    return jl_check_launch("attn_talk_kernel (single tokens)");
-}
-
 extern "C" int jl_attn_narrow(const jl_attn_args *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null arguments");
-    const jl_attn_args &a = *ap;
+    jl_attn_args a = *ap;
     if (a.n_tiles <= 0) return JL_OK;
     if (!a.q || !a.k_cache || !a.v_cache || !a.out || !a.block_tables || !a.tiles || (a.splits > 1 && !a.scratch)) return jl_fail(JL_E_INVALID, "jl_attn_narrow: null pointer");
     if (!jl_attn_narrow_ok(a.dtype, a.H, a.G, a.Gv, a.D, a.Dv, a.k_ld, a.v_ld) || a.k_ld < (int64_t)a.G * a.D || a.v_ld < (int64_t)a.Gv * a.Dv ||
@@ -491,6 +411,6 @@ extern "C" int jl_attn_narrow(const jl_attn_args *ap, void *stream) {
     if (a.out_dtype != JL_OUT_SAME && a.out_dtype != JL_OUT_F32) return jl_fail(JL_E_INVALID, "jl_attn_narrow: unknown out_dtype");
     if ((uintptr_t)a.out & (a.out_dtype == JL_OUT_F32 ? 15 : 7)) return jl_fail(JL_E_INVALID, "jl_attn_narrow: output rows start at the borders of four values");
     hipStream_t st = (hipStream_t)stream;
-    if (a.D <= 64) return a.Dv <= 64 ? an_launch<8, 8>(a, st) : an_launch<8, 16>(a, st);
-    return a.Dv <= 64 ? an_launch<16, 8>(a, st) : an_launch<16, 16>(a, st);
+    if (a.longest <= 0 || a.longest > a.TQ) a.longest = a.TQ;
+    return jl_attn_token_launch(a, false, st);
 }

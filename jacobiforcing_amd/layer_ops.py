@@ -33,10 +33,11 @@ ATTN_MAX_HEADS_ONE_LAUNCH, ATTN_MAX_VALUE_WIDTH = 16, 128   # what the matrix-co
 # values per value head, and is taken for up to 8 of them: us, two sweeps / this, 4 x 2048 tokens, 32 single ones: 8 heads over 1 688 / 102, 122 / 29; 4 over 4 1011 / 179, 196 / 81; 16 over 4
 # 1891 / 585, 299 / 93; sizes that went to float multiply-adds before: 12 over 6 51800 / 689, 16 over 8 70400 / 1270
 TALK_WORKGROUPS, TALK_SCRATCH_FLOATS = 640, 256 << 20
-NARROW_WORKGROUPS = 2048              # attention of a few tokens per request, and of portions too few for the 128-row tiles (one of 1000 / 2040 tokens, 8 heads over 2 of 128: 66 -> 36, 193 -> 67 us;
-                                      # 1000 behind 4000 290 -> 81): single wavefronts to aim at when keys are shared out
-NARROW_WHOLE = 128                    # ... up to this many keys never: one launch and no scratch (us with the host, 8 heads of 128 over 2, shared out / whole: 1 token at 64 keys 23 / 18, 32 at 128
-                                      # 24 / 19, where the form before took 16 and 17; GPU time 13 / 12 and 15 / 18; at 192 keys the shares' 15 are the better ones)
+# attention of a few tokens per request (and of portions too few for the 128-row tiles): workgroups to aim at when keys are shared out, keys of a share at least, and keys up to which they never are: one
+# launch and no scratch.  A workgroup has eight wavefronts, so one per CU has every CU's loads on their way; more only add sums to join.  us, workgroups 256 / 512: 32 tokens at 2048, 16 heads of 128 over 4
+# 31 / 34, latent of 512 30 / 30, of 256 (48 at 1000) 17 / 23, 8 mixed heads over 2 18 / 18, 16 over 4 29 / 37; 200 tokens at 1000, 16 heads over 4 21 / 29.  Keys of a share 64 / 96 / 128 / 256: one token at 700, 8 heads over
+# 2 9.5 / 9.5 / 9.8 / 11.2, mixed 13.2 / 13.4 / 14.0 / 17.8; 32 tokens at 150 9.2 / 9.5 / 9.5 / 7.9
+NARROW_WORKGROUPS, TOKEN_KEYS, NARROW_WHOLE = 256, 96, 128
 BLOCK_WORKGROUPS = 512               # a draft block's attention without key groups: workgroups to aim at when keys are shared out
 SWEEP_SPLIT_BELOW_GROUPS, SWEEP_SPLIT_WORKGROUPS = 512, 2048   # one-sweep attention: its workgroups are small (4 wavefronts, <= 32 rows)
 SWEEP_WIDE_ROWS_PER_REQUEST = 16   # one-sweep attention: from this many tokens per request on average a step takes the 128-row tiles
@@ -558,6 +559,18 @@ def _attn_args(q, k_cache, v_cache, out, batch: RaggedBatch, tiles, gate, sink, 
                       **dict(zip(("page_size", "H", "G", "Gv", "D", "Dv", "window", "keep_first", "chunk", "TQ", "splits", "out_dtype", "gate_heads"), numbers)))
 
 
+def _few(batch: RaggedBatch, heads: int, rows: int, tq: int) -> int:
+    """The most queries of a tile of up to ``tq`` where that is at most ``rows`` (query, head) rows, ``heads`` to a query (0: more)."""
+    most = tq if batch._whole is None else min(batch._whole[0], tq)
+    return most if most * heads <= rows else 0
+
+
+def _token_splits(reach: int, units: int) -> int:
+    """Shares of the keys for ``units`` workgroups' worth of rows with up to ``reach`` keys each.  The joining launch has eight shares on their way at once, so more than that from 512 keys a share on
+    only (4 tokens at 2000, 16 heads over 1, 8 / 16 / 32 shares 12.4 / 14.8 / 22.7 us)."""
+    return max(1, min(-(-reach // TOKEN_KEYS), NARROW_WORKGROUPS // units, max(8, -(-reach // 512)), 64))
+
+
 def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: torch.Tensor, batch: RaggedBatch,
                 H: int, G: int, D: int, Dv: int, scale: float, window: int, keep_first: int, rel: Optional[torch.Tensor],
                 lut: Optional[torch.Tensor], talk: Optional[torch.Tensor], value_heads: int = 0, float_out: bool = False,
@@ -591,16 +604,21 @@ def attn_window(q: torch.Tensor, gate: Optional[torch.Tensor], k_cache: torch.Te
     out = _attn_out(out, n, H * Dv, torch.float32 if float_out else dt, q.device, "attn_window")
     if (talk is not None and sink is None and chunk <= 0 and softcap <= 0 and Gv == G and N.layers().jl_attn_talk_ok(_code(dt), H, G, D, Dv, k_ld, v_ld) and _fours(out) and
             not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and not os.environ.get("JL_ATTN_NO_MFMA")):
-        wide = n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B
+        few = _few(batch, H, 16, 32 * G // H) if G in (1, 2, 4) and batch._whole is not None and batch._whole[0] * H <= 16 else 0
+        wide = not few and n >= SWEEP_WIDE_ROWS_PER_REQUEST * batch.B
         tq = int(N.layers().jl_attn_talk_tile_rows(H, G, int(wide)))
         tiles = batch.tiles(tq, longest_first=wide)
         reach = batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + int(keep_first) + tq)
-        splits = max(1, min(-(-reach // 64), (TALK_WORKGROUPS if wide else 3 * TALK_WORKGROUPS) // (tiles.shape[0] * G * G), 64))
+        if few:
+            splits = _token_splits(reach, tiles.shape[0] * -(-G // 2))
+        else:
+            splits = max(1, min(-(-reach // 64), (TALK_WORKGROUPS if wide else 3 * TALK_WORKGROUPS) // (tiles.shape[0] * G * G), 64))
         per_tile = int(N.layers().jl_attn_talk_scratch_floats(1, tq, H, G, Dv, splits))
         pass_tiles = min(tiles.shape[0], max(1, TALK_SCRATCH_FLOATS // per_tile))
         scratch = torch.empty((per_tile * pass_tiles,), dtype=torch.float32, device=q.device)
         a = _attn_args(q, k_cache, v_cache, out, batch, tiles, gate, None, rel, lut, talk, scratch, None, scale, 0.0, out_scale, H, G, Gv, D, Dv, window, max(0, int(keep_first)), 0, tq, splits,
                        N.JL_OUT_F32 if float_out and dt != torch.float32 else N.JL_OUT_SAME, gate_per_head)
+        a.longest = few
         N.check_layers(N.layers().jl_attn_talk(C.byref(a), int(wide), pass_tiles, _stream(q.device)), "jl_attn_talk")
         return out
     tq = attn_tile_rows(dt, H, G, D, Dv, k_ld, v_ld)
@@ -726,25 +744,36 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
             # what starts last should be short (4 x 2048 tokens, 16 heads of 128 over 4 key heads: 175 -> 137 us).  The 32-row kernel keeps the
             # requests' order, in which neighbours share keys (over a latent of 512 the sorted order was 3 % slower)
             tq, tiles = wide, batch.tiles(wide, longest_first=True)
-    narrow = False
+    narrow, few = False, 0
     if tiles is None and q.dtype == torch.bfloat16 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 and \
             N.layers().jl_attn_narrow_ok(N.JL_BF16, H, G, Gv, D, Dv, k_cache.stride(0), v_cache.stride(0)):
-        # few tokens per request: single wavefronts, each with a share of a tile's keys
+        # few tokens per request: every wavefront with keys of its own
         narrow, tq = True, int(N.layers().jl_attn_talk_tile_rows(H, G, 0))
         tiles = batch.tiles(tq)
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
-        splits = max(1, min(-(-reach // 64), NARROW_WORKGROUPS // (tiles.shape[0] * G), 64)) if reach > NARROW_WHOLE else 1
+        few = _few(batch, H // G, 32, tq)
+        splits = _token_splits(reach, tiles.shape[0] * G) if reach > NARROW_WHOLE else 1
         if splits > 1:
             scratch = torch.empty((int(N.layers().jl_attn_talk_scratch_floats(tiles.shape[0], tq, H, 1, Dv, splits)),), dtype=torch.float32, device=q.device)
-    elif tiles is None and groups < below:
-        tiles = batch.tiles(tq)
+    elif tiles is None:
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
-        splits = max(1, min(-(-reach // 128), SWEEP_SPLIT_WORKGROUPS // groups, 64))
+        # the same over a latent: 32 rows up to 256 values, beyond 16, which read the keys twice as often (us, 4-wavefront tiles of 32 rows / so, latent of 512, 16 heads: 200 tokens at 1000 72 / 42, 1000 at none
+        # 148 / 114, 2 x 1000 at 1000 321 / 324, 4 x 2000 998 / 1048)
+        if v_cache.data_ptr() == k_cache.data_ptr() and q.dtype == torch.bfloat16 and H <= 32 and D <= (Dv + 127) // 128 * 128 + 64 and k_cache.stride(0) % 8 == 0 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr()) % 16:
+            few = _few(batch, H, 32, tq) if Dv <= 256 else _few(batch, H, 16, 16 // H) if H <= 16 and (groups < 2 * below or batch.N == batch.B) else 0
+        if few:
+            tq = tq if Dv <= 256 else 16 // H
+            tiles = batch.tiles(tq)
+            splits = _token_splits(reach, tiles.shape[0])
+        elif groups < below:
+            tiles = batch.tiles(tq)
+            splits = max(1, min(-(-reach // 128), SWEEP_SPLIT_WORKGROUPS // groups, 64))
         if splits > 1:
             scratch = torch.empty((int(N.layers().jl_attn_sweep_scratch_floats(tiles.shape[0], H, G, Dv, splits)),), dtype=torch.float32, device=q.device)
     tiles = batch.tiles(tq) if tiles is None else tiles
     a = _attn_args(q, k_cache, v_cache, out, batch, tiles, gate, sink, None, None, None, scratch, None, scale, softcap, out_scale, H, G, Gv, D, Dv, window, 0, chunk, tq, splits,
                    N.JL_OUT_F32 if float_out else N.JL_OUT_SAME, gate_per_head)
+    a.longest = few
     if narrow:
         N.check_layers(N.layers().jl_attn_narrow(C.byref(a), _stream(q.device)), "jl_attn_narrow")
         return out
@@ -1235,14 +1264,14 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
     return parts[0] if len(parts) == 1 else torch.cat(parts, 0)
 
 
-# What the two forms of latent attention run at (this card): attention over the latent on the 32-row and (narrow latents, many rows) the 128-row tiles,
+# What the two forms of latent attention run at (this card): attention over the latent on the 32-row tiles (wide; few: latents up to 256) and (narrow latents, many rows) the 128-row tiles,
 # attention over keys and values built per head, the product that builds them.  ``key`` is the time the built form takes per key of its longest tile when the
 # chip is not full (a tile walks its keys in order; the 32-row kernel shares few tiles' keys out).  A layer wholly on built keys has fewer launches (bmm, packing, bmm
 # and head order go: 95 -> 55 us of host time for small steps), a step that mixes the forms has more.  Not counted: the tables of the built form, 70 us of the host and 7 per request
 # once per step, whatever the number of layers (8 prompts of 158 tokens, us a step over the latent / built: four layers 1357 / 1182, one layer 1168 / 1261).
-LATENT_RATES = dict(narrow=330e12, wide=140e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
+LATENT_RATES = dict(narrow=330e12, few=240e12, wide=140e12, built=420e12, product=600e12, key64=25e-9, key32=50e-9, launches=-35e-6, both=80e-6)
 # in float: the matrix form of the one-sweep kernel (narrow) or float multiply-adds (wide) over the latent
-LATENT_RATES_FLOAT = dict(narrow=60e12, wide=1.5e12, built=60e12, product=90e12, key64=130e-9, key32=180e-9, launches=-35e-6, both=80e-6)
+LATENT_RATES_FLOAT = dict(narrow=60e12, few=1.5e12, wide=1.5e12, built=60e12, product=90e12, key64=130e-9, key32=180e-9, launches=-35e-6, both=80e-6)
 LATENT_BUILT_BYTES = 2 << 30          # keys and values built at a time
 LATENT_BUILT_FROM = 16                # new tokens: no sizes make it worth building keys for fewer
 
@@ -1256,7 +1285,7 @@ def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, 
     chosen = batch._tiles.get(key)
     if chosen is None:
         r = LATENT_RATES if dtype == torch.bfloat16 else LATENT_RATES_FLOAT
-        over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["wide"])
+        over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["few"] if R <= 256 else r["wide"])
         pair, one = 2.0 * H * (D + rd + Dv) / r["built"], 2.0 * H * R * (D + Dv) / r["product"]
         step = r["key64"] if D + rd <= 128 else r["key32"]
         w, won, attend, chain, keys, chosen = window if window > 0 else 1 << 40, 0.0, 0.0, 0.0, 0, []

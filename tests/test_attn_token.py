@@ -1,0 +1,92 @@
+"""Attention of a few tokens whose wavefronts have keys of their own (jl_attn_token.hip): latents, mixed heads and grouped heads at the edges of rows, tiles and shares, against the same in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(counts, starts, page):
+    from jacobiforcing_amd import layer_ops as LO
+    need = [-(-(c + s) // page) for c, s in zip(counts, starts)]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(1)).tolist()
+    pages = [[order.pop() for _ in range(x)] for x in need]
+    return LO.RaggedBatch.build(counts, starts, list(range(len(counts))), pages, page, "cuda"), pages, sum(need) * page
+
+
+def _exact(q, k, v, scale, see, sink=None, add=None):
+    """[c, H, D], [K, H, D], [K, H, Dv] in 64 bits -> weights [H, c, K] without the sink's, values [H, K, Dv]."""
+    sc = q.permute(1, 0, 2).contiguous() @ k.permute(1, 2, 0).contiguous() * scale
+    sc = (sc if add is None else sc + add).masked_fill(~see, float("-inf"))
+    if sink is not None:
+        sc = torch.cat([sc, sink.double().view(-1, 1, 1).expand(-1, sc.shape[1], 1)], -1)
+    return torch.softmax(sc, -1)[..., :k.shape[0]].contiguous(), v.permute(1, 0, 2).contiguous()
+
+
+@pytest.mark.parametrize("H,R,rd,counts,starts,page,window,sink", [
+    (16, 512, 64, [1] * 3, [0, 15, 2040], 64, 0, False), (16, 512, 8, [3, 1], [300, 16], 48, 100, True), (5, 384, 64, [2, 1, 3], [700, 127, 0], 16, 0, False), (12, 256, 64, [2, 2], [97, 1000], 64, 0, True),
+    (32, 256, 0, [1, 1], [128, 129], 64, 50, False), (8, 128, 32, [4, 9, 1], [31, 513, 1500], 64, 1024, False), (3, 160, 24, [5, 1], [260, 33], 10, 0, False), (16, 32, 8, [2], [33], 64, 17, True),
+    (8, 128, 64, [1] * 300, [3] * 300, 4, 0, False), (1, 64, 64, [1], [9000], 64, 0, False),
+])
+def test_latents(H, R, rd, counts, starts, page, window, sink):
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(H * R + rd)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch, pages, tokens = _step(counts, starts, page)
+    n, W = sum(counts), R + rd
+    pool, q, gate = rnd(tokens, W + 8).bfloat16()[:, :W], rnd(n, H * W).bfloat16(), rnd(n, H).bfloat16()
+    sinks = rnd(H) if sink else None
+    out, r0 = LO.attn_sweep(q, pool, pool[:, :R], batch, H, 1, W, R, W ** -0.5, window, sink=sinks, gate=gate, gate_per_head=True), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        if b < 3 or b == len(counts) - 1:
+            tok = torch.tensor([pages[b][j // page] * page + j % page for j in range(c + s)], device="cuda")
+            k = pool[tok].double()[:, None].expand(-1, H, -1)
+            i, j = torch.arange(s, s + c, device="cuda").view(-1, 1), torch.arange(c + s, device="cuda").view(1, -1)
+            p, v = _exact(q[r0:r0 + c].double().view(c, H, W), k, k[..., :R], W ** -0.5, (j <= i) & ((i - j < window) | (window == 0)), sinks)
+            want = (p @ v).permute(1, 0, 2) * torch.sigmoid(gate[r0:r0 + c].double()).unsqueeze(-1)
+            # weights and results are rounded to bfloat16, 2 ** -9 each
+            assert (out[r0:r0 + c].double().view(c, H, R) - want).norm() <= 2 * 2.0 ** -8 * want.norm(), b
+        r0 += c
+
+
+@pytest.mark.parametrize("H,G,D,Dv,counts,starts,page,window,keep,bias,wgs", [
+    (16, 4, 128, 128, [1] * 3, [0, 16, 2040], 64, 1024, 4, "lut", 256), (16, 1, 128, 128, [1] * 2, [31, 32], 48, 0, 0, "direct", 256), (8, 2, 128, 128, [2, 1], [1500, 77], 64, 100, 40, "lut", 256),
+    (8, 4, 64, 64, [1, 2], [640, 0], 16, 0, 0, None, 1), (2, 2, 72, 40, [8, 3], [129, 5], 64, 33, 17, "direct", 256), (1, 1, 8, 8, [16], [300], 10, 16, 3, "direct", 4), (12, 2, 96, 96, [1], [9000], 64, 0, 0, "lut", 256),
+])
+def test_mixed_heads(monkeypatch, H, G, D, Dv, counts, starts, page, window, keep, bias, wgs):
+    from jacobiforcing_amd import layer_ops as LO
+    monkeypatch.setattr(LO, "NARROW_WORKGROUPS", wgs)
+    g = torch.Generator(device="cuda").manual_seed(H * D + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch, pages, tokens = _step(counts, starts, page)
+    n, longest, rep = sum(counts), max(c + s for c, s in zip(counts, starts)), H // G
+    assert LO._few(batch, H, 16, 32 * G // H) == max(counts)
+    kp, vp, q, gate = rnd(tokens, G * D + 8).bfloat16()[:, :G * D], rnd(tokens, G * Dv).bfloat16(), rnd(n, H * D).bfloat16(), rnd(n, H * Dv).bfloat16()
+    talk, lut = torch.eye(H, device="cuda") + 0.4 * rnd(H, H), (torch.arange(longest, device="cuda").float().sqrt() * 2).int() if bias == "lut" else None
+    rel = rnd(int(lut.max()) + 1 if bias == "lut" else 40, H) if bias else None
+    out, r0 = LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, D ** -0.5, window, keep, rel, lut, talk, float_out=True), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // page] * page + j % page for j in range(c + s)], device="cuda")
+        k, v = kp[tok].double().view(-1, G, D).repeat_interleave(rep, 1), vp[tok].double().view(-1, G, Dv).repeat_interleave(rep, 1)
+        i, j = torch.arange(s, s + c, device="cuda").view(-1, 1), torch.arange(c + s, device="cuda").view(1, -1)
+        add = None
+        if rel is not None:
+            d = (i - j).clamp(min=0)
+            add = rel.double()[lut[d].long() if lut is not None else d.clamp(max=rel.shape[0] - 1)].permute(2, 0, 1)
+        p, v = _exact(q[r0:r0 + c].double().view(c, H, D), k, v, D ** -0.5, (j <= i) & ((i - j < window) | (j < keep) | (window == 0)), add=add)
+        want = (torch.einsum("yx,xij->yij", talk.double(), p).contiguous() @ v).permute(1, 0, 2) * torch.sigmoid(gate[r0:r0 + c].double().view(c, H, Dv))
+        # float scores, weights to 16 bits of mantissa (2 ** -17), weights and sums cancel by up to 8
+        assert (out[r0:r0 + c].double().view(c, H, Dv) - want).norm() <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24) * want.norm(), b
+        r0 += c
+
+
+def test_a_request_without_tokens_beside_others():
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    pages, H, G, D = [[0, 1, 2], [3], [4, 5]], 8, 2, 64
+    kp, vp, q, pool, ql = rnd(6 * 64, G * D), rnd(6 * 64, G * D), rnd(3, H * D), rnd(6 * 64, 160), rnd(3, H * 160)
+    step = LO.RaggedBatch.build([1, 0, 2], [150, 0, 70], [0, 1, 2], pages, 64, "cuda")
+    alone = LO.RaggedBatch.build([1, 2], [150, 70], [0, 1], [pages[0], pages[2]], 64, "cuda")
+    for run in (lambda b: LO.attn_sweep(q, kp, vp, b, H, G, D, D, 0.1, 0), lambda b: LO.attn_sweep(ql, pool, pool[:, :128], b, H, 1, 160, 128, 0.1, 0)):
+        a, b = run(step).double(), run(alone).double()
+        assert (a - b).norm() <= 2 * 2.0 ** -8 * b.norm()            # tiles of as many queries, other shares of the keys
