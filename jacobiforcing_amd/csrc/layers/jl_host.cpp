@@ -13,7 +13,9 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <algorithm>
 #include <string.h>
+#include <vector>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -600,6 +602,118 @@ CALL(attention_args, 30)
     Py_RETURN_NONE;
 END_CALL
 
+// ---- a step's tables (RaggedBatch), formed on the host: nothing here touches a device ----------------------------------------------------------------
+// a list or tuple of ints within 32 bits
+bool take_ints(PyObject *o, std::vector<int64_t> &to) {
+    if (!PyList_CheckExact(o) && !PyTuple_CheckExact(o)) return false;
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
+    to.resize(n);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        int32_t v;
+        if (!take(PySequence_Fast_GET_ITEM(o, i), v)) return false;
+        to[i] = v;
+    }
+    return true;
+}
+int64_t fours(int64_t n) { return (n + 3) / 4 * 4; }
+
+// counts, starts, slots, block tables, page size, SCAN_PIECES_FROM -> (the upload as int64, N, columns of the tables, the places of seq, tables, row_req, pos and of a tile per request in it as 32-bit
+// words, words of the pieces behind that, largest position, page and slot, longest and shortest portion).  Steps that RaggedBatch.build refuses, and numbers beyond 32 bits, are its own.
+CALL(step_tables, 6)
+    std::vector<int64_t> counts, starts, slots, held;
+    int32_t page, from;
+    NEED(take_ints(arg[0], counts) && take_ints(arg[1], starts) && take_ints(arg[2], slots) && (PyList_CheckExact(arg[3]) || PyTuple_CheckExact(arg[3])) && take(arg[4], page) && page > 0 &&
+         take(arg[5], from));
+    const int64_t B = (int64_t)counts.size(), listed = PySequence_Fast_GET_SIZE(arg[3]);
+    NEED(B > 0 && (int64_t)starts.size() == B && (int64_t)slots.size() == B && listed >= B);
+    int64_t C = 1, N = 0, longest = 0, least = INT64_MAX, max_pos = 0, max_slot = slots[0], in_tables = 0;
+    held.resize(listed);
+    for (int64_t b = 0; b < listed; ++b) {
+        PyObject *t = PySequence_Fast_GET_ITEM(arg[3], b);
+        NEED(PyList_CheckExact(t) || PyTuple_CheckExact(t));
+        held[b] = PySequence_Fast_GET_SIZE(t);
+        if (held[b] > C) C = held[b];
+        if (b >= B) continue;                                       // tables of more requests count in the width alone
+        NEED(counts[b] >= 0 && starts[b] >= 0 && (!counts[b] || (starts[b] + counts[b] + page - 1) / page <= held[b]));
+        N += counts[b];
+        in_tables += held[b];
+        longest = std::max(longest, counts[b]);
+        least = std::min(least, counts[b]);
+        max_pos = std::max(max_pos, starts[b] + counts[b]);
+        max_slot = std::max(max_slot, slots[b]);
+    }
+    const int64_t pieced = longest >= from && least > 0 ? 4 * B : 0, sizes[] = {4 * B, B * C, N, N, 4 * B, pieced, pieced};
+    int64_t at[8] = {2 * (N + N % 2)};
+    for (int i = 0; i < 7; ++i) at[i + 1] = at[i] + fours(sizes[i]);
+    NEED(at[7] < INT32_MAX);
+    const Tensor up = at::empty({at[7] / 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(false));
+    int64_t *pool = up.data_ptr<int64_t>();
+    int32_t *words = (int32_t *)pool, *seq = words + at[0], *tables = words + at[1], *req = words + at[2], *pos = words + at[3], *whole = words + at[4], max_page = INT32_MIN;
+    memset(words, 0, (size_t)at[7] * 4);
+    for (int64_t b = 0, row = 0; b < B; ++b) {
+        PyObject *t = PySequence_Fast_GET_ITEM(arg[3], b);
+        int32_t *pages = tables + b * C;
+        for (int64_t i = 0; i < held[b]; ++i) {
+            NEED(take(PySequence_Fast_GET_ITEM(t, i), pages[i]));
+            max_page = std::max(max_page, pages[i]);
+        }
+        for (int64_t i = held[b]; i < C; ++i) pages[i] = -1;
+        if (held[b] < C) max_page = std::max(max_page, -1);
+        const int32_t c = (int32_t)counts[b], s = (int32_t)starts[b], sl = (int32_t)slots[b], r = (int32_t)row;
+        const int32_t s4[] = {r, c, s, sl}, w4[] = {(int32_t)b, s, c, r};
+        memcpy(seq + 4 * b, s4, 16);
+        memcpy(whole + 4 * b, w4, 16);
+        if (pieced) {
+            const int32_t piece[] = {r, c, sl, 1}, record[] = {(int32_t)b, 1, s, sl};
+            memcpy(words + at[5] + 4 * b, piece, 16);
+            memcpy(words + at[6] + 4 * b, record, 16);
+        }
+        for (int64_t j = s, pg = s / page, in = s % page; j < (int64_t)s + c; ++j, ++row) {
+            req[row] = (int32_t)b;
+            pos[row] = (int32_t)j;
+            pool[row] = (int64_t)pages[pg] * page + in;
+            if (++in == page) { in = 0; ++pg; }
+        }
+    }
+    return Py_BuildValue("(NLLLLLLLLLLLLL)", wrap(up), (long long)N, (long long)C, (long long)at[0], (long long)at[1], (long long)at[2], (long long)at[3], (long long)at[4], (long long)pieced,
+                         (long long)max_pos, (long long)max_page, (long long)max_slot, (long long)longest, (long long)least);
+END_CALL
+
+// the upload, B, N, columns, the places of seq, tables, row_req and pos -> (32-bit words, seq [B, 4], kv_slot [N], tables [B, columns], row_req [N], pos [N])
+PyObject *step_views(PyObject *, PyObject *const *arg, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    int64_t B, N, C, at[4];
+    if (n_args != 8 || !THPVariable_Check(arg[0]) || !take(arg[1], B) || !take(arg[2], N) || !take(arg[3], C)) return not_taken();
+    for (int i = 0; i < 4; ++i) NEED(take(arg[4 + i], at[i]));
+    const Tensor &up = THPVariable_Unpack(arg[0]);
+    const Tensor words = up.view(at::kInt);
+    return Py_BuildValue("(NNNNNN)", wrap(words), wrap(words.as_strided({B, 4}, {4, 1}, at[0])), wrap(up.as_strided({N}, {1}, 0)), wrap(words.as_strided({B, C}, {C, 1}, at[1])),
+                         wrap(words.as_strided({N}, {1}, at[2])), wrap(words.as_strided({N}, {1}, at[3])));
+END_CALL
+
+// counts, starts, most queries of a tile, whether those with the most positions in front of them come first -> [tiles, 4] int32 {request, first position, count, first row}
+CALL(tile_records, 4)
+    std::vector<int64_t> counts, starts;
+    int32_t tq;
+    bool sorted;
+    NEED(take_ints(arg[0], counts) && take_ints(arg[1], starts) && counts.size() == starts.size() && take(arg[2], tq) && tq > 0 && take(arg[3], sorted));
+    int64_t tiles = 0;
+    for (int64_t c : counts) { NEED(c >= 0); tiles += (c + tq - 1) / tq; }
+    struct Record { int32_t b, first, count, row; };
+    std::vector<Record> records;
+    records.reserve(tiles);
+    int64_t row = 0;
+    for (size_t b = 0; b < counts.size(); ++b) {
+        for (int64_t o = 0; o < counts[b]; o += tq)
+            records.push_back({(int32_t)b, (int32_t)(starts[b] + o), (int32_t)std::min<int64_t>(tq, counts[b] - o), (int32_t)(row + o)});
+        row += counts[b];
+    }
+    if (sorted) std::stable_sort(records.begin(), records.end(), [](const Record &x, const Record &y) { return x.first > y.first; });
+    const Tensor out = at::empty({tiles, 4}, at::TensorOptions().dtype(at::kInt));
+    if (tiles) memcpy(out.data_ptr(), records.data(), (size_t)tiles * 16);
+    return wrap(out);
+END_CALL
+
 // {symbol: address}, LINEAR_SMALL_ROWS, LINEAR_ONE_TILE, LINEAR_X_BYTES
 PyObject *bind(PyObject *, PyObject *args) {
     PyObject *symbols;
@@ -643,7 +757,7 @@ PyObject *symbols(PyObject *, PyObject *) {
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {FAST(linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
-                         FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), {"bind", bind, METH_VARARGS, nullptr},
+                         FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), FAST(step_tables), FAST(step_views), FAST(tile_records), {"bind", bind, METH_VARARGS, nullptr},
                          {"linear_rule", linear_rule, METH_VARARGS, nullptr}, {"symbols", symbols, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_jl_host", nullptr, -1, methods};
 

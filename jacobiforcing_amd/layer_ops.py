@@ -117,14 +117,14 @@ class _Gone:
             self.waiting.append((event, left))
 
 
-def _upload(host: np.ndarray, device, held: list) -> torch.Tensor:
+def _upload(host, device, held: list) -> torch.Tensor:
     """``host`` on ``device``, there for every stream when this returns.  A copy from ordinary host memory waits for its stream: on one of its own it waits for itself and not for the kernels
     queued so far.  That shows where passes queue behind one another (us a pass, tables on the kernels' stream / on this one: 32 decoding requests of Mikipel 860 / 796, 4 prompts of 2048 of Lokizen
     2402 / 2301).
     The tensor joins ``held``, the batch's list.  Its memory goes back to the copies' stream once the stream that asked for it is done with what lies in front of its first upload behind the batch's
     end: what a caller makes that stream wait for until then (kernels of another stream that read the tables) comes first, as it did when the memory was that stream's own."""
     device = torch.device(device)
-    t = torch.from_numpy(host)
+    t = torch.from_numpy(host) if isinstance(host, np.ndarray) else host
     if device.type != "cuda":
         return t.to(device)
     if torch.cuda.is_current_stream_capturing():
@@ -186,6 +186,16 @@ class RaggedBatch:
     @classmethod
     def build(cls, counts: Sequence[int], starts: Sequence[int], slots: Sequence[int], block_tables: Sequence[Sequence[int]],
               page_size: int, device) -> "RaggedBatch":
+        if _H is not None or torch.device(device).type == "cuda":
+            r = (_H or _host()).step_tables(counts, starts, slots, block_tables, page_size, SCAN_PIECES_FROM)
+            if r is not NotImplemented:                  # (us, 32 decoding requests of 33 pages each / one: so 10 / 5, below 40 / 13)
+                host, N_, C_, a_seq, a_bt, a_req, a_pos, a_whole, pieced, max_pos, max_page, max_slot, longest, least = r
+                B, held_by = len(counts), []
+                up = _upload(host, device, held_by)
+                words, seq, kv_slot, tables, row_req, pos = _H.step_views(up, B, N_, C_, a_seq, a_bt, a_req, a_pos)
+                return cls(B=B, N=N_, counts=list(counts), starts=list(starts), seq=seq, kv_slot=kv_slot, tables=tables, row_req=row_req, pos=pos, page_size=page_size, max_pos=max_pos, max_page=max_page,
+                           max_slot=max_slot, slots=list(slots), _tiles={}, _host_tables=host.numpy().view(np.int32)[a_bt:a_bt + B * C_].reshape(B, C_),
+                           _whole=(longest, words, a_whole, pieced) if least > 0 else None, _held=held_by)
         B = len(counts)
         if len(starts) != B or len(slots) != B:
             raise ValueError(f"{B} requests, {len(starts)} starts, {len(slots)} slots")
@@ -343,6 +353,10 @@ class RaggedBatch:
         t = self._tiles.get(key)
         if t is None and key == tq and self._whole is not None and self._whole[0] <= tq:
             t = self._tiles[key] = self._whole[1].as_strided((self.B, 4), (4, 1), self._whole[2])      # came with the batch's own upload
+        if t is None and _H is not None and requests is None:
+            rows = _H.tile_records(self.counts, self.starts, tq, longest_first)
+            if rows is not NotImplemented:
+                t = self._tiles[key] = _upload(rows, self.seq.device, self._held)
         if t is None:
             rows, r0 = [], 0
             for b, (c, s) in enumerate(zip(self.counts, self.starts)):
