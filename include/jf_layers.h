@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 140
+#define JL_VERSION 141
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -209,10 +209,11 @@ JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_re
 #define JL_LINEAR_SAME 0
 #define JL_LINEAR_FLOAT 1
 #define JL_LINEAR_ROUNDED_FLOAT 2
+#define JL_LINEAR_ADD 3                /* jl_linear_mid: out, of x's dtype, plus the product, rounded once */
 JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                            int32_t out_mode, void *stream);
-/* The same for more rows (a few hundred), all bfloat16, the result at a 16-byte border, operands of up to 4 GB. */
-JL_API int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O);       /* whether the launch is the better one for these sizes, whatever their type */
+/* The same for more rows (some hundred to a few thousand), all bfloat16, the result at a 16-byte border, operands of up to 4 GB. */
+JL_API int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O);       /* 1: the launch is the better one for these sizes, whatever their type; 2: so much so that products under autocast take it too */
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                          void *stream);
 

@@ -157,6 +157,11 @@ bool rule_small(int64_t n, int64_t k, int64_t o, int64_t item) {
 }
 
 // x, w, bias, float_out
+// where the launch is taken under autocast as well (2), or where that has nothing to see
+bool mid_taken(int64_t n, int64_t k, int64_t o) {
+    const int ok = p_jl_linear_mid_ok(n, k, o);
+    return ok == 2 || (ok && !at::autocast::is_autocast_enabled(at::kCUDA));
+}
 CALL(linear, 4)
     const Tensor *x, *w, *bias;
     bool as_float = false;
@@ -167,7 +172,7 @@ CALL(linear, 4)
     const bool same = w->scalar_type() == x->scalar_type();
     NEED(same || (is_float(*w) && !typed && as_float));
     const bool small = rule_small(n, k, o, size), split = !small && same && is_float(*w) && p_jl_linear_split_ok(n, k, o) && !at::autocast::is_autocast_enabled(at::kCUDA),
-               mid = !small && !split && same && !is_float(*x) && p_jl_linear_mid_ok(n, k, o);
+               mid = !small && !split && same && !is_float(*x) && mid_taken(n, k, o);
     NEED(small || split || mid);
     NEED(w->size(1) == k && w->is_contiguous() && x->stride(1) == 1 && ld >= k && k > 0 && o > 0 && o <= INT32_MAX && k * size % 16 == 0 && ld * (int64_t)x->element_size() % 16 == 0 && starts16(*x) &&
          starts16(*w) && w->device() == x->device());
@@ -184,6 +189,23 @@ CALL(linear, 4)
     else RUN(jl_linear_mid, x->data_ptr(), code(*x), n, ld, w->data_ptr(), (int32_t)k, (int32_t)o, at_(bias), out.data_ptr(), o, mode, st);
     others.back();
     return wrap(out);
+END_CALL
+
+// out += x w^T (linear_add_)
+CALL(linear_add, 3)
+    const Tensor *out, *x, *w;
+    NEED(take(arg[0], out) && take(arg[1], x) && take(arg[2], w));
+    NEED(x->dim() == 2 && w->dim() == 2 && out->dim() == 2 && x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && out->scalar_type() == at::kBFloat16);
+    const int64_t n = x->size(0), k = x->size(1), o = w->size(0), ld = x->stride(0);
+    NEED(n > 0 && k > 0 && o > 0 && o <= INT32_MAX && k <= INT32_MAX && p_jl_linear_mid_ok(n, k, o) && !at::autocast::is_autocast_enabled(at::kCUDA));
+    NEED(w->size(1) == k && w->is_contiguous() && rows(*out, n, o) && out->is_contiguous() && x->stride(1) == 1 && ld >= k && k % 8 == 0 && ld % 8 == 0 && starts16(*x) && starts16(*w) && starts16(*out) &&
+         w->device() == x->device() && out->device() == x->device() && n * ld * 2 < (int64_t)1 << 32 && !out->is_alias_of(*x) && !out->is_alias_of(*w));
+    NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad() || out->requires_grad())));
+    NEED(!x->_fw_grad(0).defined() && !w->_fw_grad(0).defined() && !out->_fw_grad(0).defined());
+    Unlocked others;
+    RUN(jl_linear_mid, x->data_ptr(), JL_BF16, n, ld, w->data_ptr(), (int32_t)k, (int32_t)o, nullptr, out->data_ptr(), o, JL_LINEAR_ADD, stream_of(*x));
+    others.back();
+    Py_RETURN_TRUE;
 END_CALL
 
 // x, y, x0, w, eps, out_dtype
@@ -756,7 +778,7 @@ PyObject *symbols(PyObject *, PyObject *) {
 }
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
+PyMethodDef methods[] = {FAST(linear), FAST(linear_add), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
                          FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), FAST(step_tables), FAST(step_views), FAST(tile_records), {"bind", bind, METH_VARARGS, nullptr},
                          {"linear_rule", linear_rule, METH_VARARGS, nullptr}, {"symbols", symbols, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_jl_host", nullptr, -1, methods};

@@ -57,34 +57,42 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 #undef LS_LAUNCH
 }
 
-// ---- a few hundred rows: 64 of x by 64 of W per workgroup ---------------------------------------------------------------------------------------
-// Stages of 128 bytes of every row go from memory straight into a ring of three buffers in LDS (16 bytes per lane, every lane fetching the unit that the permutation puts into its
-// place), two stages ahead of the products; four wavefronts hold a 32 x 32 quarter each, W's rows are the A operand, so that a lane ends with four neighbouring columns of a row.
-// What bounds it: a workgroup's way through its stages, 0.27 us each however many workgroups there are, until two per CU are busy.  us of GPU time against the library's product
-// (bfloat16, W from memory): 1024 x 1024 by 256 rows 7.8 / 8.3, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 520 x 1000 by 1024 7.0 / 10.1, by 1600 10.0 / 12.0; 192 x 768 by 1600 5.4 / 5.9;
-// 1024 x 3072 by 256 8.3 / 9.0; 2048 x 2048 by 512 13.3 / 11.2; and 11 us less of host time.  Beyond the caller's line (layer_ops.linear_mid) it loses more: 4096 x 2048 by 256 20.4 / 14.4,
-// 1024 x 3072 by 1024 16.1 / 13.6, and on the float matrix instructions everywhere (1024 x 1024 by 512 22.5 / 12.7): float rows stay with the library.  Larger tiles and deeper rings gained nothing there (128 x 128 by 8192 rows 100 / 52), nor did a share of the depth per wavefront without barriers.
-typedef float ld_f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ ld_f32x16 ld_mma(uint4 a, uint4 b, ld_f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ls_bf16x8, a), __builtin_bit_cast(ls_bf16x8, b), c, 0, 0, 0);
-}
-constexpr int LD_RING = 3, LD_UNITS = 8, LD_TILE = 64;              // 16-byte units of a row per stage
-
-__global__ __launch_bounds__(256) void linear_mid_kernel(const bf16_t *__restrict__ x, int64_t x_ld, const bf16_t *__restrict__ w, const bf16_t *__restrict__ bias, void *__restrict__ out,
-                                                         int64_t out_ld, int N, int K, int O, int out_mode, int row_tiles) {
-    typedef bf16_t T;
-    constexpr int UNIT = 16 / sizeof(T), STAGE = LD_UNITS * UNIT, BUF = 2 * LD_TILE * LD_UNITS;
-    __shared__ uint4 ldS[LD_RING * BUF];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hi = lane >> 5, wm = wave >> 1, wn = wave & 1;
-    const int n0 = blockIdx.x % row_tiles * LD_TILE, o0 = blockIdx.x / row_tiles * LD_TILE;      // neighbouring workgroups share W's rows
-    auto at = [](int row, int u) { return row * LD_UNITS + (u ^ (row & 7)); };
-    const int lr = tid / LD_UNITS, lu = (tid % LD_UNITS) ^ (lr & 7);   // the unit whose place in LDS is this thread's (rows step by 32: the permutation is the same)
-    uint32_t xo[2], wo[2];
+// ---- some hundred to a few thousand rows: TM of x by TN of W per workgroup -------------------------------------------------------------------------
+// Stages of 128 bytes of every row go from memory straight into a ring of RING buffers in LDS (16 bytes per lane, every lane fetching the unit that the permutation puts into its place).  A wavefront
+// reads the next stage's operands into registers while it multiplies this one's, so that one barrier per stage says both that the next stage is there and that this one may be written over, and multiplies
+// 16 x 16 tiles, whose sums wait for one another half as long as those of 32 x 32.  W's rows are the A operand and dealt out so that a lane ends with 4 * NT neighbouring columns of a row: 16 bytes a
+// store and more.
+// What bounds it: with few workgroups a stage's way (0.25 us before, operands read behind the barrier into one 32 x 32 tile; half of it now), with many what a CU takes in from L2, so tiles are as large
+// as still give every CU one (linear_mid_tiles).  us of GPU time, operands from memory, library / 64 x 64 with 32 x 32 tiles before / this: 1024 x 1024 by 600 rows 9.2 / 8.1 / 7.0, by 1000 9.6 / 8.3 / 7.4,
+// by 2048 11.1 / 10.6 / 9.9; 2048 x 1024 by 200 10.1 / 12.1 / 10.4, 1000 x 4864 by 896 21.9 / 27.3 / 21.3, 1536 x 1536 by 1300 14.3 / 14.0 / 12.4, 1024 x 1536 by 2048 13.9 / 16.1 / 14.1, 2048 x 2048 by
+// 2048 22.6 / 32.4 / 23.5, 1024 x 4096 by 2048 22.2 / 33.2 / 23.2; and the call takes the host 5 us, the library's 21.
+typedef uint32_t ld_u32x4 __attribute__((ext_vector_type(4)));
+template <int TM, int TN, int WM, int WN, int RING>
+__global__ __launch_bounds__(64 * WM * WN, (WM * WN >= 8 ? 1 : 2) * WM * WN / 4) void linear_mid_kernel(const bf16_t *__restrict__ x, int64_t x_ld, const bf16_t *__restrict__ w, const bf16_t *__restrict__ bias,
+                                                                                                   void *__restrict__ out, int64_t out_ld, int N, int K, int O, int out_mode, int row_tiles, int tiles) {
+    constexpr int THREADS = 64 * WM * WN, U = 8, UNIT = 8, STAGE = 64, BUF = (TM + TN) * U, XT = TM / WM / 16, NT = TN / WN / 16, XL = TM * U / THREADS, WL = TN * U / THREADS, COLS = 4 * NT;
+    static_assert(NT == 2 || NT == 4, "a lane's columns in whole stores");
+    extern __shared__ __attribute__((aligned(16))) uint4 ldS[];
+    // workgroups with the same remainder by 8 share an XCD; it walks strips of 1024 rows, column by column
+    const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;
+    const int cols = tiles / row_tiles, high = 1024 / TM < row_tiles ? 1024 / TM : row_tiles, strip = tile / (high * cols), here = row_tiles - strip * high < high ? row_tiles - strip * high : high;
+    const int in_strip = tile - strip * high * cols, n0 = (strip * high + in_strip % here) * TM, o0 = in_strip / here * TN;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, quad = lane >> 4, wm = wave / WN, wn = wave % WN;
+    // unit u of a row of LDS lies at u ^ swap: the sixteen rows that are read at once meet different banks.  Row 16 b + i of a wavefront's rows of W there is row COLS * (i / 4) + 4 b + i % 4 of them
+    auto swap = [](int row) { return (row >> 1) & 7; };
+    auto w_row = [](int m) { const int p = m % (16 * NT); return m - p + (p % 16 / 4) * COLS + p / 16 * 4 + p % 4; };
+    const int lr = tid / U, lu = (tid % U) ^ swap(lr);              // rows step by 32 or 64: the permutation is the same
+    uint32_t xo[XL], wo[WL];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {                                   // rows that do not exist repeat the last one
-        const int n = n0 + lr + 32 * i, o = o0 + lr + 32 * i;
-        xo[i] = (uint32_t)((n < N ? n : N - 1) * x_ld + lu * UNIT) * sizeof(T);
-        wo[i] = (uint32_t)((o < O ? o : O - 1) * (int64_t)K + lu * UNIT) * sizeof(T);
+    for (int i = 0; i < XL; ++i) {                                  // rows that do not exist repeat the last one
+        const int m = lr + THREADS / U * i, n = n0 + m;
+        xo[i] = (uint32_t)((n < N ? n : N - 1) * x_ld + lu * UNIT) * 2;
+    }
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+        const int o = o0 + w_row(lr + THREADS / U * i);
+        wo[i] = (uint32_t)((o < O ? o : O - 1) * (int64_t)K + lu * UNIT) * 2;
     }
     const char *xb = (const char *)x, *wb = (const char *)w;
     const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(ldS + wave * 64));
@@ -92,75 +100,157 @@ __global__ __launch_bounds__(256) void linear_mid_kernel(const bf16_t *__restric
     auto issue = [&](int s, int sel) {                              // behind the last stage, stage 0 again (never used): the number of loads on their way stays the same
         const int64_t k = s < full ? (int64_t)s * 128 : 0;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) jl_load_lds(xb + k, xo[i], lds + (sel * BUF + i * 256) * 16);
+        for (int i = 0; i < XL; ++i) jl_load_lds(xb + k, xo[i], lds + (sel * BUF + i * THREADS) * 16);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) jl_load_lds(wb + k, wo[i], lds + (sel * BUF + (2 + i) * 256) * 16);
+        for (int i = 0; i < WL; ++i) jl_load_lds(wb + k, wo[i], lds + (sel * BUF + (XL + i) * THREADS) * 16);
     };
-    ld_f32x16 acc;
+    ls_f32x4 acc[XT][NT];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    auto products = [&](const uint4 *Xs) {
-        const uint4 *Ws = Xs + LD_TILE * LD_UNITS;
+    for (int a = 0; a < XT; ++a)
 #pragma unroll
-        for (int s = 0; s < LD_UNITS / 2; ++s) acc = ld_mma(Ws[at(32 * wn + l32, 2 * s + hi)], Xs[at(32 * wm + l32, 2 * s + hi)], acc);
+        for (int b = 0; b < NT; ++b) acc[a][b] = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
+    uint4 xf[2][2][XT], wf[2][2][NT];
+    const int xs = (wm * (TM / WM) + l16) * U, ws = (TM + wn * (TN / WN) + l16) * U, p = swap(l16);
+    auto read = [&](int sel, int to) {
+        const uint4 *B = ldS + sel * BUF;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int u = (4 * k + quad) ^ p;
+#pragma unroll
+            for (int b = 0; b < NT; ++b) wf[to][k][b] = B[ws + 16 * b * U + u];
+#pragma unroll
+            for (int a = 0; a < XT; ++a) xf[to][k][a] = B[xs + 16 * a * U + u];
+        }
+    };
+    auto products = [&](int from) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int a = 0; a < XT; ++a)
+#pragma unroll
+                for (int b = 0; b < NT; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ls_bf16x8, wf[from][k][b]), __builtin_bit_cast(ls_bf16x8, xf[from][k][a]), acc[a][b], 0, 0, 0);
     };
     if (full > 0) {
 #pragma unroll
-        for (int s = 0; s < LD_RING - 1; ++s) issue(s, s);
+        for (int s = 0; s < RING; ++s) issue(s, s);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * (XL + WL)) : "memory");
+        __syncthreads();
+        read(0, 0);
         int sel = 0;
-        for (int s = 0; s < full; ++s) {
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LD_RING - 2) * 4) : "memory");
-            __syncthreads();                                        // stage s is there for everybody, stage s - 1 has been read
-            issue(s + LD_RING - 1, sel == 0 ? LD_RING - 1 : sel - 1);
-            products(ldS + sel * BUF);
-            sel = sel == LD_RING - 1 ? 0 : sel + 1;
+        auto step = [&](int s, int from) {
+            const int next = sel == RING - 1 ? 0 : sel + 1;
+            // this stage's operands are in registers, the next stage has landed: everybody may write over this one
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((RING - 2) * (XL + WL)) : "memory");
+            __builtin_amdgcn_s_barrier();
+            issue(s + RING, sel);
+            read(next, from ^ 1);
+            __builtin_amdgcn_sched_barrier(0);                      // the reads leave before the products
+            products(from);
+            __builtin_amdgcn_sched_barrier(0);
+            sel = next;
+        };
+        int s = 0;
+        for (; s + 1 < full; s += 2) {
+            step(s, 0);
+            step(s + 1, 1);
         }
+        if (s < full) step(s, 0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
     if (full * STAGE < K) {                                         // depths beyond K are zero; a lane beyond K reads its row's first unit: a row may be shorter than a stage
+        const ld_u32x4 zero = {0, 0, 0, 0};
         const bool in = full * STAGE + lu * UNIT < K;
         const int64_t k = in ? (int64_t)full * 128 : -(int64_t)lu * 16;
-        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-        const u32x4 zero = {0, 0, 0, 0};
+        auto last = [&](const char *base, uint32_t off) {
+            const ld_u32x4 v = *(const ld_u32x4 *)(base + off + k);
+            return __builtin_bit_cast(uint4, in ? v : zero);
+        };
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const u32x4 v = *(const u32x4 *)(xb + xo[i] + k), u = *(const u32x4 *)(wb + wo[i] + k);
-            ldS[i * 256 + tid] = __builtin_bit_cast(uint4, in ? v : zero);
-            ldS[(2 + i) * 256 + tid] = __builtin_bit_cast(uint4, in ? u : zero);
-        }
+        for (int i = 0; i < XL; ++i) ldS[i * THREADS + tid] = last(xb, xo[i]);
+#pragma unroll
+        for (int i = 0; i < WL; ++i) ldS[(XL + i) * THREADS + tid] = last(wb, wo[i]);
         __syncthreads();
-        products(ldS);
+        read(0, 0);
+        products(0);
     }
-    const int n = n0 + 32 * wm + l32;
-    if (n >= N) return;
-    const bool whole = O % 4 == 0 && out_ld % 4 == 0;
+    const int o = o0 + wn * (TN / WN) + quad * COLS;                // this lane's COLS columns
+    const bool whole = O % 8 == 0 && out_ld % 8 == 0, float_out = out_mode == JL_LINEAR_FLOAT || out_mode == JL_LINEAR_ROUNDED_FLOAT;
+    float add[COLS];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int o = o0 + 32 * wn + 8 * g + 4 * hi;                // four neighbouring columns
-        if (o >= O) continue;
-        float v[4];
+    for (int e = 0; e < COLS; ++e) add[e] = bias && o + e < O ? ld_f(bias + o + e) : 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[4 * g + e] + (bias && o + e < O ? ld_f(bias + o + e) : 0.f);
-        if (out_mode == JL_LINEAR_ROUNDED_FLOAT)
+    for (int a = 0; a < XT; ++a) {
+        const int n = n0 + wm * (TM / WM) + 16 * a + l16;
+        if (n >= N) continue;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { T r; st_f(&r, v[e]); v[e] = ld_f(&r); }
-        if (out_mode == JL_LINEAR_SAME) {
-            T *p = (T *)out + n * out_ld + o;
-            if (whole) st4_f(p, v);
-            else for (int e = 0; e < 4 && o + e < O; ++e) st_f(p + e, v[e]);
-        } else {
-            float *p = (float *)out + n * out_ld + o;
-            if (whole) st4_f(p, v);
-            else for (int e = 0; e < 4 && o + e < O; ++e) p[e] = v[e];
+        for (int e0 = 0; e0 < COLS; e0 += 8) {
+            if (o + e0 >= O) continue;
+            float v[2][4];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e >> 2][e & 3] = acc[a][(e0 + e) >> 2][e & 3] + add[e0 + e];
+            if (float_out) {
+                float *p = (float *)out + n * out_ld + o + e0;
+                if (out_mode == JL_LINEAR_ROUNDED_FLOAT)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) { bf16_t r; st_f(&r, v[e >> 2][e & 3]); v[e >> 2][e & 3] = ld_f(&r); }
+                if (whole) { st4_f(p, v[0]); st4_f(p + 4, v[1]); }
+                else
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (o + e0 + e < O) p[e] = v[e >> 2][e & 3];
+                continue;
+            }
+            bf16_t *p = (bf16_t *)out + n * out_ld + o + e0;
+            if (whole) {
+                if (out_mode == JL_LINEAR_ADD) {
+                    const ld_u32x4 r = *(const ld_u32x4 *)p;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e >> 1][2 * (e & 1)] += __uint_as_float(r[e] << 16);
+                        v[e >> 1][2 * (e & 1) + 1] += __uint_as_float(r[e] & 0xffff0000u);
+                    }
+                }
+                typedef float f32x8 __attribute__((ext_vector_type(8)));
+                const f32x8 all = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
+                *(ls_bf16x8 *)p = __builtin_convertvector(all, ls_bf16x8);
+            } else
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (o + e0 + e < O) st_f(p + e, v[e >> 2][e & 3] + (out_mode == JL_LINEAR_ADD ? ld_f(p + e) : 0.f));
         }
     }
 }
 
-// Up to two tiles per CU at depths of up to 1024, one at up to 2048 (layer_ops.linear_mid has the figures).
+// The largest tiles of which there is still about one per CU, since a CU takes in (TM + TN) rows for TM x TN sums: 64 x 64 up to 256 of them, 64 x 128, 128 x 128, and two of those per CU.
+// us by 64 x 64 / 64 x 128 / 128 x 128 / two per CU: 1024 x 1024 by 1000 rows (256 of 64 x 64) 7.4 / 9.0 / 11.9 / 13.0, by 2048 (512) 10.6 / 9.9 / 12.9 / 13.5, 2048 x 2048 by 2048 (1024) 32 / 24.4 / 23.5 / 26.9, 1024 x 4096 by
+// 2048 (2048) 33 / 27.3 / 27.6 / 23.2.
+static int linear_mid_tiles(int64_t N, int64_t O) {
+    auto tiles = [&](int tm, int tn) { return ((N + tm - 1) / tm) * ((O + tn - 1) / tn); };
+    return tiles(64, 64) <= 256 ? 0 : tiles(64, 128) <= 256 ? 1 : tiles(128, 128) <= 256 ? 2 : 3;
+}
+
+// 1: where the launch is the better one; 2: there, and it was so for products that autocast does not see (layer_ops.linear_mid has the figures).
 extern "C" int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O) {
-    const int64_t tiles = ((N + LD_TILE - 1) / LD_TILE) * ((O + LD_TILE - 1) / LD_TILE);
-    return N > 0 && ((K <= 1024 && tiles <= 512) || (K <= 2048 && tiles <= 256));
+    if (N <= 0 || K <= 0 || O <= 0) return 0;
+    const int64_t tiles = ((N + 63) / 64) * ((O + 63) / 64);
+    if ((K <= 1024 && tiles <= 512) || (K <= 2048 && tiles <= 256)) return 2;
+    if (N > 2304 || ((N + 127) / 128) * ((O + 127) / 128) > 512) return 0;
+    return K <= 2048 || (K <= 4096 && N >= 300 && tiles <= 512);
+}
+template <int TM, int TN, int WM, int WN, int RING>
+static int linear_mid_launch(const bf16_t *x, int64_t N, int64_t x_ld, const bf16_t *w, int32_t K, int32_t O, const bf16_t *bias, void *out, int64_t out_ld, int32_t out_mode, hipStream_t st) {
+    const int64_t row_tiles = (N + TM - 1) / TM, tiles = row_tiles * ((O + TN - 1) / TN);
+    if (tiles > INT32_MAX / (64 * WM * WN)) return jl_fail(JL_E_INVALID, "jl_linear_mid: too many tiles");
+    constexpr int lds = (TM + TN) * 128 * RING;
+    auto kern = linear_mid_kernel<TM, TN, WM, WN, RING>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_linear_mid: cannot get %d bytes of LDS: %s", lds, hipGetErrorString(e));
+    }
+    kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 64 * WM * WN, lds, st>>>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (int)row_tiles, (int)tiles);
+    return jl_check_launch("linear_mid_kernel");
 }
 extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                              void *stream) {
@@ -169,13 +259,15 @@ extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, 
     if (dtype != JL_BF16 || K % 8 || x_ld % 8 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15))
         return jl_fail(JL_E_INVALID, "jl_linear_mid: bfloat16, rows of x and W and the result at 16-byte borders");
     if (N > INT32_MAX / 64 || N * x_ld * 2 > UINT32_MAX || (int64_t)O * K * 2 > UINT32_MAX) return jl_fail(JL_E_INVALID, "jl_linear_mid: operands of up to 4 GB");
-    if (out_mode < JL_LINEAR_SAME || out_mode > JL_LINEAR_ROUNDED_FLOAT) return jl_fail(JL_E_INVALID, "jl_linear_mid: unknown out_mode");
-    const int row_tiles = (int)((N + LD_TILE - 1) / LD_TILE);
-    const int64_t groups = (int64_t)row_tiles * ((O + LD_TILE - 1) / LD_TILE);
-    if (groups > INT32_MAX / 256) return jl_fail(JL_E_INVALID, "jl_linear_mid: too many tiles");
-    linear_mid_kernel<<<dim3((unsigned)groups), 256, 0, (hipStream_t)stream>>>((const bf16_t *)x, x_ld, (const bf16_t *)w, (const bf16_t *)bias, out, out_ld, (int)N, K, O, out_mode,
-                                                                              row_tiles);
-    return jl_check_launch("linear_mid_kernel");
+    if (out_mode < JL_LINEAR_SAME || out_mode > JL_LINEAR_ADD) return jl_fail(JL_E_INVALID, "jl_linear_mid: unknown out_mode");
+    const bf16_t *xp = (const bf16_t *)x, *wp = (const bf16_t *)w, *bp = (const bf16_t *)bias;
+    hipStream_t st = (hipStream_t)stream;
+    switch (linear_mid_tiles(N, O)) {
+    case 0: return linear_mid_launch<64, 64, 2, 2, 4>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
+    case 1: return linear_mid_launch<64, 128, 2, 4, 3>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
+    case 2: return linear_mid_launch<128, 128, 2, 4, 4>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
+    }
+    return linear_mid_launch<128, 128, 2, 2, 2>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
 }
 
 // ---- float products of many rows: TM of x by 128 of W per workgroup, on the bfloat16 matrix instructions in three terms per operand (jl_split.h) -----

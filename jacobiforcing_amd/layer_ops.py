@@ -383,12 +383,13 @@ def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
     return 0 < n <= LINEAR_SMALL_ROWS and n * k * itemsize * -(-o // (tile * 256)) <= LINEAR_X_BYTES
 
 
-def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> bool:
-    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for a few hundred rows: 16-bit rows of up to 2 KB and no more than two 64 x 64 tiles per CU, or of up to 4 KB
-    and one.  There its GPU time is the library's give or take 3 us (1024 x 1024 by 128 rows 7.6 / 5.4, by 1024 8.4 / 9.1, by 1600 10.7 / 10.4; 2048 x 2048 by 512 13.3 / 11.2), and the call
-    costs 11 us less of the host, which such steps wait for (two portions of 50 beside 16 decoding requests at widths of 2048, us without / with the second line: Mikipel 1180 / 1122,
-    Safisun 1050 / 936, Voborax 1400 / 1247)."""
-    return dtype == torch.bfloat16 and bool(N.layers().jl_linear_mid_ok(n, k, o))
+def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> int:
+    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for some hundred to a few thousand rows (2: under autocast as well): bfloat16 ones of up to 4 KB, up to two 128 x 128
+    tiles per CU.  There its GPU time is about the library's and the call costs 16 us less of the host, which steps of up to some thousand tokens wait for (a block of four layers of 896 wide by 256
+    tokens 557 -> 354 us).  us of GPU time, library / own: 300 rows of 1024 by 2560 9.5 / 7.8, 1152 of 896 by 2048 11.8 / 11.6, 1196 of 2048 by 1024 14.1 / 13.6, 2048 of 1024 by 2048 16.4 / 15.5,
+    of 4096 by 1024 22.5 / 22.8.  Beyond the line: rows of 8 KB, which the library shares out, 70 of 4096 by 2048 10.7 / 18.4, 1500 32.1 / 41.2; more rows, whose steps wait for the GPU, 3000 of 2048
+    by 2048 29.4 / 32.7, 1024 of 4096 28 / 40."""
+    return int(N.layers().jl_linear_mid_ok(n, k, o)) if dtype == torch.bfloat16 else 0
 
 
 def linear_split(n: int, k: int, o: int) -> bool:
@@ -409,7 +410,7 @@ def _plain(*tensors: Optional[torch.Tensor]) -> bool:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, float_out: Optional[bool] = None) -> torch.Tensor:
-    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``), a few hundred (``linear_mid``) and many float ones
+    """x [N, K] times w [O, K] transposed (+ bias [O]): the package's launches for few rows (decoding, ``linear_small``), some hundred to a few thousand (``linear_mid``) and many float ones
     (``linear_split``), the library's product for the others and for what a launch would pass by (``_plain``).  ``float_out`` None: x's dtype; True: the float sums, unrounded; False: float, rounded to x's dtype first.  w (and bias) may be float beside a 16-bit x, which then
     counts as float: give ``float_out`` True.  What the launches do not take (other types, devices that differ, gradients wanted) is the library's to compute or refuse."""
     _dev(x)
@@ -424,7 +425,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     _need(same or (wt == torch.float32 and float_out is True), "linear: w of x's dtype, or float with a float result")
     small = launch and n <= LINEAR_SMALL_ROWS and linear_small(n, k, o, w.element_size())
     split = launch and not small and wt == torch.float32 and linear_split(n, k, o) and not torch.is_autocast_enabled("cuda")
-    if launch and (small or split or (same and linear_mid(n, k, o, dt))) and _plain(x, w, bias):
+    mid = linear_mid(n, k, o, dt) if launch and same and not small else 0
+    if launch and (small or split or mid == 2 or (mid and not torch.is_autocast_enabled("cuda"))) and _plain(x, w, bias):
         size = w.element_size()
         if (w.shape[1] == k and w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and k * size % 16 == 0 and x.stride(0) * x.element_size() % 16 == 0 and
                 (x.data_ptr() | w.data_ptr()) % 16 == 0 and (bias is None or (bias.dtype == wt and bias.shape == (o,) and bias.is_contiguous())) and dt in _LINEAR_TYPES and k > 0 and
@@ -456,6 +458,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         return torch.mm(x, w.t())
     y = F.linear(x, w, bias)
     return y if float_out is None else y.float()
+
+
+def linear_add_(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``out`` [N, O] plus x [N, K] times w [O, K] transposed, in place, rounded once: the package's launch (``linear_mid``), or the library's product."""
+    if not (is_dynamo_compiling() or (_H or _host()).linear_add(out, x, w) is NotImplemented):
+        return out
+    return out.addmm_(x, w.t())
 
 
 def embed_scale(embed: torch.Tensor, ids: torch.Tensor, scale: float, want_copy: bool,

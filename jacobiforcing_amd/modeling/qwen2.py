@@ -266,6 +266,8 @@ class Qwen2Model:
     def _mlp_residual(self, L, x2d, h2d):
         """x += down(silu(gate(h)) * up(h)) with the gate in one HIP launch and the residual in the GEMM epilogue (in place:
         an out-of-place addmm first copies x into its result, one more launch per GEMM)."""
+        if x2d.is_cuda and x2d.dtype == torch.bfloat16:
+            return LO.linear_add_(x2d, ops.swiglu(LO.linear(h2d, L["wgu"])), L["wd"])
         return x2d.addmm_(ops.swiglu(F.linear(h2d, L["wgu"])), L["wd"].t())
 
     # -- forward over a static cache -------------------------------------------------------------
@@ -411,7 +413,7 @@ class Qwen2Model:
             flat = flat[logits_rows]
         if logit_index is not None:
             flat = flat.index_select(0, logit_index.clamp(min=0).long())
-        return F.linear(flat, self.w.lm_head)
+        return LO.linear(flat, self.w.lm_head) if flat.is_cuda and flat.dtype == torch.bfloat16 else F.linear(flat, self.w.lm_head)
 
     def _forward_native(self, input_ids, positions, cache, row_prompt, row_cand, row_len, kv_len_rows, candidates, S_cur, paged, paged_slots, block_tables, n_main, logits_rows,
                         logit_index) -> torch.Tensor:
@@ -430,10 +432,10 @@ class Qwen2Model:
             slot_main, slot_cand = LO.block_slots(pos32, T, prompts, cands, lens, cache.S_max, cache.T_max, bool(candidates))
         x = w.embed[input_ids].view(R * T, cfg.hidden_size)
         for li, L in enumerate(w.layers):
-            qkv = F.linear(self._norm(x, L["ln1"]), L["wqkv"], L["bqkv"])
+            qkv = LO.linear(self._norm(x, L["ln1"]), L["wqkv"], L["bqkv"])
             ck, cv = (cache.ck[li], cache.cv[li]) if candidates else (None, None)
             qh = ops.rope_kv_append(qkv, T, nq, nkv, hd, pos32, self.cos, self.sin, cache.k[li], cache.v[li], slot_main, ck, cv, slot_cand)
             o = LO.attn_block(qh, T, cache.k[li], cache.v[li], kv, lens, S_cur, prompts, tables, cands, ck, cv)
-            x.addmm_(o, L["wo"].t())
+            LO.linear_add_(x, o, L["wo"])
             x = self._mlp_residual(L, x, self._norm(x, L["ln2"]))
         return self._head(x, logits_rows, logit_index)
