@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 141
+#define JL_VERSION 142
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -483,6 +483,20 @@ JL_API int jl_moe_router_blocks(int64_t N);
 /* in how many slices of the depth the product is better formed (1: whole): `slices`, with slices * N * E floats of scratch in `parts` when it is more than one */
 JL_API int jl_moe_router_slices(int64_t N, int32_t E, int32_t K);
 JL_API int jl_moe_router_run(const jl_moe_router *a, void *stream);
+
+/* A decode's experts, from h to every choice's weighted output, without a grouping: the choices of `router` (its x, w, bias, correction, ids, weights, N, x_ld, x_dtype, K, E, experts, top, kind, scale and
+ * renorm_eps; the others are not read), then up (relu^2, or with `gated` not 0 the unit of jl_gated_act of kind `unit`) into `act` [N*top, ff] of dtype and down into `out` float [N*top, W], rows in the choices'
+ * order; rows of choices >= experts are not written.  h [N, W], w_up [experts, ff or 2*ff, W], w_down [experts, W, ff] of dtype, everything at 16-byte borders. */
+#define JL_MOE_FEW_TOKENS 96
+#define JL_MOE_FEW_ROWS 1024
+typedef struct {
+    jl_moe_router router;
+    const void *h; const void *w_up; const void *w_down; void *act; float *out;
+    int32_t dtype, W, ff, gated, unit;
+    float limit, alpha, shift;
+} jl_moe_few;
+JL_API int jl_moe_few_ok(int dtype, int64_t N, int32_t outputs, int32_t top, int32_t W, int32_t ff);      /* whether jl_moe_few_run takes these sizes */
+JL_API int jl_moe_few_run(const jl_moe_few *a, void *stream);
 
 /* Grouped product over the sorted rows, in the tiles of a jl_moe_group with this tile_rows: C[r, :] = X[in(r), :] . W[e(r)]^T with W [E, n_out, K].
  *   mode 0 (up):   in(r) = perm[r] / top;  out[r, :] = relu(C)^2, stored in `dtype` ([N*top, n_out], sorted order)

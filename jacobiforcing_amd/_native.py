@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 141                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 142                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -262,6 +262,11 @@ class MoeRouter(C.Structure):
     """jl_moe_router (include/jf_layers.h)."""
     _fields_ = [(k, _vp) for k in ("x", "w", "bias", "correction", "ids", "weights", "perm", "offsets", "tile_expert", "tile_row0", "counts")] + [("N", _i64), ("x_ld", _i64)] + \
                [(k, _i32) for k in ("x_dtype", "K", "E", "experts", "top", "kind", "tile_rows", "max_tiles")] + [("scale", _f32), ("renorm_eps", _f32), ("parts", _vp), ("slices", _i32)]
+
+
+class MoeFew(C.Structure):
+    """jl_moe_few (include/jf_layers.h)."""
+    _fields_ = [("router", MoeRouter)] + [(n, _vp) for n in ("h", "w_up", "w_down", "act", "out")] + [(n, _i32) for n in ("dtype", "W", "ff", "gated", "unit")] + [(n, C.c_float) for n in ("limit", "alpha", "shift")]
 
 
 class LatentHeads(C.Structure):
@@ -370,12 +375,14 @@ _LAYER_SIGNATURES = {
     "jl_moe_router_blocks": (C.c_int, [_i64]),
     "jl_moe_router_slices": (C.c_int, [_i64, _i32, _i32]),
     "jl_moe_router_run": (C.c_int, [C.POINTER(MoeRouter), _vp]),
+    "jl_moe_few_ok": (C.c_int, [C.c_int, _i64, _i32, _i32, _i32, _i32]),
+    "jl_moe_few_run": (C.c_int, [C.POINTER(MoeFew), _vp]),
     "jl_moe_gemm": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp]),
     "jl_moe_gemm_gated": (C.c_int, [_vp, _vp, C.c_int, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _vp, _vp]),
 }
 LAYER_SYMBOLS = tuple(_LAYER_SIGNATURES)
 # which library a symbol lives in (jacobiforcing_amd/_build.py: LAYER_GROUPS); both carry their own jl_version / jl_last_error
-_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_float_tiles", "jl_moe_router_blocks", "jl_moe_router_slices", "jl_moe_router_run", "jl_moe_gemm", "jl_moe_gemm_gated")
+_SEQ_SYMBOLS = ("jl_retention", "jl_retention_pieces_ok", "jl_retention_pieces_run", "jl_retention_join", "jl_delta_rule", "jl_delta_chunks_ok", "jl_delta_chunks_floats", "jl_delta_chunks_run", "jl_linear_scan", "jl_linear_scan_chunked_ok", "jl_moe_route", "jl_moe_group", "jl_moe_tile_rows", "jl_moe_tile_pairs", "jl_moe_float_tiles", "jl_moe_router_blocks", "jl_moe_router_slices", "jl_moe_router_run", "jl_moe_few_ok", "jl_moe_few_run", "jl_moe_gemm", "jl_moe_gemm_gated")
 
 
 class _LayerLibs:

@@ -27,7 +27,7 @@ namespace {
 #define JL_HOST_CALLS(X)                                                                                                                              \
     X(jl_linear_small) X(jl_linear_mid_ok) X(jl_linear_mid) X(jl_linear_split_ok) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
     X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) X(jl_latent_heads_run) \
-    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
+    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_moe_few_ok) X(jl_moe_few_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
 #define DECLARE(name) decltype(&name) p_##name;
 JL_HOST_CALLS(DECLARE)
 #undef DECLARE
@@ -574,6 +574,23 @@ CALL(moe_experts, 15)
         NEED(x->dim() == 2 && known(*x) && x->size(0) == n && x->stride(1) == 1 && x->device() == h->device() && w_router->dim() == 2 && is_float(*w_router) && w_router->is_contiguous() &&
              w_router->size(0) == Er && w_router->size(1) == x->size(1) && row_weights(bias, Er));
     } else NEED(is_float(*x) && x->is_contiguous() && rows(*x, n, Er) && !bias && slices == 1);
+    if (tm == 32 && p_jl_moe_few_ok(code(*h), n, (int32_t)Er, top, (int32_t)W, (int32_t)ff) && starts16(*h) && starts16(*w_up) && starts16(*w_down) &&
+        (!w_router || (starts16(*x) && starts16(*w_router) && x->size(1) > 0 && x->size(1) % 4 == 0 && x->stride(0) >= x->size(1) && x->stride(0) * x->element_size() % 16 == 0))) {
+        Unlocked others;
+        Tensor ids = make({n, top}, at::kInt, *h), weights = make({n, top}, at::kFloat, *h), act = make({rows_, ff}, h->scalar_type(), *h), y = make({n, top, W}, at::kFloat, *h);
+        jl_moe_few f = {};
+        jl_moe_router &a = f.router;
+        a.x = x->data_ptr(); a.w = (const float *)at_(w_router); a.bias = (const float *)at_(bias); a.correction = (const float *)at_(correction);
+        a.ids = (int32_t *)ids.data_ptr(); a.weights = (float *)weights.data_ptr();
+        a.N = n; a.x_ld = x->stride(0); a.x_dtype = code(*x); a.K = (int32_t)x->size(1); a.E = (int32_t)Er; a.experts = (int32_t)E; a.top = top; a.kind = kind;
+        a.scale = (float)scale; a.renorm_eps = (float)renorm_eps;
+        f.h = h->data_ptr(); f.w_up = w_up->data_ptr(); f.w_down = w_down->data_ptr(); f.act = act.data_ptr(); f.out = (float *)y.data_ptr();
+        f.dtype = code(*h); f.W = (int32_t)W; f.ff = (int32_t)ff; f.gated = gated; f.unit = unit; f.limit = (float)limit; f.alpha = (float)alpha; f.shift = (float)shift;
+        RUN(jl_moe_few_run, &f, stream_of(*h));
+        others.back();
+        if (!identity) return wrap(y);
+        return Py_BuildValue("(NNN)", wrap(y), wrap(ids), wrap(weights));
+    }
     const int64_t max_tiles = rows_ / tm + E, blocks = p_jl_moe_router_blocks(n), lists = rows_ + E + 2 + 2 * max_tiles + blocks * E;
     Unlocked others;
     Tensor ids = make({n, top}, at::kInt, *h), weights = make({n, top}, at::kFloat, *h), list = make({lists + (slices > 1 ? slices * n * Er : 0)}, at::kInt, *h);

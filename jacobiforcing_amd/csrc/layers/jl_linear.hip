@@ -236,7 +236,7 @@ extern "C" int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O) {
     if (N <= 0 || K <= 0 || O <= 0) return 0;
     const int64_t tiles = ((N + 63) / 64) * ((O + 63) / 64);
     if ((K <= 1024 && tiles <= 512) || (K <= 2048 && tiles <= 256)) return 2;
-    if (N > 2304 || ((N + 127) / 128) * ((O + 127) / 128) > 512) return 0;
+    if (N > 2304 || ((N + 127) / 128) * ((O + 127) / 128) > 512 || K * O > (int64_t)32 << 20) return 0;
     return K <= 2048 || (K <= 4096 && N >= 300 && tiles <= 512);
 }
 template <int TM, int TN, int WM, int WN, int RING>

@@ -444,6 +444,61 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(jl_moe_router a, int ro
     if (blockIdx.x == 0) moe_tile_list(a, starts, first_tile, tid, 1024);
 }
 
+// ---- the same choice for the few tokens of a decode, a workgroup each, which group nothing (moe_few_kernel finds an expert's rows among the choices) -------------------------------------
+// What bounds it is what a CU takes in (all of W: 64 KB in 5 us of launch and choice included, 256 KB in 9) and the exchanges of the choice; the outputs are dealt out to sixteen wavefronts, each of
+// which has 2048 (up to 32 outputs) or 1024 depths of its outputs' rows on the way at once.  us, one workgroup for 32 tokens / in four slices and another launch / so: 32 x 1024 bfloat16 by 16 13.5 / - / 4.9,
+// 32 x 2048 float by 32 - / 17 / 8.7.
+constexpr int RF_NW = 16;
+template <typename TX, int RF_E>                                    // outputs of each of the wavefronts, at most
+__global__ __launch_bounds__(64 * RF_NW) void moe_router_few_kernel(jl_moe_router a) {
+    __shared__ float z[MR_MAX_E];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int64_t n = blockIdx.x;
+    if (!a.w) {
+        if (tid < a.E) z[tid] = ((const float *)a.x)[n * a.E + tid];
+    } else {
+        const TX *x = (const TX *)a.x + n * a.x_ld;
+        float sum[RF_E] = {};
+        auto of = [&](int i) { const int e = wave + RF_NW * i; return a.w + (int64_t)(e < a.E ? e : a.E - 1) * a.K; };
+        const int outputs = (a.E - wave + RF_NW - 1) / RF_NW;       // of this wavefront; none and fewer are the same for all lanes
+        constexpr int AHEAD = RF_E > 2 ? 4 : 8;
+        for (int k0 = 0; k0 < a.K; k0 += 256 * AHEAD) {             // four values per lane, of AHEAD pieces of 256
+            float xv[AHEAD][4];
+            float4 wv[RF_E][AHEAD];
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) {
+                const int k = k0 + 256 * s + 4 * lane, at = k < a.K ? k : 0;
+                ld4_f(x + at, xv[s]);
+#pragma unroll
+                for (int i = 0; i < RF_E; ++i)
+                    if (i < outputs) wv[i][s] = *(const float4 *)(of(i) + at);
+            }
+#pragma unroll
+            for (int i = 0; i < RF_E; ++i)
+                if (i < outputs)
+#pragma unroll
+                    for (int s = 0; s < AHEAD; ++s) {
+                        const bool in = k0 + 256 * s + 4 * lane < a.K;      // a weight that is not finite counts where it is, not beyond the depth
+                        sum[i] = in ? fmaf(xv[s][3], wv[i][s].w, fmaf(xv[s][2], wv[i][s].z, fmaf(xv[s][1], wv[i][s].y, fmaf(xv[s][0], wv[i][s].x, sum[i])))) : sum[i];
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < RF_E; ++i)
+            if (i < outputs) {
+                const float s = wave_sum_f32(sum[i]);
+                const int e = wave + RF_NW * i;
+                if (lane == 0) z[e] = a.bias ? s + a.bias[e] : s;
+            }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    const float *const zr[1] = {z};
+    moe_route_rows<64, 1>(zr, a.correction, a.E, a.top, a.kind, a.scale, a.renorm_eps, lane, [&](int, int s, int e, float weight) {
+        a.ids[n * a.top + s] = e;
+        a.weights[n * a.top + s] = weight;
+    });
+}
+
 extern "C" int jl_moe_router_blocks(int64_t N) { return (int)(N <= 16 ? 1 : (N + 31) / 32 < 0x7fffffff ? (N + 31) / 32 : 0x7fffffff); }
 // The product in four slices of the depth, in front of the choice, where a workgroup would take in half a MB of x and W by itself.  us of product, choice and grouping, one / four slices: 32 x 2048 float
 // by 32 outputs 20.6 / 12.9 (two 15.9, eight 13.1), by 40 27.7 / 17.0, 128 by 32 23.1 / 15.1, 1 by 32 12.7 / 8.7, 48 x 2048 bfloat16 by 32 24.7 / 15.9, 1400 x 1024 float by 20 15.4 / 13.5; below the
@@ -588,6 +643,8 @@ struct MoeMM {
     void *out;
     int mode, K, n_out, top, E, col_blocks, max_tiles, parts;       // parts: of TM rows, that a tile of the list is walked in
     MoeAct act;
+    const int32_t *ids;                                             // moe_few_kernel without a grouping: the choices of all rows, which are then where they were
+    int rows;
 };
 typedef __bf16 mm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 mm_bf16x2 __attribute__((ext_vector_type(2)));
@@ -614,8 +671,8 @@ template <> struct mm_type<float> {
 // What a wavefront's products leave: XT x NT tiles of 32 rows (from row_of(x) of the tile's) by 32 columns (from col_of(t)); a lane has sixteen rows of column lane % 32.  A store instruction writes
 // 32 neighbouring columns of two rows (float), or of four rows once neighbouring lanes have exchanged a value (bfloat16): whole lines or their halves.  (Four neighbouring columns of one row
 // per lane, 32 rows per instruction: the experts of 8192 x 4 of 32 of 2048 x 1024 took 687 us instead of 647, 8192 x 4 of 16 of 1024 x 512 174 instead of 163.)
-template <typename T, int XT, int NT, bool GATED, bool DOWN, typename Down, typename Rows, typename Cols>
-__device__ __forceinline__ void moe_store(const MoeMM &a, const mm_f32x16 (&acc)[XT][NT], int r0, int nr, int n0, Down down, Rows row_of, Cols col_of, int lane) {
+template <typename T, int XT, int NT, bool GATED, bool DOWN, typename Down, typename Rows, typename Cols, typename To>
+__device__ __forceinline__ void moe_store(const MoeMM &a, const mm_f32x16 (&acc)[XT][NT], int nr, int n0, Down down, Rows row_of, Cols col_of, int lane, To to) {
     constexpr int OT = GATED ? NT / 2 : NT;
     const int n_out = a.n_out, l32 = lane & 31, hi = lane >> 5;
     const bool pairs = n_out % 2 == 0, odd = lane & 1;
@@ -648,11 +705,11 @@ __device__ __forceinline__ void moe_store(const MoeMM &a, const mm_f32x16 (&acc)
                 } else if (sizeof(T) == 2 && pairs) {
                     const float other = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(odd ? v[0] : v[1]), 0xB1, 0xF, 0xF, true));      // quad_perm [1, 0, 3, 2]
                     const mm_f32x2 both = {odd ? other : v[0], odd ? v[1] : other};
-                    if (in && m + odd < nr) *(uint32_t *)((bf16_t *)a.out + (int64_t)(r0 + m + odd) * n_out + n - odd) = __builtin_bit_cast(uint32_t, __builtin_convertvector(both, mm_bf16x2));
+                    if (in && m + odd < nr) *(uint32_t *)((bf16_t *)a.out + (int64_t)to(m + odd) * n_out + n - odd) = __builtin_bit_cast(uint32_t, __builtin_convertvector(both, mm_bf16x2));
                 } else {
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
-                        if (in && m + i < nr) st_f((T *)a.out + (int64_t)(r0 + m + i) * n_out + n, v[i]);
+                        if (in && m + i < nr) st_f((T *)a.out + (int64_t)to(m + i) * n_out + n, v[i]);
                 }
             }
         }
@@ -771,8 +828,8 @@ __global__ __launch_bounds__(64 * NW, 3) void moe_mm_kernel(MoeMM a) {
         __syncthreads();
         products(0);
     }
-    moe_store<T, XT, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int x, int k, int &p, float &w) { const int m = wm * (TM / WM) + 32 * x + k; p = rows_out[m]; w = rows_weight[m]; },
-                                [&](int x) { return wm * (TM / WM) + 32 * x; }, w_row, lane);
+    moe_store<T, XT, NT, GATED, !GATED>(a, acc, nr, n0, [&](int x, int k, int &p, float &w) { const int m = wm * (TM / WM) + 32 * x + k; p = rows_out[m]; w = rows_weight[m]; },
+                                [&](int x) { return wm * (TM / WM) + 32 * x; }, w_row, lane, [&](int m) { return r0 + m; });
 }
 
 // ---- the same product for few rows per expert (decoding): 32 rows by 64 weight rows, the depth shared by two or four wavefronts ----------------------
@@ -780,34 +837,20 @@ __global__ __launch_bounds__(64 * NW, 3) void moe_mm_kernel(MoeMM a) {
 // products, and the shares meet in the end.  Rows of x come eight at a time, as many as there are.  (Three workgroups of four per CU do not fit the registers: spills, 106 us for the first line.)
 // us of both products, gated, weights from memory, one wavefront with all of the depth / two / four: 32 rows x 4 of 32 of 2048 x 1024 92 / 79 / 80 (402 MB: 5.0 TB/s), 1 x 4 of the same 28 / 21 / 19, 32 x 4 of
 // 16 of 1024 x 512 (plain) 22 / 18 / 16, 100 x 3 of 24 of 1536 x 704 37 / 37 / 41, 400 x 4 of 16 (plain) 27 / 25 / 28; float, 16 x 4 of 16 of 1024 x 512 62 / 38 / 27, 150 x 4 66 / 65 / 46.
-template <typename T, int MF_NW, bool GATED, bool FAR>
+template <typename T, int MF_NW, bool GATED, bool FAR, bool LIST = false, int WR = 64>
 __global__ __launch_bounds__(64 * MF_NW, 2) void moe_few_kernel(MoeMM a) {
-    constexpr int TM = 32, WR = 64, TKU = 8, NT = 2, XPF = TM * TKU / 64, WPF = WR * TKU / 64, TN = GATED ? WR / 2 : WR, UNIT = mm_type<T>::UNIT, STAGE = TKU * UNIT, OWN = (TM + WR) * TKU;
+    constexpr int TM = 32, TKU = 8, NT = WR / 32, XPF = TM * TKU / 64, WPF = WR * TKU / 64, TN = GATED ? WR / 2 : WR, UNIT = mm_type<T>::UNIT, STAGE = TKU * UNIT, OWN = (TM + WR) * TKU;
     __shared__ uint4 smem[MF_NW * OWN];
     __shared__ int rows_out[TM];                                    // way down: the flat indices and weights of the tile's rows
     __shared__ float rows_weight[TM];
-    const int tile = blockIdx.x / a.col_blocks, e = a.tile_expert[tile];
-    if (e < 0) return;
-    const int r0 = a.tile_row0[tile], K = a.K, n_out = a.n_out, n0 = (int)(blockIdx.x - tile * a.col_blocks) * TN, left = a.offsets[e + 1] - r0, nr = left < TM ? left : TM;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
-    if (!GATED && a.mode == 1 && (int)threadIdx.x < nr) {
-        const int p = a.perm[r0 + threadIdx.x];
-        rows_out[threadIdx.x] = p;
-        rows_weight[threadIdx.x] = a.weights[p];
-    }
+    const int tile = blockIdx.x / a.col_blocks, e = LIST ? tile % a.E : a.tile_expert[tile];
+    if (!LIST && e < 0) return;
+    const int K = a.K, n_out = a.n_out, n0 = (int)(blockIdx.x - tile * a.col_blocks) * TN, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
     auto at = [](int row, int u) { return row * TKU + (u ^ ((row >> 1) & 7)); };
     // loaders: unit lane % 8 of rows lane / 8 + 8 x; a row that does not exist repeats another and is not stored.  Byte offsets from a base that is the same for all lanes
-    const int lr = lane / TKU, lu = lane % TKU;
+    const int lr = lane / TKU, lu = lane % TKU, full = K / STAGE, s0 = full * wave / MF_NW, s1 = full * (wave + 1) / MF_NW;      // whole stages; what is left of K is the last wavefront's
     uint32_t xo[XPF], wo[WPF];
-    const char *xfar[FAR ? XPF : 1];
-    const char *Xb = (const char *)((const T *)a.X + (a.mode != 1 ? 0 : (int64_t)r0 * K));
-#pragma unroll
-    for (int x = 0; x < XPF; ++x) {
-        const int m = lr + 8 * x, row = m < nr ? m : 0;
-        const int64_t at_x = (a.mode != 1 ? a.perm[r0 + row] / a.top : row) * (int64_t)K + lu * UNIT;
-        if constexpr (FAR) xfar[x] = Xb + at_x * sizeof(T);
-        xo[x] = (uint32_t)at_x * sizeof(T);
-    }
+    mm_u32x4 reg[2][XPF + WPF];
     const char *Wb = (const char *)((const T *)a.Wt + ((int64_t)e * (GATED ? 2 : 1) * n_out + n0) * K), *Wl = Wb + (int64_t)(GATED ? n_out : 0) * K * sizeof(T);
 #pragma unroll
     for (int x = 0; x < WPF; ++x) {
@@ -815,8 +858,49 @@ __global__ __launch_bounds__(64 * MF_NW, 2) void moe_few_kernel(MoeMM a) {
         wo[x] = (uint32_t)((n0 + c < n_out ? c : n_out - 1 - n0) * (int64_t)K + lu * UNIT) * sizeof(T);
     }
     auto w_base = [&](int x) { return GATED && x >= WPF / 2 ? Wl : Wb; };
-    const int full = K / STAGE, s0 = full * wave / MF_NW, s1 = full * (wave + 1) / MF_NW;      // whole stages; what is left of K is the last wavefront's
-    mm_u32x4 reg[2][XPF + WPF];
+    int r0 = 0, nr;
+    if constexpr (LIST) {
+        // the rows from 32 * (tile / E) on of this expert's, in order: every wavefront looks through the choices by itself, and all write the same
+        const int first = tile / a.E * TM;
+        int found = 0;
+        for (int i0 = 0; i0 < a.rows; i0 += 256) {
+            int id[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { const int r = i0 + 64 * i + lane; id[i] = a.ids[r < a.rows ? r : a.rows - 1]; }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = i0 + 64 * i + lane;
+                const uint64_t mine = __ballot(r < a.rows && id[i] == e);
+                const int m = found + __popcll(mine & ((1ull << lane) - 1)) - first;
+                if ((mine >> lane & 1) && m >= 0 && m < TM) rows_out[m] = r;
+                found += __popcll(mine);
+            }
+        }
+        nr = found - first < TM ? found - first : TM;
+        if (nr <= 0) return;                                        // the whole workgroup
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (!GATED && a.mode == 1 && (int)threadIdx.x < nr) rows_weight[threadIdx.x] = a.weights[rows_out[threadIdx.x]];
+    } else {
+        r0 = a.tile_row0[tile];
+        const int left = a.offsets[e + 1] - r0;
+        nr = left < TM ? left : TM;
+        if (!GATED && a.mode == 1 && (int)threadIdx.x < nr) {
+            const int p = a.perm[r0 + threadIdx.x];
+            rows_out[threadIdx.x] = p;
+            rows_weight[threadIdx.x] = a.weights[p];
+        }
+    }
+    const char *xfar[FAR ? XPF : 1];
+    const char *Xb = (const char *)((const T *)a.X + (a.mode != 1 || LIST ? 0 : (int64_t)r0 * K));
+#pragma unroll
+    for (int x = 0; x < XPF; ++x) {
+        const int m = lr + 8 * x, row = m < nr ? m : 0;
+        const int from = LIST ? rows_out[row] : a.mode != 1 ? a.perm[r0 + row] : row;
+        const int64_t at_x = (a.mode != 1 ? from / a.top : from) * (int64_t)K + lu * UNIT;
+        if constexpr (FAR) xfar[x] = Xb + at_x * sizeof(T);
+        xo[x] = (uint32_t)at_x * sizeof(T);
+    }
     auto fetch = [&](mm_u32x4 (&r)[XPF + WPF], int i) {             // behind the last stage, the first again (never used)
         const int64_t k = i < s1 ? (int64_t)i * STAGE * sizeof(T) : 0;
 #pragma unroll
@@ -899,8 +983,8 @@ __global__ __launch_bounds__(64 * MF_NW, 2) void moe_few_kernel(MoeMM a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[0][t][4 * g + i] += v[i];
             }
-    moe_store<T, 1, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int, int k, int &p, float &w) { p = rows_out[k]; w = rows_weight[k]; }, [](int) { return 0; },
-                                       [&](int t) { return 32 * t; }, lane);
+    moe_store<T, 1, NT, GATED, !GATED>(a, acc, nr, n0, [&](int, int k, int &p, float &w) { p = rows_out[k]; w = rows_weight[k]; }, [](int) { return 0; },
+                                       [&](int t) { return 32 * t; }, lane, [&](int m) { return LIST ? rows_out[m] : r0 + m; });
 }
 
 // ---- the same product in tiles of 256 rows by 256 weight rows (bfloat16, depths in whole stages of 64) ----------------------------------------
@@ -1024,7 +1108,7 @@ __global__ __launch_bounds__(512, 2) void moe_big_kernel(MoeMM a) {
         products(sel, acc, [](int) {});
         sel ^= 1;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // the next tile's first stage, before the results: what this wavefront loaded of it is there
-        moe_store<bf16_t, NX, NT, GATED, false>(a, acc, now.r0, now.nr, now.n0, [](int, int, int &, float &) {}, [&](int x) { return 64 * x + 32 * wm; }, w_row, lane);
+        moe_store<bf16_t, NX, NT, GATED, false>(a, acc, now.nr, now.n0, [](int, int, int &, float &) {}, [&](int x) { return 64 * x + 32 * wm; }, w_row, lane, [&](int m) { return now.r0 + m; });
         now = next;
         q += slots;
         return more;
@@ -1064,7 +1148,7 @@ __global__ __launch_bounds__(64 * NW, NW / 2) void moe_split_kernel(MoeMM a) {
     auto w_row = [&](int t) { return GATED ? (t < NT / 2 ? 0 : TN) + wn * (TN / WN) + 32 * (t % (NT / 2 > 0 ? NT / 2 : 1)) : wn * (WR / WN) + 32 * t; };
     mm_f32x16 acc[XT][NT];
     split_products<TM, WR, NW, WM, TKU>(acc, smem, K, x_at, w_at, x_row, w_row);
-    moe_store<float, XT, NT, GATED, !GATED>(a, acc, r0, nr, n0, [&](int x, int k, int &p, float &w) { const int m = x_row(x) + k; p = rows_out[m]; w = rows_weight[m]; }, x_row, w_row, lane);
+    moe_store<float, XT, NT, GATED, !GATED>(a, acc, nr, n0, [&](int x, int k, int &p, float &w) { const int m = x_row(x) + k; p = rows_out[m]; w = rows_weight[m]; }, x_row, w_row, lane, [&](int m) { return r0 + m; });
 }
 
 template <typename T, int TM, int NW, int WR, int TKU> static int moe_mm_launch(MoeMM &a, bool gated, hipStream_t st) {
@@ -1121,7 +1205,7 @@ static int moe_gemm_launch(const void *X, const void *Wt, int dtype, int32_t mod
     static const bool no_mfma = getenv("JL_MOE_NO_MFMA") != nullptr;      // A/B switch for measurements
     if (E <= 0 || (tile_rows != 32 && tile_rows != 64 && tile_rows != 128 && tile_rows != 256)) return jl_fail(JL_E_INVALID, "jl_moe_gemm: tiles of 32, 64, 128 or 256 rows");
     const int64_t dtype_bytes = dtype == JL_BF16 ? 2 : 4;
-    MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, 1, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}};
+    MoeMM a = {X, Wt, perm, offsets, tile_expert, tile_row0, weights, out, mode, K, n_out, top, E, 0, max_tiles, 1, act ? *act : MoeAct{0, 0.f, 0.f, 0.f}, nullptr, 0};
     if (!no_mfma && moe_mm_sizes(dtype, K) && ((uintptr_t)X % 16) == 0 && ((uintptr_t)Wt % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
         256 * (int64_t)K * dtype_bytes <= UINT32_MAX) {                     // a tile's rows, of X or of W
         if (dtype == JL_BF16) return moe_mm_rows<bf16_t>(a, tile_rows, act != nullptr, (hipStream_t)stream);
@@ -1156,4 +1240,45 @@ extern "C" int jl_moe_gemm_gated(const void *X, const void *Wt, int dtype, int32
         return jl_fail(JL_E_INVALID, "jl_moe_gemm_gated: bad sizes or kind");
     const MoeAct act = {kind, limit, alpha, shift};
     return moe_gemm_launch(X, Wt, dtype, JL_MOE_UP_PLAIN, K, ff, top, perm, offsets, tile_expert, tile_row0, max_tiles, E, tile_rows, nullptr, out, &act, stream);
+}
+
+// A decode's experts without a grouping: three launches, the choice with a workgroup per token and the products in tiles of 32 of an expert's rows, whose number is not known: every expert gets as many as
+// all tokens could fill.  A product that is not gated goes in 32 columns at a time, three workgroups to a CU (64 columns, two: 9.0 us instead of 7.4, of 32 x 4 rows of 16 of 1024 x 512).
+// us, experts with choice, weights from memory, grouped / so: 16 of 1024 x 512, 1 token x 4 20.9 / 15.4, 32 31.2 / 20.8, 64 35.1 / 21.9, 96 36.0 / 23.9; 32 of 2048 x 1024, gated, 1 33.1 / 31.6, 32
+// 102 / 94, 64 105 / 94, 96 105 / 103; 64 of 1024 x 512, gated, 96 72 / 67; float, 16 of 1024 x 512, 32 45 / 39.  Beyond the line the tiles that have no rows cost more than the grouping: 128 of 32 106 / 108,
+// of 64 73 / 73, 191 of 32 107 / 133.
+static bool moe_few_sizes(int dtype, int64_t N, int32_t Er, int32_t top, int64_t W, int64_t ff) {
+    return N > 0 && N <= JL_MOE_FEW_TOKENS && Er > 0 && Er <= MR_MAX_E && top > 0 && N * top <= JL_MOE_FEW_ROWS && moe_mm_sizes(dtype, W) && moe_mm_sizes(dtype, ff) && W > 0 && ff > 0 && W <= (1 << 20) &&
+           ff <= (1 << 20);
+}
+extern "C" int jl_moe_few_ok(int dtype, int64_t N, int32_t Er, int32_t top, int32_t W, int32_t ff) {
+    static const bool no_mfma = getenv("JL_MOE_NO_MFMA") != nullptr;      // A/B switch for measurements
+    return !no_mfma && moe_few_sizes(dtype, N, Er, top, W, ff);
+}
+extern "C" int jl_moe_few_run(const jl_moe_few *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_moe_few_run: null arguments");
+    const jl_moe_few &f = *ap;
+    const jl_moe_router &a = f.router;
+    if (!a.x || !a.ids || !a.weights || !f.h || !f.w_up || !f.w_down || !f.act || !f.out) return jl_fail(JL_E_INVALID, "jl_moe_few_run: null pointer");
+    if ((f.dtype != JL_BF16 && f.dtype != JL_F32) || !moe_few_sizes(f.dtype, a.N, a.E, a.top, f.W, f.ff) || a.experts <= 0 || a.experts > a.E || a.top > a.E || a.kind < JL_ROUTE_SIGMOID ||
+        a.kind > JL_ROUTE_TOP_SOFTMAX || (f.gated && (f.unit < JL_ACT_GELU_TANH || f.unit > JL_ACT_GELU_ERF)))
+        return jl_fail(JL_E_INVALID, "jl_moe_few_run: up to %d tokens, %d choices of theirs and %d router outputs, rows at 16-byte borders", JL_MOE_FEW_TOKENS, JL_MOE_FEW_ROWS, MR_MAX_E);
+    if (((uintptr_t)f.h | (uintptr_t)f.w_up | (uintptr_t)f.w_down | (uintptr_t)f.act | (uintptr_t)f.out) & 15) return jl_fail(JL_E_INVALID, "jl_moe_few_run: operands at 16-byte borders");
+    if (!a.w && (a.x_dtype != JL_F32 || a.bias)) return jl_fail(JL_E_INVALID, "jl_moe_few_run: logits are float and whole");
+    if (a.w && ((a.x_dtype != JL_BF16 && a.x_dtype != JL_F32) || a.K <= 0 || a.K % 4 || a.x_ld < a.K || a.x_ld % (a.x_dtype == JL_BF16 ? 8 : 4) || (((uintptr_t)a.x | (uintptr_t)a.w) & 15)))
+        return jl_fail(JL_E_INVALID, "jl_moe_few_run: rows of x and W at 16-byte borders");
+    hipStream_t st = (hipStream_t)stream;
+#define RF_CASE(outputs) JL_DISPATCH(a.x_dtype, moe_router_few_kernel<T, outputs><<<dim3((unsigned)a.N), 64 * RF_NW, 0, st>>>(a))
+    if (a.E <= RF_NW) RF_CASE(1); else if (a.E <= 2 * RF_NW) RF_CASE(2); else RF_CASE(4);
+#undef RF_CASE
+    const int chunks = (int)((a.N + 31) / 32), rows = (int)(a.N * a.top);
+    auto product = [&](const void *x, const void *w, const float *weights, void *out, int mode, int K, int n_out, bool gated) {
+        const MoeMM m = {x, w, nullptr, nullptr, nullptr, nullptr, weights, out, mode, K, n_out, a.top, a.experts, (n_out + 31) / 32, 0, 1, {f.unit, f.limit, f.alpha, f.shift}, a.ids, rows};
+        const dim3 grid((unsigned)(a.experts * chunks * m.col_blocks));
+        if (gated) JL_DISPATCH(f.dtype, moe_few_kernel<T, 4, true, false, true><<<grid, 256, 0, st>>>(m));
+        else JL_DISPATCH(f.dtype, moe_few_kernel<T, 4, false, false, true, 32><<<grid, 256, 0, st>>>(m));
+    };
+    product(f.h, f.w_up, nullptr, f.act, f.gated ? JL_MOE_UP_PLAIN : 0, f.W, f.ff, f.gated);
+    product(f.act, f.w_down, a.weights, f.out, 1, f.ff, f.W, false);
+    return jl_check_launch("moe_few_kernel");
 }

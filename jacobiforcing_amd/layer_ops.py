@@ -385,10 +385,10 @@ def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
 
 def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> int:
     """Whether ``linear`` takes n rows of k values times [o, k] to the launch for some hundred to a few thousand rows (2: under autocast as well): bfloat16 ones of up to 4 KB, up to two 128 x 128
-    tiles per CU.  There its GPU time is about the library's and the call costs 16 us less of the host, which steps of up to some thousand tokens wait for (a block of four layers of 896 wide by 256
+    tiles per CU, w of up to 64 MB.  There its GPU time is about the library's and the call costs 16 us less of the host, which steps of up to some thousand tokens wait for (a block of four layers of 896 wide by 256
     tokens 557 -> 354 us).  us of GPU time, library / own: 300 rows of 1024 by 2560 9.5 / 7.8, 1152 of 896 by 2048 11.8 / 11.6, 1196 of 2048 by 1024 14.1 / 13.6, 2048 of 1024 by 2048 16.4 / 15.5,
     of 4096 by 1024 22.5 / 22.8.  Beyond the line: rows of 8 KB, which the library shares out, 70 of 4096 by 2048 10.7 / 18.4, 1500 32.1 / 41.2; more rows, whose steps wait for the GPU, 3000 of 2048
-    by 2048 29.4 / 32.7, 1024 of 4096 28 / 40."""
+    by 2048 29.4 / 32.7, 1024 of 4096 28 / 40; w that takes longer to read than to multiply, 200 of 1024 by 32000 25.2 / 27.5, 256 of 2048 45.3 / 52.4."""
     return int(N.layers().jl_linear_mid_ok(n, k, o)) if dtype == torch.bfloat16 else 0
 
 
@@ -942,6 +942,17 @@ def moe_experts(h: torch.Tensor, router_logits: Optional[torch.Tensor], correcti
             return r
     ids = torch.empty((n, top), dtype=torch.int32, device=dev)
     wts = torch.empty((n, top), dtype=torch.float32, device=dev)
+    # a decode's launches, which group nothing (moe_few_kernel and moe_router_few_kernel have the figures)
+    if (in_one or from_logits) and tm == 32 and L.jl_moe_few_ok(_code(dt), n, Er, top, W, ff) and (h.data_ptr() | w_up.data_ptr() | w_down.data_ptr()) % 16 == 0 and not os.environ.get("JL_MOE_UNFUSED_ACT"):
+        x, rw, rb = router if in_one else (router_logits, None, None)
+        act, y = torch.empty((rows, ff), dtype=dt, device=dev), torch.empty((n, top, W), dtype=torch.float32, device=dev)
+        a = N.MoeRouter(x=x.data_ptr(), w=_ptr(rw), bias=_ptr(rb), correction=_ptr(correction), ids=ids.data_ptr(), weights=wts.data_ptr(), N=n, x_ld=x.stride(0), x_dtype=_code(x.dtype),
+                        K=x.shape[1], E=Er, experts=E, top=top, kind=_ROUTES[route], scale=float(scale), renorm_eps=float(renorm_eps))
+        unit = gated or (0, 0.0, 0.0, 0.0)
+        f = N.MoeFew(router=a, h=h.data_ptr(), w_up=w_up.data_ptr(), w_down=w_down.data_ptr(), act=act.data_ptr(), out=y.data_ptr(), dtype=_code(dt), W=W, ff=ff, gated=int(gated is not None),
+                     unit=int(unit[0]), limit=float(unit[1]), alpha=float(unit[2]), shift=float(unit[3]))
+        N.check_layers(L.jl_moe_few_run(C.byref(f), st), "jl_moe_few_run")
+        return (y, ids, wts) if identity else y
     max_tiles = rows // tm + E
     blocks = int(L.jl_moe_router_blocks(n)) if in_one or from_logits else 0
     lists = torch.empty((rows + E + 2 + 2 * max_tiles + blocks * E + (slices * n * Er if slices > 1 else 0),), dtype=torch.int32, device=dev)       # the grouping's lists, one behind the other, the product's slices
