@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 142
+#define JL_VERSION 143
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -212,6 +212,24 @@ JL_API int jl_token_shift(const float *h, const float *mu, const int32_t *row_re
 #define JL_LINEAR_ADD 3                /* jl_linear_mid: out, of x's dtype, plus the product, rounded once */
 JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int w_dtype, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld,
                            int32_t out_mode, void *stream);
+/* The product of up to JL_AFTER_ROWS bfloat16 rows that the launch makes itself, as the launch before it would (`mode`):
+ *   JL_AFTER_NORM:       jl_sandwich_norm of x [N, K] float (plus y [N, K] of y_dtype, normed by w_post, when given, plus add_row) with w_next; the updated x goes into x_out, which is another buffer
+ *   JL_AFTER_ACT:        jl_gated_act of x (rows x_ld apart of bfloat16, g_col, u_col, K columns; kind, limit, alpha, shift)
+ *   JL_AFTER_GATED_NORM: jl_gated_norm of x [N, K] float in one part, y its bfloat16 gate (rows y_ld apart), w_next the norm's weight (kind, gate_first, scale)
+ * rounded to bfloat16, times w [O, K] transposed (+ bias [O], both bfloat16), into out bfloat16 [N, O].  N * K up to JL_AFTER_VALUES, K a multiple of 8, everything at 16-byte borders. */
+#define JL_AFTER_NORM 0
+#define JL_AFTER_ACT 1
+#define JL_AFTER_GATED_NORM 2
+#define JL_AFTER_ROWS 4
+#define JL_AFTER_VALUES 16384
+typedef struct {
+    const void *x; const void *y; float *x_out; const float *w_post; const float *add_row; const float *w_next; const void *w; const void *bias; void *out;
+    int64_t x_ld, y_ld;
+    int32_t mode, N, K, O, y_dtype, g_col, u_col, kind, gate_first;
+    float eps, scale, limit, alpha, shift;
+} jl_linear_after;
+JL_API int jl_linear_after_ok(int64_t N, int64_t K, int64_t O);      /* whether the launch takes these sizes and is the better one */
+JL_API int jl_linear_after_run(const jl_linear_after *a, void *stream);
 /* The same for more rows (some hundred to a few thousand), all bfloat16, the result at a 16-byte border, operands of up to 4 GB. */
 JL_API int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O);       /* 1: the launch is the better one for these sizes, whatever their type; 2: so much so that products under autocast take it too */
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,

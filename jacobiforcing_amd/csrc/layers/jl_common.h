@@ -97,6 +97,11 @@ __device__ __forceinline__ float gated_unit_f(float g, float u, int kind, float 
     return g * sigmoid_f<FAST>(alpha * g) * (u + shift);
 }
 
+// the gate of jl_gated_norm
+__device__ __forceinline__ float gate_act_f(float g, int act) {
+    const float s = 1.0f / (1.0f + expf(-g));
+    return act == JL_ACT_SILU ? g * s : s;
+}
 // out = raw / sqrt(mean(raw^2) + eps) (* norm_w) * silu(gate) per (row, head) of Dv values, gates at g_col of proj's rows (jl_delta.hip)
 int jl_heads_out(const float *raw, const void *proj, int dtype, int64_t ld, int g_col, const float *norm_w, int64_t NH, int H, int Dv, float eps, void *out, hipStream_t st);
 

@@ -27,7 +27,7 @@ namespace {
 #define JL_HOST_CALLS(X)                                                                                                                              \
     X(jl_linear_small) X(jl_linear_mid_ok) X(jl_linear_mid) X(jl_linear_split_ok) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
     X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) X(jl_latent_heads_run) \
-    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_moe_few_ok) X(jl_moe_few_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
+    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_linear_after_ok) X(jl_linear_after_run) X(jl_moe_few_ok) X(jl_moe_few_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
 #define DECLARE(name) decltype(&name) p_##name;
 JL_HOST_CALLS(DECLARE)
 #undef DECLARE
@@ -251,6 +251,78 @@ CALL(sandwich_norm, 9)
                             (const float *)at_(w_next), at_(out), out.defined() ? code(out) : 0, out.defined() ? out.stride(0) : 0, plain, n, (int32_t)W, stream_of(*x));
     others.back();
     if (into) { Py_INCREF(arg[7]); return arg[7]; }
+    return wrap(out);
+END_CALL
+
+// a product whose rows its launch makes itself: w and bias [O, K], [O], and what linear (without a choice of result) would need of rows that are whole
+bool after_taken(const Tensor &w, const Tensor *bias, int64_t n, int64_t k, const Tensor &like, jl_linear_after &a) {
+    if (w.dim() != 2 || w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.size(1) != k || !starts16(w) || w.device() != like.device() || !p_jl_linear_after_ok(n, k, w.size(0))) return false;
+    if (bias && (bias->scalar_type() != at::kBFloat16 || bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous() || bias->device() != like.device())) return false;
+    if ((c10::GradMode::is_enabled() && (w.requires_grad() || like.requires_grad() || (bias && bias->requires_grad()))) || w._fw_grad(0).defined() || like._fw_grad(0).defined() || (bias && bias->_fw_grad(0).defined())) return false;
+    a.w = w.data_ptr();
+    a.bias = at_(bias);
+    a.N = (int32_t)n; a.K = (int32_t)k; a.O = (int32_t)w.size(0);
+    return !at::autocast::is_autocast_enabled(at::kCUDA);
+}
+// x, y, w_post, eps, w_next, add_row, w, bias: the updated x and the product
+CALL(norm_linear, 8)
+    const Tensor *x, *y, *w_post, *w_next, *add_row, *w, *bias;
+    double eps;
+    NEED(take(arg[0], x) && take_maybe(arg[1], y) && take_maybe(arg[2], w_post) && take(arg[3], eps) && take(arg[4], w_next) && take_maybe(arg[5], add_row) && take(arg[6], w) && take_maybe(arg[7], bias));
+    NEED(x->dim() == 2 && is_float(*x) && x->is_contiguous() && starts16(*x));
+    const int64_t n = x->size(0), W = x->size(1);
+    jl_linear_after a = {};
+    NEED(n > 0 && W > 0 && (!y || (rows(*y, n, W) && known(*y) && y->is_contiguous() && starts16(*y) && w_post)) && row_weights(w_post, W) && row_weights(add_row, W) && row_weights(w_next, W) &&
+         after_taken(*w, bias, n, W, *x, a));
+    Unlocked others;
+    Tensor to = make({n, W}, at::kFloat, *x), out = make({n, w->size(0)}, at::kBFloat16, *x);
+    a.mode = JL_AFTER_NORM;
+    a.x = x->data_ptr(); a.y = at_(y); a.y_dtype = y ? code(*y) : 0; a.x_out = (float *)to.data_ptr(); a.w_post = (const float *)at_(w_post); a.add_row = (const float *)at_(add_row);
+    a.w_next = (const float *)w_next->data_ptr(); a.eps = (float)eps; a.out = out.data_ptr();
+    RUN(jl_linear_after_run, &a, stream_of(*x));
+    others.back();
+    return Py_BuildValue("(NN)", wrap(to), wrap(out));
+END_CALL
+
+// z, g_col, u_col, F, kind, limit, alpha, shift, w, bias
+CALL(act_linear, 10)
+    const Tensor *z, *w, *bias;
+    int32_t g_col, u_col, F, kind;
+    double limit, alpha, shift;
+    NEED(take(arg[0], z) && take(arg[1], g_col) && take(arg[2], u_col) && take(arg[3], F) && take(arg[4], kind) && take(arg[5], limit) && take(arg[6], alpha) && take(arg[7], shift) && take(arg[8], w) &&
+         take_maybe(arg[9], bias));
+    if (u_col < 0) u_col = -1;
+    NEED(z->dim() == 2 && z->scalar_type() == at::kBFloat16 && z->stride(1) == 1 && g_col >= 0 && F > 0 && (int64_t)g_col + F <= z->size(1) && (int64_t)u_col + F <= z->size(1) && starts16(*z));
+    const int64_t n = z->size(0);
+    jl_linear_after a = {};
+    NEED(after_taken(*w, bias, n, F, *z, a));
+    Unlocked others;
+    Tensor out = make({n, w->size(0)}, at::kBFloat16, *z);
+    a.mode = JL_AFTER_ACT;
+    a.x = z->data_ptr(); a.x_ld = z->stride(0); a.g_col = g_col; a.u_col = u_col; a.kind = kind; a.limit = (float)limit; a.alpha = (float)alpha; a.shift = (float)shift; a.out = out.data_ptr();
+    RUN(jl_linear_after_run, &a, stream_of(*z));
+    others.back();
+    return wrap(out);
+END_CALL
+
+// raw, gate, w_norm, eps, act, gate_first, scale, w, bias
+CALL(gated_norm_linear, 9)
+    const Tensor *raw, *gate, *wn, *w, *bias;
+    double eps, scale;
+    int32_t act;
+    bool gate_first;
+    NEED(take(arg[0], raw) && take(arg[1], gate) && take(arg[2], wn) && take(arg[3], eps) && take(arg[4], act) && take(arg[5], gate_first) && take(arg[6], scale) && take(arg[7], w) && take_maybe(arg[8], bias));
+    NEED(raw->dim() == 2 && is_float(*raw) && raw->is_contiguous() && starts16(*raw));
+    const int64_t n = raw->size(0), C = raw->size(1);
+    jl_linear_after a = {};
+    NEED(n > 0 && C > 0 && rows(*gate, n, C) && gate->scalar_type() == at::kBFloat16 && gate->stride(1) == 1 && row_weights(wn, C) && after_taken(*w, bias, n, C, *raw, a));
+    Unlocked others;
+    Tensor out = make({n, w->size(0)}, at::kBFloat16, *raw);
+    a.mode = JL_AFTER_GATED_NORM;
+    a.x = raw->data_ptr(); a.y = gate->data_ptr(); a.y_ld = gate->stride(0); a.w_next = (const float *)wn->data_ptr(); a.eps = (float)eps; a.kind = act; a.gate_first = gate_first; a.scale = (float)scale;
+    a.out = out.data_ptr();
+    RUN(jl_linear_after_run, &a, stream_of(*raw));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -795,7 +867,7 @@ PyObject *symbols(PyObject *, PyObject *) {
 }
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(linear), FAST(linear_add), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
+PyMethodDef methods[] = {FAST(linear), FAST(linear_add), FAST(norm_linear), FAST(act_linear), FAST(gated_norm_linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
                          FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), FAST(step_tables), FAST(step_views), FAST(tile_records), {"bind", bind, METH_VARARGS, nullptr},
                          {"linear_rule", linear_rule, METH_VARARGS, nullptr}, {"symbols", symbols, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_jl_host", nullptr, -1, methods};

@@ -57,6 +57,157 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 #undef LS_LAUNCH
 }
 
+// ---- one row (or a few) that every workgroup makes for itself ------------------------------------------------------------------------------
+// A token alone waits for launches: a norm, an activation or a gate in front of a product takes a launch of 4 us of the GPU and 5 of the host for a few KB.  Here each workgroup of 16 rows of W makes the
+// product's operand itself, in LDS: what the row is made of leaves memory first, this wavefront's weights right behind it, and the operand is made while they travel.  The sums are those of
+// linear_small_kernel.  us of the GPU, one row of 1024 by 1024 to 4096, the launch and the product / so: norm 4.1 + 4.6 / 6.3, unit 4.0 + 4.6 / 5.5, gated norm 4.0 + 4.3 / 5.3.  Every workgroup repeats
+// the row's work, which is why few rows go so, and why more than 512 workgroups (8192 columns) do not.
+template <int MODE, int VI>
+__global__ __launch_bounds__(512) void linear_after_kernel(jl_linear_after a) {
+    constexpr int NW = 8, STEP = 64 * NW * 4;
+    __shared__ ls_f32x4 part[NW][64];
+    __shared__ float red[16];
+    extern __shared__ __attribute__((aligned(16))) bf16_t xs[];     // [N][K]
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g4 = lane >> 4, o0 = blockIdx.x * 16, K = a.K, O = a.O, N = a.N;
+    const int steps = (K + 63) / 64, s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW, k_lane = 8 * g4;
+    const bf16_t *wp = (const bf16_t *)a.w + (int64_t)(o0 + r16 < O ? o0 + r16 : O - 1) * K + k_lane;      // rows that do not exist repeat the last one and are not stored
+    uint4 wr[LS_AHEAD][2];
+    auto load = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < LS_AHEAD; ++i)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const int k = (s + i) * 64 + 32 * y;
+                wr[i][y] = s + i < s1 && k + k_lane < K ? *(const uint4 *)(wp + k) : make_uint4(0, 0, 0, 0);
+            }
+    };
+    for (int n = 0; n < N; ++n) {
+        float x[VI][4], y[VI][4], u[VI][4], v[VI][4], add[VI][4];
+        const bool with = MODE == JL_AFTER_NORM && a.y, row = MODE == JL_AFTER_NORM && a.add_row;
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+            const int c = i * STEP + 4 * tid;
+            if (c >= K) continue;
+            if (MODE == JL_AFTER_ACT) {
+                const bf16_t *z = (const bf16_t *)a.x + n * a.x_ld;
+                ld4_f(z + a.g_col + c, x[i]);
+                if (a.u_col >= 0) ld4_f(z + a.u_col + c, u[i]);
+            } else {
+                ld4_f((const float *)a.x + (int64_t)n * K + c, x[i]);
+                if (MODE == JL_AFTER_GATED_NORM) ld4_f((const bf16_t *)a.y + n * a.y_ld + c, y[i]);
+                else if (with) {
+                    if (a.y_dtype == JL_BF16) ld4_f((const bf16_t *)a.y + (int64_t)n * K + c, y[i]);
+                    else ld4_f((const float *)a.y + (int64_t)n * K + c, y[i]);
+                    ld4_f(a.w_post + c, u[i]);
+                }
+                if (row) ld4_f(a.add_row + c, add[i]);
+                ld4_f(a.w_next + c, v[i]);
+            }
+        }
+        if (n == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(s0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float ss = 0.f, r = 1.f;
+        if (with) {
+#pragma unroll
+            for (int i = 0; i < VI; ++i)
+                if (i * STEP + 4 * tid < K) ss += y[i][0] * y[i][0] + y[i][1] * y[i][1] + y[i][2] * y[i][2] + y[i][3] * y[i][3];
+            ss = block_sum_f32(ss, red);
+            r = 1.0f / sqrtf(ss / (float)K + a.eps);
+#pragma unroll
+            for (int i = 0; i < VI; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[i][e] += y[i][e] * r * u[i][e];
+        }
+        ss = 0.f;
+        if (MODE != JL_AFTER_ACT) {
+#pragma unroll
+            for (int i = 0; i < VI; ++i) {
+                if (i * STEP + 4 * tid >= K) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (row) x[i][e] += add[i][e];
+                    if (MODE == JL_AFTER_GATED_NORM) {
+                        y[i][e] = gate_act_f(y[i][e], a.kind);
+                        if (a.gate_first) x[i][e] *= y[i][e];
+                    }
+                }
+                if (MODE == JL_AFTER_NORM && blockIdx.x == 0) st4_f(a.x_out + (int64_t)n * K + i * STEP + 4 * tid, x[i]);
+                ss += x[i][0] * x[i][0] + x[i][1] * x[i][1] + x[i][2] * x[i][2] + x[i][3] * x[i][3];
+            }
+            ss = block_sum_f32(ss, red);
+            r = (MODE == JL_AFTER_GATED_NORM ? a.scale : 1.0f) / sqrtf(ss / (float)K + a.eps);
+        }
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+            const int c = i * STEP + 4 * tid;
+            if (c >= K) continue;
+            float to[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                to[e] = MODE == JL_AFTER_ACT ? gated_unit_f<true>(x[i][e], a.u_col >= 0 ? u[i][e] : 1.0f, a.kind, a.limit, a.alpha, a.shift)
+                        : MODE == JL_AFTER_NORM ? v[i][e] * (x[i][e] * r) : v[i][e] * (x[i][e] * r * (a.gate_first ? 1.0f : y[i][e]));
+            st4_f(xs + (int64_t)n * K + c, to);
+        }
+    }
+    __syncthreads();
+    const bf16_t *xp = xs + (r16 < N ? r16 : N - 1) * K + k_lane;
+    ls_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += LS_AHEAD) {
+        if (s > s0) load(s);
+#pragma unroll
+        for (int i = 0; i < LS_AHEAD; ++i)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+                const int k = (s + i) * 64 + 32 * y;
+                acc = ls_mma((const bf16_t *)nullptr, wr[i][y], s + i < s1 && k + k_lane < K ? *(const uint4 *)(xp + k) : make_uint4(0, 0, 0, 0), acc);
+            }
+    }
+    part[wave][lane] = acc;
+    __syncthreads();
+    const int o = o0 + 4 * g4;
+    if (tid >= 64 || r16 >= N || o >= O) return;
+    ls_f32x4 sum = part[0][lane];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) sum += part[i][lane];
+    bf16_t *out = (bf16_t *)a.out + (int64_t)r16 * O + o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (o + i < O) st_f(out + i, a.bias ? sum[i] + ld_f((const bf16_t *)a.bias + o + i) : sum[i]);
+}
+
+extern "C" int jl_linear_after_ok(int64_t N, int64_t K, int64_t O) {
+    return N > 0 && N <= JL_AFTER_ROWS && K > 0 && K % 8 == 0 && K <= 8192 && N * K <= JL_AFTER_VALUES && O > 0 && O <= 8192;
+}
+extern "C" int jl_linear_after_run(const jl_linear_after *ap, void *stream) {
+    if (!ap) return jl_fail(JL_E_INVALID, "jl_linear_after_run: null arguments");
+    const jl_linear_after &a = *ap;
+    if (!a.x || !a.w || !a.out || !jl_linear_after_ok(a.N, a.K, a.O)) return jl_fail(JL_E_INVALID, "jl_linear_after_run: null pointer, or up to %d rows and %d values of theirs", JL_AFTER_ROWS, JL_AFTER_VALUES);
+    auto al = [](const void *q, uintptr_t b) { return ((uintptr_t)q % b) == 0; };
+    if (!al(a.x, 16) || !al(a.y, 8) || !al(a.w, 16) || !al(a.w_post, 16) || !al(a.add_row, 16) || !al(a.w_next, 16)) return jl_fail(JL_E_INVALID, "jl_linear_after_run: operands at 16-byte borders");
+    if (a.mode == JL_AFTER_NORM ? !a.x_out || a.x_out == a.x || !al(a.x_out, 16) || !a.w_next || (a.y && (!a.w_post || (a.y_dtype != JL_BF16 && !al(a.y, 16))))
+        : a.mode == JL_AFTER_ACT ? a.g_col < 0 || a.g_col % 4 || (a.u_col >= 0 && a.u_col % 4) || a.x_ld % 4 || a.g_col + (int64_t)a.K > a.x_ld || a.u_col + (int64_t)a.K > a.x_ld ||
+                                       a.kind < JL_ACT_GELU_TANH || a.kind > JL_ACT_GELU_ERF
+                                 : a.mode != JL_AFTER_GATED_NORM || !a.y || a.y_ld < a.K || a.y_ld % 4 || !a.w_next || (a.kind != JL_ACT_SILU && a.kind != JL_ACT_SIGMOID))
+        return jl_fail(JL_E_INVALID, "jl_linear_after_run: bad operands for the mode");
+    const dim3 grid((unsigned)((a.O + 15) / 16));
+    const int lds = a.N * a.K * 2;
+    hipStream_t st = (hipStream_t)stream;
+#define LA_MODE(M)                                                                       \
+    do {                                                                                  \
+        if (a.K <= 2048) linear_after_kernel<M, 1><<<grid, 512, lds, st>>>(a);             \
+        else if (a.K <= 4096) linear_after_kernel<M, 2><<<grid, 512, lds, st>>>(a);        \
+        else linear_after_kernel<M, 4><<<grid, 512, lds, st>>>(a);                         \
+    } while (0)
+    if (a.mode == JL_AFTER_NORM) LA_MODE(JL_AFTER_NORM);
+    else if (a.mode == JL_AFTER_ACT) LA_MODE(JL_AFTER_ACT);
+    else LA_MODE(JL_AFTER_GATED_NORM);
+#undef LA_MODE
+    return jl_check_launch("linear_after_kernel");
+}
+
 // ---- some hundred to a few thousand rows: TM of x by TN of W per workgroup -------------------------------------------------------------------------
 // Stages of 128 bytes of every row go from memory straight into a ring of RING buffers in LDS (16 bytes per lane, every lane fetching the unit that the permutation puts into its place).  A wavefront
 // reads the next stage's operands into registers while it multiplies this one's, so that one barrier per stage says both that the next stage is there and that this one may be written over, and multiplies

@@ -917,10 +917,6 @@ extern "C" int jl_output_norm(float *x, const jl_addend *addends, int32_t n_adde
 
 // ---- norm over equal parts of a mixer's output with its gate: one workgroup per (row, part) -------------------------------------------------
 //   gate first:  v = raw * act(gate);  out = v / rms(v) * w * scale          gate last:  out = raw / rms(raw) * w * act(gate) * scale
-__device__ __forceinline__ float gate_act_f(float g, int act) {
-    const float s = 1.0f / (1.0f + expf(-g));
-    return act == JL_ACT_SILU ? g * s : s;
-}
 template <typename T, int VI>
 __global__ __launch_bounds__(256) void gated_norm_vec_kernel(const float *__restrict__ raw, const T *__restrict__ gate, int64_t gate_ld, const float *__restrict__ w,
                                                               float eps, int act, int gate_first, float scale, T *__restrict__ out, int64_t out_ld, int C, int part) {

@@ -1140,6 +1140,36 @@ def gated_norm(raw: torch.Tensor, gate: torch.Tensor, w: torch.Tensor, eps: floa
     return out
 
 
+# A row alone (decoding for one user) and a few go from a norm, a unit or a gate into the product in one launch, every workgroup of which makes the rows for itself (linear_after_kernel); others take the two
+# calls.  us a pass of one token through four layers, 1024 wide: 311 in launches of their own (49), 264 so (34).
+def norm_linear(x: torch.Tensor, y: Optional[torch.Tensor], w_post: Optional[torch.Tensor], eps: float, w_next: torch.Tensor, add_row: Optional[torch.Tensor], w: torch.Tensor,
+                bias: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``sandwich_norm`` into w's dtype and ``linear`` of its result: the updated x (x itself, or another tensor, x as it was) and the product."""
+    if not is_dynamo_compiling():
+        r = (_H or _host()).norm_linear(x, y, w_post, eps, w_next, add_row, w, bias)
+        if r is not NotImplemented:
+            return r
+    return x, linear(sandwich_norm(x, y, w_post, eps, w_next, w.dtype, add_row=add_row), w, bias)
+
+
+def act_linear(z: torch.Tensor, g_col: int, u_col: int, F_: int, kind: int, w: torch.Tensor, bias: Optional[torch.Tensor] = None, limit: float = 0.0, alpha: float = 1.0, shift: float = 0.0) -> torch.Tensor:
+    """``linear`` of ``gated_act``'s result."""
+    if not is_dynamo_compiling():
+        r = (_H or _host()).act_linear(z, g_col, u_col, F_, kind, limit, alpha, shift, w, bias)
+        if r is not NotImplemented:
+            return r
+    return linear(gated_act(z, g_col, u_col, F_, kind, limit, alpha, shift), w, bias)
+
+
+def gated_norm_linear(raw: torch.Tensor, gate: torch.Tensor, w_norm: torch.Tensor, eps: float, act: int, gate_first: bool, w: torch.Tensor, parts: int = 1, scale: float = 1.0) -> torch.Tensor:
+    """``linear`` of ``gated_norm``'s result."""
+    if parts == 1 and not is_dynamo_compiling():
+        r = (_H or _host()).gated_norm_linear(raw, gate, w_norm, eps, act, gate_first, scale, w, None)
+        if r is not NotImplemented:
+            return r
+    return linear(gated_norm(raw, gate, w_norm, eps, act, gate_first, parts, scale), w)
+
+
 def polynorm(z: torch.Tensor, coef: torch.Tensor, eps: float) -> torch.Tensor:
     """c0 n(z) + c1 n(z^2) + c2 n(z^3) + c3 with n(u) = u / rms(u) over a row; z [N, F], coef four floats."""
     _dev(z)

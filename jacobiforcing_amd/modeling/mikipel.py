@@ -292,7 +292,7 @@ class MikipelModel:
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
             ff = int(f["ff"])
-            return [(LO.linear(LO.gated_act(LO.linear(h, w["w_up"]), 0, -1, ff, LO.ACT_GELU_ERF), w["w_down"]), None)]
+            return [(LO.act_linear(LO.linear(h, w["w_up"]), 0, -1, ff, LO.ACT_GELU_ERF, w["w_down"]), None)]
         return [(LO.moe_experts(h, None, None, int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="top_softmax", gated=(LO.ACT_SILU, 0.0, 1.0, 0.0),
                                 router=(h_float, w["router"], w["router_b"])), None)]
 

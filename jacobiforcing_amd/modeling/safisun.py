@@ -288,27 +288,31 @@ class SafisunModel:
                 a = torch.arange(n, dtype=torch.float32, device=self.device).view(n, 1) * f.view(1, -1)
                 self._angles[key] = (a.cos().contiguous(), a.sin().contiguous())
 
-    # ---- mixers: from the norm's output to the mixer's result (behind its output projection) ----------------------------------------------
+    # ---- mixers: from the norm's output (or its input projection, where that was the norm's launch) to the mixer's result (behind its output projection) ----------------------------------------------
     def _linear_attention(self, m, w, proj: torch.Tensor, run: int, batch: LO.RaggedBatch, cache: PagedStateCache, scale: float, out: Optional[torch.Tensor]) -> torch.Tensor:
-        """Lightning attention on the columns ``w["cols"]`` of a product, up to (not with) its output projection."""
+        """Lightning attention on the columns ``w["cols"]`` of a product, into ``out`` (without its output projection) or through its output projection."""
         H, D, Dv = _lightning_sizes(m)
         cols = w["cols"]
         raw = LO.linear_scan(proj, cols[:3], batch, H, H, D, Dv, cache.state[run], act=LO.ACT_SILU, decay=w["decay"])
-        return LO.gated_norm(raw, proj[:, cols[3]:cols[3] + H * Dv], w["out_norm"], self.cfg.norm_eps, LO.ACT_SIGMOID, False, scale=scale, out=out)
+        gate = proj[:, cols[3]:cols[3] + H * Dv]
+        if out is None:
+            return LO.gated_norm_linear(raw, gate, w["out_norm"], self.cfg.norm_eps, LO.ACT_SIGMOID, False, w["w_o"], scale=scale)
+        return LO.gated_norm(raw, gate, w["out_norm"], self.cfg.norm_eps, LO.ACT_SIGMOID, False, scale=scale, out=out)
 
-    def _lightning(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
+    def _lightning(self, run: int, li: int, h: Optional[torch.Tensor], batch: LO.RaggedBatch, cache: PagedStateCache, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         w = self.w.layers[li]
-        return LO.linear(self._linear_attention(self.cfg.layers[li]["mixer"], w, LO.linear(h, w["w_in"]), run, batch, cache, 1.0, None), w["w_o"])
+        return self._linear_attention(self.cfg.layers[li]["mixer"], w, LO.linear(h, w["w_in"]) if proj is None else proj, run, batch, cache, 1.0, None)
 
-    def _mamba2(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
+    def _mamba2(self, run: int, li: int, h: Optional[torch.Tensor], batch: LO.RaggedBatch, cache: PagedStateCache, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]
         H, G, N, Dv, taps, C_ = _mamba_sizes(m)
         inner = H * Dv
-        proj = LO.linear(h, w["w_in"])                   # z | x | B | C | dt
+        if proj is None:
+            proj = LO.linear(h, w["w_in"])               # z | x | B | C | dt
         xbc = LO.short_conv(proj, inner, C_, w["conv"], batch, cache.tails[run].get("conv"), LO.ACT_SILU, bias=w["conv_b"], out_dtype=self.dtype)
         y = LO.linear_scan(xbc, (inner + G * N, inner, 0), batch, H, G, N, Dv, cache.state[run], dt=proj[:, inner + C_:inner + C_ + H], a_log=w["a_log"],
                            dt_bias=w["dt_bias"], skip=w["skip"])
-        return LO.linear(LO.gated_norm(y, proj[:, :inner], w["out_norm"], self.cfg.norm_eps, LO.ACT_SILU, True, parts=int(m["norm_groups"])), w["w_o"])
+        return LO.gated_norm_linear(y, proj[:, :inner], w["out_norm"], self.cfg.norm_eps, LO.ACT_SILU, True, w["w_o"], parts=int(m["norm_groups"]))
 
     def _attention(self, m, w, proj: torch.Tensor, run: int, batch: LO.RaggedBatch, cache: PagedStateCache, scale: float, out: torch.Tensor) -> torch.Tensor:
         """The parallel mixer's left side on its columns of the product, up to (not with) its output projection."""
@@ -323,14 +327,15 @@ class SafisunModel:
             return LO.attn_sweep(q, kp, vp, batch, H, G, D, Dv, float(m["scale"]), 0, gate=gate, **kw)
         return LO.attn_window(q, gate, kp, vp, batch, H, G, D, Dv, float(m["scale"]), 0, 0, None, None, None, **kw)
 
-    def _parallel(self, run: int, li: int, h: torch.Tensor, batch: LO.RaggedBatch, cache: PagedStateCache) -> torch.Tensor:
+    def _parallel(self, run: int, li: int, h: Optional[torch.Tensor], batch: LO.RaggedBatch, cache: PagedStateCache, proj: Optional[torch.Tensor] = None) -> torch.Tensor:
         m, w = self.cfg.layers[li]["mixer"], self.w.layers[li]
         H, _, _, Dv = _attention_sizes(m["left"])
-        n, left, width = h.shape[0], H * Dv, w["w_o"].shape[1]
-        proj = LO.linear(h, w["w_in"], w["b_in"])
+        if proj is None:
+            proj = LO.linear(h, w["w_in"], w["b_in"])
+        n, left, width = proj.shape[0], H * Dv, w["w_o"].shape[1]
         # both sides write their columns of one matrix, scaled; the output product over all of them is the weighted sum.  Rows start at
         # 16-byte borders; the right side starts where the left one ends
-        both = torch.empty((n, width + (-width) % 8), dtype=h.dtype, device=h.device)[:, :width]
+        both = torch.empty((n, width + (-width) % 8), dtype=proj.dtype, device=proj.device)[:, :width]
         self._attention(m["left"], w, proj, run, batch, cache, float(m["left_scale"]), both[:, :left])
         self._linear_attention(m["right"], w, proj, run, batch, cache, float(m["right_scale"]), both[:, left:])
         return LO.linear(both, w["w_o"])
@@ -352,11 +357,12 @@ class SafisunModel:
             again[:, W:] = x
         pending = None                                   # the last sublayer's output and its norm's weight, folded into the next norm's launch
 
-        def norm(w_next, add_row=None):
-            nonlocal pending
+        def norm(w_next, add_row, w_in, b_in=None):      # ... and the next sublayer's first product behind that
+            nonlocal pending, x
             y, wb = pending or (None, None)
             pending = None
-            return LO.sandwich_norm(x, y, wb, eps, w_next, dt, add_row=add_row)
+            x, proj = LO.norm_linear(x, y, wb, eps, w_next, add_row, w_in, b_in)
+            return proj
 
         for run, (li, begins) in enumerate(self.runs):
             L, lw = cfg.layers[li], w.layers[li]
@@ -366,18 +372,17 @@ class SafisunModel:
                 pending = None
                 LO.sandwich_norm(x, y, wb, eps, out=again[:, :W], plain=True)
                 x, step = LO.product_f32(again, w.loop_in), w.loop_step[begins]
-            h = norm(lw["norm1"], step)
+            proj = norm(lw["norm1"], step, lw["w_in"], lw["b_in"] if L["type"] == "parallel" else None)
             mixer = self._lightning if L["type"] == "lightning" else self._mamba2 if L["type"] == "mamba2" else self._parallel
-            pending = (mixer(run, li, h, batch, cache), lw["norm1b"])
+            pending = (mixer(run, li, None, batch, cache, proj), lw["norm1b"])
             if L.get("mlp") is not None:
                 ff = int(L["mlp"]["ff"])
-                h = norm(lw["norm2"])
-                pending = (LO.linear(LO.gated_act(LO.linear(h, lw["w_gu"]), 0, ff, ff, LO.ACT_SILU), lw["w_down"]), lw["norm2b"])
+                pending = (LO.act_linear(norm(lw["norm2"], None, lw["w_gu"]), 0, ff, ff, LO.ACT_SILU, lw["w_down"]), lw["norm2b"])
             if trace is not None:
                 LO.sandwich_norm(x, *pending, eps)
                 pending = None
                 trace.append(x.clone())
-        hl = norm(w.final_norm)
+        hl = LO.sandwich_norm(x, *(pending or (None, None)), eps, w.final_norm, dt)
         if logit_rows is not None:
             hl = hl.index_select(0, logit_rows)
         return LO.linear(hl, w.head, float_out=False)

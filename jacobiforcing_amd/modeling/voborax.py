@@ -255,7 +255,7 @@ class VoboraxModel:
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
             z = LO.linear(h, w["w_up"], w["b_up"])
-            return [(LO.linear(LO.gated_act(z, 0, -1, z.shape[1], LO.ACT_GELU_TANH), w["w_down"], w["b_down"]), None)], None
+            return [(LO.act_linear(z, 0, -1, z.shape[1], LO.ACT_GELU_TANH, w["w_down"], w["b_down"]), None)], None
         E, ident = _experts(f)
         y = LO.moe_experts(h, None, w["correction"], int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm",
                            renorm_eps=ROUTER_RENORM_EPS, gated=(LO.ACT_SILU, 0.0, 1.0, 0.0), identity=ident, router=(x, w["router"], None))
@@ -263,7 +263,7 @@ class VoboraxModel:
         out = [(y, None)]
         if f.get("shared") is not None:
             fs = int(f["shared"]["ff"])
-            out.append((LO.linear(LO.gated_act(LO.linear(h, w["w_sh"]), 0, fs, fs, LO.ACT_SILU), w["w_sh_down"]), None))
+            out.append((LO.act_linear(LO.linear(h, w["w_sh"]), 0, fs, fs, LO.ACT_SILU, w["w_sh_down"]), None))
         return out, choices
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------
