@@ -17,7 +17,7 @@ extern "C" {
 #endif
 
 #define JL_API __attribute__((visibility("default")))
-#define JL_VERSION 143
+#define JL_VERSION 145
 #define JL_OK 0
 #define JL_E_INVALID (-1)
 #define JL_E_LAUNCH (-3)
@@ -234,6 +234,9 @@ JL_API int jl_linear_after_run(const jl_linear_after *a, void *stream);
 JL_API int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O);       /* 1: the launch is the better one for these sizes, whatever their type; 2: so much so that products under autocast take it too */
 JL_API int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
                          void *stream);
+/* The same with a gated unit in its epilogue: W [2 F, K], a unit's gates and behind them its linear branches; out bfloat16 [N, F] = unit(x . W[c], x . W[F + c]) of jl_gated_act's kinds, from the float sums.
+ * Where jl_linear_mid_ok(N, K, 2 F) says so. */
+JL_API int jl_linear_mid_gated(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t F, int32_t kind, float limit, float alpha, float shift, void *out, int64_t out_ld, void *stream);
 
 /* The same for float rows of any number (x [N, x_ld], W [O, K], rows at 16-byte borders, out rows out_ld floats apart), on the bfloat16 matrix instructions in three terms per operand: sums at
  * least as close to 64 bits as the float instructions' (measured at depths of 4 to 4096), but for operands below 2^-118, whose digits beyond bfloat16's last place, 2^-133, are lost.  Infinities, NaN
@@ -272,6 +275,9 @@ JL_API int jl_sandwich_norm(const float *x_in, float *x_out, const void *y, int 
 JL_API int jl_output_norm(float *x, const jl_addend *addends, int32_t n_addends, const int32_t *ids, const float *weights, int32_t top,
                           int32_t n_experts, int32_t kind, const float *w, float mult, float eps, const float *w_next, void *out, int dtype,
                           int64_t N, int32_t W, void *stream);
+
+/* out = x / sqrt(mean(x^2) + eps) * w, x and out [N, W] and w [W] of dtype, computed in float and rounded once; W up to 512 units of 16 bytes, everything at 16-byte borders. */
+JL_API int jl_rms_norm(const void *x, int dtype, const void *w, float eps, void *out, int64_t N, int32_t W, void *stream);
 
 /* Norm and gate on a recurrent mixer's float output raw [N, C], over `parts` equal parts of the row (each by its own root mean square):
  *   gate_first != 0:  v = raw * act(gate), out = v / sqrt(mean(v^2) + eps) * w * scale

@@ -231,7 +231,7 @@ def raise_state_error(code: int, what: str, aux: int = 0):
 
 # ---- libjf_layers.so (include/jf_layers.h): layer kernels of the models whose forward is not stock PyTorch ----------------------------
 JL_F32, JL_BF16 = 0, 1
-JL_VERSION = 143                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
+JL_VERSION = 145                 # include/jf_layers.h: a library of another version is not called (its signatures may differ)
 JL_OUT_SAME, JL_OUT_F32 = 0, 2
 JL_ACT_GELU_TANH, JL_ACT_CLAMPED_SWISH, JL_ACT_SILU, JL_ACT_GELU_ERF, JL_ACT_SIGMOID, JL_ACT_NONE = 0, 1, 2, 3, 4, -1
 JL_ROUTE_SIGMOID, JL_ROUTE_SOFTMAX_RENORM, JL_ROUTE_TOP_SOFTMAX = 0, 1, 2
@@ -356,6 +356,8 @@ _LAYER_SIGNATURES = {
     "jl_delta_rule": (C.c_int, [_vp, C.c_int, _i64, _i32, _i32, _i32, _vp, C.c_int, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                 _i32, _i32, _f32, _f32, _f32, _vp, _vp, _vp, _vp]),
     "jl_latent_heads_run": (C.c_int, [C.POINTER(LatentHeads), _vp]),
+    "jl_rms_norm": (C.c_int, [_vp, C.c_int, _vp, C.c_float, _vp, _i64, _i32, _vp]),
+    "jl_linear_mid_gated": (C.c_int, [_vp, C.c_int, _i64, _i64, _vp, _i32, _i32, _i32, C.c_float, C.c_float, C.c_float, _vp, _i64, _vp]),
     "jl_linear_mid_ok": (C.c_int, [_i64, _i64, _i64]),
     "jl_linear_after_ok": (C.c_int, [_i64, _i64, _i64]),
     "jl_linear_after_run": (C.c_int, [_vp, _vp]),

@@ -27,7 +27,7 @@ namespace {
 #define JL_HOST_CALLS(X)                                                                                                                              \
     X(jl_linear_small) X(jl_linear_mid_ok) X(jl_linear_mid) X(jl_linear_split_ok) X(jl_linear_split) X(jl_embed_scale) X(jl_add_rmsnorm) X(jl_sandwich_norm) X(jl_output_norm) X(jl_gated_norm) \
     X(jl_gated_act) X(jl_heads_gate) X(jl_latent_prep) X(jl_latent_q_pack) X(jl_token_shift) X(jl_depth_mix_norm) X(jl_short_conv) X(jl_linear_scan) X(jl_latent_heads_run) \
-    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_linear_after_ok) X(jl_linear_after_run) X(jl_moe_few_ok) X(jl_moe_few_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
+    X(jl_moe_router_blocks) X(jl_moe_router_run) X(jl_linear_mid_gated) X(jl_rms_norm) X(jl_linear_after_ok) X(jl_linear_after_run) X(jl_moe_few_ok) X(jl_moe_few_run) X(jl_moe_gemm) X(jl_moe_gemm_gated) X(jl_qk_norm_append)
 #define DECLARE(name) decltype(&name) p_##name;
 JL_HOST_CALLS(DECLARE)
 #undef DECLARE
@@ -251,6 +251,40 @@ CALL(sandwich_norm, 9)
                             (const float *)at_(w_next), at_(out), out.defined() ? code(out) : 0, out.defined() ? out.stride(0) : 0, plain, n, (int32_t)W, stream_of(*x));
     others.back();
     if (into) { Py_INCREF(arg[7]); return arg[7]; }
+    return wrap(out);
+END_CALL
+
+// x, w, kind, limit, alpha, shift: the unit of a product whose columns are its gates and its linear branches (linear_gated)
+CALL(linear_gated, 6)
+    const Tensor *x, *w;
+    int32_t kind;
+    double limit, alpha, shift;
+    NEED(take(arg[0], x) && take(arg[1], w) && take(arg[2], kind) && take(arg[3], limit) && take(arg[4], alpha) && take(arg[5], shift));
+    NEED(x->dim() == 2 && w->dim() == 2 && x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16);
+    const int64_t n = x->size(0), k = x->size(1), o = w->size(0), ld = x->stride(0);
+    NEED(n > 0 && k > 0 && o > 1 && o % 2 == 0 && o <= INT32_MAX && k <= INT32_MAX && !rule_small(n, k, o, 2) && p_jl_linear_mid_ok(n, k, o) && !at::autocast::is_autocast_enabled(at::kCUDA));
+    NEED(w->size(1) == k && w->is_contiguous() && x->stride(1) == 1 && ld >= k && k % 8 == 0 && ld % 8 == 0 && starts16(*x) && starts16(*w) && w->device() == x->device() && n * ld * 2 < (int64_t)1 << 32);
+    NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())) && !x->_fw_grad(0).defined() && !w->_fw_grad(0).defined());
+    Unlocked others;
+    Tensor out = make({n, o / 2}, at::kBFloat16, *x);
+    RUN(jl_linear_mid_gated, x->data_ptr(), JL_BF16, n, ld, w->data_ptr(), (int32_t)k, (int32_t)(o / 2), kind, (float)limit, (float)alpha, (float)shift, out.data_ptr(), o / 2, stream_of(*x));
+    others.back();
+    return wrap(out);
+END_CALL
+
+// x, w, eps
+CALL(rms_norm, 3)
+    const Tensor *x, *w;
+    double eps;
+    NEED(take(arg[0], x) && take(arg[1], w) && take(arg[2], eps));
+    NEED(x->dim() >= 1 && known(*x) && x->is_contiguous() && w->dim() == 1 && w->scalar_type() == x->scalar_type() && w->is_contiguous() && w->size(0) == x->size(-1) && w->device() == x->device());
+    const int64_t W = w->size(0);
+    NEED(W > 0 && W <= 512 * 8 && x->numel() > 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && !(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())) &&
+         !x->_fw_grad(0).defined() && !w->_fw_grad(0).defined());
+    Unlocked others;
+    Tensor out = at::empty(x->sizes(), x->options());
+    RUN(jl_rms_norm, x->data_ptr(), code(*x), w->data_ptr(), (float)eps, out.data_ptr(), x->numel() / W, (int32_t)W, stream_of(*x));
+    others.back();
     return wrap(out);
 END_CALL
 
@@ -867,7 +901,7 @@ PyObject *symbols(PyObject *, PyObject *) {
 }
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(linear), FAST(linear_add), FAST(norm_linear), FAST(act_linear), FAST(gated_norm_linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
+PyMethodDef methods[] = {FAST(linear), FAST(linear_add), FAST(linear_gated), FAST(rms_norm), FAST(norm_linear), FAST(act_linear), FAST(gated_norm_linear), FAST(add_rmsnorm), FAST(sandwich_norm), FAST(output_norm), FAST(gated_norm), FAST(gated_act), FAST(heads_gate), FAST(latent_prep), FAST(latent_q_pack), FAST(latent_heads),
                          FAST(token_shift), FAST(depth_mix_norm), FAST(short_conv), FAST(linear_scan), FAST(embed_scale), FAST(moe_experts), FAST(attention_args), FAST(qk_norm_append), FAST(step_tables), FAST(step_views), FAST(tile_records), {"bind", bind, METH_VARARGS, nullptr},
                          {"linear_rule", linear_rule, METH_VARARGS, nullptr}, {"symbols", symbols, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_jl_host", nullptr, -1, methods};

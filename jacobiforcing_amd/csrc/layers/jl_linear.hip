@@ -218,9 +218,12 @@ extern "C" int jl_linear_after_run(const jl_linear_after *ap, void *stream) {
 // by 2048 11.1 / 10.6 / 9.9; 2048 x 1024 by 200 10.1 / 12.1 / 10.4, 1000 x 4864 by 896 21.9 / 27.3 / 21.3, 1536 x 1536 by 1300 14.3 / 14.0 / 12.4, 1024 x 1536 by 2048 13.9 / 16.1 / 14.1, 2048 x 2048 by
 // 2048 22.6 / 32.4 / 23.5, 1024 x 4096 by 2048 22.2 / 33.2 / 23.2; and the call takes the host 5 us, the library's 21.
 typedef uint32_t ld_u32x4 __attribute__((ext_vector_type(4)));
-template <int TM, int TN, int WM, int WN, int RING>
+// GATED: W's rows are a unit's gates and behind them its O linear branches; a lane's first COLS / 2 columns are gates, the others their linear branches, and the unit leaves
+// (2048 rows of 1024 by 2 x 2048: 24.9 us and 5.9 for the unit in a launch of its own, 24.5 so).
+struct LinearUnit { int kind; float limit, alpha, shift; };
+template <int TM, int TN, int WM, int WN, int RING, bool GATED>
 __global__ __launch_bounds__(64 * WM * WN, (WM * WN >= 8 ? 1 : 2) * WM * WN / 4) void linear_mid_kernel(const bf16_t *__restrict__ x, int64_t x_ld, const bf16_t *__restrict__ w, const bf16_t *__restrict__ bias,
-                                                                                                   void *__restrict__ out, int64_t out_ld, int N, int K, int O, int out_mode, int row_tiles, int tiles) {
+                                                                                                   void *__restrict__ out, int64_t out_ld, int N, int K, int O, int out_mode, int row_tiles, int tiles, LinearUnit unit) {
     constexpr int THREADS = 64 * WM * WN, U = 8, UNIT = 8, STAGE = 64, BUF = (TM + TN) * U, XT = TM / WM / 16, NT = TN / WN / 16, XL = TM * U / THREADS, WL = TN * U / THREADS, COLS = 4 * NT;
     static_assert(NT == 2 || NT == 4, "a lane's columns in whole stores");
     extern __shared__ __attribute__((aligned(16))) uint4 ldS[];
@@ -228,7 +231,7 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN >= 8 ? 1 : 2) * WM * WN / 4)
     const int per_xcd = (tiles + 7) / 8, tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;
     const int cols = tiles / row_tiles, high = 1024 / TM < row_tiles ? 1024 / TM : row_tiles, strip = tile / (high * cols), here = row_tiles - strip * high < high ? row_tiles - strip * high : high;
-    const int in_strip = tile - strip * high * cols, n0 = (strip * high + in_strip % here) * TM, o0 = in_strip / here * TN;
+    const int in_strip = tile - strip * high * cols, n0 = (strip * high + in_strip % here) * TM, o0 = in_strip / here * (GATED ? TN / 2 : TN);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, quad = lane >> 4, wm = wave / WN, wn = wave % WN;
     // unit u of a row of LDS lies at u ^ swap: the sixteen rows that are read at once meet different banks.  Row 16 b + i of a wavefront's rows of W there is row COLS * (i / 4) + 4 b + i % 4 of them
     auto swap = [](int row) { return (row >> 1) & 7; };
@@ -242,8 +245,8 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN >= 8 ? 1 : 2) * WM * WN / 4)
     }
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
-        const int o = o0 + w_row(lr + THREADS / U * i);
-        wo[i] = (uint32_t)((o < O ? o : O - 1) * (int64_t)K + lu * UNIT) * 2;
+        const int r = w_row(lr + THREADS / U * i), linear = GATED && r % COLS >= COLS / 2, o = o0 + (GATED ? r / COLS * (COLS / 2) + r % (COLS / 2) : r);
+        wo[i] = (uint32_t)(((o < O ? o : O - 1) + (linear ? O : 0)) * (int64_t)K + lu * UNIT) * 2;
     }
     const char *xb = (const char *)x, *wb = (const char *)w;
     const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)(ldS + wave * 64));
@@ -326,6 +329,28 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN >= 8 ? 1 : 2) * WM * WN / 4)
         read(0, 0);
         products(0);
     }
+    if constexpr (GATED) {
+        constexpr int HALF = COLS / 2;
+        const int o = o0 + (wn * (TN / WN) + quad * COLS) / 2;
+#pragma unroll
+        for (int a = 0; a < XT; ++a) {
+            const int n = n0 + wm * (TM / WM) + 16 * a + l16;
+            if (n >= N || o >= O) continue;
+            float v[HALF / 4][4];
+#pragma unroll
+            for (int e = 0; e < HALF; ++e) v[e >> 2][e & 3] = gated_unit_f<true>(acc[a][e >> 2][e & 3], acc[a][(HALF + e) >> 2][e & 3], unit.kind, unit.limit, unit.alpha, unit.shift);
+            bf16_t *p = (bf16_t *)out + n * out_ld + o;
+#pragma unroll
+            for (int e = 0; e < HALF; e += 4) {
+                if (O % 4 == 0 && out_ld % 4 == 0) { if (o + e < O) st4_f(p + e, v[e >> 2]); }
+                else
+#pragma unroll
+                    for (int y = 0; y < 4; ++y)
+                        if (o + e + y < O) st_f(p + e + y, v[e >> 2][y]);
+            }
+        }
+        return;
+    }
     const int o = o0 + wn * (TN / WN) + quad * COLS;                // this lane's COLS columns
     const bool whole = O % 8 == 0 && out_ld % 8 == 0, float_out = out_mode == JL_LINEAR_FLOAT || out_mode == JL_LINEAR_ROUNDED_FLOAT;
     float add[COLS];
@@ -390,17 +415,17 @@ extern "C" int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O) {
     if (N > 2304 || ((N + 127) / 128) * ((O + 127) / 128) > 512 || K * O > (int64_t)32 << 20) return 0;
     return K <= 2048 || (K <= 4096 && N >= 300 && tiles <= 512);
 }
-template <int TM, int TN, int WM, int WN, int RING>
-static int linear_mid_launch(const bf16_t *x, int64_t N, int64_t x_ld, const bf16_t *w, int32_t K, int32_t O, const bf16_t *bias, void *out, int64_t out_ld, int32_t out_mode, hipStream_t st) {
-    const int64_t row_tiles = (N + TM - 1) / TM, tiles = row_tiles * ((O + TN - 1) / TN);
+template <int TM, int TN, int WM, int WN, int RING, bool GATED = false>
+static int linear_mid_launch(const bf16_t *x, int64_t N, int64_t x_ld, const bf16_t *w, int32_t K, int32_t O, const bf16_t *bias, void *out, int64_t out_ld, int32_t out_mode, hipStream_t st, LinearUnit unit = {0, 0.f, 0.f, 0.f}) {
+    const int64_t row_tiles = (N + TM - 1) / TM, cols = GATED ? TN / 2 : TN, tiles = row_tiles * ((O + cols - 1) / cols);
     if (tiles > INT32_MAX / (64 * WM * WN)) return jl_fail(JL_E_INVALID, "jl_linear_mid: too many tiles");
     constexpr int lds = (TM + TN) * 128 * RING;
-    auto kern = linear_mid_kernel<TM, TN, WM, WN, RING>;
+    auto kern = linear_mid_kernel<TM, TN, WM, WN, RING, GATED>;
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return jl_fail(JL_E_LAUNCH, "jl_linear_mid: cannot get %d bytes of LDS: %s", lds, hipGetErrorString(e));
     }
-    kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 64 * WM * WN, lds, st>>>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (int)row_tiles, (int)tiles);
+    kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 64 * WM * WN, lds, st>>>(x, x_ld, w, bias, out, out_ld, (int)N, K, O, out_mode, (int)row_tiles, (int)tiles, unit);
     return jl_check_launch("linear_mid_kernel");
 }
 extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t O, const void *bias, void *out, int64_t out_ld, int32_t out_mode,
@@ -419,6 +444,24 @@ extern "C" int jl_linear_mid(const void *x, int dtype, int64_t N, int64_t x_ld, 
     case 2: return linear_mid_launch<128, 128, 2, 4, 4>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
     }
     return linear_mid_launch<128, 128, 2, 2, 2>(xp, N, x_ld, wp, K, O, bp, out, out_ld, out_mode, st);
+}
+extern "C" int jl_linear_mid_gated(const void *x, int dtype, int64_t N, int64_t x_ld, const void *w, int32_t K, int32_t F, int32_t kind, float limit, float alpha, float shift, void *out, int64_t out_ld,
+                                   void *stream) {
+    if (N <= 0 || F <= 0) return JL_OK;
+    if (!x || !w || !out || K <= 0 || x_ld < K || out_ld < F || F > INT32_MAX / 2 || kind < JL_ACT_GELU_TANH || kind > JL_ACT_GELU_ERF)
+        return jl_fail(JL_E_INVALID, "jl_linear_mid_gated: null pointer, bad sizes or kind");
+    if (dtype != JL_BF16 || K % 8 || x_ld % 8 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15))
+        return jl_fail(JL_E_INVALID, "jl_linear_mid_gated: bfloat16, rows of x and W and the result at 16-byte borders");
+    if (N > INT32_MAX / 64 || N * x_ld * 2 > UINT32_MAX || (int64_t)F * K * 4 > UINT32_MAX) return jl_fail(JL_E_INVALID, "jl_linear_mid_gated: operands of up to 4 GB");
+    const bf16_t *xp = (const bf16_t *)x, *wp = (const bf16_t *)w;
+    const LinearUnit unit = {kind, limit, alpha, shift};
+    hipStream_t st = (hipStream_t)stream;
+    switch (linear_mid_tiles(N, 2 * (int64_t)F)) {
+    case 0: return linear_mid_launch<64, 64, 2, 2, 4, true>(xp, N, x_ld, wp, K, F, nullptr, out, out_ld, JL_LINEAR_SAME, st, unit);
+    case 1: return linear_mid_launch<64, 128, 2, 4, 3, true>(xp, N, x_ld, wp, K, F, nullptr, out, out_ld, JL_LINEAR_SAME, st, unit);
+    case 2: return linear_mid_launch<128, 128, 2, 4, 4, true>(xp, N, x_ld, wp, K, F, nullptr, out, out_ld, JL_LINEAR_SAME, st, unit);
+    }
+    return linear_mid_launch<128, 128, 2, 2, 2, true>(xp, N, x_ld, wp, K, F, nullptr, out, out_ld, JL_LINEAR_SAME, st, unit);
 }
 
 // ---- float products of many rows: TM of x by 128 of W per workgroup, on the bfloat16 matrix instructions in three terms per operand (jl_split.h) -----

@@ -259,7 +259,7 @@ class BamanexModel:
         f, w = self.cfg.layers[li]["mlp"], self.w.layers[li]
         if f.get("kind", "dense") == "dense":
             ff = int(f["ff"])
-            return [(LO.act_linear(LO.linear(h, w["w_gu"]), 0, ff, ff, LO.ACT_GELU_TANH, w["w_down"]), w["ls2"])]
+            return [(LO.feed_forward(h, w["w_gu"], LO.ACT_GELU_TANH, w["w_down"]), w["ls2"])]
         unit = lambda c: (LO.ACT_CLAMPED_SWISH, float(c["limit"]), SWISH_ALPHA, UNIT_SHIFT)
         out = [(LO.moe_experts(h, None, None, int(f["router"]["top"]), 1.0, w["w_gu"], w["w_down"], route="softmax_renorm", renorm_eps=ROUTER_RENORM_EPS, gated=unit(f["expert"]),
                                router=(h_float if h_float is not None else h, w["router"], None)), w["ls2"])]

@@ -254,7 +254,7 @@ class Qwen2Model:
 
     # -- pieces -----------------------------------------------------------------------------
     def _norm(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        return F.rms_norm(x, (x.shape[-1],), w, self.cfg.rms_norm_eps)
+        return LO.rms_norm(x, w, self.cfg.rms_norm_eps)
 
     @staticmethod
     def _rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
@@ -267,7 +267,8 @@ class Qwen2Model:
         """x += down(silu(gate(h)) * up(h)) with the gate in one HIP launch and the residual in the GEMM epilogue (in place:
         an out-of-place addmm first copies x into its result, one more launch per GEMM)."""
         if x2d.is_cuda and x2d.dtype == torch.bfloat16:
-            return LO.linear_add_(x2d, ops.swiglu(LO.linear(h2d, L["wgu"])), L["wd"])
+            a = LO.linear_gated(h2d, L["wgu"], LO.ACT_SILU)
+            return LO.linear_add_(x2d, ops.swiglu(LO.linear(h2d, L["wgu"])) if a is None else a, L["wd"])
         return x2d.addmm_(ops.swiglu(F.linear(h2d, L["wgu"])), L["wd"].t())
 
     # -- forward over a static cache -------------------------------------------------------------

@@ -263,7 +263,7 @@ class VoboraxModel:
         out = [(y, None)]
         if f.get("shared") is not None:
             fs = int(f["shared"]["ff"])
-            out.append((LO.act_linear(LO.linear(h, w["w_sh"]), 0, fs, fs, LO.ACT_SILU, w["w_sh_down"]), None))
+            out.append((LO.feed_forward(h, w["w_sh"], LO.ACT_SILU, w["w_sh_down"]), None))
         return out, choices
 
     # ---- one step ----------------------------------------------------------------------------------------------------------------------

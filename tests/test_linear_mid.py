@@ -46,6 +46,20 @@ def test_products_onto_what_is_there(n, k, o):
     assert (got.double() - want).abs().max() <= (2.0 ** -8 + 2.0 ** -20) * want.abs().max()
 
 
+# the same tiles with a unit in the epilogue: gates and linear branches of fewer columns than a tile's half, beside fours, and of every tile size
+@pytest.mark.parametrize("n,k,f", [(65, 8, 32), (70, 64, 36), (1000, 72, 501), (1025, 192, 512), (130, 264, 4100), (2047, 320, 508), (600, 1024, 2562), (2300, 136, 1300), (2048, 1024, 2048)])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+def test_units(n, k, f, kind):
+    from jacobiforcing_amd import layer_ops as LO
+    x, w, _, _ = _operands(n, k, 2 * f, k + 8, n + k + f)
+    got = LO.linear_gated(x, w, kind, 1.5, 1.25, 0.5)
+    z = (x.double() @ w.double().t()).float()
+    want = LO.gated_act(z, 0, f, f, kind, 1.5, 1.25, 0.5).double()     # the unit in 32 bits
+    assert got.shape == (n, f) and got.dtype == torch.bfloat16
+    # the sums as above, which a unit of slope up to two takes on; rounded once, 2 ** -9 of each at most
+    assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm() and (got.double() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+
+
 def test_which_calls_the_library_keeps(monkeypatch):
     """Sizes beyond the rule, autocast, other types, operands that share memory with the result: the library's product, as before."""
     from jacobiforcing_amd import _native as N
@@ -58,6 +72,7 @@ def test_which_calls_the_library_keeps(monkeypatch):
     with torch.autocast("cuda", dtype=torch.float16):
         assert H.linear(big, wide, None, None) is NotImplemented and LO.linear(big, wide).dtype == torch.float16
         assert H.linear_add(c, x, w) is NotImplemented
+    assert LO.linear_gated(x.half(), w.half(), 2) is None and LO.linear_gated(x, w[:1023], 2) is None and LO.linear_gated(x[:4], w, 2) is None
     assert H.linear_add(c, x.half(), w) is NotImplemented and H.linear_add(c[:, :512], x, w) is NotImplemented and H.linear_add(c, x, w[:, :256]) is NotImplemented
     square = torch.randn(64, 64, device="cuda").bfloat16()
     assert H.linear_add(square, square, square.clone()) is NotImplemented
