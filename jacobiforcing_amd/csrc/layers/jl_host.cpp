@@ -11,6 +11,7 @@
 #include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <algorithm>
@@ -200,11 +201,12 @@ CALL(linear_add, 3)
     NEED(n > 0 && k > 0 && o > 0 && o <= INT32_MAX && k <= INT32_MAX && p_jl_linear_mid_ok(n, k, o) && !at::autocast::is_autocast_enabled(at::kCUDA));
     NEED(w->size(1) == k && w->is_contiguous() && rows(*out, n, o) && out->is_contiguous() && x->stride(1) == 1 && ld >= k && k % 8 == 0 && ld % 8 == 0 && starts16(*x) && starts16(*w) && starts16(*out) &&
          w->device() == x->device() && out->device() == x->device() && n * ld * 2 < (int64_t)1 << 32 && !out->is_alias_of(*x) && !out->is_alias_of(*w));
-    NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad() || out->requires_grad())));
+    NEED(!(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad() || out->requires_grad())) && (!out->is_inference() || c10::InferenceMode::is_enabled()));
     NEED(!x->_fw_grad(0).defined() && !w->_fw_grad(0).defined() && !out->_fw_grad(0).defined());
     Unlocked others;
     RUN(jl_linear_mid, x->data_ptr(), JL_BF16, n, ld, w->data_ptr(), (int32_t)k, (int32_t)o, nullptr, out->data_ptr(), o, JL_LINEAR_ADD, stream_of(*x));
     others.back();
+    if (!out->is_inference()) out->unsafeGetTensorImpl()->bump_version();       // a graph that kept out for its backward is to see the change
     Py_RETURN_TRUE;
 END_CALL
 

@@ -78,3 +78,18 @@ def test_which_calls_the_library_keeps(monkeypatch):
     assert H.linear_add(square, square, square.clone()) is NotImplemented
     leaf = torch.randn(1024, 512, device="cuda").bfloat16().requires_grad_()
     assert H.linear_add(c, x, leaf) is NotImplemented
+
+
+def test_a_sum_in_place_is_seen():
+    """A result that a graph has kept, and one made under inference mode: as the library's product in place has it."""
+    from jacobiforcing_amd import layer_ops as LO
+    x, w, _, c = _operands(128, 64, 64, 64, 7)
+    leaf = torch.ones(128, 64, device="cuda").bfloat16().requires_grad_()
+    kept = (leaf * c).sum()
+    assert LO._host().linear_add(c, x, w) is not NotImplemented
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        kept.backward()
+    with torch.inference_mode():
+        made = torch.zeros(128, 64, device="cuda", dtype=torch.bfloat16)
+        assert LO._host().linear_add(made, x, w) is not NotImplemented
+    assert LO._host().linear_add(made, x, w) is NotImplemented
