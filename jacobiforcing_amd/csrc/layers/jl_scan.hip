@@ -8,7 +8,7 @@
 // The columns of S never interact, so a workgroup is ONE wavefront that owns 32 columns of one head's state (grid.y walks the head's
 // columns): two adjacent lanes per column, each with DMAX / 2 consecutive rows in registers.  Rows of S are read and written as 128
 // consecutive bytes.  Eight tokens at a time go through LDS; the next group's inputs travel while the current one is worked on.
-constexpr int SC_TT = 8, SC_COLS = 32;
+constexpr int SC_TT = 8, SC_COLS = 32, SC_TOKEN_COLS = 16, SC_TOKEN_HEADS = 2048;
 // silu in the activations' dtype: both forms of the recurrence see the same q, k and v, however a prompt is cut
 template <typename T> __device__ __forceinline__ float silu_as(float z) {
     T t;
@@ -101,7 +101,86 @@ __global__ __launch_bounds__(64) void scan_kernel(jl_scan_args a) {
             if (d0 + i < D) sp[(int64_t)(d0 + i) * Dv + j] = S[i];
 }
 
+// ---- a decoding step: one token for each request -----------------------------------------------------------------------------------------------
+// A token has nothing to walk: what the wavefronts above spend is two lanes' walk through half a column each, 64 dependent sums in a row behind 64 loads, in one wavefront per CU.  Here a workgroup takes
+// 16 columns, four per thread in one 16-byte access, and its 64 groups of four threads D / 64 rows each, all on their way at once; the column's sum goes through shuffles and LDS.
+// us a launch, wavefronts of two lanes a column / so (bfloat16, D and Dv 128 but as said): 1 request of 8 heads 10.0 / 4.2, 8 10.5 / 5.2, 32 of 16 heads 23.2 / 18.2, 48 32.9 / 28.9, of 64 x 64 11.4 / 10.8, 32 of 8 of 256 x 256 48.7 / 32.6.
+template <typename T, int R>
+__global__ __launch_bounds__(256) void scan_token_kernel(jl_scan_args a) {
+    __shared__ float part[4][16];
+    const int H = a.H, D = a.D, Dv = a.Dv;
+    const int b = blockIdx.x / H, h = blockIdx.x - b * H, kh = h / (H / a.G);
+    const int row0 = a.seq[4 * b], cnt = a.seq[4 * b + 1], pos0 = a.seq[4 * b + 2], slot = a.seq[4 * b + 3];
+    if (cnt <= 0) return;
+    const int tid = threadIdx.x, c = tid & 3, d0 = tid >> 2, j = (blockIdx.z * gridDim.y + blockIdx.y) * SC_TOKEN_COLS + 4 * c;
+    const bool live = j < Dv, fixed = a.decay != nullptr, act = a.act == JL_ACT_SILU;
+    float *sp = a.state + ((int64_t)slot * H + h) * D * Dv;
+    float S[R][4];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        S[i][0] = S[i][1] = S[i][2] = S[i][3] = 0.f;
+        if (live && d0 + 64 * i < D && pos0 > 0) ld4_f(sp + (int64_t)(d0 + 64 * i) * Dv + j, S[i]);
+    }
+    const float gamma = fixed ? a.decay[h] : 0.f, rate = fixed ? 0.f : -expf(a.A_log[h]), bias = fixed ? 0.f : a.dt_bias[h], skip = a.skip ? a.skip[h] : 0.f;
+    for (int t = 0; t < cnt; ++t) {                             // (a request of several tokens beside others of none)
+        const T *row = (const T *)a.src + (int64_t)(row0 + t) * a.ld, *qp = row + a.q_col + kh * D, *kp = row + a.k_col + kh * D, *vp = row + a.v_col + (int64_t)h * Dv + j;
+        float q[R], k[R], v[4], acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const bool in = d0 + 64 * i < D;
+            q[i] = in ? ld_f(qp + d0 + 64 * i) : 0.f;
+            k[i] = in ? ld_f(kp + d0 + 64 * i) : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = live ? ld_f(vp + e) : 0.f;
+        const float u = fixed ? 1.0f : softplus_f(ld_f((const T *)a.dt + (int64_t)(row0 + t) * a.dt_ld + a.dt_col + h) + bias), g = fixed ? gamma : expf(rate * u);
+        if (act) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) { q[i] = silu_as<T>(q[i]); k[i] = silu_as<T>(k[i]); }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = silu_as<T>(v[e]);
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (d0 + 64 * i < D)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    S[i][e] = g * S[i][e] + k[i] * (u * v[e]);
+                    acc[e] += S[i][e] * q[i];
+                }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int x = 4; x < 64; x *= 2) acc[e] += __shfl_xor(acc[e], x);
+        __syncthreads();                                        // the token before has been read
+        if ((tid & 63) < 4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[tid >> 6][4 * c + e] = acc[e];
+        __syncthreads();
+        if (tid < 4 && live) {
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (part[0][4 * c + e] + part[1][4 * c + e]) + (part[2][4 * c + e] + part[3][4 * c + e]) + skip * v[e];
+            st4_f(a.out + (int64_t)(row0 + t) * ((int64_t)H * Dv) + (int64_t)h * Dv + j, o);
+        }
+    }
+    if (live)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (d0 + 64 * i < D) st4_f(sp + (int64_t)(d0 + 64 * i) * Dv + j, S[i]);
+}
+
 template <typename T> static int scan_launch(const jl_scan_args &a, hipStream_t st) {
+    // no more tokens than requests: a token each (or none); rows of the state and of the result at 16-byte borders; and up to 2048 heads, since beyond that the wavefronts' 128 bytes of a row in one access
+    // read memory a little better than these 64 (200 requests of 16 heads of 128 x 128 133.4 / 135.5 us)
+    if (a.N > 0 && a.N <= a.B && (int64_t)a.B * a.H <= SC_TOKEN_HEADS && a.Dv % 4 == 0 && (((uintptr_t)a.state | (uintptr_t)a.out) & 15) == 0) {
+        const unsigned cols = (unsigned)((a.Dv + SC_TOKEN_COLS - 1) / SC_TOKEN_COLS), y = cols < 65535 ? cols : 65535;
+        const dim3 grid((unsigned)(a.B * a.H), y, (cols + y - 1) / y);
+        if (a.D <= 64) scan_token_kernel<T, 1><<<grid, 256, 0, st>>>(a);
+        else if (a.D <= 128) scan_token_kernel<T, 2><<<grid, 256, 0, st>>>(a);
+        else scan_token_kernel<T, 4><<<grid, 256, 0, st>>>(a);
+        return jl_check_launch("scan_token_kernel");
+    }
     const unsigned cols = (unsigned)((a.Dv + SC_COLS - 1) / SC_COLS), y = cols < 65535 ? cols : 65535;      // (a launch's second dimension ends there)
     const dim3 grid((unsigned)(a.B * a.H), y, (cols + y - 1) / y);
     if (a.D <= 32) scan_kernel<T, 32><<<grid, 64, 0, st>>>(a);
