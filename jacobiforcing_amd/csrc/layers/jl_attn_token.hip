@@ -1,6 +1,6 @@
 // jl_attn_token.hip — attention of single tokens and of portions of a few: every wavefront has keys of its own, the eight of a workgroup meet once, at the end.
-// Rows of the products are (query, head) pairs, up to 16 (NB = 1) or 32: the heads of one key head, or with mixed heads all of them (queries are zero where the key head is not theirs, so that one
-// accumulator takes every key head's scores and every key and value is read once for up to two value heads).  A wavefront walks every eighth tile of 16 or 32 keys: a key's units go from memory
+// Rows of the products are (query, head) pairs, up to 16 (NB = 1) or 32: the heads of one key head, or with mixed heads all of them (a row takes its scores from its own key head's product, so that
+// every key and value is read once for up to two value heads and a key that is not finite stays with its own heads).  A wavefront walks every eighth tile of 16 or 32 keys: a key's units go from memory
 // straight into the lanes that hold the operand of S^T = K Q^T, values through LDS of the wavefront's own, from where they are read turned (ds_read_b64_tr_b16) for O^T = V^T P^T; a lane holds
 // values of ONE row, so that only the maximum is exchanged, with three other lanes.  The next tile's loads leave before this one's weights are formed, and no wavefront waits for another before
 // the end, where all scale their sums to the row's maximum and add them up through LDS.
@@ -21,7 +21,7 @@ template <int U> __device__ __forceinline__ int tk_swap(int k) { return U % 16 =
 
 // Z: sixteens of keys per tile; KX: 32 depths of a key at most; VY: sixteens of value columns at most; NG: key heads (mixed heads; else 1); GV: value heads collected; VIK: values are the keys' first columns
 template <int NB, int Z, int KX, int VY, int NG, int GV, bool VIK, bool MIX> struct TkSizes {
-    static constexpr int U = 2 * VY, OWN = GV * Z * 16 * U, SLOT = GV * NB * VY * 64, QU = NB * KX * NG > 8 ? NB * KX * NG * 64 : 0;      // 16-byte units: a wavefront's values, its sums, the queries
+    static constexpr int U = 2 * VY, OWN = GV * Z * 16 * U, SLOT = GV * NB * VY * 64, QU = NB * KX > 8 ? NB * KX * 64 : 0;      // 16-byte units: a wavefront's values, its sums, the queries
     static constexpr int BODY = TK_NW * OWN > TK_NW / 2 * SLOT ? TK_NW * OWN : TK_NW / 2 * SLOT;
     static constexpr size_t BYTES = (size_t)(BODY + QU) * 16 + TK_NW * NB * 16 * 8;
 };
@@ -64,21 +64,24 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
         ok[nb] = ii[nb] < a.longest && ii[nb] < cnt;
         q_lo[nb] = lowest(i0 + ii[nb]);
     }
-    auto q_unit = [&](int nb, int c, int x) {
+    auto q_unit = [&](int nb, int x) {
         uint4 w = make_uint4(0, 0, 0, 0);
-        if (ok[nb] && (NG == 1 || h[nb] / rep == c) && 8 * (4 * x + quad) < D) w = *(const uint4 *)((const bf16_t *)a.q + ((int64_t)(row0 + ii[nb]) * H + h[nb]) * D + 8 * (4 * x + quad));
+        if (ok[nb] && 8 * (4 * x + quad) < D) w = *(const uint4 *)((const bf16_t *)a.q + ((int64_t)(row0 + ii[nb]) * H + h[nb]) * D + 8 * (4 * x + quad));
         return w;
     };
-    uint4 qf[Sizes::QU ? 1 : NB * NG * KX];
+    uint4 qf[Sizes::QU ? 1 : NB * KX];
     if constexpr (Sizes::QU == 0) {
 #pragma unroll
-        for (int e = 0; e < NB * NG * KX; ++e) qf[e] = q_unit(e / (NG * KX), e / KX % NG, e % KX);
+        for (int e = 0; e < NB * KX; ++e) qf[e] = q_unit(e / KX, e % KX);
     } else {
-        for (int e = wave; e < NG * KX; e += TK_NW)
+        for (int x = wave; x < KX; x += TK_NW)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) qS[(nb * NG * KX + e) * 64 + lane] = q_unit(nb, e / KX, e % KX);
+            for (int nb = 0; nb < NB; ++nb) qS[(nb * KX + x) * 64 + lane] = q_unit(nb, x);
         __syncthreads();
     }
+    int key_head[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) key_head[nb] = NG == 1 ? 0 : h[nb] / rep;
     const float c2 = a.scale * LOG2E;                               // scores are kept times log2(e): weights are 2 ** (s - max)
     float m_run[NB], l_run[NB];
     tk_f32x4 acc[GV][NB][VY];
@@ -171,19 +174,27 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
         }
         tk_f32x4 sc[NB][Z];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+        for (int c = 0; c < NG; ++c) {
+            tk_f32x4 of[NB][Z];
 #pragma unroll
-            for (int z = 0; z < Z; ++z) sc[nb][z] = (tk_f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int c = 0; c < NG; ++c)
+                for (int z = 0; z < Z; ++z) of[nb][z] = (tk_f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int x = 0; x < KX; ++x)
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
-                    const ar_bf16x8 q = __builtin_bit_cast(ar_bf16x8, Sizes::QU ? qS[((nb * NG + c) * KX + x) * 64 + lane] : qf[Sizes::QU ? 0 : (nb * NG + c) * KX + x]);
+                    const ar_bf16x8 q = __builtin_bit_cast(ar_bf16x8, Sizes::QU ? qS[(nb * KX + x) * 64 + lane] : qf[Sizes::QU ? 0 : nb * KX + x]);
 #pragma unroll
-                    for (int z = 0; z < Z; ++z) sc[nb][z] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ar_bf16x8, kr[c][z][x]), q, sc[nb][z], 0, 0, 0);
+                    for (int z = 0; z < Z; ++z) of[nb][z] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ar_bf16x8, kr[c][z][x]), q, of[nb][z], 0, 0, 0);
                 }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int z = 0; z < Z; ++z)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sc[nb][z][r] = c == 0 || key_head[nb] == c ? of[nb][z][r] : sc[nb][z][r];
+        }
         // the next tile's rows travel from here on
         if (t + TK_NW < t_hi) {
             load();

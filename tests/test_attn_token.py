@@ -90,3 +90,30 @@ def test_a_request_without_tokens_beside_others():
     for run in (lambda b: LO.attn_sweep(q, kp, vp, b, H, G, D, D, 0.1, 0), lambda b: LO.attn_sweep(ql, pool, pool[:, :128], b, H, 1, 160, 128, 0.1, 0)):
         a, b = run(step).double(), run(alone).double()
         assert (a - b).norm() <= 2 * 2.0 ** -8 * b.norm()            # tiles of as many queries, other shares of the keys
+
+
+@pytest.mark.parametrize("counts,starts", [([1, 2, 1], [5, 40, 900]), ([70], [0])])
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (4, 4, 64), (8, 4, 96), (6, 1, 40)])
+@pytest.mark.parametrize("head", [0, -1])
+def test_mixed_heads_with_a_key_that_one_head_never_takes(counts, starts, H, G, D, head):
+    """A key whose scores are minus infinity under one key head weighs nothing there and is any other key under the others, in this form as in that of long portions."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(H * D + G)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch, pages, tokens = _step(counts, starts, 16)
+    n, rep, c0 = sum(counts), H // G, head % G
+    kp, vp, q, talk = rnd(tokens, G * D).bfloat16(), rnd(tokens, G * D).bfloat16(), rnd(n, H * D).bfloat16(), torch.eye(H, device="cuda") + 0.3 * rnd(H, H)
+    q.view(n, H, D)[:, c0 * rep:(c0 + 1) * rep, 2] = q.view(n, H, D)[:, c0 * rep:(c0 + 1) * rep, 2].abs() + 0.5
+    for own in pages:
+        kp[own[0] * 16 + 3, c0 * D + 2] = float("-inf")
+    out, r0 = LO.attn_window(q, None, kp, vp, batch, H, G, D, D, D ** -0.5, 0, 0, None, None, talk, float_out=True), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // 16] * 16 + j % 16 for j in range(c + s)], device="cuda")
+        k, v = kp[tok].double().view(-1, G, D).repeat_interleave(rep, 1), vp[tok].double().view(-1, G, D).repeat_interleave(rep, 1)
+        i, j = torch.arange(s, s + c, device="cuda").view(-1, 1), torch.arange(c + s, device="cuda").view(1, -1)
+        p, v = _exact(q[r0:r0 + c].double().view(c, H, D), k, v, D ** -0.5, j <= i)
+        want = (torch.einsum("yx,xij->yij", talk.double(), p).contiguous() @ v).permute(1, 0, 2)
+        got = out[r0:r0 + c].double().view(c, H, D)
+        # as in test_mixed_heads
+        assert bool(want.isfinite().all()) and (got - want).norm() <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24) * want.norm(), b
+        r0 += c
