@@ -13,6 +13,9 @@
 
 constexpr int TK_NW = 8;
 
+// of a score (a sink, a share's maximum) less the row's maximum.  Scores stay as they are: times log2(e) the last third of the largest binade would be infinite
+__device__ __forceinline__ float tk_exp(float d) { return __builtin_amdgcn_exp2f(d * 1.44269504088896341f); }
+
 typedef float tk_f32x4 __attribute__((ext_vector_type(4)));
 typedef float tk_f32x8 __attribute__((ext_vector_type(8)));
 
@@ -30,7 +33,6 @@ template <int NB, int Z, int KX, int VY, int NG, int GV, bool VIK, bool MIX>
 __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args a, int rep, int tile0) {
     typedef TkSizes<NB, Z, KX, VY, NG, GV, VIK, MIX> Sizes;
     constexpr int KT = 16 * Z, U = Sizes::U, VX = VY / 2, OWN = Sizes::OWN, SLOT = Sizes::SLOT;
-    constexpr float LOG2E = 1.44269504088896341f;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int H = a.H, D = a.D, Dv = a.Dv, S = a.splits;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
@@ -82,7 +84,6 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
     int key_head[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) key_head[nb] = NG == 1 ? 0 : h[nb] / rep;
-    const float c2 = a.scale * LOG2E;                               // scores are kept times log2(e): weights are 2 ** (s - max)
     float m_run[NB], l_run[NB];
     tk_f32x4 acc[GV][NB][VY];
 #pragma unroll
@@ -205,30 +206,39 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
         for (int nb = 0; nb < NB; ++nb) {
             const int qi = i0 + ii[nb], first = ok[nb] ? q_lo[nb] - j0 : KT, last = qi - j0 < nk - 1 ? qi - j0 : nk - 1, keep = ok[nb] ? keep_first - j0 : 0;
             float mx = -INFINITY;
+            if (!MIX && a.softcap > 0.f) {
+#pragma unroll
+                for (int z = 0; z < Z; ++z)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sc[nb][z][r] = soft_cap_fast(sc[nb][z][r] * a.scale, a.softcap);
+            } else if (MIX && a.rel) {
+#pragma unroll
+                for (int z = 0; z < Z; ++z)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sc[nb][z][r] = fmaf(sc[nb][z][r], a.scale, bias[MIX ? 4 * z + r : 0]);
+            } else {
+#pragma unroll
+                for (int z = 0; z < Z; ++z) sc[nb][z] *= a.scale;
+            }
 #pragma unroll
             for (int z = 0; z < Z; ++z)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int kk = 16 * z + 4 * quad + r;
                     float s = sc[nb][z][r];
-                    if (!MIX && a.softcap > 0.f) s = soft_cap_fast(s * a.scale, a.softcap) * LOG2E;
-                    else if (MIX && a.rel) {                        // a finite bias stays finite times log2(e)
-                        const float raw = bias[MIX ? 4 * z + r : 0], v = raw * LOG2E;
-                        s = fmaf(s, c2, __builtin_isinf(v) && !__builtin_isinf(raw) ? __builtin_copysignf(__FLT_MAX__, v) : v);
-                    } else s *= c2;
                     s = (kk >= first || kk < keep) && kk <= last ? s : -INFINITY;
                     sc[nb][z][r] = s;
                     mx = fmaxf(mx, s);
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run[nb], mx), m_sub = m_new > -INFINITY ? m_new : 0.f;      // a row that has seen no key yet: all weights are 2 ** -inf
-            const float alpha = __builtin_amdgcn_exp2f(m_run[nb] - m_sub);
+            const float m_new = fmaxf(m_run[nb], mx), m_sub = m_new > -INFINITY ? m_new : 0.f;      // a row that has seen no key yet: all weights are zero
+            const float alpha = tk_exp(m_run[nb] - m_sub);
             float sum = 0.f;
 #pragma unroll
             for (int z = 0; z < Z; ++z)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) { sc[nb][z][r] = __builtin_amdgcn_exp2f(sc[nb][z][r] - m_sub); sum += sc[nb][z][r]; }
+                for (int r = 0; r < 4; ++r) { sc[nb][z][r] = tk_exp(sc[nb][z][r] - m_sub); sum += sc[nb][z][r]; }
             l_run[nb] = l_run[nb] * alpha + sum;
             m_run[nb] = m_new;
             if (__any(alpha != 1.0f)) {
@@ -299,15 +309,16 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
     for (int nb = 0; nb < NB; ++nb) {
         M[nb] = -INFINITY;
         L[nb] = 0.f;
+        float f = 0.f;                                              // of this wavefront's sums
 #pragma unroll
         for (int w = 0; w < TK_NW; ++w) M[nb] = fmaxf(M[nb], mS[(w * NB + nb) * 16 + l16]);
 #pragma unroll
         for (int w = 0; w < TK_NW; ++w) {                           // a sum that is not a number stays one
-            const float m = mS[(w * NB + nb) * 16 + l16];
-            L[nb] += lS[(w * NB + nb) * 16 + l16] * (m > -INFINITY ? __builtin_amdgcn_exp2f(m - M[nb]) : 0.f);
+            const float m = mS[(w * NB + nb) * 16 + l16], e = m > -INFINITY ? tk_exp(m - M[nb]) : 0.f;
+            L[nb] += lS[(w * NB + nb) * 16 + l16] * e;
+            f = w == wave ? e : f;
         }
         const bool any = m_run[nb] > -INFINITY;
-        const float f = any ? __builtin_amdgcn_exp2f(m_run[nb] - M[nb]) : 0.f;
 #pragma unroll
         for (int g = 0; g < GV; ++g)
 #pragma unroll
@@ -345,8 +356,8 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
         const int64_t row = ((int64_t)ti * a.TQ + ii[nb]) * S + split, n = row0 + ii[nb];      // shares: [tile, query][split][head][value head][Dv], maxima and sums [..][head][2] behind all of them
         float inv = 0.f;
         if (whole) {                                                // what the joining launch does with one share
-            const float sink = a.sink ? a.sink[h[nb]] * LOG2E : -INFINITY, Ms = fmaxf(sink, M[nb]), w = M[nb] > -INFINITY ? __builtin_amdgcn_exp2f(M[nb] - Ms) : 0.f;
-            const float Ls = (a.sink ? __builtin_amdgcn_exp2f(sink - Ms) : 0.f) + w * L[nb];
+            const float sink = a.sink ? a.sink[h[nb]] : -INFINITY, Ms = fmaxf(sink, M[nb]), w = M[nb] > -INFINITY ? tk_exp(M[nb] - Ms) : 0.f;
+            const float Ls = (a.sink ? tk_exp(sink - Ms) : 0.f) + w * L[nb];
             inv = Ls != 0.f ? w * (a.out_scale / Ls) : 0.f;         // a sum that is not a number reaches the outputs
         } else if (wave == 0 && quad == 0 && (!MIX || side == 0)) {
             float *ml = a.scratch + (int64_t)a.n_tiles * a.TQ * S * H * GW * Dv + (row * H + h[nb]) * 2;
@@ -376,7 +387,7 @@ __global__ __launch_bounds__(64 * TK_NW, 2) void attn_token_kernel(jl_attn_args 
     }
 }
 
-// Mixed heads: w[split][head] = 2 ** (m - M) / L (not a number where L is none or zero, as the softmax of such scores), out_h = sum over heads x of talk[h, x] sum over splits of w O_(x, g(h)), gated.  A
+// Mixed heads: w[split][head] = exp(m - M) / L (not a number where L is none or zero, as the softmax of such scores), out_h = sum over heads x of talk[h, x] sum over splits of w O_(x, g(h)), gated.  A
 // workgroup has 32 columns of a token's value head: its chain of loads is as long as for all of them, and a token's are on as many CUs.
 constexpr int TK_HEADS = 16, TK_SPLITS = 64;
 __global__ __launch_bounds__(128) void attn_token_mix_kernel(jl_attn_args a, int chunks) {
@@ -399,7 +410,7 @@ __global__ __launch_bounds__(128) void attn_token_mix_kernel(jl_attn_args a, int
 #pragma unroll
         for (int off = 4; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 8));
         for (int s = j; s < S; s += 8) {
-            const float m = ml[(s * H + x) * 2], e = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+            const float m = ml[(s * H + x) * 2], e = m > -INFINITY ? tk_exp(m - M) : 0.f;
             w[s][x] = e;
             L += ml[(s * H + x) * 2 + 1] * e;
         }
@@ -440,7 +451,7 @@ __global__ __launch_bounds__(128) void attn_token_mix_kernel(jl_attn_args a, int
     else st4_f((bf16_t *)a.out + n * a.out_ld + to, v);
 }
 
-// Shares of the keys added up: out = sum over shares of 2 ** (m - M) O / L, the sink as one more share that holds nothing, times the gate.  `per` lanes (a power of two) have a (query, head) row, four columns each
+// Shares of the keys added up: out = sum over shares of exp(m - M) O / L, the sink as one more share that holds nothing, times the gate.  `per` lanes (a power of two) have a (query, head) row, four columns each
 __global__ __launch_bounds__(256) void attn_token_join_kernel(jl_attn_args a, int per, int rows) {
     const int r = blockIdx.x * (256 / per) + threadIdx.x / per, lane = threadIdx.x % per;
     if (r >= rows) return;
@@ -460,16 +471,15 @@ __global__ __launch_bounds__(256) void attn_token_join_kernel(jl_attn_args a, in
         }
     };
     fetch(0);
-    constexpr float LOG2E = 1.44269504088896341f;
-    const float sink = a.sink ? a.sink[h] * LOG2E : -INFINITY;
+    const float sink = a.sink ? a.sink[h] : -INFINITY;
     float M = sink;
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s) M = fmaxf(M, st[s].x);
 #pragma unroll 8
     for (int s = AHEAD; s < S; ++s) M = fmaxf(M, ml[s * H * 2]);
-    float L = a.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
+    float L = a.sink ? tk_exp(sink - M) : 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
     auto add = [&](float2 stat, float4 o) {
-        const float w = stat.x > -INFINITY ? __builtin_amdgcn_exp2f(stat.x - M) : 0.f;
+        const float w = stat.x > -INFINITY ? tk_exp(stat.x - M) : 0.f;
         L = fmaf(w, stat.y, L);                                     // an empty share (m = -inf) holds zeros, or a sum that is not a number
         v[0] = fmaf(w, o.x, v[0]); v[1] = fmaf(w, o.y, v[1]); v[2] = fmaf(w, o.z, v[2]); v[3] = fmaf(w, o.w, v[3]);
     };

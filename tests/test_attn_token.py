@@ -117,3 +117,29 @@ def test_mixed_heads_with_a_key_that_one_head_never_takes(counts, starts, H, G, 
         # as in test_mixed_heads
         assert bool(want.isfinite().all()) and (got - want).norm() <= 8 * (2.0 ** -17 + 16 * 2.0 ** -24) * want.norm(), b
         r0 += c
+
+
+@pytest.mark.parametrize("what", ["scores", "scale", "sink"])
+@pytest.mark.parametrize("H,R,grouped", [(8, 128, False), (4, 512, False), (6, 64, True)])
+@pytest.mark.parametrize("counts,starts", [([2, 1], [9, 40]), ([1, 1], [1000, 700])])
+def test_scores_scales_and_sinks_to_the_end_of_the_floats(what, H, R, grouped, counts, starts):
+    """Finite scores, scales and sinks of the largest binade, which tie or lie so far apart that only the largest weigh anything: keys whole and shared out."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch, pages, tokens = _step(counts, starts, 64)
+    n, up, scale = sum(counts), *((-60, 3e38) if what == "scale" else (63, 1.0))
+    k, q, sinks = rnd(tokens, R).bfloat16(), torch.zeros(n, H * R, device="cuda").bfloat16(), torch.full((H,), 3e38, device="cuda") if what == "sink" else None
+    v = rnd(tokens, R).bfloat16() if grouped else k
+    q.view(n, H, R)[..., 0] = 2.0 ** up
+    k[:, 0] = torch.tensor([1.0, 1.25, 1.5, 1.75], device="cuda")[torch.arange(tokens, device="cuda") % 4] * 2.0 ** (up if what == "scale" else 64)      # the sink lies between the last two
+    out, r0 = LO.attn_sweep(q, k, v if grouped else k[:, :R], batch, H, 1, R, R, scale, 0, sink=sinks, float_out=True), 0
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // 64] * 64 + j % 64 for j in range(c + s)], device="cuda")
+        kk, vv = (x[tok].double()[:, None].expand(-1, H, -1) for x in (k, v))
+        i, j = torch.arange(s, s + c, device="cuda").view(-1, 1), torch.arange(c + s, device="cuda").view(1, -1)
+        p, vv = _exact(q[r0:r0 + c].double().view(c, H, R), kk, vv, float(torch.tensor(scale)), j <= i, sinks)
+        want, got = (p @ vv).permute(1, 0, 2)[..., 1:], out[r0:r0 + c].double().view(c, H, R)[..., 1:]
+        # weights are rounded to bfloat16; scores of a scale of 3e38 lie around 300, a few 2 ** -24 of which move a weight by less
+        assert bool(got.isfinite().all()) and (got - want).norm() <= 2 * 2.0 ** -8 * want.norm(), b
+        r0 += c
