@@ -157,12 +157,12 @@ bool rule_small(int64_t n, int64_t k, int64_t o, int64_t item) {
     return n > 0 && n <= small_rows && n * k * item * ((o + tile * 256 - 1) / (tile * 256)) <= x_bytes;
 }
 
-// x, w, bias, float_out
 // where the launch is taken under autocast as well (2), or where that has nothing to see
 bool mid_taken(int64_t n, int64_t k, int64_t o) {
     const int ok = p_jl_linear_mid_ok(n, k, o);
     return ok == 2 || (ok && !at::autocast::is_autocast_enabled(at::kCUDA));
 }
+// x, w, bias, float_out
 CALL(linear, 4)
     const Tensor *x, *w, *bias;
     bool as_float = false;
@@ -773,7 +773,7 @@ CALL(step_tables, 6)
          take(arg[5], from));
     const int64_t B = (int64_t)counts.size(), listed = PySequence_Fast_GET_SIZE(arg[3]);
     NEED(B > 0 && (int64_t)starts.size() == B && (int64_t)slots.size() == B && listed >= B);
-    int64_t C = 1, N = 0, longest = 0, least = INT64_MAX, max_pos = 0, max_slot = slots[0], in_tables = 0;
+    int64_t C = 1, N = 0, longest = 0, least = INT64_MAX, max_pos = 0, max_slot = slots[0];
     held.resize(listed);
     for (int64_t b = 0; b < listed; ++b) {
         PyObject *t = PySequence_Fast_GET_ITEM(arg[3], b);
@@ -783,7 +783,6 @@ CALL(step_tables, 6)
         if (b >= B) continue;                                       // tables of more requests count in the width alone
         NEED(counts[b] >= 0 && starts[b] >= 0 && (!counts[b] || (starts[b] + counts[b] + page - 1) / page <= held[b]));
         N += counts[b];
-        in_tables += held[b];
         longest = std::max(longest, counts[b]);
         least = std::min(least, counts[b]);
         max_pos = std::max(max_pos, starts[b] + counts[b]);
