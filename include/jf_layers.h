@@ -216,7 +216,8 @@ JL_API int jl_linear_small(const void *x, int dtype, int64_t N, int64_t x_ld, co
  *   JL_AFTER_NORM:       jl_sandwich_norm of x [N, K] float (plus y [N, K] of y_dtype, normed by w_post, when given, plus add_row) with w_next; the updated x goes into x_out, which is another buffer
  *   JL_AFTER_ACT:        jl_gated_act of x (rows x_ld apart of bfloat16, g_col, u_col, K columns; kind, limit, alpha, shift)
  *   JL_AFTER_GATED_NORM: jl_gated_norm of x [N, K] float in one part, y its bfloat16 gate (rows y_ld apart), w_next the norm's weight (kind, gate_first, scale)
- * rounded to bfloat16, times w [O, K] transposed (+ bias [O], both bfloat16), into out bfloat16 [N, O].  N * K up to JL_AFTER_VALUES, K a multiple of 8, everything at 16-byte borders. */
+ * rounded to bfloat16, times w [O, K] transposed (+ bias [O], both bfloat16), into out bfloat16 [N, O].  N * K up to JL_AFTER_VALUES (three rows count as four), K a multiple of 8; x, w and the float operands at 16-byte borders, a bfloat16 y
+ * at one of 8, rows, columns g_col and u_col of bfloat16 operands in multiples of 4, bias and out at any. */
 #define JL_AFTER_NORM 0
 #define JL_AFTER_ACT 1
 #define JL_AFTER_GATED_NORM 2

@@ -59,14 +59,33 @@ static void linear_small_launch(const void *x, int64_t x_ld, const void *w, cons
 
 // ---- one row (or a few) that every workgroup makes for itself ------------------------------------------------------------------------------
 // A token alone waits for launches: a norm, an activation or a gate in front of a product takes a launch of 4 us of the GPU and 5 of the host for a few KB.  Here each workgroup of 16 rows of W makes the
-// product's operand itself, in LDS: what the row is made of leaves memory first, this wavefront's weights right behind it, and the operand is made while they travel.  The sums are those of
-// linear_small_kernel.  us of the GPU, one row of 1024 by 1024 to 4096, the launch and the product / so: norm 4.1 + 4.6 / 6.3, unit 4.0 + 4.6 / 5.5, gated norm 4.0 + 4.3 / 5.3.  Every workgroup repeats
-// the row's work, which is why few rows go so, and why more than 512 workgroups (8192 columns) do not.
-template <int MODE, int VI>
+// product's operand itself, in LDS: what the rows are made of leaves memory first, this wavefront's weights right behind it, and the operand is made while they travel, all rows at once: their sums go
+// through two barriers together.  Up to JL_LINEAR_ONE_TILE rows of W the product's sums are those of linear_small_kernel.  us of the GPU, launch and product / so, one, two and four rows (by 1024 values and 4096):
+// norm 7.1 / 5.1, 7.2 / 5.7, 7.3 / 7.5 and 8.1 / 5.9, 7.9 / 6.6, 8.1 / 8.6; unit 6.3 / 3.6, 6.5 / 4.5, 6.7 / 5.9 and 7.2 / 4.5, 7.4 / 5.1, 7.7 / 6.5; gated norm 6.3 / 4.7, 6.5 / 5.2, 6.7 / 6.8 and
+// 7.2 / 5.5, 7.4 / 5.9, 7.5 / 7.9; and the two calls take the host 9.5 us, the one 5.  (Rows one behind the other, two barriers a sum: norm, 1024 by 1024, 5.6, 7.0 and 9.7.)  Every workgroup repeats the
+// rows' work: see jl_linear_after_ok.
+// sums of the rows' values over the workgroup's eight wavefronts, all rows at once: one barrier
+template <int R> __device__ __forceinline__ void la_sums(float (&v)[R], float (*red)[8], int wave, int lane) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] += __shfl_xor(v[r], off, 64);
+    if (lane == 0)
+#pragma unroll
+        for (int r = 0; r < R; ++r) red[r][wave] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        v[r] = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) v[r] += red[r][w];
+    }
+}
+template <int MODE, int VI, int R>                                  // R: rows, or one more than there are
 __global__ __launch_bounds__(512) void linear_after_kernel(jl_linear_after a) {
     constexpr int NW = 8, STEP = 64 * NW * 4;
     __shared__ ls_f32x4 part[NW][64];
-    __shared__ float red[16];
+    __shared__ float red[2][R][8];
     extern __shared__ __attribute__((aligned(16))) bf16_t xs[];     // [N][K]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g4 = lane >> 4, o0 = blockIdx.x * 16, K = a.K, O = a.O, N = a.N;
     const int steps = (K + 63) / 64, s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW, k_lane = 8 * g4;
@@ -81,77 +100,94 @@ __global__ __launch_bounds__(512) void linear_after_kernel(jl_linear_after a) {
                 wr[i][y] = s + i < s1 && k + k_lane < K ? *(const uint4 *)(wp + k) : make_uint4(0, 0, 0, 0);
             }
     };
-    for (int n = 0; n < N; ++n) {
-        float x[VI][4], y[VI][4], u[VI][4], v[VI][4], add[VI][4];
-        const bool with = MODE == JL_AFTER_NORM && a.y, row = MODE == JL_AFTER_NORM && a.add_row;
+    const bool with = MODE == JL_AFTER_NORM && a.y, row = MODE == JL_AFTER_NORM && a.add_row;
+    float x[R][VI][4], y[R][VI][4], post[VI][4], add[VI][4], next[VI][4];       // y: what is added, the gate, the linear branch
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+            const int c = i * STEP + 4 * tid, n = R == 1 || r < N ? r : N - 1;
+            if (c >= K) continue;
+            if (MODE == JL_AFTER_ACT) {
+                const bf16_t *z = (const bf16_t *)a.x + n * a.x_ld + c;
+                ld4_f(z + a.g_col, x[r][i]);
+                if (a.u_col >= 0) ld4_f(z + a.u_col, y[r][i]);
+            } else {
+                ld4_f((const float *)a.x + (int64_t)n * K + c, x[r][i]);
+                if (MODE == JL_AFTER_GATED_NORM) ld4_f((const bf16_t *)a.y + n * a.y_ld + c, y[r][i]);
+                else if (with) {
+                    if (a.y_dtype == JL_BF16) ld4_f((const bf16_t *)a.y + (int64_t)n * K + c, y[r][i]);
+                    else ld4_f((const float *)a.y + (int64_t)n * K + c, y[r][i]);
+                }
+            }
+        }
+    if (MODE != JL_AFTER_ACT)
 #pragma unroll
         for (int i = 0; i < VI; ++i) {
             const int c = i * STEP + 4 * tid;
             if (c >= K) continue;
-            if (MODE == JL_AFTER_ACT) {
-                const bf16_t *z = (const bf16_t *)a.x + n * a.x_ld;
-                ld4_f(z + a.g_col + c, x[i]);
-                if (a.u_col >= 0) ld4_f(z + a.u_col + c, u[i]);
-            } else {
-                ld4_f((const float *)a.x + (int64_t)n * K + c, x[i]);
-                if (MODE == JL_AFTER_GATED_NORM) ld4_f((const bf16_t *)a.y + n * a.y_ld + c, y[i]);
-                else if (with) {
-                    if (a.y_dtype == JL_BF16) ld4_f((const bf16_t *)a.y + (int64_t)n * K + c, y[i]);
-                    else ld4_f((const float *)a.y + (int64_t)n * K + c, y[i]);
-                    ld4_f(a.w_post + c, u[i]);
-                }
-                if (row) ld4_f(a.add_row + c, add[i]);
-                ld4_f(a.w_next + c, v[i]);
-            }
+            if (with) ld4_f(a.w_post + c, post[i]);
+            if (row) ld4_f(a.add_row + c, add[i]);
+            ld4_f(a.w_next + c, next[i]);
         }
-        if (n == 0) {
-            __builtin_amdgcn_sched_barrier(0);
-            load(s0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        float ss = 0.f, r = 1.f;
-        if (with) {
+    __builtin_amdgcn_sched_barrier(0);
+    load(s0);
+    __builtin_amdgcn_sched_barrier(0);
+    float ss[R], scale[R];
+    if (with) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ss[r] = 0.f;
 #pragma unroll
             for (int i = 0; i < VI; ++i)
-                if (i * STEP + 4 * tid < K) ss += y[i][0] * y[i][0] + y[i][1] * y[i][1] + y[i][2] * y[i][2] + y[i][3] * y[i][3];
-            ss = block_sum_f32(ss, red);
-            r = 1.0f / sqrtf(ss / (float)K + a.eps);
+                if (i * STEP + 4 * tid < K) ss[r] += y[r][i][0] * y[r][i][0] + y[r][i][1] * y[r][i][1] + y[r][i][2] * y[r][i][2] + y[r][i][3] * y[r][i][3];
+        }
+        la_sums<R>(ss, red[0], wave, lane);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float f = 1.0f / sqrtf(ss[r] / (float)K + a.eps);
 #pragma unroll
             for (int i = 0; i < VI; ++i)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[i][e] += y[i][e] * r * u[i][e];
+                for (int e = 0; e < 4; ++e) x[r][i][e] += y[r][i][e] * f * post[i][e];
         }
-        ss = 0.f;
-        if (MODE != JL_AFTER_ACT) {
+    }
+    if (MODE != JL_AFTER_ACT) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ss[r] = 0.f;
 #pragma unroll
             for (int i = 0; i < VI; ++i) {
                 if (i * STEP + 4 * tid >= K) continue;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    if (row) x[i][e] += add[i][e];
+                    if (row) x[r][i][e] += add[i][e];
                     if (MODE == JL_AFTER_GATED_NORM) {
-                        y[i][e] = gate_act_f(y[i][e], a.kind);
-                        if (a.gate_first) x[i][e] *= y[i][e];
+                        y[r][i][e] = gate_act_f(y[r][i][e], a.kind);
+                        if (a.gate_first) x[r][i][e] *= y[r][i][e];
                     }
                 }
-                if (MODE == JL_AFTER_NORM && blockIdx.x == 0) st4_f(a.x_out + (int64_t)n * K + i * STEP + 4 * tid, x[i]);
-                ss += x[i][0] * x[i][0] + x[i][1] * x[i][1] + x[i][2] * x[i][2] + x[i][3] * x[i][3];
+                if (MODE == JL_AFTER_NORM && blockIdx.x == 0 && (R == 1 || r < N)) st4_f(a.x_out + (int64_t)r * K + i * STEP + 4 * tid, x[r][i]);
+                ss[r] += x[r][i][0] * x[r][i][0] + x[r][i][1] * x[r][i][1] + x[r][i][2] * x[r][i][2] + x[r][i][3] * x[r][i][3];
             }
-            ss = block_sum_f32(ss, red);
-            r = (MODE == JL_AFTER_GATED_NORM ? a.scale : 1.0f) / sqrtf(ss / (float)K + a.eps);
         }
+        la_sums<R>(ss, red[1], wave, lane);
+#pragma unroll
+        for (int r = 0; r < R; ++r) scale[r] = (MODE == JL_AFTER_GATED_NORM ? a.scale : 1.0f) / sqrtf(ss[r] / (float)K + a.eps);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int i = 0; i < VI; ++i) {
             const int c = i * STEP + 4 * tid;
-            if (c >= K) continue;
+            if (c >= K || (R > 1 && r >= N)) continue;
             float to[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                to[e] = MODE == JL_AFTER_ACT ? gated_unit_f<true>(x[i][e], a.u_col >= 0 ? u[i][e] : 1.0f, a.kind, a.limit, a.alpha, a.shift)
-                        : MODE == JL_AFTER_NORM ? v[i][e] * (x[i][e] * r) : v[i][e] * (x[i][e] * r * (a.gate_first ? 1.0f : y[i][e]));
-            st4_f(xs + (int64_t)n * K + c, to);
+                to[e] = MODE == JL_AFTER_ACT ? gated_unit_f<true>(x[r][i][e], a.u_col >= 0 ? y[r][i][e] : 1.0f, a.kind, a.limit, a.alpha, a.shift)
+                        : MODE == JL_AFTER_NORM ? next[i][e] * (x[r][i][e] * scale[r]) : next[i][e] * (x[r][i][e] * scale[r] * (a.gate_first ? 1.0f : y[r][i][e]));
+            st4_f(xs + (int64_t)r * K + c, to);
         }
-    }
     __syncthreads();
     const bf16_t *xp = xs + (r16 < N ? r16 : N - 1) * K + k_lane;
     ls_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -178,8 +214,13 @@ __global__ __launch_bounds__(512) void linear_after_kernel(jl_linear_after a) {
         if (o + i < O) st_f(out + i, a.bias ? sum[i] + ld_f((const bf16_t *)a.bias + o + i) : sum[i]);
 }
 
+// One and two rows everywhere (us, launch and product / so: norm of one by 4096 values and 8192 23.3 / 18.6, of two 24.0 / 17.9, by 8192 and 8192 48.9 / 42.5; what loses there are units of two by 8192
+// values, 4096 18.9 / 21.3).  Three and four, whose time is that of four, where the host's part outweighs what 256 workgroups repeat: norm of four by 512 and 2048 6.6 / 7.1, by 2048 and 4096 11.6 / 11.0,
+// by 4096 and 1024 14.4 / 13.3, gated norm 13.0 / 14.0; beyond, by 1024 and 8192 10.2 / 11.0, by 4096 and 4096 gated norm 15.7 / 17.9, unit 13.4 / 15.4, and by 4096 and 8192, two workgroups a CU that
+// do not fit, norm 24.3 / 31.8, gated norm 22.3 / 32.8.
 extern "C" int jl_linear_after_ok(int64_t N, int64_t K, int64_t O) {
-    return N > 0 && N <= JL_AFTER_ROWS && K > 0 && K % 8 == 0 && K <= 8192 && N * K <= JL_AFTER_VALUES && O > 0 && O <= 8192;
+    if (N <= 0 || N > JL_AFTER_ROWS || K <= 0 || K % 8 || K > 8192 || (N > 2 ? 4 : N) * K > JL_AFTER_VALUES || O <= 0 || O > 8192) return 0;
+    return N <= 2 || (O <= 4096 && (K <= 2048 || O <= 1024));
 }
 extern "C" int jl_linear_after_run(const jl_linear_after *ap, void *stream) {
     if (!ap) return jl_fail(JL_E_INVALID, "jl_linear_after_run: null arguments");
@@ -195,16 +236,23 @@ extern "C" int jl_linear_after_run(const jl_linear_after *ap, void *stream) {
     const dim3 grid((unsigned)((a.O + 15) / 16));
     const int lds = a.N * a.K * 2;
     hipStream_t st = (hipStream_t)stream;
+#define LA_ROWS(M, VI)                                                                   \
+    do {                                                                                  \
+        if (a.N == 1) linear_after_kernel<M, VI, 1><<<grid, 512, lds, st>>>(a);            \
+        else if (a.N == 2) linear_after_kernel<M, VI, 2><<<grid, 512, lds, st>>>(a);       \
+        else if constexpr (VI <= 2) linear_after_kernel<M, VI, 4><<<grid, 512, lds, st>>>(a); \
+    } while (0)
 #define LA_MODE(M)                                                                       \
     do {                                                                                  \
-        if (a.K <= 2048) linear_after_kernel<M, 1><<<grid, 512, lds, st>>>(a);             \
-        else if (a.K <= 4096) linear_after_kernel<M, 2><<<grid, 512, lds, st>>>(a);        \
-        else linear_after_kernel<M, 4><<<grid, 512, lds, st>>>(a);                         \
+        if (a.K <= 2048) LA_ROWS(M, 1);                                                    \
+        else if (a.K <= 4096) LA_ROWS(M, 2);                                               \
+        else LA_ROWS(M, 4);                                                                \
     } while (0)
     if (a.mode == JL_AFTER_NORM) LA_MODE(JL_AFTER_NORM);
     else if (a.mode == JL_AFTER_ACT) LA_MODE(JL_AFTER_ACT);
     else LA_MODE(JL_AFTER_GATED_NORM);
 #undef LA_MODE
+#undef LA_ROWS
     return jl_check_launch("linear_after_kernel");
 }
 

@@ -85,3 +85,31 @@ def test_what_the_two_calls_keep():
     assert H.gated_norm_linear(one, gate.float(), v, 1e-5, N.JL_ACT_SILU, True, 1.0, w, None) is NotImplemented
     with pytest.raises(ValueError):
         LO.act_linear(gate, 60, -1, 8, LO.ACT_SILU, w[:, :8].contiguous())
+
+
+@pytest.mark.parametrize("k,o", [(64, 40), (1000, 33), (2048, 4096), (2056, 100), (4096, 1024)])
+@pytest.mark.parametrize("n", [2, 3, 4])
+def test_rows_are_what_they_are_alone(n, k, o):
+    """Rows made at once: each the row of a call of its own, to the last bit."""
+    from jacobiforcing_amd import _native as N, layer_ops as LO
+    rnd, H = _rnd(n + k + o), LO._host()
+    x, y, v, add, gate, z = rnd(n, k), rnd(n, k).bfloat16(), rnd(k), rnd(k), rnd(n, k).bfloat16(), rnd(n, 2 * k).bfloat16()
+    w, b = (rnd(o, k) * k ** -0.5).bfloat16(), rnd(o).bfloat16()
+    calls = (lambda i: H.norm_linear(x[i], y[i], v, 1e-5, add, add, w, b), lambda i: H.act_linear(z[i], 0, k, k, 1, 1.5, 1.25, 0.5, w, b), lambda i: H.gated_norm_linear(x[i], gate[i], v, 1e-5, N.JL_ACT_SIGMOID, False, 0.7, w, b))
+    for call in calls:
+        whole = call(slice(0, n))
+        assert whole is not NotImplemented
+        for r in range(n):
+            one = call(slice(r, r + 1))
+            for a, c in zip(whole if isinstance(whole, tuple) else (whole,), one if isinstance(one, tuple) else (one,)):
+                assert torch.equal(a[r], c[0]), r
+
+
+def test_where_two_launches_are_the_better_ones():
+    """Three rows and more of many columns, or deep ones of more than a few: every workgroup would repeat them."""
+    from jacobiforcing_amd import _native as N
+    ok = N.layers().jl_linear_after_ok
+    for n, k, o in ((1, 8192, 8192), (2, 8192, 8192), (3, 2048, 4096), (4, 2048, 4096), (3, 4096, 1024), (4, 4096, 1024), (4, 8, 4)):
+        assert ok(n, k, o) == 1, (n, k, o)
+    for n, k, o in ((1, 8200, 64), (2, 8192, 8193), (3, 2048, 4097), (4, 512, 4097), (3, 2056, 1025), (4, 4096, 4096), (3, 4104, 16), (5, 8, 4), (0, 8, 4), (2, 12, 4)):
+        assert ok(n, k, o) == 0, (n, k, o)
