@@ -455,13 +455,15 @@ static int linear_mid_tiles(int64_t N, int64_t O) {
     return tiles(64, 64) <= 256 ? 0 : tiles(64, 128) <= 256 ? 1 : tiles(128, 128) <= 256 ? 2 : 3;
 }
 
-// 1: where the launch is the better one; 2: there, and it was so for products that autocast does not see (layer_ops.linear_mid has the figures).
+// 1: where the launch is the better one; 2: there, and it was so for products that autocast does not see.  Tiles of 64 x 64; two of 128 x 128 per CU (linear_mid_tiles) lose to the library at depths beyond
+// 1024, many tiles and very few at depths beyond 2048 (layer_ops.linear_mid has the figures).
 extern "C" int jl_linear_mid_ok(int64_t N, int64_t K, int64_t O) {
     if (N <= 0 || K <= 0 || O <= 0) return 0;
     const int64_t tiles = ((N + 63) / 64) * ((O + 63) / 64);
     if ((K <= 1024 && tiles <= 512) || (K <= 2048 && tiles <= 256)) return 2;
-    if (N > 2304 || ((N + 127) / 128) * ((O + 127) / 128) > 512 || K * O > (int64_t)32 << 20) return 0;
-    return K <= 2048 || (K <= 4096 && N >= 300 && tiles <= 512);
+    if (N > 2304 || K > 4096 || K * O > (int64_t)32 << 20) return 0;
+    if (K > 2048) return N >= 300 && tiles >= 80 && tiles <= 256;
+    return ((N + 127) / 128) * ((O + 127) / 128) <= (K <= 1024 ? 512 : 256);
 }
 template <int TM, int TN, int WM, int WN, int RING, bool GATED = false>
 static int linear_mid_launch(const bf16_t *x, int64_t N, int64_t x_ld, const bf16_t *w, int32_t K, int32_t O, const bf16_t *bias, void *out, int64_t out_ld, int32_t out_mode, hipStream_t st, LinearUnit unit = {0, 0.f, 0.f, 0.f}) {

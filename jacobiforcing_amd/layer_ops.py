@@ -384,11 +384,14 @@ def linear_small(n: int, k: int, o: int, itemsize: int) -> bool:
 
 
 def linear_mid(n: int, k: int, o: int, dtype: torch.dtype) -> int:
-    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for some hundred to a few thousand rows (2: under autocast as well): bfloat16 ones of up to 4 KB, up to two 128 x 128
-    tiles per CU, w of up to 64 MB.  There its GPU time is about the library's and the call costs 16 us less of the host, which steps of up to some thousand tokens wait for (a block of four layers of 896 wide by 256
-    tokens 557 -> 354 us).  us of GPU time, library / own: 300 rows of 1024 by 2560 9.5 / 7.8, 1152 of 896 by 2048 11.8 / 11.6, 1196 of 2048 by 1024 14.1 / 13.6, 2048 of 1024 by 2048 16.4 / 15.5,
-    of 4096 by 1024 22.5 / 22.8.  Beyond the line: rows of 8 KB, which the library shares out, 70 of 4096 by 2048 10.7 / 18.4, 1500 32.1 / 41.2; more rows, whose steps wait for the GPU, 3000 of 2048
-    by 2048 29.4 / 32.7, 1024 of 4096 28 / 40; w that takes longer to read than to multiply, 200 of 1024 by 32000 25.2 / 27.5, 256 of 2048 45.3 / 52.4."""
+    """Whether ``linear`` takes n rows of k values times [o, k] to the launch for some hundred to a few thousand bfloat16 rows.  2 (under autocast as well), for any number of rows: up to 512 tiles of 64 x 64
+    where k is up to 1024, up to 256 where it is up to 2048.  1, up to 2304 rows and w of up to 64 MB: k up to 2048 and up to 256 tiles of 128 x 128 (k up to 1024: two of those per CU, 512); k up to 4096
+    from 300 rows on with 80 to 256 tiles of 64 x 64.  There its GPU time is about the library's and the call costs 16 us less of the host, which steps of up to some thousand tokens wait for (a block of four
+    layers of 896 wide by 256 tokens 557 -> 354 us).  us of GPU time, operands from memory, library / own: 300 rows of 512 by 6144 12.1 / 9.8, 1500 of 1536 by 1024 13.2 / 12.1, 1024 of 2048 by 4096 25.2 /
+    24.2, 2048 of 2048 by 2048 24.4 / 24.3, 300 of 4096 by 2048 21.6 / 20.1; two tiles per CU 2048 of 512 by 3072 15.2 / 13.3, of 1024 by 3072 18.4 / 19.1, at worst 1024 of 1024 by 6144 19.2 / 23.9.  Beyond
+    the line: deeper ones of two per CU, 700 of 2048 by 6144 26.8 / 33.3, 2048 of 1536 by 3072 24.6 / 32.8 (safisun's 700 tokens of 2048 wide 875 -> 813 us a pass with those at the library); of 6 and 8 KB
+    many tiles, 700 of 4096 by 2048 25.5 / 31.4, and few, which the library shares out, 512 of 4096 by 512 11.0 / 17.6; more rows, 3000 of 2048 by 512 14.7 / 17.0, 4096 of 1024 by 1024 13.9 / 14.5; w that
+    takes longer to read than to multiply, 256 of 2048 by 32000 45.3 / 52.4."""
     return int(N.layers().jl_linear_mid_ok(n, k, o)) if dtype == torch.bfloat16 else 0
 
 

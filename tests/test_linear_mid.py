@@ -93,3 +93,13 @@ def test_a_sum_in_place_is_seen():
         made = torch.zeros(128, 64, device="cuda", dtype=torch.bfloat16)
         assert LO._host().linear_add(made, x, w) is not NotImplemented
     assert LO._host().linear_add(made, x, w) is NotImplemented
+
+
+def test_where_the_launch_is_the_better_one():
+    from jacobiforcing_amd import _native as N
+    ok = N.layers().jl_linear_mid_ok
+    for want, sizes in ((2, ((1500, 512, 1024), (8192, 1024, 256), (8192, 2048, 64), (2048, 2048, 512))),
+                        (1, ((2304, 1024, 2048), (2048, 1024, 4096), (1024, 2048, 4096), (2048, 2048, 2048), (300, 4096, 1024), (512, 4096, 2048))),
+                        (0, ((2305, 1536, 1024), (700, 2048, 6144), (2048, 1536, 3072), (2048, 1024, 4097), (700, 4096, 2048), (512, 4096, 512), (299, 4096, 2048), (512, 4104, 2048), (256, 2048, 32000)))):
+        for n, k, o in sizes:
+            assert ok(n, k, o) == want, (n, k, o)
