@@ -280,8 +280,8 @@ CALL(rms_norm, 3)
     double eps;
     NEED(take(arg[0], x) && take(arg[1], w) && take(arg[2], eps));
     NEED(x->dim() >= 1 && known(*x) && x->is_contiguous() && w->dim() == 1 && w->scalar_type() == x->scalar_type() && w->is_contiguous() && w->size(0) == x->size(-1) && w->device() == x->device());
-    const int64_t W = w->size(0);
-    NEED(W > 0 && W <= 512 * 8 && x->numel() > 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && !(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())) &&
+    const int64_t W = w->size(0), vec = 16 / x->element_size();
+    NEED(W > 0 && W <= 512 * vec && W % vec == 0 && starts16(*x) && starts16(*w) && x->numel() > 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && !(c10::GradMode::is_enabled() && (x->requires_grad() || w->requires_grad())) &&
          !x->_fw_grad(0).defined() && !w->_fw_grad(0).defined());
     Unlocked others;
     Tensor out = at::empty(x->sizes(), x->options());

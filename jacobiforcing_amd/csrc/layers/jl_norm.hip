@@ -994,48 +994,58 @@ extern "C" int jl_gated_norm(const float *raw, const void *gate, int dtype, int6
 }
 
 // ---- rows of one type, normed and weighted in that type: out = x / sqrt(mean(x^2) + eps) * w -------------------------------------------------------------
-// Bound by its bytes and, for some hundred rows, by the launch: a wavefront per row, whose 16-byte units all leave at once and stay in registers.
-// 2048 rows of 1024 bfloat16 4.7 us (the library's 4.5), and the call takes the host 5 us, the library's 9: nine norms of a block's pass, which waits for the host up to some hundred tokens.
-template <typename T, int VI>
+// Bound by its bytes and, for some hundred rows, by the launch: a wavefront per row of up to 128 units of 16 bytes, or four, whose units all leave at once and stay in registers.
+// us of GPU time, the library's / so, bfloat16: 2048 rows of 1024 4.8 / 4.2, 8192 14.5 / 9.9, 64 of 2048 3.3 / 2.5, 1024
+// 5.1 / 4.1, 64 of 4096 4.3 / 2.9, 2048 10.7 / 10.0, 8192 41 / 30 (a wavefront per row there: 3.7, 5.1, 5.6, 12.6 and 37); and the call takes the host 4.4 us, the library's 7.
+template <typename T, int VI, int WAVES>                            // units a lane, wavefronts a row
 __global__ __launch_bounds__(256) void rms_norm_rows_kernel(const T *__restrict__ x, const T *__restrict__ w, float eps, T *__restrict__ out, int64_t N, int W) {
-    constexpr int VEC = 16 / sizeof(T);
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    constexpr int VEC = 16 / sizeof(T), STEP = 64 * WAVES * VEC;
+    __shared__ float part[WAVES];
+    const int64_t n = WAVES == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
     if (n >= N) return;
-    const int c0 = (threadIdx.x & 63) * VEC;
+    const int c0 = (WAVES == 1 ? threadIdx.x & 63 : threadIdx.x) * VEC;
     float v[VI][VEC], g[VI][VEC], ss = 0.f;
 #pragma unroll
     for (int i = 0; i < VI; ++i)
-        if (c0 + 64 * VEC * i < W) ld16(x + n * W + c0 + 64 * VEC * i, v[i]);
+        if (c0 + STEP * i < W) ld16(x + n * W + c0 + STEP * i, v[i]);
 #pragma unroll
     for (int i = 0; i < VI; ++i)
-        if (c0 + 64 * VEC * i < W) ld16(w + c0 + 64 * VEC * i, g[i]);
+        if (c0 + STEP * i < W) ld16(w + c0 + STEP * i, g[i]);
 #pragma unroll
     for (int i = 0; i < VI; ++i)
-        if (c0 + 64 * VEC * i < W)
+        if (c0 + STEP * i < W)
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ss += v[i][e] * v[i][e];
-    const float r = 1.0f / sqrtf(wave_sum_f32(ss) / (float)W + eps);
+    ss = wave_sum_f32(ss);
+    if (WAVES > 1) {
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) ss += part[i];
+    }
+    const float r = 1.0f / sqrtf(ss / (float)W + eps);
 #pragma unroll
     for (int i = 0; i < VI; ++i)
-        if (c0 + 64 * VEC * i < W) {
+        if (c0 + STEP * i < W) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) g[i][e] *= v[i][e] * r;
-            st16(out + n * W + c0 + 64 * VEC * i, g[i]);
+            st16(out + n * W + c0 + STEP * i, g[i]);
         }
 }
 extern "C" int jl_rms_norm(const void *x, int dtype, const void *w, float eps, void *out, int64_t N, int32_t W, void *stream) {
     if (N <= 0) return JL_OK;
-    const int vec = dtype == JL_BF16 ? 8 : 4;
-    if (!x || !w || !out || W <= 0 || W % vec || W > 64 * 8 * vec || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) || (N + 3) / 4 > 0x7fffffff)
+    const int vec = dtype == JL_BF16 ? 8 : 4, units = W / vec;
+    const int64_t groups = units <= 128 ? (N + 3) / 4 : N;
+    if (!x || !w || !out || W <= 0 || W % vec || units > 512 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) || groups > 0x7fffff)
         return jl_fail(JL_E_INVALID, "jl_rms_norm: rows of up to 512 units of 16 bytes, at 16-byte borders");
-    const dim3 grid((unsigned)((N + 3) / 4));
+    const dim3 grid((unsigned)groups);
     hipStream_t st = (hipStream_t)stream;
-    const int units = (W / vec + 63) / 64;
-#define RN_CASE(VI) JL_DISPATCH(dtype, (rms_norm_rows_kernel<T, VI><<<grid, 256, 0, st>>>((const T *)x, (const T *)w, eps, (T *)out, N, W)))
-    if (units == 1) RN_CASE(1);
-    else if (units == 2) RN_CASE(2);
-    else if (units <= 4) RN_CASE(4);
-    else RN_CASE(8);
+#define RN_CASE(VI, WAVES) JL_DISPATCH(dtype, (rms_norm_rows_kernel<T, VI, WAVES><<<grid, 256, 0, st>>>((const T *)x, (const T *)w, eps, (T *)out, N, W)))
+    if (units <= 64) RN_CASE(1, 1);
+    else if (units <= 128) RN_CASE(2, 1);
+    else if (units <= 256) RN_CASE(1, 4);
+    else RN_CASE(2, 4);
 #undef RN_CASE
     return jl_check_launch("rms_norm_rows_kernel");
 }

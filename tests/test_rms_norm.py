@@ -37,3 +37,19 @@ def test_what_the_library_keeps():
     assert leaf.grad is not None
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert H.rms_norm(x, w, 1e-6) is NotImplemented
+
+
+@pytest.mark.parametrize("W", [1024, 1032, 2048, 2056, 4096])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_row_stays_by_itself(W, dtype):
+    """Rows of one wavefront and of four, of one unit a lane and of two: each what it is alone, beside rows that are zero and not numbers."""
+    from jacobiforcing_amd import layer_ops as LO
+    W = W if dtype == torch.bfloat16 else W // 2
+    g = torch.Generator(device="cuda").manual_seed(W)
+    x, w = torch.randn(9, W, generator=g, device="cuda").to(dtype), torch.randn(W, generator=g, device="cuda").to(dtype)
+    x[2], x[5, W - 1], x[7, 0] = 0, float("nan"), float("inf")
+    got = LO._host().rms_norm(x, w, 1e-6)
+    assert got is not NotImplemented
+    for r in range(9):
+        assert torch.equal(got[r].nan_to_num(7.0), LO._host().rms_norm(x[r:r + 1], w, 1e-6)[0].nan_to_num(7.0)), r
+        assert bool(got[r].isnan().all()) == (r == 5) and (r in (5, 7) or bool(got[r].isfinite().all())), r
