@@ -600,6 +600,11 @@ def _few(batch: RaggedBatch, heads: int, rows: int, tq: int) -> int:
     return most if most * heads <= rows else 0
 
 
+def _token_latent(H: int, D: int, Dv: int) -> bool:
+    """Whether latent rows of D columns, the first Dv of them values, have the sizes of the launches for a few tokens (jl_attn_token.hip) with H heads."""
+    return H <= 32 and D <= (Dv + 127) // 128 * 128 + 64
+
+
 def _token_splits(reach: int, units: int) -> int:
     """Shares of the keys for ``units`` workgroups' worth of rows with up to ``reach`` keys each.  The joining launch has eight shares on their way at once, so more than that from 512 keys a share on
     only (4 tokens at 2000, 16 heads over 1, 8 / 16 / 32 shares 12.4 / 14.8 / 22.7 us)."""
@@ -794,7 +799,7 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
         reach = min(batch.max_pos, chunk + tq) if chunk > 0 else batch.max_pos if window <= 0 else min(batch.max_pos, int(window) + tq)
         # the same over a latent: 32 rows up to 256 values, beyond 16, which read the keys twice as often (us, 4-wavefront tiles of 32 rows / so, latent of 512, 16 heads: 200 tokens at 1000 72 / 42, 1000 at none
         # 148 / 114, 2 x 1000 at 1000 321 / 324, 4 x 2000 998 / 1048)
-        if v_cache.data_ptr() == k_cache.data_ptr() and q.dtype == torch.bfloat16 and H <= 32 and D <= (Dv + 127) // 128 * 128 + 64 and k_cache.stride(0) % 8 == 0 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr()) % 16:
+        if v_cache.data_ptr() == k_cache.data_ptr() and q.dtype == torch.bfloat16 and _token_latent(H, D, Dv) and k_cache.stride(0) % 8 == 0 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr()) % 16:
             few = _few(batch, H, 32, tq) if Dv <= 256 else _few(batch, H, 16, 16 // H) if H <= 16 and (groups < 2 * below or batch.N == batch.B) else 0
         if few:
             tq = tq if Dv <= 256 else 16 // H
@@ -1358,7 +1363,7 @@ def latent_attend(qf: torch.Tensor, pool: torch.Tensor, w_uv: torch.Tensor, batc
     return parts[0] if len(parts) == 1 else torch.cat(parts, 0)
 
 
-# What the two forms of latent attention run at (this card): attention over the latent on the 32-row tiles (wide; few: latents up to 256) and (narrow latents, many rows) the 128-row tiles,
+# What the two forms of latent attention run at (this card): attention over the latent on the 32-row tiles (wide; few: latents up to 256 in the launches for a few tokens) and (narrow latents, many rows) the 128-row tiles,
 # attention over keys and values built per head, the product that builds them.  ``key`` is the time the built form takes per key of its longest tile when the
 # chip is not full (a tile walks its keys in order; the 32-row kernel shares few tiles' keys out).  A layer wholly on built keys has fewer launches (bmm, packing, bmm
 # and head order go: 95 -> 55 us of host time for small steps), a step that mixes the forms has more.  Not counted: the tables of the built form, 70 us of the host and 7 per request
@@ -1379,7 +1384,7 @@ def _latent_built_requests(batch: RaggedBatch, H: int, D: int, R: int, rd: int, 
     chosen = batch._tiles.get(key)
     if chosen is None:
         r = LATENT_RATES if dtype == torch.bfloat16 else LATENT_RATES_FLOAT
-        over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["few"] if R <= 256 else r["wide"])
+        over = 2.0 * H * (2 * R + rd) / (r["narrow"] if R <= 128 and R + rd <= 256 and batch.N * H >= 32 * SWEEP_SPLIT_BELOW_GROUPS else r["few"] if R <= 256 and _token_latent(H, R + rd, R) else r["wide"])
         pair, one = 2.0 * H * (D + rd + Dv) / r["built"], 2.0 * H * R * (D + Dv) / r["product"]
         step = r["key64"] if D + rd <= 128 else r["key32"]
         w, won, attend, chain, keys, chosen = window if window > 0 else 1 << 40, 0.0, 0.0, 0.0, 0, []

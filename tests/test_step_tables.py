@@ -27,6 +27,18 @@ def test_keys_built_per_head_stay_within_their_bytes(monkeypatch, dtype):
         assert len(chosen) == room and sum(b.counts[i] for i in chosen) * H * (D + Dv) * dtype.itemsize <= LO.LATENT_BUILT_BYTES
 
 
+@pytest.mark.parametrize("H,R,rd,token", [(32, 256, 64, True), (40, 256, 64, False), (8, 128, 64, True), (8, 128, 96, False), (16, 512, 64, False)])
+def test_latents_are_priced_by_the_launch_that_takes_them(monkeypatch, H, R, rd, token):
+    """A step over a latent counts at the rate of the launches for a few tokens where attention takes those (heads, rotary columns) and nowhere else."""
+    assert LO._token_latent(H, R + rd, R) == (H <= 32 and R + rd <= R + 64)
+    b, chosen = batch([1000], [0]), []
+    for rate in (1e9, 1e18):
+        monkeypatch.setitem(LO.LATENT_RATES, "few", rate)
+        b._tiles.clear()
+        chosen.append(LO._latent_built_requests(b, H, 128, R, rd, 128, 0))
+    assert chosen == ([[0], []] if token else [chosen[0]] * 2)
+
+
 def test_tiles_of_some_requests_keep_the_order_they_were_asked_for():
     b = batch([5, 3, 9], [0, 7, 2])
     for first in (False, True):
