@@ -47,15 +47,27 @@ def test_one_token_each(D, H, G, Dv, counts, fixed, dtype, act):
     assert torch.equal(state.double(), want_state)                # nobody else's state
 
 
-def test_what_the_wavefronts_keep():
-    """Columns beside fours, states and more tokens than requests: the same numbers by the form before."""
+# columns beside fours, a state beside 16-byte borders, more tokens than requests, more heads than the form takes
+@pytest.mark.parametrize("H,Dv,counts,off", [(2, 18, [1, 1], 0), (2, 16, [1, 1], 1), (2, 16, [2, 1], 0), (2, 16, [1, 3], 0), (3, 20, [4, 0, 2], 0), (1100, 4, [1, 1], 0)])
+def test_what_the_wavefronts_keep(H, Dv, counts, off):
+    """The same numbers by the form before: every token of every request, and the states that it leaves."""
     from jacobiforcing_amd import layer_ops as LO
-    g = torch.Generator(device=dev).manual_seed(1)
-    for Dv, counts in ((18, [1, 1]), (16, [2, 1])):
-        batch = LO.RaggedBatch.build(counts, [3, 0], [0, 1], [[0], [1]], 64, dev)
-        src, state = torch.randn(sum(counts), 2 * 24 + 2 * Dv, generator=g, device=dev), torch.randn(2, 2, 12, Dv, generator=g, device=dev)
-        S, decay = state[0].double(), torch.tensor([0.5, 0.9], device=dev)
-        got = LO.linear_scan(src, (0, 24, 48), batch, 2, 2, 12, Dv, state, act=LO.ACT_NONE, decay=decay)
-        q, k, v = src[0, :24].double().view(2, 12), src[0, 24:48].double().view(2, 12), src[0, 48:].double().view(2, Dv)
-        want = ((decay.double()[:, None, None] * S + k[:, :, None] * v[:, None, :]) * q[:, :, None]).sum(1)
-        assert (got[0].view(2, Dv).double() - want).norm() <= 2.0 ** -20 * want.norm()
+    g = torch.Generator(device=dev).manual_seed(H + Dv)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    B, D, starts = len(counts), 12, [3, 0, 7][:len(counts)]
+    batch = LO.RaggedBatch.build(counts, starts, list(range(B)), [[b] for b in range(B)], 64, dev)
+    src, state = rnd(sum(counts), 2 * H * D + H * Dv), rnd(B * H * D * Dv + off)[off:].view(B, H, D, Dv)
+    assert sum(counts) > B or Dv % 4 or state.data_ptr() % 16 or B * H > 2048
+    kept, decay = state.double(), torch.rand(H, generator=g, device=dev)
+    got, row = LO.linear_scan(src, (0, H * D, 2 * H * D), batch, H, H, D, Dv, state, act=LO.ACT_NONE, decay=decay), 0
+    for b, c in enumerate(counts):
+        S = kept[b] if starts[b] else kept[b] * 0                  # a request that begins has no state
+        A = S.abs()
+        for _ in range(c):
+            q, k, v = src[row, :H * D].double().view(H, D), src[row, H * D:2 * H * D].double().view(H, D), src[row, 2 * H * D:].double().view(H, Dv)
+            new = k[:, :, None] * v[:, None, :]
+            S, A = decay.double()[:, None, None] * S + new, decay.double()[:, None, None] * A + new.abs()
+            # sums of twelve products and what the tokens before have left, a few 2 ** -24 of their sizes each
+            assert bool(((got[row].view(H, Dv).double() - (S * q[:, :, None]).sum(1)).abs() <= 2.0 ** -24 * 64 * (A * q[:, :, None].abs()).sum(1) + 1e-30).all()), (b, row)
+            row += 1
+        assert bool(((state[b].double() - (S if c else kept[b])).abs() <= 2.0 ** -24 * 64 * A * (c > 0)).all()), b
