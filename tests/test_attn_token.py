@@ -143,3 +143,29 @@ def test_scores_scales_and_sinks_to_the_end_of_the_floats(what, H, R, grouped, c
         # weights are rounded to bfloat16; scores of a scale of 3e38 lie around 300, a few 2 ** -24 of which move a weight by less
         assert bool(got.isfinite().all()) and (got - want).norm() <= 2 * 2.0 ** -8 * want.norm(), b
         r0 += c
+
+
+@pytest.mark.parametrize("H,R,rd,pad,counts,starts,splits", [
+    (40, 128, 64, 0, [1, 2], [700, 130], True), (8, 128, 96, 0, [3, 1], [500, 64], True), (4, 256, 64, 4, [1, 1], [900, 31], True), (33, 256, 0, 0, [2], [40], False), (20, 384, 64, 0, [1, 1], [600, 5], True),
+    (32, 512, 64, 0, [1] * 2, [1000, 31], True), (16, 512, 128, 0, [2, 1], [300, 17], True), (8, 128, 64, 4, [40, 3], [100, 0], True),
+])
+def test_latents_that_stay_with_four_wavefronts(monkeypatch, H, R, rd, pad, counts, starts, splits):
+    """More heads, wider rotary columns and rows beside 16-byte borders: attn_sweep_kernel, its keys whole and shared out."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(H * R + rd)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    batch, pages, tokens = _step(counts, starts, 64)
+    n, W, launched, args = sum(counts), R + rd, [], LO._attn_args
+    monkeypatch.setattr(LO, "_attn_args", lambda *a: launched.append(args(*a)) or launched[-1])
+    pool, q, sinks = rnd(tokens, W + pad).bfloat16()[:, :W], rnd(n, H * W).bfloat16(), rnd(H)
+    out, r0 = LO.attn_sweep(q, pool, pool[:, :R], batch, H, 1, W, R, W ** -0.5, 0, sink=sinks), 0
+    assert len(launched) == 1 and launched[0].longest == 0 and (launched[0].splits > 1) == splits
+    for b, (c, s) in enumerate(zip(counts, starts)):
+        tok = torch.tensor([pages[b][j // 64] * 64 + j % 64 for j in range(c + s)], device="cuda")
+        k = pool[tok].double()[:, None].expand(-1, H, -1)
+        i, j = torch.arange(s, s + c, device="cuda").view(-1, 1), torch.arange(c + s, device="cuda").view(1, -1)
+        p, v = _exact(q[r0:r0 + c].double().view(c, H, W), k, k[..., :R], W ** -0.5, j <= i, sinks)
+        want = (p @ v).permute(1, 0, 2)
+        # weights and results are rounded to bfloat16, 2 ** -9 each
+        assert (out[r0:r0 + c].double().view(c, H, R) - want).norm() <= 2 * 2.0 ** -8 * want.norm(), b
+        r0 += c
