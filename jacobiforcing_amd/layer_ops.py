@@ -801,6 +801,9 @@ def attn_sweep(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, ba
         # 148 / 114, 2 x 1000 at 1000 321 / 324, 4 x 2000 998 / 1048)
         if v_cache.data_ptr() == k_cache.data_ptr() and q.dtype == torch.bfloat16 and _token_latent(H, D, Dv) and k_cache.stride(0) % 8 == 0 and _fours(out) and not (q.data_ptr() | k_cache.data_ptr()) % 16:
             few = _few(batch, H, 32, tq) if Dv <= 256 else _few(batch, H, 16, 16 // H) if H <= 16 and (groups < 2 * below or batch.N == batch.B) else 0
+            # smaller tiles than the other form's may have to be copied where that one's came with the batch: not while a graph is captured
+            if few and Dv > 256 and 16 // H not in batch._tiles and (batch._whole is None or batch._whole[0] > 16 // H) and torch.cuda.is_current_stream_capturing():
+                few = 0
         if few:
             tq = tq if Dv <= 256 else 16 // H
             tiles = batch.tiles(tq)

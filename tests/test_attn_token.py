@@ -169,3 +169,24 @@ def test_latents_that_stay_with_four_wavefronts(monkeypatch, H, R, rd, pad, coun
         # weights and results are rounded to bfloat16, 2 ** -9 each
         assert (out[r0:r0 + c].double().view(c, H, R) - want).norm() <= 2 * 2.0 ** -8 * want.norm(), b
         r0 += c
+
+
+@pytest.mark.parametrize("H,R,counts", [(16, 512, [2, 1]), (8, 512, [4, 3]), (16, 128, [2, 1]), (16, 512, [1, 1])])
+def test_latents_in_a_graph(H, R, counts):
+    """Portions that the batch's own tables hold in the tiles of one form: a graph of a step that nothing has run before takes that form, and replays it."""
+    from jacobiforcing_amd import layer_ops as LO
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    (batch, _, tokens), (again, _, _) = _step(counts, [700, 90], 64), _step(counts, [700, 90], 64)
+    W = R + 64
+    pool, q = rnd(tokens, W), rnd(sum(counts), H * W)
+    run = lambda b: LO.attn_sweep(q, pool, pool[:, :R], b, H, 1, W, R, W ** -0.5, 0)
+    want = run(batch).double()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run(again)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (got.double() - want).norm() <= 2 * 2.0 ** -8 * want.norm()      # weights and results are rounded to bfloat16, 2 ** -9 each
