@@ -1161,7 +1161,7 @@ def gated_norm(raw: torch.Tensor, gate: torch.Tensor, w: torch.Tensor, eps: floa
 
 
 # A row alone (decoding for one user) and up to four go from a norm, a unit or a gate into the product in one launch, every workgroup of which makes the rows for itself (linear_after_kernel,
-# jl_linear_after_ok); others take the two calls.  us a pass of one token through four layers, 1024 wide: 311 in launches of their own (49), 264 so (34).
+# jl_linear_after_ok); others take the two calls.  us a pass of one token through four layers, 1024 wide: 311 in launches of their own (49), 254 so (34).
 def norm_linear(x: torch.Tensor, y: Optional[torch.Tensor], w_post: Optional[torch.Tensor], eps: float, w_next: torch.Tensor, add_row: Optional[torch.Tensor], w: torch.Tensor,
                 bias: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """``sandwich_norm`` into w's dtype and ``linear`` of its result: the updated x (x itself, or another tensor, x as it was) and the product."""
